@@ -48,6 +48,21 @@ template <> struct Mfma16<f16_t> {
     __device__ static f32x4_t run(Frag a, Frag b, f32x4_t c) { return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0); }
 };
 
+// One step of a 16 x 16 tile from 16-byte packets: lane l holds packet l/16 (of four) of row l%16 on either side, 32 k values for
+// the 16-bit types (one v_mfma_f32_16x16x32), 16 for fp32 (four v_mfma_f32_16x16x4_f32, instruction q multiplying element q of
+// the four packets).  D layout as Mfma16.
+template <typename T> __device__ inline f32x4_t mfma16_packet(u32x4_t a, u32x4_t b, f32x4_t c) {
+    if constexpr (sizeof(T) == 4) {
+        const f32x4_t av = __builtin_bit_cast(f32x4_t, a), bv = __builtin_bit_cast(f32x4_t, b);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) c = __builtin_amdgcn_mfma_f32_16x16x4f32(av[q], bv[q], c, 0, 0, 0);
+        return c;
+    } else {
+        using Frag = typename Mfma16<T>::Frag;
+        return Mfma16<T>::run(__builtin_bit_cast(Frag, a), __builtin_bit_cast(Frag, b), c);
+    }
+}
+
 // What the tiled kernel needs to know about a fragment shape: FR = rows (and columns) of a fragment, kChunks = 16-byte
 // pieces of a row one k-step consumes (lane l reads piece l / FR of its row l % FR), Acc with kAccRegs registers, register
 // v of lane l holding D[8*(v/4) + 4*(l/FR) + v%4][l % FR] (both shapes).

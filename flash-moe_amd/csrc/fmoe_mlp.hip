@@ -8,7 +8,7 @@
 //      and up products never go to memory.
 //   2. down: plain epilogue, optional residual add (the routed-expert output in the block).
 //
-// Main kernel (gemm_dma_kernel), used when the extents are multiples of the tile: tiles go global -> LDS
+// Main kernel (gemm_dma_kernel): tiles go global -> LDS
 // directly (global_load_lds_dwordx4, no staging registers) into NSTAGE LDS stages, issued NSTAGE-1 k-tiles
 // ahead of their use; one workgroup barrier per k-tile; MFMA fragments (v_mfma_f32_16x16x32 for the 16-bit types) are
 // read with 16-byte ds_reads.  An LDS row is one k-tile of one matrix row; its 16-byte chunks are XOR-swizzled with a key built
@@ -20,182 +20,24 @@
 // fp32 runs the same kernel on v_mfma_f32_32x32x2_f32: an LDS row is again 128 bytes (32 values), a fragment again one
 // 16-byte read, and four matrix instructions use it.
 //
-// Ragged shapes take gemm_nt_kernel (register-staged, bounds-checked), in fp32 a plain FMA kernel.
+// Extents that are no multiples of the tile run the same kernel with range-checked buffer loads (RAGGED); few output tiles take
+// gemm_splitk_kernel; fp32 whose rows are no multiples of 16 bytes takes a plain FMA kernel.
 #include "fmoe_common.h"
 #include "fmoe_mfma.h"
 
 namespace fmoe {
 namespace {
 
-constexpr int kGemmThreads = 256;
-constexpr int BK = kTileK;        // k extent of a register-staged LDS tile (elements)
-constexpr int kChunksPerRow = kTileChunks;
-
 enum Epilogue { kEpiSwiGLU = 0, kEpiPlain = 1, kEpiDual = 2 };   // Dual: the product in T and, through R, in fp32
 template <bool B> struct Flag { static constexpr bool value = B; };
-
-template <typename T, int BM, int BN, int EPI>
-__global__ __launch_bounds__(kGemmThreads) void gemm_nt_kernel(
-    const T* __restrict__ A, const T* __restrict__ B0, const T* __restrict__ B1, T* __restrict__ C,
-    const T* __restrict__ R, int M, int N, int K, int tiles_m, int tiles_n, int xcds) {
-    using Frag = typename Mfma32<T>::Frag;
-    constexpr int WM = BM / 2, WN = BN / 2;        // per-wave tile
-    constexpr int MF = WM / 32, NF = WN / 32;      // 32x32 fragments per wave
-    constexpr int A_CHUNKS = BM * kChunksPerRow / kGemmThreads;
-    constexpr int B_CHUNKS = BN * kChunksPerRow / kGemmThreads;
-    constexpr int BN_OUT = (EPI == kEpiSwiGLU) ? BN / 2 : BN;   // output columns per tile
-
-    __shared__ __attribute__((aligned(16))) T As[BM * BK];
-    __shared__ __attribute__((aligned(16))) T Bs[BN * BK];
-
-    int tm, tn;
-    tile_of_block(tiles_m, tiles_n, xcds, tm, tn);
-    const int m0 = tm * BM;
-    const int n0 = tn * BN_OUT;
-
-    const int tid = (int)threadIdx.x;
-    const int lane = tid & 63;
-    const int wave = tid >> 6;
-    const int wm = wave >> 1, wn = wave & 1;
-
-    const u32x4_t zero4 = {0u, 0u, 0u, 0u};
-    u32x4_t ra[A_CHUNKS], rb[B_CHUNKS];
-
-    auto load_global = [&](int k0) {
-#pragma unroll
-        for (int it = 0; it < A_CHUNKS; ++it) {
-            const int q = it * kGemmThreads + tid;
-            const int row = q / kChunksPerRow, ch = q % kChunksPerRow;
-            const int gm = m0 + row, gk = k0 + ch * 8;
-            ra[it] = (gm < M && gk < K) ? *reinterpret_cast<const u32x4_t*>(A + (int64_t)gm * K + gk) : zero4;
-        }
-#pragma unroll
-        for (int it = 0; it < B_CHUNKS; ++it) {
-            const int q = it * kGemmThreads + tid;
-            const int row = q / kChunksPerRow, ch = q % kChunksPerRow;
-            const int gk = k0 + ch * 8;
-            const T* base;
-            int gn;
-            if (EPI == kEpiSwiGLU) {
-                const bool is_up = row >= BN / 2;
-                base = is_up ? B1 : B0;
-                gn = n0 + (is_up ? row - BN / 2 : row);
-            } else {
-                base = B0;
-                gn = n0 + row;
-            }
-            rb[it] = (gn < N && gk < K) ? *reinterpret_cast<const u32x4_t*>(base + (int64_t)gn * K + gk) : zero4;
-        }
-    };
-    auto store_lds = [&]() {
-#pragma unroll
-        for (int it = 0; it < A_CHUNKS; ++it) {
-            const int q = it * kGemmThreads + tid;
-            *reinterpret_cast<u32x4_t*>(&As[swizzled_offset(q / kChunksPerRow, q % kChunksPerRow)]) = ra[it];
-        }
-#pragma unroll
-        for (int it = 0; it < B_CHUNKS; ++it) {
-            const int q = it * kGemmThreads + tid;
-            *reinterpret_cast<u32x4_t*>(&Bs[swizzled_offset(q / kChunksPerRow, q % kChunksPerRow)]) = rb[it];
-        }
-    };
-
-    f32x16_t acc[MF][NF];
-#pragma unroll
-    for (int i = 0; i < MF; ++i)
-#pragma unroll
-        for (int j = 0; j < NF; ++j)
-#pragma unroll
-            for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.0f;
-
-    // LDS row of this lane inside fragment f of the wave's A / B sub-tile
-    const int frag_row = lane & 31;
-    const int frag_half = lane >> 5;   // which 8 of the 16 k values of one MFMA this lane supplies
-    int b_row[NF];
-#pragma unroll
-    for (int j = 0; j < NF; ++j) {
-        if (EPI == kEpiSwiGLU)
-            b_row[j] = (j < NF / 2) ? wn * (BN / 4) + j * 32 + frag_row
-                                    : BN / 2 + wn * (BN / 4) + (j - NF / 2) * 32 + frag_row;
-        else
-            b_row[j] = wn * WN + j * 32 + frag_row;
-    }
-
-    const int k_tiles = (K + BK - 1) / BK;
-    load_global(0);
-    store_lds();
-    __syncthreads();
-
-    for (int kt = 0; kt < k_tiles; ++kt) {
-        if (kt + 1 < k_tiles) load_global((kt + 1) * BK);
-#pragma unroll
-        for (int ks = 0; ks < BK / 16; ++ks) {
-            const int chunk = ks * 2 + frag_half;
-            Frag fa[MF], fb[NF];
-#pragma unroll
-            for (int i = 0; i < MF; ++i)
-                fa[i] = *reinterpret_cast<const Frag*>(&As[swizzled_offset(wm * WM + i * 32 + frag_row, chunk)]);
-#pragma unroll
-            for (int j = 0; j < NF; ++j) fb[j] = *reinterpret_cast<const Frag*>(&Bs[swizzled_offset(b_row[j], chunk)]);
-#pragma unroll
-            for (int i = 0; i < MF; ++i)
-#pragma unroll
-                for (int j = 0; j < NF; ++j) acc[i][j] = Mfma32<T>::run(fa[i], fb[j], acc[i][j]);
-        }
-        __syncthreads();
-        if (kt + 1 < k_tiles) {
-            store_lds();
-            __syncthreads();
-        }
-    }
-
-    // D fragment layout of v_mfma_f32_32x32x*: lane l, register v holds
-    //   row = 8*(v/4) + 4*(l/32) + (v%4)   (A / M index),   col = l%32   (B / N index)
-    if (EPI == kEpiSwiGLU) {
-#pragma unroll
-        for (int i = 0; i < MF; ++i)
-#pragma unroll
-            for (int j = 0; j < NF / 2; ++j) {
-                const int col = n0 + wn * (BN / 4) + j * 32 + frag_row;
-#pragma unroll
-                for (int v = 0; v < 16; ++v) {
-                    const int row = m0 + wm * WM + i * 32 + 8 * (v / 4) + 4 * frag_half + (v % 4);
-                    if (row < M && col < N) {
-                        const float g = acc[i][j][v], u = acc[i][j + NF / 2][v];
-                        C[(int64_t)row * N + col] = Elem<T>::from_f32(silu_f32(g) * u);
-                        if (R != nullptr) {   // planes [0] and [1] of a [2, M, N] buffer keep the two products
-                            const_cast<T*>(R)[(int64_t)row * N + col] = Elem<T>::from_f32(g);
-                            const_cast<T*>(R)[((int64_t)M + row) * N + col] = Elem<T>::from_f32(u);
-                        }
-                    }
-                }
-            }
-    } else {
-#pragma unroll
-        for (int i = 0; i < MF; ++i)
-#pragma unroll
-            for (int j = 0; j < NF; ++j) {
-                const int col = n0 + wn * WN + j * 32 + frag_row;
-#pragma unroll
-                for (int v = 0; v < 16; ++v) {
-                    const int row = m0 + wm * WM + i * 32 + 8 * (v / 4) + 4 * frag_half + (v % 4);
-                    if (row < M && col < N) {
-                        float r = acc[i][j][v];
-                        if (R != nullptr) r += Elem<T>::to_f32(R[(int64_t)row * N + col]);
-                        C[(int64_t)row * N + col] = Elem<T>::from_f32(r);
-                    }
-                }
-            }
-    }
-}
-
+constexpr uint32_t kOutOfRange = 0x80000000u;    // beyond every buffer descriptor here: loads give zeros, stores are dropped
 
 // ------------------------------------------------------------------------------------------------------------
 // LDS-DMA pipelined kernel.  WAVES_M x WAVES_N waves, each (BM/WAVES_M) x (BN/WAVES_N); BKT = k extent of a stage.
 // ------------------------------------------------------------------------------------------------------------
 // FR: fragment shape (32: v_mfma_f32_32x32x16 / 32x32x2; 16: v_mfma_f32_16x16x32).  SPLIT: a k-step's A fragments are read and
 // multiplied in SPLIT parts (its B fragments stay for the whole k-step), which halves the registers the read-ahead needs.
-template <typename T, int BM, int BN, int WAVES_M, int WAVES_N, int BKT, int NSTAGE, int EPI, int PF, int FR = 32, int SPLIT = 1>
+template <typename T, int BM, int BN, int WAVES_M, int WAVES_N, int BKT, int NSTAGE, int EPI, int PF, int FR = 32, int SPLIT = 1, bool RAGGED = false>
 __global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void gemm_dma_kernel(
     const T* __restrict__ A, const T* __restrict__ B0, const T* __restrict__ B1, T* __restrict__ C,
     const T* __restrict__ R, int M, int N, int K, int tiles_m, int tiles_n, int xcds) {
@@ -240,7 +82,15 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void gemm_dma_kernel(
     // tile.  What the MFMAs make of those rows is never stored (the epilogue's buffer stores are bounds-checked).
     uint32_t a_lane_off[A_ROUNDS];
     const T *a_src, *b_src0, *b_src1 = nullptr;
+    // RAGGED: rows and the k tail are cut off by the range check of buffer descriptors over the rest of each matrix
+    __amdgpu_buffer_rsrc_t a_rsrc, b_rsrc0, b_rsrc1;
     int m0, n0;
+    const int k_tiles = (K + BKT - 1) / BKT;
+    const bool lane_in_tail = (k_tiles - 1) * BKT + (lp ^ key_dma) * EPC < K;      // the lane's chunk of the last k-tile exists
+    auto rest_of = [&](const T* base, int64_t rows) {                              // descriptor from `base` to the end of its matrix
+        const int64_t bytes = rows * K * (int64_t)sizeof(T);
+        return __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(base), 0, (int)(bytes < 0x7FFFFFFFll ? bytes : 0x7FFFFFFFll), 0x00020000);
+    };
     // The workgroup is persistent: it takes tiles t, t + gridDim.x, ...  Each XCD (workgroup id mod 8) gets a contiguous
     // run of the tile order, walked 8 tile-rows at a time so that a compact patch shares A and B tiles in the XCD's L2.
     auto set_tile = [&](int t) {
@@ -254,14 +104,37 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void gemm_dma_kernel(
 #pragma unroll
         for (int r = 0; r < A_ROUNDS; ++r) {
             int row = r * ROWS_PER_IT + wave * RPI + lrow;
-            row = m0 + row < M ? row : M - 1 - m0;
+            if (!RAGGED) row = m0 + row < M ? row : M - 1 - m0;
             a_lane_off[r] = (uint32_t)(row * K + (lp ^ key_dma) * EPC) * (uint32_t)sizeof(T);
         }
         b_src0 = B0 + (int64_t)(n0 + wave * RPI) * K;
         if (EPI == kEpiSwiGLU) b_src1 = B1 + (int64_t)(n0 + wave * RPI) * K;
+        if constexpr (RAGGED) {
+            a_rsrc = rest_of(a_src, M - m0);
+            b_rsrc0 = rest_of(B0 + (int64_t)n0 * K, N - n0);
+            if (EPI == kEpiSwiGLU) b_rsrc1 = rest_of(B1 + (int64_t)n0 * K, N - n0);
+        }
     };
     auto issue = [&](int kt, T* stage) {
         const int k0 = kt * BKT;
+        if constexpr (RAGGED) {
+            const bool drop = kt + 1 == k_tiles && !lane_in_tail;
+#pragma unroll
+            for (int r = 0; r < A_ROUNDS; ++r)
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(
+                    a_rsrc, (__attribute__((address_space(3))) void*)(stage + (r * ROWS_PER_IT + wave * RPI) * BKT), 16,
+                    (int)(drop ? kOutOfRange : a_lane_off[r]), k0 * (int)sizeof(T), 0, 0);
+#pragma unroll
+            for (int r = 0; r < B_ROUNDS; ++r) {
+                const bool second = EPI == kEpiSwiGLU && r >= B_ROUNDS / 2;
+                const uint32_t off = (uint32_t)(((second ? r - B_ROUNDS / 2 : r) * ROWS_PER_IT + wave * RPI) * K) * (uint32_t)sizeof(T) + lane_off;
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(
+                    second ? b_rsrc1 : b_rsrc0,
+                    (__attribute__((address_space(3))) void*)(stage + BM * BKT + (r * ROWS_PER_IT + wave * RPI) * BKT), 16,
+                    (int)(drop ? kOutOfRange : off), k0 * (int)sizeof(T), 0, 0);
+            }
+            return;
+        }
 #pragma unroll
         for (int r = 0; r < A_ROUNDS; ++r)
             __builtin_amdgcn_global_load_lds(
@@ -295,7 +168,6 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void gemm_dma_kernel(
 #pragma unroll
     for (int ks = 0; ks < KSTEPS; ++ks) pc[ks] = ((ks * Shape::kChunks + fhalf) ^ key_f) << 4;
 
-    const int k_tiles = K / BKT;
     int tile = (int)blockIdx.x;
     if (tile >= num_tiles) return;
     set_tile(tile);
@@ -402,13 +274,19 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void gemm_dma_kernel(
         //   row = 8*(v/4) + 4*(l/FR) + (v%4)   (A / M index),   col = l%FR   (B / N index)
         // Buffer addressing: a wave-uniform descriptor of the rows from the wave's first one on, a scalar byte offset
         // per (fragment, register) and one 32-bit byte offset per lane - no vector address arithmetic per element.
-        const int lane_bytes = ((4 * fhalf) * N + frow) * (int)sizeof(T);
+        const int lane_bytes0 = ((4 * fhalf) * N + frow) * (int)sizeof(T);
         const int64_t wave_off = (int64_t)(out_m0 + wm * WM) * N + out_n0 + wn * ((EPI == kEpiSwiGLU) ? WN / 2 : WN);
         const int64_t span = ((int64_t)M * N - wave_off) * (int64_t)sizeof(T);
         // a wave whose rows all lie beyond M gets an empty descriptor: every access of it is dropped
         const int span32 = (int)(span < 0 ? 0 : (span < 0x7FFFFFFFll ? span : 0x7FFFFFFFll));
         auto c_rsrc = __builtin_amdgcn_make_buffer_rsrc(C + wave_off, 0, span32, 0x00020000);
-        auto store_to = [&](auto rsrc, int uni_bytes, float value) {
+        // RAGGED: a lane whose column of fragment column j lies beyond N takes an offset no descriptor covers
+        auto lane_at = [&](int j, int in_range) {
+            if (!RAGGED) return in_range;
+            const int col = out_n0 + wn * ((EPI == kEpiSwiGLU) ? WN / 2 : WN) + j * FR + frow;
+            return col < N ? in_range : (int)kOutOfRange;
+        };
+        auto store_to = [&](auto rsrc, int lane_bytes, int uni_bytes, float value) {
             if constexpr (sizeof(T) == 4) {
                 __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, value), rsrc, lane_bytes, uni_bytes, 0);
             } else {
@@ -416,7 +294,6 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void gemm_dma_kernel(
                 __builtin_amdgcn_raw_buffer_store_b16(__builtin_bit_cast(short, t), rsrc, lane_bytes, uni_bytes, 0);
             }
         };
-        auto store_elem = [&](int uni_bytes, float value) { store_to(c_rsrc, uni_bytes, value); };
         // 16-bit outputs round once, so the fast reciprocal's last-bit error is invisible; fp32 divides
         auto silu = [](float v) { return sizeof(T) == 4 ? silu_f32(v) : silu_fast_f32(v); };
         // element offset of (fragment i, fragment column j, register v) from the wave's first output element
@@ -434,8 +311,8 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void gemm_dma_kernel(
 #pragma unroll
                         for (int v = 0; v < NV; ++v) {
                             const int uni = elem_at(i, j, v) * (int)sizeof(T);
-                            store_to(g_rsrc, uni, acc[i][j][v]);
-                            store_to(u_rsrc, uni, acc[i][j + NF / 2][v]);
+                            store_to(g_rsrc, lane_at(j, lane_bytes0), uni, acc[i][j][v]);
+                            store_to(u_rsrc, lane_at(j, lane_bytes0), uni, acc[i][j + NF / 2][v]);
                         }
             }
 #pragma unroll
@@ -444,7 +321,7 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void gemm_dma_kernel(
                 for (int j = 0; j < NF / 2; ++j)
 #pragma unroll
                     for (int v = 0; v < NV; ++v)
-                        store_elem(elem_at(i, j, v) * (int)sizeof(T), silu(acc[i][j][v]) * acc[i][j + NF / 2][v]);
+                        store_to(c_rsrc, lane_at(j, lane_bytes0), elem_at(i, j, v) * (int)sizeof(T), silu(acc[i][j][v]) * acc[i][j + NF / 2][v]);
         } else if (EPI == kEpiDual) {
             // R points at an fp32 [M, N] buffer that receives the unrounded sums next to the rounded ones in C
             float* out32 = reinterpret_cast<float*>(const_cast<T*>(R));
@@ -460,8 +337,8 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void gemm_dma_kernel(
                     for (int v = 0; v < NV; ++v) {
                         const int at = elem_at(i, j, v);
                         const float sum = acc[i][j][v];      // a scalar copy: the bit cast below must not see a vector element
-                        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, sum), f_rsrc, lane_bytes_f, at * 4, 0);
-                        store_elem(at * (int)sizeof(T), sum);
+                        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, sum), f_rsrc, lane_at(j, lane_bytes_f), at * 4, 0);
+                        store_to(c_rsrc, lane_at(j, lane_bytes0), at * (int)sizeof(T), sum);
                     }
         } else {
             auto r_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(R != nullptr ? R + wave_off : C), 0,
@@ -471,6 +348,7 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void gemm_dma_kernel(
 #pragma unroll
                 for (int j = 0; j < NF; ++j) {
                     float res[NV];
+                    const int lane_bytes = lane_at(j, lane_bytes0);
 #pragma unroll
                     for (int v = 0; v < NV; ++v) {
                         const int uni = elem_at(i, j, v) * (int)sizeof(T);
@@ -482,11 +360,114 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void gemm_dma_kernel(
                         }
                     }
 #pragma unroll
-                    for (int v = 0; v < NV; ++v) store_elem(elem_at(i, j, v) * (int)sizeof(T), acc[i][j][v] + res[v]);
+                    for (int v = 0; v < NV; ++v) store_to(c_rsrc, lane_bytes, elem_at(i, j, v) * (int)sizeof(T), acc[i][j][v] + res[v]);
                 }
         }
         if (next >= num_tiles) break;
         tile = next;
+    }
+}
+
+// ------------------------------------------------------------------------------------------------------------
+// Few output tiles: the waves of a workgroup share one small tile and split k.  Every wave takes its fragments straight from
+// global memory (a fragment is 16 rows of 64 bytes: lane l reads 16-byte piece l / 16 of row l % 16), kAhead k-steps ahead and
+// without a barrier; the waves' sums meet in LDS, added in wave order.  Rows beyond M or N and the k tail read as zeros (range
+// check of the descriptors).  fp32: a 16-byte piece is four k values, one per v_mfma_f32_16x16x4.
+// Bound by latency (about 4 us for a launch of one short wave per SIMD) and by what the L2s deliver (about 13 TB/s over the
+// chip): the 1024 x 4096 down product takes 7.4 us for one token and 11 us for 64 where 64 x 64 tiles with the whole k loop in
+// one chain take 14.3 us; from about 128 tokens on the larger tiles' smaller traffic wins.  Loads of whole lines (8 rows of 128
+// bytes, fragments rebuilt with lane rotations) were no faster.
+// ------------------------------------------------------------------------------------------------------------
+constexpr int kSplitWaves = 8;
+
+template <typename T, int MT, int NT, int EPI>
+__global__ __launch_bounds__(kSplitWaves * 64) void gemm_splitk_kernel(
+    const T* __restrict__ A, const T* __restrict__ B0, const T* __restrict__ B1, T* __restrict__ C,
+    const T* __restrict__ R, int M, int N, int K, int tiles_m, int tiles, int xcds) {
+    constexpr int BM = 16 * MT, BN = 16 * NT;
+    constexpr int NB = EPI == kEpiSwiGLU ? 2 * NT : NT;          // B fragments: gate rows, then the same up rows
+    constexpr int F = MT * NB;
+    constexpr int kAhead = MT + NB <= 3 ? 8 : 4;
+    constexpr int kStep = 64 / (int)sizeof(T);                   // k values of a step
+    __shared__ __attribute__((aligned(16))) f32x4_t sums[kSplitWaves][F][64];
+    const int tid = (int)threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    // XCD b % xcds takes a contiguous run of the tiles, all rows of a column first: its L2 holds B's part of the run only
+    const int tile = (int)(blockIdx.x % xcds) * ((int)gridDim.x / xcds) + (int)(blockIdx.x / xcds);
+    if (tile >= tiles) return;
+    const int m0 = (tile % tiles_m) * BM, n0 = (tile / tiles_m) * BN;
+    auto rest_of = [&](const T* base, int64_t rows) {
+        const int64_t bytes = rows * K * (int64_t)sizeof(T);
+        return __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(base), 0, (int)(bytes < 0x7FFFFFFFll ? bytes : 0x7FFFFFFFll), 0x00020000);
+    };
+    const __amdgpu_buffer_rsrc_t ar = rest_of(A + (int64_t)m0 * K, M - m0), br = rest_of(B0 + (int64_t)n0 * K, N - n0);
+    const __amdgpu_buffer_rsrc_t br1 = EPI == kEpiSwiGLU ? rest_of(B1 + (int64_t)n0 * K, N - n0) : br;
+    const int frow = lane & 15, piece = lane >> 4;
+    uint32_t row_off[MT > NT ? MT : NT];
+#pragma unroll
+    for (int i = 0; i < (MT > NT ? MT : NT); ++i) row_off[i] = (uint32_t)((i * 16 + frow) * K) * (uint32_t)sizeof(T) + (uint32_t)piece * 16u;
+    const int steps = (K + kStep - 1) / kStep;
+    const int share = ((steps + 2 * kSplitWaves - 1) / (2 * kSplitWaves)) * 2;       // two steps are one 128-byte line of a row
+    const int first = wave * share, last = first + share < steps ? first + share : steps;
+    const bool in_tail = (steps - 1) * kStep + piece * (16 / (int)sizeof(T)) < K;
+    u32x4_t fa[kAhead][MT], fb[kAhead][NB];
+    auto load = [&](int step, u32x4_t (&a)[MT], u32x4_t (&b)[NB]) {
+        const bool drop = step >= last || (step + 1 == steps && !in_tail);
+        const int at = step * 64;
+#pragma unroll
+        for (int i = 0; i < MT; ++i) a[i] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(ar, (int)(drop ? kOutOfRange : row_off[i]), at, 0));
+#pragma unroll
+        for (int j = 0; j < NB; ++j)
+            b[j] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(j < NT ? br : br1, (int)(drop ? kOutOfRange : row_off[j % NT]), at, 0));
+    };
+    f32x4_t acc[MT][NB];
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < NB; ++j) acc[i][j] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) load(first + u, fa[u], fb[u]);
+    for (int s0 = first; s0 < last; s0 += kAhead) {
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u) {
+#pragma unroll
+            for (int i = 0; i < MT; ++i)
+#pragma unroll
+                for (int j = 0; j < NB; ++j) acc[i][j] = mfma16_packet<T>(fa[u][i], fb[u][j], acc[i][j]);
+            load(s0 + u + kAhead, fa[u], fb[u]);
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < NB; ++j) sums[wave][i * NB + j][lane] = acc[i][j];
+    __syncthreads();
+    // four rows of one column per (fragment, lane)
+    for (int q = tid; q < MT * NT * 64; q += kSplitWaves * 64) {
+        const int f = q >> 6, l = q & 63, i = f / NT, j = f % NT;
+        f32x4_t g = sums[0][i * NB + j][l], u = {0.0f, 0.0f, 0.0f, 0.0f};
+        for (int w = 1; w < kSplitWaves; ++w) g += sums[w][i * NB + j][l];
+        if (EPI == kEpiSwiGLU) {
+            u = sums[0][i * NB + NT + j][l];
+            for (int w = 1; w < kSplitWaves; ++w) u += sums[w][i * NB + NT + j][l];
+        }
+        const int col = n0 + j * 16 + (l & 15);
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const int row = m0 + i * 16 + 4 * (l >> 4) + v;
+            if (row >= M || col >= N) continue;
+            const int64_t at = (int64_t)row * N + col;
+            if (EPI == kEpiSwiGLU) {
+                const float act = sizeof(T) == 4 ? silu_f32(g[v]) : silu_fast_f32(g[v]);
+                C[at] = Elem<T>::from_f32(act * u[v]);
+                if (R != nullptr) {      // planes [0] and [1] of a [2, M, N] buffer keep the two products
+                    const_cast<T*>(R)[at] = Elem<T>::from_f32(g[v]);
+                    const_cast<T*>(R)[(int64_t)M * N + at] = Elem<T>::from_f32(u[v]);
+                }
+            } else {
+                C[at] = Elem<T>::from_f32(R != nullptr ? g[v] + Elem<T>::to_f32(R[at]) : g[v]);
+            }
+        }
     }
 }
 
@@ -549,18 +530,10 @@ __global__ __launch_bounds__(256) void sgemm_nt_kernel(const float* __restrict__
         }
 }
 
-template <typename T, int BM, int BN, int EPI>
-void launch_gemm(const T* A, const T* B0, const T* B1, T* C, const T* R, int M, int N, int K, hipStream_t stream) {
-    constexpr int BN_OUT = (EPI == kEpiSwiGLU) ? BN / 2 : BN;
-    const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN_OUT - 1) / BN_OUT;
-    hipLaunchKernelGGL((gemm_nt_kernel<T, BM, BN, EPI>), dim3((unsigned)(tiles_m * tiles_n)), dim3(kGemmThreads), 0,
-                       stream, A, B0, B1, C, R, M, N, K, tiles_m, tiles_n, chip_info().xcds);
-}
-
-template <typename T, int BM, int BN, int WAVES_M, int WAVES_N, int BKT, int NSTAGE, int EPI, int PF, int FR = 32, int SPLIT = 1>
+template <typename T, int BM, int BN, int WAVES_M, int WAVES_N, int BKT, int NSTAGE, int EPI, int PF, int FR = 32, int SPLIT = 1, bool RAGGED = false>
 void launch_gemm_dma(const T* A, const T* B0, const T* B1, T* C, const T* R, int M, int N, int K, hipStream_t stream) {
     constexpr int BN_OUT = (EPI == kEpiSwiGLU) ? BN / 2 : BN;
-    const int tiles_m = (M + BM - 1) / BM, tiles_n = N / BN_OUT;      // a ragged last row of tiles is allowed
+    const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN_OUT - 1) / BN_OUT;      // without RAGGED only a ragged last row of tiles is allowed
     // persistent workgroups: as many as are resident at once (LDS-limited), a multiple of 8 so that the XCD patches hold
     constexpr int kStageBytes = (BM + BN) * BKT * (int)sizeof(T) * NSTAGE;
     constexpr int kPerCu = (160 * 1024 / kStageBytes) < 1 ? 1 : ((160 * 1024 / kStageBytes) > 2 ? 2 : (160 * 1024 / kStageBytes));
@@ -568,8 +541,16 @@ void launch_gemm_dma(const T* A, const T* B0, const T* B1, T* C, const T* R, int
     const ChipInfo& chip = chip_info();
     const int resident = chip.cus * kPerCu;
     const int grid = total < resident ? total : resident;
-    hipLaunchKernelGGL((gemm_dma_kernel<T, BM, BN, WAVES_M, WAVES_N, BKT, NSTAGE, EPI, PF, FR, SPLIT>), dim3((unsigned)grid),
+    hipLaunchKernelGGL((gemm_dma_kernel<T, BM, BN, WAVES_M, WAVES_N, BKT, NSTAGE, EPI, PF, FR, SPLIT, RAGGED>), dim3((unsigned)grid),
                        dim3(WAVES_M * WAVES_N * 64), 0, stream, A, B0, B1, C, R, M, N, K, tiles_m, tiles_n, chip.xcds);
+}
+
+template <typename T, int MT, int NT, int EPI>
+void launch_gemm_splitk(const T* A, const T* B0, const T* B1, T* C, const T* R, int M, int N, int K, hipStream_t stream) {
+    const int tiles_m = (M + 16 * MT - 1) / (16 * MT), tiles_n = (N + 16 * NT - 1) / (16 * NT);
+    const int tiles = tiles_m * tiles_n, xcds = chip_info().xcds;
+    hipLaunchKernelGGL((gemm_splitk_kernel<T, MT, NT, EPI>), dim3((unsigned)((tiles + xcds - 1) / xcds * xcds)), dim3(kSplitWaves * 64),
+                       0, stream, A, B0, B1, C, R, M, N, K, tiles_m, tiles, xcds);
 }
 
 // k extent of one LDS stage of the DMA kernel: 128 bytes of a row for every element type
@@ -581,65 +562,83 @@ template <typename T> constexpr int kFragRows = sizeof(T) == 2 ? 16 : 32;
 template <typename T> constexpr int kBigSplit = sizeof(T) == 2 ? 4 : 1;
 template <typename T> constexpr int kSmallAhead = sizeof(T) == 2 ? 1 : 3;
 
-// Ragged shapes: the bounds-checked kernels (register-staged MFMA for 16-bit, FMA for fp32).
-template <typename T, int EPI>
-void launch_ragged(const T* A, const T* B0, const T* B1, T* C, const T* R, int M, int N, int K, hipStream_t stream) {
-    if constexpr (sizeof(T) == 4)
-        hipLaunchKernelGGL((sgemm_nt_kernel<EPI>), dim3((N + 63) / 64, (M + 63) / 64), dim3(256), 0, stream, A, B0, B1, C, R, M, N, K);
-    else
-        launch_gemm<T, 128, 128, EPI>(A, B0, B1, C, R, M, N, K, stream);
+// Tile choice.  A workgroup's time per k-tile is the larger of what its CU receives from the L2 ((BM + BN) rows of 128 bytes at
+// about 70 GB/s per CU) and what its matrix pipes take (BM * BN); 128 x 128 balances the two, so in units of one received row the
+// second is BM * BN / 66.  The launch lasts as many rounds as the busiest CU has tiles.  The rule picks the shape with the
+// smallest rounds * time: 256 x 256 (8 waves, two per SIMD) once the chip has several tiles per CU, smaller ones so that every CU
+// has a tile, whatever the extents.
+// fp32 rows of 128 bytes hold half as many values for matrix pipes an eighth as fast: BM * BN / 15.  The k-splitting kernel
+// costs more per received row, and more so the more CUs receive at once (measured from 64 to 224 workgroups), but its tiles are
+// small enough for a few rows of A.
+enum TileShape { kTile256, kTile128, kTile64x128, kTile64, kSplit32, kSplit16x32, kSplit16 };
+template <typename T, int EPI> TileShape choose_tile(int M, int N, int& tiles) {
+    constexpr int kRows[7] = {256, 128, 64, 64, 32, 16, 16}, kOuts[7] = {256, 128, 128, 64, 32, 32, 16};
+    const int cus = chip_info().cus;
+    TileShape best = kTile128;
+    double best_cost = 0.0;
+    for (int i = 0; i < 7; ++i) {
+        if (i == kTile64 && EPI == kEpiSwiGLU && sizeof(T) == 4) continue;      // a 32-column wave tile is one fp32 fragment: no gate/up pair
+        const bool split_k = i >= kSplit32;
+        const int out_cols = EPI == kEpiSwiGLU && !split_k ? kOuts[i] / 2 : kOuts[i];
+        const int cols = EPI == kEpiSwiGLU ? 2 * out_cols : out_cols;
+        const int64_t n = (int64_t)((M + kRows[i] - 1) / kRows[i]) * ((N + out_cols - 1) / out_cols);
+        const double occupied = n < cus ? (double)n / cus : 1.0;
+        const double received = (kRows[i] + cols) * (split_k ? 1.45 * (1.0 + occupied) : 1.0);
+        const double multiplied = kRows[i] * (double)cols / (sizeof(T) == 4 ? 15.0 : 66.0);
+        const double cost = (double)((n + cus - 1) / cus) * (received > multiplied ? received : multiplied);
+        if (i == 0 || cost < best_cost) {
+            best = (TileShape)i;
+            best_cost = cost;
+            tiles = (int)(n < (1 << 30) ? n : (1 << 30));
+        }
+    }
+    return best;
 }
 
-// Tile choice: 256-wide tiles (8 waves, two per SIMD) halve the L2 -> LDS traffic per MFMA but need one per CU to
-// occupy the chip; otherwise 128x128 tiles of 4 waves, which read half a k-tile of fragments ahead (a whole one in fp32): one
-// workgroup per CU with four stages in flight when every tile gets a CU of its own, two per CU with two stages else.
-template <typename T, int EPI>
-void launch_small_tiles(const T* A, const T* B0, const T* B1, T* C, const T* R, int M, int N, int K, int64_t tiles,
-                        hipStream_t stream) {
-    constexpr int KT = kStageK<T>;
-    if (tiles <= chip_info().cus) launch_gemm_dma<T, 128, 128, 2, 2, KT, 4, EPI, kSmallAhead<T>, kFragRows<T>>(A, B0, B1, C, R, M, N, K, stream);
-    else launch_gemm_dma<T, 128, 128, 2, 2, KT, 2, EPI, kSmallAhead<T>, kFragRows<T>>(A, B0, B1, C, R, M, N, K, stream);
+// 128 x 128 and smaller tiles: 4 waves that read half a k-tile of fragments ahead (a whole one in fp32), one workgroup per CU
+// with four stages in flight, or (128 x 128) two per CU with two stages when there are more tiles than CUs.
+template <typename T, int EPI, bool RAGGED>
+void launch_tiles(const T* A, const T* B0, const T* B1, T* C, const T* R, int M, int N, int K, hipStream_t stream) {
+    constexpr int KT = kStageK<T>, PF = kSmallAhead<T>, FR = kFragRows<T>;
+    int tiles = 0;
+    switch (choose_tile<T, EPI>(M, N, tiles)) {
+        case kTile256: launch_gemm_dma<T, 256, 256, 2, 4, KT, 2, EPI, 1, FR, kBigSplit<T>, RAGGED>(A, B0, B1, C, R, M, N, K, stream); break;
+        case kTile128:
+            if (tiles <= chip_info().cus) launch_gemm_dma<T, 128, 128, 2, 2, KT, 4, EPI, PF, FR, 1, RAGGED>(A, B0, B1, C, R, M, N, K, stream);
+            else launch_gemm_dma<T, 128, 128, 2, 2, KT, 2, EPI, PF, FR, 1, RAGGED>(A, B0, B1, C, R, M, N, K, stream);
+            break;
+        case kSplit32: launch_gemm_splitk<T, 2, 2, EPI>(A, B0, B1, C, R, M, N, K, stream); break;
+        case kSplit16x32: launch_gemm_splitk<T, 1, 2, EPI>(A, B0, B1, C, R, M, N, K, stream); break;
+        case kSplit16: launch_gemm_splitk<T, 1, 1, EPI>(A, B0, B1, C, R, M, N, K, stream); break;
+        case kTile64x128: launch_gemm_dma<T, 64, 128, 2, 2, KT, 4, EPI, PF, FR, 1, RAGGED>(A, B0, B1, C, R, M, N, K, stream); break;
+        default:
+            if constexpr (EPI != kEpiSwiGLU || sizeof(T) == 2)
+                launch_gemm_dma<T, 64, 64, 2, 2, KT, 4, EPI, PF, FR, 1, RAGGED>(A, B0, B1, C, R, M, N, K, stream);
+    }
 }
 
-// Few tokens: 64-row tiles (wave tiles of 32 x 64 or 32 x 32), so that a batch of a few hundred tokens still gives
-// every CU a tile.  N_OUT: output columns of a tile.
 template <typename T, int EPI>
-void launch_narrow_tiles(const T* A, const T* B0, const T* B1, T* C, const T* R, int M, int N, int K, hipStream_t stream) {
-    if (EPI == kEpiPlain && (int64_t)((M + 63) / 64) * (N / 128) < chip_info().cus && N % 64 == 0)
-        launch_gemm_dma<T, 64, 64, 2, 2, kStageK<T>, 4, kEpiPlain, kSmallAhead<T>, kFragRows<T>>(A, B0, B1, C, R, M, N, K, stream);
-    else
-        launch_gemm_dma<T, 64, 128, 2, 2, kStageK<T>, 4, EPI, kSmallAhead<T>, kFragRows<T>>(A, B0, B1, C, R, M, N, K, stream);
+void launch_product(const T* A, const T* B0, const T* B1, T* C, const T* R, int M, int N, int K, hipStream_t stream) {
+    // the DMA kernel moves 16-byte pieces of rows; fp32 callers need not align their tensors or rows
+    if (sizeof(T) == 4 && !(K % 4 == 0 && aligned16(A) && aligned16(B0) && aligned16(B1))) {
+        if constexpr (sizeof(T) == 4)
+            hipLaunchKernelGGL((sgemm_nt_kernel<EPI>), dim3((N + 63) / 64, (M + 63) / 64), dim3(256), 0, stream, A, B0, B1, C, R, M, N, K);
+        return;
+    }
+    if (K % kStageK<T> == 0 && N % (EPI == kEpiSwiGLU ? 128 : 256) == 0) launch_tiles<T, EPI, false>(A, B0, B1, C, R, M, N, K, stream);
+    else launch_tiles<T, EPI, true>(A, B0, B1, C, R, M, N, K, stream);
 }
 
 template <typename T>
 int gate_up_tiled(const void* x, const void* wg, const void* wu, int M, int H, int I, void* h, void* saved, hipStream_t stream) {
-    const T *A = (const T*)x, *G = (const T*)wg, *U = (const T*)wu, *S = (const T*)saved;
-    // the DMA kernel moves 16-byte pieces (fp32 callers need not align their tensors; those take the ragged kernel)
-    const bool k_ok = H % kStageK<T> == 0 && aligned16(x) && aligned16(wg) && aligned16(wu);
-    if (k_ok && I % 128 == 0 && (int64_t)((M + 255) / 256) * (I / 128) >= chip_info().cus)
-        launch_gemm_dma<T, 256, 256, 2, 4, kStageK<T>, 2, kEpiSwiGLU, 1, kFragRows<T>, kBigSplit<T>>(A, G, U, (T*)h, S, M, I, H, stream);
-    else if (k_ok && I % 64 == 0 && (int64_t)((M + 127) / 128) * (I / 64) >= chip_info().cus)
-        launch_small_tiles<T, kEpiSwiGLU>(A, G, U, (T*)h, S, M, I, H, (int64_t)((M + 127) / 128) * (I / 64), stream);
-    else if (k_ok && I % 64 == 0)
-        launch_narrow_tiles<T, kEpiSwiGLU>(A, G, U, (T*)h, S, M, I, H, stream);
-    else
-        launch_ragged<T, kEpiSwiGLU>(A, G, U, (T*)h, S, M, I, H, stream);
+    launch_product<T, kEpiSwiGLU>((const T*)x, (const T*)wg, (const T*)wu, (T*)h, (const T*)saved, M, I, H, stream);
     FMOE_CHECK_LAUNCH("fmoe_mlp(gate/up)");
     return FMOE_OK;
 }
 
 template <typename T>
 int down_tiled(const void* h, const void* wd, int M, int H, int I, const void* residual, void* out, hipStream_t stream) {
-    const T *A = (const T*)h, *W = (const T*)wd, *R = (const T*)residual;
-    const bool k_ok = I % kStageK<T> == 0 && aligned16(h) && aligned16(wd);
-    if (k_ok && H % 256 == 0 && (int64_t)((M + 255) / 256) * (H / 256) >= chip_info().cus)
-        launch_gemm_dma<T, 256, 256, 2, 4, kStageK<T>, 2, kEpiPlain, 1, kFragRows<T>, kBigSplit<T>>(A, W, nullptr, (T*)out, R, M, H, I, stream);
-    else if (k_ok && H % 128 == 0 && (int64_t)((M + 127) / 128) * (H / 128) >= chip_info().cus)
-        launch_small_tiles<T, kEpiPlain>(A, W, nullptr, (T*)out, R, M, H, I, (int64_t)((M + 127) / 128) * (H / 128), stream);
-    else if (k_ok && H % 128 == 0)
-        launch_narrow_tiles<T, kEpiPlain>(A, W, nullptr, (T*)out, R, M, H, I, stream);
-    else
-        launch_ragged<T, kEpiPlain>(A, W, nullptr, (T*)out, R, M, H, I, stream);
+    launch_product<T, kEpiPlain>((const T*)h, (const T*)wd, nullptr, (T*)out, (const T*)residual, M, H, I, stream);
     FMOE_CHECK_LAUNCH("fmoe_mlp(down)");
     return FMOE_OK;
 }

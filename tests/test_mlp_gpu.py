@@ -116,3 +116,35 @@ def test_mlp_linearity_full_size():
     assert torch.equal(flash_mlp_func(x, wg, wu * 0.5, wd), y * 0.5)
     assert flash_mlp_func(x, wg, wu * 0, wd).abs().max() == 0
     assert torch.equal(flash_mlp_func(x, wg, wu, wd), y)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("T,H,I", [
+    (1, 8, 8), (17, 40, 24), (16, 520, 1032),          # 16-row tiles with k split over the waves
+    (33, 264, 1000), (130, 1032, 136),                 # 32 x 32 tiles, remainders on every side
+    (615, 776, 2072), (999, 1000, 2664),               # 64-row tiles
+    (3001, 1160, 3080), (5000, 1336, 3560),            # 128 x 128 and 256 x 256 tiles
+])
+def test_mlp_remainders_of_every_tile_shape(dtype, T, H, I):
+    # both products with their outputs between guard rows: nothing outside [T, N] may be written, and the gate and up
+    # products kept for a backward pass match as well
+    from flash_moe import _C
+
+    x, wg, wu, wd = cuda(*make(T, H, I, dtype, seed=T + H + I))
+    res = torch.randn(T, H, device="cuda").to(dtype)
+    L, code, stream = _C.lib(), _C.dtype_code(dtype), _C.current_stream(x.device)
+
+    def guarded(rows, cols):
+        buf = torch.full((rows + 16, cols), 7.0, device="cuda", dtype=dtype)
+        return buf, buf[8:8 + rows]
+
+    (abuf, act), (sbuf, saved), (obuf, out) = guarded(T, I), guarded(2 * T, I), guarded(T, H)
+    _C.check(L.fmoe_mlp_gate_up_save(*map(_C.ptr, (x, wg, wu)), T, H, I, code, _C.ptr(act), _C.ptr(saved), stream), "gate/up")
+    _C.check(L.fmoe_mlp_down(_C.ptr(act), _C.ptr(wd), T, H, I, code, _C.ptr(res), _C.ptr(out), stream), "down")
+    tol = {torch.float32: 2e-6, torch.bfloat16: 6e-3, torch.float16: 8e-4}[dtype]
+    a, b = x.double() @ wg.double().t(), x.double() @ wu.double().t()
+    assert rel_fro(saved[:T], a) < tol and rel_fro(saved[T:], b) < tol
+    assert rel_fro(act, torch.nn.functional.silu(a) * b) < tol
+    assert rel_fro(out, act.double() @ wd.double().t() + res.double()) < tol
+    for buf in (abuf, sbuf, obuf):
+        assert (buf[:8] == 7).all() and (buf[-8:] == 7).all()
