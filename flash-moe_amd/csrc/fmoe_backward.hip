@@ -93,8 +93,8 @@ int launch_router_backward(const void* dscores, const int64_t* indices, void* dl
 template <typename T>
 __global__ __launch_bounds__(kBwdWaves* kWave) void route_backward_kernel(
     const T* __restrict__ dgates, const int64_t* __restrict__ indices, const float* __restrict__ logits,
-    const T* __restrict__ dlogits_extra, float* __restrict__ dlogits, int64_t num_tokens, int nk, int top_k,
-    int norm_topk_prob, int waves_per_block, int chunk) {
+    const T* __restrict__ dlogits_extra, int64_t extra_token, int64_t extra_half, float* __restrict__ dlogits,
+    int64_t num_tokens, int nk, int top_k, int norm_topk_prob, int waves_per_block, int chunk) {
     extern __shared__ float acc_all[];   // [waves_per_block][2 * chunk], one private row pair per wave
     const int lane = lane_id();
     const int wave = (int)(threadIdx.x >> 6);
@@ -177,7 +177,7 @@ __global__ __launch_bounds__(kBwdWaves* kWave) void route_backward_kernel(
             for (int p = lane; p < cn; p += kWave) {
                 const int64_t at = token * 2 * nk + h * nk + c0 + p;
                 float d = acc[h * chunk + p] - expf((row[h * nk + c0 + p] - shift[h]) - lse[h]) * sum;
-                if (dlogits_extra != nullptr) d += Elem<T>::to_f32(dlogits_extra[at]);
+                if (dlogits_extra != nullptr) d += Elem<T>::to_f32(dlogits_extra[token * extra_token + h * extra_half + c0 + p]);
                 dlogits[at] = d;
             }
         }
@@ -187,14 +187,15 @@ __global__ __launch_bounds__(kBwdWaves* kWave) void route_backward_kernel(
 
 template <typename T>
 int launch_route_backward(const void* dgates, const int64_t* indices, const float* logits, const void* dlogits_extra,
-                          float* dlogits, int64_t T_, int nk, int K, int norm, hipStream_t stream) {
+                          int64_t extra_token, int64_t extra_half, float* dlogits, int64_t T_, int nk, int K, int norm, hipStream_t stream) {
     const int chunk = backward_key_chunk(nk);
     const size_t per_wave = (size_t)2 * chunk * sizeof(float);
     int waves = (int)((48 * 1024) / per_wave);
     waves = waves < 1 ? 1 : (waves > kBwdWaves ? kBwdWaves : waves);
     const unsigned grid = (unsigned)((T_ + waves - 1) / waves);
     hipLaunchKernelGGL((route_backward_kernel<T>), dim3(grid), dim3(kBwdWaves * kWave), waves * per_wave, stream,
-                       (const T*)dgates, indices, logits, (const T*)dlogits_extra, dlogits, T_, nk, K, norm, waves, chunk);
+                       (const T*)dgates, indices, logits, (const T*)dlogits_extra, extra_token, extra_half, dlogits, T_, nk, K, norm, waves,
+                       chunk);
     FMOE_CHECK_LAUNCH("fmoe_route_backward");
     return FMOE_OK;
 }
@@ -579,8 +580,15 @@ extern "C" int fmoe_router_topk_backward(const void* dscores, const int64_t* ind
 extern "C" int fmoe_route_backward(const void* dgates, const int64_t* indices, const float* logits_fp32, const void* dlogits_extra,
                                    int64_t num_tokens, int num_keys, int top_k, int dtype, int norm_topk_prob,
                                    float* dlogits_fp32, void* stream) {
+    fmoe::clear_error();
+    return fmoe::route_backward_impl(dgates, indices, logits_fp32, dlogits_extra, 2 * (int64_t)num_keys, num_keys, num_tokens, num_keys,
+                                     top_k, dtype, norm_topk_prob, dlogits_fp32, (hipStream_t)stream);
+}
+
+int fmoe::route_backward_impl(const void* dgates, const int64_t* indices, const float* logits_fp32, const void* dlogits_extra,
+                              int64_t extra_token, int64_t extra_half, int64_t num_tokens, int num_keys, int top_k, int dtype,
+                              int norm_topk_prob, float* dlogits_fp32, hipStream_t s) {
     using namespace fmoe;
-    clear_error();
     FMOE_REQUIRE(dtype_ok(dtype), FMOE_ERR_BAD_DTYPE, "fmoe_route_backward: unknown dtype %d", dtype);
     FMOE_REQUIRE(num_tokens >= 0 && num_keys > 0 && top_k >= 0, FMOE_ERR_BAD_SHAPE,
                  "fmoe_route_backward: bad shape T=%lld nk=%d K=%d", (long long)num_tokens, num_keys, top_k);
@@ -588,11 +596,10 @@ extern "C" int fmoe_route_backward(const void* dgates, const int64_t* indices, c
     if (num_tokens == 0) return FMOE_OK;
     FMOE_REQUIRE(logits_fp32 && dlogits_fp32 && (top_k == 0 || (dgates && indices)), FMOE_ERR_NULL_POINTER,
                  "fmoe_route_backward: null tensor pointer");
-    hipStream_t s = (hipStream_t)stream;
     switch (dtype) {
-        case FMOE_F32: return launch_route_backward<float>(dgates, indices, logits_fp32, dlogits_extra, dlogits_fp32, num_tokens, num_keys, top_k, norm_topk_prob, s);
-        case FMOE_BF16: return launch_route_backward<bf16_t>(dgates, indices, logits_fp32, dlogits_extra, dlogits_fp32, num_tokens, num_keys, top_k, norm_topk_prob, s);
-        default: return launch_route_backward<f16_t>(dgates, indices, logits_fp32, dlogits_extra, dlogits_fp32, num_tokens, num_keys, top_k, norm_topk_prob, s);
+        case FMOE_F32: return launch_route_backward<float>(dgates, indices, logits_fp32, dlogits_extra, extra_token, extra_half, dlogits_fp32, num_tokens, num_keys, top_k, norm_topk_prob, s);
+        case FMOE_BF16: return launch_route_backward<bf16_t>(dgates, indices, logits_fp32, dlogits_extra, extra_token, extra_half, dlogits_fp32, num_tokens, num_keys, top_k, norm_topk_prob, s);
+        default: return launch_route_backward<f16_t>(dgates, indices, logits_fp32, dlogits_extra, extra_token, extra_half, dlogits_fp32, num_tokens, num_keys, top_k, norm_topk_prob, s);
     }
 }
 

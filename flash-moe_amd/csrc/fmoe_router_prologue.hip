@@ -878,7 +878,8 @@ __global__ __launch_bounds__(256) void bn_bwd_finalize_kernel(const float* __res
 template <typename T>
 __global__ __launch_bounds__(256) void bn_bwd_apply_kernel(const T* __restrict__ x, const T* __restrict__ dq,
                                                            const float* __restrict__ mean_rstd, const float* __restrict__ sums,
-                                                           T* __restrict__ dx, int hidden, int col_blocks, int training) {
+                                                           const T* addend0, const T* addend1, T* dx, int hidden,
+                                                           int col_blocks, int training) {
     constexpr int V = Elem<T>::kVec;
     const uint32_t row = blockIdx.x / (uint32_t)col_blocks;
     const int col = ((int)(blockIdx.x % (uint32_t)col_blocks) * 256 + (int)threadIdx.x) * V;
@@ -905,6 +906,14 @@ __global__ __launch_bounds__(256) void bn_bwd_apply_kernel(const T* __restrict__
     // evaluation mode: m1 = m2 = 0 and the formula reduces to rstd * dq
 #pragma unroll
     for (int v = 0; v < V; ++v) ov[v] = rstd[v] * (gv[v] - m1[v] - (xv[v] - mean[v]) * rstd[v] * m2[v]);
+    // the block's other two token gradients; a thread reads its packet of them before it writes dx, which may be one of them
+    for (const T* addend : {addend0, addend1}) {
+        if (addend == nullptr) continue;
+        float av[V];
+        unpack16<T>(*reinterpret_cast<const u32x4_t*>(addend + at), av);
+#pragma unroll
+        for (int v = 0; v < V; ++v) ov[v] += av[v];
+    }
     *reinterpret_cast<u32x4_t*>(dx + at) = pack16<T>(ov);
 }
 
@@ -929,7 +938,8 @@ PrologueBwdPlan plan_prologue_backward(int64_t T_, int H, int nk, int dtype) {
 
 template <typename T>
 int launch_prologue_backward(const float* dlogits, const void* x, const void* gate_w, const float* mean_rstd, int training,
-                             int64_t T_, int H, int nk, int dtype, void* dx, void* dgate_w, void* workspace, hipStream_t s) {
+                             int64_t T_, int H, int nk, int dtype, void* dx, void* dgate_w, const void* addend0, const void* addend1,
+                             void* workspace, hipStream_t s) {
     constexpr int V = Elem<T>::kVec;
     const PrologueBwdPlan p = plan_prologue_backward(T_, H, nk, dtype);
     const ProloguePlan rows = plan_prologue(T_, H, nk);
@@ -969,7 +979,7 @@ int launch_prologue_backward(const float* dlogits, const void* x, const void* ga
     }
     const int apply_blocks = (H / V + 255) / 256;
     hipLaunchKernelGGL((bn_bwd_apply_kernel<T>), dim3((unsigned)(T_ * apply_blocks)), dim3(256), 0, s, (const T*)x,
-                       (const T*)dq, mean_rstd, (const float*)sums, (T*)dx, H, apply_blocks, training);
+                       (const T*)dq, mean_rstd, (const float*)sums, (const T*)addend0, (const T*)addend1, (T*)dx, H, apply_blocks, training);
     FMOE_CHECK_LAUNCH("fmoe_router_prologue_backward(apply)");
     return FMOE_OK;
 }
@@ -1032,7 +1042,7 @@ int fmoe::router_forward_impl(const void* x, const void* gate_w, void* running_m
                               int64_t num_tokens, int hidden, int num_keys, int top_k, int dtype, int norm_topk_prob,
                               void* router_logits, float* logits_fp32, float* scores, int64_t* indices, void* gates,
                               uint32_t* row_offsets, uint32_t row_bytes, void* workspace, size_t workspace_bytes,
-                              hipStream_t s, int split_query, int fixed_scratch) {
+                              hipStream_t s, int split_query, int fixed_scratch, float* mean_rstd_out) {
     using namespace fmoe;
     FMOE_REQUIRE(!split_query || (num_keys % 64 == 0 && hidden % 2 == 0), FMOE_ERR_UNSUPPORTED,
                  "fmoe_router_forward_split: num_keys=%d must be a multiple of 64 and hidden=%d even", num_keys, hidden);
@@ -1068,7 +1078,7 @@ int fmoe::router_forward_impl(const void* x, const void* gate_w, void* running_m
                  "fmoe_router_forward: workspace of %zu bytes needed, %zu given", need, workspace_bytes);
     char* ws = (char*)workspace;
     float* partial = (float*)(ws + p.off_partial);
-    float* mean_rstd = (float*)(ws + p.off_mean_rstd);
+    float* mean_rstd = mean_rstd_out ? mean_rstd_out : (float*)(ws + p.off_mean_rstd);
     float* logits32 = logits_fp32;
 
     const int M = (int)num_tokens, N = 2 * num_keys;
@@ -1178,8 +1188,16 @@ extern "C" size_t fmoe_router_prologue_backward_workspace_bytes(int64_t num_toke
 extern "C" int fmoe_router_prologue_backward(const float* dlogits_fp32, const void* x, const void* gate_w, const float* mean_rstd,
                                              int training, int64_t num_tokens, int hidden, int num_keys, int dtype, void* dx,
                                              void* dgate_w, void* workspace, size_t workspace_bytes, void* stream) {
+    fmoe::clear_error();
+    return fmoe::router_prologue_backward_impl(dlogits_fp32, x, gate_w, mean_rstd, training, num_tokens, hidden, num_keys, dtype, dx,
+                                               dgate_w, nullptr, nullptr, workspace, workspace_bytes, (hipStream_t)stream);
+}
+
+int fmoe::router_prologue_backward_impl(const float* dlogits_fp32, const void* x, const void* gate_w, const float* mean_rstd,
+                                        int training, int64_t num_tokens, int hidden, int num_keys, int dtype, void* dx,
+                                        void* dgate_w, const void* addend0, const void* addend1, void* workspace,
+                                        size_t workspace_bytes, hipStream_t s) {
     using namespace fmoe;
-    clear_error();
     FMOE_REQUIRE(dtype_ok(dtype), FMOE_ERR_BAD_DTYPE, "fmoe_router_prologue_backward: unknown dtype %d", dtype);
     FMOE_REQUIRE(num_tokens > 0 && hidden > 0 && num_keys > 0 && num_tokens < (1ll << 24), FMOE_ERR_BAD_SHAPE,
                  "fmoe_router_prologue_backward: bad shape T=%lld H=%d nk=%d", (long long)num_tokens, hidden, num_keys);
@@ -1193,10 +1211,9 @@ extern "C" int fmoe_router_prologue_backward(const float* dlogits_fp32, const vo
     const size_t need = plan_prologue_backward(num_tokens, hidden, num_keys, dtype).bytes;
     FMOE_REQUIRE(workspace && workspace_bytes >= need && aligned16(workspace), FMOE_ERR_WORKSPACE,
                  "fmoe_router_prologue_backward: workspace of %zu bytes needed, %zu given", need, workspace_bytes);
-    hipStream_t s = (hipStream_t)stream;
     switch (dtype) {
-        case FMOE_F32: return launch_prologue_backward<float>(dlogits_fp32, x, gate_w, mean_rstd, training, num_tokens, hidden, num_keys, dtype, dx, dgate_w, workspace, s);
-        case FMOE_BF16: return launch_prologue_backward<bf16_t>(dlogits_fp32, x, gate_w, mean_rstd, training, num_tokens, hidden, num_keys, dtype, dx, dgate_w, workspace, s);
-        default: return launch_prologue_backward<f16_t>(dlogits_fp32, x, gate_w, mean_rstd, training, num_tokens, hidden, num_keys, dtype, dx, dgate_w, workspace, s);
+        case FMOE_F32: return launch_prologue_backward<float>(dlogits_fp32, x, gate_w, mean_rstd, training, num_tokens, hidden, num_keys, dtype, dx, dgate_w, addend0, addend1, workspace, s);
+        case FMOE_BF16: return launch_prologue_backward<bf16_t>(dlogits_fp32, x, gate_w, mean_rstd, training, num_tokens, hidden, num_keys, dtype, dx, dgate_w, addend0, addend1, workspace, s);
+        default: return launch_prologue_backward<f16_t>(dlogits_fp32, x, gate_w, mean_rstd, training, num_tokens, hidden, num_keys, dtype, dx, dgate_w, addend0, addend1, workspace, s);
     }
 }

@@ -1,18 +1,23 @@
-"""ctypes binding of ``libflashmoe_hip.so`` (the C ABI declared in ``include/flashmoe_hip.h``).
+"""Bindings of ``libflashmoe_hip.so`` (the C ABI declared in ``include/flashmoe_hip.h``).
 
-The library is loaded from ``flash_moe/lib/`` next to this file.  It is never built at import or call
-time, and there is no fallback: if it is missing, the first op call raises.
+``native()`` is the torch extension ``_native.so`` (``csrc/fmoe_torch.cpp``) the ops call: argument checks, allocation and the
+autograd nodes in C++ on top of the C ABI.  ``lib()`` is the C ABI itself through ctypes, for callers that bring their own
+buffers.  Both are loaded from ``flash_moe/lib/`` next to this file.  They are never built at import or call time, and there is no
+fallback: if one is missing, the first op call raises.
 """
 from __future__ import annotations
 
 import ctypes
+import importlib.util
 import os
 from typing import Optional
 
 import torch
 
 _LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "lib", "libflashmoe_hip.so")
+_NATIVE_PATH = os.path.join(os.path.dirname(_LIB_PATH), "_native.so")
 _lib: Optional[ctypes.CDLL] = None
+_native = None
 
 ABI_VERSION = 1
 
@@ -48,6 +53,11 @@ SIGNATURES = {
     "fmoe_block_workspace_bytes": (_sz, [_i64, _int, _int, _int, _i64, _int, _int]),
     "fmoe_block_forward": (_int, [_vp] * 10 + [_int, _int, ctypes.c_float, ctypes.c_float, _i64, _int, _int, _i64, _int, _int,
                                   _int, _int, _vp, _vp, _vp, _vp, _vp, _sz, _vp]),
+    "fmoe_block_saved_bytes": (_sz, [_i64, _int, _int, _int, _i64, _int, _int]),
+    "fmoe_block_forward_save": (_int, [_vp] * 10 + [_int, _int, ctypes.c_float, ctypes.c_float, _i64, _int, _int, _i64, _int, _int,
+                                       _int, _int, _vp, _vp, _vp, _sz, _vp, _sz, _vp]),
+    "fmoe_block_backward_workspace_bytes": (_sz, [_i64, _int, _int, _int, _i64, _int, _int]),
+    "fmoe_block_backward": (_int, [_vp] * 10 + [_int, _i64, _int, _int, _i64, _int, _int, _int, _int] + [_vp] * 8 + [_sz, _vp]),
     "fmoe_mlp_gate_up": (_int, [_vp, _vp, _vp, _i64, _int, _int, _int, _vp, _vp]),
     "fmoe_mlp_gate_up_save": (_int, [_vp, _vp, _vp, _i64, _int, _int, _int, _vp, _vp, _vp]),
     "fmoe_mlp_down": (_int, [_vp, _vp, _i64, _int, _int, _int, _vp, _vp, _vp]),
@@ -91,26 +101,25 @@ def lib() -> ctypes.CDLL:
     return _lib
 
 
+def native():
+    """Load (once) and return the torch extension; raise if it has not been built."""
+    global _native
+    if _native is None:
+        lib()
+        if not os.path.exists(_NATIVE_PATH):
+            raise RuntimeError(f"{_NATIVE_PATH} not found: build it with `make -C flash-moe_amd/csrc`; there is no fallback path")
+        spec = importlib.util.spec_from_file_location("_native", _NATIVE_PATH)
+        module = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(module)
+        _native = module
+    return _native
+
+
 def dtype_code(dtype: torch.dtype) -> int:
     try:
         return _DTYPE_CODE[dtype]
     except KeyError:
         raise TypeError(f"unsupported dtype {dtype}; expected float32, bfloat16 or float16") from None
-
-
-def require_gpu(*tensors: torch.Tensor) -> torch.device:
-    """All tensors must live on one HIP device; returns it."""
-    dev = None
-    for t in tensors:
-        if t is None:
-            continue
-        if not t.is_cuda:
-            raise RuntimeError("flash_moe HIP ops need tensors on a ROCm GPU (got a CPU tensor); there is no CPU path")
-        if dev is None:
-            dev = t.device
-        elif t.device != dev:
-            raise RuntimeError(f"tensors on different devices: {dev} and {t.device}")
-    return dev
 
 
 def ptr(t: Optional[torch.Tensor]) -> Optional[int]:

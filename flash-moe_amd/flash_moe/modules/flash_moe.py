@@ -11,8 +11,8 @@ pair (:55-105).
   shared SwiGLU MLP + add                                           ``fmoe_mlp_forward`` (the add is the second
                                                                     GEMM's epilogue)
 ``forward_staged`` runs the same three stages as three calls.  When gradients are being recorded ``forward`` takes
-``forward_autograd`` instead: one autograd node whose forward is those three calls (keeping what the backward needs)
-and whose backward is the library's backward calls.  ``forward_autograd_ops`` is the reference's own composition
+``forward_autograd`` instead: one autograd node whose forward is ``fmoe_block_forward_save`` (which keeps what the backward
+needs) and whose backward is ``fmoe_block_backward``.  ``forward_autograd_ops`` is the reference's own composition
 (batch norm + router gate, log-softmax, then the router, expert and MLP ops, flash_moe/modules/flash_moe.py:62-101) on the
 differentiable per-op functions; both give the same gradients.
 
@@ -31,7 +31,7 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
-from flash_moe.ops.hip.flash_block import block_forward, block_forward_autograd
+from flash_moe.ops.hip.flash_block import block
 from flash_moe.ops.hip.flash_expert import expert_forward, flash_expert_func
 from flash_moe.ops.hip.flash_mlp import flash_mlp_func, mlp_forward
 from flash_moe.ops.hip.flash_router import flash_router_func, router_forward, router_prologue
@@ -90,30 +90,28 @@ class FlashMoE(nn.Module):
         return (router_logits,) + tuple(out[1:])
 
     def forward(self, hidden_states: torch.Tensor, **kwargs):
-        if torch.is_grad_enabled() and (hidden_states.requires_grad or any(p.requires_grad for p in self.parameters())):
-            return self.forward_autograd(hidden_states)
-        bsz, seq_len, _ = hidden_states.shape
-        tokens = hidden_states.reshape(bsz * seq_len, self.hidden_size)
-        out, logits = block_forward(
-            tokens, self.gate_proj.weight, self.up_proj.weight, self.down_proj.weight, self.router_gate.weight,
-            self.router_norm, self.down_embed.weight, self.up_embed.weight, self.num_keys, self.top_k, self.norm_topk_prob,
-        )
-        router_logits = logits.view(tokens.shape[0], 2, self.num_keys).transpose(0, 1)
-        return out.view(bsz, seq_len, self.hidden_size), router_logits
+        return self._block(hidden_states, torch.is_grad_enabled())
 
     def forward_autograd(self, hidden_states: torch.Tensor):
         """Differentiable forward: one autograd node around the library's forward and backward calls."""
-        bsz, seq_len, _ = hidden_states.shape
-        tokens = hidden_states.reshape(bsz * seq_len, self.hidden_size)
-        num_tokens = tokens.shape[0]
-        if num_tokens == 0 or self.top_k == 0:
-            return self.forward_autograd_ops(hidden_states)
-        out, logits = block_forward_autograd(
-            tokens, self.gate_proj.weight, self.up_proj.weight, self.down_proj.weight, self.router_gate.weight,
-            self.router_norm, self.down_embed.weight, self.up_embed.weight, self.num_keys, self.top_k, self.norm_topk_prob,
-        )
-        router_logits = logits.view(num_tokens, 2, self.num_keys).transpose(0, 1)
-        return out.view(bsz, seq_len, self.hidden_size), router_logits
+        return self._block(hidden_states, True)
+
+    def _block(self, hidden_states: torch.Tensor, differentiable: bool):
+        bsz, seq_len, _ = hidden_states.shape                # the reference's contract: [batch, sequence, hidden]
+        if differentiable and (bsz * seq_len == 0 or self.top_k == 0):
+            return self.forward_autograd_ops(hidden_states)  # nothing for the fused backward to work on
+        # straight from the submodules' tables: a call reads seven of them, and attribute lookup through nn.Module costs
+        # more than the launches of a small forward
+        modules = self._modules
+
+        def weight(name):
+            w = modules[name]._parameters.get("weight")
+            return modules[name].weight if w is None else w
+
+        out, logits = block(hidden_states, weight("gate_proj"), weight("up_proj"), weight("down_proj"), weight("router_gate"),
+                            modules["router_norm"], weight("down_embed"), weight("up_embed"), self.num_keys, self.top_k,
+                            bool(self.norm_topk_prob), differentiable)
+        return out, logits
 
     def forward_autograd_ops(self, hidden_states: torch.Tensor):
         """Differentiable forward op by op, as the reference composes it (flash_moe/modules/flash_moe.py:62-101): the

@@ -257,6 +257,35 @@ int fmoe_block_forward(const void* x, const void* gate_proj_w, const void* up_pr
                        int top_k, int dtype, int norm_topk_prob, void* out, void* router_logits, int64_t* indices_out,
                        void* gates_out, void* workspace, size_t workspace_bytes, void* stream);
 
+/* The block with gradients: fmoe_block_forward that also fills `saved` (fmoe_block_saved_bytes() bytes, 256-byte aligned: expert
+ * ids, gates, fp32 gate logits, batch-norm statistics, gate and up products) and the backward from it.  The reference reaches the
+ * same gradients through autograd of its eager ops around its three Triton functions (flash_moe/modules/flash_moe.py:55-105).
+ * fmoe_block_forward_save: arguments and workspace as fmoe_block_forward; top_k >= 1.
+ * fmoe_block_backward: dout [T,H]; dlogits [2,T,nk] (gradient of the router logits as the module returns them) or NULL; training and
+ *   norm_topk_prob as in the forward; out: dx [T,H], dgate_proj_w, dup_proj_w [I,H] (faster when they follow each other, as in
+ *   fmoe_mlp_backward), ddown_proj_w [H,I], drouter_gate_w [2*nk,H], ddown_embed, dup_embed [E,H].  The three token gradients are
+ *   added in fp32 and rounded once.  Limits: those of fmoe_mlp_backward, fmoe_expert_backward, fmoe_route_backward and
+ *   fmoe_router_prologue_backward. */
+size_t fmoe_block_saved_bytes(int64_t num_tokens, int hidden, int intermediate, int num_keys, int64_t num_experts, int top_k,
+                              int dtype);
+
+int fmoe_block_forward_save(const void* x, const void* gate_proj_w, const void* up_proj_w, const void* down_proj_w,
+                            const void* router_gate_w, const void* down_embed, const void* up_embed, void* running_mean,
+                            void* running_var, int64_t* num_batches_tracked, int stats_dtype, int training, float momentum,
+                            float eps, int64_t num_tokens, int hidden, int intermediate, int64_t num_experts, int num_keys,
+                            int top_k, int dtype, int norm_topk_prob, void* out, void* router_logits, void* saved,
+                            size_t saved_bytes, void* workspace, size_t workspace_bytes, void* stream);
+
+size_t fmoe_block_backward_workspace_bytes(int64_t num_tokens, int hidden, int intermediate, int num_keys, int64_t num_experts,
+                                           int top_k, int dtype);
+
+int fmoe_block_backward(const void* dout, const void* dlogits, const void* x, const void* gate_proj_w, const void* up_proj_w,
+                        const void* down_proj_w, const void* router_gate_w, const void* down_embed, const void* up_embed,
+                        const void* saved, int training, int64_t num_tokens, int hidden, int intermediate, int64_t num_experts,
+                        int num_keys, int top_k, int dtype, int norm_topk_prob, void* dx, void* dgate_proj_w, void* dup_proj_w,
+                        void* ddown_proj_w, void* drouter_gate_w, void* ddown_embed, void* dup_embed, void* workspace,
+                        size_t workspace_bytes, void* stream);
+
 /* ------------------------------------------------------------------------------------------------
  * The two other gather ops of the reference that share the routed-expert kernels (forward only there too).
  *
