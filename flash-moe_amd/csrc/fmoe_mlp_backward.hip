@@ -3,7 +3,8 @@
 // The forward keeps only silu(a) * b unless it was asked to keep the gate and up products a, b as well
 // (fmoe_mlp_gate_up_save); without them they are recomputed here (two launches of the forward's own NT GEMM).  The SwiGLU gradient is the fused
 // elementwise kernel of fmoe_backward.hip (it also rebuilds h = silu(a) * b for dWd).  The remaining products are
-// plain GEMMs in layouts the forward never needs (A B and A^T B); they go to rocBLAS, which is loaded on first use so
+// plain GEMMs in layouts the forward never needs (A B and A^T B): gemm_backward (fmoe_gemm_tr.hip) runs the small ones; the large
+// ones go to rocBLAS, which is loaded on first use so
 // that the forward path carries no dependency on it:
 //     dh  = dy Wd              [T,H][H,I]
 //     dWd = dy^T h             [T,H]^T [T,I]
@@ -69,10 +70,10 @@ int rocblas_for_device(rocblas_handle* out) {
 constexpr int kNN = kBlasNN, kTN = kBlasTN;
 
 struct MlpBwdPlan {
-    size_t off_a, off_b, off_dh, off_h, off_dab, bytes;
+    size_t off_a, off_b, off_dh, off_h, off_dab, off_part, part_bytes, bytes;
 };
 
-MlpBwdPlan plan_mlp_backward(int64_t T_, int I, int dtype) {
+MlpBwdPlan plan_mlp_backward(int64_t T_, int H, int I, int dtype) {
     MlpBwdPlan p;
     const size_t ti = (size_t)T_ * I * dtype_size(dtype);
     size_t o = 0;
@@ -82,6 +83,13 @@ MlpBwdPlan plan_mlp_backward(int64_t T_, int I, int dtype) {
     p.off_dh = take(ti);
     p.off_h = take(ti);
     p.off_dab = take(2 * ti);
+    p.part_bytes = 0;
+    const int t = (int)T_;
+    for (size_t n : {gemm_backward_workspace_bytes(kNN, t, I, H, 1, dtype), gemm_backward_workspace_bytes(kTN, H, I, t, 1, dtype),
+                     gemm_backward_workspace_bytes(kNN, t, H, I, 2, dtype), gemm_backward_workspace_bytes(kTN, 2 * I, H, t, 1, dtype),
+                     gemm_backward_workspace_bytes(kTN, I, H, t, 1, dtype)})
+        if (n > p.part_bytes) p.part_bytes = n;
+    p.off_part = take(p.part_bytes);
     p.bytes = o;
     return p;
 }
@@ -109,7 +117,7 @@ int blas_gemm(int layout, int M, int N, int K, const void* A, int lda, const voi
 
 extern "C" size_t fmoe_mlp_backward_workspace_bytes(int64_t num_tokens, int hidden, int intermediate, int dtype) {
     if (num_tokens <= 0 || hidden <= 0 || intermediate <= 0 || !fmoe::dtype_ok(dtype)) return 0;
-    return fmoe::plan_mlp_backward(num_tokens, intermediate, dtype).bytes;
+    return fmoe::plan_mlp_backward(num_tokens, hidden, intermediate, dtype).bytes;
 }
 
 extern "C" int fmoe_mlp_backward(const void* dy, const void* x, const void* gate_w, const void* up_w, const void* down_w,
@@ -126,13 +134,14 @@ extern "C" int fmoe_mlp_backward(const void* dy, const void* x, const void* gate
                  "fmoe_mlp_backward: hidden=%d and intermediate=%d must be multiples of %d (16-byte rows)", hidden, intermediate, vec);
     FMOE_REQUIRE(dy && x && gate_w && up_w && down_w && dx && dgate_w && dup_w && ddown_w, FMOE_ERR_NULL_POINTER,
                  "fmoe_mlp_backward: null tensor pointer");
-    const MlpBwdPlan p = plan_mlp_backward(num_tokens, intermediate, dtype);
+    const MlpBwdPlan p = plan_mlp_backward(num_tokens, hidden, intermediate, dtype);
     FMOE_REQUIRE(workspace && workspace_bytes >= p.bytes && aligned16(workspace), FMOE_ERR_WORKSPACE,
                  "fmoe_mlp_backward: workspace of %zu bytes needed, %zu given", p.bytes, workspace_bytes);
     hipStream_t s = (hipStream_t)stream;
     char* ws = (char*)workspace;
     void *a = ws + p.off_a, *b = ws + p.off_b, *dh = ws + p.off_dh, *h = ws + p.off_h;
     char* dab = ws + p.off_dab;
+    void* part = ws + p.off_part;
     const int T_ = (int)num_tokens, H = hidden, I = intermediate;
     const size_t elt = dtype_size(dtype);
 
@@ -149,24 +158,22 @@ extern "C" int fmoe_mlp_backward(const void* dy, const void* x, const void* gate
         if (rc) return rc;
     }
 
-    rc = blas_gemm(kNN, T_, I, H, dy, H, down_w, I, dh, I, 0.0f, dtype, s);                        // dh = dy Wd
+    rc = gemm_backward(kNN, T_, I, H, dy, H, down_w, nullptr, I, dh, I, dtype, part, p.part_bytes, s);                        // dh = dy Wd
     if (rc) return rc;
-    // da and db side by side: one [T, 2I] matrix [da | db], so that products over both are single library calls
+    // da and db side by side: one [T, 2I] matrix [da | db], so that products over both are single calls
     char* db = dab + (size_t)I * elt;
     const int I2 = 2 * I;
     rc = launch_swiglu_backward(dh, a, b, dab, db, h, num_tokens, I, I2, I2, dtype, s);
     if (rc) return rc;
-    rc = blas_gemm(kTN, H, I, T_, dy, H, h, I, ddown_w, I, 0.0f, dtype, s);                         // dWd = dy^T h
+    rc = gemm_backward(kTN, H, I, T_, dy, H, h, nullptr, I, ddown_w, I, dtype, part, p.part_bytes, s);                         // dWd = dy^T h
+    if (rc) return rc;
+    rc = gemm_backward(kNN, T_, H, I, dab, I2, gate_w, up_w, H, dx, H, dtype, part, p.part_bytes, s);                          // dx = da Wg + db Wu
     if (rc) return rc;
     const size_t w_bytes = (size_t)I * H * elt;
-    rc = blas_gemm(kNN, T_, H, I, dab, I2, gate_w, H, dx, H, 0.0f, dtype, s);                       // dx = da Wg
-    if (rc) return rc;
-    rc = blas_gemm(kNN, T_, H, I, db, I2, up_w, H, dx, H, 1.0f, dtype, s);                          //    + db Wu
-    if (rc) return rc;
     // the two weight gradients are one [2I, H] product when the caller's buffers follow each other: one 74 us kernel at
     // T = I = 4096, H = 1024 instead of two of 49 us
-    if ((char*)dup_w == (char*)dgate_w + w_bytes) return blas_gemm(kTN, I2, H, T_, dab, I2, x, H, dgate_w, H, 0.0f, dtype, s);
-    rc = blas_gemm(kTN, I, H, T_, dab, I2, x, H, dgate_w, H, 0.0f, dtype, s);                       // dWg = da^T x
+    if ((char*)dup_w == (char*)dgate_w + w_bytes) return gemm_backward(kTN, I2, H, T_, dab, I2, x, nullptr, H, dgate_w, H, dtype, part, p.part_bytes, s);
+    rc = gemm_backward(kTN, I, H, T_, dab, I2, x, nullptr, H, dgate_w, H, dtype, part, p.part_bytes, s);                       // dWg = da^T x
     if (rc) return rc;
-    return blas_gemm(kTN, I, H, T_, db, I2, x, H, dup_w, H, 0.0f, dtype, s);                        // dWu = db^T x
+    return gemm_backward(kTN, I, H, T_, db, I2, x, nullptr, H, dup_w, H, dtype, part, p.part_bytes, s);                        // dWu = db^T x
 }

@@ -694,14 +694,14 @@ void launch_finalize(const float* partial, const ProloguePlan& p, int H, int tra
 // ------------------------------------------------------------------------------------------------------------
 // Backward of the prologue (batch norm + gate product), for the differentiable composition of the block.
 //   d   = dlogits (fp32) rounded to the activation dtype          q = round((x - mean) * rstd)     [recomputed]
-//   dWr = d^T q,  dq = d Wr                                        (library GEMMs)
+//   dWr = d^T q,  dq = d Wr                                        (gemm_backward)
 //   dx  = rstd * (dq - mean_t(dq) - xhat * mean_t(dq * xhat))      (training; xhat unrounded)   |   rstd * dq  (evaluation)
 // ------------------------------------------------------------------------------------------------------------
 // Workgroup b: row b / col_blocks of q (and of d), packets (b % col_blocks) * 256 + thread of that row.
 template <typename T>
 __global__ __launch_bounds__(256) void prologue_bwd_prepare_kernel(const float* __restrict__ dlogits, const T* __restrict__ x,
                                                                   const float* __restrict__ mean_rstd, T* __restrict__ d16,
-                                                                  T* __restrict__ q, int hidden, int n_out, int col_blocks) {
+                                                                  T* __restrict__ q, int hidden, int n_out, int n_pad, int col_blocks) {
     constexpr int V = Elem<T>::kVec;
     const uint32_t row = blockIdx.x / (uint32_t)col_blocks;
     const int pc = (int)(blockIdx.x % (uint32_t)col_blocks) * 256 + (int)threadIdx.x;
@@ -719,21 +719,22 @@ __global__ __launch_bounds__(256) void prologue_bwd_prepare_kernel(const float* 
         }
         *reinterpret_cast<u32x4_t*>(q + at) = pack16<T>(qv);
     }
-    if (col < n_out) {
+    if (col < n_pad) {
+        // rows of d are padded with zeros to a whole number of packets
         const int64_t at = (int64_t)row * n_out + col;
+        float dv[V];
         if (n_out % V == 0) {
-            float dv[V];
 #pragma unroll
             for (int h = 0; h < V / 4; ++h) {
                 const f32x4_t g = *reinterpret_cast<const f32x4_t*>(dlogits + at + 4 * h);
 #pragma unroll
                 for (int j = 0; j < 4; ++j) dv[4 * h + j] = g[j];
             }
-            *reinterpret_cast<u32x4_t*>(d16 + at) = pack16<T>(dv);
         } else {
-            // rows of d that are not a whole number of 16-byte packets (2*nk not a multiple of V): element by element
-            for (int j = 0; j < V && col + j < n_out; ++j) d16[at + j] = Elem<T>::from_f32(dlogits[at + j]);
+#pragma unroll
+            for (int j = 0; j < V; ++j) dv[j] = col + j < n_out ? dlogits[at + j] : 0.0f;
         }
+        *reinterpret_cast<u32x4_t*>(d16 + (int64_t)row * n_pad + col) = pack16<T>(dv);
     }
 }
 
@@ -918,7 +919,8 @@ __global__ __launch_bounds__(256) void bn_bwd_apply_kernel(const T* __restrict__
 }
 
 struct PrologueBwdPlan {
-    size_t off_d16, off_dT, off_q, off_dq, off_partial, off_sums, bytes;
+    int n_pad;            // row length of d in the activation dtype: 2 * nk rounded up to whole packets
+    size_t off_d16, off_dT, off_q, off_dq, off_partial, off_sums, off_part, part_bytes, bytes;
 };
 
 PrologueBwdPlan plan_prologue_backward(int64_t T_, int H, int nk, int dtype) {
@@ -926,12 +928,18 @@ PrologueBwdPlan plan_prologue_backward(int64_t T_, int H, int nk, int dtype) {
     const size_t elt = dtype_size(dtype);
     size_t o = 0;
     auto take = [&](size_t n) { const size_t at = o; o = round_up(o + n, 256); return at; };
-    p.off_d16 = take((size_t)T_ * 2 * nk * elt);
+    const int vec = (int)(16 / elt), t = (int)T_;
+    p.n_pad = (2 * nk + vec - 1) / vec * vec;
+    p.off_d16 = take((size_t)T_ * p.n_pad * elt);
     p.off_dT = take((size_t)T_ * 2 * nk * elt);
     p.off_q = take((size_t)T_ * H * elt);
     p.off_dq = take((size_t)T_ * H * elt);
     p.off_partial = take((size_t)kMaxRowBlocks * 2 * H * 4);
     p.off_sums = take((size_t)2 * H * 4);
+    p.part_bytes = gemm_backward_workspace_bytes(kBlasTN, 2 * nk, H, t, 1, dtype);
+    const size_t dq = gemm_backward_workspace_bytes(kBlasNN, t, H, 2 * nk, 1, dtype);
+    if (dq > p.part_bytes) p.part_bytes = dq;
+    p.off_part = take(p.part_bytes);
     p.bytes = o;
     return p;
 }
@@ -947,11 +955,12 @@ int launch_prologue_backward(const float* dlogits, const void* x, const void* ga
     T *d16 = (T*)(ws + p.off_d16), *q = (T*)(ws + p.off_q), *dq = (T*)(ws + p.off_dq);
     float *partial = (float*)(ws + p.off_partial), *sums = (float*)(ws + p.off_sums);
     const int N = 2 * nk;
-    const int widest = H > N ? H : N;
+    const int widest = H > p.n_pad ? H : p.n_pad;
+    void* part = ws + p.off_part;
     const int col_blocks = ((widest + V - 1) / V + 255) / 256;
     bool transposed = false;
     if constexpr (sizeof(T) == 2) {
-        if (T_ % 64 == 0 && H % 64 == 0 && N % 64 == 0) {
+        if (!gemm_backward_own(N, H, (int)T_, dtype) && T_ % 64 == 0 && H % 64 == 0 && N % 64 == 0) {
             // dWr[N, H] = dT[N, T] qT[H, T]^T: both operands K-contiguous, the forward's own GEMM ("down" form)
             T* dT = (T*)(ws + p.off_dT);
             hipLaunchKernelGGL((prologue_bwd_prepare_transposed_kernel<T>), dim3((unsigned)(T_ / 64), (unsigned)((H + N) / 64)),
@@ -963,11 +972,11 @@ int launch_prologue_backward(const float* dlogits, const void* x, const void* ga
     }
     if (!transposed) {
         hipLaunchKernelGGL((prologue_bwd_prepare_kernel<T>), dim3((unsigned)(T_ * col_blocks)), dim3(256), 0, s, dlogits,
-                           (const T*)x, mean_rstd, d16, q, H, N, col_blocks);
+                           (const T*)x, mean_rstd, d16, q, H, N, p.n_pad, col_blocks);
         FMOE_CHECK_LAUNCH("fmoe_router_prologue_backward(prepare)");
-        if (int rc = blas_gemm(kBlasTN, N, H, (int)T_, d16, N, q, H, dgate_w, H, 0.0f, dtype, s)) return rc;      // dWr = d^T q
+        if (int rc = gemm_backward(kBlasTN, N, H, (int)T_, d16, p.n_pad, q, nullptr, H, dgate_w, H, dtype, part, p.part_bytes, s)) return rc;   // dWr = d^T q
     }
-    if (int rc = blas_gemm(kBlasNN, (int)T_, H, N, d16, N, gate_w, H, dq, H, 0.0f, dtype, s)) return rc;       // dq = d Wr
+    if (int rc = gemm_backward(kBlasNN, (int)T_, H, N, d16, p.n_pad, gate_w, nullptr, H, dq, H, dtype, part, p.part_bytes, s)) return rc;   // dq = d Wr
     if (training) {
         const int strips = (H + kWave * V - 1) / (kWave * V);
         hipLaunchKernelGGL((bn_bwd_partial_kernel<T>), dim3((unsigned)rows.row_blocks, (unsigned)strips), dim3(kStatsThreads), 0, s,

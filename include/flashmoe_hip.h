@@ -338,7 +338,7 @@ int fmoe_route_backward(const void* dgates, const int64_t* indices, const float*
  * fp32, at byte offset fmoe_router_workspace_stats_offset() of its workspace; pass that as mean_rstd.
  *   dlogits_fp32 [T, 2*nk] fp32 (rounded to dtype for the two GEMMs); dx [T,H], dgate_w [2*nk,H]: dtype.
  * training != 0: batch statistics were used (the gradient flows through mean and variance); else running statistics
- * (constants).  The two GEMMs are rocBLAS calls.
+ * (constants).  The two GEMMs are rocBLAS calls, or this library's own kernels up to 5 GFLOP in the 16-bit dtypes.
  * Limits of this build: num_tokens < 2^24; hidden a whole number of 16-byte packets; any num_keys the forward accepts. */
 size_t fmoe_router_workspace_stats_offset(int64_t num_tokens, int hidden, int num_keys);
 size_t fmoe_router_prologue_backward_workspace_bytes(int64_t num_tokens, int hidden, int num_keys, int dtype);
@@ -354,7 +354,8 @@ int fmoe_swiglu_backward(const void* dc, const void* a, const void* b, int64_t r
 /* Backward of triton_flash_mlp_func (flash_moe/ops/triton/flash_mlp.py:169-181: two matmuls, TritonSwiGLUFunc, one
  * matmul, differentiated by autograd in the reference): from dy [T,H] the gradients dx [T,H], dgate_w, dup_w [I,H],
  * ddown_w [H,I].  saved_products: the [2,T,I] buffer fmoe_mlp_gate_up_save() filled in the forward, or NULL to
- * recompute the gate and up products here.  The transposed-operand GEMMs are rocBLAS calls (loaded on first use;
+ * recompute the gate and up products here.  The transposed-operand GEMMs are rocBLAS calls (loaded on first use, from 5 GFLOP on
+ * in the 16-bit dtypes and always in fp32; this library's own kernels below;
  * FMOE_ERR_LIBRARY if unavailable).  When dup_w starts where dgate_w ends (one [2I,H] buffer) the two weight gradients
  * are formed as one product (faster; the sums may differ in the last bit from two products); separate buffers work as well. */
 size_t fmoe_mlp_backward_workspace_bytes(int64_t num_tokens, int hidden, int intermediate, int dtype);

@@ -529,3 +529,27 @@ def test_expert_backward_with_skewed_routing_is_exact_and_quick():
     u_e = do64[tok] @ wu64[e]
     assert rel_fro(got[2][e], (s_e * sig_e * g64[tok, slot]) @ do64[tok]) < 1.5e-2
     assert rel_fro(got[1][e], (u_e * g64[tok, slot] * (sig_e * (1 + s_e * (1 - sig_e)))) @ x64[tok]) < 1.5e-2
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("T,H,I", [
+    (1, 8, 8), (9, 72, 136),                           # less than a tile on every side
+    (65, 64, 1032), (127, 136, 264),                   # a row or a packet more or less than whole 64 x 64 tiles
+    (48, 128, 4104),                                   # few tiles, long k: k split over workgroups (dx) and one k-tile (dW)
+    (300, 264, 2056),                                  # one tile per compute unit at most: two k groups (dx)
+    (1000, 2048, 1032),                                # 128 x 128 tiles with remainders
+])
+def test_mlp_backward_remainders_of_the_transposing_products(dtype, T, H, I):
+    from flash_moe.ops.hip.flash_mlp import mlp_backward, mlp_forward_saving
+
+    g = gen(T + I)
+    x, dy = (torch.randn(T, H, generator=g).to(dtype).cuda() for _ in range(2))
+    ws = [(torch.randn(s, generator=g) * 0.05).to(dtype).cuda() for s in ((I, H), (I, H), (H, I))]
+    saved = mlp_forward_saving(x, *ws)[1]
+    got = mlp_backward(dy, x, *ws, saved)
+    leaves = [t.double().requires_grad_(True) for t in (x, *ws)]
+    h = torch.nn.functional.silu(leaves[0] @ leaves[1].t()) * (leaves[0] @ leaves[2].t())
+    (h @ leaves[3].t()).backward(dy.double())
+    for name, a, leaf in zip(("dx", "dgate", "dup", "ddown"), got, leaves):
+        assert rel_fro(a, leaf.grad) < GRAD_FRO[dtype], name
+    assert all(torch.equal(a, b) for a, b in zip(got, mlp_backward(dy, x, *ws, saved)))      # bit for bit the same twice
