@@ -334,26 +334,32 @@ __global__ __launch_bounds__(kBwdWaves* kWave) void expert_backward_token_kernel
 }
 
 // Column-slice schedule of the per-token part (same kernels as the forward, fmoe_expert.hip): the partial dot products
-// s = <x, down[e]> and u = <dout, up[e]> come per slice; this kernel sums them and forms every pair's coefficients,
-// gate gradient and histogram entry; dx is then the forward's `states` pass over `down` with coef_down.
+// s = <x, down[e]> and u = <dout, up[e]> come per slice; this kernel sums them (or takes the scores the forward kept) and forms
+// every pair's coefficients, gate gradient and histogram entry; dx is then the forward's `states` pass over `down` with coef_down.
+// place: NULL, or the (token, k) position of every list position: the states pass then needs coef_down in list order as well.
 template <typename T>
 __global__ __launch_bounds__(256) void expert_backward_gate_kernel(
-    const float* __restrict__ spart_s, const float* __restrict__ spart_u, const T* __restrict__ gates,
-    const uint32_t* __restrict__ off32, const int64_t* __restrict__ indices, T* __restrict__ dgates,
-    float* __restrict__ coef_up, float* __restrict__ coef_down, int32_t* __restrict__ counts, int64_t pairs, int num_slices) {
-    const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= pairs) return;
+    const float* __restrict__ spart_s, const float* __restrict__ scores, const float* __restrict__ spart_u,
+    const T* __restrict__ gates, const uint32_t* __restrict__ off32, const uint16_t* __restrict__ place,
+    const int64_t* __restrict__ indices, T* __restrict__ dgates, float* __restrict__ coef_up, float* __restrict__ coef_down,
+    float* __restrict__ coef_list, int32_t* __restrict__ counts, int64_t pairs, int num_slices, int top_k) {
+    const int64_t at = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (at >= pairs) return;
+    const int64_t p = place == nullptr ? at : at / top_k * top_k + place[at];
     float s = 0.0f, u = 0.0f;
     for (int sl = 0; sl < num_slices; ++sl) {
-        s += spart_s[(int64_t)sl * pairs + p];
-        u += spart_u[(int64_t)sl * pairs + p];
+        if (scores == nullptr) s += spart_s[(int64_t)sl * pairs + at];
+        u += spart_u[(int64_t)sl * pairs + at];
     }
-    const bool valid = off32[p] != kExpertBadOffset;
+    if (scores != nullptr) s = scores[p];
+    const bool valid = off32[at] != kExpertBadOffset;
     const float gate = Elem<T>::to_f32(gates[p]);
     const float sig = 1.0f / (1.0f + __expf(-s));
     const float act = s * sig;
     coef_up[p] = valid ? act * gate : 0.0f;
-    coef_down[p] = valid ? u * gate * (sig * (1.0f + s * (1.0f - sig))) : 0.0f;
+    const float cd = valid ? u * gate * (sig * (1.0f + s * (1.0f - sig))) : 0.0f;
+    coef_down[p] = cd;
+    if (place != nullptr) coef_list[at] = cd;
     dgates[p] = Elem<T>::from_f32(valid ? u * act : 0.0f);
     if (valid) atomicAdd(&counts[indices[p]], 1);   // integer histogram: the result does not depend on order
 }
@@ -432,9 +438,9 @@ __global__ __launch_bounds__(kBwdWaves* kWave) void expert_backward_weight_kerne
 }
 
 struct ExpertBwdPlan {
-    bool slices;
+    bool slices, ordered;      // slices: column slices of the tables, on ordered lists or not
     int num_slices;
-    size_t off_coef_up, off_coef_down, off_pairs, off_counts, off_cursor, off_offsets, off_off32, off_spart_s, off_spart_u, bytes;
+    size_t off_coef_up, off_coef_down, off_pairs, off_counts, off_cursor, off_offsets, off_off32, off_place, off_coef_list, off_spart_s, off_spart_u, bytes;
 };
 
 ExpertBwdPlan plan_expert_backward(int64_t T_, int H, int64_t E, int K, int dtype) {
@@ -448,11 +454,15 @@ ExpertBwdPlan plan_expert_backward(int64_t T_, int H, int64_t E, int K, int dtyp
     p.off_counts = take(bucket_workspace_bytes(E));     // per-expert counts, then the fill's cursors, and the scan state
     p.off_cursor = p.off_counts;
     p.off_offsets = take((size_t)(E + 1) * 4);
-    p.slices = expert_slices_usable(T_, H, E, K, dtype);
-    p.num_slices = p.slices ? expert_slice_count(T_, H, E, K, dtype) : 0;
-    p.off_off32 = p.off_spart_s = p.off_spart_u = o;
+    const ExpertSavedPlan kept = expert_saved_plan(T_, H, E, K, dtype);
+    p.slices = kept.kept;
+    p.ordered = kept.ordered;
+    p.num_slices = p.slices ? expert_slice_count(T_, H, E, K, dtype, p.ordered) : 0;
+    p.off_off32 = p.off_place = p.off_coef_list = p.off_spart_s = p.off_spart_u = o;
     if (p.slices) {
         p.off_off32 = take(pairs * 4);
+        p.off_place = take(p.ordered ? pairs * 2 : 0);
+        p.off_coef_list = take(p.ordered ? pairs * 4 : 0);
         p.off_spart_s = take((size_t)p.num_slices * pairs * 4);
         p.off_spart_u = take((size_t)p.num_slices * pairs * 4);
     }
@@ -463,7 +473,7 @@ ExpertBwdPlan plan_expert_backward(int64_t T_, int H, int64_t E, int K, int dtyp
 template <typename T>
 int launch_expert_backward(const void* dout, const void* x, const void* down, const void* up, const int64_t* indices,
                            const void* gates, int64_t T_, int H, int64_t E, int K, int dtype, void* dx, void* ddown, void* dup,
-                           void* dgates, void* workspace, hipStream_t stream) {
+                           void* dgates, const void* saved, void* workspace, hipStream_t stream) {
     constexpr int V = Elem<T>::kVec;
     const ExpertBwdPlan p = plan_expert_backward(T_, H, E, K, dtype);
     char* ws = (char*)workspace;
@@ -482,16 +492,28 @@ int launch_expert_backward(const void* dout, const void* x, const void* down, co
     if (int rc = bucket_clear(bucket_ws, E, stream)) return rc;
     if (p.slices) {
         uint32_t* off32 = (uint32_t*)(ws + p.off_off32);
+        uint16_t* place = p.ordered ? (uint16_t*)(ws + p.off_place) : nullptr;
         float* spart_s = (float*)(ws + p.off_spart_s);
         float* spart_u = (float*)(ws + p.off_spart_u);
-        if (int rc = expert_slice_prepare(indices, off32, pairs, H, E, dtype, stream)) return rc;
-        if (int rc = expert_slice_scores(x, down, off32, spart_s, T_, H, E, K, dtype, stream)) return rc;
-        if (int rc = expert_slice_scores(dout, up, off32, spart_u, T_, H, E, K, dtype, stream)) return rc;
+        float* coef_list = p.ordered ? (float*)(ws + p.off_coef_list) : coef_down;
+        const float* scores = nullptr;
+        if (saved != nullptr) {
+            const ExpertSaved kept = expert_saved_plan(T_, H, E, K, dtype).at(saved);
+            off32 = kept.off32;
+            if (p.ordered) place = kept.place;
+            scores = kept.scores;
+        } else {
+            if (int rc = p.ordered ? expert_order(indices, off32, place, T_, H, E, K, dtype, stream)
+                                   : expert_slice_prepare(indices, off32, pairs, H, E, dtype, stream))
+                return rc;
+            if (int rc = expert_slice_scores(x, down, off32, spart_s, T_, H, E, K, dtype, p.ordered, stream)) return rc;
+        }
+        if (int rc = expert_slice_scores(dout, up, off32, spart_u, T_, H, E, K, dtype, p.ordered, stream)) return rc;
         hipLaunchKernelGGL((expert_backward_gate_kernel<T>), dim3((unsigned)((pairs + 255) / 256)), dim3(256), 0, stream,
-                           (const float*)spart_s, (const float*)spart_u, (const T*)gates, (const uint32_t*)off32, indices,
-                           (T*)dgates, coef_up, coef_down, counts, pairs, p.num_slices);
+                           (const float*)spart_s, scores, (const float*)spart_u, (const T*)gates, (const uint32_t*)off32,
+                           (const uint16_t*)place, indices, (T*)dgates, coef_up, coef_down, coef_list, counts, pairs, p.num_slices, K);
         FMOE_CHECK_LAUNCH("fmoe_expert_backward(coefficients)");
-        if (int rc = expert_slice_states(coef_down, down, off32, dx, T_, H, E, K, dtype, stream)) return rc;
+        if (int rc = expert_slice_states(coef_list, down, off32, dx, T_, H, E, K, dtype, p.ordered, stream)) return rc;
     } else {
 #define FMOE_LAUNCH_TOKEN(N)                                                                                          \
         hipLaunchKernelGGL((expert_backward_token_kernel<T, N>), token_grid, block, 0, stream, (const T*)dout, (const T*)x, \
@@ -626,6 +648,14 @@ extern "C" int fmoe_expert_backward(const void* dout, const void* x, const void*
                                     const void* gates, int64_t num_tokens, int hidden, int64_t num_experts, int top_k, int dtype,
                                     void* dx, void* ddown, void* dup, void* dgates, void* workspace, size_t workspace_bytes,
                                     void* stream) {
+    return fmoe_expert_backward_saved(dout, x, down, up, indices, gates, nullptr, num_tokens, hidden, num_experts, top_k, dtype, dx, ddown,
+                                      dup, dgates, workspace, workspace_bytes, stream);
+}
+
+extern "C" int fmoe_expert_backward_saved(const void* dout, const void* x, const void* down, const void* up, const int64_t* indices,
+                                          const void* gates, const void* saved, int64_t num_tokens, int hidden, int64_t num_experts,
+                                          int top_k, int dtype, void* dx, void* ddown, void* dup, void* dgates, void* workspace,
+                                          size_t workspace_bytes, void* stream) {
     using namespace fmoe;
     clear_error();
     FMOE_REQUIRE(dtype_ok(dtype), FMOE_ERR_BAD_DTYPE, "fmoe_expert_backward: unknown dtype %d", dtype);
@@ -658,8 +688,8 @@ extern "C" int fmoe_expert_backward(const void* dout, const void* x, const void*
     FMOE_REQUIRE(workspace && workspace_bytes >= need && aligned16(workspace), FMOE_ERR_WORKSPACE,
                  "fmoe_expert_backward: workspace of %zu bytes needed, %zu given", need, workspace_bytes);
     switch (dtype) {
-        case FMOE_F32: return launch_expert_backward<float>(dout, x, down, up, indices, gates, num_tokens, hidden, num_experts, top_k, dtype, dx, ddown, dup, dgates, workspace, s);
-        case FMOE_BF16: return launch_expert_backward<bf16_t>(dout, x, down, up, indices, gates, num_tokens, hidden, num_experts, top_k, dtype, dx, ddown, dup, dgates, workspace, s);
-        default: return launch_expert_backward<f16_t>(dout, x, down, up, indices, gates, num_tokens, hidden, num_experts, top_k, dtype, dx, ddown, dup, dgates, workspace, s);
+        case FMOE_F32: return launch_expert_backward<float>(dout, x, down, up, indices, gates, num_tokens, hidden, num_experts, top_k, dtype, dx, ddown, dup, dgates, saved, workspace, s);
+        case FMOE_BF16: return launch_expert_backward<bf16_t>(dout, x, down, up, indices, gates, num_tokens, hidden, num_experts, top_k, dtype, dx, ddown, dup, dgates, saved, workspace, s);
+        default: return launch_expert_backward<f16_t>(dout, x, down, up, indices, gates, num_tokens, hidden, num_experts, top_k, dtype, dx, ddown, dup, dgates, saved, workspace, s);
     }
 }

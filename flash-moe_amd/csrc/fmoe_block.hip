@@ -44,10 +44,10 @@ namespace {
 
 // What a training forward leaves for the backward, in one caller-owned buffer.
 struct SavedPlan {
-    size_t off_logits32, off_indices, off_gates, off_stats, off_products, bytes;
+    size_t off_logits32, off_indices, off_gates, off_stats, off_products, off_experts, bytes;
 };
 
-SavedPlan plan_saved(int64_t T_, int H, int I, int nk, int K, int dtype) {
+SavedPlan plan_saved(int64_t T_, int H, int I, int nk, int64_t E, int K, int dtype) {
     SavedPlan p;
     const size_t elt = dtype_size(dtype);
     size_t o = 0;
@@ -57,6 +57,7 @@ SavedPlan plan_saved(int64_t T_, int H, int I, int nk, int K, int dtype) {
     p.off_gates = take((size_t)T_ * K * elt);
     p.off_stats = take((size_t)2 * H * 4);
     p.off_products = take((size_t)2 * T_ * I * elt);
+    p.off_experts = take(fmoe_expert_saved_bytes(T_, H, E, K, dtype));
     p.bytes = o;
     return p;
 }
@@ -128,8 +129,10 @@ int block_forward_impl(const char* who, const void* x, const void* gate_proj_w, 
     void* gates = gates_out ? gates_out : (void*)(ws + p.off_gates);
     float* stats = nullptr;
     void* products = nullptr;
+    void* expert_saved = nullptr;
     if (saved != nullptr) {
-        const SavedPlan sp = plan_saved(num_tokens, hidden, intermediate, num_keys, top_k, dtype);
+        const SavedPlan sp = plan_saved(num_tokens, hidden, intermediate, num_keys, num_experts, top_k, dtype);
+        expert_saved = saved + sp.off_experts;
         logits32 = (float*)(saved + sp.off_logits32);
         indices = (int64_t*)(saved + sp.off_indices);
         gates = saved + sp.off_gates;
@@ -142,16 +145,27 @@ int block_forward_impl(const char* who, const void* x, const void* gate_proj_w, 
     const size_t elt = dtype_size(dtype);
 
     const bool slices = expert_slices_usable(num_tokens, hidden, num_experts, top_k, dtype);
+    uint32_t* offsets = slices ? expert_workspace_offsets(expert_ws) : nullptr;
+    float* expert_scores = nullptr;
+    if (slices && expert_saved != nullptr) {
+        const ExpertSaved kept = expert_saved_plan(num_tokens, hidden, num_experts, top_k, dtype).at(expert_saved);
+        offsets = kept.off32;
+        expert_scores = kept.scores;
+    }
     int rc = router_forward_impl(x, router_gate_w, running_mean, running_var, num_batches_tracked, stats_dtype, training,
                                  momentum, eps, num_tokens, hidden, num_keys, top_k, dtype, norm_topk_prob, router_logits,
-                                 logits32, scores, indices, gates, slices ? expert_workspace_offsets(expert_ws) : nullptr,
+                                 logits32, scores, indices, gates, offsets,
                                  (uint32_t)(hidden * elt), ws + p.off_router, p.off_logits32 - p.off_router, s, 0, 0, stats);
     if (rc) return rc;
     const void* residual = nullptr;
     if (top_k > 0) {
         if (slices)
             rc = expert_slices_prepared(x, down_embed, up_embed, gates, num_tokens, hidden, num_experts, top_k, dtype, experts,
-                                        expert_ws, s);
+                                        expert_ws, offsets, expert_scores, s);
+        else if (expert_saved != nullptr)
+            rc = fmoe_expert_forward_save(x, down_embed, up_embed, indices, gates, num_tokens, hidden, num_experts, top_k, dtype, experts,
+                                          expert_saved, fmoe_expert_saved_bytes(num_tokens, hidden, num_experts, top_k, dtype), expert_ws,
+                                          p.off_act - p.off_expert, stream);
         else
             rc = fmoe_expert_forward(x, down_embed, up_embed, indices, gates, num_tokens, hidden, num_experts, top_k, dtype,
                                      experts, expert_ws, p.off_act - p.off_expert, stream);
@@ -185,7 +199,7 @@ extern "C" size_t fmoe_block_saved_bytes(int64_t num_tokens, int hidden, int int
                                          int top_k, int dtype) {
     if (num_tokens <= 0 || hidden <= 0 || intermediate <= 0 || num_keys <= 0 || num_experts <= 0 || top_k <= 0 || !fmoe::dtype_ok(dtype))
         return 0;
-    return fmoe::plan_saved(num_tokens, hidden, intermediate, num_keys, top_k, dtype).bytes;
+    return fmoe::plan_saved(num_tokens, hidden, intermediate, num_keys, num_experts, top_k, dtype).bytes;
 }
 
 extern "C" int fmoe_block_forward_save(const void* x, const void* gate_proj_w, const void* up_proj_w, const void* down_proj_w,
@@ -229,7 +243,7 @@ extern "C" int fmoe_block_backward(const void* dout, const void* dlogits, const 
     const BlockBackwardPlan p = plan_block_backward(num_tokens, hidden, intermediate, num_keys, num_experts, top_k, dtype);
     FMOE_REQUIRE(workspace && workspace_bytes >= p.bytes && aligned16(workspace), FMOE_ERR_WORKSPACE,
                  "fmoe_block_backward: workspace of %zu bytes needed, %zu given", p.bytes, workspace_bytes);
-    const SavedPlan sp = plan_saved(num_tokens, hidden, intermediate, num_keys, top_k, dtype);
+    const SavedPlan sp = plan_saved(num_tokens, hidden, intermediate, num_keys, num_experts, top_k, dtype);
     const char* sv = (const char*)saved;
     const float* logits32 = (const float*)(sv + sp.off_logits32);
     const int64_t* indices = (const int64_t*)(sv + sp.off_indices);
@@ -239,8 +253,8 @@ extern "C" int fmoe_block_backward(const void* dout, const void* dlogits, const 
     int rc = fmoe_mlp_backward(dout, x, gate_proj_w, up_proj_w, down_proj_w, sv + sp.off_products, num_tokens, hidden, intermediate,
                                dtype, dx, dgate_proj_w, dup_proj_w, ddown_proj_w, stage, p.stage_bytes, stream);
     if (rc) return rc;
-    rc = fmoe_expert_backward(dout, x, down_embed, up_embed, indices, sv + sp.off_gates, num_tokens, hidden, num_experts, top_k, dtype,
-                              dx_experts, ddown_embed, dup_embed, dgates, stage, p.stage_bytes, stream);
+    rc = fmoe_expert_backward_saved(dout, x, down_embed, up_embed, indices, sv + sp.off_gates, sv + sp.off_experts, num_tokens, hidden,
+                                    num_experts, top_k, dtype, dx_experts, ddown_embed, dup_embed, dgates, stage, p.stage_bytes, stream);
     if (rc) return rc;
     rc = route_backward_impl(dgates, indices, logits32, dlogits, num_keys, num_tokens * num_keys, num_tokens, num_keys, top_k, dtype,
                              norm_topk_prob, dlogits32, (hipStream_t)stream);

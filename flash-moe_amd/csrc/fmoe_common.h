@@ -74,24 +74,41 @@ int route_backward_impl(const void* dgates, const int64_t* indices, const float*
                         int64_t extra_token, int64_t extra_half, int64_t num_tokens, int num_keys, int top_k, int dtype,
                         int norm_topk_prob, float* dlogits_fp32, hipStream_t stream);
 
-// Column-slice schedule of the routed experts on row offsets that are already in place at the start of `workspace`
-// (the layout fmoe_expert_workspace_bytes describes); defined in fmoe_expert.hip.
+// Column-slice schedule of the routed experts on row offsets that are already in place (off32; expert_workspace_offsets is where a
+// caller without a place of its own puts them), `workspace` as fmoe_expert_workspace_bytes describes; scores: NULL, or where the
+// complete scores go; defined in fmoe_expert.hip.
 bool expert_slices_usable(int64_t num_tokens, int hidden, int64_t num_experts, int top_k, int dtype);
 uint32_t* expert_workspace_offsets(void* workspace);
 int expert_slices_prepared(const void* x, const void* down, const void* up, const void* gates, int64_t num_tokens,
                            int hidden, int64_t num_experts, int top_k, int dtype, void* out, void* workspace,
-                           hipStream_t stream);
+                           const uint32_t* off32, float* scores, hipStream_t stream);
+// What a forward leaves for the backward: complete scores in (token, k) order, the row offsets of every list position and, with
+// ordered lists, the position each came from.  kept: the schedule of these extents leaves it at all.
+struct ExpertSaved {
+    float* scores;
+    uint32_t* off32;
+    uint16_t* place;
+};
+struct ExpertSavedPlan {
+    bool kept, ordered;
+    size_t off_off32, off_place, bytes;
+    ExpertSaved at(const void* buffer) const;
+};
+ExpertSavedPlan expert_saved_plan(int64_t num_tokens, int hidden, int64_t num_experts, int top_k, int dtype);
+int expert_order(const int64_t* indices, uint32_t* off32, uint16_t* place, int64_t num_tokens, int hidden, int64_t num_experts, int top_k,
+                 int dtype, hipStream_t stream);
 // The same schedule stage by stage (for the backward pass): row byte offsets of the ids (kExpertBadOffset for an id
 // outside [0,E)), per-slice partial dot products spart[slice][pair] = <x[token, slice], table[expert, slice]>, and
-// out[token, :] = sum_k coef[token,k] * table[expert_k, :].  expert_slice_count is the number of slices.
+// out[token, :] = sum_k coef[token,k] * table[expert_k, :].  expert_slice_count is the number of slices.  ordered: on ordered lists
+// (expert_order) of the ordered schedule.
 constexpr uint32_t kExpertBadOffset = 0xFFF00000u;   // beyond any table the slice schedule accepts
-int expert_slice_count(int64_t num_tokens, int hidden, int64_t num_experts, int top_k, int dtype);
+int expert_slice_count(int64_t num_tokens, int hidden, int64_t num_experts, int top_k, int dtype, bool ordered);
 int expert_slice_prepare(const int64_t* indices, uint32_t* off32, int64_t pairs, int hidden, int64_t num_experts, int dtype,
                          hipStream_t stream);
 int expert_slice_scores(const void* x, const void* table, const uint32_t* off32, float* spart, int64_t num_tokens, int hidden,
-                        int64_t num_experts, int top_k, int dtype, hipStream_t stream);
+                        int64_t num_experts, int top_k, int dtype, bool ordered, hipStream_t stream);
 int expert_slice_states(const float* coef, const void* table, const uint32_t* off32, void* out, int64_t num_tokens, int hidden,
-                        int64_t num_experts, int top_k, int dtype, hipStream_t stream);
+                        int64_t num_experts, int top_k, int dtype, bool ordered, hipStream_t stream);
 
 // C[M,N] = A[M,K] * B[N,K]^T written in the 16-bit dtype and in fp32, on the shared MLP's tiled kernel (fmoe_mlp.hip);
 // usable when the extents are whole tiles and there are enough of them.

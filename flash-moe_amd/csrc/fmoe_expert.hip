@@ -357,15 +357,20 @@ __global__ __launch_bounds__(256) void expert_scores_slice_kernel(
     }
 }
 
+// place: NULL, or the position in its token's row that list position p came from (ordered lists).  scores: NULL, or where the
+// complete scores go, in (token, k) order, for a backward pass
 template <typename T, int ACT>
 __global__ __launch_bounds__(256) void expert_gate_kernel(const float* __restrict__ spart, const T* __restrict__ gates,
-                                                          const uint32_t* __restrict__ off32, float* __restrict__ a,
-                                                          int64_t pairs, int num_slices) {
+                                                          const uint32_t* __restrict__ off32, const uint16_t* __restrict__ place,
+                                                          float* __restrict__ a, float* __restrict__ scores, int64_t pairs,
+                                                          int num_slices, int top_k) {
     const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= pairs) return;
     float s = 0.0f;
     for (int sl = 0; sl < num_slices; ++sl) s += spart[(int64_t)sl * pairs + p];
-    a[p] = off32[p] != kBadOffset ? activate<ACT>(s) * Elem<T>::to_f32(gates[p]) : 0.0f;
+    const int64_t q = place == nullptr ? p : p / top_k * top_k + place[p];
+    a[p] = off32[p] != kBadOffset ? activate<ACT>(s) * Elem<T>::to_f32(gates[q]) : 0.0f;
+    if (scores != nullptr) scores[q] = s;
 }
 
 // acc[0..kVec) += a0 * w0 + a1 * w1 for two 16-byte packets of two different rows
@@ -457,16 +462,16 @@ __global__ __launch_bounds__(256) void expert_states_slice_kernel(
 struct SlicePlan {
     int chunk_lanes, num_slices, blocks_per_slice, tokens_per_block, xcds;
     unsigned grid;
-    size_t off_idx32, off_a, off_spart, bytes;
+    size_t off_idx32, off_a, off_spart, off_place, bytes;
 };
 
 // A slice is as wide as one XCD's 4 MiB L2 can keep resident: 256 bytes per row up to 16384 rows (fewer passes over
 // the offsets, coefficients and partial sums), 128 bytes beyond.
-SlicePlan plan_slices(int64_t T_, int H, int64_t E, int K, size_t elt) {
+SlicePlan plan_slices(int64_t T_, int H, int64_t E, int K, size_t elt, bool ordered = false, bool scored = true) {
     SlicePlan p;
     const ChipInfo& chip = chip_info();
     p.xcds = chip.xcds;
-    p.chunk_lanes = E * 256 <= chip.l2_bytes ? 16 : 8;
+    p.chunk_lanes = ordered || E * 256 <= chip.l2_bytes ? 16 : 8;
     const size_t chunk_bytes = (size_t)p.chunk_lanes * 16;
     p.num_slices = (int)((H * elt + chunk_bytes - 1) / chunk_bytes);
     const int64_t want = (T_ + 3) / 4;                       // at least one token per wave
@@ -477,15 +482,15 @@ SlicePlan plan_slices(int64_t T_, int H, int64_t E, int K, size_t elt) {
     p.off_idx32 = 0;
     p.off_a = round_up(p.off_idx32 + pairs * 4, 256);
     p.off_spart = round_up(p.off_a + pairs * 4, 256);
-    p.bytes = round_up(p.off_spart + (size_t)p.num_slices * pairs * 4, 256);
+    p.off_place = round_up(p.off_spart + (ordered && !scored ? 0 : (size_t)p.num_slices * pairs * 4), 256);
+    p.bytes = ordered ? round_up(p.off_place + pairs * 2, 256) : p.off_place;
     return p;
 }
 
 // ids != nullptr: off32 is written by this launch (from the ids) instead of read
 template <typename T>
-int launch_slice_scores(const void* x, const void* table, const uint32_t* off32, float* spart, int64_t T_, int H, int64_t E,
-                        int K, hipStream_t stream, const int64_t* ids = nullptr) {
-    const SlicePlan p = plan_slices(T_, H, E, K, sizeof(T));
+int launch_slice_scores(const SlicePlan& p, const void* x, const void* table, const uint32_t* off32, float* spart, int64_t T_, int H,
+                        int64_t E, int K, hipStream_t stream, const int64_t* ids = nullptr) {
     const uint32_t table_bytes = (uint32_t)(E * (int64_t)H * (int64_t)sizeof(T));
     if (ids != nullptr) {
         if (p.chunk_lanes == 16)
@@ -509,9 +514,14 @@ int launch_slice_scores(const void* x, const void* table, const uint32_t* off32,
 }
 
 template <typename T>
-int launch_slice_states(const float* a, const void* table, const uint32_t* off32, void* out, int64_t T_, int H, int64_t E,
-                        int K, hipStream_t stream) {
-    const SlicePlan p = plan_slices(T_, H, E, K, sizeof(T));
+int launch_slice_scores_prepared(const SlicePlan& p, const void* x, const void* table, const uint32_t* off32, float* spart, int64_t T_, int H,
+                                 int64_t E, int K, hipStream_t stream) {
+    return launch_slice_scores<T>(p, x, table, off32, spart, T_, H, E, K, stream);
+}
+
+template <typename T>
+int launch_slice_states(const SlicePlan& p, const float* a, const void* table, const uint32_t* off32, void* out, int64_t T_, int H,
+                        int64_t E, int K, hipStream_t stream) {
     const uint32_t table_bytes = (uint32_t)(E * (int64_t)H * (int64_t)sizeof(T));
     if (p.chunk_lanes == 16)
         hipLaunchKernelGGL((expert_states_slice_kernel<T, 16>), dim3(p.grid), dim3(256), 0, stream, a, (const T*)table,
@@ -523,47 +533,287 @@ int launch_slice_states(const float* a, const void* table, const uint32_t* off32
     return FMOE_OK;
 }
 
-// Scores, gate and states launches on row offsets that already sit at the start of the workspace.
-// ids != nullptr: the offsets are not in the workspace yet; the score launch writes them on its way
+// Sum of the partial scores, activation, gate.  Without a score (product-key memory) the coefficient is the routing weight: no
+// partial sums are read.
 template <typename T>
-int launch_expert_slices_prepared(int act, const void* x, const void* down, const void* up, const void* gates, int64_t T_,
-                                  int H, int64_t E, int K, void* out, void* workspace, hipStream_t stream,
-                                  const int64_t* ids = nullptr) {
-    const SlicePlan p = plan_slices(T_, H, E, K, sizeof(T));
+int launch_expert_gate(int act, const float* spart, const void* gates, const uint32_t* off32, const uint16_t* place, float* a, float* scores,
+                       int64_t pairs, int num_slices, int K, hipStream_t stream) {
+    const dim3 grid((unsigned)((pairs + 255) / 256));
+    if (act == kActSilu)
+        hipLaunchKernelGGL((expert_gate_kernel<T, kActSilu>), grid, dim3(256), 0, stream, spart, (const T*)gates, off32, place, a, scores, pairs, num_slices, K);
+    else if (act == kActGelu)
+        hipLaunchKernelGGL((expert_gate_kernel<T, kActGelu>), grid, dim3(256), 0, stream, spart, (const T*)gates, off32, place, a, scores, pairs, num_slices, K);
+    else
+        hipLaunchKernelGGL((expert_gate_kernel<T, kActNone>), grid, dim3(256), 0, stream, spart, (const T*)gates, off32, place, a, scores, pairs, 0, K);
+    FMOE_CHECK_LAUNCH("fmoe_expert_forward(gate)");
+    return FMOE_OK;
+}
+
+// Scores, gate and states launches on row offsets.
+// ids != nullptr: the offsets are not there yet; the score launch writes them on its way
+template <typename T>
+int launch_expert_slices_prepared(const SlicePlan& p, int act, const void* x, const void* down, const void* up, const void* gates,
+                                  int64_t T_, int H, int64_t E, int K, void* out, void* workspace, const uint32_t* off32, float* scores,
+                                  hipStream_t stream, const int64_t* ids = nullptr) {
     char* ws = (char*)workspace;
-    const uint32_t* off32 = (const uint32_t*)(ws + p.off_idx32);
     float* a = (float*)(ws + p.off_a);
     float* spart = (float*)(ws + p.off_spart);
-    const int64_t pairs = T_ * K;
-    const unsigned flat_grid = (unsigned)((pairs + 255) / 256);
     if (act != kActNone)
-        if (int rc = launch_slice_scores<T>(x, down, off32, spart, T_, H, E, K, stream, ids)) return rc;
-    // without a score (product-key memory) the coefficient is the routing weight: no partial sums are read
-    if (act == kActSilu)
-        hipLaunchKernelGGL((expert_gate_kernel<T, kActSilu>), dim3(flat_grid), dim3(256), 0, stream, (const float*)spart,
-                           (const T*)gates, off32, a, pairs, p.num_slices);
-    else if (act == kActGelu)
-        hipLaunchKernelGGL((expert_gate_kernel<T, kActGelu>), dim3(flat_grid), dim3(256), 0, stream, (const float*)spart,
-                           (const T*)gates, off32, a, pairs, p.num_slices);
-    else
-        hipLaunchKernelGGL((expert_gate_kernel<T, kActNone>), dim3(flat_grid), dim3(256), 0, stream, (const float*)spart,
-                           (const T*)gates, off32, a, pairs, 0);
-    FMOE_CHECK_LAUNCH("fmoe_expert_forward(gate)");
-    return launch_slice_states<T>(a, up, off32, out, T_, H, E, K, stream);
+        if (int rc = launch_slice_scores<T>(p, x, down, off32, spart, T_, H, E, K, stream, ids)) return rc;
+    if (int rc = launch_expert_gate<T>(act, spart, gates, off32, nullptr, a, scores, T_ * K, p.num_slices, K, stream)) return rc;
+    return launch_slice_states<T>(p, a, up, off32, out, T_, H, E, K, stream);
 }
 
 template <typename T>
 int launch_expert_slices(int act, const void* x, const void* down, const void* up, const int64_t* indices, const void* gates,
-                         int64_t T_, int H, int64_t E, int K, void* out, void* workspace, hipStream_t stream) {
-    // with a score phase the score launch turns the ids into row offsets itself (and stores them for the launches after it)
-    if (act != kActNone) return launch_expert_slices_prepared<T>(act, x, down, up, gates, T_, H, E, K, out, workspace, stream, indices);
+                         int64_t T_, int H, int64_t E, int K, void* out, void* workspace, const ExpertSaved* saved, hipStream_t stream) {
     const SlicePlan p = plan_slices(T_, H, E, K, sizeof(T));
-    uint32_t* off32 = (uint32_t*)((char*)workspace + p.off_idx32);
+    uint32_t* off32 = saved ? saved->off32 : (uint32_t*)((char*)workspace + p.off_idx32);
+    float* scores = saved ? saved->scores : nullptr;
+    // with a score phase the score launch turns the ids into row offsets itself (and stores them for the launches after it)
+    if (act != kActNone)
+        return launch_expert_slices_prepared<T>(p, act, x, down, up, gates, T_, H, E, K, out, workspace, off32, scores, stream, indices);
     const int64_t pairs = T_ * K;
     hipLaunchKernelGGL(expert_prepare_kernel, dim3((unsigned)((pairs + 255) / 256)), dim3(256), 0, stream, indices, off32,
                        pairs, E, (uint32_t)(H * sizeof(T)));
     FMOE_CHECK_LAUNCH("fmoe_expert_forward(prepare)");
-    return launch_expert_slices_prepared<T>(act, x, down, up, gates, T_, H, E, K, out, workspace, stream);
+    return launch_expert_slices_prepared<T>(p, act, x, down, up, gates, T_, H, E, K, out, workspace, off32, scores, stream);
+}
+
+// ---- ordered slices: column slices of tables far larger than the L2s -----------------------------------------------------
+// A slice of such a table does not stay in an XCD's L2, but the part of it that all resident tokens are at does, if every
+// token's list is in ascending expert order: the waves start together, have lists of one length and gather at one pace, so at
+// any moment they read from one window of the slice, which leaves the fabric once per generation of resident tokens instead of
+// once per pair.  One launch orders the lists, then scores, gate and states run on them as in the slice schedule.
+//
+// One workgroup per token: a stable partition of its list into at most 255 blocks of 2^shift consecutive experts (and one for ids
+// outside the table), in one pass.  Wave w has the w-th eighth of the list; counts per (block, wave), their scan in that order,
+// then every wave hands out its slots 64 positions at a time, the rank among equal blocks from eight ballots.
+constexpr int kOrderMaxTopK = 65536;      // a list position is kept in 16 bits
+constexpr int kOrderBlocks = 256, kOrderTokenWaves = 8;
+inline int order_shift(int64_t E) {
+    int shift = 0;
+    while (((E - 1) >> shift) > kOrderBlocks - 2) ++shift;
+    return shift;
+}
+__global__ __launch_bounds__(kOrderTokenWaves* kWave) void expert_order_kernel(const int64_t* __restrict__ indices, uint32_t* __restrict__ off32,
+                                                                              uint16_t* __restrict__ place, int64_t num_experts, int top_k,
+                                                                              int shift, uint32_t row_bytes) {
+    __shared__ int32_t slots[kOrderBlocks][kOrderTokenWaves];
+    __shared__ int32_t wave_total[kOrderTokenWaves];
+    constexpr int THREADS = kOrderTokenWaves * kWave, PER = kOrderBlocks * kOrderTokenWaves / THREADS;
+    const int tid = (int)threadIdx.x, lane = tid & (kWave - 1), wave = tid >> 6;
+    const int64_t base = (int64_t)blockIdx.x * top_k;
+    const int share = ((top_k + THREADS - 1) / THREADS) * kWave;       // list positions per wave
+    const int begin = wave * share, end = begin + share < top_k ? begin + share : top_k;
+    auto block_of = [&](int64_t e) { return e >= 0 && e < num_experts ? (int)(e >> shift) : kOrderBlocks - 1; };
+#pragma unroll
+    for (int i = 0; i < PER; ++i) (&slots[0][0])[i * THREADS + tid] = 0;
+    __syncthreads();
+    for (int i = begin + lane; i < end; i += kWave) atomicAdd(&slots[block_of(indices[base + i])][wave], 1);
+    __syncthreads();
+    int32_t c[PER], mine = 0;
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+        c[i] = (&slots[0][0])[tid * PER + i];
+        mine += c[i];
+    }
+    int32_t incl = mine;
+#pragma unroll
+    for (int d = 1; d < kWave; d <<= 1) {
+        const int32_t up = __shfl_up(incl, d, kWave);
+        if (lane >= d) incl += up;
+    }
+    if (lane == kWave - 1) wave_total[wave] = incl;
+    __syncthreads();
+    int32_t run = incl - mine;
+    for (int w = 0; w < wave; ++w) run += wave_total[w];
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+        (&slots[0][0])[tid * PER + i] = run;
+        run += c[i];
+    }
+    __syncthreads();
+    for (int i0 = begin; i0 < end; i0 += kWave) {
+        const int i = i0 + lane;
+        const bool live = i < end;
+        const int64_t e = live ? indices[base + i] : -1;
+        const int b = block_of(e);
+        uint64_t same = __ballot(live);
+#pragma unroll
+        for (int bit = 0; bit < 8; ++bit) {
+            const uint64_t m = __ballot((b >> bit) & 1);
+            same &= ((b >> bit) & 1) ? m : ~m;
+        }
+        if (live) {
+            const int at = slots[b][wave] + __popcll(same & ((1ull << lane) - 1ull));
+            off32[base + at] = e >= 0 && e < num_experts ? (uint32_t)e * row_bytes : kBadOffset;
+            place[base + at] = (uint16_t)i;
+        }
+        __builtin_amdgcn_wave_barrier();                               // every lane has read its block's slot
+        if (live && (same >> lane) == 1ull) slots[b][wave] += __popcll(same);      // the block's last lane
+        __builtin_amdgcn_wave_barrier();
+    }
+}
+
+// NT tokens per wave, walked together: a step takes 64 / NT list positions of each (the same 16 gathers in flight as the slice
+// kernels), so that NT times as many tokens are at the same place of their lists.  256-byte slices.
+template <typename T, int NT>
+__global__ __launch_bounds__(256) void expert_scores_ordered_kernel(const T* __restrict__ x, const T* __restrict__ down, uint32_t table_bytes,
+                                                                    const uint32_t* __restrict__ off32, float* __restrict__ spart,
+                                                                    int64_t num_tokens, int hidden, int top_k, int num_slices,
+                                                                    int blocks_per_slice, int xcds) {
+    constexpr int V = Elem<T>::kVec, CL = 16, PPL = kWave / CL;
+    constexpr int QL = CL / NT, QP = QL * PPL;                   // loads and list positions per token and step
+    int slice, tb;
+    if (!slice_of_block(num_slices, blocks_per_slice, xcds, slice, tb)) return;
+    const int lane = lane_id(), wave = (int)(threadIdx.x >> 6);
+    const int c = lane & (CL - 1), pg = lane / CL;
+    const int col = slice * (CL * V) + c * V;
+    const bool col_ok = col < hidden;
+    const uint32_t col_bytes = col_ok ? (uint32_t)col * sizeof(T) : 0u;
+    const u32x4_t zero4 = {0u, 0u, 0u, 0u};
+    const __amdgpu_buffer_rsrc_t rsrc = table_resource(down, table_bytes);
+    const int64_t t0 = ((int64_t)tb * 4 + wave) * NT;
+    if (t0 >= num_tokens) return;                                // whole wave leaves; nobody waits on it
+    const int tokens = (int)(num_tokens - t0 < NT ? num_tokens - t0 : NT);
+    u32x4_t xq[NT];
+#pragma unroll
+    for (int n = 0; n < NT; ++n) xq[n] = col_ok && n < tokens ? *reinterpret_cast<const u32x4_t*>(x + (t0 + n) * hidden + col) : zero4;
+    const int my_token = lane / QP, my_at = lane % QP;           // the list position this lane fetches per step
+    const uint32_t* my_list = off32 + (t0 + my_token) * top_k;
+    float* out = spart + (int64_t)slice * num_tokens * top_k + t0 * top_k;
+    uint32_t mine = my_token < tokens && my_at < top_k ? my_list[my_at] : kBadOffset;
+    for (int k0 = 0; k0 < top_k; k0 += QP) {
+        u32x4_t w[CL];
+#pragma unroll
+        for (int u = 0; u < CL; ++u) {
+            const uint32_t o = (uint32_t)__builtin_amdgcn_ds_bpermute((u / QL * QP + (u % QL) * PPL + pg) * 4, (int)mine);
+            w[u] = load_row_piece(rsrc, o + col_bytes);
+        }
+        const int next = k0 + QP + my_at;
+        mine = my_token < tokens && next < top_k ? my_list[next] : kBadOffset;
+        float part[CL];
+#pragma unroll
+        for (int u = 0; u < CL; ++u) part[u] = dot16<T>(xq[u / QL], w[u], 0.0f);
+        const float total = transpose_sum<CL, 1>(part, c);          // load u = c: token c / QL, position (c % QL) * PPL + pg
+        const int kk = k0 + (c % QL) * PPL + pg;
+        if (c / QL < tokens && kk < top_k) out[(int64_t)(c / QL) * top_k + kk] = total;
+    }
+}
+
+template <typename T, int NT>
+__global__ __launch_bounds__(256) void expert_states_ordered_kernel(const float* __restrict__ a, const T* __restrict__ up, uint32_t table_bytes,
+                                                                    const uint32_t* __restrict__ off32, T* __restrict__ out,
+                                                                    int64_t num_tokens, int hidden, int top_k, int num_slices,
+                                                                    int blocks_per_slice, int xcds) {
+    constexpr int V = Elem<T>::kVec, CL = 16, PPL = kWave / CL;
+    constexpr int QL = CL / NT, QP = QL * PPL;
+    int slice, tb;
+    if (!slice_of_block(num_slices, blocks_per_slice, xcds, slice, tb)) return;
+    const int lane = lane_id(), wave = (int)(threadIdx.x >> 6);
+    const int c = lane & (CL - 1), pg = lane / CL;
+    const int col = slice * (CL * V) + c * V;
+    const bool col_ok = col < hidden;
+    const uint32_t col_bytes = col_ok ? (uint32_t)col * sizeof(T) : 0u;
+    const __amdgpu_buffer_rsrc_t rsrc = table_resource(up, table_bytes);
+    const int64_t t0 = ((int64_t)tb * 4 + wave) * NT;
+    if (t0 >= num_tokens) return;                                // whole wave leaves; nobody waits on it
+    const int tokens = (int)(num_tokens - t0 < NT ? num_tokens - t0 : NT);
+    float acc[NT][V];
+#pragma unroll
+    for (int n = 0; n < NT; ++n)
+#pragma unroll
+        for (int v = 0; v < V; ++v) acc[n][v] = 0.0f;
+    const int my_token = lane / QP, my_at = lane % QP;
+    const uint32_t* my_list = off32 + (t0 + my_token) * top_k;
+    const float* my_coef = a + (t0 + my_token) * top_k;
+    bool live = my_token < tokens && my_at < top_k;
+    uint32_t mine = live ? my_list[my_at] : kBadOffset;
+    float mine_a = live ? my_coef[my_at] : 0.0f;
+    for (int k0 = 0; k0 < top_k; k0 += QP) {
+        u32x4_t w[CL];
+        float av[CL];
+#pragma unroll
+        for (int u = 0; u < CL; ++u) {
+            const int src = (u / QL * QP + (u % QL) * PPL + pg) * 4;
+            const uint32_t o = (uint32_t)__builtin_amdgcn_ds_bpermute(src, (int)mine);
+            av[u] = __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(src, __builtin_bit_cast(int, mine_a)));
+            w[u] = load_row_piece(rsrc, o + col_bytes);          // zeros for an invalid id (out of bounds)
+        }
+        const int next = k0 + QP + my_at;
+        live = my_token < tokens && next < top_k;
+        mine = live ? my_list[next] : kBadOffset;
+        mine_a = live ? my_coef[next] : 0.0f;
+        // fp32 coefficients, as in the row kernel: the loads, not these instructions, set the pace
+#pragma unroll
+        for (int u = 0; u < CL; ++u) axpy16<T>(av[u], w[u], acc[u / QL]);
+    }
+#pragma unroll
+    for (int n = 0; n < NT; ++n) {
+#pragma unroll
+        for (int v = 0; v < V; ++v) {
+            acc[n][v] += __shfl_xor(acc[n][v], 16, kWave);
+            acc[n][v] += __shfl_xor(acc[n][v], 32, kWave);
+        }
+        if (pg == 0 && col_ok && n < tokens) *reinterpret_cast<u32x4_t*>(out + (t0 + n) * hidden + col) = pack16<T>(acc[n]);
+    }
+}
+
+int launch_expert_order(const int64_t* indices, uint32_t* off32, uint16_t* place, int64_t T_, int64_t E, int K, uint32_t row_bytes,
+                        hipStream_t stream) {
+    hipLaunchKernelGGL(expert_order_kernel, dim3((unsigned)T_), dim3(kOrderTokenWaves * kWave), 0, stream, indices, off32, place, E, K,
+                       order_shift(E), row_bytes);
+    FMOE_CHECK_LAUNCH("routed experts (ordered lists)");
+    return FMOE_OK;
+}
+
+// Tokens per wave: until all of them are resident at once (about 20 waves per CU), at most eight.
+int ordered_tokens_per_wave(int64_t T_) {
+    const int64_t resident = (int64_t)chip_info().cus / chip_info().xcds * 20;
+    int nt = 1;
+    while (nt < 8 && T_ > resident * nt) nt *= 2;
+    return nt;
+}
+#define FMOE_LAUNCH_ORDERED(KERNEL, ...)                                                                                      \
+    do {                                                                                                                      \
+        const int nt = ordered_tokens_per_wave(T_);                                                                           \
+        const int blocks = (int)((T_ + 4 * nt - 1) / (4 * nt));                                                               \
+        const dim3 grid((unsigned)(p.xcds * slice_grid_rows(p.num_slices, blocks, p.xcds)));                                  \
+        if (nt == 1) hipLaunchKernelGGL((KERNEL<T, 1>), grid, dim3(256), 0, stream, __VA_ARGS__, T_, H, K, p.num_slices, blocks, p.xcds); \
+        else if (nt == 2) hipLaunchKernelGGL((KERNEL<T, 2>), grid, dim3(256), 0, stream, __VA_ARGS__, T_, H, K, p.num_slices, blocks, p.xcds); \
+        else if (nt == 4) hipLaunchKernelGGL((KERNEL<T, 4>), grid, dim3(256), 0, stream, __VA_ARGS__, T_, H, K, p.num_slices, blocks, p.xcds); \
+        else hipLaunchKernelGGL((KERNEL<T, 8>), grid, dim3(256), 0, stream, __VA_ARGS__, T_, H, K, p.num_slices, blocks, p.xcds); \
+    } while (0)
+
+template <typename T>
+int launch_ordered_scores(const SlicePlan& p, const void* x, const void* table, const uint32_t* off32, float* spart, int64_t T_, int H,
+                          int64_t E, int K, hipStream_t stream) {
+    FMOE_LAUNCH_ORDERED(expert_scores_ordered_kernel, (const T*)x, (const T*)table, (uint32_t)(E * (int64_t)H * (int64_t)sizeof(T)), off32, spart);
+    FMOE_CHECK_LAUNCH("routed experts (ordered scores)");
+    return FMOE_OK;
+}
+template <typename T>
+int launch_ordered_states(const SlicePlan& p, const float* a, const void* table, const uint32_t* off32, void* out, int64_t T_, int H,
+                          int64_t E, int K, hipStream_t stream) {
+    FMOE_LAUNCH_ORDERED(expert_states_ordered_kernel, a, (const T*)table, (uint32_t)(E * (int64_t)H * (int64_t)sizeof(T)), off32, (T*)out);
+    FMOE_CHECK_LAUNCH("routed experts (ordered states)");
+    return FMOE_OK;
+}
+
+template <typename T>
+int launch_expert_ordered(int act, const void* x, const void* down, const void* up, const int64_t* indices, const void* gates,
+                          int64_t T_, int H, int64_t E, int K, void* out, void* workspace, const ExpertSaved* saved, hipStream_t stream) {
+    const SlicePlan p = plan_slices(T_, H, E, K, sizeof(T), true, act != kActNone);
+    char* ws = (char*)workspace;
+    uint32_t* off32 = saved ? saved->off32 : (uint32_t*)(ws + p.off_idx32);
+    uint16_t* place = saved ? saved->place : (uint16_t*)(ws + p.off_place);
+    float *a = (float*)(ws + p.off_a), *spart = (float*)(ws + p.off_spart);
+    if (int rc = launch_expert_order(indices, off32, place, T_, E, K, (uint32_t)(H * sizeof(T)), stream)) return rc;
+    if (act != kActNone)
+        if (int rc = launch_ordered_scores<T>(p, x, down, off32, spart, T_, H, E, K, stream)) return rc;
+    if (int rc = launch_expert_gate<T>(act, spart, gates, off32, place, a, saved ? saved->scores : nullptr, T_ * K, p.num_slices, K, stream)) return rc;
+    return launch_ordered_states<T>(p, a, up, off32, out, T_, H, E, K, stream);
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -1088,11 +1338,21 @@ bool slices_chosen(int64_t T_, int H, int64_t E, int K, size_t elt) {
 // Grouping the pairs by expert pays once an expert's row serves about a dozen pairs (measured: 16 pairs per expert, bucketed
 // 10-25 % ahead of whole-row gathers; 8 pairs per expert, 15 % behind): below that the rows are better gathered whole, straight
 // from HBM.
+// Ordered slices pay when the slices of the table do not stay in L2 and 400 tokens name every expert about once or more, so that a
+// window of the slice serves several of the gathers in flight.  Measured at H = 1024, E = 102400, bf16 (ordered against the better
+// of whole rows and buckets): 1024 tokens x 160 experts 104 against 96 us, x 512 227 against 290, x 1250 428 against 722;
+// 4096 x 512 655 against 907; 300 x 1000 160 against 243.
+bool ordered_possible(int64_t E, int H, int K, size_t elt) { return slices_possible(E, H, elt) && K <= kOrderMaxTopK; }
+bool ordered_pays(int64_t T_, int64_t E, int K) {
+    const int64_t resident = T_ < 400 ? T_ : 400;
+    return !slices_pay(T_, E, K) && T_ * K >= (1ll << 16) && resident * K >= E;
+}
 bool buckets_pay(int64_t T_, int64_t E, int K) { return !slices_pay(T_, E, K) && T_ * K >= (1ll << 16) && T_ * K >= 12 * E; }
 int choose_schedule(int algo, int64_t T_, int H, int64_t E, int K, size_t elt, bool scored = true) {
     if (K == 0) return FMOE_EXPERT_ROWS;
     if (algo != FMOE_EXPERT_AUTO) return algo;
     if (slices_chosen(T_, H, E, K, elt)) return FMOE_EXPERT_SLICES;
+    if (ordered_pays(T_, E, K) && ordered_possible(E, H, K, elt)) return FMOE_EXPERT_ORDERED;
     // grouping by expert serves the score phase; an op without scores (product-key memory) has nothing to group
     if (scored && buckets_pay(T_, E, K) && bucketed_possible(T_, E, H, K, elt)) return FMOE_EXPERT_BUCKETS;
     return FMOE_EXPERT_ROWS;
@@ -1106,19 +1366,43 @@ bool expert_slices_usable(int64_t num_tokens, int hidden, int64_t num_experts, i
 
 uint32_t* expert_workspace_offsets(void* workspace) { return (uint32_t*)workspace; }   // SlicePlan::off_idx32 == 0
 
+// What a forward in the slice or ordered schedule leaves for the backward (which takes the same schedule for these extents).
+ExpertSavedPlan expert_saved_plan(int64_t num_tokens, int hidden, int64_t num_experts, int top_k, int dtype) {
+    ExpertSavedPlan p = {};
+    if (num_tokens <= 0 || top_k <= 0) return p;
+    const int schedule = choose_schedule(FMOE_EXPERT_AUTO, num_tokens, hidden, num_experts, top_k, dtype_size(dtype));
+    p.kept = schedule == FMOE_EXPERT_SLICES || schedule == FMOE_EXPERT_ORDERED;
+    p.ordered = schedule == FMOE_EXPERT_ORDERED;
+    if (!p.kept) return p;
+    const size_t pairs = (size_t)num_tokens * top_k;
+    p.off_off32 = round_up(pairs * 4, 256);
+    p.off_place = round_up(p.off_off32 + pairs * 4, 256);
+    p.bytes = p.ordered ? round_up(p.off_place + pairs * 2, 256) : p.off_place;
+    return p;
+}
+ExpertSaved ExpertSavedPlan::at(const void* buffer) const {
+    char* b = (char*)const_cast<void*>(buffer);
+    return {(float*)b, (uint32_t*)(b + off_off32), (uint16_t*)(b + off_place)};
+}
+int expert_order(const int64_t* indices, uint32_t* off32, uint16_t* place, int64_t num_tokens, int hidden, int64_t num_experts, int top_k,
+                 int dtype, hipStream_t stream) {
+    return launch_expert_order(indices, off32, place, num_tokens, num_experts, top_k, (uint32_t)(hidden * dtype_size(dtype)), stream);
+}
+
 int expert_slices_prepared(const void* x, const void* down, const void* up, const void* gates, int64_t num_tokens,
                            int hidden, int64_t num_experts, int top_k, int dtype, void* out, void* workspace,
-                           hipStream_t stream) {
+                           const uint32_t* off32, float* scores, hipStream_t stream) {
+    const SlicePlan p = plan_slices(num_tokens, hidden, num_experts, top_k, dtype_size(dtype));
     switch (dtype) {
-        case FMOE_F32: return launch_expert_slices_prepared<float>(kActSilu, x, down, up, gates, num_tokens, hidden, num_experts, top_k, out, workspace, stream);
-        case FMOE_BF16: return launch_expert_slices_prepared<bf16_t>(kActSilu, x, down, up, gates, num_tokens, hidden, num_experts, top_k, out, workspace, stream);
-        default: return launch_expert_slices_prepared<f16_t>(kActSilu, x, down, up, gates, num_tokens, hidden, num_experts, top_k, out, workspace, stream);
+        case FMOE_F32: return launch_expert_slices_prepared<float>(p, kActSilu, x, down, up, gates, num_tokens, hidden, num_experts, top_k, out, workspace, off32, scores, stream);
+        case FMOE_BF16: return launch_expert_slices_prepared<bf16_t>(p, kActSilu, x, down, up, gates, num_tokens, hidden, num_experts, top_k, out, workspace, off32, scores, stream);
+        default: return launch_expert_slices_prepared<f16_t>(p, kActSilu, x, down, up, gates, num_tokens, hidden, num_experts, top_k, out, workspace, off32, scores, stream);
     }
 }
 
 // The stages of the column-slice schedule one by one, for the backward pass (fmoe_backward.hip).
-int expert_slice_count(int64_t num_tokens, int hidden, int64_t num_experts, int top_k, int dtype) {
-    return plan_slices(num_tokens, hidden, num_experts, top_k, dtype_size(dtype)).num_slices;
+int expert_slice_count(int64_t num_tokens, int hidden, int64_t num_experts, int top_k, int dtype, bool ordered) {
+    return plan_slices(num_tokens, hidden, num_experts, top_k, dtype_size(dtype), ordered).num_slices;
 }
 
 int expert_slice_prepare(const int64_t* indices, uint32_t* off32, int64_t pairs, int hidden, int64_t num_experts, int dtype,
@@ -1130,20 +1414,22 @@ int expert_slice_prepare(const int64_t* indices, uint32_t* off32, int64_t pairs,
 }
 
 int expert_slice_scores(const void* x, const void* table, const uint32_t* off32, float* spart, int64_t num_tokens, int hidden,
-                        int64_t num_experts, int top_k, int dtype, hipStream_t stream) {
+                        int64_t num_experts, int top_k, int dtype, bool ordered, hipStream_t stream) {
+    const SlicePlan p = plan_slices(num_tokens, hidden, num_experts, top_k, dtype_size(dtype), ordered);
     switch (dtype) {
-        case FMOE_F32: return launch_slice_scores<float>(x, table, off32, spart, num_tokens, hidden, num_experts, top_k, stream);
-        case FMOE_BF16: return launch_slice_scores<bf16_t>(x, table, off32, spart, num_tokens, hidden, num_experts, top_k, stream);
-        default: return launch_slice_scores<f16_t>(x, table, off32, spart, num_tokens, hidden, num_experts, top_k, stream);
+        case FMOE_F32: return (ordered ? launch_ordered_scores<float> : launch_slice_scores_prepared<float>)(p, x, table, off32, spart, num_tokens, hidden, num_experts, top_k, stream);
+        case FMOE_BF16: return (ordered ? launch_ordered_scores<bf16_t> : launch_slice_scores_prepared<bf16_t>)(p, x, table, off32, spart, num_tokens, hidden, num_experts, top_k, stream);
+        default: return (ordered ? launch_ordered_scores<f16_t> : launch_slice_scores_prepared<f16_t>)(p, x, table, off32, spart, num_tokens, hidden, num_experts, top_k, stream);
     }
 }
 
 int expert_slice_states(const float* coef, const void* table, const uint32_t* off32, void* out, int64_t num_tokens, int hidden,
-                        int64_t num_experts, int top_k, int dtype, hipStream_t stream) {
+                        int64_t num_experts, int top_k, int dtype, bool ordered, hipStream_t stream) {
+    const SlicePlan p = plan_slices(num_tokens, hidden, num_experts, top_k, dtype_size(dtype), ordered);
     switch (dtype) {
-        case FMOE_F32: return launch_slice_states<float>(coef, table, off32, out, num_tokens, hidden, num_experts, top_k, stream);
-        case FMOE_BF16: return launch_slice_states<bf16_t>(coef, table, off32, out, num_tokens, hidden, num_experts, top_k, stream);
-        default: return launch_slice_states<f16_t>(coef, table, off32, out, num_tokens, hidden, num_experts, top_k, stream);
+        case FMOE_F32: return (ordered ? launch_ordered_states<float> : launch_slice_states<float>)(p, coef, table, off32, out, num_tokens, hidden, num_experts, top_k, stream);
+        case FMOE_BF16: return (ordered ? launch_ordered_states<bf16_t> : launch_slice_states<bf16_t>)(p, coef, table, off32, out, num_tokens, hidden, num_experts, top_k, stream);
+        default: return (ordered ? launch_ordered_states<f16_t> : launch_slice_states<f16_t>)(p, coef, table, off32, out, num_tokens, hidden, num_experts, top_k, stream);
     }
 }
 
@@ -1157,6 +1443,7 @@ extern "C" size_t fmoe_expert_workspace_bytes_algo(int64_t num_tokens, int hidde
     switch (choose_schedule(algo, num_tokens, hidden, num_experts, top_k, elt)) {
         case FMOE_EXPERT_SLICES: return plan_slices(num_tokens, hidden, num_experts, top_k, elt).bytes;
         case FMOE_EXPERT_BUCKETS: return plan_bucketed(num_tokens, hidden, num_experts, top_k, elt).bytes;
+        case FMOE_EXPERT_ORDERED: return plan_slices(num_tokens, hidden, num_experts, top_k, elt, true).bytes;
         default: return 0;   // the row schedule needs no scratch
     }
 }
@@ -1169,9 +1456,11 @@ extern "C" size_t fmoe_pkm_workspace_bytes(int64_t num_tokens, int hidden, int64
     using namespace fmoe;
     if (num_tokens <= 0 || hidden <= 0 || num_experts <= 0 || top_k <= 0 || !dtype_ok(dtype)) return 0;
     const size_t elt = dtype_size(dtype);
-    return choose_schedule(FMOE_EXPERT_AUTO, num_tokens, hidden, num_experts, top_k, elt, false) == FMOE_EXPERT_SLICES
-               ? plan_slices(num_tokens, hidden, num_experts, top_k, elt).bytes
-               : 0;
+    switch (choose_schedule(FMOE_EXPERT_AUTO, num_tokens, hidden, num_experts, top_k, elt, false)) {
+        case FMOE_EXPERT_SLICES: return plan_slices(num_tokens, hidden, num_experts, top_k, elt).bytes;
+        case FMOE_EXPERT_ORDERED: return plan_slices(num_tokens, hidden, num_experts, top_k, elt, true, false).bytes;
+        default: return 0;
+    }
 }
 
 namespace fmoe {
@@ -1180,13 +1469,13 @@ namespace {
 // Shared body of the three gather ops; `who` names the entry point in messages, `down` is unused for kActNone.
 int expert_dispatch(const char* who, int act, const void* x, const void* down, const void* up, const int64_t* indices,
                     const void* gates, int64_t num_tokens, int hidden, int64_t num_experts, int top_k, int dtype, void* out,
-                    void* workspace, size_t workspace_bytes, int algo, void* stream) {
+                    void* workspace, size_t workspace_bytes, int algo, void* stream, const ExpertSaved* saved = nullptr) {
     clear_error();
     FMOE_REQUIRE(dtype_ok(dtype), FMOE_ERR_BAD_DTYPE, "%s: unknown dtype %d", who, dtype);
     FMOE_REQUIRE(num_tokens >= 0 && hidden > 0 && num_experts > 0 && top_k >= 0, FMOE_ERR_BAD_SHAPE,
                  "%s: bad shape T=%lld H=%d E=%lld K=%d", who, (long long)num_tokens, hidden,
                  (long long)num_experts, top_k);
-    FMOE_REQUIRE(algo >= FMOE_EXPERT_AUTO && algo <= FMOE_EXPERT_BUCKETS, FMOE_ERR_UNSUPPORTED,
+    FMOE_REQUIRE(algo >= FMOE_EXPERT_AUTO && algo <= FMOE_EXPERT_ORDERED, FMOE_ERR_UNSUPPORTED,
                  "%s: unknown algo %d", who, algo);
     if (num_tokens == 0) return FMOE_OK;
     FMOE_REQUIRE((x || act == kActNone) && (down || act == kActNone) && up && out, FMOE_ERR_NULL_POINTER, "%s: null tensor pointer", who);
@@ -1217,14 +1506,26 @@ int expert_dispatch(const char* who, int act, const void* x, const void* down, c
             default: return launch_expert_bucketed<f16_t>(act, x, down, up, indices, gates, num_tokens, hidden, num_experts, top_k, out, workspace, s);
         }
     }
+    FMOE_REQUIRE(schedule != FMOE_EXPERT_ORDERED || ordered_possible(num_experts, hidden, top_k, elt), FMOE_ERR_UNSUPPORTED,
+                 "%s: the ordered schedule needs tables below 4 GiB and at most %d experts per token", who, kOrderMaxTopK);
+    if (schedule == FMOE_EXPERT_ORDERED) {
+        const size_t need = plan_slices(num_tokens, hidden, num_experts, top_k, elt, true, act != kActNone).bytes;
+        FMOE_REQUIRE(workspace && workspace_bytes >= need && aligned16(workspace), FMOE_ERR_WORKSPACE,
+                     "%s: workspace of %zu bytes needed, %zu given", who, need, workspace_bytes);
+        switch (dtype) {
+            case FMOE_F32: return launch_expert_ordered<float>(act, x, down, up, indices, gates, num_tokens, hidden, num_experts, top_k, out, workspace, saved, s);
+            case FMOE_BF16: return launch_expert_ordered<bf16_t>(act, x, down, up, indices, gates, num_tokens, hidden, num_experts, top_k, out, workspace, saved, s);
+            default: return launch_expert_ordered<f16_t>(act, x, down, up, indices, gates, num_tokens, hidden, num_experts, top_k, out, workspace, saved, s);
+        }
+    }
     if (schedule == FMOE_EXPERT_SLICES) {
         const size_t need = fmoe_expert_workspace_bytes_algo(num_tokens, hidden, num_experts, top_k, dtype, FMOE_EXPERT_SLICES);
         FMOE_REQUIRE(workspace && workspace_bytes >= need && aligned16(workspace), FMOE_ERR_WORKSPACE,
                      "%s: workspace of %zu bytes needed, %zu given", who, need, workspace_bytes);
         switch (dtype) {
-            case FMOE_F32: return launch_expert_slices<float>(act, x, down, up, indices, gates, num_tokens, hidden, num_experts, top_k, out, workspace, s);
-            case FMOE_BF16: return launch_expert_slices<bf16_t>(act, x, down, up, indices, gates, num_tokens, hidden, num_experts, top_k, out, workspace, s);
-            default: return launch_expert_slices<f16_t>(act, x, down, up, indices, gates, num_tokens, hidden, num_experts, top_k, out, workspace, s);
+            case FMOE_F32: return launch_expert_slices<float>(act, x, down, up, indices, gates, num_tokens, hidden, num_experts, top_k, out, workspace, saved, s);
+            case FMOE_BF16: return launch_expert_slices<bf16_t>(act, x, down, up, indices, gates, num_tokens, hidden, num_experts, top_k, out, workspace, saved, s);
+            default: return launch_expert_slices<f16_t>(act, x, down, up, indices, gates, num_tokens, hidden, num_experts, top_k, out, workspace, saved, s);
         }
     }
     switch (dtype) {
@@ -1243,6 +1544,25 @@ extern "C" int fmoe_expert_forward_algo(const void* x, const void* down, const v
                                         int algo, void* stream) {
     return fmoe::expert_dispatch("fmoe_expert_forward", fmoe::kActSilu, x, down, up, indices, gates, num_tokens, hidden,
                                  num_experts, top_k, dtype, out, workspace, workspace_bytes, algo, stream);
+}
+
+extern "C" size_t fmoe_expert_saved_bytes(int64_t num_tokens, int hidden, int64_t num_experts, int top_k, int dtype) {
+    if (num_tokens <= 0 || hidden <= 0 || num_experts <= 0 || top_k <= 0 || !fmoe::dtype_ok(dtype)) return 0;
+    return fmoe::expert_saved_plan(num_tokens, hidden, num_experts, top_k, dtype).bytes;
+}
+
+extern "C" int fmoe_expert_forward_save(const void* x, const void* down, const void* up, const int64_t* indices, const void* gates,
+                                        int64_t num_tokens, int hidden, int64_t num_experts, int top_k, int dtype, void* out, void* saved,
+                                        size_t saved_bytes, void* workspace, size_t workspace_bytes, void* stream) {
+    using namespace fmoe;
+    clear_error();
+    const size_t need = fmoe_expert_saved_bytes(num_tokens, hidden, num_experts, top_k, dtype);
+    FMOE_REQUIRE(need == 0 || (saved && saved_bytes >= need && aligned16(saved)), FMOE_ERR_WORKSPACE,
+                 "fmoe_expert_forward_save: buffer of %zu bytes needed, %zu given", need, saved_bytes);
+    ExpertSaved kept = {};
+    if (need) kept = expert_saved_plan(num_tokens, hidden, num_experts, top_k, dtype).at(saved);
+    return expert_dispatch("fmoe_expert_forward_save", kActSilu, x, down, up, indices, gates, num_tokens, hidden, num_experts, top_k, dtype,
+                           out, workspace, workspace_bytes, FMOE_EXPERT_AUTO, stream, need ? &kept : nullptr);
 }
 
 extern "C" int fmoe_peer_forward(const void* x, const void* down, const void* up, const void* routing_weights,

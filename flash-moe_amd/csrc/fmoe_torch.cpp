@@ -216,7 +216,9 @@ std::tuple<Tensor, Tensor> router_prologue(const Tensor& tokens, const Tensor& g
 }
 
 // ---- routed experts, PEER, PKM -------------------------------------------------------------------------------------------
-Tensor expert_forward(const Tensor& hidden_states, const Tensor& down, const Tensor& up, const Tensor& indices, const Tensor& weights, int64_t algo) {
+// saved: where to put what a backward pass wants kept (undefined where the schedule keeps nothing), or NULL
+Tensor expert_forward_impl(const Tensor& hidden_states, const Tensor& down, const Tensor& up, const Tensor& indices, const Tensor& weights,
+                           int64_t algo, Tensor* saved) {
     TORCH_CHECK_VALUE(hidden_states.dim() == 2 && down.dim() == 2 && up.dim() == 2, "hidden_states, down_weights and up_weights must be 2-D");
     TORCH_CHECK_VALUE(indices.dim() == 2 && weights.sizes() == indices.sizes(), "indices and routing_weights must both be (num_tokens, num_experts_per_tok)");
     const int64_t T = hidden_states.size(0), H = hidden_states.size(1), E = down.size(0), K = indices.size(1);
@@ -233,13 +235,25 @@ Tensor expert_forward(const Tensor& hidden_states, const Tensor& down, const Ten
     Tensor out = at::empty_like(x);
     const size_t bytes = fmoe_expert_workspace_bytes_algo(T, (int)H, E, (int)K, code, (int)algo);
     Tensor ws = bytes ? workspace(x, bytes) : Tensor();
+    if (saved != nullptr) {
+        const size_t kept = fmoe_expert_saved_bytes(T, (int)H, E, (int)K, code);
+        if (kept) *saved = workspace(x, kept);
+        check(fmoe_expert_forward_save(ptr(x), ptr(wd), ptr(wu), (const int64_t*)ptr(idx), ptr(g), T, (int)H, E, (int)K, code, ptr(out),
+                                       ptr(*saved), kept, ptr(ws), bytes, call.stream), "flash_expert");
+        return out;
+    }
     check(fmoe_expert_forward_algo(ptr(x), ptr(wd), ptr(wu), (const int64_t*)ptr(idx), ptr(g), T, (int)H, E, (int)K, code, ptr(out),
                                    ptr(ws), bytes, (int)algo, call.stream), "flash_expert");
     return out;
 }
 
-std::tuple<Tensor, Tensor, Tensor, Tensor> expert_backward(const Tensor& dout, const Tensor& hidden_states, const Tensor& down,
-                                                           const Tensor& up, const Tensor& indices, const Tensor& weights) {
+Tensor expert_forward(const Tensor& hidden_states, const Tensor& down, const Tensor& up, const Tensor& indices, const Tensor& weights, int64_t algo) {
+    return expert_forward_impl(hidden_states, down, up, indices, weights, algo, nullptr);
+}
+
+std::tuple<Tensor, Tensor, Tensor, Tensor> expert_backward_impl(const Tensor& dout, const Tensor& hidden_states, const Tensor& down,
+                                                                const Tensor& up, const Tensor& indices, const Tensor& weights,
+                                                                const Tensor& saved) {
     require_gpu({&dout, &hidden_states, &down, &up, &indices, &weights});
     TORCH_CHECK_VALUE(dout.sizes() == hidden_states.sizes() && dout.scalar_type() == hidden_states.scalar_type(),
                       "the output gradient must have the shape and dtype of hidden_states");
@@ -250,19 +264,26 @@ std::tuple<Tensor, Tensor, Tensor, Tensor> expert_backward(const Tensor& dout, c
     Tensor dx = at::empty_like(x), dwd = at::empty_like(wd), dwu = at::empty_like(wu), dg = at::empty_like(g);
     const size_t bytes = fmoe_expert_backward_workspace_bytes(T, (int)H, E, (int)K, code);
     Tensor ws = workspace(x, bytes);
-    check(fmoe_expert_backward(ptr(d), ptr(x), ptr(wd), ptr(wu), (const int64_t*)ptr(idx), ptr(g), T, (int)H, E, (int)K, code, ptr(dx),
-                               ptr(dwd), ptr(dwu), ptr(dg), ptr(ws), bytes, call.stream), "flash_expert backward");
+    check(fmoe_expert_backward_saved(ptr(d), ptr(x), ptr(wd), ptr(wu), (const int64_t*)ptr(idx), ptr(g), ptr(saved), T, (int)H, E, (int)K,
+                                     code, ptr(dx), ptr(dwd), ptr(dwu), ptr(dg), ptr(ws), bytes, call.stream), "flash_expert backward");
     return {dx, dwd, dwu, dg};
+}
+
+std::tuple<Tensor, Tensor, Tensor, Tensor> expert_backward(const Tensor& dout, const Tensor& hidden_states, const Tensor& down,
+                                                           const Tensor& up, const Tensor& indices, const Tensor& weights) {
+    return expert_backward_impl(dout, hidden_states, down, up, indices, weights, Tensor());
 }
 
 struct ExpertNode : torch::autograd::Function<ExpertNode> {
     static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& down, const Tensor& up, const Tensor& indices, const Tensor& weights) {
-        ctx->save_for_backward({x, down, up, indices, weights});
-        return expert_forward(x, down, up, indices, weights, FMOE_EXPERT_AUTO);
+        Tensor saved;
+        Tensor out = expert_forward_impl(x, down, up, indices, weights, FMOE_EXPERT_AUTO, &saved);
+        ctx->save_for_backward({x, down, up, indices, weights, saved});
+        return out;
     }
     static variable_list backward(AutogradContext* ctx, variable_list grads) {
         const auto s = ctx->get_saved_variables();
-        auto [dx, dwd, dwu, dg] = expert_backward(grads[0], s[0], s[1], s[2], s[3], s[4]);
+        auto [dx, dwd, dwu, dg] = expert_backward_impl(grads[0], s[0], s[1], s[2], s[3], s[4], s[5]);
         return {dx, dwd, dwu, Tensor(), dg};
     }
 };

@@ -26,7 +26,7 @@ _DTYPE_CODE = {torch.float32: F32, torch.bfloat16: BF16, torch.float16: F16}
 
 ERR_TOPK_RANGE = -3
 
-EXPERT_AUTO, EXPERT_ROWS, EXPERT_SLICES, EXPERT_BUCKETS = 0, 1, 2, 3
+EXPERT_AUTO, EXPERT_ROWS, EXPERT_SLICES, EXPERT_BUCKETS, EXPERT_ORDERED = 0, 1, 2, 3, 4
 
 _vp, _i64, _int, _sz = ctypes.c_void_p, ctypes.c_int64, ctypes.c_int, ctypes.c_size_t
 
@@ -46,6 +46,8 @@ SIGNATURES = {
     "fmoe_expert_workspace_bytes_algo": (_sz, [_i64, _int, _i64, _int, _int, _int]),
     "fmoe_expert_forward": (_int, [_vp, _vp, _vp, _vp, _vp, _i64, _int, _i64, _int, _int, _vp, _vp, _sz, _vp]),
     "fmoe_expert_forward_algo": (_int, [_vp, _vp, _vp, _vp, _vp, _i64, _int, _i64, _int, _int, _vp, _vp, _sz, _int, _vp]),
+    "fmoe_expert_saved_bytes": (_sz, [_i64, _int, _i64, _int, _int]),
+    "fmoe_expert_forward_save": (_int, [_vp] * 5 + [_i64, _int, _i64, _int, _int, _vp, _vp, _sz, _vp, _sz, _vp]),
     "fmoe_expert_bucket_workspace_bytes": (_sz, [_i64]),
     "fmoe_expert_bucket": (_int, [_vp, _i64, _int, _i64, _vp, _vp, _vp, _vp, _vp, _sz, _vp]),
     "fmoe_mlp_workspace_bytes": (_sz, [_i64, _int, _int, _int]),
@@ -73,6 +75,7 @@ SIGNATURES = {
     "fmoe_mlp_backward_workspace_bytes": (_sz, [_i64, _int, _int, _int]),
     "fmoe_mlp_backward": (_int, [_vp] * 6 + [_i64, _int, _int, _int] + [_vp] * 5 + [_sz, _vp]),
     "fmoe_expert_backward_workspace_bytes": (_sz, [_i64, _int, _i64, _int, _int]),
+    "fmoe_expert_backward_saved": (_int, [_vp] * 7 + [_i64, _int, _i64, _int, _int] + [_vp] * 5 + [_sz, _vp]),
     "fmoe_expert_backward": (_int, [_vp] * 6 + [_i64, _int, _i64, _int, _int] + [_vp] * 5 + [_sz, _vp]),
 }
 

@@ -154,8 +154,10 @@ int fmoe_router_forward_noalloc(const void* x, const void* gate_w, void* running
  *   slices   each table below 4 GiB (rows are addressed with 32-bit byte offsets)
  *   buckets  rows a multiple of 128 bytes; x and each table below 4 GiB; T*K < 2^31 - 4096; T < 2^24 (its second
  *            phase sweeps the experts when the dtype is 16-bit, K <= 256 and E < 2^22; else it gathers whole rows)
+ *   ordered  tables below 4 GiB, K <= 65536
  * fmoe_expert_forward picks slices when E*128 bytes fit twice the L2 of one XCD and there are at least 65536 pairs, or
- * when the rows are too long for the row schedule; else buckets when there are at least 65536 pairs and 12 pairs per
+ * when the rows are too long for the row schedule; else ordered when there are at least 65536 pairs and min(T, 400) * K >= E
+ * (the tokens in flight then share the table's rows); else buckets when there are at least 65536 pairs and 12 pairs per
  * expert (each table row then serves enough pairs to pay for the grouping) and its limits hold; else rows.  So any
  * hidden size works as long as each table stays below 4 GiB.
  */
@@ -183,6 +185,15 @@ int fmoe_expert_bucket(const int64_t* indices, int64_t num_tokens, int top_k, in
                        int32_t* sorted_pair_ids, int32_t* sorted_token_ids, int32_t* sorted_expert_ids, void* workspace,
                        size_t workspace_bytes, void* stream);
 
+/* fmoe_expert_forward that also keeps what fmoe_expert_backward_saved would recompute: the scores and the addressing of every pair,
+ * in `saved` (fmoe_expert_saved_bytes() bytes, 256-byte aligned; 0 bytes, and `saved` may be NULL, where the schedule of these
+ * extents has nothing to keep). */
+size_t fmoe_expert_saved_bytes(int64_t num_tokens, int hidden, int64_t num_experts, int top_k, int dtype);
+
+int fmoe_expert_forward_save(const void* x, const void* down, const void* up, const int64_t* indices, const void* gates,
+                             int64_t num_tokens, int hidden, int64_t num_experts, int top_k, int dtype, void* out, void* saved,
+                             size_t saved_bytes, void* workspace, size_t workspace_bytes, void* stream);
+
 /* Same operation with the schedule chosen by the caller instead of by problem size (fmoe_expert_forward
  * passes FMOE_EXPERT_AUTO).  All schedules compute the formula above; they differ in how the table rows
  * travel: whole rows per (token, expert) pair; 128- or 256-byte column slices of the tables, each worked through by
@@ -193,6 +204,8 @@ typedef enum {
     FMOE_EXPERT_AUTO = 0,
     FMOE_EXPERT_ROWS = 1,     /* one wavefront per token, whole rows; no workspace needed */
     FMOE_EXPERT_SLICES = 2,   /* column slices of the tables resident in L2; needs the workspace */
+    FMOE_EXPERT_ORDERED = 4,  /* column slices of tables larger than the L2s, every token's list in expert order so that the
+                                 tokens in flight share a window of the slice; needs the workspace, top_k <= 65536 */
     FMOE_EXPERT_BUCKETS = 3   /* pairs grouped by expert (the fmoe_expert_bucket stage), column bands of x resident in
                                  L2, each down row streamed once; needs the workspace */
 } fmoe_expert_algo_t;
@@ -375,6 +388,12 @@ int fmoe_expert_backward(const void* dout, const void* x, const void* down, cons
                          const void* gates, int64_t num_tokens, int hidden, int64_t num_experts, int top_k, int dtype,
                          void* dx, void* ddown, void* dup, void* dgates, void* workspace, size_t workspace_bytes,
                          void* stream);
+
+/* The same from what fmoe_expert_forward_save kept for these inputs (NULL: nothing was kept, everything is recomputed). */
+int fmoe_expert_backward_saved(const void* dout, const void* x, const void* down, const void* up, const int64_t* indices,
+                               const void* gates, const void* saved, int64_t num_tokens, int hidden, int64_t num_experts, int top_k,
+                               int dtype, void* dx, void* ddown, void* dup, void* dgates, void* workspace, size_t workspace_bytes,
+                               void* stream);
 
 #ifdef __cplusplus
 }

@@ -289,3 +289,53 @@ def test_expert_on_router_produced_ids_at_the_block_size():
         assert rel_fro(out[sample], ref) < 4e-3, algo
         assert_output_close(out[sample], orc.expert_forward(x[sample], wd, wu, idx[sample], g[sample]), torch.bfloat16, algo)
     assert rel_fro(outs["slices"], outs["rows"]) < 5e-3 and rel_fro(outs["buckets"], outs["rows"]) < 5e-3
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("T,H,E,K", [
+    (3, 8, 4, 1), (37, 72, 50, 5),                     # fewer list positions than a step takes; one partial slice
+    (641, 136, 700, 33), (1281, 264, 300, 70),         # two and four tokens per wave, the last wave short of tokens
+    (2570, 64, 1000, 130),                             # eight tokens per wave
+    (70, 1000, 70000, 1100),                           # more positions than the ordering pass has lanes; the automatic choice
+])
+def test_expert_ordered_lists(dtype, T, H, E, K):
+    # every token's list walked in expert order: against the float64 oracle (a sample of the tokens) and whole rows, with ids
+    # outside the table, duplicates, and the same result twice
+    from flash_moe import _C
+    from flash_moe.ops.hip.flash_expert import expert_forward
+
+    g = torch.Generator().manual_seed(T + K)
+    x, wd, wu = (torch.randn(n, H, generator=g).mul(s).to(dtype) for n, s in ((T, 1.0), (E, 0.05), (E, 0.05)))
+    idx = torch.randint(0, E, (T, K), generator=g)
+    gates = torch.softmax(torch.randn(T, K, generator=g), -1).to(dtype)
+    idx[0, 0], idx[T - 1, K - 1] = -1, E
+    args = cuda(x, wd, wu, idx, gates)
+    got = expert_forward(*args, algo=_C.EXPERT_ORDERED)
+    assert torch.equal(got, expert_forward(*args, algo=_C.EXPERT_ORDERED))
+    tol = {torch.float32: 2e-6, torch.bfloat16: 5e-3, torch.float16: 6e-4}[dtype]
+    assert rel_fro(got, expert_forward(*args, algo=_C.EXPERT_ROWS)) < tol
+    sample = torch.arange(0, T, max(1, T // 40))
+    valid = (idx[sample] >= 0) & (idx[sample] < E)
+    ref = truth64(x[sample], wd, wu, idx[sample].clamp(0, E - 1), gates[sample] * valid)
+    assert rel_fro(got[sample.cuda()], ref) < tol
+
+
+@pytest.mark.parametrize("T,H,E,K", [(64, 128, 256, 8), (300, 264, 700, 230), (70, 64, 66000, 1000)])    # rows, slices, ordered lists
+def test_expert_backward_from_what_the_forward_kept(T, H, E, K):
+    # the op's autograd keeps scores and list addresses where its schedule has them; the stand-alone backward recomputes them
+    from flash_moe.ops import flash_expert_func
+    from flash_moe.ops.hip.flash_expert import expert_backward
+
+    g = torch.Generator().manual_seed(K)
+    x, wd, wu, dy = (torch.randn(n, H, generator=g).mul(s).cuda() for n, s in ((T, 1.0), (E, 0.1), (E, 0.1), (T, 1.0)))
+    idx = torch.randint(0, E, (T, K), generator=g).cuda()
+    gates = torch.softmax(torch.randn(T, K, generator=g), -1).cuda()
+    leaves = [t.clone().requires_grad_(True) for t in (x, wd, wu, gates)]
+    flash_expert_func(leaves[0], leaves[1], leaves[2], idx, leaves[3]).backward(dy)
+    alone = expert_backward(dy, x, wd, wu, idx, gates)
+    refs = [t.double().requires_grad_(True) for t in (x, wd, wu, gates)]
+    s = torch.stack([(refs[0][t] * refs[1][idx[t]]).sum(-1) for t in range(T)])
+    out = torch.stack([((torch.nn.functional.silu(s[t]) * refs[3][t])[:, None] * refs[2][idx[t]]).sum(0) for t in range(T)])
+    out.backward(dy.double())
+    for leaf, other, ref in zip(leaves, alone, refs):
+        assert rel_fro(leaf.grad, ref.grad) < 2e-5 and rel_fro(other, ref.grad) < 2e-5
