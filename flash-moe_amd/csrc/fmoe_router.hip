@@ -126,6 +126,19 @@ __device__ inline void bitonic_sort(uint64_t (&v)[RK], int lane) {
     bitonic_stages_from<RK, DESC, 2>(v, lane);
 }
 
+// One key per lane: every aligned block of N lanes sorted descending on its own (block size 0 in the last stage: all blocks alike).
+template <int N>
+__device__ inline void bitonic_sort_blocks(uint64_t& v, int lane) {
+    uint64_t a[1] = {v};
+    if constexpr (N >= 4) bitonic_stage<1, true, 2, 1>(a, lane);
+    if constexpr (N >= 8) bitonic_stage<1, true, 4, 2>(a, lane);
+    if constexpr (N >= 16) bitonic_stage<1, true, 8, 4>(a, lane);
+    if constexpr (N >= 32) bitonic_stage<1, true, 16, 8>(a, lane);
+    if constexpr (N >= 64) bitonic_stage<1, true, 32, 16>(a, lane);
+    bitonic_stage<1, true, 0, N / 2>(a, lane);
+    v = a[0];
+}
+
 // v holds a bitonic sequence of N keys; sort it descending.
 template <int RK>
 __device__ inline void bitonic_merge_desc(uint64_t (&v)[RK], int lane) {
@@ -281,13 +294,17 @@ __global__ __launch_bounds__(kRouterWaves* kWave) __attribute__((amdgpu_waves_pe
 // ------------------------------------------------------------------------------------------------------------
 // Selection by threshold (num_keys <= 64*RH, candidates <= 64*RC): the same result as the group scan above, for the
 // sizes where a whole list fits the wave's registers (R keys per lane).
-//   1. tau = K-th largest score of the list, found bit by bit from the top: the largest value with at least K scores
-//      >= it (per bit one compare per register, the counts come from the ballots on the scalar unit);
-//   2. the keys above tau, then keys equal to tau in list order until K are taken, go to K slots in LDS (positions from
-//      ballot prefix counts);
-//   3. one bitonic sort of the KP slots on the 64-bit keys.
-// List order is key index order for a half (position p = r*64 + lane), so ties at the cut go to the lowest index there;
-// among candidate sums tied at the cut the earlier candidate (lower rank in half 0) is taken.
+//   1. a score tau that at least K and at most CAP keys reach (CAP: the slots that are sorted), found bit by bit from the top (per
+//      bit one compare per register, the counts come from the ballots on the scalar unit): any such tau will do, so the search
+//      ends after 3 to 9 of the 32 bits, where the exact K-th largest score would take about 22;
+//   2. the keys at or above tau go to slots in LDS (positions from ballot prefix counts);
+//   3. one bitonic sort of the slots on the 64-bit keys; the first K are the result.
+// List order is key index order for a half (position p = r*64 + lane), so ties at the cut go to the lowest index there; among
+// candidate sums tied at the cut the earlier candidate (lower rank in half 0) is taken: where the sorted keys show such a tie, or
+// more than CAP keys tie with the K-th, the keys above that score and then the equal ones in list order are taken again.
+// Up to 32 experts per token (SMALL) CAP is 32 and one sort orders both halves, 32 lanes each.
+// Bound by instruction issue, 4 to 8 tokens per SIMD: at 32768 tokens, 128 keys, 16 experts the kernel took 92 us with the exact
+// search and three 64-lane sorts, now 36; 128 tokens or fewer, 32 experts: 10.3 -> 7.1; 4096 tokens, 64 experts: 16 -> 12.5.
 // ------------------------------------------------------------------------------------------------------------
 __device__ inline uint32_t wave_max_u32(uint32_t v) {
 #pragma unroll
@@ -297,13 +314,13 @@ __device__ inline uint32_t wave_max_u32(uint32_t v) {
     }
     return (uint32_t)__builtin_amdgcn_readfirstlane((int)v);
 }
-// RK = registers whose 64 * RK entries cover at least k: their smallest score bounds tau from below (k entries are at
+// RK = registers whose 64 * RK entries cover at least k: their smallest score bounds the K-th largest from below (k entries are at
 // least that large), the largest score of the list bounds it from above, and tau shares the leading bits the two bounds
-// share - the search starts below them (log-probabilities of one token typically share the sign, the exponent and a
-// few mantissa bits: about 22 of the 32 steps remain).  A padding entry (key 0) among those registers just gives the
-// bound 0.
-template <int R, int RK>
-__device__ inline uint32_t kth_largest_score(const uint64_t (&key)[R], int k) {
+// share - the search starts below them.  A padding entry (key 0) among those registers just gives the bound 0.
+// Ends at the first tau that at most `cap` keys reach, or at the exact K-th largest score.  LOW: low bits that every score of the
+// list shares with its sign (those a 16-bit type does not have); ties are common there and would run the search through them.
+template <int R, int RK, int LOW>
+__device__ inline uint32_t selecting_score(const uint64_t (&key)[R], int k, int cap) {
     uint32_t hi = 0u, lo_inv = 0u;
 #pragma unroll
     for (int r = 0; r < R; ++r) {
@@ -315,13 +332,17 @@ __device__ inline uint32_t kth_largest_score(const uint64_t (&key)[R], int k) {
     const uint32_t lo = ~wave_max_u32(lo_inv);
     const int bits = 32 - __builtin_clz((hi ^ lo) | 1u);         // low bits in which the bounds may differ
     uint32_t tau = bits >= 32 ? 0u : (hi >> bits) << bits;
-    for (int bit = bits - 1; bit >= 0; --bit) {
+    for (int bit = bits - 1; bit >= LOW; --bit) {
         const uint32_t trial = tau | (1u << bit);
         int count = 0;
 #pragma unroll
         for (int r = 0; r < R; ++r)
             count += __builtin_popcountll(__builtin_amdgcn_ballot_w64((uint32_t)(key[r] >> 32) >= trial));
         tau = count >= k ? trial : tau;
+        if (count >= k && count <= cap) break;
+    }
+    if constexpr (LOW > 0) {                                     // make tau a score: the low bits of a negative one are ones
+        if (!(tau >> 31)) tau |= (1u << LOW) - 1u;
     }
     return tau;
 }
@@ -330,11 +351,9 @@ __device__ inline int lanes_below(uint64_t mask) {
     return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
 }
 
-// slots: KP wave-private LDS entries.  Unused list entries hold key 0 (below every score).
-template <int R, int RK>
-__device__ inline void select_topk_sorted(const uint64_t (&key)[R], int k, uint64_t* slots, uint64_t (&best)[RK], int lane) {
-    constexpr int KP = RK * kWave;
-    const uint32_t tau = kth_largest_score<R, RK>(key, k);
+// The keys above tau, then those equal to it in list order, until k are taken.
+template <int R>
+__device__ inline void collect_exactly(const uint64_t (&key)[R], uint32_t tau, int k, int cap, uint64_t* slots, int lane) {
     int base = 0;
 #pragma unroll
     for (int r = 0; r < R; ++r) {
@@ -351,12 +370,42 @@ __device__ inline void select_topk_sorted(const uint64_t (&key)[R], int k, uint6
         if (equal && pos < k) slots[pos] = key[r];
         base += __builtin_popcountll(m);
     }
-    for (int p = k + lane; p < KP; p += kWave) slots[p] = 0ull;
+    for (int p = k + lane; p < cap; p += kWave) slots[p] = 0ull;
+}
+
+// At least k of the list's keys, all that reach a common score (or exactly k of them), into slots[0 .. cap), the rest of them 0;
+// cap wave-private LDS entries.  n: keys in the list; unused entries hold key 0 (below every score).
+template <int R, int RK, int LOW>
+__device__ inline void collect_top(const uint64_t (&key)[R], int n, int k, int cap, uint64_t* slots, int lane) {
+    const uint32_t tau = n <= cap ? 1u : selecting_score<R, RK, LOW>(key, k, cap);
+    uint64_t m[R];
+    int total = 0;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        m[r] = __builtin_amdgcn_ballot_w64((uint32_t)(key[r] >> 32) >= tau);
+        total += __builtin_popcountll(m[r]);
+    }
+    if (total > cap) {                    // more ties with the k-th score than there are slots
+        collect_exactly<R>(key, tau, k, cap, slots, lane);
+        return;
+    }
+    int base = 0;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        if ((m[r] >> lane) & 1) slots[base + lanes_below(m[r])] = key[r];
+        base += __builtin_popcountll(m[r]);
+    }
+    for (int p = base + lane; p < cap; p += kWave) slots[p] = 0ull;
+}
+
+template <int RK, bool SMALL>
+__device__ inline void sort_slots(const uint64_t* slots, uint64_t (&best)[RK], int lane) {
     __builtin_amdgcn_wave_barrier();      // LDS operations of one wave complete in order; keep the compiler from moving them
 #pragma unroll
     for (int r = 0; r < RK; ++r) best[r] = slots[lane * RK + r];
     __builtin_amdgcn_wave_barrier();
-    bitonic_sort<RK, true>(best, lane);
+    if constexpr (SMALL) bitonic_sort_blocks<32>(best[0], lane);
+    else bitonic_sort<RK, true>(best, lane);
 }
 
 // The candidate pairs (rank in half 0) | (rank in half 1) << 8, listed by rank in half 0: the list depends on top_k only,
@@ -367,13 +416,16 @@ struct CandidateTable { uint16_t pair[kSelectMaxCand]; };
 // OCC: waves per SIMD the register allocation must leave room for.  With more than four tokens per SIMD eight resident
 // waves (at most 64 registers, a few of them spilled for the larger lists) finish sooner than seven, whose eighth token
 // per SIMD would wait for a second round; with at most four tokens per SIMD the unconstrained allocation is faster.
-template <typename T, typename TG, int RK, int RH, int RC, bool FROM_LOGITS, int OCC>
+template <typename T, typename TG, int RK, int RH, int RC, bool FROM_LOGITS, int OCC, bool SMALL = false>
 __global__ __launch_bounds__(kRouterWaves* kWave, OCC) void router_select_kernel(
     const T* __restrict__ lp, int64_t num_tokens, int nk, int top_k, int num_cand, T* __restrict__ scores,
     int64_t* __restrict__ indices, TG* __restrict__ gates, int norm_topk_prob, uint32_t* __restrict__ row_offsets,
     uint32_t row_bytes, const CandidateTable table) {
     constexpr int KP = RK * kWave;
+    constexpr int LOW = sizeof(T) == 4 ? 0 : __is_same(T, bf16_t) ? 16 : 13;      // fp32 bits below the type's mantissa
+    constexpr int CAP = SMALL ? kWave / 2 : KP;
     static_assert(RC * kWave <= kSelectMaxCand, "candidate table");
+    static_assert(!SMALL || RK == 1, "one key per lane");
     __shared__ uint16_t cand[RC * kWave];
     __shared__ float half_score[kRouterWaves][2][KP];
     __shared__ uint32_t half_index[kRouterWaves][2][KP];
@@ -418,13 +470,17 @@ __global__ __launch_bounds__(kRouterWaves* kWave, OCC) void router_select_kernel
                 const int p = r * kWave + lane;
                 key[r] = p < nk ? make_key(FROM_LOGITS ? (v[r] - shift) - lse : v[r], (uint32_t)p) : 0ull;
             }
-            uint64_t best[RK];
-            // every rank up to KP is looked up by the candidates (entries past nk stay key 0)
-            select_topk_sorted<RH, RK>(key, nk < KP ? nk : KP, slot[wave], best, lane);
+            // the candidates look up ranks below top_k (entries past nk stay key 0)
+            collect_top<RH, RK, FROM_LOGITS ? 0 : LOW>(key, nk, top_k < nk ? top_k : nk, CAP, slot[wave] + (SMALL ? h * CAP : 0), lane);
+            if (!SMALL || h == 1) {
+                uint64_t best[RK];
+                sort_slots<RK, SMALL>(slot[wave], best, lane);
 #pragma unroll
-            for (int r = 0; r < RK; ++r) {
-                half_score[wave][h][lane * RK + r] = key_score(best[r]);
-                half_index[wave][h][lane * RK + r] = key_index(best[r]);
+                for (int r = 0; r < RK; ++r) {
+                    const int which = SMALL ? lane / CAP : h, rank = SMALL ? lane % CAP : lane * RK + r;
+                    half_score[wave][which][rank] = key_score(best[r]);
+                    half_index[wave][which][rank] = key_index(best[r]);
+                }
             }
         }
         __builtin_amdgcn_wave_barrier();
@@ -442,7 +498,17 @@ __global__ __launch_bounds__(kRouterWaves* kWave, OCC) void router_select_kernel
             }
         }
         uint64_t best[RK];
-        select_topk_sorted<RC, RK>(ckey, top_k, slot[wave], best, lane);
+        if (SMALL && lane >= CAP) slot[wave][lane] = 0ull;                 // the sort's other block
+        collect_top<RC, RK, LOW>(ckey, num_cand, top_k, CAP, slot[wave], lane);
+        sort_slots<RK, SMALL>(slot[wave], best, lane);
+        {
+            // a tie across the cut: the first candidates in list order among the equal sums are the ones to keep
+            const uint32_t cut = (uint32_t)(key_at<RK>(best, top_k - 1) >> 32);
+            if (top_k < CAP && cut == (uint32_t)(key_at<RK>(best, top_k) >> 32)) {
+                collect_exactly<RC>(ckey, cut, top_k, CAP, slot[wave], lane);
+                sort_slots<RK, SMALL>(slot[wave], best, lane);
+            }
+        }
         float e[RK];
         float total = 0.0f;
 #pragma unroll
@@ -758,36 +824,41 @@ int launch_router(const void* lp, int64_t T_, int nk, int K, void* scores, int64
     }
     // lists that fit the registers of a wave take the threshold selection
     const bool crowded = T_ > (int64_t)chip_info().cus * 4 * kRouterWaves;      // more than four tokens per SIMD
-#define FMOE_LAUNCH_SELECT(RK_, RH_, RC_)                                                                                    \
-    do {                                                                                                                     \
-        if (crowded)                                                                                                         \
-            hipLaunchKernelGGL((router_select_kernel<T, TG, RK_, RH_, RC_, FROM_LOGITS, 8>), grid, block, 0, stream,         \
-                               (const T*)lp, T_, nk, K, num_cand, (T*)scores, indices, (TG*)gates, norm, row_offsets,        \
-                               row_bytes, table);                                                                            \
-        else                                                                                                                 \
-            hipLaunchKernelGGL((router_select_kernel<T, TG, RK_, RH_, RC_, FROM_LOGITS, 1>), grid, block, 0, stream,         \
-                               (const T*)lp, T_, nk, K, num_cand, (T*)scores, indices, (TG*)gates, norm, row_offsets,        \
-                               row_bytes, table);                                                                            \
+#define FMOE_LAUNCH_SELECT_OCC(RK_, RH_, RC_, OCC_, SMALL_)                                                                   \
+    hipLaunchKernelGGL((router_select_kernel<T, TG, RK_, RH_, RC_, FROM_LOGITS, OCC_, SMALL_>), grid, block, 0, stream, (const T*)lp, \
+                       T_, nk, K, num_cand, (T*)scores, indices, (TG*)gates, norm, row_offsets, row_bytes, table)
+// Many tokens: one key per lane lets the kernel run in the registers of eight waves per SIMD at no or little spilling (K = 16, nk =
+// 128, 32768 tokens: 36 us against 40 at five waves); the instances of two keys per lane would spill 25 to 59 registers (nk = 512,
+// K = 128: 165 us against 138 without the bound).  Few tokens are one latency chain, spills would lengthen it.
+#define FMOE_LAUNCH_SELECT(RK_, RH_, RC_, SMALL_)                              \
+    do {                                                                       \
+        if (crowded && RK_ == 1) FMOE_LAUNCH_SELECT_OCC(1, RH_, RC_, 8, SMALL_); \
+        else FMOE_LAUNCH_SELECT_OCC(RK_, RH_, RC_, 1, SMALL_);                 \
     } while (0)
-    CandidateTable table;
     if (K <= 128 && nk <= 512) {
+        CandidateTable table;
         int c = 0;
         for (int i = 0; i < K; ++i)
             for (int j = 0; j < K / (i + 1); ++j) table.pair[c++] = (uint16_t)(i | (j << 8));
         for (; c < kSelectMaxCand; ++c) table.pair[c] = 0;
-    }
-    if (K <= 64 && nk <= 512) {
-        if (nk <= 128) FMOE_LAUNCH_SELECT(1, 2, 5);
-        else FMOE_LAUNCH_SELECT(1, 8, 5);
+        if (K <= 32 && num_cand <= kWave) {          // up to 19 experts: the candidates are one key per lane
+            if (nk <= 128) FMOE_LAUNCH_SELECT(1, 2, 1, true);
+            else FMOE_LAUNCH_SELECT(1, 8, 1, true);
+        } else if (K <= 32) {
+            if (nk <= 128) FMOE_LAUNCH_SELECT(1, 2, 2, true);
+            else FMOE_LAUNCH_SELECT(1, 8, 2, true);
+        } else if (K <= 64) {
+            if (nk <= 128) FMOE_LAUNCH_SELECT(1, 2, 5, false);
+            else if (nk <= 256) FMOE_LAUNCH_SELECT(1, 4, 5, false);
+            else FMOE_LAUNCH_SELECT(1, 8, 5, false);
+        } else {
+            if (nk <= 128) FMOE_LAUNCH_SELECT(2, 2, 11, false);
+            else FMOE_LAUNCH_SELECT(2, 8, 11, false);
+        }
         FMOE_CHECK_LAUNCH("fmoe_router_topk");
         return FMOE_OK;
     }
-    if (K <= 128 && nk <= 512) {
-        if (nk <= 128) FMOE_LAUNCH_SELECT(2, 2, 11);
-        else FMOE_LAUNCH_SELECT(2, 8, 11);
-        FMOE_CHECK_LAUNCH("fmoe_router_topk");
-        return FMOE_OK;
-    }
+#undef FMOE_LAUNCH_SELECT_OCC
 #undef FMOE_LAUNCH_SELECT
 #define FMOE_LAUNCH_ROUTER(R)                                                                                      \
     hipLaunchKernelGGL((router_topk_kernel<T, TG, R, FROM_LOGITS>), grid, block, 0, stream, (const T*)lp, T_, nk, K, \

@@ -93,6 +93,35 @@ def test_router_matches_exhaustive_scan_with_lowest_index_ties():
         assert want <= set(i[t].tolist())
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("T,nk,K", [
+    # a choice of the selection each side of its edges: 19 | 20 and 32 | 33 experts, 128 | 129 and 256 | 257 keys, lists that fill
+    # their slots exactly, and enough tokens for the eight-wave instances
+    (60, 19, 19), (60, 128, 20), (4200, 128, 16), (60, 129, 32), (60, 32, 32), (60, 33, 33), (60, 256, 64), (4200, 257, 64), (60, 130, 65),
+])
+@pytest.mark.parametrize("step", [0.0, 0.25, 8.0])
+def test_router_selection_is_exact_with_ties(dtype, T, nk, K, step):
+    # rounded scores tie within and across the cut, down to lists of two distinct values; the choice among equals is fixed:
+    # lowest key in a half, lowest rank of half 0 among the sums, and the result by descending score, then ascending index
+    from flash_moe.ops import flash_router_func
+
+    lp = orc.make_router_inputs(T, nk, seed=T + nk + K)
+    lp = ((lp / step).round() * step if step else lp).to(dtype)
+    s, i = flash_router_func(cuda(lp), nk, K)
+    s, i = s.cpu(), i.cpu()
+    top, ids = lp.float().sort(dim=-1, descending=True, stable=True)
+    pairs = [(a, b) for a in range(K) for b in range(K // (a + 1))]
+    a, b = torch.tensor([p[0] for p in pairs]), torch.tensor([p[1] for p in pairs])
+    sums = (top[0][:, a] + top[1][:, b]).to(dtype).float()
+    flat = ids[0][:, a] * nk + ids[1][:, b]
+    kept = sums.sort(dim=-1, descending=True, stable=True)[1][:, :K]
+    sums, flat = sums.gather(-1, kept), flat.gather(-1, kept)
+    order = flat.sort(-1)[1]
+    order = order.gather(-1, sums.gather(-1, order).sort(dim=-1, descending=True, stable=True)[1])
+    assert torch.equal(s, sums.gather(-1, order).to(dtype))
+    assert torch.equal(i, flat.gather(-1, order))
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_router_16bit_scores(dtype):
     # sums are rounded to the input dtype as the reference adds in the input dtype (flash_router.py:51-53)
