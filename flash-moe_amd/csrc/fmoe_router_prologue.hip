@@ -3,20 +3,21 @@
 //   logits = q Wr^T     [T, 2*nk]
 //   log-softmax per half, top-k over the pair sums, exp / renormalise   (router_topk_kernel, logits-input mode)
 //
-// Launches, 16-bit activations (three in training mode, two in evaluation mode):
+// Launches (three in training mode, two in evaluation mode):
 //   bn_block_stats_kernel  per (row block, 128-byte column strip): shifted sums -> (mean, M2) of the block   [training]
-//   router_gate_kernel     MFMA GEMM.  Its prologue combines the (at most 16) row blocks per column (Chan's parallel
-//                          formula) into mean and 1/sqrt(var+eps) - or takes the running statistics - for the columns
-//                          it multiplies, and a few workgroups also store them and update the running statistics
-//                          (momentum, unbiased variance) and the batch counter.  The A tile is normalised while it is
-//                          staged: (x - mean) * rstd is rounded to the activation dtype exactly as a stand-alone
-//                          batch-norm would emit it, then multiplied with the gate weights with fp32 accumulation;
-//                          writes the logits in fp32 (for the routing) and in the activation dtype (the tensor the
-//                          module returns).  With at most one tile per compute unit (4096 tokens) a workgroup is 16
-//                          waves: four groups that each take every fourth k-tile and add their accumulators at the end
-//   router_topk_kernel     (fmoe_router.hip)
-// fp32 activations (a parity configuration, not tuned): bn_partial_kernel per (row block, 512-column strip),
-// bn_finalize_kernel per column, router_gate_f32_kernel, router_topk_kernel.
+//   router_gate_splitk_kernel   few tiles and fp32: MFMA product, the waves of a workgroup split k; or
+//   router_gate_kernel     MFMA product on 64 x 64 tiles, operands shared through LDS.  With at most one tile per compute unit (4096
+//                          tokens) a workgroup is 16 waves: four groups that each take every fourth k-tile and add their
+//                          accumulators at the end.
+//                          Either combines the (at most 16) row blocks per column (Chan's parallel formula) into mean and
+//                          1/sqrt(var+eps) - or takes the running statistics - for the columns it multiplies, and a few workgroups
+//                          also store them and update the running statistics (momentum, unbiased variance) and the batch counter.
+//                          (x - mean) * rstd is rounded to the activation dtype exactly as a stand-alone batch-norm would emit
+//                          it, then multiplied with the gate weights with fp32 accumulation; writes the logits in fp32 (for the
+//                          routing) and in the activation dtype (the tensor the module returns).
+//   router_select_kernel   (fmoe_router.hip)
+// With many tiles the statistics are combined once instead: bn_partial_kernel per (row block, column strip), bn_finalize_kernel per
+// column.
 #include <math.h>
 
 #include <mutex>
@@ -359,6 +360,96 @@ template <> __device__ inline u32x4_t normalise16<f16_t>(u32x4_t raw, const floa
     return out;
 }
 
+template <> __device__ inline u32x4_t normalise16<float>(u32x4_t raw, const float* mean, const float* rstd) {
+    u32x4_t out;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const uint32_t r = raw[i];
+        out[i] = __float_as_uint((__uint_as_float(r) - mean[i]) * rstd[i]);
+    }
+    return out;
+}
+
+// mean and 1/std of columns [k_off, k_off + K) into LDS (zeros up to kpad), by all threads of a workgroup.  keeper: the one column of
+// tiles per k range that also stores them (for a backward pass) and updates the running statistics: its tile row (i / 64) mod
+// tiles_m takes column i, so every column is written by exactly one workgroup.  CPT columns per thread and round: all their
+// block statistics are loaded together, one memory round trip per round.
+template <int CPT>
+__device__ inline void stage_stats(const GateStats& st, float* stats, int kpad, int K, int K_full, int k_off, bool keeper, int tm, int tiles_m) {
+    const int threads = (int)blockDim.x, tid = (int)threadIdx.x;
+    if (blockIdx.x == 0 && tid == 0 && st.training && !st.ready && st.num_batches_tracked != nullptr) *st.num_batches_tracked += 1;
+    const float n = (float)st.num_tokens;
+    const float full = (float)st.rows_per_block;
+    const float last = (float)(st.num_tokens - (int64_t)(st.row_blocks - 1) * st.rows_per_block);
+    for (int i0 = tid; st.ready && i0 < kpad; i0 += threads) {
+        stats[i0] = i0 < K ? st.mean_rstd[k_off + i0] : 0.0f;
+        stats[kpad + i0] = i0 < K ? st.mean_rstd[K_full + k_off + i0] : 0.0f;
+    }
+    for (int i0 = tid; !st.ready && i0 < kpad; i0 += threads * CPT) {
+        float mean[CPT], var[CPT], m2[CPT];
+        if (st.training) {
+            float mb[CPT][kFoldMaxRowBlocks], m2b[CPT][kFoldMaxRowBlocks];
+#pragma unroll
+            for (int u = 0; u < CPT; ++u) {
+                const int i = i0 + u * threads;
+                const float* pc = st.partial + k_off + (i < K ? i : 0);
+#pragma unroll
+                for (int b = 0; b < kFoldMaxRowBlocks; ++b) {
+                    const bool ok = b < st.row_blocks;
+                    mb[u][b] = ok ? pc[(int64_t)b * 2 * K_full] : 0.0f;
+                    m2b[u][b] = ok ? pc[(int64_t)b * 2 * K_full + K_full] : 0.0f;
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < CPT; ++u) {
+                float snm = 0.0f;
+#pragma unroll
+                for (int b = 0; b < kFoldMaxRowBlocks; ++b) {
+                    const float nb = b + 1 < st.row_blocks ? full : (b + 1 == st.row_blocks ? last : 0.0f);
+                    snm = __builtin_fmaf(nb, mb[u][b], snm);
+                }
+                mean[u] = snm / n;
+                float acc2 = 0.0f;
+#pragma unroll
+                for (int b = 0; b < kFoldMaxRowBlocks; ++b) {
+                    const float nb = b + 1 < st.row_blocks ? full : (b + 1 == st.row_blocks ? last : 0.0f);
+                    const float d = mb[u][b] - mean[u];
+                    acc2 += __builtin_fmaf(nb * d, d, m2b[u][b]);
+                }
+                m2[u] = acc2;
+                var[u] = acc2 / n;                              // biased: what normalises the batch
+            }
+        } else {
+#pragma unroll
+            for (int u = 0; u < CPT; ++u) {
+                const int i = i0 + u * threads;
+                const int c = k_off + (i < K ? i : 0);
+                mean[u] = load_stat_rt(st.running_mean, c, st.stats_dtype);
+                var[u] = load_stat_rt(st.running_var, c, st.stats_dtype);
+                m2[u] = 0.0f;
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < CPT; ++u) {
+            const int i = i0 + u * threads;
+            if (i >= kpad) continue;
+            const int c = k_off + i;
+            const float rstd = 1.0f / sqrtf(var[u] + st.eps);
+            if (i < K && keeper && tm == (i / 64) % tiles_m) {
+                if (st.training && st.running_mean != nullptr && st.running_var != nullptr) {
+                    const float unbiased = n > 1.0f ? m2[u] / (n - 1.0f) : var[u];
+                    store_stat_rt(st.running_mean, c, (1.0f - st.momentum) * load_stat_rt(st.running_mean, c, st.stats_dtype) + st.momentum * mean[u], st.stats_dtype);
+                    store_stat_rt(st.running_var, c, (1.0f - st.momentum) * load_stat_rt(st.running_var, c, st.stats_dtype) + st.momentum * unbiased, st.stats_dtype);
+                }
+                st.mean_rstd[c] = mean[u];
+                st.mean_rstd[K_full + c] = rstd;
+            }
+            stats[i] = i < K ? mean[u] : 0.0f;
+            stats[kpad + i] = i < K ? rstd : 0.0f;
+        }
+    }
+}
+
 // logits[M, N] = normalise(x)[M, K] * W[N, K]^T for 16-bit activations: 64x64 tiles (256 of them at T=4096, 2*nk=256),
 // 4 waves of one 32x32 MFMA tile each, register-staged LDS tiles (the A tile is normalised between the global load and
 // the LDS store).  With one such workgroup per CU nothing else hides the global-load latency, so the packets of the
@@ -379,7 +470,6 @@ __global__ __launch_bounds__(256 * KG) __attribute__((amdgpu_waves_per_eu(4, 4))
     using Frag = typename Mfma32<T>::Frag;
     constexpr int BM = 64, BN = 64, CH = 2;   // CH = 16-byte packets per thread per tile and operand
     constexpr int D = KG > 1 ? 4 : kGatePrefetch;
-    constexpr int THREADS = 256 * KG;
     __shared__ __attribute__((aligned(16))) T tiles[KG][2][BM * kTileK];
     extern __shared__ __attribute__((aligned(16))) float stats[];   // [2][Kpad]: mean, rstd
     int tm, tn;
@@ -440,85 +530,7 @@ __global__ __launch_bounds__(256 * KG) __attribute__((amdgpu_waves_per_eu(4, 4))
 #pragma unroll
         for (int d = 0; d < 2; ++d) load_global(d, d);
     }
-    // mean and 1/std of this tile's k range into LDS.  One column of tiles per k range also stores them (for a backward
-    // pass) and updates the running statistics: tile row (i / 64) mod tiles_m takes column i, so every column is written
-    // by exactly one workgroup.  CPT columns per thread and round: all their block statistics are loaded together (one
-    // memory round trip per round), before the operand prefetch below claims its registers.
-    {
-        constexpr int CPT = KG > 1 ? 1 : 2;
-        const bool keeper = tn == (k_off ? tiles_n / 2 : 0);
-        if (blockIdx.x == 0 && tid_all == 0 && st.training && !st.ready && st.num_batches_tracked != nullptr) *st.num_batches_tracked += 1;
-        const float n = (float)st.num_tokens;
-        const float full = (float)st.rows_per_block;
-        const float last = (float)(st.num_tokens - (int64_t)(st.row_blocks - 1) * st.rows_per_block);
-        for (int i0 = tid_all; st.ready && i0 < kpad; i0 += THREADS) {
-            stats[i0] = i0 < K ? st.mean_rstd[k_off + i0] : 0.0f;
-            stats[kpad + i0] = i0 < K ? st.mean_rstd[K_full + k_off + i0] : 0.0f;
-        }
-        for (int i0 = tid_all; !st.ready && i0 < kpad; i0 += THREADS * CPT) {
-            float mean[CPT], var[CPT], m2[CPT];
-            if (st.training) {
-                float mb[CPT][kFoldMaxRowBlocks], m2b[CPT][kFoldMaxRowBlocks];
-#pragma unroll
-                for (int u = 0; u < CPT; ++u) {
-                    const int i = i0 + u * THREADS;
-                    const float* pc = st.partial + k_off + (i < K ? i : 0);
-#pragma unroll
-                    for (int b = 0; b < kFoldMaxRowBlocks; ++b) {
-                        const bool ok = b < st.row_blocks;
-                        mb[u][b] = ok ? pc[(int64_t)b * 2 * K_full] : 0.0f;
-                        m2b[u][b] = ok ? pc[(int64_t)b * 2 * K_full + K_full] : 0.0f;
-                    }
-                }
-#pragma unroll
-                for (int u = 0; u < CPT; ++u) {
-                    float snm = 0.0f;
-#pragma unroll
-                    for (int b = 0; b < kFoldMaxRowBlocks; ++b) {
-                        const float nb = b + 1 < st.row_blocks ? full : (b + 1 == st.row_blocks ? last : 0.0f);
-                        snm = __builtin_fmaf(nb, mb[u][b], snm);
-                    }
-                    mean[u] = snm / n;
-                    float acc2 = 0.0f;
-#pragma unroll
-                    for (int b = 0; b < kFoldMaxRowBlocks; ++b) {
-                        const float nb = b + 1 < st.row_blocks ? full : (b + 1 == st.row_blocks ? last : 0.0f);
-                        const float d = mb[u][b] - mean[u];
-                        acc2 += __builtin_fmaf(nb * d, d, m2b[u][b]);
-                    }
-                    m2[u] = acc2;
-                    var[u] = acc2 / n;                              // biased: what normalises the batch
-                }
-            } else {
-#pragma unroll
-                for (int u = 0; u < CPT; ++u) {
-                    const int i = i0 + u * THREADS;
-                    const int c = k_off + (i < K ? i : 0);
-                    mean[u] = load_stat_rt(st.running_mean, c, st.stats_dtype);
-                    var[u] = load_stat_rt(st.running_var, c, st.stats_dtype);
-                    m2[u] = 0.0f;
-                }
-            }
-#pragma unroll
-            for (int u = 0; u < CPT; ++u) {
-                const int i = i0 + u * THREADS;
-                if (i >= kpad) continue;
-                const int c = k_off + i;
-                const float rstd = 1.0f / sqrtf(var[u] + st.eps);
-                if (i < K && keeper && tm == (i / 64) % tiles_m) {
-                    if (st.training && st.running_mean != nullptr && st.running_var != nullptr) {
-                        const float unbiased = n > 1.0f ? m2[u] / (n - 1.0f) : var[u];
-                        store_stat_rt(st.running_mean, c, (1.0f - st.momentum) * load_stat_rt(st.running_mean, c, st.stats_dtype) + st.momentum * mean[u], st.stats_dtype);
-                        store_stat_rt(st.running_var, c, (1.0f - st.momentum) * load_stat_rt(st.running_var, c, st.stats_dtype) + st.momentum * unbiased, st.stats_dtype);
-                    }
-                    st.mean_rstd[c] = mean[u];
-                    st.mean_rstd[K_full + c] = rstd;
-                }
-                stats[i] = i < K ? mean[u] : 0.0f;
-                stats[kpad + i] = i < K ? rstd : 0.0f;
-            }
-        }
-    }
+    stage_stats<KG == 1 ? 2 : 1>(st, stats, kpad, K, K_full, k_off, tn == (k_off ? tiles_n / 2 : 0), tm, tiles_m);   // before the other loads claim its registers
 #pragma unroll
     for (int d = KG > 1 ? 2 : 0; d < D; ++d) load_global(d, d);
     __syncthreads();               // stats[] visible
@@ -569,53 +581,134 @@ __global__ __launch_bounds__(256 * KG) __attribute__((amdgpu_waves_per_eu(4, 4))
     }
 }
 
-// fp32 activations (the small parity configuration): plain FMA, 64x64 tile, 4x4 outputs per thread.
-__global__ __launch_bounds__(256) void router_gate_f32_kernel(const float* __restrict__ x, const float* __restrict__ w,
-                                                              const float* __restrict__ mean_rstd,
-                                                              float* __restrict__ logits32, float* __restrict__ logits,
-                                                              int M, int N, int K_full, int split) {
-    constexpr int TS = 64, KS = 16;
-    __shared__ float As[KS][TS + 1];
-    __shared__ float Bs[KS][TS + 1];
-    const int m0 = blockIdx.y * TS, n0 = blockIdx.x * TS;
-    const int tx = threadIdx.x % 16, ty = threadIdx.x / 16;
-    const int K = split ? K_full / 2 : K_full;              // split: the tile's columns score one half of the activations
+// logits[M, N] = normalise(x)[M, K] * W[N, K]^T while there are few tiles: the waves of a workgroup share one tile of 16 MT rows and 16
+// NT columns and split k, line l (128 bytes of k) to wave l mod kGateWaves.  Every wave takes its fragments straight from global
+// memory (lane l reads 16-byte piece l / 16 of row l % 16), kAhead steps of 64 bytes ahead and without a barrier, and normalises
+// the activations in registers; the waves' sums meet in LDS and are added in wave order, so the result depends neither on the
+// tile shape nor, the zero blocks of a block-diagonal gate adding nothing, on split.
+// STAGED: mean and 1/std of the tile's k range are made (or copied) in LDS first, overlapping the first loads; otherwise
+// st.ready, and they are read from mean_rstd as the operands are.
+constexpr int kGateWaves = 8;
+constexpr int kGateStagedK = 4096;       // 8 bytes of LDS per column
+constexpr uint32_t kOutOfRange = 0x80000000u;
+
+template <typename T, int MT, int NT, bool STAGED>
+__global__ __launch_bounds__(kGateWaves* kWave) void router_gate_splitk_kernel(
+    const T* __restrict__ x, const T* __restrict__ w, GateStats st, float* __restrict__ logits32, T* __restrict__ logits, int M, int N,
+    int K_full, int tiles_m, int tiles_n, int split, int xcds) {
+    constexpr int BM = 16 * MT, BN = 16 * NT, F = MT * NT, V = Elem<T>::kVec;
+    constexpr int kStep = 64 / (int)sizeof(T);                   // k values of a step; two steps are a line
+    constexpr int kAhead = MT + NT <= 3 ? 8 : 4;
+    constexpr int kRound = F < 8 ? F : 8;                        // fragments exchanged at a time
+    __shared__ __attribute__((aligned(16))) f32x4_t sums[kGateWaves][kRound][kWave];
+    extern __shared__ __attribute__((aligned(16))) float stats[];   // [2][kpad]: mean, rstd
+    const int tid = (int)threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    // XCD b % xcds takes a contiguous run of the tiles, all columns of a row first: its L2 holds the run's part of x only
+    const int tile = (int)(blockIdx.x % xcds) * ((int)gridDim.x / xcds) + (int)(blockIdx.x / xcds);
+    if (tile >= tiles_m * tiles_n) return;
+    const int tm = tile / tiles_n, tn = tile % tiles_n;
+    const int m0 = tm * BM, n0 = tn * BN;
+    // the k range of this tile: all of it, or the half of the activations its columns score (tiles do not straddle halves)
+    const int K = split ? K_full / 2 : K_full;
     const int k_off = (split && n0 >= N / 2) ? K : 0;
-    const float* mean = mean_rstd + k_off;
-    const float* rstd = mean_rstd + K_full + k_off;
-    float acc[4][4] = {};
-    for (int k0 = 0; k0 < K; k0 += KS) {
-        for (int q = threadIdx.x; q < TS * KS; q += 256) {
-            const int r = q / KS, kk = q % KS, gk = k0 + kk;
-            As[kk][r] = (m0 + r < M && gk < K) ? (x[(int64_t)(m0 + r) * K_full + k_off + gk] - mean[gk]) * rstd[gk] : 0.0f;
-            Bs[kk][r] = (n0 + r < N && gk < K) ? w[(int64_t)(n0 + r) * K + gk] : 0.0f;
-        }
-        __syncthreads();
+    auto rsrc = [&](const void* base, int64_t bytes) {
+        return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, (int)(bytes < 0x7FFFFFFFll ? bytes : 0x7FFFFFFFll), 0x00020000);
+    };
+    const __amdgpu_buffer_rsrc_t ar = rsrc(x + (int64_t)m0 * K_full + k_off, ((int64_t)(M - m0) * K_full - k_off) * (int64_t)sizeof(T));
+    const __amdgpu_buffer_rsrc_t br = rsrc(w + (int64_t)n0 * K, (int64_t)(N - n0) * K * (int64_t)sizeof(T));
+    const __amdgpu_buffer_rsrc_t sr = rsrc(st.mean_rstd + k_off, ((int64_t)2 * K_full - k_off) * 4);
+    const int frow = lane & 15, piece = lane >> 4;
+    uint32_t a_off[MT], b_off[NT];
 #pragma unroll
-        for (int kk = 0; kk < KS; ++kk) {
-            float a[4], b[4];
+    for (int i = 0; i < MT; ++i) a_off[i] = (uint32_t)((i * 16 + frow) * K_full) * (uint32_t)sizeof(T) + (uint32_t)piece * 16u;
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                a[i] = As[kk][ty * 4 + i];
-                b[i] = Bs[kk][tx * 4 + i];
-            }
+    for (int j = 0; j < NT; ++j) b_off[j] = (uint32_t)((j * 16 + frow) * K) * (uint32_t)sizeof(T) + (uint32_t)piece * 16u;
+    // step u of this wave: half u % 2 of its line u / 2; lines are numbered over all of k, whichever half the tile scores
+    const int lines = (K + 2 * kStep - 1) / (2 * kStep);
+    const int first_line = (wave + kGateWaves - (k_off / (2 * kStep)) % kGateWaves) % kGateWaves;
+    const int steps = first_line < lines ? 2 * ((lines - first_line + kGateWaves - 1) / kGateWaves) : 0;
+    u32x4_t fa[kAhead][MT], fb[kAhead][NT];
+    auto k_of = [&](int u) { return ((first_line + (u >> 1) * kGateWaves) * 2 + (u & 1)) * kStep; };
+    auto load = [&](int u, u32x4_t (&a)[MT], u32x4_t (&b)[NT]) {
+        const int k0 = k_of(u);
+        const bool drop = u >= steps || k0 + piece * V >= K;
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
+        for (int i = 0; i < MT; ++i)
+            a[i] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(ar, (int)(drop ? kOutOfRange : a_off[i]), k0 * (int)sizeof(T), 0));
 #pragma unroll
-                for (int j = 0; j < 4; ++j) acc[i][j] = __builtin_fmaf(a[i], b[j], acc[i][j]);
-        }
+        for (int j = 0; j < NT; ++j)
+            b[j] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(br, (int)(drop ? kOutOfRange : b_off[j]), k0 * (int)sizeof(T), 0));
+    };
+    f32x4_t acc[MT][NT];
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j) acc[i][j] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) load(u, fa[u], fb[u]);
+    const int kpad = (K + 2 * kStep - 1) / (2 * kStep) * (2 * kStep);
+    if constexpr (STAGED) {
+        stage_stats<1>(st, stats, kpad, K, K_full, k_off, tn == (k_off ? tiles_n / 2 : 0), tm, tiles_m);
         __syncthreads();
     }
+    for (int u0 = 0; u0 < steps; u0 += kAhead) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+        for (int d = 0; d < kAhead; ++d) {
+            const int u = u0 + d;
+            // steps past the end multiply zeros; their statistics are read from the last valid place
+            const int k0 = u < steps ? k_of(u) : 0;
+            float mean[V], rstd[V];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int row = m0 + ty * 4 + i, col = n0 + tx * 4 + j;
-            if (row < M && col < N) {
-                logits32[(int64_t)row * N + col] = acc[i][j];
-                logits[(int64_t)row * N + col] = acc[i][j];
+            for (int c = 0; c < V / 4; ++c) {
+                u32x4_t mv, rv;
+                if constexpr (STAGED) {
+                    mv = *reinterpret_cast<const u32x4_t*>(stats + k0 + piece * V + c * 4);
+                    rv = *reinterpret_cast<const u32x4_t*>(stats + kpad + k0 + piece * V + c * 4);
+                } else {
+                    const int at = (piece * V + c * 4) * 4;
+                    mv = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(sr, at, k0 * 4, 0));
+                    rv = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(sr, at, (K_full + k0) * 4, 0));
+                }
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    const uint32_t mw = mv[v], rw = rv[v];
+                    mean[c * 4 + v] = __uint_as_float(mw);
+                    rstd[c * 4 + v] = __uint_as_float(rw);
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < MT; ++i) {
+                const u32x4_t q = normalise16<T>(fa[d][i], mean, rstd);
+#pragma unroll
+                for (int j = 0; j < NT; ++j) acc[i][j] = mfma16_packet<T>(q, fb[d][j], acc[i][j]);
+            }
+            load(u + kAhead, fa[d], fb[d]);
+        }
+    }
+#pragma unroll
+    for (int f0 = 0; f0 < F; f0 += kRound) {
+        if (f0 > 0) __syncthreads();
+#pragma unroll
+        for (int f = f0; f < f0 + kRound; ++f) sums[wave][f - f0][lane] = acc[f / NT][f % NT];
+        __syncthreads();
+        // four rows of one column per (fragment, lane)
+        for (int q = tid; q < kRound * kWave; q += kGateWaves * kWave) {
+            const int f = f0 + (q >> 6), l = q & 63;
+            f32x4_t g = sums[0][q >> 6][l];
+#pragma unroll
+            for (int v = 1; v < kGateWaves; ++v) g += sums[v][q >> 6][l];
+            const int col = n0 + (f % NT) * 16 + (l & 15);
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const int row = m0 + (f / NT) * 16 + 4 * (l >> 4) + v;
+                if (row >= M || col >= N) continue;
+                const float sum = g[v];
+                logits32[(int64_t)row * N + col] = sum;
+                logits[(int64_t)row * N + col] = Elem<T>::from_f32(sum);
             }
         }
+    }
 }
 
 // q = round_T((x - mean) * rstd), 16 bytes per thread: the normalised activations as a stand-alone batch-norm emits them,
@@ -689,6 +782,42 @@ void launch_finalize(const float* partial, const ProloguePlan& p, int H, int tra
                      void* rm, void* rv, int64_t* nbt, float* mean_rstd, hipStream_t stream) {
     hipLaunchKernelGGL((bn_finalize_kernel<TS>), dim3((unsigned)((H + kWave - 1) / kWave)), dim3(kFinalizeWaves * kWave), 0, stream, partial,
                        p.row_blocks, H, training, momentum, eps, rm, rv, nbt, mean_rstd);
+}
+
+// The smallest tiles that still are one round of workgroups: 1024 tokens, 1024 columns, 256 outputs in bf16 take 14.7 us with the
+// statistics launch on 32 x 32 tiles (256 of them), 23 on 16 x 32 and 17 on 32 x 64; the 64 x 64 tiles of router_gate_kernel 18.2, and
+// with one tile 11.2 against 7.0 here.  16-bit products beyond a round of 32 x 64 tiles are left to that kernel, whose waves share
+// the operands through LDS (4096 tokens: 20.6 us against 22.4 on 64 x 64 tiles here); fp32 (bound by its matrix rate) goes on with
+// 64 x 64 tiles (2048 tokens: 25 us where a kernel of plain FMAs took 196; 207 tokens, 1232 columns, 436 outputs: 13 for 194).
+inline int64_t gate_tiles(int M, int N, int mt, int nt) { return (int64_t)((M + 16 * mt - 1) / (16 * mt)) * ((N + 16 * nt - 1) / (16 * nt)); }
+bool gate_splitk_pays(int M, int N, int dtype) { return dtype == FMOE_F32 || gate_tiles(M, N, 2, 4) <= chip_info().cus; }
+
+template <typename T>
+void launch_gate_splitk(const void* x, const void* w, const GateStats& st, float* logits32, void* logits, int M, int N, int K, int split,
+                        hipStream_t stream) {
+    const int cus = chip_info().cus, xcds = chip_info().xcds;
+    const bool staged = K <= kGateStagedK;
+    const int k_pad = (K + 63) / 64 * 64;
+#define FMOE_GATE_GO(MT, NT, STAGED)                                                                                            \
+    do {                                                                                                                        \
+        const int tiles_m = (M + 16 * MT - 1) / (16 * MT), tiles_n = (N + 16 * NT - 1) / (16 * NT);                             \
+        const int grid = (tiles_m * tiles_n + xcds - 1) / xcds * xcds;                                                          \
+        hipLaunchKernelGGL((router_gate_splitk_kernel<T, MT, NT, STAGED>), dim3((unsigned)grid), dim3(kGateWaves * kWave),      \
+                           STAGED ? (size_t)k_pad * 8 : 0, stream, (const T*)x, (const T*)w, st, logits32, (T*)logits, M, N, K, \
+                           tiles_m, tiles_n, split, xcds);                                                                      \
+    } while (0)
+#define FMOE_GATE_TILE(MT, NT)                     \
+    do {                                           \
+        if (staged) FMOE_GATE_GO(MT, NT, true);    \
+        else FMOE_GATE_GO(MT, NT, false);          \
+    } while (0)
+    if (gate_tiles(M, N, 1, 1) <= cus) FMOE_GATE_TILE(1, 1);
+    else if (gate_tiles(M, N, 1, 2) <= cus) FMOE_GATE_TILE(1, 2);
+    else if (gate_tiles(M, N, 2, 2) <= cus) FMOE_GATE_TILE(2, 2);
+    else if (sizeof(T) == 2 || gate_tiles(M, N, 2, 4) <= cus) FMOE_GATE_TILE(2, 4);
+    else FMOE_GATE_TILE(4, 4);
+#undef FMOE_GATE_TILE
+#undef FMOE_GATE_GO
 }
 
 // ------------------------------------------------------------------------------------------------------------
@@ -1091,59 +1220,49 @@ int fmoe::router_forward_impl(const void* x, const void* gate_w, void* running_m
     float* logits32 = logits_fp32;
 
     const int M = (int)num_tokens, N = 2 * num_keys;
-    if (dtype == FMOE_F32) {
-        if (training) {
-            launch_stats<float>(x, num_tokens, hidden, p, partial, s);
-            FMOE_CHECK_LAUNCH("fmoe_router_forward(batch statistics)");
+    const BlockStatsPlan bp = plan_block_stats(num_tokens);
+    const int64_t tiles64 = (int64_t)((M + 63) / 64) * ((N + 63) / 64);
+    // Every gate workgroup combining the block statistics itself saves a launch, but repeats the combination per tile: with more
+    // than a couple of tiles per CU one finalize launch is cheaper.
+    const bool splitk = gate_splitk_pays(M, N, dtype);
+    const bool fold = tiles64 <= 2 * (int64_t)chip_info().cus && hidden <= (splitk ? kGateStagedK : kGateMaxK);
+    if (training) {
+        if (fold) {
+            switch (dtype) {
+                case FMOE_F32: launch_block_stats<float>(x, num_tokens, hidden, bp, partial, s); break;
+                case FMOE_BF16: launch_block_stats<bf16_t>(x, num_tokens, hidden, bp, partial, s); break;
+                default: launch_block_stats<f16_t>(x, num_tokens, hidden, bp, partial, s); break;
+            }
+        } else {
+            switch (dtype) {
+                case FMOE_F32: launch_stats<float>(x, num_tokens, hidden, p, partial, s); break;
+                case FMOE_BF16: launch_stats<bf16_t>(x, num_tokens, hidden, p, partial, s); break;
+                default: launch_stats<f16_t>(x, num_tokens, hidden, p, partial, s); break;
+            }
         }
+        FMOE_CHECK_LAUNCH("fmoe_router_forward(batch statistics)");
+    }
+    if (!fold) {
         switch (stats_dtype) {
             case FMOE_F32: launch_finalize<float>(partial, p, hidden, training, momentum, eps, running_mean, running_var, num_batches_tracked, mean_rstd, s); break;
             case FMOE_BF16: launch_finalize<bf16_t>(partial, p, hidden, training, momentum, eps, running_mean, running_var, num_batches_tracked, mean_rstd, s); break;
             default: launch_finalize<f16_t>(partial, p, hidden, training, momentum, eps, running_mean, running_var, num_batches_tracked, mean_rstd, s); break;
         }
         FMOE_CHECK_LAUNCH("fmoe_router_forward(finalize)");
-        hipLaunchKernelGGL(router_gate_f32_kernel, dim3((N + 63) / 64, (M + 63) / 64), dim3(256), 0, s, (const float*)x,
-                           (const float*)gate_w, (const float*)mean_rstd, logits32, (float*)router_logits, M, N, hidden, split_query);
+    }
+    if (tiled_gate) {
+        // fold is false here (at least one 256 x 256 tile per compute unit): mean and 1/std are in the workspace
+        void* q = ws + p.off_q;
+        const int64_t packets = num_tokens * (int64_t)(hidden / 8);
+        if (dtype == FMOE_BF16)
+            hipLaunchKernelGGL((bn_apply_kernel<bf16_t>), dim3((unsigned)((packets + 255) / 256)), dim3(256), 0, s,
+                               (const u32x4_t*)x, (const float*)mean_rstd, (u32x4_t*)q, packets, hidden);
+        else
+            hipLaunchKernelGGL((bn_apply_kernel<f16_t>), dim3((unsigned)((packets + 255) / 256)), dim3(256), 0, s,
+                               (const u32x4_t*)x, (const float*)mean_rstd, (u32x4_t*)q, packets, hidden);
+        FMOE_CHECK_LAUNCH("fmoe_router_forward(normalise)");
+        if (int rc = gemm_nt_dual(q, gate_w, router_logits, logits32, M, N, hidden, dtype, s)) return rc;
     } else {
-        const BlockStatsPlan bp = plan_block_stats(num_tokens);
-        const int tiles_m = (M + 63) / 64, tiles_n = (N + 63) / 64;
-        // Every gate workgroup combining the block statistics itself saves a launch, but repeats the combination per
-        // tile: with more than a couple of tiles per CU one finalize launch is cheaper.
-        const bool fold = (int64_t)tiles_m * tiles_n <= 2 * (int64_t)chip_info().cus;
-        if (fold && training) {
-            if (dtype == FMOE_BF16) launch_block_stats<bf16_t>(x, num_tokens, hidden, bp, partial, s);
-            else launch_block_stats<f16_t>(x, num_tokens, hidden, bp, partial, s);
-            FMOE_CHECK_LAUNCH("fmoe_router_forward(batch statistics)");
-        }
-        if (!fold) {
-            if (training) {
-                if (dtype == FMOE_BF16) launch_stats<bf16_t>(x, num_tokens, hidden, p, partial, s);
-                else launch_stats<f16_t>(x, num_tokens, hidden, p, partial, s);
-                FMOE_CHECK_LAUNCH("fmoe_router_forward(batch statistics)");
-            }
-            switch (stats_dtype) {
-                case FMOE_F32: launch_finalize<float>(partial, p, hidden, training, momentum, eps, running_mean, running_var, num_batches_tracked, mean_rstd, s); break;
-                case FMOE_BF16: launch_finalize<bf16_t>(partial, p, hidden, training, momentum, eps, running_mean, running_var, num_batches_tracked, mean_rstd, s); break;
-                default: launch_finalize<f16_t>(partial, p, hidden, training, momentum, eps, running_mean, running_var, num_batches_tracked, mean_rstd, s); break;
-            }
-            FMOE_CHECK_LAUNCH("fmoe_router_forward(finalize)");
-        }
-        if (tiled_gate) {
-            // fold is false here (at least one 256 x 256 tile per compute unit): mean and 1/std are in the workspace
-            void* q = ws + p.off_q;
-            const int64_t packets = num_tokens * (int64_t)(hidden / 8);
-            if (dtype == FMOE_BF16)
-                hipLaunchKernelGGL((bn_apply_kernel<bf16_t>), dim3((unsigned)((packets + 255) / 256)), dim3(256), 0, s,
-                                   (const u32x4_t*)x, (const float*)mean_rstd, (u32x4_t*)q, packets, hidden);
-            else
-                hipLaunchKernelGGL((bn_apply_kernel<f16_t>), dim3((unsigned)((packets + 255) / 256)), dim3(256), 0, s,
-                                   (const u32x4_t*)x, (const float*)mean_rstd, (u32x4_t*)q, packets, hidden);
-            FMOE_CHECK_LAUNCH("fmoe_router_forward(normalise)");
-            if (int rc = gemm_nt_dual(q, gate_w, router_logits, logits32, M, N, hidden, dtype, s)) return rc;
-            if (top_k == 0) return FMOE_OK;
-            return launch_router_from_logits(logits32, num_tokens, num_keys, top_k, scores, indices, gates, dtype, norm_topk_prob,
-                                             row_offsets, row_bytes, s);
-        }
         GateStats st;
         st.ready = fold ? 0 : 1;
         st.partial = partial;
@@ -1158,25 +1277,34 @@ int fmoe::router_forward_impl(const void* x, const void* gate_w, void* running_m
         st.running_var = running_var;
         st.num_batches_tracked = num_batches_tracked;
         st.mean_rstd = mean_rstd;
-        const size_t stats_bytes = (size_t)((hidden + kTileK - 1) / kTileK) * kTileK * 2 * sizeof(float);
-        // few tiles with a long k loop: four k groups per workgroup, two for up to two tiles per compute unit; many tiles
-        // already fill the chip
-        const bool k_groups = (int64_t)tiles_m * tiles_n <= chip_info().cus && (split_query ? hidden / 2 : hidden) >= 8 * kTileK;
+        if (splitk) {
+            switch (dtype) {
+                case FMOE_F32: launch_gate_splitk<float>(x, gate_w, st, logits32, router_logits, M, N, hidden, split_query, s); break;
+                case FMOE_BF16: launch_gate_splitk<bf16_t>(x, gate_w, st, logits32, router_logits, M, N, hidden, split_query, s); break;
+                default: launch_gate_splitk<f16_t>(x, gate_w, st, logits32, router_logits, M, N, hidden, split_query, s); break;
+            }
+        } else {
+            const int tiles_m = (M + 63) / 64, tiles_n = (N + 63) / 64;
+            const size_t stats_bytes = (size_t)((hidden + kTileK - 1) / kTileK) * kTileK * 2 * sizeof(float);
+            // few tiles with a long k loop: four k groups per workgroup, two for up to two tiles per compute unit; many tiles
+            // already fill the chip
+            const bool long_k = (split_query ? hidden / 2 : hidden) >= 8 * kTileK;
+            const int groups = !long_k || tiles64 > 2 * chip_info().cus ? 1 : (tiles64 > chip_info().cus ? 2 : 4);
 #define FMOE_LAUNCH_GATE(TT, KG)                                                                                            \
     hipLaunchKernelGGL((router_gate_kernel<TT, KG>), dim3((unsigned)(tiles_m * tiles_n)), dim3(256 * KG), stats_bytes, s,  \
                        (const TT*)x, (const TT*)gate_w, st, logits32, (TT*)router_logits, M, N, hidden, tiles_m, tiles_n,   \
                        split_query, chip_info().xcds)
-        const bool k_pairs = !k_groups && (int64_t)tiles_m * tiles_n <= 2 * chip_info().cus && (split_query ? hidden / 2 : hidden) >= 8 * kTileK;
-        if (dtype == FMOE_BF16) {
-            if (k_groups) FMOE_LAUNCH_GATE(bf16_t, 4);
-            else if (k_pairs) FMOE_LAUNCH_GATE(bf16_t, 2);
-            else FMOE_LAUNCH_GATE(bf16_t, 1);
-        } else {
-            if (k_groups) FMOE_LAUNCH_GATE(f16_t, 4);
-            else if (k_pairs) FMOE_LAUNCH_GATE(f16_t, 2);
-            else FMOE_LAUNCH_GATE(f16_t, 1);
-        }
+            if (dtype == FMOE_BF16) {
+                if (groups == 4) FMOE_LAUNCH_GATE(bf16_t, 4);
+                else if (groups == 2) FMOE_LAUNCH_GATE(bf16_t, 2);
+                else FMOE_LAUNCH_GATE(bf16_t, 1);
+            } else {
+                if (groups == 4) FMOE_LAUNCH_GATE(f16_t, 4);
+                else if (groups == 2) FMOE_LAUNCH_GATE(f16_t, 2);
+                else FMOE_LAUNCH_GATE(f16_t, 1);
+            }
 #undef FMOE_LAUNCH_GATE
+        }
     }
     FMOE_CHECK_LAUNCH("fmoe_router_forward(gate)");
     if (top_k == 0) return FMOE_OK;

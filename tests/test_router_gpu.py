@@ -234,6 +234,32 @@ def test_fused_router_matches_oracle_prologue(T, H, nk, K, dtype):
     torch.testing.assert_close(gates.float().cpu(), orc.routing_weights(o_s[:, :K], False), rtol=g_tol, atol=g_atol)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("training", [True, False])
+@pytest.mark.parametrize("T,H,nk", [
+    # each tile shape of the k-splitting gate kernel with remainders in rows, columns and k (fewer k lines than waves, a half line, a
+    # last line of one packet), statistics read instead of staged (above 4096 columns), and one tile beyond a round of tiles
+    (2, 8, 2), (33, 72, 12), (600, 264, 61), (1000, 1000, 100), (2000, 520, 125), (4130, 776, 125), (40, 4104, 33),
+])
+def test_gate_logits_at_the_edges_of_the_tile_shapes(dtype, training, T, H, nk):
+    g = torch.Generator().manual_seed(T + H)
+    x = (torch.randn(T, H, generator=g) * 1.7 + 0.3).to(dtype)
+    wr = (torch.randn(2 * nk, H, generator=g) * 0.02).to(dtype)
+    rm, rv = torch.randn(H, generator=g).to(dtype), (torch.rand(H, generator=g) + 0.5).to(dtype)
+    (logits, *_, logits32), bn = _fused(x.float(), wr.float(), nk, 2, False, dtype, training=training, rm=rm.float(), rv=rv.float())
+    x64 = x.double()
+    mean, var = (x64.mean(0), x64.var(0, unbiased=False)) if training else (rm.double(), rv.double())
+    q = ((x64 - mean) / (var + 1e-5).sqrt()).to(dtype).double()
+    want = q @ wr.double().t()
+    err = (logits32.cpu().double() - want).norm() / want.norm()
+    assert err < {torch.float32: 1e-6, torch.bfloat16: 5e-4, torch.float16: 1e-4}[dtype], err
+    assert torch.equal(logits, logits32.to(dtype))
+    if training:
+        tol = {torch.float32: 1e-5, torch.bfloat16: 1e-2, torch.float16: 2e-3}[dtype]
+        torch.testing.assert_close(bn.running_mean.cpu().double(), 0.9 * rm.double() + 0.1 * mean, rtol=tol, atol=tol)
+        torch.testing.assert_close(bn.running_var.cpu().double(), 0.9 * rv.double() + 0.1 * x64.var(0), rtol=tol, atol=tol)
+
+
 def test_fused_router_eval_mode_and_normalised_gates():
     T, H, nk, K = 300, 128, 64, 32
     g = torch.Generator().manual_seed(5)
