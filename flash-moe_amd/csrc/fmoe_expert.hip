@@ -25,25 +25,44 @@ template <int ACT> __device__ inline float activate(float s) {
     return 1.0f;
 }
 
-constexpr int kPairsInFlight = 4;   // (down,up) row pairs requested ahead per wave
+// (down, up) row pairs requested ahead per wave: what fits 128 registers with sixteen waves in the workgroup, 256 with eight
+constexpr int kPairsInFlight = 4;
+constexpr int pairs_in_flight(int nch, int waves) {
+    if (waves == 16) return nch == 1 ? 4 : (nch == 2 ? 2 : 1);
+    if (waves == 8 && nch == 8) return 2;
+    return kPairsInFlight;
+}
 constexpr int kWavesPerBlock = 4;
 
+template <typename T> __device__ inline void store4(T* p, f32x4_t v) {
+    if constexpr (sizeof(T) == 4) {
+        *reinterpret_cast<f32x4_t*>(p) = v;
+    } else {
+        T r[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) r[i] = Elem<T>::from_f32(v[i]);
+        *reinterpret_cast<uint64_t*>(p) = __builtin_bit_cast(uint64_t, r);
+    }
+}
+
 // NCH = number of 16-byte packets each lane holds per row: a row has at most NCH*64 packets.
-// SPLIT = false: one wave per token, kWavesPerBlock tokens per workgroup.  SPLIT = true (few tokens): the workgroup's
-// waves share one token, wave w taking pairs w*P .. w*P+P-1, (w+4)*P .. of it (P = pairs in flight), and their partial rows
-// are added in wave order through LDS: four times shorter dependency chains when there are not enough tokens to fill the
-// chip with one wave each.
-template <typename T, typename TG, int NCH, int ACT, bool SPLIT>
-__global__ __launch_bounds__(kWavesPerBlock* kWave) void expert_token_kernel(
+// WAVES = 1: one wave per token, kWavesPerBlock tokens per workgroup.  WAVES > 1 (few tokens): the workgroup's waves share one
+// token, wave w taking pairs w*P .. w*P+P-1, (w+WAVES)*P .. of it (P = pairs in flight), and their partial rows are added in wave
+// order through LDS: dependency chains shorter by WAVES when there are not enough tokens to fill the chip with one wave each.
+template <typename T, typename TG, int NCH, int ACT, int WAVES>
+__global__ __launch_bounds__((WAVES > 1 ? WAVES : kWavesPerBlock) * kWave) void expert_token_kernel(
     const T* __restrict__ x, const T* __restrict__ down, const T* __restrict__ up,
     const int64_t* __restrict__ indices, const TG* __restrict__ gates, T* __restrict__ out,
     int64_t num_tokens, int hidden, int64_t num_experts, int top_k) {
+    constexpr bool SPLIT = WAVES > 1;
+    constexpr int P = pairs_in_flight(NCH, WAVES);
     constexpr int V = Elem<T>::kVec;
     const int lane = lane_id();
     const int wave = (int)(threadIdx.x >> 6);
     const int64_t token = SPLIT ? (int64_t)blockIdx.x : (int64_t)blockIdx.x * kWavesPerBlock + wave;
     if (token >= num_tokens) return;   // whole wave leaves together (SPLIT: the whole workgroup)
-    __shared__ float partial_rows[SPLIT ? (kWavesPerBlock - 1) * NCH * V * kWave : 1];
+    constexpr int ROW = NCH * V * kWave;
+    __shared__ __attribute__((aligned(16))) float partial_rows[SPLIT ? WAVES * ROW : 4];
 
     const int packets = hidden / V;   // 16-byte packets per row (hidden % V == 0 is checked on the host)
     const u32x4_t zero4 = {0u, 0u, 0u, 0u};
@@ -66,14 +85,14 @@ __global__ __launch_bounds__(kWavesPerBlock* kWave) void expert_token_kernel(
     const int64_t* my_idx = indices + token * top_k;
     const TG* my_gate = gates + token * top_k;
 
-    const int k_first = SPLIT ? wave * kPairsInFlight : 0;
-    const int k_step = SPLIT ? kWavesPerBlock * kPairsInFlight : kPairsInFlight;
+    const int k_first = SPLIT ? wave * P : 0;
+    const int k_step = WAVES * P;
     for (int k0 = k_first; k0 < top_k; k0 += k_step) {
-        u32x4_t dn[kPairsInFlight][NCH];
-        u32x4_t uq[kPairsInFlight][NCH];
-        float gate[kPairsInFlight];
+        u32x4_t dn[P][NCH];
+        u32x4_t uq[P][NCH];
+        float gate[P];
 #pragma unroll
-        for (int u = 0; u < kPairsInFlight; ++u) {
+        for (int u = 0; u < P; ++u) {
             const int k = k0 + u;
             int64_t e = -1;
             gate[u] = 0.0f;
@@ -96,9 +115,9 @@ __global__ __launch_bounds__(kWavesPerBlock* kWave) void expert_token_kernel(
                 uq[u][c] = (ok && live[c]) ? urow[p] : zero4;
             }
         }
-        float s[kPairsInFlight];
+        float s[P];
 #pragma unroll
-        for (int u = 0; u < kPairsInFlight; ++u) {
+        for (int u = 0; u < P; ++u) {
             float part = 0.0f;
 #pragma unroll
             for (int c = 0; c < NCH; ++c) part = dot16<T>(xr[c], dn[u][c], part);
@@ -106,10 +125,10 @@ __global__ __launch_bounds__(kWavesPerBlock* kWave) void expert_token_kernel(
         }
         if (ACT != kActNone) {
 #pragma unroll
-            for (int u = 0; u < kPairsInFlight; ++u) s[u] = wave_sum(s[u]);
+            for (int u = 0; u < P; ++u) s[u] = wave_sum(s[u]);
         }
 #pragma unroll
-        for (int u = 0; u < kPairsInFlight; ++u) {
+        for (int u = 0; u < P; ++u) {
             const float a = activate<ACT>(s[u]) * gate[u];
 #pragma unroll
             for (int c = 0; c < NCH; ++c) axpy16<T>(a, uq[u][c], acc[c]);
@@ -117,20 +136,20 @@ __global__ __launch_bounds__(kWavesPerBlock* kWave) void expert_token_kernel(
     }
 
     if (SPLIT) {
-        if (wave > 0) {
 #pragma unroll
-            for (int c = 0; c < NCH; ++c)
+        for (int c = 0; c < NCH; ++c)
 #pragma unroll
-                for (int v = 0; v < V; ++v) partial_rows[(((wave - 1) * NCH + c) * V + v) * kWave + lane] = acc[c][v];
-        }
+            for (int v = 0; v < V; v += 4)
+                *reinterpret_cast<f32x4_t*>(&partial_rows[wave * ROW + (c * kWave + lane) * V + v]) =
+                    f32x4_t{acc[c][v], acc[c][v + 1], acc[c][v + 2], acc[c][v + 3]};
         __syncthreads();
-        if (wave > 0) return;
+        for (int at = (int)threadIdx.x * 4; at < hidden; at += WAVES * kWave * 4) {
+            f32x4_t sum = *reinterpret_cast<const f32x4_t*>(&partial_rows[at]);
 #pragma unroll
-        for (int w = 0; w < kWavesPerBlock - 1; ++w)
-#pragma unroll
-            for (int c = 0; c < NCH; ++c)
-#pragma unroll
-                for (int v = 0; v < V; ++v) acc[c][v] += partial_rows[((w * NCH + c) * V + v) * kWave + lane];
+            for (int w = 1; w < WAVES; ++w) sum += *reinterpret_cast<const f32x4_t*>(&partial_rows[w * ROW + at]);
+            store4(out + token * hidden + at, sum);
+        }
+        return;
     }
 #pragma unroll
     for (int c = 0; c < NCH; ++c) {
@@ -145,18 +164,21 @@ int launch_expert_rows(int act, const void* x, const void* down, const void* up,
     constexpr int V = Elem<T>::kVec;
     const int packets = H / V;
     const int nch = (packets + kWave - 1) / kWave;
-    const dim3 block(kWavesPerBlock * kWave);
-    // with at most 2048 tokens a workgroup per token still fits the chip at once
-    const bool split = T_ <= 2048 && K > kPairsInFlight;
-    const dim3 grid((unsigned)(split ? T_ : (T_ + kWavesPerBlock - 1) / kWavesPerBlock));
-#define FMOE_LAUNCH_EXPERT_ACT(N, A)                                                                                  \
-    do {                                                                                                              \
-        if (split)                                                                                                    \
-            hipLaunchKernelGGL((expert_token_kernel<T, T, N, A, true>), grid, block, 0, stream, (const T*)x, (const T*)down, \
-                               (const T*)up, indices, (const T*)gates, (T*)out, T_, H, E, K);                         \
-        else                                                                                                          \
-            hipLaunchKernelGGL((expert_token_kernel<T, T, N, A, false>), grid, block, 0, stream, (const T*)x, (const T*)down, \
-                               (const T*)up, indices, (const T*)gates, (T*)out, T_, H, E, K);                         \
+    // Waves per token: sixteen while every token has a compute unit of its own (8 tokens of 1024 columns, 64 pairs: 5.8 us against
+    // 8.8 with four; 128 tokens: 7.3 against 12.4), four up to 2048 tokens (more only crowd each other out: 512 tokens
+    // take 21 us with 4, 8 or 16), one beyond.  Rows of more than four packets per lane leave registers for eight.
+    const int waves = K <= kPairsInFlight || T_ > 2048 ? 1 : (T_ > chip_info().cus ? 4 : (nch > 4 ? 8 : 16));
+    const dim3 block((waves > 1 ? waves : kWavesPerBlock) * kWave);
+    const dim3 grid((unsigned)(waves > 1 ? T_ : (T_ + kWavesPerBlock - 1) / kWavesPerBlock));
+#define FMOE_LAUNCH_EXPERT_WAVES(N, A, W)                                                                             \
+    hipLaunchKernelGGL((expert_token_kernel<T, T, N, A, W>), grid, block, 0, stream, (const T*)x, (const T*)down,     \
+                       (const T*)up, indices, (const T*)gates, (T*)out, T_, H, E, K)
+#define FMOE_LAUNCH_EXPERT_ACT(N, A)                                 \
+    do {                                                             \
+        if (waves == 16 && N < 8) FMOE_LAUNCH_EXPERT_WAVES(N, A, (N < 8 ? 16 : 8)); \
+        else if (waves >= 8) FMOE_LAUNCH_EXPERT_WAVES(N, A, 8);      \
+        else if (waves == 4) FMOE_LAUNCH_EXPERT_WAVES(N, A, 4);      \
+        else FMOE_LAUNCH_EXPERT_WAVES(N, A, 1);                      \
     } while (0)
 #define FMOE_LAUNCH_EXPERT(N)                                     \
     do {                                                          \
@@ -175,6 +197,7 @@ int launch_expert_rows(int act, const void* x, const void* down, const void* up,
     }
 #undef FMOE_LAUNCH_EXPERT
 #undef FMOE_LAUNCH_EXPERT_ACT
+#undef FMOE_LAUNCH_EXPERT_WAVES
     FMOE_CHECK_LAUNCH("fmoe_expert_forward");
     return FMOE_OK;
 }
@@ -189,7 +212,7 @@ int launch_expert_rows_coef(const void* up, const int64_t* indices, const float*
     const dim3 block(kWavesPerBlock * kWave);
     const dim3 grid((unsigned)((T_ + kWavesPerBlock - 1) / kWavesPerBlock));
 #define FMOE_LAUNCH_COEF(N)                                                                                             \
-    hipLaunchKernelGGL((expert_token_kernel<T, float, N, kActNone, false>), grid, block, 0, stream, (const T*)up, (const T*)up, \
+    hipLaunchKernelGGL((expert_token_kernel<T, float, N, kActNone, 1>), grid, block, 0, stream, (const T*)up, (const T*)up, \
                        (const T*)up, indices, coef, (T*)out, T_, H, E, K)
     if (nch <= 1) FMOE_LAUNCH_COEF(1);
     else if (nch <= 2) FMOE_LAUNCH_COEF(2);

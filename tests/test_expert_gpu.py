@@ -51,6 +51,19 @@ def test_expert_matches_oracle(dtype, T, H, E, K, algo):
     assert fro < {torch.float32: 2e-6, torch.bfloat16: 4e-3, torch.float16: 5e-4}[dtype], fro
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("T", [1, 256, 257, 2049])
+@pytest.mark.parametrize("H,K", [(24, 4), (264, 5), (520, 67), (1032, 17), (2048, 9)])
+def test_expert_rows_at_the_edges_of_the_waves_per_token(dtype, T, H, K):
+    # sixteen (or eight), four and one wave per token; rows of one to eight packets per lane, the last ones partial; the fewest
+    # pairs that are split, and more pairs than the waves take in a round
+    x, wd, wu, idx, g = orc.make_expert_inputs(T, H, 300, K, seed=T + H)
+    x, wd, wu, g = (t.to(dtype) for t in (x, wd, wu, g))
+    got = run(x, wd, wu, idx, g, "rows")
+    fro = rel_fro(got, truth64(x, wd, wu, idx, g))
+    assert fro < {torch.float32: 2e-6, torch.bfloat16: 4e-3, torch.float16: 5e-4}[dtype], fro
+
+
 @pytest.mark.parametrize("dtype,H", [(torch.bfloat16, 8192), (torch.bfloat16, 5120), (torch.float16, 4104), (torch.float32, 2304)])
 def test_expert_long_rows_take_the_column_slices(dtype, H):
     # rows of more than 8192 bytes do not fit the registers of the one-wave-per-token kernel: the op takes the column-slice
