@@ -8,7 +8,8 @@ namespace fmoe {
 namespace {
 
 struct BlockPlan {
-    size_t off_router, off_logits32, off_scores, off_indices, off_gates, off_expert, off_act, off_experts_out, bytes;
+    size_t off_router, off_logits32, off_scores, off_indices, off_gates, off_expert, off_act, off_experts_out, off_sums, bytes;
+    bool small;      // evaluation mode takes the three launches of fmoe_small.hip
 };
 
 BlockPlan plan_block(int64_t T_, int H, int I, int nk, int64_t E, int K, int dtype) {
@@ -24,6 +25,8 @@ BlockPlan plan_block(int64_t T_, int H, int I, int nk, int64_t E, int K, int dty
     p.off_expert = take(fmoe_expert_workspace_bytes(T_, H, E, K, dtype));
     p.off_act = take(fmoe_mlp_workspace_bytes(T_, H, I, dtype));
     p.off_experts_out = take((size_t)T_ * H * elt);
+    p.small = block_small_usable(T_, H, I, nk, E, K, dtype);
+    p.off_sums = take(p.small ? block_small_sums_bytes(T_, H, I, dtype) : 0);
     p.bytes = o;
     return p;
 }
@@ -143,6 +146,12 @@ int block_forward_impl(const char* who, const void* x, const void* gate_proj_w, 
     void* act = ws + p.off_act;
     void* experts = ws + p.off_experts_out;
     const size_t elt = dtype_size(dtype);
+
+    if (p.small && !training && saved == nullptr && running_mean && running_var && dtype_ok(stats_dtype))
+        return block_small_forward(x, gate_proj_w, up_proj_w, down_proj_w, router_gate_w, down_embed, up_embed, running_mean, running_var,
+                                   stats_dtype, eps, num_tokens, hidden, intermediate, num_experts, num_keys, top_k, dtype, norm_topk_prob,
+                                   out, router_logits, logits32, scores, indices, gates, act, (float*)(ws + p.off_router),
+                                   (float*)(ws + p.off_sums), s);
 
     const bool slices = expert_slices_usable(num_tokens, hidden, num_experts, top_k, dtype);
     uint32_t* offsets = slices ? expert_workspace_offsets(expert_ws) : nullptr;

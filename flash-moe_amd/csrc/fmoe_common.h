@@ -51,6 +51,22 @@ int launch_router_from_logits(const float* logits, int64_t num_tokens, int num_k
 // Whether a top-k kernel exists for these extents: top_k <= 256 with any num_keys, or top_k <= 1024 with num_keys <= 8192.
 bool router_topk_supported(int num_keys, int top_k);
 
+// The whole block for up to kSmallMaxTokens tokens in evaluation mode in three launches (fmoe_small.hip); usable says whether these
+// extents have it, sums_bytes what `sums` needs.  mean_rstd: [2][H] scratch.
+constexpr int kSmallMaxTokens = 256, kSmallMaxSlices = 4;
+bool block_small_usable(int64_t num_tokens, int hidden, int intermediate, int num_keys, int64_t num_experts, int top_k, int dtype);
+size_t block_small_sums_bytes(int64_t num_tokens, int hidden, int intermediate, int dtype);
+int block_small_forward(const void* x, const void* gate_proj_w, const void* up_proj_w, const void* down_proj_w, const void* router_gate_w,
+                        const void* down_embed, const void* up_embed, void* running_mean, void* running_var, int stats_dtype, float eps,
+                        int64_t num_tokens, int hidden, int intermediate, int64_t num_experts, int num_keys, int top_k, int dtype,
+                        int norm_topk_prob, void* out, void* router_logits, float* logits32, float* scores, int64_t* indices, void* gates,
+                        void* act, float* mean_rstd, float* sums, hipStream_t stream);
+// The row schedule of the routed experts: whether these extents take it, and with `slices` fp32 planes [T,H] added to its result
+// (few tokens, at most 2048 columns).
+bool expert_rows_chosen(int64_t num_tokens, int hidden, int64_t num_experts, int top_k, int dtype);
+int expert_rows_added(const void* x, const void* down, const void* up, const int64_t* indices, const void* gates, int64_t num_tokens,
+                      int hidden, int64_t num_experts, int top_k, int dtype, const float* planes, int slices, void* out, hipStream_t stream);
+
 // The fused router (fmoe_router_forward) with the optional row-offset output; defined in fmoe_router_prologue.hip.
 // fixed_scratch: the workspace is the fixed scratch of the no-allocation entry point, which has no room for the normalised
 // copy of x that many tokens would otherwise use.

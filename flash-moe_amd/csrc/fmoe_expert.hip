@@ -49,11 +49,12 @@ template <typename T> __device__ inline void store4(T* p, f32x4_t v) {
 // WAVES = 1: one wave per token, kWavesPerBlock tokens per workgroup.  WAVES > 1 (few tokens): the workgroup's waves share one
 // token, wave w taking pairs w*P .. w*P+P-1, (w+WAVES)*P .. of it (P = pairs in flight), and their partial rows are added in wave
 // order through LDS: dependency chains shorter by WAVES when there are not enough tokens to fill the chip with one wave each.
-template <typename T, typename TG, int NCH, int ACT, int WAVES>
+// ADDED (at most WAVES * 256 columns): `slices` planes [T, H] of fp32 sums are added to the rounded result, as the residual of the down product would be.
+template <typename T, typename TG, int NCH, int ACT, int WAVES, bool ADDED = false>
 __global__ __launch_bounds__((WAVES > 1 ? WAVES : kWavesPerBlock) * kWave) void expert_token_kernel(
     const T* __restrict__ x, const T* __restrict__ down, const T* __restrict__ up,
     const int64_t* __restrict__ indices, const TG* __restrict__ gates, T* __restrict__ out,
-    int64_t num_tokens, int hidden, int64_t num_experts, int top_k) {
+    int64_t num_tokens, int hidden, int64_t num_experts, int top_k, const float* __restrict__ planes, int slices) {
     constexpr bool SPLIT = WAVES > 1;
     constexpr int P = pairs_in_flight(NCH, WAVES);
     constexpr int V = Elem<T>::kVec;
@@ -81,6 +82,15 @@ __global__ __launch_bounds__((WAVES > 1 ? WAVES : kWavesPerBlock) * kWave) void 
     for (int c = 0; c < NCH; ++c)
 #pragma unroll
         for (int v = 0; v < V; ++v) acc[c][v] = 0.0f;
+
+    f32x4_t added[ADDED ? kSmallMaxSlices : 1];
+    if constexpr (ADDED) {
+        const int at = (int)threadIdx.x * 4;
+#pragma unroll
+        for (int s = 0; s < kSmallMaxSlices; ++s)
+            added[s] = s < slices && at < hidden ? *reinterpret_cast<const f32x4_t*>(planes + (s * num_tokens + token) * hidden + at)
+                                                 : f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    }
 
     const int64_t* my_idx = indices + token * top_k;
     const TG* my_gate = gates + token * top_k;
@@ -147,6 +157,13 @@ __global__ __launch_bounds__((WAVES > 1 ? WAVES : kWavesPerBlock) * kWave) void 
             f32x4_t sum = *reinterpret_cast<const f32x4_t*>(&partial_rows[at]);
 #pragma unroll
             for (int w = 1; w < WAVES; ++w) sum += *reinterpret_cast<const f32x4_t*>(&partial_rows[w * ROW + at]);
+            if constexpr (ADDED) {
+                f32x4_t mlp = added[0];
+#pragma unroll
+                for (int s = 1; s < kSmallMaxSlices; ++s) mlp += added[s];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) sum[i] = mlp[i] + round_through<T>(sum[i]);
+            }
             store4(out + token * hidden + at, sum);
         }
         return;
@@ -172,7 +189,7 @@ int launch_expert_rows(int act, const void* x, const void* down, const void* up,
     const dim3 grid((unsigned)(waves > 1 ? T_ : (T_ + kWavesPerBlock - 1) / kWavesPerBlock));
 #define FMOE_LAUNCH_EXPERT_WAVES(N, A, W)                                                                             \
     hipLaunchKernelGGL((expert_token_kernel<T, T, N, A, W>), grid, block, 0, stream, (const T*)x, (const T*)down,     \
-                       (const T*)up, indices, (const T*)gates, (T*)out, T_, H, E, K)
+                       (const T*)up, indices, (const T*)gates, (T*)out, T_, H, E, K, nullptr, 0)
 #define FMOE_LAUNCH_EXPERT_ACT(N, A)                                 \
     do {                                                             \
         if (waves == 16 && N < 8) FMOE_LAUNCH_EXPERT_WAVES(N, A, (N < 8 ? 16 : 8)); \
@@ -202,6 +219,20 @@ int launch_expert_rows(int act, const void* x, const void* down, const void* up,
     return FMOE_OK;
 }
 
+template <typename T>
+void launch_expert_rows_added(const void* x, const void* down, const void* up, const int64_t* indices, const void* gates, int64_t T_, int H,
+                              int64_t E, int K, const float* planes, int slices, void* out, hipStream_t stream) {
+    const int nch = (H / Elem<T>::kVec + kWave - 1) / kWave;
+#define FMOE_LAUNCH_ADDED(N, W)                                                                                                      \
+    hipLaunchKernelGGL((expert_token_kernel<T, T, N, kActSilu, W, true>), dim3((unsigned)T_), dim3(W * kWave), 0, stream, (const T*)x, \
+                       (const T*)down, (const T*)up, indices, (const T*)gates, (T*)out, T_, H, E, K, planes, slices)
+    if (nch <= 1) FMOE_LAUNCH_ADDED(1, 16);
+    else if (nch <= 2) FMOE_LAUNCH_ADDED(2, 16);
+    else if (nch <= 4) FMOE_LAUNCH_ADDED(4, 16);
+    else if constexpr (sizeof(T) == 4) FMOE_LAUNCH_ADDED(8, 8);
+#undef FMOE_LAUNCH_ADDED
+}
+
 // out[t] = sum_k coef[t,k] * up[idx[t,k]] with fp32 coefficients that are already complete (the second phase of the
 // bucketed schedule): the row kernel without its score phase.
 template <typename T>
@@ -213,7 +244,7 @@ int launch_expert_rows_coef(const void* up, const int64_t* indices, const float*
     const dim3 grid((unsigned)((T_ + kWavesPerBlock - 1) / kWavesPerBlock));
 #define FMOE_LAUNCH_COEF(N)                                                                                             \
     hipLaunchKernelGGL((expert_token_kernel<T, float, N, kActNone, 1>), grid, block, 0, stream, (const T*)up, (const T*)up, \
-                       (const T*)up, indices, coef, (T*)out, T_, H, E, K)
+                       (const T*)up, indices, coef, (T*)out, T_, H, E, K, nullptr, 0)
     if (nch <= 1) FMOE_LAUNCH_COEF(1);
     else if (nch <= 2) FMOE_LAUNCH_COEF(2);
     else if (nch <= 4) FMOE_LAUNCH_COEF(4);
@@ -1388,6 +1419,21 @@ bool expert_slices_usable(int64_t num_tokens, int hidden, int64_t num_experts, i
 }
 
 uint32_t* expert_workspace_offsets(void* workspace) { return (uint32_t*)workspace; }   // SlicePlan::off_idx32 == 0
+
+bool expert_rows_chosen(int64_t num_tokens, int hidden, int64_t num_experts, int top_k, int dtype) {
+    return choose_schedule(FMOE_EXPERT_AUTO, num_tokens, hidden, num_experts, top_k, dtype_size(dtype)) == FMOE_EXPERT_ROWS;
+}
+
+int expert_rows_added(const void* x, const void* down, const void* up, const int64_t* indices, const void* gates, int64_t num_tokens,
+                      int hidden, int64_t num_experts, int top_k, int dtype, const float* planes, int slices, void* out, hipStream_t stream) {
+    switch (dtype) {
+        case FMOE_F32: launch_expert_rows_added<float>(x, down, up, indices, gates, num_tokens, hidden, num_experts, top_k, planes, slices, out, stream); break;
+        case FMOE_BF16: launch_expert_rows_added<bf16_t>(x, down, up, indices, gates, num_tokens, hidden, num_experts, top_k, planes, slices, out, stream); break;
+        default: launch_expert_rows_added<f16_t>(x, down, up, indices, gates, num_tokens, hidden, num_experts, top_k, planes, slices, out, stream); break;
+    }
+    FMOE_CHECK_LAUNCH("fmoe_block(experts)");
+    return FMOE_OK;
+}
 
 // What a forward in the slice or ordered schedule leaves for the backward (which takes the same schedule for these extents).
 ExpertSavedPlan expert_saved_plan(int64_t num_tokens, int hidden, int64_t num_experts, int top_k, int dtype) {

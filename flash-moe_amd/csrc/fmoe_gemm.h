@@ -1,0 +1,501 @@
+// Tiles of C[M,N] = A[M,K] * B[N,K]^T on the matrix cores (gfx950), the parts of kernels that form such products: the shared MLP
+// (fmoe_mlp.hip) and the launches that put a product beside other work (fmoe_small.hip).  `block` of `blocks` workgroups.
+#pragma once
+
+#include "fmoe_common.h"
+#include "fmoe_mfma.h"
+
+namespace fmoe {
+namespace {
+
+enum Epilogue { kEpiSwiGLU = 0, kEpiPlain = 1, kEpiDual = 2, kEpiPart = 3 };   // Dual: the product in T and, through R, in fp32
+template <bool B> struct Flag { static constexpr bool value = B; };
+constexpr uint32_t kOutOfRange = 0x80000000u;    // beyond every buffer descriptor here: loads give zeros, stores are dropped
+
+// ------------------------------------------------------------------------------------------------------------
+// LDS-DMA pipelined kernel.  WAVES_M x WAVES_N waves, each (BM/WAVES_M) x (BN/WAVES_N); BKT = k extent of a stage.
+// ------------------------------------------------------------------------------------------------------------
+// FR: fragment shape (32: v_mfma_f32_32x32x16 / 32x32x2; 16: v_mfma_f32_16x16x32).  SPLIT: a k-step's A fragments are read and
+// multiplied in SPLIT parts (its B fragments stay for the whole k-step), which halves the registers the read-ahead needs.
+template <typename T, int BM, int BN, int WAVES_M, int WAVES_N, int BKT, int NSTAGE, int EPI, int PF, int FR = 32, int SPLIT = 1, bool RAGGED = false>
+__device__ __forceinline__ void gemm_dma_tiles(
+    const T* __restrict__ A, const T* __restrict__ B0, const T* __restrict__ B1, T* __restrict__ C,
+    const T* __restrict__ R, int M, int N, int K, int tiles_m, int tiles_n, int xcds, int block, int blocks) {
+    using Shape = MfmaShape<T, FR>;
+    using Frag = typename Shape::Frag;
+    using Acc = typename Shape::Acc;
+    constexpr int NV = Shape::kAccRegs;
+    constexpr int NWAVES = WAVES_M * WAVES_N;
+    constexpr int WM = BM / WAVES_M, WN = BN / WAVES_N, MF = WM / FR, NF = WN / FR;
+    constexpr int EPC = 16 / (int)sizeof(T);        // elements per 16-byte chunk
+    constexpr int CPR = BKT / EPC;                  // 16-byte chunks per LDS row
+    constexpr int RPI = 64 / CPR;                   // rows one wave-wide DMA load covers
+    constexpr int ROWS_PER_IT = NWAVES * RPI;       // rows all waves cover per DMA round
+    constexpr int STAGE = (BM + BN) * BKT;          // elements per stage
+    constexpr int KSTEPS = BKT / (Shape::kChunks * EPC);   // a k-step is kChunks 16-byte pieces of a row: one per lane group
+    constexpr int SPK = KSTEPS * SPLIT;             // steps (a part of a k-step's A fragments against all its B fragments) per k-tile
+    constexpr int MFS = MF / SPLIT;
+    static_assert(MF % SPLIT == 0 && WM % FR == 0 && WN % FR == 0, "fragments tile the wave tile");
+    constexpr int ROW_SHIFT = (CPR == 8) ? 1 : 2;   // log2(rows per 256 bytes)
+    constexpr int BN_OUT = (EPI == kEpiSwiGLU) ? BN / 2 : BN;
+    constexpr int A_ROUNDS = BM / ROWS_PER_IT, B_ROUNDS = BN / ROWS_PER_IT;
+    constexpr int DMA_PER_TILE = A_ROUNDS + B_ROUNDS;
+    static_assert(CPR == 4 || CPR == 8, "stage depth: LDS rows of 64 or 128 bytes");
+    static_assert(ROWS_PER_IT % 16 == 0 && BM % ROWS_PER_IT == 0 && BN % ROWS_PER_IT == 0, "DMA rounds");
+    static_assert(EPI != kEpiSwiGLU || ((BN / 2) % ROWS_PER_IT == 0 && NF % 2 == 0), "gate/up split");
+    static_assert((NSTAGE - 2) * DMA_PER_TILE < 64, "vmcnt range");
+
+    __shared__ __attribute__((aligned(1024))) T lds[NSTAGE * STAGE];
+
+    const int tid = (int)threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = wave / WAVES_N, wn = wave % WAVES_N;
+    const int num_tiles = tiles_m * tiles_n;
+
+    // DMA: the lane's LDS position is row (round*ROWS_PER_IT + wave*RPI + lrow), physical chunk lp; it holds the
+    // logical chunk lp ^ key(row), key(row) = (row >> ROW_SHIFT) & (CPR-1).  ROWS_PER_IT is a multiple of 16, so the
+    // key does not depend on the round and one element offset per lane serves every load.
+    const int lrow = lane / CPR, lp = lane % CPR;
+    const int key_dma = ((wave * RPI + lrow) >> ROW_SHIFT) & (CPR - 1);
+    const uint32_t lane_off = (uint32_t)(lrow * K + (lp ^ key_dma) * EPC) * (uint32_t)sizeof(T);   // bytes
+    // A rows beyond M (a ragged last tile row) are read from row M-1 instead: one byte offset per DMA round, set per
+    // tile.  What the MFMAs make of those rows is never stored (the epilogue's buffer stores are bounds-checked).
+    uint32_t a_lane_off[A_ROUNDS];
+    const T *a_src, *b_src0, *b_src1 = nullptr;
+    // RAGGED: rows and the k tail are cut off by the range check of buffer descriptors over the rest of each matrix
+    __amdgpu_buffer_rsrc_t a_rsrc, b_rsrc0, b_rsrc1;
+    int m0, n0;
+    const int k_tiles = (K + BKT - 1) / BKT;
+    const bool lane_in_tail = (k_tiles - 1) * BKT + (lp ^ key_dma) * EPC < K;      // the lane's chunk of the last k-tile exists
+    auto rest_of = [&](const T* base, int64_t rows) {                              // descriptor from `base` to the end of its matrix
+        const int64_t bytes = rows * K * (int64_t)sizeof(T);
+        return __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(base), 0, (int)(bytes < 0x7FFFFFFFll ? bytes : 0x7FFFFFFFll), 0x00020000);
+    };
+    // The workgroup is persistent: it takes tiles t, t + blocks, ...  Each XCD (workgroup id mod 8) gets a contiguous
+    // run of the tile order, walked 8 tile-rows at a time so that a compact patch shares A and B tiles in the XCD's L2.
+    auto set_tile = [&](int t) {
+        if (num_tiles % xcds == 0) t = (t % xcds) * (num_tiles / xcds) + t / xcds;
+        constexpr int GM = 8;
+        const int width = GM * tiles_n, group = t / width, first_m = group * GM;
+        const int gsz = (tiles_m - first_m) < GM ? (tiles_m - first_m) : GM;
+        m0 = (first_m + (t % width) % gsz) * BM;
+        n0 = ((t % width) / gsz) * BN_OUT;
+        a_src = A + (int64_t)m0 * K;                     // wave-uniform; the lane's part is the 32-bit a_lane_off[r]
+#pragma unroll
+        for (int r = 0; r < A_ROUNDS; ++r) {
+            int row = r * ROWS_PER_IT + wave * RPI + lrow;
+            if (!RAGGED) row = m0 + row < M ? row : M - 1 - m0;
+            a_lane_off[r] = (uint32_t)(row * K + (lp ^ key_dma) * EPC) * (uint32_t)sizeof(T);
+        }
+        b_src0 = B0 + (int64_t)(n0 + wave * RPI) * K;
+        if (EPI == kEpiSwiGLU) b_src1 = B1 + (int64_t)(n0 + wave * RPI) * K;
+        if constexpr (RAGGED) {
+            a_rsrc = rest_of(a_src, M - m0);
+            b_rsrc0 = rest_of(B0 + (int64_t)n0 * K, N - n0);
+            if (EPI == kEpiSwiGLU) b_rsrc1 = rest_of(B1 + (int64_t)n0 * K, N - n0);
+        }
+    };
+    auto issue = [&](int kt, T* stage) {
+        const int k0 = kt * BKT;
+        if constexpr (RAGGED) {
+            const bool drop = kt + 1 == k_tiles && !lane_in_tail;
+#pragma unroll
+            for (int r = 0; r < A_ROUNDS; ++r)
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(
+                    a_rsrc, (__attribute__((address_space(3))) void*)(stage + (r * ROWS_PER_IT + wave * RPI) * BKT), 16,
+                    (int)(drop ? kOutOfRange : a_lane_off[r]), k0 * (int)sizeof(T), 0, 0);
+#pragma unroll
+            for (int r = 0; r < B_ROUNDS; ++r) {
+                const bool second = EPI == kEpiSwiGLU && r >= B_ROUNDS / 2;
+                const uint32_t off = (uint32_t)(((second ? r - B_ROUNDS / 2 : r) * ROWS_PER_IT + wave * RPI) * K) * (uint32_t)sizeof(T) + lane_off;
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(
+                    second ? b_rsrc1 : b_rsrc0,
+                    (__attribute__((address_space(3))) void*)(stage + BM * BKT + (r * ROWS_PER_IT + wave * RPI) * BKT), 16,
+                    (int)(drop ? kOutOfRange : off), k0 * (int)sizeof(T), 0, 0);
+            }
+            return;
+        }
+#pragma unroll
+        for (int r = 0; r < A_ROUNDS; ++r)
+            __builtin_amdgcn_global_load_lds(
+                (const __attribute__((address_space(1))) void*)((const char*)(a_src + k0) + a_lane_off[r]),
+                (__attribute__((address_space(3))) void*)(stage + (r * ROWS_PER_IT + wave * RPI) * BKT), 16, 0, 0);
+#pragma unroll
+        for (int r = 0; r < B_ROUNDS; ++r) {
+            const T* src;
+            if (EPI == kEpiSwiGLU && r >= B_ROUNDS / 2) src = b_src1 + (int64_t)(r - B_ROUNDS / 2) * ROWS_PER_IT * K + k0;
+            else src = b_src0 + (int64_t)r * ROWS_PER_IT * K + k0;
+            __builtin_amdgcn_global_load_lds(
+                (const __attribute__((address_space(1))) void*)((const char*)src + lane_off),
+                (__attribute__((address_space(3))) void*)(stage + BM * BKT + (r * ROWS_PER_IT + wave * RPI) * BKT), 16, 0, 0);
+        }
+    };
+
+    // Fragment rows of a lane are (multiple of FR) + frow: the swizzle key is the same for all of them, so the
+    // address is (row base + one per-k-step offset) + an immediate per fragment.
+    const int frow = lane % FR, fhalf = lane / FR;       // fhalf: which 16-byte piece of a k-step the lane supplies
+    const int key_f = (frow >> ROW_SHIFT) & (CPR - 1);
+    const int a_row_bytes = (wm * WM + frow) * BKT * (int)sizeof(T);
+    int b_row_bytes[NF];
+#pragma unroll
+    for (int j = 0; j < NF; ++j) {
+        int row;
+        if (EPI == kEpiSwiGLU) row = (j < NF / 2) ? wn * (WN / 2) + j * FR : BN / 2 + wn * (WN / 2) + (j - NF / 2) * FR;
+        else row = wn * WN + j * FR;
+        b_row_bytes[j] = (BM + row + frow) * BKT * (int)sizeof(T);
+    }
+    int pc[KSTEPS];
+#pragma unroll
+    for (int ks = 0; ks < KSTEPS; ++ks) pc[ks] = ((ks * Shape::kChunks + fhalf) ^ key_f) << 4;
+
+    int tile = block;
+    if (tile >= num_tiles) return;
+    set_tile(tile);
+#pragma unroll
+    for (int s = 0; s < NSTAGE - 1; ++s)
+        if (s < k_tiles) issue(s, lds + s * STAGE);
+
+    // Fragments of step q+PF are read from LDS while the MFMAs of step q run (PF+1 register buffers for the A parts; B
+    // fragments are read with the first part of their k-step); the read-ahead crosses k-tile boundaries, so the barrier
+    // that publishes the next stage sits PF steps before the end of a k-tile and the matrix pipe always has work queued
+    // while a wave waits.
+    constexpr int RING = PF + 1;
+    constexpr int RINGB = SPLIT == 1 ? RING : 2;
+    static_assert(SPK % RING == 0 && PF >= 1 && PF < SPK + 1, "fragment buffers rotate with period RING");
+    static_assert(SPLIT == 1 || (PF <= SPLIT && KSTEPS % 2 == 0), "with split k-steps at most the next k-step's B fragments are in flight");
+    Frag fa[RING][MFS], fb[RINGB][NF];
+    auto b_slot = [](int q) { return SPLIT == 1 ? q % RING : (q / SPLIT) % 2; };     // q: step inside the k-tile (may exceed SPK by PF)
+    auto read_frags = [&](const char* stage, int q, Frag (&a)[MFS], Frag (&b)[NF]) {
+        const int ks = q / SPLIT, part = q % SPLIT;
+#pragma unroll
+        for (int i = 0; i < MFS; ++i)
+            a[i] = *reinterpret_cast<const Frag*>(stage + a_row_bytes + pc[ks] + (part * MFS + i) * FR * BKT * (int)sizeof(T));
+        if (part == 0) {
+#pragma unroll
+            for (int j = 0; j < NF; ++j) b[j] = *reinterpret_cast<const Frag*>(stage + b_row_bytes[j] + pc[ks]);
+        }
+    };
+    // Entering k-tile kt (kt = 0: from the tile prologue): my share of its stage has landed once at most the loads of
+    // the NSTAGE-2 younger k-tiles are outstanding; my reads of the stage that is overwritten next are complete (all
+    // reads of k-tile kt-1 have been issued by then); after the barrier both hold for every wave, so the load of k-tile
+    // kt+NSTAGE-1 can go into the stage kt-1 used.
+    auto enter_k_tile = [&](int kt) {
+        constexpr int kKeep = (NSTAGE - 2) * DMA_PER_TILE;
+        if (kt + NSTAGE - 2 < k_tiles) __builtin_amdgcn_s_waitcnt(0x0070 | (kKeep & 0xF) | ((kKeep >> 4) << 14));
+        else __builtin_amdgcn_s_waitcnt(0x0070);
+        __builtin_amdgcn_s_barrier();
+        if (kt + NSTAGE - 1 < k_tiles) issue(kt + NSTAGE - 1, lds + ((kt + NSTAGE - 1) % NSTAGE) * STAGE);
+    };
+    while (true) {
+        Acc acc[MF][NF];
+#pragma unroll
+        for (int i = 0; i < MF; ++i)
+#pragma unroll
+            for (int j = 0; j < NF; ++j)
+#pragma unroll
+                for (int v = 0; v < NV; ++v) acc[i][j][v] = 0.0f;
+
+        enter_k_tile(0);
+#pragma unroll
+        for (int s = 0; s < PF; ++s) read_frags(reinterpret_cast<const char*>(lds), s, fa[s % RING], fb[b_slot(s)]);
+        // the last k-tile has no successor to read ahead into: it is a separate copy of the body, so that no branch
+        // merges a path with reads in flight into the MFMA sequence
+        auto k_tile_body = [&](int kt, auto last_tag) {
+            constexpr bool kLast = decltype(last_tag)::value;
+            const char* stage = reinterpret_cast<const char*>(lds + (kt % NSTAGE) * STAGE);
+            const char* next_stage = reinterpret_cast<const char*>(lds + ((kt + 1) % NSTAGE) * STAGE);
+#pragma unroll
+            for (int q = 0; q < SPK; ++q) {
+                const int nxt = q + PF;
+                constexpr int kMfmas = MFS * NF;     // runs of Shape::kInstr instructions
+                const bool reads = nxt < SPK || !kLast;
+                const int n_reads = MFS + ((nxt % SPLIT) == 0 ? NF : 0);
+                __builtin_amdgcn_sched_barrier(0);
+                if (nxt < SPK) {
+                    read_frags(stage, nxt, fa[nxt % RING], fb[b_slot(nxt)]);
+                } else if (!kLast) {
+                    if (nxt == SPK) {
+                        enter_k_tile(kt + 1);
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                    read_frags(next_stage, nxt - SPK, fa[nxt % RING], fb[b_slot(nxt)]);
+                }
+                const int part = q % SPLIT;
+#pragma unroll
+                for (int i = 0; i < MFS; ++i)
+#pragma unroll
+                    for (int j = 0; j < NF; ++j)
+                        acc[part * MFS + i][j] = Shape::run(fa[q % RING][i], fb[b_slot(q)][j], acc[part * MFS + i][j]);
+                // issue order: the LDS reads spread evenly behind the MFMAs
+                constexpr int kPer = (MFS + NF + kMfmas - 1) / kMfmas;
+#pragma unroll
+                for (int m = 0; m < kMfmas; ++m) {
+                    __builtin_amdgcn_sched_group_barrier(0x008, Shape::kInstr, 0);
+                    if (reads && m * kPer < n_reads) __builtin_amdgcn_sched_group_barrier(0x100, kPer, 0);
+                }
+            }
+        };
+        for (int kt = 0; kt + 1 < k_tiles; ++kt) k_tile_body(kt, Flag<false>{});
+        k_tile_body(k_tiles - 1, Flag<true>{});
+        __builtin_amdgcn_sched_barrier(0);
+
+        // start the next tile's first stages before this tile's epilogue, so that its global-load latency is covered
+        const int out_m0 = m0, out_n0 = n0;
+        const int next = tile + blocks;
+        if (next < num_tiles) {
+            set_tile(next);
+            __builtin_amdgcn_s_barrier();     // every wave has consumed its reads of the last stage
+#pragma unroll
+            for (int s = 0; s < NSTAGE - 1; ++s)
+                if (s < k_tiles) issue(s, lds + s * STAGE);
+        }
+
+        // D fragment layout (both shapes): lane l, register v holds
+        //   row = 8*(v/4) + 4*(l/FR) + (v%4)   (A / M index),   col = l%FR   (B / N index)
+        // Buffer addressing: a wave-uniform descriptor of the rows from the wave's first one on, a scalar byte offset
+        // per (fragment, register) and one 32-bit byte offset per lane - no vector address arithmetic per element.
+        const int lane_bytes0 = ((4 * fhalf) * N + frow) * (int)sizeof(T);
+        const int64_t wave_off = (int64_t)(out_m0 + wm * WM) * N + out_n0 + wn * ((EPI == kEpiSwiGLU) ? WN / 2 : WN);
+        const int64_t span = ((int64_t)M * N - wave_off) * (int64_t)sizeof(T);
+        // a wave whose rows all lie beyond M gets an empty descriptor: every access of it is dropped
+        const int span32 = (int)(span < 0 ? 0 : (span < 0x7FFFFFFFll ? span : 0x7FFFFFFFll));
+        auto c_rsrc = __builtin_amdgcn_make_buffer_rsrc(C + wave_off, 0, span32, 0x00020000);
+        // RAGGED: a lane whose column of fragment column j lies beyond N takes an offset no descriptor covers
+        auto lane_at = [&](int j, int in_range) {
+            if (!RAGGED) return in_range;
+            const int col = out_n0 + wn * ((EPI == kEpiSwiGLU) ? WN / 2 : WN) + j * FR + frow;
+            return col < N ? in_range : (int)kOutOfRange;
+        };
+        auto store_to = [&](auto rsrc, int lane_bytes, int uni_bytes, float value) {
+            if constexpr (sizeof(T) == 4) {
+                __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, value), rsrc, lane_bytes, uni_bytes, 0);
+            } else {
+                const T t = Elem<T>::from_f32(value);
+                __builtin_amdgcn_raw_buffer_store_b16(__builtin_bit_cast(short, t), rsrc, lane_bytes, uni_bytes, 0);
+            }
+        };
+        // 16-bit outputs round once, so the fast reciprocal's last-bit error is invisible; fp32 divides
+        auto silu = [](float v) { return sizeof(T) == 4 ? silu_f32(v) : silu_fast_f32(v); };
+        // element offset of (fragment i, fragment column j, register v) from the wave's first output element
+        auto elem_at = [&](int i, int j, int v) { return (i * FR + 8 * (v / 4) + (v % 4)) * N + j * FR; };
+        if (EPI == kEpiSwiGLU) {
+            if (R != nullptr) {
+                // keep the gate and up products for a backward pass: planes [0] and [1] of a [2, M, N] buffer
+                T* planes = const_cast<T*>(R);
+                auto g_rsrc = __builtin_amdgcn_make_buffer_rsrc(planes + wave_off, 0, span32, 0x00020000);
+                auto u_rsrc = __builtin_amdgcn_make_buffer_rsrc(planes + (int64_t)M * N + wave_off, 0, span32, 0x00020000);
+#pragma unroll
+                for (int i = 0; i < MF; ++i)
+#pragma unroll
+                    for (int j = 0; j < NF / 2; ++j)
+#pragma unroll
+                        for (int v = 0; v < NV; ++v) {
+                            const int uni = elem_at(i, j, v) * (int)sizeof(T);
+                            store_to(g_rsrc, lane_at(j, lane_bytes0), uni, acc[i][j][v]);
+                            store_to(u_rsrc, lane_at(j, lane_bytes0), uni, acc[i][j + NF / 2][v]);
+                        }
+            }
+#pragma unroll
+            for (int i = 0; i < MF; ++i)
+#pragma unroll
+                for (int j = 0; j < NF / 2; ++j)
+#pragma unroll
+                    for (int v = 0; v < NV; ++v)
+                        store_to(c_rsrc, lane_at(j, lane_bytes0), elem_at(i, j, v) * (int)sizeof(T), silu(acc[i][j][v]) * acc[i][j + NF / 2][v]);
+        } else if (EPI == kEpiDual) {
+            // R points at an fp32 [M, N] buffer that receives the unrounded sums next to the rounded ones in C
+            float* out32 = reinterpret_cast<float*>(const_cast<T*>(R));
+            const int64_t span_f = ((int64_t)M * N - wave_off) * 4;
+            const int span32_f = (int)(span_f < 0 ? 0 : (span_f < 0x7FFFFFFFll ? span_f : 0x7FFFFFFFll));
+            auto f_rsrc = __builtin_amdgcn_make_buffer_rsrc(out32 + wave_off, 0, span32_f, 0x00020000);
+            const int lane_bytes_f = ((4 * fhalf) * N + frow) * 4;
+#pragma unroll
+            for (int i = 0; i < MF; ++i)
+#pragma unroll
+                for (int j = 0; j < NF; ++j)
+#pragma unroll
+                    for (int v = 0; v < NV; ++v) {
+                        const int at = elem_at(i, j, v);
+                        const float sum = acc[i][j][v];      // a scalar copy: the bit cast below must not see a vector element
+                        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, sum), f_rsrc, lane_at(j, lane_bytes_f), at * 4, 0);
+                        store_to(c_rsrc, lane_at(j, lane_bytes0), at * (int)sizeof(T), sum);
+                    }
+        } else {
+            auto r_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(R != nullptr ? R + wave_off : C), 0,
+                                                            R != nullptr ? span32 : 0, 0x00020000);   // no residual: reads give 0
+#pragma unroll
+            for (int i = 0; i < MF; ++i)
+#pragma unroll
+                for (int j = 0; j < NF; ++j) {
+                    float res[NV];
+                    const int lane_bytes = lane_at(j, lane_bytes0);
+#pragma unroll
+                    for (int v = 0; v < NV; ++v) {
+                        const int uni = elem_at(i, j, v) * (int)sizeof(T);
+                        if constexpr (sizeof(T) == 4) {
+                            res[v] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r_rsrc, lane_bytes, uni, 0));
+                        } else {
+                            const short raw = __builtin_amdgcn_raw_buffer_load_b16(r_rsrc, lane_bytes, uni, 0);
+                            res[v] = Elem<T>::to_f32(__builtin_bit_cast(T, raw));
+                        }
+                    }
+#pragma unroll
+                    for (int v = 0; v < NV; ++v) store_to(c_rsrc, lane_bytes, elem_at(i, j, v) * (int)sizeof(T), acc[i][j][v] + res[v]);
+                }
+        }
+        if (next >= num_tiles) break;
+        tile = next;
+    }
+}
+
+// ------------------------------------------------------------------------------------------------------------
+// Few output tiles: the waves of a workgroup share one small tile and split k.  Every wave takes its fragments straight from
+// global memory (a fragment is 16 rows of 64 bytes: lane l reads 16-byte piece l / 16 of row l % 16), kAhead k-steps ahead and
+// without a barrier; the waves' sums meet in LDS, added in wave order.  Rows beyond M or N and the k tail read as zeros (range
+// check of the descriptors).  fp32: a 16-byte piece is four k values, one per v_mfma_f32_16x16x4.
+// Bound by latency (about 4 us for a launch of one short wave per SIMD) and by what the L2s deliver (about 13 TB/s over the
+// chip): the 1024 x 4096 down product takes 7.4 us for one token and 11 us for 64 where 64 x 64 tiles with the whole k loop in
+// one chain take 14.3 us; from about 128 tokens on the larger tiles' smaller traffic wins.  Loads of whole lines (8 rows of 128
+// bytes, fragments rebuilt with lane rotations) were no faster.
+// kEpiPart: slice `slice` of `slices` of k, its sums in fp32 to plane `slice` of C.
+// ------------------------------------------------------------------------------------------------------------
+constexpr int kSplitWaves = 8;
+
+template <typename T, int MT, int NT, int EPI>
+__device__ __forceinline__ void gemm_splitk_tile(
+    const T* __restrict__ A, const T* __restrict__ B0, const T* __restrict__ B1, T* __restrict__ C,
+    const T* __restrict__ R, int M, int N, int K, int tiles_m, int tiles, int xcds, int block, int blocks, int slice = 0, int slices = 1) {
+    constexpr int BM = 16 * MT, BN = 16 * NT;
+    constexpr int NB = EPI == kEpiSwiGLU ? 2 * NT : NT;          // B fragments: gate rows, then the same up rows
+    constexpr int F = MT * NB;
+    constexpr int kAhead = MT + NB <= 3 ? 8 : 4;
+    constexpr int kStep = 64 / (int)sizeof(T);                   // k values of a step
+    __shared__ __attribute__((aligned(16))) f32x4_t sums[kSplitWaves][F][64];
+    const int tid = (int)threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    // XCD b % xcds takes a contiguous run of the tiles, all rows of a column first: its L2 holds B's part of the run only
+    const int tile = (block % xcds) * (blocks / xcds) + block / xcds;
+    if (tile >= tiles) return;
+    const int m0 = (tile % tiles_m) * BM, n0 = (tile / tiles_m) * BN;
+    auto rest_of = [&](const T* base, int64_t rows) {
+        const int64_t bytes = rows * K * (int64_t)sizeof(T);
+        return __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(base), 0, (int)(bytes < 0x7FFFFFFFll ? bytes : 0x7FFFFFFFll), 0x00020000);
+    };
+    const __amdgpu_buffer_rsrc_t ar = rest_of(A + (int64_t)m0 * K, M - m0), br = rest_of(B0 + (int64_t)n0 * K, N - n0);
+    const __amdgpu_buffer_rsrc_t br1 = EPI == kEpiSwiGLU ? rest_of(B1 + (int64_t)n0 * K, N - n0) : br;
+    const int frow = lane & 15, piece = lane >> 4;
+    uint32_t row_off[MT > NT ? MT : NT];
+#pragma unroll
+    for (int i = 0; i < (MT > NT ? MT : NT); ++i) row_off[i] = (uint32_t)((i * 16 + frow) * K) * (uint32_t)sizeof(T) + (uint32_t)piece * 16u;
+    const int steps = (K + kStep - 1) / kStep;
+    const int parts = kSplitWaves * slices;
+    const int share = ((steps + 2 * parts - 1) / (2 * parts)) * 2;                   // two steps are one 128-byte line of a row
+    const int first = (slice * kSplitWaves + wave) * share, last = first + share < steps ? first + share : steps;
+    const bool in_tail = (steps - 1) * kStep + piece * (16 / (int)sizeof(T)) < K;
+    u32x4_t fa[kAhead][MT], fb[kAhead][NB];
+    auto load = [&](int step, u32x4_t (&a)[MT], u32x4_t (&b)[NB]) {
+        const bool drop = step >= last || (step + 1 == steps && !in_tail);
+        const int at = step * 64;
+#pragma unroll
+        for (int i = 0; i < MT; ++i) a[i] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(ar, (int)(drop ? kOutOfRange : row_off[i]), at, 0));
+#pragma unroll
+        for (int j = 0; j < NB; ++j)
+            b[j] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(j < NT ? br : br1, (int)(drop ? kOutOfRange : row_off[j % NT]), at, 0));
+    };
+    f32x4_t acc[MT][NB];
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < NB; ++j) acc[i][j] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) load(first + u, fa[u], fb[u]);
+    for (int s0 = first; s0 < last; s0 += kAhead) {
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u) {
+#pragma unroll
+            for (int i = 0; i < MT; ++i)
+#pragma unroll
+                for (int j = 0; j < NB; ++j) acc[i][j] = mfma16_packet<T>(fa[u][i], fb[u][j], acc[i][j]);
+            load(s0 + u + kAhead, fa[u], fb[u]);
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < NB; ++j) sums[wave][i * NB + j][lane] = acc[i][j];
+    __syncthreads();
+    // four rows of one column per (fragment, lane)
+    for (int q = tid; q < MT * NT * 64; q += kSplitWaves * 64) {
+        const int f = q >> 6, l = q & 63, i = f / NT, j = f % NT;
+        f32x4_t g = sums[0][i * NB + j][l], u = {0.0f, 0.0f, 0.0f, 0.0f};
+        for (int w = 1; w < kSplitWaves; ++w) g += sums[w][i * NB + j][l];
+        if (EPI == kEpiSwiGLU) {
+            u = sums[0][i * NB + NT + j][l];
+            for (int w = 1; w < kSplitWaves; ++w) u += sums[w][i * NB + NT + j][l];
+        }
+        const int col = n0 + j * 16 + (l & 15);
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const int row = m0 + i * 16 + 4 * (l >> 4) + v;
+            if (row >= M || col >= N) continue;
+            const int64_t at = (int64_t)row * N + col;
+            if (EPI == kEpiPart) {
+                reinterpret_cast<float*>(C)[(int64_t)slice * M * N + at] = g[v];
+            } else if (EPI == kEpiSwiGLU) {
+                const float act = sizeof(T) == 4 ? silu_f32(g[v]) : silu_fast_f32(g[v]);
+                C[at] = Elem<T>::from_f32(act * u[v]);
+                if (R != nullptr) {      // planes [0] and [1] of a [2, M, N] buffer keep the two products
+                    const_cast<T*>(R)[at] = Elem<T>::from_f32(g[v]);
+                    const_cast<T*>(R)[(int64_t)M * N + at] = Elem<T>::from_f32(u[v]);
+                }
+            } else {
+                C[at] = Elem<T>::from_f32(R != nullptr ? g[v] + Elem<T>::to_f32(R[at]) : g[v]);
+            }
+        }
+    }
+}
+
+// k extent of one LDS stage of the DMA kernel: 128 bytes of a row for every element type
+template <typename T> constexpr int kStageK = 128 / (int)sizeof(T);
+// 16-bit products run on v_mfma_f32_16x16x32 (more multiply-adds per joule than 32x32x16, which is what bounds these
+// kernels); a k-step is then half a stage, so the read-ahead is one step, and the 256 x 256 tile reads a k-step's A
+// fragments in four parts to stay inside 256 registers per wave (in two parts it spills 24).  fp32 keeps 32x32x2.
+template <typename T> constexpr int kFragRows = sizeof(T) == 2 ? 16 : 32;
+template <typename T> constexpr int kBigSplit = sizeof(T) == 2 ? 4 : 1;
+template <typename T> constexpr int kSmallAhead = sizeof(T) == 2 ? 1 : 3;
+
+// Tile choice.  A workgroup's time per k-tile is the larger of what its CU receives from the L2 ((BM + BN) rows of 128 bytes at
+// about 70 GB/s per CU) and what its matrix pipes take (BM * BN); 128 x 128 balances the two, so in units of one received row the
+// second is BM * BN / 66.  The launch lasts as many rounds as the busiest CU has tiles.  The rule picks the shape with the
+// smallest rounds * time: 256 x 256 (8 waves, two per SIMD) once the chip has several tiles per CU, smaller ones so that every CU
+// has a tile, whatever the extents.
+// fp32 rows of 128 bytes hold half as many values for matrix pipes an eighth as fast: BM * BN / 15.  The k-splitting kernel
+// costs more per received row, and more so the more CUs receive at once (measured from 64 to 224 workgroups), but its tiles are
+// small enough for a few rows of A.
+enum TileShape { kTile256, kTile128, kTile64x128, kTile64, kSplit32, kSplit16x32, kSplit16 };
+template <typename T, int EPI> TileShape choose_tile(int M, int N, int& tiles) {
+    constexpr int kRows[7] = {256, 128, 64, 64, 32, 16, 16}, kOuts[7] = {256, 128, 128, 64, 32, 32, 16};
+    const int cus = chip_info().cus;
+    TileShape best = kTile128;
+    double best_cost = 0.0;
+    for (int i = 0; i < 7; ++i) {
+        if (i == kTile64 && EPI == kEpiSwiGLU && sizeof(T) == 4) continue;      // a 32-column wave tile is one fp32 fragment: no gate/up pair
+        const bool split_k = i >= kSplit32;
+        const int out_cols = EPI == kEpiSwiGLU && !split_k ? kOuts[i] / 2 : kOuts[i];
+        const int cols = EPI == kEpiSwiGLU ? 2 * out_cols : out_cols;
+        const int64_t n = (int64_t)((M + kRows[i] - 1) / kRows[i]) * ((N + out_cols - 1) / out_cols);
+        const double occupied = n < cus ? (double)n / cus : 1.0;
+        const double received = (kRows[i] + cols) * (split_k ? 1.45 * (1.0 + occupied) : 1.0);
+        const double multiplied = kRows[i] * (double)cols / (sizeof(T) == 4 ? 15.0 : 66.0);
+        const double cost = (double)((n + cus - 1) / cus) * (received > multiplied ? received : multiplied);
+        if (i == 0 || cost < best_cost) {
+            best = (TileShape)i;
+            best_cost = cost;
+            tiles = (int)(n < (1 << 30) ? n : (1 << 30));
+        }
+    }
+    return best;
+}
+
+}  // namespace
+}  // namespace fmoe

@@ -1,0 +1,408 @@
+// Product-key selection on one wave per token, for lists that fit the wave's registers (gfx950): the keys and sorting networks all
+// selections share, and the selection by threshold of the kernels in fmoe_router.hip and fmoe_small.hip.
+#pragma once
+
+#include <math.h>
+
+#include "fmoe_common.h"
+
+namespace fmoe {
+namespace {
+
+__device__ inline uint32_t order_bits(float f) {
+    const uint32_t u = __float_as_uint(f);
+    return u ^ ((u >> 31) ? 0xffffffffu : 0x80000000u);
+}
+__device__ inline float order_value(uint32_t o) {
+    return __uint_as_float(o ^ ((o >> 31) ? 0x80000000u : 0xffffffffu));
+}
+__device__ inline uint64_t make_key(float score, uint32_t index) {
+    return ((uint64_t)order_bits(score) << 32) | (uint64_t)(~index);
+}
+__device__ inline float key_score(uint64_t k) { return order_value((uint32_t)(k >> 32)); }
+__device__ inline uint32_t key_index(uint64_t k) { return ~(uint32_t)(k & 0xffffffffu); }
+
+// Value of lane (lane ^ mask) for mask in {1,2,4,8,16,32}; `mask` must be a compile-time constant after inlining.
+// Distances 1, 2 and 8 are single DPP moves.  Distances 4, 16 and 32 would cost 2-4 vector instructions each on the
+// DPP / permlane path; the kernel is bound by vector-ALU issue, so they go through the LDS crossbar instead
+// (ds_swizzle / ds_bpermute: no LDS memory is touched, no vector-ALU slot is used, other waves cover the latency).
+__device__ inline uint32_t xor_lane_u32(uint32_t v, int mask, int lane) {
+    const int iv = (int)v;
+    switch (mask) {
+        case 1: return (uint32_t)__builtin_amdgcn_update_dpp(0, iv, 0xB1, 0xF, 0xF, true);    // quad_perm [1,0,3,2]
+        case 2: return (uint32_t)__builtin_amdgcn_update_dpp(0, iv, 0x4E, 0xF, 0xF, true);    // quad_perm [2,3,0,1]
+        case 4: return (uint32_t)__builtin_amdgcn_ds_swizzle(iv, (4 << 10) | 0x1F);          // bit mode: lane ^ 4
+        case 8: return (uint32_t)__builtin_amdgcn_update_dpp(0, iv, 0x128, 0xF, 0xF, true);   // row_ror:8
+        case 16: return (uint32_t)__builtin_amdgcn_ds_swizzle(iv, (16 << 10) | 0x1F);        // bit mode: lane ^ 16
+        default: return (uint32_t)__builtin_amdgcn_ds_bpermute((lane ^ 32) << 2, iv);
+    }
+}
+__device__ inline uint64_t xor_lane_u64(uint64_t v, int mask, int lane) {
+    const uint32_t lo = xor_lane_u32((uint32_t)v, mask, lane);
+    const uint32_t hi = xor_lane_u32((uint32_t)(v >> 32), mask, lane);
+    return ((uint64_t)hi << 32) | lo;
+}
+
+// Position of a key in the wave-wide sequence: p = lane*RK + r.
+// One compare-exchange layer of a bitonic network: partner = p ^ J, blocks of size K alternate direction.
+// Which lanes keep the larger key is a function of the lane number alone, so it is a 64-bit compile-time constant per
+// (layer, register), handed to the selects as a lane mask (inverse ballot): no vector instruction and no live scalar
+// register per layer, where lane-number compares hoisted out of the token loop would be spilled.
+template <int RK> struct LaneMasks { uint64_t m[RK]; };
+template <int RK, int K, bool DESC> constexpr LaneMasks<RK> descending_block_lanes() {
+    LaneMasks<RK> out{};
+    for (int r = 0; r < RK; ++r)
+        for (int l = 0; l < kWave; ++l) out.m[r] |= (uint64_t)((((l * RK + r) & K) == 0) == DESC) << l;
+    return out;
+}
+template <int RK, int K, int J, bool DESC> constexpr LaneMasks<RK> keep_max_lanes() {
+    LaneMasks<RK> out{};
+    for (int r = 0; r < RK; ++r)
+        for (int l = 0; l < kWave; ++l) {
+            const int p = l * RK + r;
+            const bool desc_block = (((p & K) == 0) == DESC), first = (p & J) == 0;
+            out.m[r] |= (uint64_t)(first == desc_block) << l;
+        }
+    return out;
+}
+
+template <int RK, bool DESC, int K, int J>
+__device__ inline void bitonic_layer(uint64_t (&v)[RK], int lane) {
+    if constexpr (J < RK) {
+        constexpr LaneMasks<RK> desc = descending_block_lanes<RK, K, DESC>();
+#pragma unroll
+        for (int r = 0; r < RK; ++r) {
+            if ((r & J) == 0) {
+                const bool desc_block = __builtin_amdgcn_inverse_ballot_w64(desc.m[r]);
+                const uint64_t a = v[r], b = v[r | J];
+                const uint64_t hi = a > b ? a : b, lo = a > b ? b : a;
+                v[r] = desc_block ? hi : lo;
+                v[r | J] = desc_block ? lo : hi;
+            }
+        }
+    } else {
+        constexpr LaneMasks<RK> keep = keep_max_lanes<RK, K, J, DESC>();
+#pragma unroll
+        for (int r = 0; r < RK; ++r) {
+            const uint64_t other = xor_lane_u64(v[r], J / RK, lane);
+            const bool keep_max = __builtin_amdgcn_inverse_ballot_w64(keep.m[r]);
+            // keep my key if it is the larger one and I keep the max, or the smaller one and I keep the min
+            v[r] = ((v[r] > other) == keep_max) ? v[r] : other;
+        }
+    }
+}
+
+// layers J, J/2, ..., 1 of the stage with block size K
+template <int RK, bool DESC, int K, int J>
+__device__ inline void bitonic_stage(uint64_t (&v)[RK], int lane) {
+    bitonic_layer<RK, DESC, K, J>(v, lane);
+    if constexpr (J > 1) bitonic_stage<RK, DESC, K, J / 2>(v, lane);
+}
+// stages K, 2K, ..., N
+template <int RK, bool DESC, int K>
+__device__ inline void bitonic_stages_from(uint64_t (&v)[RK], int lane) {
+    bitonic_stage<RK, DESC, K, K / 2>(v, lane);
+    if constexpr (K < RK * kWave) bitonic_stages_from<RK, DESC, 2 * K>(v, lane);
+}
+
+template <int RK, bool DESC>
+__device__ inline void bitonic_sort(uint64_t (&v)[RK], int lane) {
+    bitonic_stages_from<RK, DESC, 2>(v, lane);
+}
+
+// One key per lane: every aligned block of N lanes sorted descending on its own (block size 0 in the last stage: all blocks alike).
+template <int N>
+__device__ inline void bitonic_sort_blocks(uint64_t& v, int lane) {
+    uint64_t a[1] = {v};
+    if constexpr (N >= 4) bitonic_stage<1, true, 2, 1>(a, lane);
+    if constexpr (N >= 8) bitonic_stage<1, true, 4, 2>(a, lane);
+    if constexpr (N >= 16) bitonic_stage<1, true, 8, 4>(a, lane);
+    if constexpr (N >= 32) bitonic_stage<1, true, 16, 8>(a, lane);
+    if constexpr (N >= 64) bitonic_stage<1, true, 32, 16>(a, lane);
+    bitonic_stage<1, true, 0, N / 2>(a, lane);
+    v = a[0];
+}
+
+// v holds a bitonic sequence of N keys; sort it descending.
+template <int RK>
+__device__ inline void bitonic_merge_desc(uint64_t (&v)[RK], int lane) {
+    constexpr int N = RK * kWave;
+    bitonic_stage<RK, true, N, N / 2>(v, lane);
+}
+
+// Key at position `pos` of the wave-wide sequence (wave-uniform `pos`).
+template <int RK>
+__device__ inline uint64_t key_at(const uint64_t (&v)[RK], int pos) {
+    uint64_t k = v[0];
+#pragma unroll
+    for (int r = 1; r < RK; ++r) k = (pos % RK == r) ? v[r] : k;
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)k, pos / RK);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(k >> 32), pos / RK);
+    return ((uint64_t)hi << 32) | lo;
+}
+
+// ------------------------------------------------------------------------------------------------------------
+// Selection by threshold (num_keys <= 64*RH, candidates <= 64*RC): the same result as the group scan above, for the
+// sizes where a whole list fits the wave's registers (R keys per lane).
+//   1. a score tau that at least K and at most CAP keys reach (CAP: the slots that are sorted), found bit by bit from the top (per
+//      bit one compare per register, the counts come from the ballots on the scalar unit): any such tau will do, so the search
+//      ends after 3 to 9 of the 32 bits, where the exact K-th largest score would take about 22;
+//   2. the keys at or above tau go to slots in LDS (positions from ballot prefix counts);
+//   3. one bitonic sort of the slots on the 64-bit keys; the first K are the result.
+// List order is key index order for a half (position p = r*64 + lane), so ties at the cut go to the lowest index there; among
+// candidate sums tied at the cut the earlier candidate (lower rank in half 0) is taken: where the sorted keys show such a tie, or
+// more than CAP keys tie with the K-th, the keys above that score and then the equal ones in list order are taken again.
+// Up to 32 experts per token (SMALL) CAP is 32 and one sort orders both halves, 32 lanes each.
+// Bound by instruction issue, 4 to 8 tokens per SIMD: at 32768 tokens, 128 keys, 16 experts the kernel took 92 us with the exact
+// search and three 64-lane sorts, now 36; 128 tokens or fewer, 32 experts: 10.3 -> 7.1; 4096 tokens, 64 experts: 16 -> 12.5.
+// ------------------------------------------------------------------------------------------------------------
+template <int CTRL> __device__ inline uint32_t dpp_max_step(uint32_t v) {      // lanes without a source read 0
+    const uint32_t o = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xF, 0xF, true);
+    return v > o ? v : o;
+}
+__device__ inline uint32_t wave_max_u32(uint32_t v) {
+    v = dpp_max_step<0xB1>(v);       // lane ^ 1
+    v = dpp_max_step<0x4E>(v);       // lane ^ 2
+    v = dpp_max_step<0x141>(v);      // mirrored in 8 lanes
+    v = dpp_max_step<0x140>(v);      // mirrored in 16 lanes
+    v = dpp_max_step<0x142>(v);      // lane 15 of a row into the next row
+    v = dpp_max_step<0x143>(v);      // lane 31 into rows 2 and 3
+    return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
+}
+// RK = registers whose 64 * RK entries cover at least k: their smallest score bounds the K-th largest from below (k entries are at
+// least that large), the largest score of the list bounds it from above, and tau shares the leading bits the two bounds
+// share - the search starts below them.  A padding entry (key 0) among those registers just gives the bound 0.
+// Ends at the first tau that at most `cap` keys reach, or at the exact K-th largest score.  LOW: low bits that every score of the
+// list shares with its sign (those a 16-bit type does not have); ties are common there and would run the search through them.
+template <int R, int RK, int LOW>
+__device__ inline uint32_t selecting_score(const uint64_t (&key)[R], int k, int cap) {
+    uint32_t hi = 0u, lo_inv = 0u;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const uint32_t s = (uint32_t)(key[r] >> 32);
+        hi = hi > s ? hi : s;
+        if (r < RK) lo_inv = lo_inv > ~s ? lo_inv : ~s;        // max of the complements = complement of the min
+    }
+    hi = wave_max_u32(hi);
+    const uint32_t lo = ~wave_max_u32(lo_inv);
+    const int bits = 32 - __builtin_clz((hi ^ lo) | 1u);         // low bits in which the bounds may differ
+    uint32_t tau = bits >= 32 ? 0u : (hi >> bits) << bits;
+    for (int bit = bits - 1; bit >= LOW; --bit) {
+        const uint32_t trial = tau | (1u << bit);
+        int count = 0;
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+            count += __builtin_popcountll(__builtin_amdgcn_ballot_w64((uint32_t)(key[r] >> 32) >= trial));
+        tau = count >= k ? trial : tau;
+        if (count >= k && count <= cap) break;
+    }
+    if constexpr (LOW > 0) {                                     // make tau a score: the low bits of a negative one are ones
+        if (!(tau >> 31)) tau |= (1u << LOW) - 1u;
+    }
+    return tau;
+}
+
+__device__ inline int lanes_below(uint64_t mask) {
+    return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
+}
+
+// The keys above tau, then those equal to it in list order, until k are taken.
+template <int R>
+__device__ inline void collect_exactly(const uint64_t (&key)[R], uint32_t tau, int k, int cap, uint64_t* slots, int lane) {
+    int base = 0;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const bool above = (uint32_t)(key[r] >> 32) > tau;
+        const uint64_t m = __builtin_amdgcn_ballot_w64(above);
+        if (above) slots[base + lanes_below(m)] = key[r];
+        base += __builtin_popcountll(m);
+    }
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const bool equal = (uint32_t)(key[r] >> 32) == tau;
+        const uint64_t m = __builtin_amdgcn_ballot_w64(equal);
+        const int pos = base + lanes_below(m);
+        if (equal && pos < k) slots[pos] = key[r];
+        base += __builtin_popcountll(m);
+    }
+    for (int p = k + lane; p < cap; p += kWave) slots[p] = 0ull;
+}
+
+// At least k of the list's keys, all that reach a common score (or exactly k of them), into slots[0 .. cap), the rest of them 0;
+// cap wave-private LDS entries.  n: keys in the list; unused entries hold key 0 (below every score).
+template <int R, int RK, int LOW>
+__device__ inline void collect_top(const uint64_t (&key)[R], int n, int k, int cap, uint64_t* slots, int lane) {
+    const uint32_t tau = n <= cap ? 1u : selecting_score<R, RK, LOW>(key, k, cap);
+    uint64_t m[R];
+    int total = 0;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        m[r] = __builtin_amdgcn_ballot_w64((uint32_t)(key[r] >> 32) >= tau);
+        total += __builtin_popcountll(m[r]);
+    }
+    if (total > cap) {                    // more ties with the k-th score than there are slots
+        collect_exactly<R>(key, tau, k, cap, slots, lane);
+        return;
+    }
+    int base = 0;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        if ((m[r] >> lane) & 1) slots[base + lanes_below(m[r])] = key[r];
+        base += __builtin_popcountll(m[r]);
+    }
+    for (int p = base + lane; p < cap; p += kWave) slots[p] = 0ull;
+}
+
+template <int RK, bool SMALL>
+__device__ inline void sort_slots(const uint64_t* slots, uint64_t (&best)[RK], int lane) {
+    __builtin_amdgcn_wave_barrier();      // LDS operations of one wave complete in order; keep the compiler from moving them
+#pragma unroll
+    for (int r = 0; r < RK; ++r) best[r] = slots[lane * RK + r];
+    __builtin_amdgcn_wave_barrier();
+    if constexpr (SMALL) bitonic_sort_blocks<32>(best[0], lane);
+    else bitonic_sort<RK, true>(best, lane);
+}
+
+// The candidate pairs (rank in half 0) | (rank in half 1) << 8, listed by rank in half 0: the list depends on top_k only,
+// so the host writes it and it travels as a kernel argument (at most 64 * 11 entries for top_k <= 128).
+constexpr int kSelectMaxCand = 11 * kWave;
+struct CandidateTable { uint16_t pair[kSelectMaxCand]; };
+
+// ... and what a launch needs with it: top_k <= 128.
+inline int candidate_table(int top_k, CandidateTable& table) {
+    int c = 0;
+    for (int i = 0; i < top_k; ++i)
+        for (int j = 0; j < top_k / (i + 1); ++j) table.pair[c++] = (uint16_t)(i | (j << 8));
+    const int used = c;
+    for (; c < kSelectMaxCand; ++c) table.pair[c] = 0;
+    return used;
+}
+
+// WAVES waves per workgroup, a token each; PAIRED: two waves per token (one launch round of few tokens), one per half, the first of
+// them going on with the candidates.
+template <typename T, typename TG, int RK, int RH, int RC, bool FROM_LOGITS, bool SMALL, int WAVES, bool PAIRED>
+__device__ __forceinline__ void router_select_tokens(
+    const T* __restrict__ lp, int64_t num_tokens, int nk, int top_k, int num_cand, T* __restrict__ scores,
+    int64_t* __restrict__ indices, TG* __restrict__ gates, int norm_topk_prob, uint32_t* __restrict__ row_offsets,
+    uint32_t row_bytes, const CandidateTable& table, int block, int blocks) {
+    constexpr int KP = RK * kWave;
+    constexpr int LOW = sizeof(T) == 4 ? 0 : __is_same(T, bf16_t) ? 16 : 13;      // fp32 bits below the type's mantissa
+    constexpr int CAP = SMALL ? kWave / 2 : KP;
+    static_assert(RC * kWave <= kSelectMaxCand, "candidate table");
+    static_assert(!SMALL || RK == 1, "one key per lane");
+    __shared__ uint16_t cand[RC * kWave];
+    constexpr int TOKENS = PAIRED ? WAVES / 2 : WAVES;
+    __shared__ float half_score[TOKENS][2][KP];
+    __shared__ uint32_t half_index[TOKENS][2][KP];
+    __shared__ uint64_t slot[WAVES][KP];
+
+    for (int i = (int)threadIdx.x; i < RC * kWave; i += (int)blockDim.x) cand[i] = table.pair[i];
+    __syncthreads();
+    const int lane = lane_id();
+    const int wave = (int)(threadIdx.x >> 6);
+    const int mine = PAIRED ? wave >> 1 : wave;          // the wave's token of the workgroup
+    const int64_t tokens_total = (int64_t)blocks * TOKENS;
+    const int64_t rounds = PAIRED ? 1 : (num_tokens + tokens_total - 1) / tokens_total;
+
+    for (int64_t round = 0; round < rounds; ++round) {
+        const int64_t token = round * tokens_total + (int64_t)block * TOKENS + mine;
+        if (!PAIRED && token >= num_tokens) continue;    // nothing below synchronises across waves
+#pragma unroll
+        for (int h = PAIRED ? __builtin_amdgcn_readfirstlane(wave & 1) : 0; h < 2; ++h) {
+            if (PAIRED && token >= num_tokens) break;
+            const T* row = FROM_LOGITS ? lp + (token * 2 + h) * nk : lp + ((int64_t)h * num_tokens + token) * nk;
+            float v[RH];
+#pragma unroll
+            for (int r = 0; r < RH; ++r) {
+                const int p = r * kWave + lane;
+                v[r] = p < nk ? Elem<T>::to_f32(row[p]) : 0.0f;
+            }
+            float shift = 0.0f, lse = 0.0f;
+            if (FROM_LOGITS) {
+                float mx = -INFINITY;
+#pragma unroll
+                for (int r = 0; r < RH; ++r)
+                    if (r * kWave + lane < nk) mx = fmaxf(mx, v[r]);
+                mx = wave_max(mx);
+                float se = 0.0f;
+#pragma unroll
+                for (int r = 0; r < RH; ++r)
+                    if (r * kWave + lane < nk) se += expf(v[r] - mx);
+                shift = mx;
+                lse = logf(wave_sum(se));
+            }
+            uint64_t key[RH];
+#pragma unroll
+            for (int r = 0; r < RH; ++r) {
+                const int p = r * kWave + lane;
+                key[r] = p < nk ? make_key(FROM_LOGITS ? (v[r] - shift) - lse : v[r], (uint32_t)p) : 0ull;
+            }
+            // the candidates look up ranks below top_k (entries past nk stay key 0)
+            collect_top<RH, RK, FROM_LOGITS ? 0 : LOW>(key, nk, top_k < nk ? top_k : nk, CAP, slot[wave] + (SMALL && !PAIRED ? h * CAP : 0), lane);
+            if (!SMALL || PAIRED || h == 1) {
+                uint64_t best[RK];
+                sort_slots<RK, SMALL>(slot[wave], best, lane);
+#pragma unroll
+                for (int r = 0; r < RK; ++r) {
+                    const int which = SMALL && !PAIRED ? lane / CAP : h, rank = SMALL && !PAIRED ? lane % CAP : lane * RK + r;
+                    half_score[mine][which][rank] = key_score(best[r]);
+                    half_index[mine][which][rank] = key_index(best[r]);
+                }
+            }
+            if (PAIRED) break;
+        }
+        if (PAIRED) {
+            __syncthreads();
+            if ((wave & 1) != 0 || token >= num_tokens) return;
+        }
+        __builtin_amdgcn_wave_barrier();
+        uint64_t ckey[RC];
+#pragma unroll
+        for (int r = 0; r < RC; ++r) {
+            const int c = r * kWave + lane;
+            ckey[r] = 0ull;
+            if (c < num_cand) {
+                const int ij = cand[c];
+                const int i = ij & 0xff, j = ij >> 8;
+                const float s = round_through<T>(half_score[mine][0][i] + half_score[mine][1][j]);
+                const uint32_t flat = half_index[mine][0][i] * (uint32_t)nk + half_index[mine][1][j];
+                ckey[r] = make_key(s, flat);
+            }
+        }
+        uint64_t best[RK];
+        if (SMALL && lane >= CAP) slot[wave][lane] = 0ull;                 // the sort's other block
+        collect_top<RC, RK, LOW>(ckey, num_cand, top_k, CAP, slot[wave], lane);
+        sort_slots<RK, SMALL>(slot[wave], best, lane);
+        {
+            // a tie across the cut: the first candidates in list order among the equal sums are the ones to keep
+            const uint32_t cut = (uint32_t)(key_at<RK>(best, top_k - 1) >> 32);
+            if (top_k < CAP && cut == (uint32_t)(key_at<RK>(best, top_k) >> 32)) {
+                collect_exactly<RC>(ckey, cut, top_k, CAP, slot[wave], lane);
+                sort_slots<RK, SMALL>(slot[wave], best, lane);
+            }
+        }
+        float e[RK];
+        float total = 0.0f;
+#pragma unroll
+        for (int r = 0; r < RK; ++r) {
+            const int p = lane * RK + r;
+            e[r] = p < top_k ? expf(key_score(best[r])) : 0.0f;
+            total += e[r];
+        }
+        if (gates != nullptr && norm_topk_prob) total = wave_sum(total);
+#pragma unroll
+        for (int r = 0; r < RK; ++r) {
+            const int p = lane * RK + r;
+            if (p < top_k) {
+                const int64_t o = token * top_k + p;
+                scores[o] = Elem<T>::from_f32(key_score(best[r]));
+                indices[o] = (int64_t)key_index(best[r]);
+                if (row_offsets != nullptr) row_offsets[o] = key_index(best[r]) * row_bytes;
+                if (gates != nullptr) gates[o] = Elem<TG>::from_f32(norm_topk_prob ? e[r] / total : e[r]);
+            }
+        }
+    }
+}
+
+}  // namespace
+}  // namespace fmoe

@@ -191,6 +191,39 @@ def test_single_call_block_equals_the_three_stage_calls(dtype, T, H, I, E, K, tr
     assert torch.equal(idx, idx_ref) and torch.equal(gates, gates_ref) and torch.equal(y3.view_as(y1), y1)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("T,H,I,E,K", [
+    # the three-launch forward of few tokens: one token; 16 | 17 rows; each kind of gate/up tile with remainders, k split over
+    # workgroups, 32 x 32 down tiles; both selections and more than 128 keys; the most tokens, and one more than it takes
+    (1, 8, 8, 9, 1), (16, 264, 520, 1200, 33), (17, 1000, 2664, 10000, 24), (64, 1024, 4096, 17000, 64), (255, 520, 1032, 400, 17),
+    (256, 1032, 1040, 5000, 5), (257, 264, 520, 1024, 8), (40, 2048, 5464, 2500, 50),
+])
+def test_block_of_few_tokens_in_evaluation_mode(dtype, T, H, I, E, K):
+    from flash_moe.ops.hip.flash_block import block_forward
+
+    m, w = build(H, I, E, K, True, dtype, seed=T)
+    g = torch.Generator().manual_seed(T + H)
+    m.router_norm.running_mean.copy_(torch.randn(H, generator=g) * 0.1)
+    m.router_norm.running_var.copy_(torch.rand(H, generator=g) + 0.5)
+    m.eval()
+    x = torch.randn(1, T, H, generator=g).to(dtype).cuda()
+    y, logits = m(x)
+    y2, _, idx, gates = block_forward(x.view(T, H), m.gate_proj.weight, m.up_proj.weight, m.down_proj.weight,
+                                            m.router_gate.weight, m.router_norm, m.down_embed.weight, m.up_embed.weight,
+                                            m.num_keys, K, True, return_routing=True)
+    staged, staged_logits = m.forward_staged(x)
+    _, _, idx_staged, gates_staged = m.route(x.view(T, H))
+    assert torch.equal(y, y2.view_as(y))
+    assert torch.equal(logits, staged_logits) and torch.equal(idx, idx_staged) and torch.equal(gates, gates_staged)
+    assert rel_fro(y, staged.cpu()) < {torch.float32: 3e-6, torch.bfloat16: 3e-3, torch.float16: 4e-4}[dtype]
+    # the two halves of the output in float64
+    x64, idx, gates = x.view(T, H).double().cpu(), idx.cpu(), gates.double().cpu()
+    experts = orc.expert_forward(x64, w.down_embed.double(), w.up_embed.double(), idx, gates)
+    hidden = torch.nn.functional.silu(x64 @ w.gate_proj.double().t()) * (x64 @ w.up_proj.double().t())
+    want = experts + hidden.to(dtype).double() @ w.down_proj.double().t()
+    assert rel_fro(y.view(T, H), want) < {torch.float32: 3e-6, torch.bfloat16: 6e-3, torch.float16: 8e-4}[dtype]
+
+
 def test_single_call_block_without_routed_experts():
     """num_experts_per_tok = 0: the block is the shared MLP alone."""
     from flash_moe.ops.hip.flash_mlp import mlp_forward
