@@ -9,7 +9,7 @@ namespace {
 
 struct BlockPlan {
     size_t off_router, off_logits32, off_scores, off_indices, off_gates, off_expert, off_act, off_experts_out, off_sums, bytes;
-    bool small;      // evaluation mode takes the three launches of fmoe_small.hip
+    SmallPlan small;
 };
 
 BlockPlan plan_block(int64_t T_, int H, int I, int nk, int64_t E, int K, int dtype) {
@@ -25,8 +25,8 @@ BlockPlan plan_block(int64_t T_, int H, int I, int nk, int64_t E, int K, int dty
     p.off_expert = take(fmoe_expert_workspace_bytes(T_, H, E, K, dtype));
     p.off_act = take(fmoe_mlp_workspace_bytes(T_, H, I, dtype));
     p.off_experts_out = take((size_t)T_ * H * elt);
-    p.small = block_small_usable(T_, H, I, nk, E, K, dtype);
-    p.off_sums = take(p.small ? block_small_sums_bytes(T_, H, I, dtype) : 0);
+    p.small = plan_small(T_, H, I, nk, E, K, dtype);
+    p.off_sums = take(p.small.sums_bytes);
     p.bytes = o;
     return p;
 }
@@ -147,12 +147,6 @@ int block_forward_impl(const char* who, const void* x, const void* gate_proj_w, 
     void* experts = ws + p.off_experts_out;
     const size_t elt = dtype_size(dtype);
 
-    if (p.small && !training && saved == nullptr && running_mean && running_var && dtype_ok(stats_dtype))
-        return block_small_forward(x, gate_proj_w, up_proj_w, down_proj_w, router_gate_w, down_embed, up_embed, running_mean, running_var,
-                                   stats_dtype, eps, num_tokens, hidden, intermediate, num_experts, num_keys, top_k, dtype, norm_topk_prob,
-                                   out, router_logits, logits32, scores, indices, gates, act, (float*)(ws + p.off_router),
-                                   (float*)(ws + p.off_sums), s);
-
     const bool slices = expert_slices_usable(num_tokens, hidden, num_experts, top_k, dtype);
     uint32_t* offsets = slices ? expert_workspace_offsets(expert_ws) : nullptr;
     float* expert_scores = nullptr;
@@ -161,11 +155,36 @@ int block_forward_impl(const char* who, const void* x, const void* gate_proj_w, 
         offsets = kept.off32;
         expert_scores = kept.scores;
     }
-    int rc = router_forward_impl(x, router_gate_w, running_mean, running_var, num_batches_tracked, stats_dtype, training,
-                                 momentum, eps, num_tokens, hidden, num_keys, top_k, dtype, norm_topk_prob, router_logits,
-                                 logits32, scores, indices, gates, offsets,
-                                 (uint32_t)(hidden * elt), ws + p.off_router, p.off_logits32 - p.off_router, s, 0, 0, stats);
+    auto gate_up = [&]() {
+        return products ? fmoe_mlp_gate_up_save(x, gate_proj_w, up_proj_w, num_tokens, hidden, intermediate, dtype, act, products, stream)
+                        : fmoe_mlp_gate_up(x, gate_proj_w, up_proj_w, num_tokens, hidden, intermediate, dtype, act, stream);
+    };
+    // The statistics a call lacks, and the shapes the router refuses, are reported by the router's own entry
+    const bool up_beside = p.small.gate_and_up && dtype_ok(stats_dtype) &&
+                           (training ? num_tokens > 1 : running_mean != nullptr && running_var != nullptr);
+    const bool down_beside = p.small.select_and_down;
+    int rc;
+    if (up_beside) {
+        float* scratch = (float*)(ws + p.off_router);
+        rc = small_gate_and_up(x, gate_proj_w, up_proj_w, router_gate_w, running_mean, running_var, num_batches_tracked, stats_dtype, training,
+                               momentum, eps, num_tokens, hidden, intermediate, num_keys, dtype, router_logits, logits32, act, products,
+                               scratch, stats ? stats : scratch + router_block_stats_bytes(hidden) / sizeof(float), s);
+        if (rc == FMOE_OK && !down_beside && top_k > 0)
+            rc = launch_router_from_logits(logits32, num_tokens, num_keys, top_k, scores, indices, gates, dtype, norm_topk_prob, offsets,
+                                           (uint32_t)(hidden * elt), s);
+    } else {
+        rc = router_forward_impl(x, router_gate_w, running_mean, running_var, num_batches_tracked, stats_dtype, training, momentum, eps,
+                                 num_tokens, hidden, num_keys, down_beside ? 0 : top_k, dtype, norm_topk_prob, router_logits, logits32, scores,
+                                 indices, gates, offsets, (uint32_t)(hidden * elt), ws + p.off_router, p.off_logits32 - p.off_router, s, 0, 0,
+                                 stats);
+    }
     if (rc) return rc;
+    if (down_beside) {
+        if (!up_beside)
+            if ((rc = gate_up())) return rc;
+        return small_select_down_experts(x, down_proj_w, down_embed, up_embed, num_tokens, hidden, intermediate, num_experts, num_keys, top_k,
+                                         dtype, norm_topk_prob, out, logits32, scores, indices, gates, act, (float*)(ws + p.off_sums), s);
+    }
     const void* residual = nullptr;
     if (top_k > 0) {
         if (slices)
@@ -181,9 +200,8 @@ int block_forward_impl(const char* who, const void* x, const void* gate_proj_w, 
         if (rc) return rc;
         residual = experts;
     }
-    rc = products ? fmoe_mlp_gate_up_save(x, gate_proj_w, up_proj_w, num_tokens, hidden, intermediate, dtype, act, products, stream)
-                  : fmoe_mlp_gate_up(x, gate_proj_w, up_proj_w, num_tokens, hidden, intermediate, dtype, act, stream);
-    if (rc) return rc;
+    if (!up_beside)
+        if ((rc = gate_up())) return rc;
     return fmoe_mlp_down(act, down_proj_w, num_tokens, hidden, intermediate, dtype, residual, out, stream);
 }
 

@@ -51,16 +51,27 @@ int launch_router_from_logits(const float* logits, int64_t num_tokens, int num_k
 // Whether a top-k kernel exists for these extents: top_k <= 256 with any num_keys, or top_k <= 1024 with num_keys <= 8192.
 bool router_topk_supported(int num_keys, int top_k);
 
-// The whole block for up to kSmallMaxTokens tokens in evaluation mode in three launches (fmoe_small.hip); usable says whether these
-// extents have it, sums_bytes what `sums` needs.  mean_rstd: [2][H] scratch.
-constexpr int kSmallMaxTokens = 256, kSmallMaxSlices = 4;
-bool block_small_usable(int64_t num_tokens, int hidden, int intermediate, int num_keys, int64_t num_experts, int top_k, int dtype);
-size_t block_small_sums_bytes(int64_t num_tokens, int hidden, int intermediate, int dtype);
-int block_small_forward(const void* x, const void* gate_proj_w, const void* up_proj_w, const void* down_proj_w, const void* router_gate_w,
-                        const void* down_embed, const void* up_embed, void* running_mean, void* running_var, int stats_dtype, float eps,
-                        int64_t num_tokens, int hidden, int intermediate, int64_t num_experts, int num_keys, int top_k, int dtype,
-                        int norm_topk_prob, void* out, void* router_logits, float* logits32, float* scores, int64_t* indices, void* gates,
-                        void* act, float* mean_rstd, float* sums, hipStream_t stream);
+// Stages of the block that share a launch while there are few tokens (fmoe_small.hip), and which of them these extents have.
+//   gate_and_up: everything up to the router logits, and act (products: NULL, or where the two products of the MLP are kept);
+//     scratch: router_block_stats_bytes(hidden), mean_rstd: [2][H].
+//   select_and_down: the rest, from logits and act to out; sums: sums_bytes of scratch.
+constexpr int kSmallMaxTokens = 2048, kSmallMaxSlices = 4;
+struct SmallPlan {
+    bool gate_and_up, select_and_down;
+    size_t sums_bytes;
+};
+SmallPlan plan_small(int64_t num_tokens, int hidden, int intermediate, int num_keys, int64_t num_experts, int top_k, int dtype);
+int small_gate_and_up(const void* x, const void* gate_proj_w, const void* up_proj_w, const void* router_gate_w, void* running_mean,
+                      void* running_var, int64_t* num_batches_tracked, int stats_dtype, int training, float momentum, float eps,
+                      int64_t num_tokens, int hidden, int intermediate, int num_keys, int dtype, void* router_logits, float* logits32,
+                      void* act, void* products, float* scratch, float* mean_rstd, hipStream_t stream);
+int small_select_down_experts(const void* x, const void* down_proj_w, const void* down_embed, const void* up_embed, int64_t num_tokens,
+                              int hidden, int intermediate, int64_t num_experts, int num_keys, int top_k, int dtype, int norm_topk_prob,
+                              void* out, const float* logits32, float* scores, int64_t* indices, void* gates, const void* act,
+                              float* sums, hipStream_t stream);
+size_t router_block_stats_bytes(int hidden);
+int router_block_stats(const void* x, int64_t num_tokens, int hidden, int dtype, float* partial, int* row_blocks, int* rows_per_block,
+                       hipStream_t stream);
 // The row schedule of the routed experts: whether these extents take it, and with `slices` fp32 planes [T,H] added to its result
 // (few tokens, at most 2048 columns).
 bool expert_rows_chosen(int64_t num_tokens, int hidden, int64_t num_experts, int top_k, int dtype);

@@ -49,7 +49,7 @@ template <typename T> __device__ inline void store4(T* p, f32x4_t v) {
 // WAVES = 1: one wave per token, kWavesPerBlock tokens per workgroup.  WAVES > 1 (few tokens): the workgroup's waves share one
 // token, wave w taking pairs w*P .. w*P+P-1, (w+WAVES)*P .. of it (P = pairs in flight), and their partial rows are added in wave
 // order through LDS: dependency chains shorter by WAVES when there are not enough tokens to fill the chip with one wave each.
-// ADDED (at most WAVES * 256 columns): `slices` planes [T, H] of fp32 sums are added to the rounded result, as the residual of the down product would be.
+// ADDED: `slices` planes [T, H] of fp32 sums are added to the rounded result, as the residual of the down product would be.
 template <typename T, typename TG, int NCH, int ACT, int WAVES, bool ADDED = false>
 __global__ __launch_bounds__((WAVES > 1 ? WAVES : kWavesPerBlock) * kWave) void expert_token_kernel(
     const T* __restrict__ x, const T* __restrict__ down, const T* __restrict__ up,
@@ -83,14 +83,19 @@ __global__ __launch_bounds__((WAVES > 1 ? WAVES : kWavesPerBlock) * kWave) void 
 #pragma unroll
         for (int v = 0; v < V; ++v) acc[c][v] = 0.0f;
 
-    f32x4_t added[ADDED ? kSmallMaxSlices : 1];
-    if constexpr (ADDED) {
-        const int at = (int)threadIdx.x * 4;
+    // the planes of the thread's first columns are requested before the rows
+    auto planes_at = [&](int at) {
+        f32x4_t v[kSmallMaxSlices];
 #pragma unroll
         for (int s = 0; s < kSmallMaxSlices; ++s)
-            added[s] = s < slices && at < hidden ? *reinterpret_cast<const f32x4_t*>(planes + (s * num_tokens + token) * hidden + at)
-                                                 : f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-    }
+            v[s] = s < slices && at < hidden ? *reinterpret_cast<const f32x4_t*>(planes + (s * num_tokens + token) * hidden + at)
+                                             : f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int s = 1; s < kSmallMaxSlices; ++s) v[0] += v[s];
+        return v[0];
+    };
+    f32x4_t added = {0.0f, 0.0f, 0.0f, 0.0f};
+    if constexpr (ADDED) added = planes_at((int)threadIdx.x * 4);
 
     const int64_t* my_idx = indices + token * top_k;
     const TG* my_gate = gates + token * top_k;
@@ -158,11 +163,9 @@ __global__ __launch_bounds__((WAVES > 1 ? WAVES : kWavesPerBlock) * kWave) void 
 #pragma unroll
             for (int w = 1; w < WAVES; ++w) sum += *reinterpret_cast<const f32x4_t*>(&partial_rows[w * ROW + at]);
             if constexpr (ADDED) {
-                f32x4_t mlp = added[0];
+                if (at != (int)threadIdx.x * 4) added = planes_at(at);
 #pragma unroll
-                for (int s = 1; s < kSmallMaxSlices; ++s) mlp += added[s];
-#pragma unroll
-                for (int i = 0; i < 4; ++i) sum[i] = mlp[i] + round_through<T>(sum[i]);
+                for (int i = 0; i < 4; ++i) sum[i] = added[i] + round_through<T>(sum[i]);
             }
             store4(out + token * hidden + at, sum);
         }
@@ -226,7 +229,12 @@ void launch_expert_rows_added(const void* x, const void* down, const void* up, c
 #define FMOE_LAUNCH_ADDED(N, W)                                                                                                      \
     hipLaunchKernelGGL((expert_token_kernel<T, T, N, kActSilu, W, true>), dim3((unsigned)T_), dim3(W * kWave), 0, stream, (const T*)x, \
                        (const T*)down, (const T*)up, indices, (const T*)gates, (T*)out, T_, H, E, K, planes, slices)
-    if (nch <= 1) FMOE_LAUNCH_ADDED(1, 16);
+    if (T_ > chip_info().cus) {
+        if (nch <= 1) FMOE_LAUNCH_ADDED(1, 4);
+        else if (nch <= 2) FMOE_LAUNCH_ADDED(2, 4);
+        else if (nch <= 4) FMOE_LAUNCH_ADDED(4, 4);
+        else if constexpr (sizeof(T) == 4) FMOE_LAUNCH_ADDED(8, 4);
+    } else if (nch <= 1) FMOE_LAUNCH_ADDED(1, 16);
     else if (nch <= 2) FMOE_LAUNCH_ADDED(2, 16);
     else if (nch <= 4) FMOE_LAUNCH_ADDED(4, 16);
     else if constexpr (sizeof(T) == 4) FMOE_LAUNCH_ADDED(8, 8);

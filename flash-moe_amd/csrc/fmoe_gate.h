@@ -167,15 +167,18 @@ constexpr int kGateWaves = 8;
 constexpr int kGateStagedK = 4096;       // 8 bytes of LDS per column
 constexpr uint32_t kGateOutOfRange = 0x80000000u;
 
-template <typename T, int MT, int NT, bool STAGED>
+// lds: kGateLds bytes.
+template <int MT, int NT> constexpr int kGateLds = kGateWaves * (MT * NT < 8 ? MT * NT : 8) * kWave * 16;
+// WAVES of the kernel: with half of kGateWaves each takes the lines of two, one after the other - the same sums.
+template <typename T, int MT, int NT, bool STAGED, int WAVES = kGateWaves>
 __device__ __forceinline__ void router_gate_splitk_tile(
     const T* __restrict__ x, const T* __restrict__ w, const GateStats& st, float* __restrict__ logits32, T* __restrict__ logits, int M, int N,
-    int K_full, int tiles_m, int tiles_n, int split, int xcds, float* stats, int block, int blocks) {
+    int K_full, int tiles_m, int tiles_n, int split, int xcds, void* lds, float* stats, int block, int blocks) {
     constexpr int BM = 16 * MT, BN = 16 * NT, F = MT * NT, V = Elem<T>::kVec;
     constexpr int kStep = 64 / (int)sizeof(T);                   // k values of a step; two steps are a line
     constexpr int kAhead = MT + NT <= 3 ? 8 : 4;
     constexpr int kRound = F < 8 ? F : 8;                        // fragments exchanged at a time
-    __shared__ __attribute__((aligned(16))) f32x4_t sums[kGateWaves][kRound][kWave];
+    f32x4_t(*sums)[kRound][kWave] = reinterpret_cast<f32x4_t(*)[kRound][kWave]>(lds);      // [kGateWaves]
     const int tid = (int)threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     // XCD b % xcds takes a contiguous run of the tiles, all columns of a row first: its L2 holds the run's part of x only
@@ -198,10 +201,14 @@ __device__ __forceinline__ void router_gate_splitk_tile(
     for (int i = 0; i < MT; ++i) a_off[i] = (uint32_t)((i * 16 + frow) * K_full) * (uint32_t)sizeof(T) + (uint32_t)piece * 16u;
 #pragma unroll
     for (int j = 0; j < NT; ++j) b_off[j] = (uint32_t)((j * 16 + frow) * K) * (uint32_t)sizeof(T) + (uint32_t)piece * 16u;
-    // step u of this wave: half u % 2 of its line u / 2; lines are numbered over all of k, whichever half the tile scores
     const int lines = (K + 2 * kStep - 1) / (2 * kStep);
-    const int first_line = (wave + kGateWaves - (k_off / (2 * kStep)) % kGateWaves) % kGateWaves;
-    const int steps = first_line < lines ? 2 * ((lines - first_line + kGateWaves - 1) / kGateWaves) : 0;
+    // step u of part `part` of k: half u % 2 of its line u / 2; lines are numbered over all of k, whichever half the tile scores
+    int first_line = 0, steps = 0;
+    auto set_part = [&](int part) {
+        first_line = (part + kGateWaves - (k_off / (2 * kStep)) % kGateWaves) % kGateWaves;
+        steps = first_line < lines ? 2 * ((lines - first_line + kGateWaves - 1) / kGateWaves) : 0;
+    };
+    set_part(wave);
     u32x4_t fa[kAhead][MT], fb[kAhead][NT];
     auto k_of = [&](int u) { return ((first_line + (u >> 1) * kGateWaves) * 2 + (u & 1)) * kStep; };
     auto load = [&](int u, u32x4_t (&a)[MT], u32x4_t (&b)[NT]) {
@@ -214,11 +221,6 @@ __device__ __forceinline__ void router_gate_splitk_tile(
         for (int j = 0; j < NT; ++j)
             b[j] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(br, (int)(drop ? kGateOutOfRange : b_off[j]), k0 * (int)sizeof(T), 0));
     };
-    f32x4_t acc[MT][NT];
-#pragma unroll
-    for (int i = 0; i < MT; ++i)
-#pragma unroll
-        for (int j = 0; j < NT; ++j) acc[i][j] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
     for (int u = 0; u < kAhead; ++u) load(u, fa[u], fb[u]);
     const int kpad = (K + 2 * kStep - 1) / (2 * kStep) * (2 * kStep);
@@ -226,48 +228,66 @@ __device__ __forceinline__ void router_gate_splitk_tile(
         stage_stats<1>(st, stats, kpad, K, K_full, k_off, tn == (k_off ? tiles_n / 2 : 0), tm, tiles_m, tile == 0);
         __syncthreads();
     }
-    for (int u0 = 0; u0 < steps; u0 += kAhead) {
+    f32x4_t acc[MT][NT];
+    auto multiply = [&]() {
 #pragma unroll
-        for (int d = 0; d < kAhead; ++d) {
-            const int u = u0 + d;
-            // steps past the end multiply zeros; their statistics are read from the last valid place
-            const int k0 = u < steps ? k_of(u) : 0;
-            float mean[V], rstd[V];
+        for (int i = 0; i < MT; ++i)
 #pragma unroll
-            for (int c = 0; c < V / 4; ++c) {
-                u32x4_t mv, rv;
-                if constexpr (STAGED) {
-                    mv = *reinterpret_cast<const u32x4_t*>(stats + k0 + piece * V + c * 4);
-                    rv = *reinterpret_cast<const u32x4_t*>(stats + kpad + k0 + piece * V + c * 4);
-                } else {
-                    const int at = (piece * V + c * 4) * 4;
-                    mv = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(sr, at, k0 * 4, 0));
-                    rv = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(sr, at, (K_full + k0) * 4, 0));
+            for (int j = 0; j < NT; ++j) acc[i][j] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+        for (int u0 = 0; u0 < steps; u0 += kAhead) {
+#pragma unroll
+            for (int d = 0; d < kAhead; ++d) {
+                const int u = u0 + d;
+                // steps past the end multiply zeros; their statistics are read from the last valid place
+                const int k0 = u < steps ? k_of(u) : 0;
+                float mean[V], rstd[V];
+#pragma unroll
+                for (int c = 0; c < V / 4; ++c) {
+                    u32x4_t mv, rv;
+                    if constexpr (STAGED) {
+                        mv = *reinterpret_cast<const u32x4_t*>(stats + k0 + piece * V + c * 4);
+                        rv = *reinterpret_cast<const u32x4_t*>(stats + kpad + k0 + piece * V + c * 4);
+                    } else {
+                        const int at = (piece * V + c * 4) * 4;
+                        mv = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(sr, at, k0 * 4, 0));
+                        rv = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(sr, at, (K_full + k0) * 4, 0));
+                    }
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) {
+                        const uint32_t mw = mv[v], rw = rv[v];
+                        mean[c * 4 + v] = __uint_as_float(mw);
+                        rstd[c * 4 + v] = __uint_as_float(rw);
+                    }
                 }
 #pragma unroll
-                for (int v = 0; v < 4; ++v) {
-                    const uint32_t mw = mv[v], rw = rv[v];
-                    mean[c * 4 + v] = __uint_as_float(mw);
-                    rstd[c * 4 + v] = __uint_as_float(rw);
+                for (int i = 0; i < MT; ++i) {
+                    const u32x4_t q = normalise16<T>(fa[d][i], mean, rstd);
+#pragma unroll
+                    for (int j = 0; j < NT; ++j) acc[i][j] = mfma16_packet<T>(q, fb[d][j], acc[i][j]);
                 }
+                load(u + kAhead, fa[d], fb[d]);
             }
-#pragma unroll
-            for (int i = 0; i < MT; ++i) {
-                const u32x4_t q = normalise16<T>(fa[d][i], mean, rstd);
-#pragma unroll
-                for (int j = 0; j < NT; ++j) acc[i][j] = mfma16_packet<T>(q, fb[d][j], acc[i][j]);
-            }
-            load(u + kAhead, fa[d], fb[d]);
         }
+    };
+    multiply();
+    static_assert(WAVES == kGateWaves || F <= kRound, "one exchange");
+#pragma unroll
+    for (int part = WAVES; part < kGateWaves; part += WAVES) {
+#pragma unroll
+        for (int f = 0; f < F; ++f) sums[part - WAVES + wave][f][lane] = acc[f / NT][f % NT];
+        set_part(part + wave);
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u) load(u, fa[u], fb[u]);
+        multiply();
     }
 #pragma unroll
     for (int f0 = 0; f0 < F; f0 += kRound) {
         if (f0 > 0) __syncthreads();
 #pragma unroll
-        for (int f = f0; f < f0 + kRound; ++f) sums[wave][f - f0][lane] = acc[f / NT][f % NT];
+        for (int f = f0; f < f0 + kRound; ++f) sums[kGateWaves - WAVES + wave][f - f0][lane] = acc[f / NT][f % NT];
         __syncthreads();
         // four rows of one column per (fragment, lane)
-        for (int q = tid; q < kRound * kWave; q += kGateWaves * kWave) {
+        for (int q = tid; q < kRound * kWave; q += WAVES * kWave) {
             const int f = f0 + (q >> 6), l = q & 63;
             f32x4_t g = sums[0][q >> 6][l];
 #pragma unroll

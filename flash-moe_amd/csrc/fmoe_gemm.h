@@ -1,5 +1,6 @@
 // Tiles of C[M,N] = A[M,K] * B[N,K]^T on the matrix cores (gfx950), the parts of kernels that form such products: the shared MLP
-// (fmoe_mlp.hip) and the launches that put a product beside other work (fmoe_small.hip).  `block` of `blocks` workgroups.
+// (fmoe_mlp.hip) and the launches that put a product beside other work (fmoe_small.hip).  `block` of `blocks` workgroups; lds: kSplitLds bytes
+// of the kernel's memory.
 #pragma once
 
 #include "fmoe_common.h"
@@ -12,12 +13,23 @@ enum Epilogue { kEpiSwiGLU = 0, kEpiPlain = 1, kEpiDual = 2, kEpiPart = 3 };   /
 template <bool B> struct Flag { static constexpr bool value = B; };
 constexpr uint32_t kOutOfRange = 0x80000000u;    // beyond every buffer descriptor here: loads give zeros, stores are dropped
 
+// The stages of a kernel's pipeline tiles.  The memory is reached by this function, not through a pointer handed down: with a pointer
+// the compiler schedules the address arithmetic of the 256 x 256 tiles differently, which costs the large products 1 to 2 %.
+template <typename T, int N> struct DmaLds {
+    __device__ __forceinline__ static T* at() {
+        __shared__ __attribute__((aligned(1024))) T stages[N];
+        return stages;
+    }
+};
+constexpr int kSplitWaves = 8;
+template <int MT, int NT, int EPI> constexpr int kSplitLds = kSplitWaves * MT * NT * (EPI == kEpiSwiGLU ? 2 : 1) * 64 * 16;
+
 // ------------------------------------------------------------------------------------------------------------
 // LDS-DMA pipelined kernel.  WAVES_M x WAVES_N waves, each (BM/WAVES_M) x (BN/WAVES_N); BKT = k extent of a stage.
 // ------------------------------------------------------------------------------------------------------------
 // FR: fragment shape (32: v_mfma_f32_32x32x16 / 32x32x2; 16: v_mfma_f32_16x16x32).  SPLIT: a k-step's A fragments are read and
 // multiplied in SPLIT parts (its B fragments stay for the whole k-step), which halves the registers the read-ahead needs.
-template <typename T, int BM, int BN, int WAVES_M, int WAVES_N, int BKT, int NSTAGE, int EPI, int PF, int FR = 32, int SPLIT = 1, bool RAGGED = false>
+template <typename T, int BM, int BN, int WAVES_M, int WAVES_N, int BKT, int NSTAGE, int EPI, int PF, int FR, int SPLIT, bool RAGGED>
 __device__ __forceinline__ void gemm_dma_tiles(
     const T* __restrict__ A, const T* __restrict__ B0, const T* __restrict__ B1, T* __restrict__ C,
     const T* __restrict__ R, int M, int N, int K, int tiles_m, int tiles_n, int xcds, int block, int blocks) {
@@ -45,7 +57,7 @@ __device__ __forceinline__ void gemm_dma_tiles(
     static_assert(EPI != kEpiSwiGLU || ((BN / 2) % ROWS_PER_IT == 0 && NF % 2 == 0), "gate/up split");
     static_assert((NSTAGE - 2) * DMA_PER_TILE < 64, "vmcnt range");
 
-    __shared__ __attribute__((aligned(1024))) T lds[NSTAGE * STAGE];
+    using Lds = DmaLds<T, NSTAGE * STAGE>;
 
     const int tid = (int)threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -153,7 +165,7 @@ __device__ __forceinline__ void gemm_dma_tiles(
     set_tile(tile);
 #pragma unroll
     for (int s = 0; s < NSTAGE - 1; ++s)
-        if (s < k_tiles) issue(s, lds + s * STAGE);
+        if (s < k_tiles) issue(s, Lds::at() + s * STAGE);
 
     // Fragments of step q+PF are read from LDS while the MFMAs of step q run (PF+1 register buffers for the A parts; B
     // fragments are read with the first part of their k-step); the read-ahead crosses k-tile boundaries, so the barrier
@@ -184,7 +196,7 @@ __device__ __forceinline__ void gemm_dma_tiles(
         if (kt + NSTAGE - 2 < k_tiles) __builtin_amdgcn_s_waitcnt(0x0070 | (kKeep & 0xF) | ((kKeep >> 4) << 14));
         else __builtin_amdgcn_s_waitcnt(0x0070);
         __builtin_amdgcn_s_barrier();
-        if (kt + NSTAGE - 1 < k_tiles) issue(kt + NSTAGE - 1, lds + ((kt + NSTAGE - 1) % NSTAGE) * STAGE);
+        if (kt + NSTAGE - 1 < k_tiles) issue(kt + NSTAGE - 1, Lds::at() + ((kt + NSTAGE - 1) % NSTAGE) * STAGE);
     };
     while (true) {
         Acc acc[MF][NF];
@@ -197,13 +209,13 @@ __device__ __forceinline__ void gemm_dma_tiles(
 
         enter_k_tile(0);
 #pragma unroll
-        for (int s = 0; s < PF; ++s) read_frags(reinterpret_cast<const char*>(lds), s, fa[s % RING], fb[b_slot(s)]);
+        for (int s = 0; s < PF; ++s) read_frags(reinterpret_cast<const char*>(Lds::at()), s, fa[s % RING], fb[b_slot(s)]);
         // the last k-tile has no successor to read ahead into: it is a separate copy of the body, so that no branch
         // merges a path with reads in flight into the MFMA sequence
         auto k_tile_body = [&](int kt, auto last_tag) {
             constexpr bool kLast = decltype(last_tag)::value;
-            const char* stage = reinterpret_cast<const char*>(lds + (kt % NSTAGE) * STAGE);
-            const char* next_stage = reinterpret_cast<const char*>(lds + ((kt + 1) % NSTAGE) * STAGE);
+            const char* stage = reinterpret_cast<const char*>(Lds::at() + (kt % NSTAGE) * STAGE);
+            const char* next_stage = reinterpret_cast<const char*>(Lds::at() + ((kt + 1) % NSTAGE) * STAGE);
 #pragma unroll
             for (int q = 0; q < SPK; ++q) {
                 const int nxt = q + PF;
@@ -247,7 +259,7 @@ __device__ __forceinline__ void gemm_dma_tiles(
             __builtin_amdgcn_s_barrier();     // every wave has consumed its reads of the last stage
 #pragma unroll
             for (int s = 0; s < NSTAGE - 1; ++s)
-                if (s < k_tiles) issue(s, lds + s * STAGE);
+                if (s < k_tiles) issue(s, Lds::at() + s * STAGE);
         }
 
         // D fragment layout (both shapes): lane l, register v holds
@@ -302,6 +314,21 @@ __device__ __forceinline__ void gemm_dma_tiles(
 #pragma unroll
                     for (int v = 0; v < NV; ++v)
                         store_to(c_rsrc, lane_at(j, lane_bytes0), elem_at(i, j, v) * (int)sizeof(T), silu(acc[i][j][v]) * acc[i][j + NF / 2][v]);
+        } else if (EPI == kEpiPart) {
+            // the unrounded sums, C being an fp32 [M, N] buffer
+            const int64_t span_f = ((int64_t)M * N - wave_off) * 4;
+            const int span32_f = (int)(span_f < 0 ? 0 : (span_f < 0x7FFFFFFFll ? span_f : 0x7FFFFFFFll));
+            auto f_rsrc = __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<float*>(C) + wave_off, 0, span32_f, 0x00020000);
+            const int lane_bytes_f = ((4 * fhalf) * N + frow) * 4;
+#pragma unroll
+            for (int i = 0; i < MF; ++i)
+#pragma unroll
+                for (int j = 0; j < NF; ++j)
+#pragma unroll
+                    for (int v = 0; v < NV; ++v) {
+                        const float sum = acc[i][j][v];
+                        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, sum), f_rsrc, lane_at(j, lane_bytes_f), elem_at(i, j, v) * 4, 0);
+                    }
         } else if (EPI == kEpiDual) {
             // R points at an fp32 [M, N] buffer that receives the unrounded sums next to the rounded ones in C
             float* out32 = reinterpret_cast<float*>(const_cast<T*>(R));
@@ -359,18 +386,17 @@ __device__ __forceinline__ void gemm_dma_tiles(
 // bytes, fragments rebuilt with lane rotations) were no faster.
 // kEpiPart: slice `slice` of `slices` of k, its sums in fp32 to plane `slice` of C.
 // ------------------------------------------------------------------------------------------------------------
-constexpr int kSplitWaves = 8;
-
 template <typename T, int MT, int NT, int EPI>
 __device__ __forceinline__ void gemm_splitk_tile(
     const T* __restrict__ A, const T* __restrict__ B0, const T* __restrict__ B1, T* __restrict__ C,
-    const T* __restrict__ R, int M, int N, int K, int tiles_m, int tiles, int xcds, int block, int blocks, int slice = 0, int slices = 1) {
+    const T* __restrict__ R, int M, int N, int K, int tiles_m, int tiles, int xcds, int block, int blocks, void* lds,
+    int slice = 0, int slices = 1) {
     constexpr int BM = 16 * MT, BN = 16 * NT;
     constexpr int NB = EPI == kEpiSwiGLU ? 2 * NT : NT;          // B fragments: gate rows, then the same up rows
     constexpr int F = MT * NB;
     constexpr int kAhead = MT + NB <= 3 ? 8 : 4;
     constexpr int kStep = 64 / (int)sizeof(T);                   // k values of a step
-    __shared__ __attribute__((aligned(16))) f32x4_t sums[kSplitWaves][F][64];
+    f32x4_t(*sums)[F][64] = reinterpret_cast<f32x4_t(*)[F][64]>(lds);      // [kSplitWaves]
     const int tid = (int)threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     // XCD b % xcds takes a contiguous run of the tiles, all rows of a column first: its L2 holds B's part of the run only

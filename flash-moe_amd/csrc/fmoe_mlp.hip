@@ -40,7 +40,8 @@ template <typename T, int MT, int NT, int EPI>
 __global__ __launch_bounds__(kSplitWaves * 64) void gemm_splitk_kernel(
     const T* __restrict__ A, const T* __restrict__ B0, const T* __restrict__ B1, T* __restrict__ C,
     const T* __restrict__ R, int M, int N, int K, int tiles_m, int tiles, int xcds) {
-    gemm_splitk_tile<T, MT, NT, EPI>(A, B0, B1, C, R, M, N, K, tiles_m, tiles, xcds, (int)blockIdx.x, (int)gridDim.x);
+    __shared__ __attribute__((aligned(16))) char lds[kSplitLds<MT, NT, EPI>];
+    gemm_splitk_tile<T, MT, NT, EPI>(A, B0, B1, C, R, M, N, K, tiles_m, tiles, xcds, (int)blockIdx.x, (int)gridDim.x, lds);
 }
 
 // fp32 with ragged extents or unaligned tensors (not a tuned kernel): 64x64 tile, 16-deep LDS slabs, 4x4 outputs

@@ -168,8 +168,9 @@ __global__ __launch_bounds__(kRouterWaves* kWave, OCC) void router_select_kernel
     const T* __restrict__ lp, int64_t num_tokens, int nk, int top_k, int num_cand, T* __restrict__ scores,
     int64_t* __restrict__ indices, TG* __restrict__ gates, int norm_topk_prob, uint32_t* __restrict__ row_offsets,
     uint32_t row_bytes, const CandidateTable table) {
+    __shared__ SelectLds<RK, RC, kRouterWaves, false> lds;
     router_select_tokens<T, TG, RK, RH, RC, FROM_LOGITS, SMALL, kRouterWaves, false>(
-        lp, num_tokens, nk, top_k, num_cand, scores, indices, gates, norm_topk_prob, row_offsets, row_bytes, table, (int)blockIdx.x,
+        lp, num_tokens, nk, top_k, num_cand, scores, indices, gates, norm_topk_prob, row_offsets, row_bytes, table, lds, (int)blockIdx.x,
         (int)gridDim.x);
 }
 

@@ -441,7 +441,8 @@ __global__ __launch_bounds__(kGateWaves* kWave) void router_gate_splitk_kernel(
     const T* __restrict__ x, const T* __restrict__ w, GateStats st, float* __restrict__ logits32, T* __restrict__ logits, int M, int N,
     int K_full, int tiles_m, int tiles_n, int split, int xcds) {
     extern __shared__ __attribute__((aligned(16))) float stats[];
-    router_gate_splitk_tile<T, MT, NT, STAGED>(x, w, st, logits32, logits, M, N, K_full, tiles_m, tiles_n, split, xcds, stats,
+    __shared__ __attribute__((aligned(16))) char lds[kGateLds<MT, NT>];
+    router_gate_splitk_tile<T, MT, NT, STAGED>(x, w, st, logits32, logits, M, N, K_full, tiles_m, tiles_n, split, xcds, lds, stats,
                                                (int)blockIdx.x, (int)gridDim.x);
 }
 
@@ -906,6 +907,22 @@ extern "C" int fmoe_router_forward_noalloc(const void* x, const void* gate_w, vo
     return router_forward_impl(x, gate_w, running_mean, running_var, num_batches_tracked, stats_dtype, training, momentum,
                                eps, num_tokens, hidden, num_keys, top_k, dtype, norm_topk_prob, router_logits, logits_fp32,
                                scores, indices, gates, nullptr, 0u, ws, (size_t)FMOE_NOALLOC_SCRATCH_BYTES, (hipStream_t)stream, 0, 1);
+}
+
+// Statistics of the batch per row block, for a gate product that combines them itself: what to pass it.
+size_t fmoe::router_block_stats_bytes(int hidden) { return (size_t)kFoldMaxRowBlocks * 2 * (size_t)hidden * 4; }
+int fmoe::router_block_stats(const void* x, int64_t num_tokens, int hidden, int dtype, float* partial, int* row_blocks, int* rows_per_block,
+                             hipStream_t s) {
+    const BlockStatsPlan bp = plan_block_stats(num_tokens);
+    *row_blocks = bp.row_blocks;
+    *rows_per_block = bp.rows_per_block;
+    switch (dtype) {
+        case FMOE_F32: launch_block_stats<float>(x, num_tokens, hidden, bp, partial, s); break;
+        case FMOE_BF16: launch_block_stats<bf16_t>(x, num_tokens, hidden, bp, partial, s); break;
+        default: launch_block_stats<f16_t>(x, num_tokens, hidden, bp, partial, s); break;
+    }
+    FMOE_CHECK_LAUNCH("fmoe_block(batch statistics)");
+    return FMOE_OK;
 }
 
 int fmoe::router_forward_impl(const void* x, const void* gate_w, void* running_mean, void* running_var,

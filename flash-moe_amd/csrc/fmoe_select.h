@@ -278,23 +278,31 @@ inline int candidate_table(int top_k, CandidateTable& table) {
     return used;
 }
 
+template <int RK, int RC, int WAVES, bool PAIRED> struct SelectLds {
+    static constexpr int kTokens = PAIRED ? WAVES / 2 : WAVES;
+    uint64_t slot[WAVES][RK * kWave];
+    float half_score[kTokens][2][RK * kWave];
+    uint32_t half_index[kTokens][2][RK * kWave];
+    uint16_t cand[RC * kWave];
+};
+
 // WAVES waves per workgroup, a token each; PAIRED: two waves per token (one launch round of few tokens), one per half, the first of
 // them going on with the candidates.
 template <typename T, typename TG, int RK, int RH, int RC, bool FROM_LOGITS, bool SMALL, int WAVES, bool PAIRED>
 __device__ __forceinline__ void router_select_tokens(
     const T* __restrict__ lp, int64_t num_tokens, int nk, int top_k, int num_cand, T* __restrict__ scores,
     int64_t* __restrict__ indices, TG* __restrict__ gates, int norm_topk_prob, uint32_t* __restrict__ row_offsets,
-    uint32_t row_bytes, const CandidateTable& table, int block, int blocks) {
+    uint32_t row_bytes, const CandidateTable& table, SelectLds<RK, RC, WAVES, PAIRED>& lds, int block, int blocks) {
     constexpr int KP = RK * kWave;
     constexpr int LOW = sizeof(T) == 4 ? 0 : __is_same(T, bf16_t) ? 16 : 13;      // fp32 bits below the type's mantissa
     constexpr int CAP = SMALL ? kWave / 2 : KP;
     static_assert(RC * kWave <= kSelectMaxCand, "candidate table");
     static_assert(!SMALL || RK == 1, "one key per lane");
-    __shared__ uint16_t cand[RC * kWave];
     constexpr int TOKENS = PAIRED ? WAVES / 2 : WAVES;
-    __shared__ float half_score[TOKENS][2][KP];
-    __shared__ uint32_t half_index[TOKENS][2][KP];
-    __shared__ uint64_t slot[WAVES][KP];
+    auto& cand = lds.cand;
+    auto& half_score = lds.half_score;
+    auto& half_index = lds.half_index;
+    auto& slot = lds.slot;
 
     for (int i = (int)threadIdx.x; i < RC * kWave; i += (int)blockDim.x) cand[i] = table.pair[i];
     __syncthreads();
