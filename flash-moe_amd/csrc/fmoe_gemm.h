@@ -490,11 +490,12 @@ template <typename T> constexpr int kFragRows = sizeof(T) == 2 ? 16 : 32;
 template <typename T> constexpr int kBigSplit = sizeof(T) == 2 ? 4 : 1;
 template <typename T> constexpr int kSmallAhead = sizeof(T) == 2 ? 1 : 3;
 
-// Tile choice.  A workgroup's time per k-tile is the larger of what its CU receives from the L2 ((BM + BN) rows of 128 bytes at
-// about 70 GB/s per CU) and what its matrix pipes take (BM * BN); 128 x 128 balances the two, so in units of one received row the
-// second is BM * BN / 66.  The launch lasts as many rounds as the busiest CU has tiles.  The rule picks the shape with the
-// smallest rounds * time: 256 x 256 (8 waves, two per SIMD) once the chip has several tiles per CU, smaller ones so that every CU
-// has a tile, whatever the extents.
+// Tile choice.  A workgroup's time per k-tile is the larger of what its CU receives from the L2 ((BM + BN) rows of 128 bytes, at 40
+// to 70 GB/s per CU) and what its matrix pipes take (BM * BN), in units of one received row BM * BN / 95: with every CU busy a
+// k-tile of 256 x 256 takes 1.65 us where 128 x 128 takes 0.6, 64 x 128 0.45 and 64 x 64 0.25.  The launch lasts as many rounds as
+// the busiest CU has tiles.  The rule picks the shape with the smallest rounds * time: 256 x 256 (8 waves, two per SIMD) once that
+// means fewer rounds, smaller ones so that every CU has a tile, whatever the extents.  (Pricing 256 x 256 at / 66 gave 1675 tokens
+// of 2904 -> 7744 seven rounds of 128 x 128, 227 us; two of 256 x 256 take 157.)
 // fp32 rows of 128 bytes hold half as many values for matrix pipes an eighth as fast: BM * BN / 15.  The k-splitting kernel
 // costs more per received row, and more so the more CUs receive at once (measured from 64 to 224 workgroups), but its tiles are
 // small enough for a few rows of A.
@@ -512,7 +513,7 @@ template <typename T, int EPI> TileShape choose_tile(int M, int N, int& tiles) {
         const int64_t n = (int64_t)((M + kRows[i] - 1) / kRows[i]) * ((N + out_cols - 1) / out_cols);
         const double occupied = n < cus ? (double)n / cus : 1.0;
         const double received = (kRows[i] + cols) * (split_k ? 1.45 * (1.0 + occupied) : 1.0);
-        const double multiplied = kRows[i] * (double)cols / (sizeof(T) == 4 ? 15.0 : 66.0);
+        const double multiplied = kRows[i] * (double)cols / (sizeof(T) == 4 ? 15.0 : 95.0);
         const double cost = (double)((n + cus - 1) / cus) * (received > multiplied ? received : multiplied);
         if (i == 0 || cost < best_cost) {
             best = (TileShape)i;

@@ -17,10 +17,11 @@ static_assert(kGateWaves == kSplitWaves, "one workgroup size");
 
 // How a product is cut into workgroups: the k-splitting tiles (16 x 16, 32 x 32), or tiles of the LDS pipeline on four waves
 // instead of eight, with as many stages as let two workgroups share a compute unit (all workgroups of a launch hold the same LDS).
-enum Cut { kCutSplit16, kCutSplit32, kCut64, kCut64x128, kCut128, kCutNone };
+enum Cut { kCutSplit16, kCutSplit32, kCut64, kCut64x128, kCut128, kCut256, kCutNone };
 template <int CUT> struct CutShape {
     static constexpr bool kDma = CUT >= kCut64;
-    static constexpr int BM = CUT >= kCut128 ? 128 : 64, BN = CUT == kCut64 ? 64 : 128, kStages = CUT == kCut128 ? 2 : (CUT == kCut64x128 ? 3 : 4);
+    static constexpr int BM = CUT == kCut256 ? 256 : (CUT == kCut128 ? 128 : 64), BN = CUT == kCut256 ? 256 : (CUT == kCut64 ? 64 : 128);
+    static constexpr int kStages = CUT >= kCut128 ? 2 : (CUT == kCut64x128 ? 3 : 4), kWavesN = CUT == kCut256 ? 4 : 2;
     static constexpr int MT = CUT == kCutSplit32 ? 2 : 1;
 };
 // The memory of a launch: the stages of its pipeline tiles, or what the larger of its two kinds of work exchanges sums in.
@@ -40,7 +41,7 @@ template <typename T, int CUT, int EPI, int BESIDE> __device__ __forceinline__ c
 // Waves of a workgroup.  The pipeline's tiles use four.  With few gate tiles, or in fp32 (whose gate product is bound by the matrix
 // pipes), the gate's eight matter more, and the tile's other four end at once; else, and with the registers of a 128 x 128 tile, the
 // four more would keep a second tile off the compute unit.
-template <typename T, int CUT, int GT> constexpr int kGateUpWaves = (CutShape<CUT>::kDma && GT == 2 && sizeof(T) == 2) || CUT == kCut128 ? 4 : kSplitWaves;
+template <typename T, int CUT, int GT> constexpr int kGateUpWaves = (CutShape<CUT>::kDma && CUT != kCut256 && GT == 2 && sizeof(T) == 2) || CUT == kCut128 ? 4 : kSplitWaves;
 template <int CUT> constexpr int kSelectDownWaves = CutShape<CUT>::kDma ? 4 : kSplitWaves;
 
 struct Product { int cut, tiles_m, tiles_n, blocks, slices; };     // blocks: workgroups of a slice of k, whole rounds of XCDs
@@ -50,8 +51,9 @@ __device__ __forceinline__ void product_tiles(const T* A, const T* B0, const T* 
                                               int xcds, int block, char* lds) {
     using S = CutShape<CUT>;
     if constexpr (S::kDma) {
-        if (threadIdx.x >= 256) return;          // whole waves; the barriers of the tile count those that are left
-        gemm_dma_tiles<T, S::BM, S::BN, 2, 2, kStageK<T>, S::kStages, EPI, kSmallAhead<T>, kFragRows<T>, 1, true>(
+        if (threadIdx.x >= 2 * S::kWavesN * kWave) return;          // whole waves; the barriers of the tile count those that are left
+        gemm_dma_tiles<T, S::BM, S::BN, 2, S::kWavesN, kStageK<T>, S::kStages, EPI, CUT == kCut256 ? 1 : kSmallAhead<T>, kFragRows<T>,
+                       CUT == kCut256 ? kBigSplit<T> : 1, true>(
             A, B0, B1, C, R, M, N, K, p.tiles_m, p.tiles_n, xcds, block, p.blocks);
     } else {
         gemm_splitk_tile<T, S::MT, S::MT, EPI>(A, B0, B1, C, R, M, N, K, p.tiles_m, p.tiles_m * p.tiles_n, xcds, block % p.blocks, p.blocks,
@@ -98,7 +100,8 @@ template <typename T, int EPI> Product plan_product(int M, int N) {
     int tiles = 0;
     const int cus = chip_info().cus;
     Product p = {kCutNone, 0, 0, 0, 1};
-    switch (choose_tile<T, EPI>(M, N, tiles)) {
+    const TileShape shape = choose_tile<T, EPI>(M, N, tiles);
+    switch (shape) {
         case kSplit16: p.cut = kCutSplit16; break;
         case kSplit16x32: p.cut = M <= 16 ? kCutSplit16 : kCutSplit32; break;
         case kSplit32: p.cut = kCutSplit32; break;
@@ -108,14 +111,17 @@ template <typename T, int EPI> Product plan_product(int M, int N) {
             if (EPI == kEpiPart) return p;      // gains nothing: without four stages of its own it is slower by what the selection takes
             p.cut = kCut128;
             break;
-        default: return p;
+        default:
+            // a 256 x 256 tile fills its compute unit: only those without one in the last round have room for the gate
+            if (EPI == kEpiPart || sizeof(T) == 4 || (cus - tiles % cus) % cus < cus / 4) return p;
+            p.cut = kCut256;
     }
     if (EPI == kEpiSwiGLU && sizeof(T) == 4 && M <= 256 && p.cut > kCutSplit32) p.cut = M <= 16 ? kCutSplit16 : kCutSplit32;
-    const int rows = p.cut == kCutSplit16 ? 16 : (p.cut == kCutSplit32 ? 32 : (p.cut >= kCut128 ? 128 : 64));
-    const int cols = p.cut == kCutSplit16 ? 16 : (p.cut == kCutSplit32 ? 32 : (p.cut == kCut64 ? 64 : 128) / (EPI == kEpiSwiGLU ? 2 : 1));
+    const int rows = p.cut == kCutSplit16 ? 16 : (p.cut == kCutSplit32 ? 32 : (p.cut == kCut256 ? 256 : (p.cut == kCut128 ? 128 : 64)));
+    const int cols = p.cut == kCutSplit16 ? 16 : (p.cut == kCutSplit32 ? 32 : (p.cut == kCut64 ? 64 : (p.cut == kCut256 ? 256 : 128)) / (EPI == kEpiSwiGLU ? 2 : 1));
     p.tiles_m = (M + rows - 1) / rows;
     p.tiles_n = (N + cols - 1) / cols;
-    const int64_t n = (int64_t)p.tiles_m * p.tiles_n, resident = 2 * cus;
+    const int64_t n = (int64_t)p.tiles_m * p.tiles_n, resident = p.cut == kCut256 ? cus : 2 * cus;
     p.blocks = whole(p.cut >= kCut64 && n > resident ? resident : n, chip_info().xcds);
     return p;
 }
@@ -162,7 +168,8 @@ int gate_and_up(const void* x, const void* gate_w, const GateStats& st, float* l
         case kCutSplit32: FMOE_GO(kCutSplit32); break;
         case kCut64: if constexpr (sizeof(T) == 2) FMOE_GO(kCut64); break;
         case kCut64x128: FMOE_GO(kCut64x128); break;
-        default: FMOE_GO(kCut128); break;
+        case kCut128: FMOE_GO(kCut128); break;
+        default: if constexpr (sizeof(T) == 2) FMOE_GO(kCut256); break;
     }
 #undef FMOE_GO
     FMOE_CHECK_LAUNCH("fmoe_block(gate and up)");

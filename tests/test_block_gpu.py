@@ -199,7 +199,7 @@ def test_single_call_block_equals_the_three_stage_calls(dtype, T, H, I, E, K, tr
     (1, 8, 8, 9, 1), (16, 264, 520, 1200, 33), (17, 1000, 2664, 10000, 24), (64, 1024, 4096, 17000, 64), (255, 520, 1032, 400, 17),
     (256, 1032, 1040, 5000, 5), (257, 264, 520, 1024, 8), (40, 2048, 5464, 2500, 50),
     (300, 1032, 4104, 5000, 40), (999, 1000, 2664, 10000, 24), (1500, 520, 1032, 4200, 3), (2048, 264, 1048, 20000, 40),
-    (1030, 776, 3000, 700, 20), (2049, 264, 520, 1024, 8),
+    (1030, 776, 3000, 700, 20), (1000, 1608, 4264, 2000, 9), (2049, 264, 520, 1024, 8),
 ])
 def test_block_of_few_tokens(dtype, training, T, H, I, E, K):
     from flash_moe.ops.hip.flash_block import block_forward
