@@ -202,7 +202,10 @@ int block_forward_impl(const char* who, const void* x, const void* gate_proj_w, 
     }
     if (!up_beside)
         if ((rc = gate_up())) return rc;
-    return fmoe_mlp_down(act, down_proj_w, num_tokens, hidden, intermediate, dtype, residual, out, stream);
+    const size_t act_bytes = fmoe_mlp_workspace_bytes(num_tokens, hidden, intermediate, dtype);
+    const size_t planes = fmoe_mlp_down_workspace_bytes(num_tokens, hidden, intermediate, dtype);
+    return fmoe_mlp_down_ws(act, down_proj_w, num_tokens, hidden, intermediate, dtype, residual, out, (char*)act + (act_bytes - planes), planes,
+                            stream);
 }
 
 }  // namespace

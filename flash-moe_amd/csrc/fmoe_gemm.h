@@ -29,10 +29,10 @@ template <int MT, int NT, int EPI> constexpr int kSplitLds = kSplitWaves * MT * 
 // ------------------------------------------------------------------------------------------------------------
 // FR: fragment shape (32: v_mfma_f32_32x32x16 / 32x32x2; 16: v_mfma_f32_16x16x32).  SPLIT: a k-step's A fragments are read and
 // multiplied in SPLIT parts (its B fragments stay for the whole k-step), which halves the registers the read-ahead needs.
-template <typename T, int BM, int BN, int WAVES_M, int WAVES_N, int BKT, int NSTAGE, int EPI, int PF, int FR, int SPLIT, bool RAGGED>
+template <typename T, int BM, int BN, int WAVES_M, int WAVES_N, int BKT, int NSTAGE, int EPI, int PF, int FR, int SPLIT, bool RAGGED, bool SLICED = false>
 __device__ __forceinline__ void gemm_dma_tiles(
     const T* __restrict__ A, const T* __restrict__ B0, const T* __restrict__ B1, T* __restrict__ C,
-    const T* __restrict__ R, int M, int N, int K, int tiles_m, int tiles_n, int xcds, int block, int blocks) {
+    const T* __restrict__ R, int M, int N, int K, int tiles_m, int tiles_n, int xcds, int block, int blocks, int slice = 0, int slices = 1) {
     using Shape = MfmaShape<T, FR>;
     using Frag = typename Shape::Frag;
     using Acc = typename Shape::Acc;
@@ -77,10 +77,18 @@ __device__ __forceinline__ void gemm_dma_tiles(
     // RAGGED: rows and the k tail are cut off by the range check of buffer descriptors over the rest of each matrix
     __amdgpu_buffer_rsrc_t a_rsrc, b_rsrc0, b_rsrc1;
     int m0, n0;
-    const int k_tiles = (K + BKT - 1) / BKT;
-    const bool lane_in_tail = (k_tiles - 1) * BKT + (lp ^ key_dma) * EPC < K;      // the lane's chunk of the last k-tile exists
+    // SLICED: k-tiles [k_first, k_first + k_tiles) of the product (every slice has some), one tile per workgroup
+    static_assert(!SLICED || (RAGGED && EPI == kEpiPart), "slices of k leave partial sums");
+    const int k_all = (K + BKT - 1) / BKT, k_share = SLICED ? (k_all + slices - 1) / slices : k_all, k_first = SLICED ? slice * k_share : 0;
+    const int k_tiles = SLICED ? (k_all - k_first < k_share ? k_all - k_first : k_share) : (K + BKT - 1) / BKT;
+    if (SLICED) {
+        A += k_first * BKT;
+        B0 += k_first * BKT;
+        C = reinterpret_cast<T*>(reinterpret_cast<float*>(C) + (int64_t)slice * M * N);
+    }
+    const bool lane_in_tail = (k_first + k_tiles - 1) * BKT + (lp ^ key_dma) * EPC < K;      // the lane's chunk of the last k-tile exists
     auto rest_of = [&](const T* base, int64_t rows) {                              // descriptor from `base` to the end of its matrix
-        const int64_t bytes = rows * K * (int64_t)sizeof(T);
+        const int64_t bytes = SLICED ? (rows * K - k_first * BKT) * (int64_t)sizeof(T) : rows * K * (int64_t)sizeof(T);
         return __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(base), 0, (int)(bytes < 0x7FFFFFFFll ? bytes : 0x7FFFFFFFll), 0x00020000);
     };
     // The workgroup is persistent: it takes tiles t, t + blocks, ...  Each XCD (workgroup id mod 8) gets a contiguous
@@ -500,25 +508,65 @@ template <typename T> constexpr int kSmallAhead = sizeof(T) == 2 ? 1 : 3;
 // costs more per received row, and more so the more CUs receive at once (measured from 64 to 224 workgroups), but its tiles are
 // small enough for a few rows of A.
 enum TileShape { kTile256, kTile128, kTile64x128, kTile64, kSplit32, kSplit16x32, kSplit16 };
-template <typename T, int EPI> TileShape choose_tile(int M, int N, int& tiles) {
-    constexpr int kRows[7] = {256, 128, 64, 64, 32, 16, 16}, kOuts[7] = {256, 128, 128, 64, 32, 32, 16};
+constexpr int kTileRows[7] = {256, 128, 64, 64, 32, 16, 16}, kTileCols[7] = {256, 128, 128, 64, 32, 32, 16};
+
+// Workgroups of tile i, and the time of a round of them per k-tile.
+template <typename T, int EPI> double tile_cost(int i, int M, int N, int64_t& n) {
+    const int cus = chip_info().cus;
+    const bool split_k = i >= kSplit32;
+    const int out_cols = EPI == kEpiSwiGLU && !split_k ? kTileCols[i] / 2 : kTileCols[i];
+    const int cols = EPI == kEpiSwiGLU ? 2 * out_cols : out_cols;
+    n = (int64_t)((M + kTileRows[i] - 1) / kTileRows[i]) * ((N + out_cols - 1) / out_cols);
+    const double occupied = n < cus ? (double)n / cus : 1.0;
+    const double received = (kTileRows[i] + cols) * (split_k ? 1.45 * (1.0 + occupied) : 1.0);
+    const double multiplied = kTileRows[i] * (double)cols / (sizeof(T) == 4 ? 15.0 : 95.0);
+    return received > multiplied ? received : multiplied;
+}
+template <typename T, int EPI> TileShape choose_tile(int M, int N, int& tiles, double* cost_out = nullptr) {
     const int cus = chip_info().cus;
     TileShape best = kTile128;
     double best_cost = 0.0;
     for (int i = 0; i < 7; ++i) {
         if (i == kTile64 && EPI == kEpiSwiGLU && sizeof(T) == 4) continue;      // a 32-column wave tile is one fp32 fragment: no gate/up pair
-        const bool split_k = i >= kSplit32;
-        const int out_cols = EPI == kEpiSwiGLU && !split_k ? kOuts[i] / 2 : kOuts[i];
-        const int cols = EPI == kEpiSwiGLU ? 2 * out_cols : out_cols;
-        const int64_t n = (int64_t)((M + kRows[i] - 1) / kRows[i]) * ((N + out_cols - 1) / out_cols);
-        const double occupied = n < cus ? (double)n / cus : 1.0;
-        const double received = (kRows[i] + cols) * (split_k ? 1.45 * (1.0 + occupied) : 1.0);
-        const double multiplied = kRows[i] * (double)cols / (sizeof(T) == 4 ? 15.0 : 95.0);
-        const double cost = (double)((n + cus - 1) / cus) * (received > multiplied ? received : multiplied);
+        int64_t n = 0;
+        const double round = tile_cost<T, EPI>(i, M, N, n), cost = (double)((n + cus - 1) / cus) * round;
         if (i == 0 || cost < best_cost) {
             best = (TileShape)i;
             best_cost = cost;
             tiles = (int)(n < (1 << 30) ? n : (1 << 30));
+        }
+    }
+    if (cost_out != nullptr) *cost_out = best_cost;
+    return best;
+}
+
+// A long k loop on few tiles: slices of k to workgroups of their own, which leave fp32 sums in planes [slices][M][N] that one more
+// launch adds.  The rule prices both ways, a received row and k-tile at 2.3 ns, that launch at 4 us and the planes written and read
+// at 6 TB/s, and wants the slices to gain a tenth; against the k-splitting tiles, which this price makes too dear when they are
+// short, 8.5 us and a fifth.  Down products, us: 47 tokens, 15360 -> 3840 49.6 -> 25.4; 128 tokens, 8192 -> 2048 29 -> 15.6; 300
+// tokens, 10920 -> 4096 69 -> 51; 479 tokens, 13216 -> 3304 77 -> 61; fp32, 803 tokens, 5632 -> 1408 195 -> 130.
+struct SlicePlan { int shape, slices; };
+constexpr int kMaxSlices = 16;
+template <typename T> SlicePlan plan_slices_of_k(int M, int N, int K) {
+    SlicePlan best = {-1, 1};
+    int tiles = 0;
+    double whole = 0.0;
+    const bool split_k = choose_tile<T, kEpiPlain>(M, N, tiles, &whole) >= kSplit32;
+    const int cus = chip_info().cus, k_tiles = (K + kStageK<T> - 1) / kStageK<T>;
+    const double kRow = 2.3e-3, launch = split_k ? 8.5 : 4.0;
+    double best_time = (split_k ? 0.8 : 0.9) * whole * k_tiles * kRow;
+    if (sizeof(T) == 4 && K % 4 != 0) return best;
+    for (int i = kTile128; i <= kTile64; ++i) {
+        int64_t n = 0;
+        const double round = tile_cost<T, kEpiPlain>(i, M, N, n);
+        for (int s = 2; s <= kMaxSlices && n * s <= cus && s * 4 <= k_tiles; ++s) {
+            const int share = (k_tiles + s - 1) / s;
+            if ((s - 1) * share >= k_tiles) continue;           // a slice would have no k-tile
+            const double time = round * share * kRow + launch + 8.0e-6 * s * (double)M * N / 6.0;
+            if (time < best_time) {
+                best = {i, s};
+                best_time = time;
+            }
         }
     }
     return best;

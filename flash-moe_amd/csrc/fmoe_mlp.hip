@@ -44,6 +44,35 @@ __global__ __launch_bounds__(kSplitWaves * 64) void gemm_splitk_kernel(
     gemm_splitk_tile<T, MT, NT, EPI>(A, B0, B1, C, R, M, N, K, tiles_m, tiles, xcds, (int)blockIdx.x, (int)gridDim.x, lds);
 }
 
+template <typename T, int BM, int BN, int NSTAGE>
+__global__ __launch_bounds__(256) void gemm_sliced_kernel(const T* __restrict__ A, const T* __restrict__ B, float* __restrict__ planes, int M,
+                                                          int N, int K, int tiles_m, int tiles_n, int xcds, int slices) {
+    const int tiles = tiles_m * tiles_n;
+    gemm_dma_tiles<T, BM, BN, 2, 2, kStageK<T>, NSTAGE, kEpiPart, kSmallAhead<T>, kFragRows<T>, 1, true, true>(
+        A, B, nullptr, reinterpret_cast<T*>(planes), nullptr, M, N, K, tiles_m, tiles_n, xcds, (int)blockIdx.x % tiles, tiles,
+        (int)blockIdx.x / tiles, slices);
+}
+
+// C = sum of the planes in slice order [+ R]; four elements per thread.
+template <typename T>
+__global__ __launch_bounds__(256) void add_slices_kernel(const float* __restrict__ planes, const T* __restrict__ R, T* __restrict__ C,
+                                                         int64_t elements, int slices) {
+    const int64_t at = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
+    if (at >= elements) return;
+    const bool whole = at + 4 <= elements && elements % 4 == 0;      // planes of a size that keeps 16-byte alignment
+    if (whole) {
+        f32x4_t sum = *reinterpret_cast<const f32x4_t*>(planes + at);
+        for (int s = 1; s < slices; ++s) sum += *reinterpret_cast<const f32x4_t*>(planes + s * elements + at);
+        for (int i = 0; i < 4; ++i) C[at + i] = Elem<T>::from_f32(R != nullptr ? sum[i] + Elem<T>::to_f32(R[at + i]) : sum[i]);
+    } else {
+        for (int64_t e = at; e < at + 4 && e < elements; ++e) {
+            float sum = planes[e];
+            for (int s = 1; s < slices; ++s) sum += planes[s * elements + e];
+            C[e] = Elem<T>::from_f32(R != nullptr ? sum + Elem<T>::to_f32(R[e]) : sum);
+        }
+    }
+}
+
 // fp32 with ragged extents or unaligned tensors (not a tuned kernel): 64x64 tile, 16-deep LDS slabs, 4x4 outputs
 // per thread, plain FMA.
 template <int EPI>
@@ -168,7 +197,31 @@ int gate_up_tiled(const void* x, const void* wg, const void* wu, int M, int H, i
 }
 
 template <typename T>
-int down_tiled(const void* h, const void* wd, int M, int H, int I, const void* residual, void* out, hipStream_t stream) {
+void launch_sliced(const T* A, const T* B, T* C, const T* R, int M, int N, int K, const SlicePlan& p, float* planes, hipStream_t stream) {
+    const int tiles_m = (M + kTileRows[p.shape] - 1) / kTileRows[p.shape], tiles_n = (N + kTileCols[p.shape] - 1) / kTileCols[p.shape];
+    const dim3 grid((unsigned)(tiles_m * tiles_n * p.slices)), block(256);
+#define FMOE_GO(BM, BN) \
+    hipLaunchKernelGGL((gemm_sliced_kernel<T, BM, BN, 4>), grid, block, 0, stream, A, B, planes, M, N, K, tiles_m, tiles_n, chip_info().xcds, p.slices)
+    if (p.shape == kTile128) FMOE_GO(128, 128);
+    else if (p.shape == kTile64x128) FMOE_GO(64, 128);
+    else FMOE_GO(64, 64);
+#undef FMOE_GO
+    const int64_t elements = (int64_t)M * N;
+    hipLaunchKernelGGL((add_slices_kernel<T>), dim3((unsigned)((elements + 1023) / 1024)), dim3(256), 0, stream, (const float*)planes, R, C,
+                       elements, p.slices);
+}
+
+// planes: room for the fp32 sums of a product cut into slices of k (NULL: it is not cut)
+template <typename T>
+int down_tiled(const void* h, const void* wd, int M, int H, int I, const void* residual, void* out, float* planes, hipStream_t stream) {
+    if (planes != nullptr && (sizeof(T) == 2 || (aligned16(h) && aligned16(wd)))) {
+        const SlicePlan p = plan_slices_of_k<T>(M, H, I);
+        if (p.slices > 1) {
+            launch_sliced<T>((const T*)h, (const T*)wd, (T*)out, (const T*)residual, M, H, I, p, planes, stream);
+            FMOE_CHECK_LAUNCH("fmoe_mlp(down)");
+            return FMOE_OK;
+        }
+    }
     launch_product<T, kEpiPlain>((const T*)h, (const T*)wd, nullptr, (T*)out, (const T*)residual, M, H, I, stream);
     FMOE_CHECK_LAUNCH("fmoe_mlp(down)");
     return FMOE_OK;
@@ -209,9 +262,9 @@ int check_mlp_shape(const char* who, int64_t T_, int H, int I, int dtype) {
 }  // namespace fmoe
 
 extern "C" size_t fmoe_mlp_workspace_bytes(int64_t num_tokens, int hidden, int intermediate, int dtype) {
-    (void)hidden;
     if (num_tokens <= 0 || intermediate <= 0 || !fmoe::dtype_ok(dtype)) return 0;
-    return fmoe::round_up((size_t)num_tokens * (size_t)intermediate * fmoe::dtype_size(dtype), 256);
+    return fmoe::round_up((size_t)num_tokens * (size_t)intermediate * fmoe::dtype_size(dtype), 256) +
+           fmoe_mlp_down_workspace_bytes(num_tokens, hidden, intermediate, dtype);
 }
 
 namespace fmoe {
@@ -251,22 +304,51 @@ extern "C" int fmoe_mlp_gate_up_save(const void* x, const void* gate_w, const vo
     return mlp_gate_up_impl("fmoe_mlp_gate_up_save", x, gate_w, up_w, num_tokens, hidden, intermediate, dtype, act, saved, stream);
 }
 
-extern "C" int fmoe_mlp_down(const void* act, const void* down_w, int64_t num_tokens, int hidden, int intermediate,
-                             int dtype, const void* residual, void* out, void* stream) {
-    using namespace fmoe;
+namespace fmoe {
+namespace {
+int mlp_down_impl(const char* who, const void* act, const void* down_w, int64_t num_tokens, int hidden, int intermediate, int dtype,
+                  const void* residual, void* out, float* planes, void* stream) {
     clear_error();
-    if (int rc = check_mlp_shape("fmoe_mlp_down", num_tokens, hidden, intermediate, dtype)) return rc;
+    if (int rc = check_mlp_shape(who, num_tokens, hidden, intermediate, dtype)) return rc;
     if (num_tokens == 0) return FMOE_OK;
-    FMOE_REQUIRE(act && down_w && out, FMOE_ERR_NULL_POINTER, "fmoe_mlp_down: null tensor pointer");
+    FMOE_REQUIRE(act && down_w && out, FMOE_ERR_NULL_POINTER, "%s: null tensor pointer", who);
     FMOE_REQUIRE(dtype == FMOE_F32 || (aligned16(act) && aligned16(down_w)), FMOE_ERR_ALIGNMENT,
-                 "fmoe_mlp_down: tensor pointers must be 16-byte aligned");
+                 "%s: tensor pointers must be 16-byte aligned", who);
     hipStream_t s = (hipStream_t)stream;
     const int M = (int)num_tokens;
     switch (dtype) {
-        case FMOE_F32: return down_tiled<float>(act, down_w, M, hidden, intermediate, residual, out, s);
-        case FMOE_BF16: return down_tiled<bf16_t>(act, down_w, M, hidden, intermediate, residual, out, s);
-        default: return down_tiled<f16_t>(act, down_w, M, hidden, intermediate, residual, out, s);
+        case FMOE_F32: return down_tiled<float>(act, down_w, M, hidden, intermediate, residual, out, planes, s);
+        case FMOE_BF16: return down_tiled<bf16_t>(act, down_w, M, hidden, intermediate, residual, out, planes, s);
+        default: return down_tiled<f16_t>(act, down_w, M, hidden, intermediate, residual, out, planes, s);
     }
+}
+}  // namespace
+}  // namespace fmoe
+
+extern "C" int fmoe_mlp_down(const void* act, const void* down_w, int64_t num_tokens, int hidden, int intermediate,
+                             int dtype, const void* residual, void* out, void* stream) {
+    return fmoe::mlp_down_impl("fmoe_mlp_down", act, down_w, num_tokens, hidden, intermediate, dtype, residual, out, nullptr, stream);
+}
+
+extern "C" size_t fmoe_mlp_down_workspace_bytes(int64_t num_tokens, int hidden, int intermediate, int dtype) {
+    using namespace fmoe;
+    if (num_tokens <= 0 || num_tokens >= (1ll << 31) || hidden <= 0 || intermediate <= 0 || !dtype_ok(dtype)) return 0;
+    const SlicePlan p = dtype == FMOE_F32 ? plan_slices_of_k<float>((int)num_tokens, hidden, intermediate)
+                                          : plan_slices_of_k<bf16_t>((int)num_tokens, hidden, intermediate);
+    return p.slices > 1 ? round_up((size_t)p.slices * (size_t)num_tokens * (size_t)hidden * 4, 256) : 0;
+}
+
+extern "C" int fmoe_mlp_down_ws(const void* act, const void* down_w, int64_t num_tokens, int hidden, int intermediate, int dtype,
+                                const void* residual, void* out, void* workspace, size_t workspace_bytes, void* stream) {
+    using namespace fmoe;
+    const size_t need = fmoe_mlp_down_workspace_bytes(num_tokens, hidden, intermediate, dtype);
+    if (need > 0 && (workspace == nullptr || workspace_bytes < need || !aligned16(workspace))) {
+        clear_error();
+        set_error("fmoe_mlp_down_ws: workspace of %zu bytes needed, %zu given", need, workspace_bytes);
+        return FMOE_ERR_WORKSPACE;
+    }
+    return mlp_down_impl("fmoe_mlp_down_ws", act, down_w, num_tokens, hidden, intermediate, dtype, residual, out,
+                         need > 0 ? (float*)workspace : nullptr, stream);
 }
 
 extern "C" int fmoe_mlp_forward(const void* x, const void* gate_w, const void* up_w, const void* down_w,
@@ -281,5 +363,7 @@ extern "C" int fmoe_mlp_forward(const void* x, const void* gate_w, const void* u
     FMOE_REQUIRE(workspace && workspace_bytes >= need, FMOE_ERR_WORKSPACE,
                  "fmoe_mlp_forward: workspace of %zu bytes needed, %zu given", need, workspace_bytes);
     if (int rc = fmoe_mlp_gate_up(x, gate_w, up_w, num_tokens, hidden, intermediate, dtype, workspace, stream)) return rc;
-    return fmoe_mlp_down(workspace, down_w, num_tokens, hidden, intermediate, dtype, residual, out, stream);
+    const size_t planes = fmoe_mlp_down_workspace_bytes(num_tokens, hidden, intermediate, dtype);
+    return fmoe_mlp_down_ws(workspace, down_w, num_tokens, hidden, intermediate, dtype, residual, out, (char*)workspace + (need - planes),
+                            planes, stream);
 }

@@ -410,8 +410,10 @@ std::tuple<Tensor, Tensor> mlp_forward_saving(const Tensor& x_in, const Tensor& 
     const int64_t H = x.size(-1), I = wg.size(0), T = H ? x.numel() / H : 0;
     Launch call(x);
     Tensor act = at::empty({T, I}, x.options()), saved = at::empty({2, T, I}, x.options()), out = at::empty_like(x);
+    const size_t bytes = fmoe_mlp_down_workspace_bytes(T, (int)H, (int)I, code);
+    Tensor ws = bytes ? workspace(x, bytes) : Tensor();
     check(fmoe_mlp_gate_up_save(ptr(x), ptr(wg), ptr(wu), T, (int)H, (int)I, code, ptr(act), ptr(saved), call.stream), "flash_mlp");
-    check(fmoe_mlp_down(ptr(act), ptr(wd), T, (int)H, (int)I, code, ptr(res), ptr(out), call.stream), "flash_mlp");
+    check(fmoe_mlp_down_ws(ptr(act), ptr(wd), T, (int)H, (int)I, code, ptr(res), ptr(out), ptr(ws), bytes, call.stream), "flash_mlp");
     return {out, saved};
 }
 

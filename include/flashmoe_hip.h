@@ -223,7 +223,7 @@ int fmoe_expert_forward_algo(const void* x, const void* down, const void* up, co
  *
  *   x [T,H], gate_w [I,H], up_w [I,H], down_w [H,I], residual [T,H] or NULL, out [T,H]: dtype.
  * The gate/up products are kept in fp32 until after silu(.)*(.), then rounded once to dtype.
- * workspace: fmoe_mlp_workspace_bytes() bytes (the [T,I] activation), 256-byte aligned.
+ * workspace: fmoe_mlp_workspace_bytes() bytes (the [T,I] activation, and the sums of a sliced k loop), 256-byte aligned.
  */
 size_t fmoe_mlp_workspace_bytes(int64_t num_tokens, int hidden, int intermediate, int dtype);
 
@@ -246,6 +246,11 @@ int fmoe_mlp_gate_up_save(const void* x, const void* gate_w, const void* up_w, i
 
 int fmoe_mlp_down(const void* act, const void* down_w, int64_t num_tokens, int hidden, int intermediate, int dtype,
                   const void* residual, void* out, void* stream);
+/* fmoe_mlp_down that may cut a long k loop over few output tiles into slices, with the workspace for their sums
+ * (fmoe_mlp_down_workspace_bytes(), 0 where it does not; 16-byte aligned), as fmoe_mlp_forward does. */
+size_t fmoe_mlp_down_workspace_bytes(int64_t num_tokens, int hidden, int intermediate, int dtype);
+int fmoe_mlp_down_ws(const void* act, const void* down_w, int64_t num_tokens, int hidden, int intermediate, int dtype,
+                     const void* residual, void* out, void* workspace, size_t workspace_bytes, void* stream);
 
 /* ------------------------------------------------------------------------------------------------
  * The whole block: FlashMoE.forward (flash_moe/modules/flash_moe.py:55-105) in one call, on the flattened tokens.

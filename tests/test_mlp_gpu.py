@@ -148,3 +148,34 @@ def test_mlp_remainders_of_every_tile_shape(dtype, T, H, I):
     assert rel_fro(out, act.double() @ wd.double().t() + res.double()) < tol
     for buf in (abuf, sbuf, obuf):
         assert (buf[:8] == 7).all() and (buf[-8:] == 7).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("T,H,I", [(47, 1032, 8200), (129, 520, 4104), (203, 1032, 12296), (300, 2056, 8008), (129, 1001, 4004)])
+@pytest.mark.parametrize("with_residual", [False, True])
+def test_mlp_down_with_slices_of_k(dtype, T, H, I, with_residual):
+    # each tile shape with remainders in rows, columns and k; guard rows around the output and the sums; planes of a size that is no
+    # multiple of four elements (fp32); and the result of the uncut product up to the order of the sums
+    from flash_moe import _C
+
+    if dtype != torch.float32 and H % 8:
+        H += 8 - H % 8
+        I += 8 - I % 8
+    _, _, _, wd = cuda(*make(T, H, I, dtype, seed=T + I))
+    act = torch.randn(T, I, device="cuda").to(dtype)
+    res = torch.randn(T, H, device="cuda").to(dtype) if with_residual else None
+    L, code, stream = _C.lib(), _C.dtype_code(dtype), _C.current_stream(act.device)
+    need = L.fmoe_mlp_down_workspace_bytes(T, H, I, code)
+    assert need > 0 and need % 256 == 0 and L.fmoe_mlp_down_workspace_bytes(4096, 4096, 1024, code) == 0
+    ws = torch.full((need + 512,), 7, device="cuda", dtype=torch.uint8)
+    buf = torch.full((T + 16, H), 7.0, device="cuda", dtype=dtype)
+    out = buf[8:8 + T]
+    args = (_C.ptr(act), _C.ptr(wd), T, H, I, code, _C.ptr(res) if res is not None else None)
+    assert L.fmoe_mlp_down_ws(*args, _C.ptr(out), _C.ptr(ws), need - 1, stream) == -7
+    _C.check(L.fmoe_mlp_down_ws(*args, _C.ptr(out), _C.ptr(ws[256:]), need, stream), "down")
+    whole = torch.empty_like(out)
+    _C.check(L.fmoe_mlp_down(*args, _C.ptr(whole), stream), "down")
+    want = act.double() @ wd.double().t() + (res.double() if res is not None else 0.0)
+    tol = {torch.float32: 2e-6, torch.bfloat16: 6e-3, torch.float16: 8e-4}[dtype]
+    assert rel_fro(out, want) < tol and rel_fro(out, whole.cpu()) < tol
+    assert (buf[:8] == 7).all() and (buf[-8:] == 7).all() and (ws[:256] == 7).all() and (ws[-256:] == 7).all()
