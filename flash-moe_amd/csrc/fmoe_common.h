@@ -170,14 +170,13 @@ enum { kBlasNN = 0, kBlasTN = 1 };
 int blas_gemm(int layout, int M, int N, int K, const void* A, int lda, const void* B, int ldb, void* C, int ldc, float beta,
               int dtype, hipStream_t stream);
 
-// The same products on this library's own kernel where that is the faster one (fmoe_gemm_tr.hip), else through blas_gemm.  With
-// B1 (NN only) the product has a second range of K values: C = A[:, :K] B0 + A[:, K:2K] B1.
-int gemm_backward(int layout, int M, int N, int K, const void* A, int lda, const void* B0, const void* B1, int ldb, void* C, int ldc,
-                  int dtype, void* workspace, size_t workspace_bytes, hipStream_t stream);
-// A's rows may be padded (lda) with zeros to whole 16-byte packets.  gemm_backward_own: whether the size is this kernel's.
-bool gemm_backward_own(int M, int N, int K, int dtype);
-// Scratch of gemm_backward for the sums of a split k range (0 when it needs none); segments = 2 with B1, else 1.
-size_t gemm_backward_workspace_bytes(int layout, int M, int N, int K, int segments, int dtype);
+// The same products (C is [M,N]) on this library's own kernels in the 16-bit types (fmoe_gemm_tr.hip), else through blas_gemm.  With B1
+// (NN only) the product has a second range of K values: C = A[:, :K] B0 + A[:, K:2K] B1.  A's rows may be padded (lda) with zeros to
+// whole 16-byte packets.
+int gemm_backward(int layout, int M, int N, int K, const void* A, int lda, const void* B0, const void* B1, int ldb, void* C, int dtype,
+                  void* workspace, size_t workspace_bytes, hipStream_t stream);
+// Scratch of gemm_backward for the sums of a sliced k range (0 when it needs none); segments = 2 with B1, else 1.
+size_t gemm_backward_workspace_bytes(int M, int N, int K, int segments, int dtype);
 
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 inline size_t dtype_size(int dtype) { return dtype == FMOE_F32 ? 4 : 2; }

@@ -29,10 +29,12 @@ template <int MT, int NT, int EPI> constexpr int kSplitLds = kSplitWaves * MT * 
 // ------------------------------------------------------------------------------------------------------------
 // FR: fragment shape (32: v_mfma_f32_32x32x16 / 32x32x2; 16: v_mfma_f32_16x16x32).  SPLIT: a k-step's A fragments are read and
 // multiplied in SPLIT parts (its B fragments stay for the whole k-step), which halves the registers the read-ahead needs.
-template <typename T, int BM, int BN, int WAVES_M, int WAVES_N, int BKT, int NSTAGE, int EPI, int PF, int FR, int SPLIT, bool RAGGED, bool SLICED = false>
+template <typename T, int BM, int BN, int WAVES_M, int WAVES_N, int BKT, int NSTAGE, int EPI, int PF, int FR, int SPLIT, bool RAGGED, bool SLICED = false,
+          bool TA = false, bool TB = false>
 __device__ __forceinline__ void gemm_dma_tiles(
     const T* __restrict__ A, const T* __restrict__ B0, const T* __restrict__ B1, T* __restrict__ C,
-    const T* __restrict__ R, int M, int N, int K, int tiles_m, int tiles_n, int xcds, int block, int blocks, int slice = 0, int slices = 1) {
+    const T* __restrict__ R, int M, int N, int K, int tiles_m, int tiles_n, int xcds, int block, int blocks, int slice = 0, int slices = 1,
+    int lda = 0, int ldb = 0, int segments = 1) {
     using Shape = MfmaShape<T, FR>;
     using Frag = typename Shape::Frag;
     using Acc = typename Shape::Acc;
@@ -52,6 +54,14 @@ __device__ __forceinline__ void gemm_dma_tiles(
     constexpr int BN_OUT = (EPI == kEpiSwiGLU) ? BN / 2 : BN;
     constexpr int A_ROUNDS = BM / ROWS_PER_IT, B_ROUNDS = BN / ROWS_PER_IT;
     constexpr int DMA_PER_TILE = A_ROUNDS + B_ROUNDS;
+    // Turned operands (TA, TB) lie k-row by k-row: a stage holds them as they lie, BKT rows of BM (BN) values, and a lane's 8 k values
+    // come from two transposing LDS reads (lane l of 16 addresses piece l % 4 of row l / 4, and receives column l of the four
+    // rows).  The 32-byte pieces of a row are XOR-ed with a key of the row number, so that the 16 rows a wave-wide read touches lie
+    // in different banks.  NN (TB only) may have a second range of K values, in A further along the rows and in B1.
+    constexpr bool kTurned = TA || TB;
+    static_assert(!kTurned || (RAGGED && sizeof(T) == 2 && FR == 16 && BKT == 64 && EPI != kEpiSwiGLU && EPI != kEpiDual), "turned operands");
+    constexpr int CHA = BM / 8, CHB = BN / 8;        // 16-byte chunks of a k-row
+    auto row_key = [](int k, int chunks) { return chunks >= 16 ? (k & 3) | ((k >> 3) & 1) << 2 : ((k >> 1) & 1) | ((k >> 3) & 1) << 1; };
     static_assert(CPR == 4 || CPR == 8, "stage depth: LDS rows of 64 or 128 bytes");
     static_assert(ROWS_PER_IT % 16 == 0 && BM % ROWS_PER_IT == 0 && BN % ROWS_PER_IT == 0, "DMA rounds");
     static_assert(EPI != kEpiSwiGLU || ((BN / 2) % ROWS_PER_IT == 0 && NF % 2 == 0), "gate/up split");
@@ -70,6 +80,10 @@ __device__ __forceinline__ void gemm_dma_tiles(
     const int lrow = lane / CPR, lp = lane % CPR;
     const int key_dma = ((wave * RPI + lrow) >> ROW_SHIFT) & (CPR - 1);
     const uint32_t lane_off = (uint32_t)(lrow * K + (lp ^ key_dma) * EPC) * (uint32_t)sizeof(T);   // bytes
+    // turned: the lane's row of the round and logical chunk; rounds cover a multiple of 16 rows, so the key is the same in all
+    const int ta_row = wave * (64 / CHA) + lane / CHA, tb_row = wave * (64 / CHB) + lane / CHB;
+    const uint32_t ta_off = (uint32_t)(ta_row * lda + ((lane % CHA) ^ (row_key(ta_row, CHA) << 1)) * 8) * (uint32_t)sizeof(T);
+    const uint32_t tb_off = (uint32_t)(tb_row * ldb + ((lane % CHB) ^ (row_key(tb_row, CHB) << 1)) * 8) * (uint32_t)sizeof(T);
     // A rows beyond M (a ragged last tile row) are read from row M-1 instead: one byte offset per DMA round, set per
     // tile.  What the MFMAs make of those rows is never stored (the epilogue's buffer stores are bounds-checked).
     uint32_t a_lane_off[A_ROUNDS];
@@ -79,16 +93,22 @@ __device__ __forceinline__ void gemm_dma_tiles(
     int m0, n0;
     // SLICED: k-tiles [k_first, k_first + k_tiles) of the product (every slice has some), one tile per workgroup
     static_assert(!SLICED || (RAGGED && EPI == kEpiPart), "slices of k leave partial sums");
-    const int k_all = (K + BKT - 1) / BKT, k_share = SLICED ? (k_all + slices - 1) / slices : k_all, k_first = SLICED ? slice * k_share : 0;
-    const int k_tiles = SLICED ? (k_all - k_first < k_share ? k_all - k_first : k_share) : (K + BKT - 1) / BKT;
-    if (SLICED) {
+    const int k_range = (K + BKT - 1) / BKT;                     // k-tiles of a range of K values
+    const int k_all = kTurned ? k_range * segments : k_range, k_share = SLICED ? (k_all + slices - 1) / slices : k_all, k_first = SLICED ? slice * k_share : 0;
+    const int k_tiles = SLICED ? (k_all - k_first < k_share ? k_all - k_first : k_share) : (kTurned ? k_all : (K + BKT - 1) / BKT);
+    if (SLICED && kTurned) C = reinterpret_cast<T*>(reinterpret_cast<float*>(C) + (int64_t)slice * M * N);
+    if (SLICED && !kTurned) {
         A += k_first * BKT;
         B0 += k_first * BKT;
         C = reinterpret_cast<T*>(reinterpret_cast<float*>(C) + (int64_t)slice * M * N);
     }
-    const bool lane_in_tail = (k_first + k_tiles - 1) * BKT + (lp ^ key_dma) * EPC < K;      // the lane's chunk of the last k-tile exists
+    const bool lane_in_tail = kTurned ? (k_range - 1) * BKT + (lp ^ key_dma) * EPC < K : (k_first + k_tiles - 1) * BKT + (lp ^ key_dma) * EPC < K;      // the lane's chunk of the last k-tile exists
     auto rest_of = [&](const T* base, int64_t rows) {                              // descriptor from `base` to the end of its matrix
         const int64_t bytes = SLICED ? (rows * K - k_first * BKT) * (int64_t)sizeof(T) : rows * K * (int64_t)sizeof(T);
+        return __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(base), 0, (int)(bytes < 0x7FFFFFFFll ? bytes : 0x7FFFFFFFll), 0x00020000);
+    };
+    auto rest_of_rows = [&](const T* base, int64_t rows, int ld, int cols) {        // turned launches: rows of `cols` values, ld apart
+        const int64_t bytes = rows > 0 ? ((rows - 1) * ld + cols) * (int64_t)sizeof(T) : 0;
         return __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(base), 0, (int)(bytes < 0x7FFFFFFFll ? bytes : 0x7FFFFFFFll), 0x00020000);
     };
     // The workgroup is persistent: it takes tiles t, t + blocks, ...  Each XCD (workgroup id mod 8) gets a contiguous
@@ -105,7 +125,15 @@ __device__ __forceinline__ void gemm_dma_tiles(
         for (int r = 0; r < A_ROUNDS; ++r) {
             int row = r * ROWS_PER_IT + wave * RPI + lrow;
             if (!RAGGED) row = m0 + row < M ? row : M - 1 - m0;
-            a_lane_off[r] = (uint32_t)(row * K + (lp ^ key_dma) * EPC) * (uint32_t)sizeof(T);
+            a_lane_off[r] = (uint32_t)(row * (kTurned ? lda : K) + (lp ^ key_dma) * EPC) * (uint32_t)sizeof(T);
+        }
+        if constexpr (kTurned) {
+            auto packets = [](int cols) { return (cols + 7) / 8 * 8; };      // A's rows are padded to whole chunks
+            a_rsrc = TA ? rest_of_rows(A + m0, K, lda, packets(M - m0)) : rest_of_rows(A + (int64_t)m0 * lda, M - m0, lda, packets(K * segments));
+            static_assert(TB, "B is turned wherever A may be");
+            b_rsrc0 = rest_of_rows(B0 + n0, K, ldb, N - n0);
+            b_rsrc1 = segments > 1 ? rest_of_rows(B1 + n0, K, ldb, N - n0) : b_rsrc0;
+            return;
         }
         b_src0 = B0 + (int64_t)(n0 + wave * RPI) * K;
         if (EPI == kEpiSwiGLU) b_src1 = B1 + (int64_t)(n0 + wave * RPI) * K;
@@ -117,6 +145,23 @@ __device__ __forceinline__ void gemm_dma_tiles(
     };
     auto issue = [&](int kt, T* stage) {
         const int k0 = kt * BKT;
+        if constexpr (kTurned) {
+            const int at = k_first + kt, seg = at >= k_range ? 1 : 0, kr = at - seg * k_range;
+            const bool drop = kr + 1 == k_range && !lane_in_tail;
+#pragma unroll
+            for (int r = 0; r < A_ROUNDS; ++r)
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(
+                    a_rsrc, (__attribute__((address_space(3))) void*)(stage + (r * ROWS_PER_IT + wave * RPI) * BKT), 16,
+                    (int)(TA ? ta_off : (drop ? kOutOfRange : a_lane_off[r])),
+                    TA ? (kr * BKT + r * (BKT / A_ROUNDS)) * lda * (int)sizeof(T) : (seg * K + kr * BKT) * (int)sizeof(T), 0, 0);
+            const __amdgpu_buffer_rsrc_t b = seg ? b_rsrc1 : b_rsrc0;
+#pragma unroll
+            for (int r = 0; r < B_ROUNDS; ++r)
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(
+                    b, (__attribute__((address_space(3))) void*)(stage + BM * BKT + (r * ROWS_PER_IT + wave * RPI) * BKT), 16, (int)tb_off,
+                    (kr * BKT + r * (BKT / B_ROUNDS)) * ldb * (int)sizeof(T), 0, 0);
+            return;
+        }
         if constexpr (RAGGED) {
             const bool drop = kt + 1 == k_tiles && !lane_in_tail;
 #pragma unroll
@@ -168,6 +213,21 @@ __device__ __forceinline__ void gemm_dma_tiles(
 #pragma unroll
     for (int ks = 0; ks < KSTEPS; ++ks) pc[ks] = ((ks * Shape::kChunks + fhalf) ^ key_f) << 4;
 
+    // turned: byte address of the lane's piece in fragment 0's place (bits 5 and up of it are XOR-ed per fragment)
+    const int t_row = fhalf * 8 + frow / 4;
+    int ta_lane = t_row * BM * (int)sizeof(T) + row_key(t_row, CHA) * 32 + (frow % 4) * 8;
+    int tb_lane = BM * BKT * (int)sizeof(T) + t_row * BN * (int)sizeof(T) + row_key(t_row, CHB) * 32 + (frow % 4) * 8;
+    auto turned_frag = [&](const char* stage, int lane_at, int piece, int ks, int cols) {
+        typedef short i16x4_t __attribute__((__vector_size__(8)));
+        typedef __attribute__((address_space(3))) i16x4_t* tr_ptr;
+        const char* at = stage + (lane_at ^ ((piece & 7) * 32)) + (piece >> 3) * 256 + ks * 32 * cols * (int)sizeof(T);
+        const i16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((tr_ptr)at);
+        const i16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((tr_ptr)(at + 4 * cols * (int)sizeof(T)));
+        typedef short i16x8_t __attribute__((__vector_size__(16)));
+        const i16x8_t both = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+        return __builtin_bit_cast(Frag, both);
+    };
+
     int tile = block;
     if (tile >= num_tiles) return;
     set_tile(tile);
@@ -188,11 +248,16 @@ __device__ __forceinline__ void gemm_dma_tiles(
     auto read_frags = [&](const char* stage, int q, Frag (&a)[MFS], Frag (&b)[NF]) {
         const int ks = q / SPLIT, part = q % SPLIT;
 #pragma unroll
-        for (int i = 0; i < MFS; ++i)
-            a[i] = *reinterpret_cast<const Frag*>(stage + a_row_bytes + pc[ks] + (part * MFS + i) * FR * BKT * (int)sizeof(T));
+        for (int i = 0; i < MFS; ++i) {
+            if constexpr (TA) a[i] = turned_frag(stage, ta_lane, wm * (WM / 16) + part * MFS + i, ks, BM);
+            else a[i] = *reinterpret_cast<const Frag*>(stage + a_row_bytes + pc[ks] + (part * MFS + i) * FR * BKT * (int)sizeof(T));
+        }
         if (part == 0) {
 #pragma unroll
-            for (int j = 0; j < NF; ++j) b[j] = *reinterpret_cast<const Frag*>(stage + b_row_bytes[j] + pc[ks]);
+            for (int j = 0; j < NF; ++j) {
+                if constexpr (TB) b[j] = turned_frag(stage, tb_lane, wn * (WN / 16) + j, ks, BN);
+                else b[j] = *reinterpret_cast<const Frag*>(stage + b_row_bytes[j] + pc[ks]);
+            }
         }
     };
     // Entering k-tile kt (kt = 0: from the tile prologue): my share of its stage has landed once at most the loads of
@@ -222,6 +287,8 @@ __device__ __forceinline__ void gemm_dma_tiles(
         // merges a path with reads in flight into the MFMA sequence
         auto k_tile_body = [&](int kt, auto last_tag) {
             constexpr bool kLast = decltype(last_tag)::value;
+            // with both operands turned the per-fragment XORs stay inside the k-tile: hoisted, they spill in the 256 x 256 tile
+            if constexpr (TA && BM == 256) asm volatile("" : "+v"(ta_lane), "+v"(tb_lane));
             const char* stage = reinterpret_cast<const char*>(Lds::at() + (kt % NSTAGE) * STAGE);
             const char* next_stage = reinterpret_cast<const char*>(Lds::at() + ((kt + 1) % NSTAGE) * STAGE);
 #pragma unroll
@@ -229,7 +296,8 @@ __device__ __forceinline__ void gemm_dma_tiles(
                 const int nxt = q + PF;
                 constexpr int kMfmas = MFS * NF;     // runs of Shape::kInstr instructions
                 const bool reads = nxt < SPK || !kLast;
-                const int n_reads = MFS + ((nxt % SPLIT) == 0 ? NF : 0);
+                constexpr int RA = TA ? 2 : 1, RB = TB ? 2 : 1;       // LDS reads per fragment
+                const int n_reads = RA * MFS + ((nxt % SPLIT) == 0 ? RB * NF : 0);
                 __builtin_amdgcn_sched_barrier(0);
                 if (nxt < SPK) {
                     read_frags(stage, nxt, fa[nxt % RING], fb[b_slot(nxt)]);
@@ -247,7 +315,7 @@ __device__ __forceinline__ void gemm_dma_tiles(
                     for (int j = 0; j < NF; ++j)
                         acc[part * MFS + i][j] = Shape::run(fa[q % RING][i], fb[b_slot(q)][j], acc[part * MFS + i][j]);
                 // issue order: the LDS reads spread evenly behind the MFMAs
-                constexpr int kPer = (MFS + NF + kMfmas - 1) / kMfmas;
+                constexpr int kPer = (RA * MFS + RB * NF + kMfmas - 1) / kMfmas;
 #pragma unroll
                 for (int m = 0; m < kMfmas; ++m) {
                     __builtin_amdgcn_sched_group_barrier(0x008, Shape::kInstr, 0);
@@ -355,6 +423,13 @@ __device__ __forceinline__ void gemm_dma_tiles(
                         __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, sum), f_rsrc, lane_at(j, lane_bytes_f), at * 4, 0);
                         store_to(c_rsrc, lane_at(j, lane_bytes0), at * (int)sizeof(T), sum);
                     }
+        } else if (kTurned) {
+#pragma unroll
+            for (int i = 0; i < MF; ++i)
+#pragma unroll
+                for (int j = 0; j < NF; ++j)
+#pragma unroll
+                    for (int v = 0; v < NV; ++v) store_to(c_rsrc, lane_at(j, lane_bytes0), elem_at(i, j, v) * (int)sizeof(T), acc[i][j][v]);
         } else {
             auto r_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(R != nullptr ? R + wave_off : C), 0,
                                                             R != nullptr ? span32 : 0, 0x00020000);   // no residual: reads give 0

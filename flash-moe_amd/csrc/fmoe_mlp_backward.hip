@@ -3,9 +3,8 @@
 // The forward keeps only silu(a) * b unless it was asked to keep the gate and up products a, b as well
 // (fmoe_mlp_gate_up_save); without them they are recomputed here (two launches of the forward's own NT GEMM).  The SwiGLU gradient is the fused
 // elementwise kernel of fmoe_backward.hip (it also rebuilds h = silu(a) * b for dWd).  The remaining products are
-// plain GEMMs in layouts the forward never needs (A B and A^T B): gemm_backward (fmoe_gemm_tr.hip) runs the small ones; the large
-// ones go to rocBLAS, which is loaded on first use so
-// that the forward path carries no dependency on it:
+// plain GEMMs in layouts the forward never needs (A B and A^T B): gemm_backward (fmoe_gemm_tr.hip) runs them in the 16-bit types;
+// fp32 goes to rocBLAS, which is loaded on first use so that the other paths carry no dependency on it:
 //     dh  = dy Wd              [T,H][H,I]
 //     dWd = dy^T h             [T,H]^T [T,I]
 //     dx  = da Wg + db Wu      [T,I][I,H] twice, the second accumulating
@@ -85,9 +84,9 @@ MlpBwdPlan plan_mlp_backward(int64_t T_, int H, int I, int dtype) {
     p.off_dab = take(2 * ti);
     p.part_bytes = 0;
     const int t = (int)T_;
-    for (size_t n : {gemm_backward_workspace_bytes(kNN, t, I, H, 1, dtype), gemm_backward_workspace_bytes(kTN, H, I, t, 1, dtype),
-                     gemm_backward_workspace_bytes(kNN, t, H, I, 2, dtype), gemm_backward_workspace_bytes(kTN, 2 * I, H, t, 1, dtype),
-                     gemm_backward_workspace_bytes(kTN, I, H, t, 1, dtype)})
+    for (size_t n : {gemm_backward_workspace_bytes(t, I, H, 1, dtype), gemm_backward_workspace_bytes(H, I, t, 1, dtype),
+                     gemm_backward_workspace_bytes(t, H, I, 2, dtype), gemm_backward_workspace_bytes(2 * I, H, t, 1, dtype),
+                     gemm_backward_workspace_bytes(I, H, t, 1, dtype)})
         if (n > p.part_bytes) p.part_bytes = n;
     p.off_part = take(p.part_bytes);
     p.bytes = o;
@@ -158,22 +157,22 @@ extern "C" int fmoe_mlp_backward(const void* dy, const void* x, const void* gate
         if (rc) return rc;
     }
 
-    rc = gemm_backward(kNN, T_, I, H, dy, H, down_w, nullptr, I, dh, I, dtype, part, p.part_bytes, s);                        // dh = dy Wd
+    rc = gemm_backward(kNN, T_, I, H, dy, H, down_w, nullptr, I, dh, dtype, part, p.part_bytes, s);                        // dh = dy Wd
     if (rc) return rc;
     // da and db side by side: one [T, 2I] matrix [da | db], so that products over both are single calls
     char* db = dab + (size_t)I * elt;
     const int I2 = 2 * I;
     rc = launch_swiglu_backward(dh, a, b, dab, db, h, num_tokens, I, I2, I2, dtype, s);
     if (rc) return rc;
-    rc = gemm_backward(kTN, H, I, T_, dy, H, h, nullptr, I, ddown_w, I, dtype, part, p.part_bytes, s);                         // dWd = dy^T h
+    rc = gemm_backward(kTN, H, I, T_, dy, H, h, nullptr, I, ddown_w, dtype, part, p.part_bytes, s);                         // dWd = dy^T h
     if (rc) return rc;
-    rc = gemm_backward(kNN, T_, H, I, dab, I2, gate_w, up_w, H, dx, H, dtype, part, p.part_bytes, s);                          // dx = da Wg + db Wu
+    rc = gemm_backward(kNN, T_, H, I, dab, I2, gate_w, up_w, H, dx, dtype, part, p.part_bytes, s);                          // dx = da Wg + db Wu
     if (rc) return rc;
     const size_t w_bytes = (size_t)I * H * elt;
     // the two weight gradients are one [2I, H] product when the caller's buffers follow each other: one 74 us kernel at
     // T = I = 4096, H = 1024 instead of two of 49 us
-    if ((char*)dup_w == (char*)dgate_w + w_bytes) return gemm_backward(kTN, I2, H, T_, dab, I2, x, nullptr, H, dgate_w, H, dtype, part, p.part_bytes, s);
-    rc = gemm_backward(kTN, I, H, T_, dab, I2, x, nullptr, H, dgate_w, H, dtype, part, p.part_bytes, s);                       // dWg = da^T x
+    if ((char*)dup_w == (char*)dgate_w + w_bytes) return gemm_backward(kTN, I2, H, T_, dab, I2, x, nullptr, H, dgate_w, dtype, part, p.part_bytes, s);
+    rc = gemm_backward(kTN, I, H, T_, dab, I2, x, nullptr, H, dgate_w, dtype, part, p.part_bytes, s);                       // dWg = da^T x
     if (rc) return rc;
-    return gemm_backward(kTN, I, H, T_, db, I2, x, nullptr, H, dup_w, H, dtype, part, p.part_bytes, s);                        // dWu = db^T x
+    return gemm_backward(kTN, I, H, T_, db, I2, x, nullptr, H, dup_w, dtype, part, p.part_bytes, s);                        // dWu = db^T x
 }
