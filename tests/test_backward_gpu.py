@@ -553,3 +553,14 @@ def test_mlp_backward_remainders_of_the_transposing_products(dtype, T, H, I):
     for name, a, leaf in zip(("dx", "dgate", "dup", "ddown"), got, leaves):
         assert rel_fro(a, leaf.grad) < GRAD_FRO[dtype], name
     assert all(torch.equal(a, b) for a, b in zip(got, mlp_backward(dy, x, *ws, saved)))      # bit for bit the same twice
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("T,H,I", [
+    (500, 2056, 4104),       # 128 x 128 tiles, one and two to a compute unit, and slices of k
+    (600, 3080, 6152),       # dW on 256 x 256 tiles
+    (2500, 264, 5000),       # dh on 256 x 256 tiles; slices for the weight gradients
+    (260, 3080, 13000),      # dx on 256 x 256 tiles in slices
+])
+def test_mlp_backward_on_the_large_tiles_of_the_turned_products(dtype, T, H, I):
+    test_mlp_backward_remainders_of_the_transposing_products(dtype, T, H, I)
