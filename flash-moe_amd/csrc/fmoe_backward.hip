@@ -235,8 +235,10 @@ __global__ __launch_bounds__(256) void swiglu_backward_kernel(const T* __restric
 // ------------------------------------------------------------------------------------------------------------
 // routed experts, per-token part: dx, dgates and the two coefficients of every pair
 // ------------------------------------------------------------------------------------------------------------
-template <typename T, int NCH>
-__global__ __launch_bounds__(kBwdWaves* kWave) void expert_backward_token_kernel(
+// WAVES = 1: a wave per token.  WAVES > 1 (few tokens): the workgroup's waves share one token as in the forward, their partial rows of
+// dx are added in wave order through LDS.
+template <typename T, int NCH, int WAVES>
+__global__ __launch_bounds__((WAVES > 1 ? WAVES : kBwdWaves) * kWave) void expert_backward_token_kernel(
     const T* __restrict__ dout, const T* __restrict__ x, const T* __restrict__ down, const T* __restrict__ up,
     const int64_t* __restrict__ indices, const T* __restrict__ gates, T* __restrict__ dx, T* __restrict__ dgates,
     float* __restrict__ coef_up, float* __restrict__ coef_down, int32_t* __restrict__ counts, int64_t num_tokens,
@@ -244,8 +246,11 @@ __global__ __launch_bounds__(kBwdWaves* kWave) void expert_backward_token_kernel
     constexpr int V = Elem<T>::kVec;
     constexpr int PIF = NCH >= 8 ? 1 : (NCH >= 4 ? 2 : 4);   // (down, up) row pairs requested ahead
     const int lane = lane_id();
-    const int64_t token = (int64_t)blockIdx.x * kBwdWaves + (threadIdx.x >> 6);
+    const int wave = (int)(threadIdx.x >> 6);
+    const int64_t token = WAVES > 1 ? (int64_t)blockIdx.x : (int64_t)blockIdx.x * kBwdWaves + wave;
     if (token >= num_tokens) return;
+    constexpr int ROW = NCH * V * kWave;
+    __shared__ __attribute__((aligned(16))) float partial_rows[WAVES > 1 ? WAVES * ROW : 4];
 
     const int packets = hidden / V;
     const u32x4_t zero4 = {0u, 0u, 0u, 0u};
@@ -264,7 +269,7 @@ __global__ __launch_bounds__(kBwdWaves* kWave) void expert_backward_token_kernel
 #pragma unroll
         for (int v = 0; v < V; ++v) acc[c][v] = 0.0f;
 
-    for (int k0 = 0; k0 < top_k; k0 += PIF) {
+    for (int k0 = WAVES > 1 ? wave * PIF : 0; k0 < top_k; k0 += WAVES * PIF) {
         u32x4_t dn[PIF][NCH], uq[PIF][NCH];
         float gate[PIF];
         bool valid[PIF];
@@ -326,6 +331,26 @@ __global__ __launch_bounds__(kBwdWaves* kWave) void expert_backward_token_kernel
             }
         }
     }
+    if constexpr (WAVES > 1) {
+#pragma unroll
+        for (int c = 0; c < NCH; ++c)
+#pragma unroll
+            for (int v = 0; v < V; v += 4)
+                *reinterpret_cast<f32x4_t*>(&partial_rows[wave * ROW + (c * kWave + lane) * V + v]) =
+                    f32x4_t{acc[c][v], acc[c][v + 1], acc[c][v + 2], acc[c][v + 3]};
+        __syncthreads();
+        for (int p = (int)threadIdx.x; p < packets; p += WAVES * kWave) {
+            float sum[V];
+#pragma unroll
+            for (int v = 0; v < V; ++v) sum[v] = partial_rows[p * V + v];
+#pragma unroll
+            for (int w = 1; w < WAVES; ++w)
+#pragma unroll
+                for (int v = 0; v < V; ++v) sum[v] += partial_rows[w * ROW + p * V + v];
+            reinterpret_cast<u32x4_t*>(dx + token * hidden)[p] = pack16<T>(sum);
+        }
+        return;
+    }
 #pragma unroll
     for (int c = 0; c < NCH; ++c) {
         const int p = c * kWave + lane;
@@ -364,75 +389,93 @@ __global__ __launch_bounds__(256) void expert_backward_gate_kernel(
     if (valid) atomicAdd(&counts[indices[p]], 1);   // integer histogram: the result does not depend on order
 }
 
-// One wave per expert and column chunk (blockIdx.y; NCH * 64 packets each): its rows of ddown and dup, summed over its
-// pairs in ascending pair index.
+// A wave takes `span` consecutive experts (lane l holds the end of the l-th one's segment) and a chunk of the columns (NCH * 1024 bytes):
+// their pieces of ddown and dup, each summed over its pairs in ascending pair index.  The segments follow each other, so the wave walks
+// one list, 64 pairs per round, with the pieces of the next pairs in flight whether or not an expert ends between them.
+// Bound by what the caches deliver (x and dout, 4 KB per pair at 1024 columns), so the work is ordered chunk by chunk and every XCD
+// gets a run of it: its L2 holds a chunk of x and dout instead of their whole rows.  Weight gradients, us: 4096 tokens x 64 pairs,
+// 16384 experts, 1024 columns 90 -> 70; 1024 x 512, 102400 experts 172 -> 145; 1024 x 64, 2048 columns 90 -> 60.
+// Where x and dout fit the L2 whole, chunks of two packets per lane save walking the lists twice.
 template <typename T, int NCH>
 __global__ __launch_bounds__(kBwdWaves* kWave) void expert_backward_weight_kernel(
     const T* __restrict__ dout, const T* __restrict__ x, const float* __restrict__ coef_up,
     const float* __restrict__ coef_down, const uint32_t* __restrict__ pairs, const int32_t* __restrict__ offsets,
-    T* __restrict__ ddown, T* __restrict__ dup, int hidden, int64_t num_experts, int top_k) {
-    constexpr int V = Elem<T>::kVec;
-    constexpr int PIF = NCH >= 8 ? 1 : 2;
+    T* __restrict__ ddown, T* __restrict__ dup, int hidden, int64_t num_experts, int top_k, int span, int units, int chunks, int xcds) {
+    constexpr int V = Elem<T>::kVec, PIF = 8 / NCH;
     const int lane = lane_id();
-    const int64_t e = (int64_t)blockIdx.x * kBwdWaves + (threadIdx.x >> 6);
-    if (e >= num_experts) return;
-    const int packets = hidden / V;
-    const int first = (int)blockIdx.y * NCH * kWave;          // first packet of this column chunk
-    const u32x4_t zero4 = {0u, 0u, 0u, 0u};
+    const int item = ((int)blockIdx.x % xcds) * ((int)gridDim.x / xcds) + (int)blockIdx.x / xcds;      // chunk-major
+    if (item >= units * chunks) return;
+    const int64_t e0 = ((int64_t)(item % units) * kBwdWaves + (threadIdx.x >> 6)) * span;
+    if (e0 >= num_experts) return;
+    const int count = num_experts - e0 < span ? (int)(num_experts - e0) : span;
     bool live[NCH];
-#pragma unroll
-    for (int c = 0; c < NCH; ++c) live[c] = first + c * kWave + lane < packets;
-    float acc_d[NCH][V], acc_u[NCH][V];
-#pragma unroll
-    for (int c = 0; c < NCH; ++c)
-#pragma unroll
-        for (int v = 0; v < V; ++v) acc_d[c][v] = acc_u[c][v] = 0.0f;
-
-    const int begin = offsets[e], end = offsets[e + 1];
-    const int n_total = end - begin;
-    // The segment lists the expert's pairs in ascending pair index (the bucketing stage orders it), kWave pairs per round.
-    for (int done = 0; done < n_total; done += kWave) {
-        const int n = n_total - done < kWave ? n_total - done : kWave;
-        const uint32_t mine = lane < n ? pairs[begin + done + lane] : 0u;
-        uint32_t tok = 0;
-        float cu = 0.0f, cd = 0.0f;
-        if (lane < n) {
-            tok = mine / (uint32_t)top_k;
-            cu = coef_up[mine];
-            cd = coef_down[mine];
-        }
-        for (int j0 = 0; j0 < n; j0 += PIF) {
-            u32x4_t xq[PIF][NCH], gq[PIF][NCH];
-            float su[PIF], sd[PIF];
-#pragma unroll
-            for (int u = 0; u < PIF; ++u) {
-                const int j = j0 + u < n ? j0 + u : n - 1;
-                const bool on = j0 + u < n;
-                const int64_t t = (int64_t)(uint32_t)__builtin_amdgcn_readlane((int)tok, j);
-                su[u] = on ? __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, cu), j)) : 0.0f;
-                sd[u] = on ? __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, cd), j)) : 0.0f;
-#pragma unroll
-                for (int c = 0; c < NCH; ++c) {
-                    const int p = first + c * kWave + lane;
-                    xq[u][c] = (on && live[c]) ? reinterpret_cast<const u32x4_t*>(x + t * hidden)[p] : zero4;
-                    gq[u][c] = (on && live[c]) ? reinterpret_cast<const u32x4_t*>(dout + t * hidden)[p] : zero4;
-                }
-            }
-#pragma unroll
-            for (int u = 0; u < PIF; ++u)
-#pragma unroll
-                for (int c = 0; c < NCH; ++c) {
-                    axpy16<T>(sd[u], xq[u][c], acc_d[c]);
-                    axpy16<T>(su[u], gq[u][c], acc_u[c]);
-                }
-        }
-    }
+    int at[NCH];                                              // lanes past the row read its first packet and store nothing
 #pragma unroll
     for (int c = 0; c < NCH; ++c) {
-        const int p = first + c * kWave + lane;
-        if (live[c]) {
-            reinterpret_cast<u32x4_t*>(ddown + e * hidden)[p] = pack16<T>(acc_d[c]);
-            reinterpret_cast<u32x4_t*>(dup + e * hidden)[p] = pack16<T>(acc_u[c]);
+        const int packet = (item / units * NCH + c) * kWave + lane;
+        live[c] = packet < hidden / V;
+        at[c] = live[c] ? packet : 0;
+    }
+    float acc_d[NCH][V], acc_u[NCH][V];
+    auto clear = [&]() {
+#pragma unroll
+        for (int c = 0; c < NCH; ++c)
+#pragma unroll
+            for (int v = 0; v < V; ++v) acc_d[c][v] = acc_u[c][v] = 0.0f;
+    };
+    clear();
+
+    const int ends = offsets[e0 + (lane < count ? lane + 1 : count)];
+    const int begin = __builtin_amdgcn_readfirstlane(offsets[e0]), end = __builtin_amdgcn_readlane(ends, count - 1);
+    int cur = 0, cur_end = __builtin_amdgcn_readlane(ends, 0);
+    // rows of the experts whose segments end at list position `pos`
+    auto flush = [&](int pos) {
+        while (cur < count && cur_end == pos) {
+#pragma unroll
+            for (int c = 0; c < NCH; ++c) {
+                if (live[c]) {
+                    reinterpret_cast<u32x4_t*>(ddown + (e0 + cur) * hidden)[at[c]] = pack16<T>(acc_d[c]);
+                    reinterpret_cast<u32x4_t*>(dup + (e0 + cur) * hidden)[at[c]] = pack16<T>(acc_u[c]);
+                }
+            }
+            clear();
+            ++cur;
+            cur_end = __builtin_amdgcn_readlane(ends, cur < count ? cur : count - 1);
+        }
+    };
+    flush(begin);
+    for (int done = begin; done < end; done += kWave) {
+        const int n = end - done < kWave ? end - done : kWave;
+        const uint32_t mine = pairs[done + (lane < n ? lane : n - 1)];
+        const uint32_t tok = mine / (uint32_t)top_k;
+        const float cu = coef_up[mine], cd = coef_down[mine];
+        u32x4_t xq[PIF][NCH], gq[PIF][NCH];
+        auto load = [&](int j, u32x4_t (&xr)[NCH], u32x4_t (&gr)[NCH]) {
+            const int64_t t = (int64_t)(uint32_t)__builtin_amdgcn_readlane((int)tok, j < n ? j : n - 1);
+#pragma unroll
+            for (int c = 0; c < NCH; ++c) {
+                xr[c] = reinterpret_cast<const u32x4_t*>(x + t * hidden)[at[c]];
+                gr[c] = reinterpret_cast<const u32x4_t*>(dout + t * hidden)[at[c]];
+            }
+        };
+#pragma unroll
+        for (int u = 0; u < PIF; ++u) load(u, xq[u], gq[u]);
+        for (int j0 = 0; j0 < n; j0 += PIF) {
+#pragma unroll
+            for (int u = 0; u < PIF; ++u) {
+                const int j = j0 + u;
+                if (j < n) {
+                    const float sd = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, cd), j));
+                    const float su = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, cu), j));
+#pragma unroll
+                    for (int c = 0; c < NCH; ++c) {
+                        axpy16<T>(sd, xq[u][c], acc_d[c]);
+                        axpy16<T>(su, gq[u][c], acc_u[c]);
+                    }
+                    flush(done + j + 1);
+                }
+                load(j + PIF, xq[u], gq[u]);
+            }
         }
     }
 }
@@ -486,9 +529,6 @@ int launch_expert_backward(const void* dout, const void* x, const void* down, co
     const int64_t pairs = T_ * K;
     const int nch = (H / V + kWave - 1) / kWave;
     const dim3 block(kBwdWaves * kWave);
-    const dim3 token_grid((unsigned)((T_ + kBwdWaves - 1) / kBwdWaves));
-    const dim3 expert_grid((unsigned)((E + kBwdWaves - 1) / kBwdWaves), (unsigned)((nch + 7) / 8));   // y: column chunks of long rows
-
     if (int rc = bucket_clear(bucket_ws, E, stream)) return rc;
     if (p.slices) {
         uint32_t* off32 = (uint32_t*)(ws + p.off_off32);
@@ -515,14 +555,23 @@ int launch_expert_backward(const void* dout, const void* x, const void* down, co
         FMOE_CHECK_LAUNCH("fmoe_expert_backward(coefficients)");
         if (int rc = expert_slice_states(coef_list, down, off32, dx, T_, H, E, K, dtype, p.ordered, stream)) return rc;
     } else {
-#define FMOE_LAUNCH_TOKEN(N)                                                                                          \
-        hipLaunchKernelGGL((expert_backward_token_kernel<T, N>), token_grid, block, 0, stream, (const T*)dout, (const T*)x, \
-                           (const T*)down, (const T*)up, indices, (const T*)gates, (T*)dx, (T*)dgates, coef_up, coef_down,  \
-                           counts, T_, H, E, K)
-        if (nch <= 1) FMOE_LAUNCH_TOKEN(1);
-        else if (nch <= 2) FMOE_LAUNCH_TOKEN(2);
-        else if (nch <= 4) FMOE_LAUNCH_TOKEN(4);
-        else FMOE_LAUNCH_TOKEN(8);
+        // waves per token: as the forward's rows; sixteen fit their registers up to two packets per lane
+        const int waves = K <= 4 || T_ > 2048 ? 1 : (T_ > chip_info().cus ? 4 : (nch > 2 ? 8 : 16));
+#define FMOE_LAUNCH_TOKEN(N, W)                                                                                                       \
+        hipLaunchKernelGGL((expert_backward_token_kernel<T, N, W>), dim3((unsigned)(W > 1 ? T_ : (T_ + kBwdWaves - 1) / kBwdWaves)), \
+                           dim3((W > 1 ? W : kBwdWaves) * kWave), 0, stream, (const T*)dout, (const T*)x, (const T*)down,            \
+                           (const T*)up, indices, (const T*)gates, (T*)dx, (T*)dgates, coef_up, coef_down, counts, T_, H, E, K)
+#define FMOE_LAUNCH_TOKENS(N, MOST)                                      \
+        do {                                                             \
+            if (waves >= 8) FMOE_LAUNCH_TOKEN(N, MOST);                  \
+            else if (waves == 4) FMOE_LAUNCH_TOKEN(N, 4);                \
+            else FMOE_LAUNCH_TOKEN(N, 1);                                \
+        } while (0)
+        if (nch <= 1) FMOE_LAUNCH_TOKENS(1, 16);
+        else if (nch <= 2) FMOE_LAUNCH_TOKENS(2, 16);
+        else if (nch <= 4) FMOE_LAUNCH_TOKENS(4, 8);
+        else FMOE_LAUNCH_TOKENS(8, 8);
+#undef FMOE_LAUNCH_TOKENS
 #undef FMOE_LAUNCH_TOKEN
         FMOE_CHECK_LAUNCH("fmoe_expert_backward(tokens)");
     }
@@ -532,14 +581,21 @@ int launch_expert_backward(const void* dout, const void* x, const void* down, co
                                   nullptr, 0, 1, stream))
         return rc;
 
-#define FMOE_LAUNCH_WEIGHT(N)                                                                                            \
-    hipLaunchKernelGGL((expert_backward_weight_kernel<T, N>), expert_grid, block, 0, stream, (const T*)dout, (const T*)x, \
-                       (const float*)coef_up, (const float*)coef_down, (const uint32_t*)pairs_by_expert,                  \
-                       (const int32_t*)offsets, (T*)ddown, (T*)dup, H, E, K)
-    if (nch <= 1) FMOE_LAUNCH_WEIGHT(1);
-    else if (nch <= 2) FMOE_LAUNCH_WEIGHT(2);
-    else if (nch <= 4) FMOE_LAUNCH_WEIGHT(4);
-    else FMOE_LAUNCH_WEIGHT(8);
+    // experts per wave: about a round of 64 pairs, as long as every SIMD keeps four waves
+    const int xcds = chip_info().xcds;
+    const bool resident = 2 * T_ * H * (int64_t)sizeof(T) < chip_info().l2_bytes;
+    const int chunks = resident ? (nch + 1) / 2 : nch;
+    int64_t span = pairs > 0 ? 64 * E / pairs : 32;
+    const int64_t most = E * chunks / (chip_info().cus * 16);
+    if (span > most) span = most;
+    span = span < 1 ? 1 : (span > 32 ? 32 : span);
+    const int64_t units = (E + span * kBwdWaves - 1) / (span * kBwdWaves);
+#define FMOE_LAUNCH_WEIGHT(N)                                                                                                             \
+    hipLaunchKernelGGL((expert_backward_weight_kernel<T, N>), dim3((unsigned)((units * chunks + xcds - 1) / xcds * xcds)), block, 0, stream, \
+                       (const T*)dout, (const T*)x, (const float*)coef_up, (const float*)coef_down, (const uint32_t*)pairs_by_expert,     \
+                       (const int32_t*)offsets, (T*)ddown, (T*)dup, H, E, K, (int)span, (int)units, chunks, xcds)
+    if (resident && nch > 1) FMOE_LAUNCH_WEIGHT(2);
+    else FMOE_LAUNCH_WEIGHT(1);
 #undef FMOE_LAUNCH_WEIGHT
     FMOE_CHECK_LAUNCH("fmoe_expert_backward(weights)");
     return FMOE_OK;

@@ -564,3 +564,29 @@ def test_mlp_backward_remainders_of_the_transposing_products(dtype, T, H, I):
 ])
 def test_mlp_backward_on_the_large_tiles_of_the_turned_products(dtype, T, H, I):
     test_mlp_backward_remainders_of_the_transposing_products(dtype, T, H, I)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("T,H,E,K", [
+    (3, 24, 40, 4), (256, 264, 900, 5), (257, 520, 300, 33), (2049, 136, 5000, 9),      # waves per token of the row schedule
+    (120, 2048, 70, 17), (64, 1032, 20000, 70),        # rows of several packets per lane; experts without pairs, spans of experts
+    (1500, 1544, 700, 20),                             # x and dout beyond an L2: column chunks, the last one partial
+    (200, 64, 3, 2), (700, 72, 2, 2),                  # segments of more than a round of pairs
+])
+def test_expert_backward_edges_of_the_waves_and_spans(dtype, T, H, E, K):
+    from flash_moe.ops.hip.flash_expert import expert_backward
+
+    g = gen(T + H)
+    x, dy = (torch.randn(T, H, generator=g).to(dtype).cuda() for _ in range(2))
+    wd, wu = (torch.randn(E, H, generator=g).mul(0.05).to(dtype).cuda() for _ in range(2))
+    idx = torch.randint(0, E, (T, K), generator=g).cuda()
+    gates = torch.softmax(torch.randn(T, K, generator=g), -1).to(dtype).cuda()
+    got = expert_backward(dy, x, wd, wu, idx, gates)
+    leaves = [t.double().requires_grad_(True) for t in (x, wd, wu, gates)]
+    out = torch.zeros(T, H, device="cuda", dtype=torch.float64)
+    for k in range(K):
+        s = (leaves[0] * leaves[1][idx[:, k]]).sum(-1)
+        out = out + (torch.nn.functional.silu(s) * leaves[3][:, k])[:, None] * leaves[2][idx[:, k]]
+    out.backward(dy.double())
+    for name, a, leaf in zip(("dx", "ddown", "dup", "dgates"), got, leaves):
+        assert rel_fro(a, leaf.grad) < GRAD_FRO[dtype], name
