@@ -170,7 +170,7 @@ enum { kBlasNN = 0, kBlasTN = 1 };
 int blas_gemm(int layout, int M, int N, int K, const void* A, int lda, const void* B, int ldb, void* C, int ldc, float beta,
               int dtype, hipStream_t stream);
 
-// The same products (C is [M,N]) on this library's own kernels in the 16-bit types (fmoe_gemm_tr.hip), else through blas_gemm.  With B1
+// The same products (C is [M,N]) on this library's own kernels (fmoe_gemm_tr.hip), through blas_gemm where those cannot address them.  With B1
 // (NN only) the product has a second range of K values: C = A[:, :K] B0 + A[:, K:2K] B1.  A's rows may be padded (lda) with zeros to
 // whole 16-byte packets.
 int gemm_backward(int layout, int M, int N, int K, const void* A, int lda, const void* B0, const void* B1, int ldb, void* C, int dtype,

@@ -54,14 +54,19 @@ __device__ __forceinline__ void gemm_dma_tiles(
     constexpr int BN_OUT = (EPI == kEpiSwiGLU) ? BN / 2 : BN;
     constexpr int A_ROUNDS = BM / ROWS_PER_IT, B_ROUNDS = BN / ROWS_PER_IT;
     constexpr int DMA_PER_TILE = A_ROUNDS + B_ROUNDS;
-    // Turned operands (TA, TB) lie k-row by k-row: a stage holds them as they lie, BKT rows of BM (BN) values, and a lane's 8 k values
-    // come from two transposing LDS reads (lane l of 16 addresses piece l % 4 of row l / 4, and receives column l of the four
-    // rows).  The 32-byte pieces of a row are XOR-ed with a key of the row number, so that the 16 rows a wave-wide read touches lie
-    // in different banks.  NN (TB only) may have a second range of K values, in A further along the rows and in B1.
+    // Turned operands (TA, TB) lie k-row by k-row: a stage holds them as they lie, BKT rows of BM (BN) values.  16-bit: a lane's 8 k
+    // values come from two transposing LDS reads (lane l of 16 addresses piece l % 4 of row l / 4, and receives column l of the four
+    // rows); fp32: from four plain ones, one per k value.  The 16-byte chunks of a row are XOR-ed with a key of the row number, so
+    // that the rows a wave-wide read touches lie in different banks.  NN (TB only) may have a second range of K values, in A
+    // further along the rows and in B1.
     constexpr bool kTurned = TA || TB;
-    static_assert(!kTurned || (RAGGED && sizeof(T) == 2 && FR == 16 && BKT == 64 && EPI != kEpiSwiGLU && EPI != kEpiDual), "turned operands");
-    constexpr int CHA = BM / 8, CHB = BN / 8;        // 16-byte chunks of a k-row
-    auto row_key = [](int k, int chunks) { return chunks >= 16 ? (k & 3) | ((k >> 3) & 1) << 2 : ((k >> 1) & 1) | ((k >> 3) & 1) << 1; };
+    static_assert(!kTurned || (RAGGED && ((sizeof(T) == 2 && FR == 16 && BKT == 64) || (sizeof(T) == 4 && FR == 32 && BKT == 32)) &&
+                               EPI != kEpiSwiGLU && EPI != kEpiDual), "turned operands");
+    constexpr int CHA = BM / EPC, CHB = BN / EPC;    // 16-byte chunks of a k-row
+    auto row_key = [](int k, int chunks) {
+        if (sizeof(T) == 4) return ((k >> 2) & 1) << 3;
+        return chunks >= 16 ? ((k & 3) | ((k >> 3) & 1) << 2) << 1 : (((k >> 1) & 1) | ((k >> 3) & 1) << 1) << 1;
+    };
     static_assert(CPR == 4 || CPR == 8, "stage depth: LDS rows of 64 or 128 bytes");
     static_assert(ROWS_PER_IT % 16 == 0 && BM % ROWS_PER_IT == 0 && BN % ROWS_PER_IT == 0, "DMA rounds");
     static_assert(EPI != kEpiSwiGLU || ((BN / 2) % ROWS_PER_IT == 0 && NF % 2 == 0), "gate/up split");
@@ -80,10 +85,10 @@ __device__ __forceinline__ void gemm_dma_tiles(
     const int lrow = lane / CPR, lp = lane % CPR;
     const int key_dma = ((wave * RPI + lrow) >> ROW_SHIFT) & (CPR - 1);
     const uint32_t lane_off = (uint32_t)(lrow * K + (lp ^ key_dma) * EPC) * (uint32_t)sizeof(T);   // bytes
-    // turned: the lane's row of the round and logical chunk; rounds cover a multiple of 16 rows, so the key is the same in all
+    // turned: the lane's row of the round and logical chunk; rounds cover a multiple of 16 rows (8 in fp32), so the key is the same in all
     const int ta_row = wave * (64 / CHA) + lane / CHA, tb_row = wave * (64 / CHB) + lane / CHB;
-    const uint32_t ta_off = (uint32_t)(ta_row * lda + ((lane % CHA) ^ (row_key(ta_row, CHA) << 1)) * 8) * (uint32_t)sizeof(T);
-    const uint32_t tb_off = (uint32_t)(tb_row * ldb + ((lane % CHB) ^ (row_key(tb_row, CHB) << 1)) * 8) * (uint32_t)sizeof(T);
+    const uint32_t ta_off = (uint32_t)(ta_row * lda + ((lane % CHA) ^ row_key(ta_row, CHA)) * EPC) * (uint32_t)sizeof(T);
+    const uint32_t tb_off = (uint32_t)(tb_row * ldb + ((lane % CHB) ^ row_key(tb_row, CHB)) * EPC) * (uint32_t)sizeof(T);
     // A rows beyond M (a ragged last tile row) are read from row M-1 instead: one byte offset per DMA round, set per
     // tile.  What the MFMAs make of those rows is never stored (the epilogue's buffer stores are bounds-checked).
     uint32_t a_lane_off[A_ROUNDS];
@@ -128,7 +133,7 @@ __device__ __forceinline__ void gemm_dma_tiles(
             a_lane_off[r] = (uint32_t)(row * (kTurned ? lda : K) + (lp ^ key_dma) * EPC) * (uint32_t)sizeof(T);
         }
         if constexpr (kTurned) {
-            auto packets = [](int cols) { return (cols + 7) / 8 * 8; };      // A's rows are padded to whole chunks
+            auto packets = [](int cols) { return (cols + EPC - 1) / EPC * EPC; };      // A's rows are padded to whole chunks
             a_rsrc = TA ? rest_of_rows(A + m0, K, lda, packets(M - m0)) : rest_of_rows(A + (int64_t)m0 * lda, M - m0, lda, packets(K * segments));
             static_assert(TB, "B is turned wherever A may be");
             b_rsrc0 = rest_of_rows(B0 + n0, K, ldb, N - n0);
@@ -213,19 +218,27 @@ __device__ __forceinline__ void gemm_dma_tiles(
 #pragma unroll
     for (int ks = 0; ks < KSTEPS; ++ks) pc[ks] = ((ks * Shape::kChunks + fhalf) ^ key_f) << 4;
 
-    // turned: byte address of the lane's piece in fragment 0's place (bits 5 and up of it are XOR-ed per fragment)
-    const int t_row = fhalf * 8 + frow / 4;
-    int ta_lane = t_row * BM * (int)sizeof(T) + row_key(t_row, CHA) * 32 + (frow % 4) * 8;
-    int tb_lane = BM * BKT * (int)sizeof(T) + t_row * BN * (int)sizeof(T) + row_key(t_row, CHB) * 32 + (frow % 4) * 8;
+    // turned: byte address of the lane's piece in fragment 0's place; bits 5 to 7 (7 in fp32) of it are XOR-ed per fragment
+    const int t_row = sizeof(T) == 4 ? fhalf * 4 : fhalf * 8 + frow / 4, t_piece = sizeof(T) == 4 ? frow * 4 : (frow % 4) * 8;
+    int ta_lane = t_row * BM * (int)sizeof(T) + (row_key(t_row, CHA) * 16 ^ t_piece);
+    int tb_lane = BM * BKT * (int)sizeof(T) + t_row * BN * (int)sizeof(T) + (row_key(t_row, CHB) * 16 ^ t_piece);
     auto turned_frag = [&](const char* stage, int lane_at, int piece, int ks, int cols) {
-        typedef short i16x4_t __attribute__((__vector_size__(8)));
-        typedef __attribute__((address_space(3))) i16x4_t* tr_ptr;
-        const char* at = stage + (lane_at ^ ((piece & 7) * 32)) + (piece >> 3) * 256 + ks * 32 * cols * (int)sizeof(T);
-        const i16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((tr_ptr)at);
-        const i16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((tr_ptr)(at + 4 * cols * (int)sizeof(T)));
-        typedef short i16x8_t __attribute__((__vector_size__(16)));
-        const i16x8_t both = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
-        return __builtin_bit_cast(Frag, both);
+        constexpr int kBytes = FR * (int)sizeof(T), kInKey = 256 / kBytes;       // bytes of a fragment's columns in a k-row
+        const char* at = stage + (lane_at ^ ((piece % kInKey) * kBytes)) + (piece / kInKey) * 256 + ks * (BKT / KSTEPS) * cols * (int)sizeof(T);
+        if constexpr (sizeof(T) == 4) {
+            Frag f;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) f[q] = *reinterpret_cast<const float*>(at + q * cols * 4);
+            return f;
+        } else {
+            typedef short i16x4_t __attribute__((__vector_size__(8)));
+            typedef short i16x8_t __attribute__((__vector_size__(16)));
+            typedef __attribute__((address_space(3))) i16x4_t* tr_ptr;
+            const i16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((tr_ptr)at);
+            const i16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((tr_ptr)(at + 4 * cols * (int)sizeof(T)));
+            const i16x8_t both = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+            return __builtin_bit_cast(Frag, both);
+        }
     };
 
     int tile = block;
@@ -249,13 +262,13 @@ __device__ __forceinline__ void gemm_dma_tiles(
         const int ks = q / SPLIT, part = q % SPLIT;
 #pragma unroll
         for (int i = 0; i < MFS; ++i) {
-            if constexpr (TA) a[i] = turned_frag(stage, ta_lane, wm * (WM / 16) + part * MFS + i, ks, BM);
+            if constexpr (TA) a[i] = turned_frag(stage, ta_lane, wm * (WM / FR) + part * MFS + i, ks, BM);
             else a[i] = *reinterpret_cast<const Frag*>(stage + a_row_bytes + pc[ks] + (part * MFS + i) * FR * BKT * (int)sizeof(T));
         }
         if (part == 0) {
 #pragma unroll
             for (int j = 0; j < NF; ++j) {
-                if constexpr (TB) b[j] = turned_frag(stage, tb_lane, wn * (WN / 16) + j, ks, BN);
+                if constexpr (TB) b[j] = turned_frag(stage, tb_lane, wn * (WN / FR) + j, ks, BN);
                 else b[j] = *reinterpret_cast<const Frag*>(stage + b_row_bytes[j] + pc[ks]);
             }
         }
@@ -296,7 +309,7 @@ __device__ __forceinline__ void gemm_dma_tiles(
                 const int nxt = q + PF;
                 constexpr int kMfmas = MFS * NF;     // runs of Shape::kInstr instructions
                 const bool reads = nxt < SPK || !kLast;
-                constexpr int RA = TA ? 2 : 1, RB = TB ? 2 : 1;       // LDS reads per fragment
+                constexpr int RT = sizeof(T) == 4 ? 4 : 2, RA = TA ? RT : 1, RB = TB ? RT : 1;       // LDS reads per fragment
                 const int n_reads = RA * MFS + ((nxt % SPLIT) == 0 ? RB * NF : 0);
                 __builtin_amdgcn_sched_barrier(0);
                 if (nxt < SPK) {

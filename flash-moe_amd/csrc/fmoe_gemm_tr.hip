@@ -1,15 +1,16 @@
 // Products of the backward passes whose operands do not lie K-contiguous, for gfx950:
 //   NN   C[M,N] = A[M,K] B[K,N]          (dh = dy Wd, dx = [da | db] [Wg; Wu], dq = d Wr)
 //   TN   C[M,N] = A[K,M]^T B[K,N]        (the weight gradients)
-// 16-bit operands run on the LDS pipeline of the forward's products (fmoe_gemm.h): a turned operand is brought into the LDS as it lies, k-row
-// by k-row, and turned by the LDS itself on the way to the matrix cores (ds_read_b64_tr_b16).  fp32 has no such read and goes to the library.
+// They run on the LDS pipeline of the forward's products (fmoe_gemm.h): a turned operand is brought into the LDS as it lies, k-row by
+// k-row, and turned on the way to the matrix cores, in the 16-bit types by the LDS itself (ds_read_b64_tr_b16), in fp32 because a
+// lane reads its k values one by one.  Operands that are not whole 16-byte packets go to the library.
 //
 // What bounds it is what bounds the forward's products: what a compute unit receives on small tiles, the matrix pipes on 256 x 256,
 // and, with few tiles and a long k loop, the length of one chain, which slices of k cut (their sums are added by a second launch, in
-// slice order).  Against the library's kernels, us: training step of 2048 tokens, 4096 -> 16384: dh 208 for 211, dx 381 for 446, dWd
-// 228 for 254, dWg and dWu 458 for 509; 479 tokens, 3304 -> 13216: 53 for 65, 100 for 258, 58 for 109, 123 for 191; 615 tokens, 776
-// -> 2072: 9 for 20, 16 for 28, 8 for 19, 11 for 21.  A kernel that turned the operands in registers reached 600 TFLOP/s where these
-// reach 1000 to 1300.
+// slice order).  Against the library's kernels, us: 2048 tokens, 4096 -> 16384: dh 211 for 207, dx 435 for 435, dWd 225 for 252, dWg
+// and dWu 445 for 494; 479 tokens, 3304 -> 13216: 60 for 67, 105 for 258, 60 for 110, 114 for 192; 615 tokens, 776 -> 2072: 8 for 19,
+// 20 for 28, 8 for 19, 11 for 20; fp32, 383 tokens, 1880 -> 7520: 114 for 97, 207 for 826, 111 for 118, 182 for 228.  A kernel that
+// turned the operands in registers reached 600 TFLOP/s in bf16 where these reach 1000 to 1200.
 #include "fmoe_common.h"
 #include "fmoe_gemm.h"
 #include "fmoe_vec.h"
@@ -23,7 +24,7 @@ __global__ __launch_bounds__(2 * WAVES_N * kWave) void gemm_turned_kernel(
     const T* __restrict__ A, int lda, const T* __restrict__ B0, const T* __restrict__ B1, int ldb, T* __restrict__ C, int M, int N, int K,
     int segments, int tiles_m, int tiles_n, int xcds, int slices) {
     const int tiles = tiles_m * tiles_n, block = (int)blockIdx.x;
-    gemm_dma_tiles<T, BM, BN, 2, WAVES_N, kStageK<T>, NSTAGE, SLICED ? kEpiPart : kEpiPlain, 1, 16, BM == 256 ? kBigSplit<T> : 1, true, SLICED,
+    gemm_dma_tiles<T, BM, BN, 2, WAVES_N, kStageK<T>, NSTAGE, SLICED ? kEpiPart : kEpiPlain, kSmallAhead<T>, kFragRows<T>, BM == 256 ? kBigSplit<T> : 1, true, SLICED,
                    TA, true>(A, B0, B1, C, nullptr, M, N, K, tiles_m, tiles_n, xcds, SLICED ? block % tiles : block,
                              SLICED ? tiles : (int)gridDim.x, SLICED ? block / tiles : 0, slices, lda, ldb, segments);
 }
@@ -50,13 +51,13 @@ __global__ __launch_bounds__(256) void gemm_turned_add_kernel(const float* __res
 // Tile shape and slices of k by price (us): a round of tiles costs what the forward's rule says, 2.3 ns per received row and k-tile,
 // plus the stores of its tiles, which nothing hides on 256 x 256 (7 us; the smaller tiles overlap them with other workgroups); slices,
 // as long as they are one round, add a launch of 4 us and their planes, written and read at 6 TB/s.
-SlicePlan plan_turned(int M, int N, int K, int segments) {
-    const int cus = chip_info().cus, k_tiles = (K + kStageK<bf16_t> - 1) / kStageK<bf16_t> * segments;
+template <typename T> SlicePlan plan_turned(int M, int N, int K, int segments) {
+    const int cus = chip_info().cus, k_tiles = (K + kStageK<T> - 1) / kStageK<T> * segments;
     SlicePlan best = {kTile64, 1};
     double best_time = 0.0;
-    for (int i = kTile256; i <= kTile64; ++i) {
+    for (int i = sizeof(T) == 4 ? kTile128 : kTile256; i <= kTile64; ++i) {
         int64_t n = 0;
-        const double row = tile_cost<bf16_t, kEpiPlain>(i, M, N, n) * 2.3e-3, stores = i == kTile256 ? 7.0 : 1.0;
+        const double row = tile_cost<T, kEpiPlain>(i, M, N, n) * 2.3e-3, stores = i == kTile256 ? 7.0 : 1.0;
         for (int s = 1; s <= kMaxSlices && (s == 1 || (n * s <= cus && 2 * s <= k_tiles)); ++s) {
             const int share = (k_tiles + s - 1) / s;
             if ((s - 1) * share >= k_tiles) continue;                 // a slice would have no k-tile
@@ -86,7 +87,7 @@ void launch_turned(const void* A, int lda, const void* B0, const void* B1, int l
                        0, stream, (const T*)A, lda, (const T*)B0, (const T*)B1, ldb, (T*)planes, M, N, K, segments, tm, tn, xcds, p.slices)
     if (p.slices > 1) {
         switch (p.shape) {
-            case kTile256: FMOE_SLICED(256, 256, 4, 2); break;
+            case kTile256: if constexpr (sizeof(T) == 2) FMOE_SLICED(256, 256, 4, 2); break;
             case kTile128: FMOE_SLICED(128, 128, 2, 4); break;
             case kTile64x128: FMOE_SLICED(64, 128, 2, 4); break;
             default: FMOE_SLICED(64, 64, 2, 4); break;
@@ -97,7 +98,7 @@ void launch_turned(const void* A, int lda, const void* B0, const void* B1, int l
         return;
     }
     switch (p.shape) {
-        case kTile256: FMOE_WHOLE(256, 256, 4, 2, 1); break;
+        case kTile256: if constexpr (sizeof(T) == 2) FMOE_WHOLE(256, 256, 4, 2, 1); break;
         case kTile128:
             if (n <= cus) FMOE_WHOLE(128, 128, 2, 4, 1);
             else FMOE_WHOLE(128, 128, 2, 2, 2);
@@ -112,8 +113,7 @@ void launch_turned(const void* A, int lda, const void* B0, const void* B1, int l
 }  // namespace
 
 size_t gemm_backward_workspace_bytes(int M, int N, int K, int segments, int dtype) {
-    if (dtype == FMOE_F32) return 0;
-    const int slices = plan_turned(M, N, K, segments).slices;
+    const int slices = (dtype == FMOE_F32 ? plan_turned<float>(M, N, K, segments) : plan_turned<bf16_t>(M, N, K, segments)).slices;
     return slices > 1 ? (size_t)slices * M * N * sizeof(float) : 0;
 }
 
@@ -121,22 +121,25 @@ int gemm_backward(int layout, int M, int N, int K, const void* A, int lda, const
                   void* workspace, size_t workspace_bytes, hipStream_t stream) {
     const int segments = B1 != nullptr ? 2 : 1;
     // whole packets: where M (TN) or K (NN) is none, the rows of A are padded with zeros up to lda
-    const int a_cols = layout == kBlasTN ? M : K * segments;
-    const bool packets = lda % 8 == 0 && ldb % 8 == 0 && N % 8 == 0 && (a_cols + 7) / 8 * 8 <= lda && (segments == 1 || K % 8 == 0) &&
-                         aligned16(A) && aligned16(B0) && aligned16(B1) && aligned16(C);
+    const int a_cols = layout == kBlasTN ? M : K * segments, vec = dtype == FMOE_F32 ? 4 : 8;
+    const bool packets = lda % vec == 0 && ldb % vec == 0 && N % vec == 0 && (a_cols + vec - 1) / vec * vec <= lda &&
+                         (segments == 1 || K % vec == 0) && aligned16(A) && aligned16(B0) && aligned16(B1) && aligned16(C);
     // 32-bit byte offsets inside a descriptor
-    const bool reach = (double)K * ldb < 1.0e9 && (layout == kBlasTN ? (double)K * lda < 1.0e9 : 256.0 * lda < 1.0e9);
-    if (dtype != FMOE_F32 && packets && reach) {
-        SlicePlan p = plan_turned(M, N, K, segments);
+    const double most = dtype == FMOE_F32 ? 5.0e8 : 1.0e9;
+    const bool reach = (double)K * ldb < most && (layout == kBlasTN ? (double)K * lda < most : 256.0 * lda < most);
+    if (packets && reach) {
+        SlicePlan p = dtype == FMOE_F32 ? plan_turned<float>(M, N, K, segments) : plan_turned<bf16_t>(M, N, K, segments);
         if ((size_t)p.slices * M * N * sizeof(float) > workspace_bytes) p.slices = 1;
         float* planes = (float*)workspace;
-#define FMOE_TURNED(TT, TA) launch_turned<TT, TA>(A, lda, B0, B1, ldb, C, M, N, K, segments, p, planes, stream)
-        if (layout == kBlasTN) {
-            if (dtype == FMOE_BF16) FMOE_TURNED(bf16_t, true);
-            else FMOE_TURNED(f16_t, true);
-        } else {
-            if (dtype == FMOE_BF16) FMOE_TURNED(bf16_t, false);
-            else FMOE_TURNED(f16_t, false);
+#define FMOE_TURNED(TT)                                                                                                       \
+    do {                                                                                                                      \
+        if (layout == kBlasTN) launch_turned<TT, true>(A, lda, B0, B1, ldb, C, M, N, K, segments, p, planes, stream);         \
+        else launch_turned<TT, false>(A, lda, B0, B1, ldb, C, M, N, K, segments, p, planes, stream);                          \
+    } while (0)
+        switch (dtype) {
+            case FMOE_F32: FMOE_TURNED(float); break;
+            case FMOE_BF16: FMOE_TURNED(bf16_t); break;
+            default: FMOE_TURNED(f16_t); break;
         }
 #undef FMOE_TURNED
         FMOE_CHECK_LAUNCH("backward product");

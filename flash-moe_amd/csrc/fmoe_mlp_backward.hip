@@ -3,8 +3,8 @@
 // The forward keeps only silu(a) * b unless it was asked to keep the gate and up products a, b as well
 // (fmoe_mlp_gate_up_save); without them they are recomputed here (two launches of the forward's own NT GEMM).  The SwiGLU gradient is the fused
 // elementwise kernel of fmoe_backward.hip (it also rebuilds h = silu(a) * b for dWd).  The remaining products are
-// plain GEMMs in layouts the forward never needs (A B and A^T B): gemm_backward (fmoe_gemm_tr.hip) runs them in the 16-bit types;
-// fp32 goes to rocBLAS, which is loaded on first use so that the other paths carry no dependency on it:
+// plain GEMMs in layouts the forward never needs (A B and A^T B): gemm_backward (fmoe_gemm_tr.hip).  What its kernels cannot
+// address goes to rocBLAS, which is loaded on first use so that nothing else depends on it:
 //     dh  = dy Wd              [T,H][H,I]
 //     dWd = dy^T h             [T,H]^T [T,I]
 //     dx  = da Wg + db Wu      [T,I][I,H] twice, the second accumulating

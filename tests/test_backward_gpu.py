@@ -555,6 +555,11 @@ def test_mlp_backward_remainders_of_the_transposing_products(dtype, T, H, I):
     assert all(torch.equal(a, b) for a, b in zip(got, mlp_backward(dy, x, *ws, saved)))      # bit for bit the same twice
 
 
+@pytest.mark.parametrize("T,H,I", [(1, 4, 8), (65, 68, 1028), (300, 264, 2060), (383, 516, 1544), (900, 1032, 2056), (2500, 264, 2052)])
+def test_mlp_backward_remainders_of_the_transposing_products_fp32(T, H, I):
+    test_mlp_backward_remainders_of_the_transposing_products(torch.float32, T, H, I)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("T,H,I", [
     (500, 2056, 4104),       # 128 x 128 tiles, one and two to a compute unit, and slices of k
