@@ -59,7 +59,7 @@ SavedPlan plan_saved(int64_t T_, int H, int I, int nk, int64_t E, int K, int dty
     p.off_indices = take((size_t)T_ * K * 8);
     p.off_gates = take((size_t)T_ * K * elt);
     p.off_stats = take((size_t)2 * H * 4);
-    p.off_products = take((size_t)2 * T_ * I * elt);
+    p.off_products = take((size_t)3 * T_ * I * elt);      // gate, up, and silu(gate) * up
     p.off_experts = take(fmoe_expert_saved_bytes(T_, H, E, K, dtype));
     p.bytes = o;
     return p;
@@ -132,6 +132,7 @@ int block_forward_impl(const char* who, const void* x, const void* gate_proj_w, 
     void* gates = gates_out ? gates_out : (void*)(ws + p.off_gates);
     float* stats = nullptr;
     void* products = nullptr;
+    void* act = ws + p.off_act;
     void* expert_saved = nullptr;
     if (saved != nullptr) {
         const SavedPlan sp = plan_saved(num_tokens, hidden, intermediate, num_keys, num_experts, top_k, dtype);
@@ -141,9 +142,9 @@ int block_forward_impl(const char* who, const void* x, const void* gate_proj_w, 
         gates = saved + sp.off_gates;
         stats = (float*)(saved + sp.off_stats);
         products = saved + sp.off_products;
+        act = saved + sp.off_products + (size_t)2 * num_tokens * intermediate * dtype_size(dtype);
     }
     void* expert_ws = ws + p.off_expert;
-    void* act = ws + p.off_act;
     void* experts = ws + p.off_experts_out;
     const size_t elt = dtype_size(dtype);
 
@@ -204,7 +205,7 @@ int block_forward_impl(const char* who, const void* x, const void* gate_proj_w, 
         if ((rc = gate_up())) return rc;
     const size_t act_bytes = fmoe_mlp_workspace_bytes(num_tokens, hidden, intermediate, dtype);
     const size_t planes = fmoe_mlp_down_workspace_bytes(num_tokens, hidden, intermediate, dtype);
-    return fmoe_mlp_down_ws(act, down_proj_w, num_tokens, hidden, intermediate, dtype, residual, out, (char*)act + (act_bytes - planes), planes,
+    return fmoe_mlp_down_ws(act, down_proj_w, num_tokens, hidden, intermediate, dtype, residual, out, ws + p.off_act + (act_bytes - planes), planes,
                             stream);
 }
 
@@ -280,7 +281,9 @@ extern "C" int fmoe_block_backward(const void* dout, const void* dlogits, const 
     char* ws = (char*)workspace;
     void *dgates = ws + p.off_dgates, *dx_experts = ws + p.off_dx_experts, *stage = ws + p.off_stage;
     float* dlogits32 = (float*)(ws + p.off_dlogits32);
-    int rc = fmoe_mlp_backward(dout, x, gate_proj_w, up_proj_w, down_proj_w, sv + sp.off_products, num_tokens, hidden, intermediate,
+    const char* products = sv + sp.off_products;
+    int rc = fmoe_mlp_backward_act(dout, x, gate_proj_w, up_proj_w, down_proj_w, products,
+                               products + (size_t)2 * num_tokens * intermediate * dtype_size(dtype), num_tokens, hidden, intermediate,
                                dtype, dx, dgate_proj_w, dup_proj_w, ddown_proj_w, stage, p.stage_bytes, stream);
     if (rc) return rc;
     rc = fmoe_expert_backward_saved(dout, x, down_embed, up_embed, indices, sv + sp.off_gates, sv + sp.off_experts, num_tokens, hidden,

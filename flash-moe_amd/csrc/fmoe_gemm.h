@@ -639,18 +639,20 @@ template <typename T> SlicePlan plan_slices_of_k(int M, int N, int K) {
     SlicePlan best = {-1, 1};
     int tiles = 0;
     double whole = 0.0;
-    const bool split_k = choose_tile<T, kEpiPlain>(M, N, tiles, &whole) >= kSplit32;
+    const TileShape shape = choose_tile<T, kEpiPlain>(M, N, tiles, &whole);
+    const bool split_k = shape >= kSplit32;
     const int cus = chip_info().cus, k_tiles = (K + kStageK<T> - 1) / kStageK<T>;
     const double kRow = 2.3e-3, launch = split_k ? 8.5 : 4.0;
     double best_time = (split_k ? 0.8 : 0.9) * whole * k_tiles * kRow;
+    if (shape == kTile128 && tiles > cus) best_time *= 0.65;       // two to a compute unit hide each other's latency
     if (sizeof(T) == 4 && K % 4 != 0) return best;
-    for (int i = kTile128; i <= kTile64; ++i) {
+    for (int i = sizeof(T) == 2 ? kTile256 : kTile128; i <= kTile64; ++i) {
         int64_t n = 0;
         const double round = tile_cost<T, kEpiPlain>(i, M, N, n);
         for (int s = 2; s <= kMaxSlices && n * s <= cus && s * 4 <= k_tiles; ++s) {
             const int share = (k_tiles + s - 1) / s;
             if ((s - 1) * share >= k_tiles) continue;           // a slice would have no k-tile
-            const double time = round * share * kRow + launch + 8.0e-6 * s * (double)M * N / 6.0;
+            const double time = round * share * kRow + launch + (i == kTile256 ? 7.0 : 0.0) + 8.0e-6 * s * (double)M * N / 6.0;
             if (time < best_time) {
                 best = {i, s};
                 best_time = time;

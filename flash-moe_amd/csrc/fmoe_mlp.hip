@@ -44,11 +44,12 @@ __global__ __launch_bounds__(kSplitWaves * 64) void gemm_splitk_kernel(
     gemm_splitk_tile<T, MT, NT, EPI>(A, B0, B1, C, R, M, N, K, tiles_m, tiles, xcds, (int)blockIdx.x, (int)gridDim.x, lds);
 }
 
-template <typename T, int BM, int BN, int NSTAGE>
-__global__ __launch_bounds__(256) void gemm_sliced_kernel(const T* __restrict__ A, const T* __restrict__ B, float* __restrict__ planes, int M,
+template <typename T, int BM, int BN, int WAVES_N, int NSTAGE>
+__global__ __launch_bounds__(2 * WAVES_N * 64) void gemm_sliced_kernel(const T* __restrict__ A, const T* __restrict__ B, float* __restrict__ planes, int M,
                                                           int N, int K, int tiles_m, int tiles_n, int xcds, int slices) {
     const int tiles = tiles_m * tiles_n;
-    gemm_dma_tiles<T, BM, BN, 2, 2, kStageK<T>, NSTAGE, kEpiPart, kSmallAhead<T>, kFragRows<T>, 1, true, true>(
+    gemm_dma_tiles<T, BM, BN, 2, WAVES_N, kStageK<T>, NSTAGE, kEpiPart, BM == 256 ? 1 : kSmallAhead<T>, kFragRows<T>,
+                   BM == 256 ? kBigSplit<T> : 1, true, true>(
         A, B, nullptr, reinterpret_cast<T*>(planes), nullptr, M, N, K, tiles_m, tiles_n, xcds, (int)blockIdx.x % tiles, tiles,
         (int)blockIdx.x / tiles, slices);
 }
@@ -199,12 +200,16 @@ int gate_up_tiled(const void* x, const void* wg, const void* wu, int M, int H, i
 template <typename T>
 void launch_sliced(const T* A, const T* B, T* C, const T* R, int M, int N, int K, const SlicePlan& p, float* planes, hipStream_t stream) {
     const int tiles_m = (M + kTileRows[p.shape] - 1) / kTileRows[p.shape], tiles_n = (N + kTileCols[p.shape] - 1) / kTileCols[p.shape];
-    const dim3 grid((unsigned)(tiles_m * tiles_n * p.slices)), block(256);
-#define FMOE_GO(BM, BN) \
-    hipLaunchKernelGGL((gemm_sliced_kernel<T, BM, BN, 4>), grid, block, 0, stream, A, B, planes, M, N, K, tiles_m, tiles_n, chip_info().xcds, p.slices)
-    if (p.shape == kTile128) FMOE_GO(128, 128);
-    else if (p.shape == kTile64x128) FMOE_GO(64, 128);
-    else FMOE_GO(64, 64);
+    const dim3 grid((unsigned)(tiles_m * tiles_n * p.slices));
+#define FMOE_GO(BM, BN, WAVES_N, NSTAGE)                                                                                            \
+    hipLaunchKernelGGL((gemm_sliced_kernel<T, BM, BN, WAVES_N, NSTAGE>), grid, dim3(128 * WAVES_N), 0, stream, A, B, planes, M, N, K, \
+                       tiles_m, tiles_n, chip_info().xcds, p.slices)
+    switch (p.shape) {
+        case kTile256: if constexpr (sizeof(T) == 2) FMOE_GO(256, 256, 4, 2); break;
+        case kTile128: FMOE_GO(128, 128, 2, 4); break;
+        case kTile64x128: FMOE_GO(64, 128, 2, 4); break;
+        default: FMOE_GO(64, 64, 2, 4); break;
+    }
 #undef FMOE_GO
     const int64_t elements = (int64_t)M * N;
     hipLaunchKernelGGL((add_slices_kernel<T>), dim3((unsigned)((elements + 1023) / 1024)), dim3(256), 0, stream, (const float*)planes, R, C,

@@ -2,7 +2,8 @@
 //
 // The forward keeps only silu(a) * b unless it was asked to keep the gate and up products a, b as well
 // (fmoe_mlp_gate_up_save); without them they are recomputed here (two launches of the forward's own NT GEMM).  The SwiGLU gradient is the fused
-// elementwise kernel of fmoe_backward.hip (it also rebuilds h = silu(a) * b for dWd).  The remaining products are
+// elementwise kernel of fmoe_backward.hip (it also rebuilds h = silu(a) * b for dWd unless the caller kept that too: a sixth of
+// what it moves).  The remaining products are
 // plain GEMMs in layouts the forward never needs (A B and A^T B): gemm_backward (fmoe_gemm_tr.hip).  What its kernels cannot
 // address goes to rocBLAS, which is loaded on first use so that nothing else depends on it:
 //     dh  = dy Wd              [T,H][H,I]
@@ -122,6 +123,13 @@ extern "C" size_t fmoe_mlp_backward_workspace_bytes(int64_t num_tokens, int hidd
 extern "C" int fmoe_mlp_backward(const void* dy, const void* x, const void* gate_w, const void* up_w, const void* down_w,
                                  const void* saved_products, int64_t num_tokens, int hidden, int intermediate, int dtype, void* dx, void* dgate_w, void* dup_w,
                                  void* ddown_w, void* workspace, size_t workspace_bytes, void* stream) {
+    return fmoe_mlp_backward_act(dy, x, gate_w, up_w, down_w, saved_products, nullptr, num_tokens, hidden, intermediate, dtype, dx, dgate_w,
+                                 dup_w, ddown_w, workspace, workspace_bytes, stream);
+}
+
+extern "C" int fmoe_mlp_backward_act(const void* dy, const void* x, const void* gate_w, const void* up_w, const void* down_w,
+                                     const void* saved_products, const void* act, int64_t num_tokens, int hidden, int intermediate, int dtype,
+                                     void* dx, void* dgate_w, void* dup_w, void* ddown_w, void* workspace, size_t workspace_bytes, void* stream) {
     using namespace fmoe;
     clear_error();
     FMOE_REQUIRE(dtype_ok(dtype), FMOE_ERR_BAD_DTYPE, "fmoe_mlp_backward: unknown dtype %d", dtype);
@@ -162,9 +170,10 @@ extern "C" int fmoe_mlp_backward(const void* dy, const void* x, const void* gate
     // da and db side by side: one [T, 2I] matrix [da | db], so that products over both are single calls
     char* db = dab + (size_t)I * elt;
     const int I2 = 2 * I;
-    rc = launch_swiglu_backward(dh, a, b, dab, db, h, num_tokens, I, I2, I2, dtype, s);
+    // h = silu(a) * b is what the forward multiplied with Wd: kept, or rebuilt here
+    rc = launch_swiglu_backward(dh, a, b, dab, db, act != nullptr ? nullptr : h, num_tokens, I, I2, I2, dtype, s);
     if (rc) return rc;
-    rc = gemm_backward(kTN, H, I, T_, dy, H, h, nullptr, I, ddown_w, dtype, part, p.part_bytes, s);                         // dWd = dy^T h
+    rc = gemm_backward(kTN, H, I, T_, dy, H, act != nullptr ? act : h, nullptr, I, ddown_w, dtype, part, p.part_bytes, s);                         // dWd = dy^T h
     if (rc) return rc;
     rc = gemm_backward(kNN, T_, H, I, dab, I2, gate_w, up_w, H, dx, dtype, part, p.part_bytes, s);                          // dx = da Wg + db Wu
     if (rc) return rc;

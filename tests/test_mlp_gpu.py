@@ -179,3 +179,8 @@ def test_mlp_down_with_slices_of_k(dtype, T, H, I, with_residual):
     tol = {torch.float32: 2e-6, torch.bfloat16: 6e-3, torch.float16: 8e-4}[dtype]
     assert rel_fro(out, want) < tol and rel_fro(out, whole.cpu()) < tol
     assert (buf[:8] == 7).all() and (buf[-8:] == 7).all() and (ws[:256] == 7).all() and (ws[-256:] == 7).all()
+
+
+@pytest.mark.parametrize("T,H,I", [(300, 4104, 16392), (1000, 2056, 16392)])
+def test_mlp_down_with_slices_of_k_on_the_largest_tiles(T, H, I):
+    test_mlp_down_with_slices_of_k(torch.bfloat16, T, H, I, True)
