@@ -238,8 +238,10 @@ __device__ __forceinline__ void router_gate_splitk_tile(
 #pragma unroll
             for (int d = 0; d < kAhead; ++d) {
                 const int u = u0 + d;
-                // steps past the end multiply zeros; their statistics are read from the last valid place
+                // Steps and pieces past the end multiply zeros.  Their q has to be zero as well as their weights: their statistics are
+                // other columns' (staged ones are zero beyond K), whose (0 - mean) * rstd may be infinite in T.
                 const int k0 = u < steps ? k_of(u) : 0;
+                const uint32_t keep = u < steps && (STAGED || k0 + piece * V < K) ? ~0u : 0u;
                 float mean[V], rstd[V];
 #pragma unroll
                 for (int c = 0; c < V / 4; ++c) {
@@ -261,7 +263,7 @@ __device__ __forceinline__ void router_gate_splitk_tile(
                 }
 #pragma unroll
                 for (int i = 0; i < MT; ++i) {
-                    const u32x4_t q = normalise16<T>(fa[d][i], mean, rstd);
+                    const u32x4_t q = normalise16<T>(fa[d][i], mean, rstd) & keep;
 #pragma unroll
                     for (int j = 0; j < NT; ++j) acc[i][j] = mfma16_packet<T>(q, fb[d][j], acc[i][j]);
                 }

@@ -260,6 +260,57 @@ def test_gate_logits_at_the_edges_of_the_tile_shapes(dtype, training, T, H, nk):
         torch.testing.assert_close(bn.running_var.cpu().double(), 0.9 * rv.double() + 0.1 * x64.var(0), rtol=tol, atol=tol)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("training", [True, False])
+@pytest.mark.parametrize("T,H", [(8, 1024), (64, 520), (300, 1536), (40, 1024), (2000, 1024)])
+def test_gate_logits_with_a_constant_column_of_large_mean(dtype, training, T, H):
+    """A constant column has 1/std = 316, so its mean of 300 times that is beyond fp16.  Its normalised value is zero and so are its
+    contributions, also where a wave of the k-splitting kernel multiplies steps past the end of its share of k."""
+    from flash_moe.modules.flash_moe import FlashMoE, FlashMoEConfig
+
+    nk = 32
+    g = torch.Generator().manual_seed(T + H)
+    x = (torch.randn(T, H, generator=g) * 1.7 + 0.3).to(dtype)
+    wr = (torch.randn(2 * nk, H, generator=g) * 0.02).to(dtype)
+    rm, rv = torch.randn(H, generator=g).to(dtype), (torch.rand(H, generator=g) + 0.5).to(dtype)
+    constant = [5, 31, H // 2 + 3]
+    x[:, constant], rm[constant], rv[constant] = 300.0, 300.0, 0.0
+    (logits, *_, logits32), bn = _fused(x.float(), wr.float(), nk, 2, False, dtype, training=training, rm=rm.float(), rv=rv.float())
+    x64 = x.double()
+    mean, var = (x64.mean(0), x64.var(0, unbiased=False)) if training else (rm.double(), rv.double())
+    want = ((x64 - mean) / (var + 1e-5).sqrt()).to(dtype).double() @ wr.double().t()
+    err = (logits32.cpu().double() - want).norm() / want.norm()
+    assert err < {torch.float32: 1e-6, torch.bfloat16: 5e-4, torch.float16: 1e-4}[dtype], err
+    # the same gate inside the block, beside the MLP's gate and up products
+    m = FlashMoE(FlashMoEConfig(H, 264, "silu", nk * nk, 4)).to(device="cuda", dtype=dtype).train(training)
+    with torch.no_grad():
+        m.router_gate.weight.copy_(wr)
+        m.router_norm.running_mean.copy_(rm), m.router_norm.running_var.copy_(rv)
+        _, block_logits = m(x.cuda().unsqueeze(0))
+    # one more rounding, to dtype
+    err = (block_logits.transpose(0, 1).reshape(T, 2 * nk).cpu().double() - want).norm() / want.norm()
+    assert err < {torch.float32: 1e-6, torch.bfloat16: 4e-3, torch.float16: 5e-4}[dtype], err
+
+
+def test_split_gate_logits_with_a_half_that_is_not_whole_lines():
+    """Above 4096 columns the statistics are read, not staged: past the end of the first half they are those of the second half's
+    columns, whose zero activations may normalise to infinity."""
+    from flash_moe.ops.hip.flash_router import router_forward
+
+    T, H, nk, dtype = 40, 4112, 64, torch.float16
+    g = torch.Generator().manual_seed(9)
+    x = torch.randn(T, H, generator=g).to(dtype)
+    x[:, H // 2:H // 2 + 24] = 300.0
+    tables = (torch.randn(2 * nk, H // 2, generator=g) * 0.02).to(dtype)
+    bn = torch.nn.BatchNorm1d(H, affine=False).to(device="cuda", dtype=dtype)
+    logits32 = router_forward(x.cuda(), tables.cuda(), bn, nk, 2, False, return_logits32=True, split_query=True)[4]
+    x64 = x.double()
+    q = ((x64 - x64.mean(0)) / (x64.var(0, unbiased=False) + 1e-5).sqrt()).to(dtype).double()
+    want = torch.cat([q[:, :H // 2] @ tables[:nk].double().t(), q[:, H // 2:] @ tables[nk:].double().t()], dim=1)
+    err = (logits32.cpu().double() - want).norm() / want.norm()
+    assert err < 1e-4, err
+
+
 def test_fused_router_eval_mode_and_normalised_gates():
     T, H, nk, K = 300, 128, 64, 32
     g = torch.Generator().manual_seed(5)
