@@ -65,6 +65,15 @@ bool records_gradient(std::initializer_list<const Tensor*> tensors) {
     return false;
 }
 
+// Forward-mode derivatives are not implemented.  An input that carries a tangent is refused, as torch refuses it for an autograd
+// function without one, whether or not a node would be recorded: an output without a tangent reads as a zero derivative.
+void refuse_tangents(std::initializer_list<const Tensor*> tensors) {
+    if (!c10::AutogradState::get_tls_state().get_fw_grad_mode()) return;
+    for (const Tensor* t : tensors)
+        if (t->defined() && t->_fw_grad(/*level=*/0).defined())
+            C10_THROW_ERROR(NotImplementedError, "forward-mode differentiation is not implemented for the flash_moe ops");
+}
+
 // ---- router -----------------------------------------------------------------------------------------------------------
 std::tuple<Tensor, Tensor, OptTensor> router_topk(const Tensor& router_logits, int64_t nk, int64_t K, bool with_gates, bool norm) {
     TORCH_CHECK_VALUE(router_logits.size(2) == nk, "router_logits.size(-1)=", router_logits.size(2), " does not match num_expert_keys=", nk);
@@ -108,6 +117,7 @@ struct RouterNode : torch::autograd::Function<RouterNode> {
 };
 
 std::tuple<Tensor, Tensor> router_func(const Tensor& router_logits, int64_t nk, int64_t K) {
+    refuse_tangents({&router_logits});
     if (records_gradient({&router_logits})) {
         auto out = RouterNode::apply(router_logits, nk, K);
         return {out[0], out[1]};
@@ -210,6 +220,7 @@ struct PrologueNode : torch::autograd::Function<PrologueNode> {
 
 std::tuple<Tensor, Tensor> router_prologue(const Tensor& tokens, const Tensor& gate_weight, const Tensor& mean, const Tensor& var,
                                            const OptTensor& batches, bool training, double momentum, double eps) {
+    refuse_tangents({&tokens, &gate_weight});
     const Norm norm{mean, var, value(batches), training, momentum, eps};
     auto out = PrologueNode::apply(tokens, gate_weight, &norm);
     return {out[0], out[1]};
@@ -289,6 +300,7 @@ struct ExpertNode : torch::autograd::Function<ExpertNode> {
 };
 
 Tensor expert_func(const Tensor& x, const Tensor& down, const Tensor& up, const Tensor& indices, const Tensor& weights) {
+    refuse_tangents({&x, &down, &up, &weights});
     if (records_gradient({&x, &down, &up, &weights})) return ExpertNode::apply(x, down, up, indices, weights);
     return expert_forward(x, down, up, indices, weights, FMOE_EXPERT_AUTO);
 }
@@ -355,6 +367,7 @@ struct PeerNode : torch::autograd::Function<PeerNode> {
     }
 };
 Tensor peer_func(const Tensor& x, const Tensor& down, const Tensor& up, const Tensor& weights, const Tensor& indices) {
+    refuse_tangents({&x, &down, &up, &weights});
     if (records_gradient({&x, &down, &up, &weights})) return PeerNode::apply(x, down, up, weights, indices);
     return peer_forward(x, down, up, weights, indices);
 }
@@ -366,6 +379,7 @@ struct PkmNode : torch::autograd::Function<PkmNode> {
     }
 };
 Tensor pkm_func(const Tensor& values, const Tensor& weights, const Tensor& indices) {
+    refuse_tangents({&values, &weights});
     if (records_gradient({&values, &weights})) return PkmNode::apply(values, weights, indices);
     return pkm_forward(values, weights, indices);
 }
@@ -468,6 +482,7 @@ struct MlpNode : torch::autograd::Function<MlpNode> {
 };
 
 Tensor mlp_func(const Tensor& x, const Tensor& gate, const Tensor& up, const Tensor& down) {
+    refuse_tangents({&x, &gate, &up, &down});
     if (records_gradient({&x, &gate, &up, &down})) return MlpNode::apply(x, gate, up, down);
     return mlp_forward(x, gate, up, down, std::nullopt);
 }
@@ -584,6 +599,7 @@ struct BlockNode : torch::autograd::Function<BlockNode> {
 std::vector<Tensor> block(const Tensor& hidden_states, const Tensor& gate, const Tensor& up, const Tensor& down, const Tensor& router_gate,
                           const Tensor& down_embed, const Tensor& up_embed, const Tensor& mean, const Tensor& var, const OptTensor& batches,
                           bool training, double momentum, double eps, int64_t nk, int64_t K, bool norm, bool differentiable, bool return_routing) {
+    refuse_tangents({&hidden_states, &gate, &up, &down, &router_gate, &down_embed, &up_embed});
     const Norm bn{mean, var, value(batches), training, momentum, eps};
     if (differentiable && records_gradient({&hidden_states, &gate, &up, &down, &router_gate, &down_embed, &up_embed}))
         return BlockNode::apply(hidden_states, gate, up, down, router_gate, down_embed, up_embed, &bn, nk, K, norm);

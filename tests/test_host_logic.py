@@ -71,6 +71,42 @@ def test_router_assertions_match_reference_wording():
         flash_router_func(torch.zeros(2, 4, 8), 8, 9)
 
 
+@pytest.mark.parametrize("device", ["cpu", pytest.param("cuda", marks=pytest.mark.gpu)])
+@pytest.mark.parametrize("op", ["router", "expert", "mlp", "peer", "pkm", "prologue", "block", "frozen block"])
+def test_forward_mode_is_refused(op, device):
+    """A dual input raises, with and without gradients recorded: an output without a tangent would read as a zero derivative."""
+    import torch.autograd.forward_ad as fwAD
+
+    from flash_moe.ops import flash_expert_func, flash_mlp_func, flash_router_func, peer_func, pkm_func
+    from flash_moe.ops.hip.flash_router import router_prologue
+
+    T, H, I, E, K = 4, 16, 32, 100, 3
+    rand = lambda *shape: torch.randn(*shape, device=device)
+    x, table, gates, idx = rand(T, H), rand(E, H), rand(T, K), torch.zeros(T, K, dtype=torch.int64, device=device)
+    module = FlashMoE(FlashMoEConfig(H, I, "silu", E, K)).requires_grad_(op == "block").to(device)
+    calls = {
+        "router": (rand(2, T, 10), lambda d: flash_router_func(d, 10, K)),
+        "expert": (x, lambda d: flash_expert_func(d, table, table, idx, gates)),
+        "mlp": (x, lambda d: flash_mlp_func(d, rand(I, H), rand(I, H), rand(H, I))),
+        "peer": (gates, lambda d: peer_func(x, table, table, d, idx)),
+        "pkm": (table, lambda d: pkm_func(d, gates, idx)),
+        "prologue": (x, lambda d: router_prologue(d, rand(20, H), torch.nn.BatchNorm1d(H, affine=False).to(device))),
+        "block": (x.unsqueeze(0), module), "frozen block": (x.unsqueeze(0), module),
+    }
+    primal, call = calls[op]
+    with fwAD.dual_level():
+        dual = fwAD.make_dual(primal, torch.ones_like(primal))
+        with pytest.raises(NotImplementedError):
+            call(dual)
+        with torch.no_grad(), pytest.raises(NotImplementedError):
+            call(dual)
+        if device == "cuda":
+            call(primal)
+        else:
+            with pytest.raises(RuntimeError, match="GPU"):      # without a tangent the call goes on, to the refusal of CPU tensors
+                call(primal)
+
+
 def test_utils():
     assert [next_power_of_2(n) for n in (0, 1, 2, 3, 4, 5, 1023, 1024, 1025)] == [1, 1, 2, 4, 4, 8, 1024, 1024, 2048]
     seen = {}
