@@ -310,5 +310,12 @@ __device__ __forceinline__ void router_gate_splitk_tile(
 // Tiles of a launch with 16 mt x 16 nt outputs each.
 inline int64_t gate_tiles(int M, int N, int mt, int nt) { return (int64_t)((M + 16 * mt - 1) / (16 * mt)) * ((N + 16 * nt - 1) / (16 * nt)); }
 
+// Whether the gate product of these extents is the k-splitting kernel's, for the router alone and inside the block: the two have to
+// agree to the last bit, so one rule decides for both.  16-bit products beyond a round of 32 x 64 tiles are left to router_gate_kernel,
+// whose waves share the operands through LDS (4096 tokens, 1024 columns, 256 outputs: 20.6 us against 22.4 on 64 x 64 tiles here; 1024
+// tokens 18.2 there against 14.7 here); fp32 is bound by its matrix rate (2048 tokens: 25 us where a kernel of plain FMAs took 196;
+// 207 tokens, 1232 columns, 436 outputs: 13 for 194).
+inline bool gate_splitk_pays(int M, int N, int dtype) { return dtype == FMOE_F32 || gate_tiles(M, N, 2, 4) <= chip_info().cus; }
+
 }  // namespace
 }  // namespace fmoe

@@ -520,12 +520,7 @@ void launch_finalize(const float* partial, const ProloguePlan& p, int H, int tra
 }
 
 // The smallest tiles that still are one round of workgroups: 1024 tokens, 1024 columns, 256 outputs in bf16 take 14.7 us with the
-// statistics launch on 32 x 32 tiles (256 of them), 23 on 16 x 32 and 17 on 32 x 64; the 64 x 64 tiles of router_gate_kernel 18.2, and
-// with one tile 11.2 against 7.0 here.  16-bit products beyond a round of 32 x 64 tiles are left to that kernel, whose waves share
-// the operands through LDS (4096 tokens: 20.6 us against 22.4 on 64 x 64 tiles here); fp32 (bound by its matrix rate) goes on with
-// 64 x 64 tiles (2048 tokens: 25 us where a kernel of plain FMAs took 196; 207 tokens, 1232 columns, 436 outputs: 13 for 194).
-bool gate_splitk_pays(int M, int N, int dtype) { return dtype == FMOE_F32 || gate_tiles(M, N, 2, 4) <= chip_info().cus; }
-
+// statistics launch on 32 x 32 tiles (256 of them), 23 on 16 x 32 and 17 on 32 x 64.  fp32 beyond a round goes on with 64 x 64 tiles.
 template <typename T>
 void launch_gate_splitk(const void* x, const void* w, const GateStats& st, float* logits32, void* logits, int M, int N, int K, int split,
                         hipStream_t stream) {

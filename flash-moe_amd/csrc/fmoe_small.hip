@@ -217,7 +217,7 @@ int select_and_down(const float* logits32, int T_, int nk, int K, float* scores,
 
 bool gate_beside_up(int64_t T_, int H, int I, int nk, int dtype) {
     if (T_ > kSmallMaxTokens || H > kGateStagedK || (dtype == FMOE_F32 && I % 4 != 0) || nk > 32767) return false;
-    if (gate_tiles((int)T_, 2 * nk, 2, 2) > 2 * chip_info().cus) return false;
+    if (gate_tiles((int)T_, 2 * nk, 2, 2) > 2 * chip_info().cus || !gate_splitk_pays((int)T_, 2 * nk, dtype)) return false;
     switch (dtype) {
         case FMOE_F32: return plan_product<float, kEpiSwiGLU>((int)T_, I).cut != kCutNone;
         default: return plan_product<bf16_t, kEpiSwiGLU>((int)T_, I).cut != kCutNone;

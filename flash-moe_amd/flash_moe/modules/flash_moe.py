@@ -137,7 +137,8 @@ class FlashMoE(nn.Module):
         return out.view(bsz, seq_len, self.hidden_size), router_logits
 
     def forward_staged(self, hidden_states: torch.Tensor):
-        """``forward`` as three library calls (router, experts, MLP) instead of one; same results."""
+        """``forward`` as three library calls (router, experts, MLP) instead of one; the same routing, and the same output up
+        to the order of the MLP's fp32 sums (for at most 2048 tokens)."""
         bsz, seq_len, _ = hidden_states.shape
         tokens = hidden_states.reshape(bsz * seq_len, self.hidden_size)
         router_logits, _, indices, gates = self.route(tokens)

@@ -1,9 +1,11 @@
 """The whole FlashMoE block forward as one call of ``fmoe_block_forward``.
 
 ``block_forward`` computes what FlashMoE.forward computes on the flattened tokens
-(flash_moe/modules/flash_moe.py:55-105): router -> routed experts -> shared SwiGLU MLP + add.  It gives the same
-results as calling ``router_forward``, ``expert_forward`` and ``mlp_forward(residual=...)`` in turn; the single call
-keeps every intermediate in one workspace and skips the conversion of expert ids to table offsets.
+(flash_moe/modules/flash_moe.py:55-105): router -> routed experts -> shared SwiGLU MLP + add.  The routing
+(logits, expert ids, gates, statistics) is that of ``router_forward`` to the last bit, and the output that of calling
+``expert_forward`` and ``mlp_forward(residual=...)`` with it; for at most 2048 tokens, where stages share launches, the MLP's
+fp32 sums may be taken in another order, beyond that the output is the same to the last bit too.  The single call keeps
+every intermediate in one workspace and skips the conversion of expert ids to table offsets.
 """
 from __future__ import annotations
 

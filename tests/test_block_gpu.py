@@ -200,6 +200,8 @@ def test_single_call_block_equals_the_three_stage_calls(dtype, T, H, I, E, K, tr
     (256, 1032, 1040, 5000, 5), (257, 264, 520, 1024, 8), (40, 2048, 5464, 2500, 50),
     (300, 1032, 4104, 5000, 40), (999, 1000, 2664, 10000, 24), (1500, 520, 1032, 4200, 3), (2048, 264, 1048, 20000, 40),
     (1030, 776, 3000, 700, 20), (1000, 1608, 4264, 2000, 9), (2049, 264, 520, 1024, 8),
+    # at most two rounds of 32 x 32 gate tiles, but more than one of 32 x 64: the router alone does not split k in 16 bits
+    (1700, 264, 520, 16900, 9), (1760, 520, 1032, 16641, 4),
 ])
 def test_block_of_few_tokens(dtype, training, T, H, I, E, K):
     from flash_moe.ops.hip.flash_block import block_forward
@@ -226,12 +228,9 @@ def test_block_of_few_tokens(dtype, training, T, H, I, E, K):
     fresh(); staged, staged_logits = m.forward_staged(x); staged_kept = statistics()
     fresh(); _, _, idx_staged, gates_staged = m.route(x.view(T, H))
     assert torch.equal(y, y2.view_as(y)) and torch.equal(kept, staged_kept) and int(kept[-1]) == (1 if training else 0)
-    assert rel_fro(logits, staged_logits.cpu()) < {torch.float32: 1e-6, torch.bfloat16: 1e-3, torch.float16: 1e-4}[dtype]
-    if torch.equal(logits, staged_logits):           # the same tile kernel: everything that follows from the logits is the same
-        assert torch.equal(idx, idx_staged) and torch.equal(gates, gates_staged)
-        assert rel_fro(y, staged.cpu()) < {torch.float32: 3e-6, torch.bfloat16: 3e-3, torch.float16: 4e-4}[dtype]
-    else:
-        assert dtype != torch.float32 and T > 512
+    # the routing is the staged calls' to the last bit; the down product may sum k in another order
+    assert torch.equal(logits, staged_logits) and torch.equal(idx, idx_staged) and torch.equal(gates, gates_staged)
+    assert rel_fro(y, staged.cpu()) < {torch.float32: 3e-6, torch.bfloat16: 3e-3, torch.float16: 4e-4}[dtype]
     # the two parts of the output in float64, for a sample of the tokens
     sample = torch.arange(0, T, max(1, T // 100))
     x64, idx, gates = x.view(T, H)[sample.cuda()].double().cpu(), idx.cpu()[sample], gates.double().cpu()[sample]
