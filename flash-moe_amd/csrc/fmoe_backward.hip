@@ -204,11 +204,11 @@ int launch_route_backward(const void* dgates, const int64_t* indices, const floa
 // SwiGLU
 // ------------------------------------------------------------------------------------------------------------
 // One 16-byte packet per thread; workgroup b works on row b / col_blocks.  Row strides (elements) let da / db / h live
-// side by side in wider buffers.
+// side by side in wider buffers.  h may be dc: a thread reads its packet of dc before it writes h.
 template <typename T>
-__global__ __launch_bounds__(256) void swiglu_backward_kernel(const T* __restrict__ dc, const T* __restrict__ a,
+__global__ __launch_bounds__(256) void swiglu_backward_kernel(const T* dc, const T* __restrict__ a,
                                                               const T* __restrict__ b, T* __restrict__ da,
-                                                              T* __restrict__ db, T* __restrict__ h, int col_blocks,
+                                                              T* __restrict__ db, T* h, int col_blocks,
                                                               int cols, int64_t da_stride, int64_t db_stride) {
     constexpr int V = Elem<T>::kVec;
     const uint32_t row = blockIdx.x / (uint32_t)col_blocks;

@@ -59,7 +59,7 @@ SavedPlan plan_saved(int64_t T_, int H, int I, int nk, int64_t E, int K, int dty
     p.off_indices = take((size_t)T_ * K * 8);
     p.off_gates = take((size_t)T_ * K * elt);
     p.off_stats = take((size_t)2 * H * 4);
-    p.off_products = take((size_t)3 * T_ * I * elt);      // gate, up, and silu(gate) * up
+    p.off_products = take((size_t)2 * T_ * I * elt);
     p.off_experts = take(fmoe_expert_saved_bytes(T_, H, E, K, dtype));
     p.bytes = o;
     return p;
@@ -78,7 +78,7 @@ BlockBackwardPlan plan_block_backward(int64_t T_, int H, int I, int nk, int64_t 
     p.off_dgates = take((size_t)T_ * K * elt);
     p.off_dlogits32 = take((size_t)T_ * 2 * nk * 4);
     p.off_dx_experts = take((size_t)T_ * H * elt);
-    p.stage_bytes = fmoe_mlp_backward_workspace_bytes(T_, H, I, dtype);
+    p.stage_bytes = fmoe_mlp_backward_saved_workspace_bytes(T_, H, I, dtype);
     const size_t experts = fmoe_expert_backward_workspace_bytes(T_, H, E, K, dtype);
     const size_t prologue = fmoe_router_prologue_backward_workspace_bytes(T_, H, nk, dtype);
     if (experts > p.stage_bytes) p.stage_bytes = experts;
@@ -142,7 +142,6 @@ int block_forward_impl(const char* who, const void* x, const void* gate_proj_w, 
         gates = saved + sp.off_gates;
         stats = (float*)(saved + sp.off_stats);
         products = saved + sp.off_products;
-        act = saved + sp.off_products + (size_t)2 * num_tokens * intermediate * dtype_size(dtype);
     }
     void* expert_ws = ws + p.off_expert;
     void* experts = ws + p.off_experts_out;
@@ -281,9 +280,7 @@ extern "C" int fmoe_block_backward(const void* dout, const void* dlogits, const 
     char* ws = (char*)workspace;
     void *dgates = ws + p.off_dgates, *dx_experts = ws + p.off_dx_experts, *stage = ws + p.off_stage;
     float* dlogits32 = (float*)(ws + p.off_dlogits32);
-    const char* products = sv + sp.off_products;
-    int rc = fmoe_mlp_backward_act(dout, x, gate_proj_w, up_proj_w, down_proj_w, products,
-                               products + (size_t)2 * num_tokens * intermediate * dtype_size(dtype), num_tokens, hidden, intermediate,
+    int rc = fmoe_mlp_backward(dout, x, gate_proj_w, up_proj_w, down_proj_w, sv + sp.off_products, num_tokens, hidden, intermediate,
                                dtype, dx, dgate_proj_w, dup_proj_w, ddown_proj_w, stage, p.stage_bytes, stream);
     if (rc) return rc;
     rc = fmoe_expert_backward_saved(dout, x, down_embed, up_embed, indices, sv + sp.off_gates, sv + sp.off_experts, num_tokens, hidden,

@@ -1,11 +1,11 @@
 // Backward of the shared SwiGLU MLP  y = (silu(x Wg^T) * (x Wu^T)) Wd^T  for gfx950.
 //
-// The forward keeps only silu(a) * b unless it was asked to keep the gate and up products a, b as well
-// (fmoe_mlp_gate_up_save); without them they are recomputed here (two launches of the forward's own NT GEMM).  The SwiGLU gradient is the fused
-// elementwise kernel of fmoe_backward.hip (it also rebuilds h = silu(a) * b for dWd unless the caller kept that too: a sixth of
-// what it moves).  The remaining products are
-// plain GEMMs in layouts the forward never needs (A B and A^T B): gemm_backward (fmoe_gemm_tr.hip).  What its kernels cannot
-// address goes to rocBLAS, which is loaded on first use so that nothing else depends on it:
+// The forward keeps the gate and up products a, b if it was asked to (fmoe_mlp_gate_up_save); without them they are recomputed here
+// (two launches of the forward's own NT GEMM).  The SwiGLU gradient is the fused elementwise kernel of fmoe_backward.hip, which also
+// rebuilds h = silu(a) * b for dWd.  Written in place of dh it costs 2 us in a training step of 4096 tokens of 1024 -> 4096 in
+// bf16 (743 us); keeping it from the forward instead would make the largest tensor a training step holds half as large again.  The
+// remaining products are plain GEMMs in layouts the forward never needs (A B and A^T B): gemm_backward (fmoe_gemm_tr.hip).  What its
+// kernels cannot address goes to rocBLAS, which is loaded on first use so that nothing else depends on it:
 //     dh  = dy Wd              [T,H][H,I]
 //     dWd = dy^T h             [T,H]^T [T,I]
 //     dx  = da Wg + db Wu      [T,I][I,H] twice, the second accumulating
@@ -73,15 +73,16 @@ struct MlpBwdPlan {
     size_t off_a, off_b, off_dh, off_h, off_dab, off_part, part_bytes, bytes;
 };
 
-MlpBwdPlan plan_mlp_backward(int64_t T_, int H, int I, int dtype) {
+// kept: the caller has the products.  Their planes are left out, and h takes the place of dh, element by element as that is read.
+MlpBwdPlan plan_mlp_backward(int64_t T_, int H, int I, int dtype, bool kept) {
     MlpBwdPlan p;
     const size_t ti = (size_t)T_ * I * dtype_size(dtype);
     size_t o = 0;
     auto take = [&](size_t n) { const size_t at = o; o = round_up(o + n, 256); return at; };
-    p.off_a = take(ti);
-    p.off_b = take(ti);
+    p.off_a = take(kept ? 0 : ti);
+    p.off_b = take(kept ? 0 : ti);
     p.off_dh = take(ti);
-    p.off_h = take(ti);
+    p.off_h = kept ? p.off_dh : take(ti);
     p.off_dab = take(2 * ti);
     p.part_bytes = 0;
     const int t = (int)T_;
@@ -117,19 +118,17 @@ int blas_gemm(int layout, int M, int N, int K, const void* A, int lda, const voi
 
 extern "C" size_t fmoe_mlp_backward_workspace_bytes(int64_t num_tokens, int hidden, int intermediate, int dtype) {
     if (num_tokens <= 0 || hidden <= 0 || intermediate <= 0 || !fmoe::dtype_ok(dtype)) return 0;
-    return fmoe::plan_mlp_backward(num_tokens, hidden, intermediate, dtype).bytes;
+    return fmoe::plan_mlp_backward(num_tokens, hidden, intermediate, dtype, false).bytes;
+}
+
+extern "C" size_t fmoe_mlp_backward_saved_workspace_bytes(int64_t num_tokens, int hidden, int intermediate, int dtype) {
+    if (num_tokens <= 0 || hidden <= 0 || intermediate <= 0 || !fmoe::dtype_ok(dtype)) return 0;
+    return fmoe::plan_mlp_backward(num_tokens, hidden, intermediate, dtype, true).bytes;
 }
 
 extern "C" int fmoe_mlp_backward(const void* dy, const void* x, const void* gate_w, const void* up_w, const void* down_w,
                                  const void* saved_products, int64_t num_tokens, int hidden, int intermediate, int dtype, void* dx, void* dgate_w, void* dup_w,
                                  void* ddown_w, void* workspace, size_t workspace_bytes, void* stream) {
-    return fmoe_mlp_backward_act(dy, x, gate_w, up_w, down_w, saved_products, nullptr, num_tokens, hidden, intermediate, dtype, dx, dgate_w,
-                                 dup_w, ddown_w, workspace, workspace_bytes, stream);
-}
-
-extern "C" int fmoe_mlp_backward_act(const void* dy, const void* x, const void* gate_w, const void* up_w, const void* down_w,
-                                     const void* saved_products, const void* act, int64_t num_tokens, int hidden, int intermediate, int dtype,
-                                     void* dx, void* dgate_w, void* dup_w, void* ddown_w, void* workspace, size_t workspace_bytes, void* stream) {
     using namespace fmoe;
     clear_error();
     FMOE_REQUIRE(dtype_ok(dtype), FMOE_ERR_BAD_DTYPE, "fmoe_mlp_backward: unknown dtype %d", dtype);
@@ -141,7 +140,7 @@ extern "C" int fmoe_mlp_backward_act(const void* dy, const void* x, const void* 
                  "fmoe_mlp_backward: hidden=%d and intermediate=%d must be multiples of %d (16-byte rows)", hidden, intermediate, vec);
     FMOE_REQUIRE(dy && x && gate_w && up_w && down_w && dx && dgate_w && dup_w && ddown_w, FMOE_ERR_NULL_POINTER,
                  "fmoe_mlp_backward: null tensor pointer");
-    const MlpBwdPlan p = plan_mlp_backward(num_tokens, hidden, intermediate, dtype);
+    const MlpBwdPlan p = plan_mlp_backward(num_tokens, hidden, intermediate, dtype, saved_products != nullptr);
     FMOE_REQUIRE(workspace && workspace_bytes >= p.bytes && aligned16(workspace), FMOE_ERR_WORKSPACE,
                  "fmoe_mlp_backward: workspace of %zu bytes needed, %zu given", p.bytes, workspace_bytes);
     hipStream_t s = (hipStream_t)stream;
@@ -170,10 +169,9 @@ extern "C" int fmoe_mlp_backward_act(const void* dy, const void* x, const void* 
     // da and db side by side: one [T, 2I] matrix [da | db], so that products over both are single calls
     char* db = dab + (size_t)I * elt;
     const int I2 = 2 * I;
-    // h = silu(a) * b is what the forward multiplied with Wd: kept, or rebuilt here
-    rc = launch_swiglu_backward(dh, a, b, dab, db, act != nullptr ? nullptr : h, num_tokens, I, I2, I2, dtype, s);
+    rc = launch_swiglu_backward(dh, a, b, dab, db, h, num_tokens, I, I2, I2, dtype, s);
     if (rc) return rc;
-    rc = gemm_backward(kTN, H, I, T_, dy, H, act != nullptr ? act : h, nullptr, I, ddown_w, dtype, part, p.part_bytes, s);                         // dWd = dy^T h
+    rc = gemm_backward(kTN, H, I, T_, dy, H, h, nullptr, I, ddown_w, dtype, part, p.part_bytes, s);                         // dWd = dy^T h
     if (rc) return rc;
     rc = gemm_backward(kNN, T_, H, I, dab, I2, gate_w, up_w, H, dx, dtype, part, p.part_bytes, s);                          // dx = da Wg + db Wu
     if (rc) return rc;

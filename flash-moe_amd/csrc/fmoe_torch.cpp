@@ -415,8 +415,8 @@ Tensor mlp_forward(const Tensor& x_in, const Tensor& gate, const Tensor& up, con
     return out;
 }
 
-// out and a [3, T, I] buffer: the gate and up products and the activation
-std::tuple<Tensor, Tensor> mlp_forward_keeping(const Tensor& x_in, const Tensor& gate, const Tensor& up, const Tensor& down, const OptTensor& residual) {
+// out and a [2, T, I] buffer: the gate and up products
+std::tuple<Tensor, Tensor> mlp_forward_saving(const Tensor& x_in, const Tensor& gate, const Tensor& up, const Tensor& down, const OptTensor& residual) {
     check_mlp_weights(x_in, gate, up, down);
     const Tensor res_in = value(residual);
     require_gpu({&x_in, &gate, &up, &down, &res_in});
@@ -424,21 +424,14 @@ std::tuple<Tensor, Tensor> mlp_forward_keeping(const Tensor& x_in, const Tensor&
     const Tensor x = x_in.contiguous(), wg = gate.contiguous(), wu = up.contiguous(), wd = down.contiguous(), res = contiguous_residual(res_in, x_in);
     const int64_t H = x.size(-1), I = wg.size(0), T = H ? x.numel() / H : 0;
     Launch call(x);
-    Tensor saved = at::empty({3, T, I}, x.options()), out = at::empty_like(x);
-    void* act = (char*)ptr(saved) + (size_t)2 * T * I * x.element_size();
+    Tensor saved = at::empty({2, T, I}, x.options()), act = at::empty({T, I}, x.options()), out = at::empty_like(x);
     const size_t bytes = fmoe_mlp_down_workspace_bytes(T, (int)H, (int)I, code);
     Tensor ws = bytes ? workspace(x, bytes) : Tensor();
-    check(fmoe_mlp_gate_up_save(ptr(x), ptr(wg), ptr(wu), T, (int)H, (int)I, code, act, ptr(saved), call.stream), "flash_mlp");
-    check(fmoe_mlp_down_ws(act, ptr(wd), T, (int)H, (int)I, code, ptr(res), ptr(out), ptr(ws), bytes, call.stream), "flash_mlp");
+    check(fmoe_mlp_gate_up_save(ptr(x), ptr(wg), ptr(wu), T, (int)H, (int)I, code, ptr(act), ptr(saved), call.stream), "flash_mlp");
+    check(fmoe_mlp_down_ws(ptr(act), ptr(wd), T, (int)H, (int)I, code, ptr(res), ptr(out), ptr(ws), bytes, call.stream), "flash_mlp");
     return {out, saved};
 }
 
-std::tuple<Tensor, Tensor> mlp_forward_saving(const Tensor& x, const Tensor& gate, const Tensor& up, const Tensor& down, const OptTensor& residual) {
-    auto [out, saved] = mlp_forward_keeping(x, gate, up, down, residual);
-    return {out, saved.narrow(0, 0, 2)};
-}
-
-// products: NULL, [2, T, I], or (from the autograd node) with the activation as a third plane
 std::tuple<Tensor, Tensor, Tensor, Tensor> mlp_backward(const Tensor& dout, const Tensor& x_in, const Tensor& gate, const Tensor& up,
                                                         const Tensor& down, const OptTensor& products) {
     const Tensor saved = value(products);
@@ -447,7 +440,7 @@ std::tuple<Tensor, Tensor, Tensor, Tensor> mlp_backward(const Tensor& dout, cons
     const int code = dtype_code(x_in.scalar_type());
     const Tensor x = x_in.contiguous(), dy = dout.contiguous(), wg = gate.contiguous(), wu = up.contiguous(), wd = down.contiguous();
     const int64_t H = x.size(-1), I = wg.size(0), T = H ? x.numel() / H : 0;
-    TORCH_CHECK_VALUE(!saved.defined() || (saved.dim() == 3 && (saved.size(0) == 2 || saved.size(0) == 3) && saved.size(1) == T && saved.size(2) == I &&
+    TORCH_CHECK_VALUE(!saved.defined() || (saved.dim() == 3 && saved.size(0) == 2 && saved.size(1) == T && saved.size(2) == I &&
                                            saved.scalar_type() == x.scalar_type() && saved.is_contiguous()),
                       "saved must be the contiguous [2, T, I] tensor mlp_forward_saving returned");
     Launch call(x);
@@ -455,10 +448,10 @@ std::tuple<Tensor, Tensor, Tensor, Tensor> mlp_backward(const Tensor& dout, cons
     Tensor dwgu = at::empty({2 * I, H}, wg.options());
     Tensor dwg = dwgu.narrow(0, 0, I), dwu = dwgu.narrow(0, I, I), dx = at::empty_like(x), dwd = at::empty_like(wd);
     if (T == 0) return {dx, dwg.zero_(), dwu.zero_(), dwd.zero_()};
-    const size_t bytes = fmoe_mlp_backward_workspace_bytes(T, (int)H, (int)I, code);
+    const size_t bytes = saved.defined() ? fmoe_mlp_backward_saved_workspace_bytes(T, (int)H, (int)I, code)
+                                         : fmoe_mlp_backward_workspace_bytes(T, (int)H, (int)I, code);
     Tensor ws = workspace(x, bytes);
-    const void* act = saved.defined() && saved.size(0) == 3 ? (const char*)ptr(saved) + (size_t)2 * T * I * x.element_size() : nullptr;
-    check(fmoe_mlp_backward_act(ptr(dy), ptr(x), ptr(wg), ptr(wu), ptr(wd), ptr(saved), act, T, (int)H, (int)I, code, ptr(dx), ptr(dwg), ptr(dwu),
+    check(fmoe_mlp_backward(ptr(dy), ptr(x), ptr(wg), ptr(wu), ptr(wd), ptr(saved), T, (int)H, (int)I, code, ptr(dx), ptr(dwg), ptr(dwu),
                             ptr(dwd), ptr(ws), bytes, call.stream), "flash_mlp backward");
     return {dx, dwg, dwu, dwd};
 }
@@ -470,7 +463,7 @@ struct MlpNode : torch::autograd::Function<MlpNode> {
             ctx->save_for_backward({x, gate, up, down});
             return mlp_forward(x, gate, up, down, std::nullopt);
         }
-        auto [out, saved] = mlp_forward_keeping(x, gate, up, down, std::nullopt);
+        auto [out, saved] = mlp_forward_saving(x, gate, up, down, std::nullopt);
         ctx->save_for_backward({x, gate, up, down, saved});
         return out;
     }

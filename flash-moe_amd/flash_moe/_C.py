@@ -75,8 +75,8 @@ SIGNATURES = {
     "fmoe_router_prologue_backward": (_int, [_vp, _vp, _vp, _vp, _int, _i64, _int, _int, _int, _vp, _vp, _vp, _sz, _vp]),
     "fmoe_swiglu_backward": (_int, [_vp, _vp, _vp, _i64, _int, _int, _vp, _vp, _vp]),
     "fmoe_mlp_backward_workspace_bytes": (_sz, [_i64, _int, _int, _int]),
+    "fmoe_mlp_backward_saved_workspace_bytes": (_sz, [_i64, _int, _int, _int]),
     "fmoe_mlp_backward": (_int, [_vp] * 6 + [_i64, _int, _int, _int] + [_vp] * 5 + [_sz, _vp]),
-    "fmoe_mlp_backward_act": (_int, [_vp] * 7 + [_i64, _int, _int, _int] + [_vp] * 5 + [_sz, _vp]),
     "fmoe_expert_backward_workspace_bytes": (_sz, [_i64, _int, _i64, _int, _int]),
     "fmoe_expert_backward_saved": (_int, [_vp] * 7 + [_i64, _int, _i64, _int, _int] + [_vp] * 5 + [_sz, _vp]),
     "fmoe_expert_backward": (_int, [_vp] * 6 + [_i64, _int, _i64, _int, _int] + [_vp] * 5 + [_sz, _vp]),

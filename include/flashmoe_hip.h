@@ -276,8 +276,8 @@ int fmoe_block_forward(const void* x, const void* gate_proj_w, const void* up_pr
                        void* gates_out, void* workspace, size_t workspace_bytes, void* stream);
 
 /* The block with gradients: fmoe_block_forward that also fills `saved` (fmoe_block_saved_bytes() bytes, 256-byte aligned: expert
- * ids, gates, fp32 gate logits, batch-norm statistics, gate and up products and the activation) and the backward from it.  The reference reaches the
- * same gradients through autograd of its eager ops around its three Triton functions (flash_moe/modules/flash_moe.py:55-105).
+ * ids, gates, fp32 gate logits, batch-norm statistics, gate and up products, and what fmoe_expert_forward_save keeps) and the
+ * backward from it.  The reference reaches the same gradients through autograd of its eager ops around its three Triton functions (flash_moe/modules/flash_moe.py:55-105).
  * fmoe_block_forward_save: arguments and workspace as fmoe_block_forward; top_k >= 1.
  * fmoe_block_backward: dout [T,H]; dlogits [2,T,nk] (gradient of the router logits as the module returns them) or NULL; training and
  *   norm_topk_prob as in the forward; out: dx [T,H], dgate_proj_w, dup_proj_w [I,H] (faster when they follow each other, as in
@@ -375,16 +375,15 @@ int fmoe_swiglu_backward(const void* dc, const void* a, const void* b, int64_t r
  * recompute the gate and up products here.  The transposed-operand GEMMs run on this library's kernels; operands those
  * cannot address (beyond 2 GB, or not whole 16-byte packets) are rocBLAS calls (loaded on first use; FMOE_ERR_LIBRARY if
  * unavailable).  When dup_w starts where dgate_w ends (one [2I,H] buffer) the two weight gradients
- * are formed as one product (faster; the sums may differ in the last bit from two products); separate buffers work as well. */
+ * are formed as one product (faster; the sums may differ in the last bit from two products); separate buffers work as well.
+ * Workspace: fmoe_mlp_backward_workspace_bytes() is enough for either kind of call, fmoe_mlp_backward_saved_workspace_bytes() (half
+ * of it: three [T,I] planes and what slices of k need) for one with saved_products. */
 size_t fmoe_mlp_backward_workspace_bytes(int64_t num_tokens, int hidden, int intermediate, int dtype);
+size_t fmoe_mlp_backward_saved_workspace_bytes(int64_t num_tokens, int hidden, int intermediate, int dtype);
 
 int fmoe_mlp_backward(const void* dy, const void* x, const void* gate_w, const void* up_w, const void* down_w,
                       const void* saved_products, int64_t num_tokens, int hidden, int intermediate, int dtype, void* dx, void* dgate_w, void* dup_w,
                       void* ddown_w, void* workspace, size_t workspace_bytes, void* stream);
-/* The same with the [T,I] activation the forward formed (act; NULL: it is rebuilt from the products). */
-int fmoe_mlp_backward_act(const void* dy, const void* x, const void* gate_w, const void* up_w, const void* down_w,
-                          const void* saved_products, const void* act, int64_t num_tokens, int hidden, int intermediate, int dtype,
-                          void* dx, void* dgate_w, void* dup_w, void* ddown_w, void* workspace, size_t workspace_bytes, void* stream);
 
 /* FlashExpertFunc.backward / _flash_expert_backward (flash_moe/ops/triton/flash_expert.py:654-745, kernels :234-525):
  * from dout [T,H] the gradients dx [T,H], ddown, dup [E,H] (rows of experts no pair selects are zero) and

@@ -214,6 +214,8 @@ def test_backward_argument_checks():
     assert ecall(ws_bytes=need - 1) == -7
     mneed = lib.fmoe_mlp_backward_workspace_bytes(8, 64, 128, _C.BF16)
     assert mneed >= 6 * 8 * 128 * 2 and mneed % 256 == 0
+    sneed = lib.fmoe_mlp_backward_saved_workspace_bytes(8, 64, 128, _C.BF16)
+    assert 3 * 8 * 128 * 2 <= sneed <= mneed - 3 * 8 * 128 * 2
     mb = lib.fmoe_mlp_backward
 
     def mcall(T=8, H=64, I=128, dtype=_C.BF16, dy=a, ws_bytes=mneed):
@@ -224,6 +226,16 @@ def test_backward_argument_checks():
     assert mcall(I=100) == -6
     assert mcall(dy=None) == -1
     assert mcall(ws_bytes=mneed - 1) == -7
+    assert mb(a, a, a, a, a, a, 8, 64, 128, _C.BF16, a, a, a, a, a, sneed - 1, None) == -7      # with saved products
+
+
+def test_training_keeps_two_planes_of_the_intermediate_width():
+    """What a block's forward leaves for its backward grows by the gate and up products, [2, T, I], with the intermediate width."""
+    lib = _C.lib()
+    T, H, nk, E, K = 512, 256, 32, 1024, 16
+    for code, elt in ((_C.F32, 4), (_C.BF16, 2), (_C.F16, 2)):
+        narrow, wide = (lib.fmoe_block_saved_bytes(T, H, I, nk, E, K, code) for I in (1024, 4096))
+        assert wide - narrow == 2 * T * (4096 - 1024) * elt
 
 
 def test_python_wrappers_refuse_cpu_tensors():

@@ -408,6 +408,31 @@ def test_mlp_backward_with_saved_products_equals_recomputation(dtype):
         assert rel_fro(a, b) < (1e-6 if dtype == torch.float32 else 2e-3)
 
 
+@pytest.mark.parametrize("what", ["mlp", "block"])
+def test_memory_of_a_training_step(what):
+    """In planes of [T, I], the largest tensors of a step: the forward keeps two (gate and up product), the backward works in three
+    more (dh, da, db) beside the gradients."""
+    from flash_moe.modules.flash_moe import FlashMoE, FlashMoEConfig
+    from flash_moe.ops import flash_mlp_func
+
+    T, H, I = 4096, 128, 8192
+    plane = T * I * 2
+    m = FlashMoE(FlashMoEConfig(H, I, "silu", 1024, 8)).to(device="cuda", dtype=torch.bfloat16)
+    x = torch.randn(1, T, H, generator=gen(0)).bfloat16().cuda().requires_grad_()
+    run = (lambda: m(x)[0]) if what == "block" else (lambda: flash_mlp_func(x, m.gate_proj.weight, m.up_proj.weight, m.down_proj.weight))
+    run().sum().backward()                                   # gradients exist from here on: they are not counted below
+    torch.cuda.synchronize()
+    before = torch.cuda.memory_allocated()
+    y = run()
+    kept = torch.cuda.memory_allocated() - before
+    dy = torch.ones_like(y)
+    torch.cuda.reset_peak_memory_stats()
+    y.backward(dy)
+    peak = torch.cuda.max_memory_allocated() - before
+    # a quarter of a plane: tensors of the hidden and the routing width; half a plane more: new gradients and slices of k
+    assert 2 * plane <= kept <= 2.25 * plane and peak <= 5.75 * plane, (kept / plane, peak / plane)
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("stacked_weights", [False, True])
 @pytest.mark.parametrize("stacked_grads", [False, True])
