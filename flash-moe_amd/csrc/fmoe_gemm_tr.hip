@@ -7,10 +7,19 @@
 //
 // What bounds it is what bounds the forward's products: what a compute unit receives on small tiles, the matrix pipes on 256 x 256,
 // and, with few tiles and a long k loop, the length of one chain, which slices of k cut (their sums are added by a second launch, in
-// slice order).  Against the library's kernels, us: 2048 tokens, 4096 -> 16384: dh 211 for 207, dx 435 for 435, dWd 225 for 252, dWg
-// and dWu 445 for 494; 479 tokens, 3304 -> 13216: 60 for 67, 105 for 258, 60 for 110, 114 for 192; 615 tokens, 776 -> 2072: 8 for 19,
-// 20 for 28, 8 for 19, 11 for 20; fp32, 383 tokens, 1880 -> 7520: 114 for 97, 207 for 826, 111 for 118, 182 for 228.  A kernel that
-// turned the operands in registers reached 600 TFLOP/s in bf16 where these reach 1000 to 1200.
+// slice order).  A kernel that turned the operands in registers reached 600 TFLOP/s in bf16 where these reach 1000 to 1300.
+//
+// Against the library's kernels (rocBLAS), us:
+//   bf16  2048 tokens, 4096 -> 16384: dh 208 for 204, dx 447 for 496, dWd 222 for 243, dWg and dWu 463 for 516; 615 tokens, 776 -> 2072: 8
+//         for 16, 20 for 35, 8 for 17, 11 for 18; 32768 tokens, 2048 -> 8192: 1018 for 890, 1711 for 1726, 833 for 980, 1709 for 1891.
+//         Slower only for dh of many tokens on 256 x 256 tiles (4096 tokens and more, by 3 to 14 %) and dx of 12000 tokens of 3072 -> 768
+//         (124 for 106).
+//   fp32  383 tokens, 1880 -> 7520: dh 97 for 88, dx 200 for 828, dWd 100 for 105, dWg and dWu 191 for 218; 1000 tokens, 1024 -> 4096: 71
+//         for 64, 136 for 120, 69 for 71, 125 for 152; 4096 tokens, 1024 -> 4096: 257 for 242, 520 for 460, 260 for 231, 479 for 455; 5000
+//         tokens, 2048 -> 5464: 897 for 812, 1791 for 2426, 867 for 1094, 1746 for 1913; 16384 tokens, 512 -> 2048: 258 for 246, 488 for
+//         913, 259 for 235, 516 for 788.  At 120 to 143 TFLOP/s these kernels are 5 to 15 % behind the library's best and far ahead of what
+//         it takes at other extents; over the backward passes of 16 extents 21.0 ms for 25.0, the worst of them 9 % longer (4096 tokens).
+//         Products of less than a round of tiles take up to 3 us longer (dq of 600 tokens, 256 -> 256: 7.6 for 6.1).
 #include "fmoe_common.h"
 #include "fmoe_gemm.h"
 #include "fmoe_vec.h"
@@ -49,19 +58,27 @@ __global__ __launch_bounds__(256) void gemm_turned_add_kernel(const float* __res
 }
 
 // Tile shape and slices of k by price (us): a round of tiles costs what the forward's rule says, 2.3 ns per received row and k-tile,
-// plus the stores of its tiles, which nothing hides on 256 x 256 (7 us; the smaller tiles overlap them with other workgroups); slices,
+// plus the stores of its tiles, which nothing hides on 256 x 256 (8.5 us; the smaller tiles overlap them with other workgroups); slices,
 // as long as they are one round, add a launch of 4 us and their planes, written and read at 6 TB/s.
+// fp32 tiles are bound by the matrix pipes, which two workgroups of a compute unit keep a tenth busier than one (a k-tile of 128 x 128
+// 2.0 us for 2.25), so slices of 64 x 64 tiles may be two rounds: dx of 1000 tokens, 1024 -> 4096 156 -> 138 in two slices.  64 x 128 has
+// the faults of both its neighbours there and is left out (dx of 2048 tokens 279 for 268 on 64 x 64).
+// The 8.5 us: dq of 32768 tokens, 256 -> 2048 in bf16 takes 66 on 256 x 256 tiles and 54 on 128 x 128; dWd of 384 tokens, 7520 -> 1880, 19
+// for 23.
 template <typename T> SlicePlan plan_turned(int M, int N, int K, int segments) {
     const int cus = chip_info().cus, k_tiles = (K + kStageK<T> - 1) / kStageK<T> * segments;
     SlicePlan best = {kTile64, 1};
     double best_time = 0.0;
     for (int i = sizeof(T) == 4 ? kTile128 : kTile256; i <= kTile64; ++i) {
         int64_t n = 0;
-        const double row = tile_cost<T, kEpiPlain>(i, M, N, n) * 2.3e-3, stores = i == kTile256 ? 7.0 : 1.0;
-        for (int s = 1; s <= kMaxSlices && (s == 1 || (n * s <= cus && 2 * s <= k_tiles)); ++s) {
+        if (sizeof(T) == 4 && i == kTile64x128) continue;
+        const double row = tile_cost<T, kEpiPlain>(i, M, N, n) * 2.3e-3, stores = i == kTile256 ? 8.5 : 1.0;
+        const int64_t most = sizeof(T) == 4 && i == kTile64 ? 2 * cus : cus;
+        for (int s = 1; s <= kMaxSlices && (s == 1 || (n * s <= most && 2 * s <= k_tiles)); ++s) {
             const int share = (k_tiles + s - 1) / s;
             if ((s - 1) * share >= k_tiles) continue;                 // a slice would have no k-tile
-            const double time = (double)((n * s + cus - 1) / cus) * (row * share + stores) + (s > 1 ? 4.0 + 8.0e-6 * s * (double)M * N / 6.0 : 0.0);
+            const double shared = sizeof(T) == 4 && n * s > cus ? 0.9 : 1.0;
+            const double time = (double)((n * s + cus - 1) / cus) * (shared * row * share + stores) + (s > 1 ? 4.0 + 8.0e-6 * s * (double)M * N / 6.0 : 0.0);
             if (best_time == 0.0 || time < best_time) {
                 best = {i, s};
                 best_time = time;
@@ -89,7 +106,7 @@ void launch_turned(const void* A, int lda, const void* B0, const void* B1, int l
         switch (p.shape) {
             case kTile256: if constexpr (sizeof(T) == 2) FMOE_SLICED(256, 256, 4, 2); break;
             case kTile128: FMOE_SLICED(128, 128, 2, 4); break;
-            case kTile64x128: FMOE_SLICED(64, 128, 2, 4); break;
+            case kTile64x128: if constexpr (sizeof(T) == 2) FMOE_SLICED(64, 128, 2, 4); break;
             default: FMOE_SLICED(64, 64, 2, 4); break;
         }
         const int64_t packets = (int64_t)M * N / Elem<T>::kVec;
@@ -103,7 +120,7 @@ void launch_turned(const void* A, int lda, const void* B0, const void* B1, int l
             if (n <= cus) FMOE_WHOLE(128, 128, 2, 4, 1);
             else FMOE_WHOLE(128, 128, 2, 2, 2);
             break;
-        case kTile64x128: FMOE_WHOLE(64, 128, 2, 4, 1); break;
+        case kTile64x128: if constexpr (sizeof(T) == 2) FMOE_WHOLE(64, 128, 2, 4, 1); break;
         default: FMOE_WHOLE(64, 64, 2, 4, 2); break;
     }
 #undef FMOE_SLICED

@@ -580,7 +580,8 @@ def test_mlp_backward_remainders_of_the_transposing_products(dtype, T, H, I):
     assert all(torch.equal(a, b) for a, b in zip(got, mlp_backward(dy, x, *ws, saved)))      # bit for bit the same twice
 
 
-@pytest.mark.parametrize("T,H,I", [(1, 4, 8), (65, 68, 1028), (300, 264, 2060), (383, 516, 1544), (900, 1032, 2056), (2500, 264, 2052)])
+@pytest.mark.parametrize("T,H,I", [(1, 4, 8), (65, 68, 1028), (300, 264, 2060), (383, 516, 1544), (900, 1032, 2056), (2500, 264, 2052),
+                                   (1000, 520, 1032)])       # slices of 64 x 64 tiles beyond a round (dx, dWd)
 def test_mlp_backward_remainders_of_the_transposing_products_fp32(T, H, I):
     test_mlp_backward_remainders_of_the_transposing_products(torch.float32, T, H, I)
 
