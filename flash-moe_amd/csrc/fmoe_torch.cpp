@@ -614,7 +614,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     FMOE_DEF(expert_backward);
     FMOE_DEF(expert_func);
     FMOE_DEF(expert_bucketing);
+    FMOE_DEF(peer_forward);
     FMOE_DEF(peer_func);
+    FMOE_DEF(pkm_forward);
     FMOE_DEF(pkm_func);
     FMOE_DEF(mlp_forward);
     FMOE_DEF(mlp_forward_saving);

@@ -12,7 +12,9 @@ from __future__ import annotations
 import torch
 
 from flash_moe import _C
-from flash_moe.ops.hip.flash_router import check_norm
+from flash_moe.ops.hip.flash_expert import expert_backward, expert_forward
+from flash_moe.ops.hip.flash_mlp import mlp_backward, mlp_forward_saving
+from flash_moe.ops.hip.flash_router import check_norm, route_backward, router_forward, router_prologue_backward
 
 
 def block_forward(tokens: torch.Tensor, gate_proj: torch.Tensor, up_proj: torch.Tensor, down_proj: torch.Tensor,
@@ -40,3 +42,37 @@ def block(hidden_states, gate_proj, up_proj, down_proj, router_gate, norm, down_
     )
     return _C.native().block(hidden_states, gate_proj, up_proj, down_proj, router_gate, down_embed, up_embed, *check_norm(norm),
                              num_expert_keys, num_experts_per_tok, norm_topk_prob, differentiable, return_routing)
+
+
+class FlashMoEBlockFunc(torch.autograd.Function):
+    """The block with gradients for the tokens and every weight as an autograd function over the per-op calls: ``(out [T, H],
+    router_logits [T, 2*nk])``, for callers that apply or subclass it; ``block`` takes the native node, one library call each way."""
+
+    @staticmethod
+    def forward(ctx, tokens, gate_proj, up_proj, down_proj, router_gate, down_embed, up_embed, norm, num_expert_keys,
+                num_experts_per_tok, norm_topk_prob):
+        x = tokens.contiguous()
+        logits, _, indices, gates, logits32, stats = router_forward(
+            x, router_gate, norm, num_expert_keys, num_experts_per_tok, norm_topk_prob, return_logits32=True, return_stats=True)
+        experts = expert_forward(x, down_embed, up_embed, indices, gates)
+        out, products = mlp_forward_saving(x, gate_proj, up_proj, down_proj, residual=experts)
+        ctx.save_for_backward(x, gate_proj, up_proj, down_proj, router_gate, down_embed, up_embed, indices, gates, logits32,
+                              stats.clone(), products)
+        ctx.training, ctx.num_expert_keys, ctx.norm_topk_prob = norm.training, num_expert_keys, norm_topk_prob
+        return out, logits
+
+    @staticmethod
+    def backward(ctx, dout, dlogits):
+        x, wg, wu, wd, wr, ed, eu, indices, gates, logits32, stats, products = ctx.saved_tensors
+        dx, dwg, dwu, dwd = mlp_backward(dout, x, wg, wu, wd, products)
+        dx_experts, ded, deu, dgates = expert_backward(dout, x, ed, eu, indices, gates)
+        dlogits32 = route_backward(dgates, indices, logits32, ctx.num_expert_keys, ctx.norm_topk_prob, dlogits)
+        dx_router, dwr = router_prologue_backward(dlogits32, x, wr, stats, ctx.training)
+        return dx.add_(dx_experts).add_(dx_router), dwg, dwu, dwd, dwr, ded, deu, None, None, None, None
+
+
+def block_forward_autograd(tokens, gate_proj, up_proj, down_proj, router_gate, norm, down_embed, up_embed, num_expert_keys,
+                           num_experts_per_tok, norm_topk_prob=False):
+    """Differentiable ``block_forward``: ``(out [T, H], router_logits [T, 2*nk])``."""
+    return FlashMoEBlockFunc.apply(tokens, gate_proj, up_proj, down_proj, router_gate, down_embed, up_embed, norm,
+                                   num_expert_keys, num_experts_per_tok, norm_topk_prob)

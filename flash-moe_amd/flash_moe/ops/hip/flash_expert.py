@@ -9,6 +9,7 @@ from __future__ import annotations
 import torch
 
 from flash_moe import _C
+from flash_moe.ops.utils import ensure_contiguous
 
 
 def expert_forward(hidden_states, down_weights, up_weights, indices, routing_weights, algo: int = _C.EXPERT_AUTO) -> torch.Tensor:
@@ -49,8 +50,18 @@ def flash_expert_func(hidden_states, down_weights, up_weights, indices, routing_
     return _C.native().expert_func(hidden_states, down_weights, up_weights, indices, routing_weights)
 
 
-class FlashExpertFunc:
-    """The differentiable op under the reference's class name (flash_moe/ops/triton/flash_expert.py:748); the autograd node is
-    native."""
+class FlashExpertFunc(torch.autograd.Function):
+    """``flash_expert_func`` as an autograd function under the reference's class name (flash_moe/ops/triton/flash_expert.py:748), for
+    callers that apply or subclass it; the op itself takes the native node, which keeps the scores as well."""
 
-    apply = staticmethod(flash_expert_func)
+    @staticmethod
+    @ensure_contiguous
+    def forward(ctx, hidden_states, down_weights, up_weights, indices, routing_weights):
+        ctx.save_for_backward(hidden_states, down_weights, up_weights, indices, routing_weights)
+        return expert_forward(hidden_states, down_weights, up_weights, indices, routing_weights)
+
+    @staticmethod
+    @ensure_contiguous
+    def backward(ctx, dexperts_states):
+        dx, dwd, dwu, dg = expert_backward(dexperts_states, *ctx.saved_tensors)
+        return dx, dwd, dwu, None, dg

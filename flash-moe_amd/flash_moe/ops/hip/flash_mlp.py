@@ -11,6 +11,7 @@ from typing import Optional
 import torch
 
 from flash_moe import _C
+from flash_moe.ops.utils import ensure_contiguous
 
 
 def mlp_forward(x, gate_weight, up_weight, down_weight, residual: Optional[torch.Tensor] = None) -> torch.Tensor:
@@ -42,7 +43,20 @@ def flash_mlp_func(x: torch.Tensor, gate_weight: torch.Tensor, up_weight: torch.
     return _C.native().mlp_func(x, gate_weight, up_weight, down_weight)
 
 
-class FlashMLPFunc:
-    """The differentiable op as a class, as autograd functions are called; the autograd node is native."""
+class FlashMLPFunc(torch.autograd.Function):
+    """``flash_mlp_func`` as an autograd function, for callers that apply or subclass it; the op itself takes the native node."""
 
-    apply = staticmethod(flash_mlp_func)
+    @staticmethod
+    @ensure_contiguous
+    def forward(ctx, x, gate_weight, up_weight, down_weight):
+        if x.numel() == 0 or not any(ctx.needs_input_grad):
+            ctx.save_for_backward(x, gate_weight, up_weight, down_weight)
+            return mlp_forward(x, gate_weight, up_weight, down_weight)
+        out, saved = mlp_forward_saving(x, gate_weight, up_weight, down_weight)
+        ctx.save_for_backward(x, gate_weight, up_weight, down_weight, saved)
+        return out
+
+    @staticmethod
+    @ensure_contiguous
+    def backward(ctx, dout):
+        return mlp_backward(dout, *ctx.saved_tensors)

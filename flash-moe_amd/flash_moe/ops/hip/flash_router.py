@@ -11,6 +11,7 @@ from typing import Optional, Tuple
 import torch
 
 from flash_moe import _C
+from flash_moe.ops.utils import ensure_contiguous
 
 
 def router_topk_gates(
@@ -131,8 +132,38 @@ def flash_router_func(router_logits, num_expert_keys, num_experts_per_tok):
     return _C.native().router_func(router_logits, num_expert_keys, num_experts_per_tok)
 
 
-class FlashRouterFunc:
-    """The differentiable op under the reference's class name (flash_moe/ops/triton/flash_router.py:347); the autograd node is
-    native."""
+class FlashRouterFunc(torch.autograd.Function):
+    """``flash_router_func`` as an autograd function under the reference's class name (flash_moe/ops/triton/flash_router.py:347),
+    for callers that apply or subclass it; the op itself takes the native node."""
 
-    apply = staticmethod(flash_router_func)
+    @staticmethod
+    @ensure_contiguous
+    def forward(ctx, router_logits, num_expert_keys, num_experts_per_tok):
+        scores, indices, _ = router_topk_gates(router_logits, num_expert_keys, num_experts_per_tok)
+        ctx.mark_non_differentiable(indices)
+        ctx.save_for_backward(indices)
+        ctx.num_expert_keys = num_expert_keys
+        return scores, indices
+
+    @staticmethod
+    @ensure_contiguous
+    def backward(ctx, dscores, dindices):
+        (indices,) = ctx.saved_tensors
+        return router_topk_backward(dscores, indices, ctx.num_expert_keys), None, None
+
+
+class RouterPrologueFunc(torch.autograd.Function):
+    """``router_prologue`` as an autograd function."""
+
+    @staticmethod
+    def forward(ctx, tokens, gate_weight, norm):
+        logits, _, _, _, logits32, stats = router_forward(tokens, gate_weight, norm, gate_weight.shape[0] // 2, 0,
+                                                          return_logits32=True, return_stats=True)
+        ctx.save_for_backward(tokens, gate_weight, stats.clone())
+        ctx.training = norm.training
+        return logits32, logits
+
+    @staticmethod
+    def backward(ctx, dlogits32, dlogits):
+        tokens, gate_weight, stats = ctx.saved_tensors
+        return (*router_prologue_backward(dlogits32 + dlogits.float(), tokens, gate_weight, stats, ctx.training), None)

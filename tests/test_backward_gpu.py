@@ -107,6 +107,49 @@ def test_block_autograd_node_equals_the_composition_of_ops(dtype, norm):
         assert rel_fro(gp0[k], gp1[k]) < tol, (k, rel_fro(gp0[k], gp1[k]))
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("what", ["router", "prologue", "expert", "mlp", "block"])
+def test_autograd_functions_by_class_equal_the_native_nodes(what, dtype):
+    """The classes under the reference's names give the outputs and gradients of the ops, whose nodes are native."""
+    from flash_moe.modules.flash_moe import FlashMoE, FlashMoEConfig
+    from flash_moe.ops import flash_expert_func, flash_mlp_func, flash_router_func
+    from flash_moe.ops.hip import flash_block as fb, flash_expert as fe, flash_mlp as fm, flash_router as fr
+
+    T, H, I, E, K = 96, 128, 264, 1024, 8
+    g = gen(3)
+    m = FlashMoE(FlashMoEConfig(H, I, "silu", E, K, True)).to(device="cuda", dtype=dtype)
+    wg, wu, wd, wr, ed, eu = (p.detach() for p in (m.gate_proj.weight, m.up_proj.weight, m.down_proj.weight, m.router_gate.weight,
+                                                   m.down_embed.weight, m.up_embed.weight))
+    x = torch.randn(T, H, generator=g).to(dtype).cuda()
+    idx = torch.randint(0, E, (T, K), generator=g).cuda()
+    gates = torch.rand(T, K, generator=g).to(dtype).cuda()
+    logs = torch.log_softmax(torch.randn(2, T, 32, generator=g), -1).to(dtype).cuda()
+
+    def native_block(*leaves):
+        out, logits = fb.block(*leaves[:5], m.router_norm, *leaves[5:], 32, K, True, differentiable=True)
+        return out, logits.transpose(0, 1).reshape(T, 64)
+
+    leaves, by_class, native = {
+        "router": ([logs], lambda t: fr.FlashRouterFunc.apply(t, 32, K), lambda t: flash_router_func(t, 32, K)),
+        "prologue": ([x, wr], lambda *t: fr.RouterPrologueFunc.apply(*t, m.router_norm), lambda *t: fr.router_prologue(*t, m.router_norm)),
+        "expert": ([x, ed, eu, gates], lambda a, d, u, w: fe.FlashExpertFunc.apply(a, d, u, idx, w),
+                   lambda a, d, u, w: flash_expert_func(a, d, u, idx, w)),
+        "mlp": ([x, wg, wu, wd], fm.FlashMLPFunc.apply, flash_mlp_func),
+        "block": ([x, wg, wu, wd, wr, ed, eu],
+                  lambda *t: fb.block_forward_autograd(*t[:5], m.router_norm, *t[5:], 32, K, True), native_block),
+    }[what]
+    results = []
+    for fn in (by_class, native):
+        ts = [t.clone().requires_grad_() for t in leaves]
+        out = fn(*ts)
+        out = [o for o in (out if isinstance(out, tuple) else (out,)) if o.requires_grad]
+        torch.autograd.backward(out, [torch.randn(o.shape, generator=gen(5)).to(o.dtype).cuda() for o in out])
+        results.append([o.detach() for o in out] + [t.grad for t in ts])
+    # two library paths in the same types: sums in another order, the block's token gradients rounded once or three times
+    for a, b in zip(*results):
+        assert a.dtype == b.dtype and rel_fro(a, b.cpu()) < (1e-5 if dtype == torch.float32 else 1e-2)
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("shape", [(7, 64), (3, 5, 256), (128, 1024)])
 def test_swiglu_backward(dtype, shape):

@@ -59,6 +59,18 @@ def test_reference_import_paths_resolve_to_the_hip_ops():
     assert list(inspect.signature(m1).parameters) == ["x", "gate_weight", "up_weight", "down_weight"]
 
 
+def test_op_classes_are_autograd_functions_and_forward_names_exist():
+    from flash_moe.ops.hip import flash_block, flash_expert, flash_mlp, flash_router, peer, pkm
+    from flash_moe.ops.triton.peer import TritonPEERFunc
+    from flash_moe.ops.triton.pkm import TritonPKMFunc
+
+    for cls in (flash_router.FlashRouterFunc, flash_router.RouterPrologueFunc, flash_expert.FlashExpertFunc, flash_mlp.FlashMLPFunc,
+                flash_block.FlashMoEBlockFunc, peer.PEERFunc, pkm.PKMFunc, TritonPEERFunc, TritonPKMFunc):
+        assert issubclass(cls, torch.autograd.Function) and "forward" in vars(cls) and "backward" in vars(cls)
+    for fn in (flash_block.block_forward_autograd, peer.peer_forward, pkm.pkm_forward):
+        assert inspect.isfunction(fn)
+
+
 def test_router_assertions_match_reference_wording():
     # flash_router.py:257-263: AssertionError for a non-3D input, a first dimension != 2, K outside [0, nk]
     from flash_moe.ops import flash_router_func

@@ -58,6 +58,24 @@ def test_pkm_forward(dtype, T, H, E, K):
     assert_output_close(out, ref.to(dtype), dtype, "pkm")
 
 
+def test_peer_and_pkm_by_class_and_by_forward_name():
+    from flash_moe.ops.hip.peer import PEERFunc, peer_forward, peer_func
+    from flash_moe.ops.hip.pkm import PKMFunc, pkm_forward, pkm_func
+
+    g = torch.Generator().manual_seed(2)
+    x, wd, wu = (torch.randn(*s, generator=g).cuda() for s in ((20, 64), (300, 64), (300, 64)))
+    w, idx = torch.rand(20, 7, generator=g).cuda(), torch.randint(0, 300, (20, 7), generator=g).cuda()
+    want = peer_func(x, wd, wu, w, idx)
+    assert torch.equal(peer_forward(x, wd, wu, w, idx), want)
+    want_pkm = pkm_func(wd, w, idx)
+    assert torch.equal(pkm_forward(wd, w, idx), want_pkm)
+    x.requires_grad_(), wd.requires_grad_()
+    for out, same in ((PEERFunc.apply(x, wd, wu, w, idx), want), (PKMFunc.apply(wd, w, idx), want_pkm)):
+        assert torch.equal(out.detach(), same)
+        with pytest.raises(NotImplementedError):
+            out.sum().backward()
+
+
 def test_pkm_closed_forms():
     from flash_moe.ops import pkm_func
 
