@@ -14,7 +14,7 @@ import torch
 from flash_moe import _C
 from flash_moe.ops.hip.flash_expert import expert_backward, expert_forward
 from flash_moe.ops.hip.flash_mlp import mlp_backward, mlp_forward_saving
-from flash_moe.ops.hip.flash_router import check_norm, route_backward, router_forward, router_prologue_backward
+from flash_moe.ops.hip.flash_router import check_norm, check_router_args, route_backward, router_forward, router_prologue_backward
 
 
 def block_forward(tokens: torch.Tensor, gate_proj: torch.Tensor, up_proj: torch.Tensor, down_proj: torch.Tensor,
@@ -24,6 +24,7 @@ def block_forward(tokens: torch.Tensor, gate_proj: torch.Tensor, up_proj: torch.
     """tokens [T, H] -> ``(out [T, H], router_logits [T, 2*nk])`` in tokens.dtype, plus ``(indices int64, gates)``
     [T, K] when ``return_routing`` is set.  ``norm.training`` selects batch or running statistics; the running
     statistics are updated in place in training mode."""
+    check_router_args(tokens, router_gate, norm, num_expert_keys, num_experts_per_tok)      # tokens are 2-D here, unlike in block()
     out, logits, *routing = block(tokens, gate_proj, up_proj, down_proj, router_gate, norm, down_embed, up_embed, num_expert_keys,
                                   num_experts_per_tok, norm_topk_prob, return_routing=return_routing)
     return (out, logits.transpose(0, 1).reshape(tokens.shape[0], 2 * num_expert_keys), *routing)

@@ -119,6 +119,20 @@ def test_forward_mode_is_refused(op, device):
                 call(primal)
 
 
+@pytest.mark.parametrize("shape", [(2, 3, 16), (2, 1, 16), (1, 16, 16)])
+def test_block_forward_takes_tokens_in_two_dimensions_only(shape):
+    """Refused before a kernel runs or the running statistics change."""
+    from flash_moe.ops.hip.flash_block import block_forward, block_forward_autograd
+
+    m = FlashMoE(FlashMoEConfig(16, 32, "silu", 100, 3)).requires_grad_(False)
+    args = (torch.randn(shape), m.gate_proj.weight, m.up_proj.weight, m.down_proj.weight, m.router_gate.weight, m.router_norm,
+            m.down_embed.weight, m.up_embed.weight, 10, 3)
+    for fn in (block_forward, block_forward_autograd):
+        with pytest.raises(ValueError, match=r"tokens \[T, H\]"):
+            fn(*args)
+    assert int(m.router_norm.num_batches_tracked) == 0
+
+
 def test_utils():
     assert [next_power_of_2(n) for n in (0, 1, 2, 3, 4, 5, 1023, 1024, 1025)] == [1, 1, 2, 4, 4, 8, 1024, 1024, 2048]
     seen = {}
