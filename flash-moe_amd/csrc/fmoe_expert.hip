@@ -1400,24 +1400,35 @@ bool slices_chosen(int64_t T_, int H, int64_t E, int K, size_t elt) {
 // Grouping the pairs by expert pays once an expert's row serves about a dozen pairs (measured: 16 pairs per expert, bucketed
 // 10-25 % ahead of whole-row gathers; 8 pairs per expert, 15 % behind): below that the rows are better gathered whole, straight
 // from HBM.
-// Ordered slices pay when the slices of the table do not stay in L2 and 400 tokens name every expert about once or more, so that a
-// window of the slice serves several of the gathers in flight.  Measured at H = 1024, E = 102400, bf16 (ordered against the better
-// of whole rows and buckets): 1024 tokens x 160 experts 104 against 96 us, x 512 227 against 290, x 1250 428 against 722;
-// 4096 x 512 655 against 907; 300 x 1000 160 against 243.
+// Ordered slices pay when the slices of the table do not stay in L2 and 400 tokens name every expert about once or more, so that the
+// gathers in flight (400 to 5000 tokens of an XCD, ordered_tokens_per_wave) meet in a window of the slice.  Measured in bf16, ordered
+// against the better of whole rows and buckets, us, ids uniform | ids a product-key router selects, whose lists keep less in step:
+//   H 1024, E 102400   1024 tokens x 256 139 for 150 | 145 for 148, x 512 227 for 290 | 243 for 290;  4096 x 256 406 for 573 | 529 for 578,
+//                      x 512 660 for 906 | 977 for 900;  16384 x 512 2807 for 3920 | 4205 for 3854
+//   H 2048, E 160000   2048 tokens x 800 1339 for 1446 | 1685 for 1440;  8192 x 512 3443 for 3555 | 4562 for 3523
+//   H 512, E 75076     1024 tokens x 512 79 for 142 | 97 for 142;  8192 x 400: 547 for 825 | 787 for 809 (E 102400)
+// Fewer experts per token do not pay however many tokens there are: H 1024, E 102400, 16384 tokens x 64 599 for 556 | 627 for 552, x 16
+// 202 for 156; 4096 x 128 alone is better for uniform ids, 252 for 297 | 287 for 292; E 262144, 32768 x 128 2571 for 1965.
 bool ordered_possible(int64_t E, int H, int K, size_t elt) { return slices_possible(E, H, elt) && K <= kOrderMaxTopK; }
 bool ordered_pays(int64_t T_, int64_t E, int K) {
     const int64_t resident = T_ < 400 ? T_ : 400;
     return !slices_pay(T_, E, K) && T_ * K >= (1ll << 16) && resident * K >= E;
 }
 bool buckets_pay(int64_t T_, int64_t E, int K) { return !slices_pay(T_, E, K) && T_ * K >= (1ll << 16) && T_ * K >= 12 * E; }
-int choose_schedule(int algo, int64_t T_, int H, int64_t E, int K, size_t elt, bool scored = true) {
+// Where both pay, rows of 4 KB and hardly more than 400 K = E ids in step leave the forward to the buckets: at H 2048, E 102400, 256 experts
+// per token, ordered takes 3440 us of 16384 tokens for 3218 in buckets and 7641 of 32768 for 6653 (uniform ids), 4429 for 3183 and 9065 for
+// 6444 (a router's).  The training step keeps the ordered lists, which its backward walks too: 12.1 ms for 13.7 and 26.2 for 28.2 | 11.3
+// for 12.5 and 24.0 for 26.3.
+bool buckets_ahead(int64_t E, int H, int K, size_t elt) { return (size_t)H * elt >= 4096 && 400ll * K * 100 < E * 135; }
+// keeps: the forward of a training step
+int choose_schedule(int algo, int64_t T_, int H, int64_t E, int K, size_t elt, bool scored = true, bool keeps = false) {
     if (K == 0) return FMOE_EXPERT_ROWS;
     if (algo != FMOE_EXPERT_AUTO) return algo;
     if (slices_chosen(T_, H, E, K, elt)) return FMOE_EXPERT_SLICES;
-    if (ordered_pays(T_, E, K) && ordered_possible(E, H, K, elt)) return FMOE_EXPERT_ORDERED;
     // grouping by expert serves the score phase; an op without scores (product-key memory) has nothing to group
-    if (scored && buckets_pay(T_, E, K) && bucketed_possible(T_, E, H, K, elt)) return FMOE_EXPERT_BUCKETS;
-    return FMOE_EXPERT_ROWS;
+    const bool buckets = scored && buckets_pay(T_, E, K) && bucketed_possible(T_, E, H, K, elt);
+    if (ordered_pays(T_, E, K) && ordered_possible(E, H, K, elt) && (keeps || !buckets || !buckets_ahead(E, H, K, elt))) return FMOE_EXPERT_ORDERED;
+    return buckets ? FMOE_EXPERT_BUCKETS : FMOE_EXPERT_ROWS;
 }
 
 }  // namespace
@@ -1443,11 +1454,12 @@ int expert_rows_added(const void* x, const void* down, const void* up, const int
     return FMOE_OK;
 }
 
-// What a forward in the slice or ordered schedule leaves for the backward (which takes the same schedule for these extents).
+// What the forward of a training step in the slice or ordered schedule leaves for the backward (which takes the same schedule for these
+// extents).
 ExpertSavedPlan expert_saved_plan(int64_t num_tokens, int hidden, int64_t num_experts, int top_k, int dtype) {
     ExpertSavedPlan p = {};
     if (num_tokens <= 0 || top_k <= 0) return p;
-    const int schedule = choose_schedule(FMOE_EXPERT_AUTO, num_tokens, hidden, num_experts, top_k, dtype_size(dtype));
+    const int schedule = choose_schedule(FMOE_EXPERT_AUTO, num_tokens, hidden, num_experts, top_k, dtype_size(dtype), true, true);
     p.kept = schedule == FMOE_EXPERT_SLICES || schedule == FMOE_EXPERT_ORDERED;
     p.ordered = schedule == FMOE_EXPERT_ORDERED;
     if (!p.kept) return p;
@@ -1526,7 +1538,11 @@ extern "C" size_t fmoe_expert_workspace_bytes_algo(int64_t num_tokens, int hidde
 }
 
 extern "C" size_t fmoe_expert_workspace_bytes(int64_t num_tokens, int hidden, int64_t num_experts, int top_k, int dtype) {
-    return fmoe_expert_workspace_bytes_algo(num_tokens, hidden, num_experts, top_k, dtype, FMOE_EXPERT_AUTO);
+    // enough for the forward of a training step as well, which may take another schedule
+    const size_t plain = fmoe_expert_workspace_bytes_algo(num_tokens, hidden, num_experts, top_k, dtype, FMOE_EXPERT_AUTO);
+    if (plain == 0 || !fmoe::expert_saved_plan(num_tokens, hidden, num_experts, top_k, dtype).ordered) return plain;
+    const size_t ordered = fmoe_expert_workspace_bytes_algo(num_tokens, hidden, num_experts, top_k, dtype, FMOE_EXPERT_ORDERED);
+    return ordered > plain ? ordered : plain;
 }
 
 extern "C" size_t fmoe_pkm_workspace_bytes(int64_t num_tokens, int hidden, int64_t num_experts, int top_k, int dtype) {
@@ -1637,9 +1653,10 @@ extern "C" int fmoe_expert_forward_save(const void* x, const void* down, const v
     FMOE_REQUIRE(need == 0 || (saved && saved_bytes >= need && aligned16(saved)), FMOE_ERR_WORKSPACE,
                  "fmoe_expert_forward_save: buffer of %zu bytes needed, %zu given", need, saved_bytes);
     ExpertSaved kept = {};
-    if (need) kept = expert_saved_plan(num_tokens, hidden, num_experts, top_k, dtype).at(saved);
+    const ExpertSavedPlan plan = expert_saved_plan(num_tokens, hidden, num_experts, top_k, dtype);
+    if (need) kept = plan.at(saved);
     return expert_dispatch("fmoe_expert_forward_save", kActSilu, x, down, up, indices, gates, num_tokens, hidden, num_experts, top_k, dtype,
-                           out, workspace, workspace_bytes, FMOE_EXPERT_AUTO, stream, need ? &kept : nullptr);
+                           out, workspace, workspace_bytes, plan.ordered ? FMOE_EXPERT_ORDERED : FMOE_EXPERT_AUTO, stream, need ? &kept : nullptr);
 }
 
 extern "C" int fmoe_peer_forward(const void* x, const void* down, const void* up, const void* routing_weights,

@@ -244,7 +244,8 @@ Tensor expert_forward_impl(const Tensor& hidden_states, const Tensor& down, cons
     const Tensor x = hidden_states.contiguous(), wd = down.contiguous(), wu = up.contiguous(), idx = indices.contiguous(), g = weights.contiguous();
     Launch call(x);
     Tensor out = at::empty_like(x);
-    const size_t bytes = fmoe_expert_workspace_bytes_algo(T, (int)H, E, (int)K, code, (int)algo);
+    const size_t bytes = saved != nullptr ? fmoe_expert_workspace_bytes(T, (int)H, E, (int)K, code)
+                                          : fmoe_expert_workspace_bytes_algo(T, (int)H, E, (int)K, code, (int)algo);
     Tensor ws = bytes ? workspace(x, bytes) : Tensor();
     if (saved != nullptr) {
         const size_t kept = fmoe_expert_saved_bytes(T, (int)H, E, (int)K, code);
@@ -335,7 +336,7 @@ Tensor peer_forward(const Tensor& hidden_states, const Tensor& down, const Tenso
     const Tensor x = hidden_states.contiguous(), wd = down.contiguous(), wu = up.contiguous(), w = weights.contiguous(), idx = indices.contiguous();
     Launch call(x);
     Tensor out = at::empty_like(x);
-    const size_t bytes = fmoe_expert_workspace_bytes(T, (int)H, E, (int)K, code);
+    const size_t bytes = fmoe_expert_workspace_bytes_algo(T, (int)H, E, (int)K, code, FMOE_EXPERT_AUTO);
     Tensor ws = workspace(x, bytes);
     check(fmoe_peer_forward(ptr(x), ptr(wd), ptr(wu), ptr(w), (const int64_t*)ptr(idx), T, (int)H, E, (int)K, code, ptr(out), ptr(ws),
                             bytes, call.stream), "peer");

@@ -229,6 +229,16 @@ def test_backward_argument_checks():
     assert mb(a, a, a, a, a, a, 8, 64, 128, _C.BF16, a, a, a, a, a, sneed - 1, None) == -7      # with saved products
 
 
+def test_expert_workspace_is_enough_for_both_forwards():
+    """The forward of a training step may take the ordered lists where the other takes buckets: one size for both."""
+    lib = _C.lib()
+    for T, H, E, K in ((4800, 2048, 66049, 222), (16384, 2048, 102400, 256), (1024, 1024, 102400, 512), (4096, 1024, 16384, 64)):
+        need = lib.fmoe_expert_workspace_bytes(T, H, E, K, _C.BF16)
+        assert need >= lib.fmoe_expert_workspace_bytes_algo(T, H, E, K, _C.BF16, _C.EXPERT_AUTO)
+        if K > 64:
+            assert need >= lib.fmoe_expert_workspace_bytes_algo(T, H, E, K, _C.BF16, _C.EXPERT_ORDERED)
+
+
 def test_training_keeps_two_planes_of_the_intermediate_width():
     """What a block's forward leaves for its backward grows by the gate and up products, [2, T, I], with the intermediate width."""
     lib = _C.lib()

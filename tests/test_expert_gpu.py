@@ -333,6 +333,29 @@ def test_expert_ordered_lists(dtype, T, H, E, K):
     assert rel_fro(got[sample.cuda()], ref) < tol
 
 
+@pytest.mark.parametrize("dtype,H,K", [(torch.float32, 1024, 166), (torch.bfloat16, 2048, 222), (torch.bfloat16, 2048, 223), (torch.bfloat16, 2040, 166)])
+def test_expert_forward_and_training_step_where_buckets_and_ordered_lists_both_pay(dtype, H, K):
+    """Rows of 4 KB, 400 tokens that name every expert hardly more than once, twelve pairs per expert: without gradients the forward
+    groups by expert, in a training step it walks ordered lists.  One expert per token more, and rows shorter than 4 KB, are ordered
+    in both.  Both against the float64 oracle on a sample."""
+    from flash_moe.ops import flash_expert_func
+
+    T, E = 4800, 66049
+    g = torch.Generator().manual_seed(K)
+    x, wd, wu = (torch.randn(n, H, generator=g).mul(s).to(dtype) for n, s in ((T, 1.0), (E, 0.05), (E, 0.05)))
+    idx = torch.randint(0, E, (T, K), generator=g)
+    gates = torch.softmax(torch.randn(T, K, generator=g), -1).to(dtype)
+    args = cuda(x, wd, wu, idx, gates)
+    with torch.no_grad():
+        plain = flash_expert_func(*args)
+    trained = flash_expert_func(args[0].requires_grad_(), *args[1:]).detach()
+    sample = torch.arange(0, T, 120)
+    ref = truth64(x[sample], wd, wu, idx[sample], gates[sample])
+    tol = {torch.float32: 2e-6, torch.bfloat16: 5e-3}[dtype]
+    for out in (plain, trained):
+        assert rel_fro(out[sample.cuda()], ref) < tol
+
+
 @pytest.mark.parametrize("T,H,E,K", [(64, 128, 256, 8), (300, 264, 700, 230), (70, 64, 66000, 1000)])    # rows, slices, ordered lists
 def test_expert_backward_from_what_the_forward_kept(T, H, E, K):
     # the op's autograd keeps scores and list addresses where its schedule has them; the stand-alone backward recomputes them
