@@ -644,7 +644,10 @@ template <typename T> SlicePlan plan_slices_of_k(int M, int N, int K) {
     const int cus = chip_info().cus, k_tiles = (K + kStageK<T> - 1) / kStageK<T>;
     const double kRow = 2.3e-3, launch = split_k ? 8.5 : 4.0;
     double best_time = (split_k ? 0.8 : 0.9) * whole * k_tiles * kRow;
-    if (shape == kTile128 && tiles > cus) best_time *= 0.65;       // two to a compute unit hide each other's latency
+    // Two 128 x 128 tiles to a compute unit hide each other's latency, by how much depends on the extents in ways the price does not
+    // see: of 53 down products that would otherwise be sliced (bf16) 38 would gain, up to a third (1692 tokens, 10576 -> 3968: 192 whole,
+    // 131 in two slices), and 15 lose, up to a seventh (4918 tokens, 3456 -> 864: 41 whole, 47).  0.65 keeps all of them whole.
+    if (shape == kTile128 && tiles > cus) best_time *= 0.65;
     if (sizeof(T) == 4 && K % 4 != 0) return best;
     for (int i = sizeof(T) == 2 ? kTile256 : kTile128; i <= kTile64; ++i) {
         int64_t n = 0;

@@ -4,7 +4,7 @@
 //   gate_and_up_kernel       logits = BatchNorm(x) Wr^T   beside   act = silu(x Wg^T) * (x Wu^T)
 //   select_and_down_kernel   product-key selection and gates   beside   the fp32 sums of act Wd^T
 //   expert_token_kernel (fmoe_expert.hip)   the routed experts, plus those sums -> out
-// README block in bf16, evaluation mode: 8 tokens 39.0 -> 22.1 us, 64 tokens 42.6 -> 25.6.  @@
+// README block in bf16, evaluation mode: 8 tokens 39.0 -> 23.6 us, 64 tokens 42.6 -> 25.6.
 #include "fmoe_common.h"
 #include "fmoe_gate.h"
 #include "fmoe_gemm.h"

@@ -39,7 +39,7 @@ typedef enum {
     FMOE_ERR_UNSUPPORTED = -5,    /* extent beyond what the kernels are built for (message says which) */
     FMOE_ERR_ALIGNMENT = -6,      /* pointer not 16-byte aligned or row length not a multiple of 16 bytes */
     FMOE_ERR_WORKSPACE = -7,      /* workspace NULL or smaller than the *_workspace_bytes() figure */
-    FMOE_ERR_LIBRARY = -8         /* rocBLAS (backward GEMMs only) could not be loaded or reported a failure */
+    FMOE_ERR_LIBRARY = -8         /* rocBLAS (backward GEMMs whose operands this library's kernels cannot address) could not be loaded or reported a failure */
 } fmoe_status_t;
 
 /* ABI version of the loaded library (== FMOE_ABI_VERSION it was built with). */
@@ -145,8 +145,8 @@ int fmoe_router_forward_noalloc(const void* x, const void* gate_w, void* running
  * Duplicate ids in a row add, as in the reference.  An id outside [0,E) contributes nothing (the
  * reference reads out of bounds).  Accumulation is fp32 and deterministic (no atomics); `out` is
  * written once, it need not be zeroed.
- * fmoe_expert_workspace_bytes() gives the scratch fmoe_expert_forward needs for these extents (0 when it takes the
- * row schedule); pass a 256-byte aligned buffer of at least that size.  fmoe_expert_workspace_bytes_algo() gives it
+ * fmoe_expert_workspace_bytes() gives the scratch fmoe_expert_forward and fmoe_expert_forward_save need for these extents (0 when
+ * they take the row schedule); pass a 256-byte aligned buffer of at least that size.  fmoe_expert_workspace_bytes_algo() gives it
  * for a schedule forced through fmoe_expert_forward_algo().
  * Limits of this build: hidden a whole number of 16-byte packets (FMOE_ERR_ALIGNMENT); E < 2^31 and T*K < 2^40; and per
  * schedule (FMOE_ERR_UNSUPPORTED when a call can take none of them, or when the forced one does not apply):
@@ -157,7 +157,8 @@ int fmoe_router_forward_noalloc(const void* x, const void* gate_w, void* running
  *   ordered  tables below 4 GiB, K <= 65536
  * fmoe_expert_forward picks slices when E*128 bytes fit twice the L2 of one XCD and there are at least 65536 pairs, or
  * when the rows are too long for the row schedule; else ordered when there are at least 65536 pairs and min(T, 400) * K >= E
- * (the tokens in flight then share the table's rows); else buckets when there are at least 65536 pairs and 12 pairs per
+ * (the tokens in flight then share the table's rows; without gradients rows of 4 KB and more go to buckets while 400 * K is below
+ * 1.35 * E and those apply); else buckets when there are at least 65536 pairs and 12 pairs per
  * expert (each table row then serves enough pairs to pay for the grouping) and its limits hold; else rows.  So any
  * hidden size works as long as each table stays below 4 GiB.
  */
@@ -356,7 +357,7 @@ int fmoe_route_backward(const void* dgates, const int64_t* indices, const float*
  * fp32, at byte offset fmoe_router_workspace_stats_offset() of its workspace; pass that as mean_rstd.
  *   dlogits_fp32 [T, 2*nk] fp32 (rounded to dtype for the two GEMMs); dx [T,H], dgate_w [2*nk,H]: dtype.
  * training != 0: batch statistics were used (the gradient flows through mean and variance); else running statistics
- * (constants).  The two GEMMs are rocBLAS calls, or this library's own kernels up to 5 GFLOP in the 16-bit dtypes.
+ * (constants).  The two GEMMs run on this library's kernels, as those of fmoe_mlp_backward.
  * Limits of this build: num_tokens < 2^24; hidden a whole number of 16-byte packets; any num_keys the forward accepts. */
 size_t fmoe_router_workspace_stats_offset(int64_t num_tokens, int hidden, int num_keys);
 size_t fmoe_router_prologue_backward_workspace_bytes(int64_t num_tokens, int hidden, int num_keys, int dtype);
