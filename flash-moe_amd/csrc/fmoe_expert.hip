@@ -1403,7 +1403,7 @@ bool slices_chosen(int64_t T_, int H, int64_t E, int K, size_t elt) {
 // Ordered slices pay when the slices of the table do not stay in L2 and 400 tokens name every expert about once or more, so that the
 // gathers in flight (400 to 5000 tokens of an XCD, ordered_tokens_per_wave) meet in a window of the slice.  Measured in bf16, ordered
 // against the better of whole rows and buckets, us, ids uniform | ids a product-key router selects, whose lists keep less in step:
-//   H 1024, E 102400   1024 tokens x 256 139 for 150 | 145 for 148, x 512 227 for 290 | 243 for 290;  4096 x 256 406 for 573 | 529 for 578,
+//   H 1024, E 102400   1024 tokens x 256 139 for 150 | 145 for 148, x 512 223 for 291 | 252 for 291;  4096 x 256 406 for 573 | 529 for 578,
 //                      x 512 660 for 906 | 977 for 900;  16384 x 512 2807 for 3920 | 4205 for 3854
 //   H 2048, E 160000   2048 tokens x 800 1339 for 1446 | 1685 for 1440;  8192 x 512 3443 for 3555 | 4562 for 3523
 //   H 512, E 75076     1024 tokens x 512 79 for 142 | 97 for 142;  8192 x 400: 547 for 825 | 787 for 809 (E 102400)
