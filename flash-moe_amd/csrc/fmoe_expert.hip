@@ -407,7 +407,7 @@ __global__ __launch_bounds__(256) void expert_scores_slice_kernel(
 #pragma unroll
             for (int u = 0; u < CL; ++u) {
                 const uint32_t o = (uint32_t)__builtin_amdgcn_ds_bpermute((u * PPL + pg) * 4, (int)mine);
-                w[u] = load_row_piece(rsrc, o + col_bytes);
+                w[u] = load_row_piece(rsrc, col_ok ? o + col_bytes : kBadOffset);      // zeros beyond the row: x is zero there, and so must w be
             }
             float part[CL];
 #pragma unroll
@@ -751,7 +751,7 @@ __global__ __launch_bounds__(256) void expert_scores_ordered_kernel(const T* __r
 #pragma unroll
         for (int u = 0; u < CL; ++u) {
             const uint32_t o = (uint32_t)__builtin_amdgcn_ds_bpermute((u / QL * QP + (u % QL) * PPL + pg) * 4, (int)mine);
-            w[u] = load_row_piece(rsrc, o + col_bytes);
+            w[u] = load_row_piece(rsrc, col_ok ? o + col_bytes : kBadOffset);          // as in the slice kernel
         }
         const int next = k0 + QP + my_at;
         mine = my_token < tokens && next < top_k ? my_list[next] : kBadOffset;

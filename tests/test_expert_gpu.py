@@ -333,6 +333,30 @@ def test_expert_ordered_lists(dtype, T, H, E, K):
     assert rel_fro(got[sample.cuda()], ref) < tol
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("algo", ["ROWS", "SLICES", "ORDERED"])
+@pytest.mark.parametrize("T,H,E,K", [(70, 72, 300, 5), (40, 8, 20000, 33), (700, 200, 500, 20)])
+def test_expert_infinite_weights_and_a_partial_last_slice(dtype, algo, T, H, E, K):
+    """Lanes beyond the last column multiply zeros by zeros: an infinite weight makes the scores of its own expert infinite and
+    nothing else, and those are not NaN."""
+    from flash_moe import _C
+    from flash_moe.ops.hip.flash_expert import expert_forward
+
+    g = torch.Generator().manual_seed(T)
+    x, wd, wu = (torch.randn(n, H, generator=g).mul(s).to(dtype) for n, s in ((T, 1.0), (E, 0.05), (E, 0.05)))
+    x[:, 0] = x[:, 0].abs() + 0.1
+    wu[wu == 0] = 0.01
+    idx = torch.randint(1, E, (T, K), generator=g)
+    idx[::3, K // 2] = 0                                        # expert 0: score +inf, so its row times +inf
+    wd[0, 0] = float("inf")
+    gates = torch.softmax(torch.randn(T, K, generator=g), -1).to(dtype)
+    got = expert_forward(*cuda(x, wd, wu, idx, gates), algo=getattr(_C, "EXPERT_" + algo)).cpu()
+    assert torch.equal(got[::3].double(), wu[0].double().sign().mul(float("inf")).expand_as(got[::3]))
+    others = torch.arange(T) % 3 != 0
+    ref = truth64(x[others], wd, wu, idx[others], gates[others])
+    assert rel_fro(got[others], ref) < {torch.float32: 2e-6, torch.bfloat16: 5e-3, torch.float16: 6e-4}[dtype]
+
+
 @pytest.mark.parametrize("dtype,H,K", [(torch.float32, 1024, 166), (torch.bfloat16, 2048, 222), (torch.bfloat16, 2048, 223), (torch.bfloat16, 2040, 166)])
 def test_expert_forward_and_training_step_where_buckets_and_ordered_lists_both_pay(dtype, H, K):
     """Rows of 4 KB, 400 tokens that name every expert hardly more than once, twelve pairs per expert: without gradients the forward
