@@ -27,9 +27,8 @@ template <int MT, int NT, int EPI> constexpr int kSplitLds = kSplitWaves * MT * 
 // ------------------------------------------------------------------------------------------------------------
 // LDS-DMA pipelined kernel.  WAVES_M x WAVES_N waves, each (BM/WAVES_M) x (BN/WAVES_N); BKT = k extent of a stage.
 // ------------------------------------------------------------------------------------------------------------
-// FR: fragment shape (32: v_mfma_f32_32x32x16 / 32x32x2; 16: v_mfma_f32_16x16x32).  SPLIT: a k-step's A fragments are read and
-// multiplied in SPLIT parts (its B fragments stay for the whole k-step), which halves the registers the read-ahead needs.
-template <typename T, int BM, int BN, int WAVES_M, int WAVES_N, int BKT, int NSTAGE, int EPI, int PF, int FR, int SPLIT, bool RAGGED, bool SLICED = false,
+// FR: fragment shape (32: v_mfma_f32_32x32x16 / 32x32x2; 16: v_mfma_f32_16x16x32).
+template <typename T, int BM, int BN, int WAVES_M, int WAVES_N, int BKT, int NSTAGE, int EPI, int PF, int FR, bool RAGGED, bool SLICED = false,
           bool TA = false, bool TB = false>
 __device__ __forceinline__ void gemm_dma_tiles(
     const T* __restrict__ A, const T* __restrict__ B0, const T* __restrict__ B1, T* __restrict__ C,
@@ -47,9 +46,7 @@ __device__ __forceinline__ void gemm_dma_tiles(
     constexpr int ROWS_PER_IT = NWAVES * RPI;       // rows all waves cover per DMA round
     constexpr int STAGE = (BM + BN) * BKT;          // elements per stage
     constexpr int KSTEPS = BKT / (Shape::kChunks * EPC);   // a k-step is kChunks 16-byte pieces of a row: one per lane group
-    constexpr int SPK = KSTEPS * SPLIT;             // steps (a part of a k-step's A fragments against all its B fragments) per k-tile
-    constexpr int MFS = MF / SPLIT;
-    static_assert(MF % SPLIT == 0 && WM % FR == 0 && WN % FR == 0, "fragments tile the wave tile");
+    static_assert(WM % FR == 0 && WN % FR == 0, "fragments tile the wave tile");
     constexpr int ROW_SHIFT = (CPR == 8) ? 1 : 2;   // log2(rows per 256 bytes)
     constexpr int BN_OUT = (EPI == kEpiSwiGLU) ? BN / 2 : BN;
     constexpr int A_ROUNDS = BM / ROWS_PER_IT, B_ROUNDS = BN / ROWS_PER_IT;
@@ -220,8 +217,8 @@ __device__ __forceinline__ void gemm_dma_tiles(
 
     // turned: byte address of the lane's piece in fragment 0's place; bits 5 to 7 (7 in fp32) of it are XOR-ed per fragment
     const int t_row = sizeof(T) == 4 ? fhalf * 4 : fhalf * 8 + frow / 4, t_piece = sizeof(T) == 4 ? frow * 4 : (frow % 4) * 8;
-    int ta_lane = t_row * BM * (int)sizeof(T) + (row_key(t_row, CHA) * 16 ^ t_piece);
-    int tb_lane = BM * BKT * (int)sizeof(T) + t_row * BN * (int)sizeof(T) + (row_key(t_row, CHB) * 16 ^ t_piece);
+    const int ta_lane = t_row * BM * (int)sizeof(T) + (row_key(t_row, CHA) * 16 ^ t_piece);
+    const int tb_lane = BM * BKT * (int)sizeof(T) + t_row * BN * (int)sizeof(T) + (row_key(t_row, CHB) * 16 ^ t_piece);
     auto turned_frag = [&](const char* stage, int lane_at, int piece, int ks, int cols) {
         constexpr int kBytes = FR * (int)sizeof(T), kInKey = 256 / kBytes;       // bytes of a fragment's columns in a k-row
         const char* at = stage + (lane_at ^ ((piece % kInKey) * kBytes)) + (piece / kInKey) * 256 + ks * (BKT / KSTEPS) * cols * (int)sizeof(T);
@@ -248,29 +245,22 @@ __device__ __forceinline__ void gemm_dma_tiles(
     for (int s = 0; s < NSTAGE - 1; ++s)
         if (s < k_tiles) issue(s, Lds::at() + s * STAGE);
 
-    // Fragments of step q+PF are read from LDS while the MFMAs of step q run (PF+1 register buffers for the A parts; B
-    // fragments are read with the first part of their k-step); the read-ahead crosses k-tile boundaries, so the barrier
+    // Fragments of k-step q+PF are read from LDS while the MFMAs of k-step q run (PF+1 register buffers); the read-ahead crosses k-tile boundaries, so the barrier
     // that publishes the next stage sits PF steps before the end of a k-tile and the matrix pipe always has work queued
     // while a wave waits.
     constexpr int RING = PF + 1;
-    constexpr int RINGB = SPLIT == 1 ? RING : 2;
-    static_assert(SPK % RING == 0 && PF >= 1 && PF < SPK + 1, "fragment buffers rotate with period RING");
-    static_assert(SPLIT == 1 || (PF <= SPLIT && KSTEPS % 2 == 0), "with split k-steps at most the next k-step's B fragments are in flight");
-    Frag fa[RING][MFS], fb[RINGB][NF];
-    auto b_slot = [](int q) { return SPLIT == 1 ? q % RING : (q / SPLIT) % 2; };     // q: step inside the k-tile (may exceed SPK by PF)
-    auto read_frags = [&](const char* stage, int q, Frag (&a)[MFS], Frag (&b)[NF]) {
-        const int ks = q / SPLIT, part = q % SPLIT;
+    static_assert(KSTEPS % RING == 0 && PF >= 1 && PF < KSTEPS + 1, "fragment buffers rotate with period RING");
+    Frag fa[RING][MF], fb[RING][NF];
+    auto read_frags = [&](const char* stage, int ks, Frag (&a)[MF], Frag (&b)[NF]) {
 #pragma unroll
-        for (int i = 0; i < MFS; ++i) {
-            if constexpr (TA) a[i] = turned_frag(stage, ta_lane, wm * (WM / FR) + part * MFS + i, ks, BM);
-            else a[i] = *reinterpret_cast<const Frag*>(stage + a_row_bytes + pc[ks] + (part * MFS + i) * FR * BKT * (int)sizeof(T));
+        for (int i = 0; i < MF; ++i) {
+            if constexpr (TA) a[i] = turned_frag(stage, ta_lane, wm * (WM / FR) + i, ks, BM);
+            else a[i] = *reinterpret_cast<const Frag*>(stage + a_row_bytes + pc[ks] + i * FR * BKT * (int)sizeof(T));
         }
-        if (part == 0) {
 #pragma unroll
-            for (int j = 0; j < NF; ++j) {
-                if constexpr (TB) b[j] = turned_frag(stage, tb_lane, wn * (WN / FR) + j, ks, BN);
-                else b[j] = *reinterpret_cast<const Frag*>(stage + b_row_bytes[j] + pc[ks]);
-            }
+        for (int j = 0; j < NF; ++j) {
+            if constexpr (TB) b[j] = turned_frag(stage, tb_lane, wn * (WN / FR) + j, ks, BN);
+            else b[j] = *reinterpret_cast<const Frag*>(stage + b_row_bytes[j] + pc[ks]);
         }
     };
     // Entering k-tile kt (kt = 0: from the tile prologue): my share of its stage has landed once at most the loads of
@@ -295,40 +285,36 @@ __device__ __forceinline__ void gemm_dma_tiles(
 
         enter_k_tile(0);
 #pragma unroll
-        for (int s = 0; s < PF; ++s) read_frags(reinterpret_cast<const char*>(Lds::at()), s, fa[s % RING], fb[b_slot(s)]);
+        for (int s = 0; s < PF; ++s) read_frags(reinterpret_cast<const char*>(Lds::at()), s, fa[s % RING], fb[s % RING]);
         // the last k-tile has no successor to read ahead into: it is a separate copy of the body, so that no branch
         // merges a path with reads in flight into the MFMA sequence
         auto k_tile_body = [&](int kt, auto last_tag) {
             constexpr bool kLast = decltype(last_tag)::value;
-            // with both operands turned the per-fragment XORs stay inside the k-tile: hoisted, they spill in the 256 x 256 tile
-            if constexpr (TA && BM == 256) asm volatile("" : "+v"(ta_lane), "+v"(tb_lane));
             const char* stage = reinterpret_cast<const char*>(Lds::at() + (kt % NSTAGE) * STAGE);
             const char* next_stage = reinterpret_cast<const char*>(Lds::at() + ((kt + 1) % NSTAGE) * STAGE);
 #pragma unroll
-            for (int q = 0; q < SPK; ++q) {
+            for (int q = 0; q < KSTEPS; ++q) {
                 const int nxt = q + PF;
-                constexpr int kMfmas = MFS * NF;     // runs of Shape::kInstr instructions
-                const bool reads = nxt < SPK || !kLast;
+                constexpr int kMfmas = MF * NF;     // runs of Shape::kInstr instructions
+                const bool reads = nxt < KSTEPS || !kLast;
                 constexpr int RT = sizeof(T) == 4 ? 4 : 2, RA = TA ? RT : 1, RB = TB ? RT : 1;       // LDS reads per fragment
-                const int n_reads = RA * MFS + ((nxt % SPLIT) == 0 ? RB * NF : 0);
+                constexpr int n_reads = RA * MF + RB * NF;
                 __builtin_amdgcn_sched_barrier(0);
-                if (nxt < SPK) {
-                    read_frags(stage, nxt, fa[nxt % RING], fb[b_slot(nxt)]);
+                if (nxt < KSTEPS) {
+                    read_frags(stage, nxt, fa[nxt % RING], fb[nxt % RING]);
                 } else if (!kLast) {
-                    if (nxt == SPK) {
+                    if (nxt == KSTEPS) {
                         enter_k_tile(kt + 1);
                         __builtin_amdgcn_sched_barrier(0);
                     }
-                    read_frags(next_stage, nxt - SPK, fa[nxt % RING], fb[b_slot(nxt)]);
+                    read_frags(next_stage, nxt - KSTEPS, fa[nxt % RING], fb[nxt % RING]);
                 }
-                const int part = q % SPLIT;
 #pragma unroll
-                for (int i = 0; i < MFS; ++i)
+                for (int i = 0; i < MF; ++i)
 #pragma unroll
-                    for (int j = 0; j < NF; ++j)
-                        acc[part * MFS + i][j] = Shape::run(fa[q % RING][i], fb[b_slot(q)][j], acc[part * MFS + i][j]);
+                    for (int j = 0; j < NF; ++j) acc[i][j] = Shape::run(fa[q % RING][i], fb[q % RING][j], acc[i][j]);
                 // issue order: the LDS reads spread evenly behind the MFMAs
-                constexpr int kPer = (RA * MFS + RB * NF + kMfmas - 1) / kMfmas;
+                constexpr int kPer = (n_reads + kMfmas - 1) / kMfmas;
 #pragma unroll
                 for (int m = 0; m < kMfmas; ++m) {
                     __builtin_amdgcn_sched_group_barrier(0x008, Shape::kInstr, 0);
@@ -580,10 +566,9 @@ __device__ __forceinline__ void gemm_splitk_tile(
 // k extent of one LDS stage of the DMA kernel: 128 bytes of a row for every element type
 template <typename T> constexpr int kStageK = 128 / (int)sizeof(T);
 // 16-bit products run on v_mfma_f32_16x16x32 (more multiply-adds per joule than 32x32x16, which is what bounds these
-// kernels); a k-step is then half a stage, so the read-ahead is one step, and the 256 x 256 tile reads a k-step's A
-// fragments in four parts to stay inside 256 registers per wave (in two parts it spills 24).  fp32 keeps 32x32x2.
+// kernels); a k-step is then half a stage, so the read-ahead is one step.  Their 256 x 256 tiles are in fmoe_gemm256.h.  fp32 keeps
+// 32x32x2.
 template <typename T> constexpr int kFragRows = sizeof(T) == 2 ? 16 : 32;
-template <typename T> constexpr int kBigSplit = sizeof(T) == 2 ? 4 : 1;
 template <typename T> constexpr int kSmallAhead = sizeof(T) == 2 ? 1 : 3;
 
 // Tile choice.  A workgroup's time per k-tile is the larger of what its CU receives from the L2 ((BM + BN) rows of 128 bytes, at 40

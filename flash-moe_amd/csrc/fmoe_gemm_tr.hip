@@ -5,15 +5,16 @@
 // k-row, and turned on the way to the matrix cores, in the 16-bit types by the LDS itself (ds_read_b64_tr_b16), in fp32 because a
 // lane reads its k values one by one.  Operands that are not whole 16-byte packets go to the library.
 //
-// What bounds it is what bounds the forward's products: what a compute unit receives on small tiles, the matrix pipes on 256 x 256,
+// What bounds it is what bounds the forward's products: what a compute unit receives on small tiles, the matrix pipes on 256 x 256
+// (fmoe_gemm256.h),
 // and, with few tiles and a long k loop, the length of one chain, which slices of k cut (their sums are added by a second launch, in
 // slice order).  A kernel that turned the operands in registers reached 600 TFLOP/s in bf16 where these reach 1000 to 1300.
 //
 // Against the library's kernels (rocBLAS), us:
-//   bf16  2048 tokens, 4096 -> 16384: dh 208 for 204, dx 447 for 496, dWd 222 for 243, dWg and dWu 463 for 516; 615 tokens, 776 -> 2072: 8
-//         for 16, 20 for 35, 8 for 17, 11 for 18; 32768 tokens, 2048 -> 8192: 1018 for 890, 1711 for 1726, 833 for 980, 1709 for 1891.
-//         Slower only for dh of many tokens on 256 x 256 tiles (4096 tokens and more, by 3 to 14 %) and dx of 12000 tokens of 3072 -> 768
-//         (124 for 106).
+//   bf16  2048 tokens, 4096 -> 16384: dh 187 for 203, dx 414 for 502, dWd 213 for 258, dWg and dWu 418 for 512; 4096 tokens, 1024 -> 4096:
+//         31 for 33, 71 for 79, 39 for 45, 62 for 69; 615 tokens, 776 -> 2072: 8 for 17, 20 for 36, 7 for 17, 11 for 18; 32768 tokens, 2048
+//         -> 8192: 871 for 871, 1501 for 1648, 783 for 944, 1613 for 1891.  Before the waves of a 256 x 256 tile worked in two groups
+//         (fmoe_gemm256.h): 2048 tokens 206, 442, 221, 438; 8192 tokens of 2048 -> 8192 223, 406, 199, 428 for 198, 370, 193, 409 now.
 //   fp32  383 tokens, 1880 -> 7520: dh 97 for 88, dx 200 for 828, dWd 100 for 105, dWg and dWu 191 for 218; 1000 tokens, 1024 -> 4096: 71
 //         for 64, 136 for 120, 69 for 71, 125 for 152; 4096 tokens, 1024 -> 4096: 257 for 242, 520 for 460, 260 for 231, 479 for 455; 5000
 //         tokens, 2048 -> 5464: 897 for 812, 1791 for 2426, 867 for 1094, 1746 for 1913; 16384 tokens, 512 -> 2048: 258 for 246, 488 for
@@ -22,6 +23,7 @@
 //         Products of less than a round of tiles take up to 3 us longer (dq of 600 tokens, 256 -> 256: 7.6 for 6.1).
 #include "fmoe_common.h"
 #include "fmoe_gemm.h"
+#include "fmoe_gemm256.h"
 #include "fmoe_vec.h"
 
 namespace fmoe {
@@ -33,9 +35,19 @@ __global__ __launch_bounds__(2 * WAVES_N * kWave) void gemm_turned_kernel(
     const T* __restrict__ A, int lda, const T* __restrict__ B0, const T* __restrict__ B1, int ldb, T* __restrict__ C, int M, int N, int K,
     int segments, int tiles_m, int tiles_n, int xcds, int slices) {
     const int tiles = tiles_m * tiles_n, block = (int)blockIdx.x;
-    gemm_dma_tiles<T, BM, BN, 2, WAVES_N, kStageK<T>, NSTAGE, SLICED ? kEpiPart : kEpiPlain, kSmallAhead<T>, kFragRows<T>, BM == 256 ? kBigSplit<T> : 1, true, SLICED,
+    gemm_dma_tiles<T, BM, BN, 2, WAVES_N, kStageK<T>, NSTAGE, SLICED ? kEpiPart : kEpiPlain, kSmallAhead<T>, kFragRows<T>, true, SLICED,
                    TA, true>(A, B0, B1, C, nullptr, M, N, K, tiles_m, tiles_n, xcds, SLICED ? block % tiles : block,
                              SLICED ? tiles : (int)gridDim.x, SLICED ? block / tiles : 0, slices, lda, ldb, segments);
+}
+
+template <typename T, bool TA, bool SLICED, bool RAGGED>
+__global__ __launch_bounds__(kWideThreads, 2) void gemm_wide_turned_kernel(
+    const T* __restrict__ A, int lda, const T* __restrict__ B0, const T* __restrict__ B1, int ldb, T* __restrict__ C, int M, int N, int K,
+    int segments, int tiles_m, int tiles_n, int xcds, int slices) {
+    const int tiles = tiles_m * tiles_n, block = (int)blockIdx.x;
+    gemm_wide_tiles<T, SLICED ? kEpiPart : kEpiPlain, RAGGED, SLICED, TA, true>(
+        A, B0, B1, C, nullptr, M, N, K, tiles_m, tiles_n, xcds, SLICED ? block % tiles : block, SLICED ? tiles : (int)gridDim.x,
+        SLICED ? block / tiles : 0, slices, lda, ldb, segments);
 }
 
 // C = sum over the slices, in order; one packet of C per thread
@@ -104,7 +116,11 @@ void launch_turned(const void* A, int lda, const void* B0, const void* B1, int l
                        0, stream, (const T*)A, lda, (const T*)B0, (const T*)B1, ldb, (T*)planes, M, N, K, segments, tm, tn, xcds, p.slices)
     if (p.slices > 1) {
         switch (p.shape) {
-            case kTile256: if constexpr (sizeof(T) == 2) FMOE_SLICED(256, 256, 4, 2); break;
+            case kTile256:
+                if constexpr (sizeof(T) == 2)
+                    hipLaunchKernelGGL((gemm_wide_turned_kernel<T, TA, true, true>), dim3((unsigned)(n * p.slices)), dim3(kWideThreads), 0, stream, (const T*)A,
+                                       lda, (const T*)B0, (const T*)B1, ldb, (T*)planes, M, N, K, segments, tm, tn, xcds, p.slices);
+                break;
             case kTile128: FMOE_SLICED(128, 128, 2, 4); break;
             case kTile64x128: if constexpr (sizeof(T) == 2) FMOE_SLICED(64, 128, 2, 4); break;
             default: FMOE_SLICED(64, 64, 2, 4); break;
@@ -115,7 +131,18 @@ void launch_turned(const void* A, int lda, const void* B0, const void* B1, int l
         return;
     }
     switch (p.shape) {
-        case kTile256: if constexpr (sizeof(T) == 2) FMOE_WHOLE(256, 256, 4, 2, 1); break;
+        case kTile256:
+            if constexpr (sizeof(T) == 2) {
+                const dim3 grid((unsigned)(n < cus ? n : cus));
+                const bool whole = M % kWide == 0 && N % kWide == 0 && K % kWideK == 0 && (K / kWideK * segments) % 2 == 0;
+#define FMOE_WIDE(RAGGED)                                                                                                               \
+    hipLaunchKernelGGL((gemm_wide_turned_kernel<T, TA, false, RAGGED>), grid, dim3(kWideThreads), 0, stream, (const T*)A, lda, (const T*)B0, \
+                       (const T*)B1, ldb, (T*)C, M, N, K, segments, tm, tn, xcds, 1)
+                if (whole) FMOE_WIDE(false);
+                else FMOE_WIDE(true);
+#undef FMOE_WIDE
+            }
+            break;
         case kTile128:
             if (n <= cus) FMOE_WHOLE(128, 128, 2, 4, 1);
             else FMOE_WHOLE(128, 128, 2, 2, 2);

@@ -8,7 +8,8 @@
 //      and up products never go to memory.
 //   2. down: plain epilogue, optional residual add (the routed-expert output in the block).
 //
-// Main kernel (gemm_dma_kernel; its tiles and those of gemm_splitk_kernel are in fmoe_gemm.h): tiles go global -> LDS
+// 256 x 256 tiles of the 16-bit types are gemm_wide_kernel's (fmoe_gemm256.h).  The other tiles (gemm_dma_kernel; they and those of
+// gemm_splitk_kernel are in fmoe_gemm.h) go global -> LDS
 // directly (global_load_lds_dwordx4, no staging registers) into NSTAGE LDS stages, issued NSTAGE-1 k-tiles
 // ahead of their use; one workgroup barrier per k-tile; MFMA fragments (v_mfma_f32_16x16x32 for the 16-bit types) are
 // read with 16-byte ds_reads.  An LDS row is one k-tile of one matrix row; its 16-byte chunks are XOR-swizzled with a key built
@@ -24,15 +25,16 @@
 // gemm_splitk_kernel; fp32 whose rows are no multiples of 16 bytes takes a plain FMA kernel.
 #include "fmoe_common.h"
 #include "fmoe_gemm.h"
+#include "fmoe_gemm256.h"
 
 namespace fmoe {
 namespace {
 
-template <typename T, int BM, int BN, int WAVES_M, int WAVES_N, int BKT, int NSTAGE, int EPI, int PF, int FR, int SPLIT, bool RAGGED>
+template <typename T, int BM, int BN, int WAVES_M, int WAVES_N, int BKT, int NSTAGE, int EPI, int PF, int FR, bool RAGGED>
 __global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void gemm_dma_kernel(
     const T* __restrict__ A, const T* __restrict__ B0, const T* __restrict__ B1, T* __restrict__ C,
     const T* __restrict__ R, int M, int N, int K, int tiles_m, int tiles_n, int xcds) {
-    gemm_dma_tiles<T, BM, BN, WAVES_M, WAVES_N, BKT, NSTAGE, EPI, PF, FR, SPLIT, RAGGED>(A, B0, B1, C, R, M, N, K, tiles_m, tiles_n, xcds,
+    gemm_dma_tiles<T, BM, BN, WAVES_M, WAVES_N, BKT, NSTAGE, EPI, PF, FR, RAGGED>(A, B0, B1, C, R, M, N, K, tiles_m, tiles_n, xcds,
                                                                                          (int)blockIdx.x, (int)gridDim.x);
 }
 
@@ -44,12 +46,26 @@ __global__ __launch_bounds__(kSplitWaves * 64) void gemm_splitk_kernel(
     gemm_splitk_tile<T, MT, NT, EPI>(A, B0, B1, C, R, M, N, K, tiles_m, tiles, xcds, (int)blockIdx.x, (int)gridDim.x, lds);
 }
 
+template <typename T, int EPI, bool RAGGED>
+__global__ __launch_bounds__(kWideThreads, 2) void gemm_wide_kernel(const T* __restrict__ A, const T* __restrict__ B0, const T* __restrict__ B1,
+                                                                 T* __restrict__ C, const T* __restrict__ R, int M, int N, int K,
+                                                                 int tiles_m, int tiles_n, int xcds) {
+    gemm_wide_tiles<T, EPI, RAGGED>(A, B0, B1, C, R, M, N, K, tiles_m, tiles_n, xcds, (int)blockIdx.x, (int)gridDim.x);
+}
+
+template <typename T>
+__global__ __launch_bounds__(kWideThreads, 2) void gemm_wide_sliced_kernel(const T* __restrict__ A, const T* __restrict__ B, float* __restrict__ planes, int M,
+                                                                        int N, int K, int tiles_m, int tiles_n, int xcds, int slices) {
+    const int tiles = tiles_m * tiles_n;
+    gemm_wide_tiles<T, kEpiPart, true, true>(A, B, nullptr, reinterpret_cast<T*>(planes), nullptr, M, N, K, tiles_m, tiles_n, xcds,
+                                             (int)blockIdx.x % tiles, tiles, (int)blockIdx.x / tiles, slices);
+}
+
 template <typename T, int BM, int BN, int WAVES_N, int NSTAGE>
 __global__ __launch_bounds__(2 * WAVES_N * 64) void gemm_sliced_kernel(const T* __restrict__ A, const T* __restrict__ B, float* __restrict__ planes, int M,
                                                           int N, int K, int tiles_m, int tiles_n, int xcds, int slices) {
     const int tiles = tiles_m * tiles_n;
-    gemm_dma_tiles<T, BM, BN, 2, WAVES_N, kStageK<T>, NSTAGE, kEpiPart, BM == 256 ? 1 : kSmallAhead<T>, kFragRows<T>,
-                   BM == 256 ? kBigSplit<T> : 1, true, true>(
+    gemm_dma_tiles<T, BM, BN, 2, WAVES_N, kStageK<T>, NSTAGE, kEpiPart, kSmallAhead<T>, kFragRows<T>, true, true>(
         A, B, nullptr, reinterpret_cast<T*>(planes), nullptr, M, N, K, tiles_m, tiles_n, xcds, (int)blockIdx.x % tiles, tiles,
         (int)blockIdx.x / tiles, slices);
 }
@@ -133,7 +149,7 @@ __global__ __launch_bounds__(256) void sgemm_nt_kernel(const float* __restrict__
         }
 }
 
-template <typename T, int BM, int BN, int WAVES_M, int WAVES_N, int BKT, int NSTAGE, int EPI, int PF, int FR = 32, int SPLIT = 1, bool RAGGED = false>
+template <typename T, int BM, int BN, int WAVES_M, int WAVES_N, int BKT, int NSTAGE, int EPI, int PF, int FR = 32, bool RAGGED = false>
 void launch_gemm_dma(const T* A, const T* B0, const T* B1, T* C, const T* R, int M, int N, int K, hipStream_t stream) {
     constexpr int BN_OUT = (EPI == kEpiSwiGLU) ? BN / 2 : BN;
     const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN_OUT - 1) / BN_OUT;      // without RAGGED only a ragged last row of tiles is allowed
@@ -144,8 +160,20 @@ void launch_gemm_dma(const T* A, const T* B0, const T* B1, T* C, const T* R, int
     const ChipInfo& chip = chip_info();
     const int resident = chip.cus * kPerCu;
     const int grid = total < resident ? total : resident;
-    hipLaunchKernelGGL((gemm_dma_kernel<T, BM, BN, WAVES_M, WAVES_N, BKT, NSTAGE, EPI, PF, FR, SPLIT, RAGGED>), dim3((unsigned)grid),
+    hipLaunchKernelGGL((gemm_dma_kernel<T, BM, BN, WAVES_M, WAVES_N, BKT, NSTAGE, EPI, PF, FR, RAGGED>), dim3((unsigned)grid),
                        dim3(WAVES_M * WAVES_N * 64), 0, stream, A, B0, B1, C, R, M, N, K, tiles_m, tiles_n, chip.xcds);
+}
+
+template <typename T, int EPI>
+void launch_gemm_wide(const T* A, const T* B0, const T* B1, T* C, const T* R, int M, int N, int K, hipStream_t stream) {
+    constexpr int BN_OUT = EPI == kEpiSwiGLU ? kWide / 2 : kWide;
+    const int tiles_m = (M + kWide - 1) / kWide, tiles_n = (N + BN_OUT - 1) / BN_OUT, total = tiles_m * tiles_n;
+    const ChipInfo& chip = chip_info();
+    const dim3 grid((unsigned)(total < chip.cus ? total : chip.cus));
+    if (M % kWide == 0 && N % BN_OUT == 0 && K % (2 * kWideK) == 0)
+        hipLaunchKernelGGL((gemm_wide_kernel<T, EPI, false>), grid, dim3(kWideThreads), 0, stream, A, B0, B1, C, R, M, N, K, tiles_m, tiles_n, chip.xcds);
+    else
+        hipLaunchKernelGGL((gemm_wide_kernel<T, EPI, true>), grid, dim3(kWideThreads), 0, stream, A, B0, B1, C, R, M, N, K, tiles_m, tiles_n, chip.xcds);
 }
 
 template <typename T, int MT, int NT, int EPI>
@@ -162,19 +190,27 @@ template <typename T, int EPI, bool RAGGED>
 void launch_tiles(const T* A, const T* B0, const T* B1, T* C, const T* R, int M, int N, int K, hipStream_t stream) {
     constexpr int KT = kStageK<T>, PF = kSmallAhead<T>, FR = kFragRows<T>;
     int tiles = 0;
-    switch (choose_tile<T, EPI>(M, N, tiles)) {
-        case kTile256: launch_gemm_dma<T, 256, 256, 2, 4, KT, 2, EPI, 1, FR, kBigSplit<T>, RAGGED>(A, B0, B1, C, R, M, N, K, stream); break;
+    TileShape shape = choose_tile<T, EPI>(M, N, tiles);
+    if (sizeof(T) == 2 && shape == kTile256 && !(aligned16(C) && aligned16(R))) {          // its results and residual move in 16-byte pieces
+        shape = kTile128;
+        tiles = ((M + 127) / 128) * ((N + kTileCols[kTile128] / (EPI == kEpiSwiGLU ? 2 : 1) - 1) / (kTileCols[kTile128] / (EPI == kEpiSwiGLU ? 2 : 1)));
+    }
+    switch (shape) {
+        case kTile256:
+            if constexpr (sizeof(T) == 2) launch_gemm_wide<T, EPI>(A, B0, B1, C, R, M, N, K, stream);
+            else launch_gemm_dma<T, 256, 256, 2, 4, KT, 2, EPI, 1, FR, RAGGED>(A, B0, B1, C, R, M, N, K, stream);
+            break;
         case kTile128:
-            if (tiles <= chip_info().cus) launch_gemm_dma<T, 128, 128, 2, 2, KT, 4, EPI, PF, FR, 1, RAGGED>(A, B0, B1, C, R, M, N, K, stream);
-            else launch_gemm_dma<T, 128, 128, 2, 2, KT, 2, EPI, PF, FR, 1, RAGGED>(A, B0, B1, C, R, M, N, K, stream);
+            if (tiles <= chip_info().cus) launch_gemm_dma<T, 128, 128, 2, 2, KT, 4, EPI, PF, FR, RAGGED>(A, B0, B1, C, R, M, N, K, stream);
+            else launch_gemm_dma<T, 128, 128, 2, 2, KT, 2, EPI, PF, FR, RAGGED>(A, B0, B1, C, R, M, N, K, stream);
             break;
         case kSplit32: launch_gemm_splitk<T, 2, 2, EPI>(A, B0, B1, C, R, M, N, K, stream); break;
         case kSplit16x32: launch_gemm_splitk<T, 1, 2, EPI>(A, B0, B1, C, R, M, N, K, stream); break;
         case kSplit16: launch_gemm_splitk<T, 1, 1, EPI>(A, B0, B1, C, R, M, N, K, stream); break;
-        case kTile64x128: launch_gemm_dma<T, 64, 128, 2, 2, KT, 4, EPI, PF, FR, 1, RAGGED>(A, B0, B1, C, R, M, N, K, stream); break;
+        case kTile64x128: launch_gemm_dma<T, 64, 128, 2, 2, KT, 4, EPI, PF, FR, RAGGED>(A, B0, B1, C, R, M, N, K, stream); break;
         default:
             if constexpr (EPI != kEpiSwiGLU || sizeof(T) == 2)
-                launch_gemm_dma<T, 64, 64, 2, 2, KT, 4, EPI, PF, FR, 1, RAGGED>(A, B0, B1, C, R, M, N, K, stream);
+                launch_gemm_dma<T, 64, 64, 2, 2, KT, 4, EPI, PF, FR, RAGGED>(A, B0, B1, C, R, M, N, K, stream);
     }
 }
 
@@ -205,7 +241,11 @@ void launch_sliced(const T* A, const T* B, T* C, const T* R, int M, int N, int K
     hipLaunchKernelGGL((gemm_sliced_kernel<T, BM, BN, WAVES_N, NSTAGE>), grid, dim3(128 * WAVES_N), 0, stream, A, B, planes, M, N, K, \
                        tiles_m, tiles_n, chip_info().xcds, p.slices)
     switch (p.shape) {
-        case kTile256: if constexpr (sizeof(T) == 2) FMOE_GO(256, 256, 4, 2); break;
+        case kTile256:
+            if constexpr (sizeof(T) == 2)
+                hipLaunchKernelGGL((gemm_wide_sliced_kernel<T>), grid, dim3(kWideThreads), 0, stream, A, B, planes, M, N, K, tiles_m, tiles_n, chip_info().xcds,
+                                   p.slices);
+            break;
         case kTile128: FMOE_GO(128, 128, 2, 4); break;
         case kTile64x128: FMOE_GO(64, 128, 2, 4); break;
         default: FMOE_GO(64, 64, 2, 4); break;

@@ -8,6 +8,7 @@
 #include "fmoe_common.h"
 #include "fmoe_gate.h"
 #include "fmoe_gemm.h"
+#include "fmoe_gemm256.h"
 #include "fmoe_select.h"
 
 namespace fmoe {
@@ -52,9 +53,11 @@ __device__ __forceinline__ void product_tiles(const T* A, const T* B0, const T* 
     using S = CutShape<CUT>;
     if constexpr (S::kDma) {
         if (threadIdx.x >= 2 * S::kWavesN * kWave) return;          // whole waves; the barriers of the tile count those that are left
-        gemm_dma_tiles<T, S::BM, S::BN, 2, S::kWavesN, kStageK<T>, S::kStages, EPI, CUT == kCut256 ? 1 : kSmallAhead<T>, kFragRows<T>,
-                       CUT == kCut256 ? kBigSplit<T> : 1, true>(
-            A, B0, B1, C, R, M, N, K, p.tiles_m, p.tiles_n, xcds, block, p.blocks);
+        if constexpr (CUT == kCut256 && sizeof(T) == 2 && EPI == kEpiSwiGLU)
+            gemm_wide_tiles<T, EPI, true>(A, B0, B1, C, R, M, N, K, p.tiles_m, p.tiles_n, xcds, block, p.blocks);
+        else
+            gemm_dma_tiles<T, S::BM, S::BN, 2, S::kWavesN, kStageK<T>, S::kStages, EPI, kSmallAhead<T>, kFragRows<T>, true>(
+                A, B0, B1, C, R, M, N, K, p.tiles_m, p.tiles_n, xcds, block, p.blocks);
     } else {
         gemm_splitk_tile<T, S::MT, S::MT, EPI>(A, B0, B1, C, R, M, N, K, p.tiles_m, p.tiles_m * p.tiles_n, xcds, block % p.blocks, p.blocks,
                                                lds, block / p.blocks, p.slices);

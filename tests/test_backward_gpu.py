@@ -635,6 +635,8 @@ def test_mlp_backward_remainders_of_the_transposing_products_fp32(T, H, I):
     (600, 3080, 6152),       # dW on 256 x 256 tiles
     (2500, 264, 5000),       # dh on 256 x 256 tiles; slices for the weight gradients
     (260, 3080, 13000),      # dx on 256 x 256 tiles in slices
+    (2048, 256, 8192), (512, 2048, 4096),      # nothing but whole 256 x 256 tiles: dh, dW
+    (4096, 4096, 192), (4096, 4096, 328),      # dx on 256 x 256 tiles, two ranges of k: three k-tiles each, and with a tail
 ])
 def test_mlp_backward_on_the_large_tiles_of_the_turned_products(dtype, T, H, I):
     test_mlp_backward_remainders_of_the_transposing_products(dtype, T, H, I)

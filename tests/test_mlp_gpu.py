@@ -184,3 +184,37 @@ def test_mlp_down_with_slices_of_k(dtype, T, H, I, with_residual):
 @pytest.mark.parametrize("T,H,I", [(300, 4104, 16392), (1000, 2056, 16392)])
 def test_mlp_down_with_slices_of_k_on_the_largest_tiles(T, H, I):
     test_mlp_down_with_slices_of_k(torch.bfloat16, T, H, I, True)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("T,N,K", [
+    (8200, 2056, 8), (8200, 2056, 64), (8200, 2056, 136),        # one, one and three k-tiles: the loop takes two at a time
+    (8192, 2048, 200), (8192, 2048, 256),                        # whole tiles with a k tail, and nothing but whole tiles
+    (8449, 2312, 72),                                            # a last row and a last column of tiles of one and eight
+])
+def test_mlp_on_the_widest_tiles(dtype, T, N, K):
+    """256 x 256 tiles: several to a workgroup, remainders in every extent, guard rows around every output, a residual large against
+    the sums; and tensors off the 16-byte grid, which smaller tiles take.  Bound: the sums are exact in fp32 up to K roundings of 2^-24,
+    so the one rounding to the type remains (2^-9 and 2^-12 relative), twice for the activation, which multiplies two of them."""
+    from flash_moe import _C
+
+    g = torch.Generator(device="cuda").manual_seed(T + N + K)
+    x, wg, wu = (torch.randn(*s, device="cuda", generator=g).to(dtype) for s in ((T, K), (N, K), (N, K)))
+    res = (100 * torch.randn(T, N, device="cuda", generator=g)).to(dtype)
+    L, code, stream = _C.lib(), _C.dtype_code(dtype), _C.current_stream(x.device)
+
+    def guarded(rows, shift=0):
+        buf = torch.full(((rows + 16) * N + 8,), 7.0, device="cuda", dtype=dtype)
+        return buf, buf[8 * N + shift:(8 + rows) * N + shift].view(rows, N)
+
+    tol = {torch.bfloat16: 2.0 ** -9, torch.float16: 2.0 ** -12}[dtype]
+    a, b = (torch.cat([x[i:i + 1024].double() @ w.double().t() for i in range(0, T, 1024)]) for w in (wg, wu))
+    for shift in (0, 1):
+        (abuf, act), (sbuf, saved), (obuf, out) = guarded(T), guarded(2 * T), guarded(T, shift)
+        _C.check(L.fmoe_mlp_gate_up_save(*map(_C.ptr, (x, wg, wu)), T, K, N, code, _C.ptr(act), _C.ptr(saved), stream), "gate/up")
+        _C.check(L.fmoe_mlp_down(_C.ptr(x), _C.ptr(wg), T, N, K, code, _C.ptr(res), _C.ptr(out), stream), "down")
+        for got, want, times in ((saved[:T], a, 1), (saved[T:], b, 1), (act, torch.nn.functional.silu(a) * b, 2), (out, a + res.double(), 1)):
+            off = (got.double() - want).abs()
+            assert off.norm() < times * tol * want.norm() and (off <= 2 * times * tol * want.abs() + 1e-5 * K).all()
+        for buf, rows, at in ((abuf, T, 0), (sbuf, 2 * T, 0), (obuf, T, shift)):
+            assert (buf[:8 * N + at] == 7).all() and (buf[(8 + rows) * N + at:] == 7).all()
