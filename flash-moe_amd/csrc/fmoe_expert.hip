@@ -718,98 +718,137 @@ __global__ __launch_bounds__(kOrderTokenWaves* kWave) void expert_order_kernel(c
     }
 }
 
-// NT tokens per wave, walked together: a step takes 64 / NT list positions of each (the same 16 gathers in flight as the slice
-// kernels), so that NT times as many tokens are at the same place of their lists.  256-byte slices.
-template <typename T, int NT>
-__global__ __launch_bounds__(256) void expert_scores_ordered_kernel(const T* __restrict__ x, const T* __restrict__ down, uint32_t table_bytes,
-                                                                    const uint32_t* __restrict__ off32, float* __restrict__ spart,
-                                                                    int64_t num_tokens, int hidden, int top_k, int num_slices,
-                                                                    int blocks_per_slice, int xcds) {
-    constexpr int V = Elem<T>::kVec, CL = 16, PPL = kWave / CL;
-    constexpr int QL = CL / NT, QP = QL * PPL;                   // loads and list positions per token and step
+// NT tokens per wave, walked together, a step taking U gathers of four rows: 4 U / NT list positions of each token.  256-byte
+// slices.  What bounds these kernels is the fabric: pieces of the window that left the L2 before the last token came by.  Left alone
+// the waves of a compute unit drift apart (the older ones are served first), 60 % of the lines of 1024 x 512 ids of 102400 missed where
+// 20 % do with all in step.  So the waves of a workgroup, as many as a compute unit holds, keep within two steps of each other; they
+// count steps in LDS, and a wave waits only while others are behind it, so the last one never does.  1024 x 512: 224 -> 196 us, 16384 x
+// 512 2831 -> 2284, 2048 x 800 of 160000 1339 -> 1130.  A step of 16 gathers is a wider window (391 for 389 us at 1024 x 1250, 392 for
+// 340 at 2048 x 512); keeping all workgroups of an XCD in step through counters in its L2 costs more than it saves (6 us each time,
+// under this load); 128-byte slices read lists and leave sums twice as often (250 us).
+constexpr int kOrderSlack = 2, kOrderMaxWaves = 16;
+struct Pace {
+    uint32_t* done;               // steps of all waves of the workgroup, zero before the first
+    uint32_t waves, step;
+    __device__ __forceinline__ void wait() const {
+        if (step < kOrderSlack) return;
+        const uint32_t want = (step - kOrderSlack + 1) * waves;
+        while (*(volatile const uint32_t*)done < want) __builtin_amdgcn_s_sleep(1);
+    }
+    __device__ __forceinline__ void tick() {
+        if (lane_id() == 0) atomicAdd(done, 1u);
+        ++step;
+    }
+};
+
+// Lane l of a wave: columns of the slice, row of a gather, and which token's list positions it fetches for a step.
+template <typename T, int NT, int U> struct OrderedWalk {
+    static constexpr int V = Elem<T>::kVec, CL = 16, PPL = kWave / CL;
+    static constexpr int QL = U / NT, QP = QL * PPL;             // gathers and list positions per token and step
+    static_assert(U % NT == 0 && U * PPL <= kWave, "every token has gathers of its own");
+    int c, pg, col, tokens, my_token, my_at;
+    bool col_ok;
+    uint32_t col_bytes;
+    int64_t t0;
+    __device__ __forceinline__ OrderedWalk(int slice, int tb, int64_t num_tokens, int hidden) {
+        const int lane = lane_id(), wave = (int)(threadIdx.x >> 6);
+        c = lane & (CL - 1);
+        pg = lane / CL;
+        col = slice * (CL * V) + c * V;
+        col_ok = col < hidden;
+        col_bytes = col_ok ? (uint32_t)col * sizeof(T) : 0u;
+        t0 = ((int64_t)tb * (blockDim.x / kWave) + wave) * NT;
+        tokens = (int)(num_tokens - t0 < NT ? (num_tokens > t0 ? num_tokens - t0 : 0) : NT);      // 0: the wave only keeps the pace
+        my_token = (lane / QP) % NT;
+        my_at = lane % QP;
+    }
+    __device__ __forceinline__ bool lists(int k, int top_k) const { return lane_id() < QP * NT && my_token < tokens && k + my_at < top_k; }
+    // the lane that fetched what gather u of this lane's row needs
+    __device__ __forceinline__ int source(int u) const { return (u / QL * QP + (u % QL) * PPL + pg) * 4; }
+};
+
+template <typename T, int NT, int U>
+__global__ __launch_bounds__(kOrderMaxWaves * kWave, 4) void expert_scores_ordered_kernel(
+    const T* __restrict__ x, const T* __restrict__ down, uint32_t table_bytes, const uint32_t* __restrict__ off32, float* __restrict__ spart,
+    int64_t num_tokens, int hidden, int top_k, int num_slices, int blocks_per_slice, int xcds) {
+    using Walk = OrderedWalk<T, NT, U>;
+    constexpr int QL = Walk::QL, QP = Walk::QP;
+    __shared__ uint32_t done;
     int slice, tb;
-    if (!slice_of_block(num_slices, blocks_per_slice, xcds, slice, tb)) return;
-    const int lane = lane_id(), wave = (int)(threadIdx.x >> 6);
-    const int c = lane & (CL - 1), pg = lane / CL;
-    const int col = slice * (CL * V) + c * V;
-    const bool col_ok = col < hidden;
-    const uint32_t col_bytes = col_ok ? (uint32_t)col * sizeof(T) : 0u;
-    const u32x4_t zero4 = {0u, 0u, 0u, 0u};
+    if (!slice_of_block(num_slices, blocks_per_slice, xcds, slice, tb)) return;      // the whole workgroup
+    if (threadIdx.x == 0) done = 0;
+    __syncthreads();
+    const Walk at(slice, tb, num_tokens, hidden);
     const __amdgpu_buffer_rsrc_t rsrc = table_resource(down, table_bytes);
-    const int64_t t0 = ((int64_t)tb * 4 + wave) * NT;
-    if (t0 >= num_tokens) return;                                // whole wave leaves; nobody waits on it
-    const int tokens = (int)(num_tokens - t0 < NT ? num_tokens - t0 : NT);
+    const u32x4_t zero4 = {0u, 0u, 0u, 0u};
     u32x4_t xq[NT];
 #pragma unroll
-    for (int n = 0; n < NT; ++n) xq[n] = col_ok && n < tokens ? *reinterpret_cast<const u32x4_t*>(x + (t0 + n) * hidden + col) : zero4;
-    const int my_token = lane / QP, my_at = lane % QP;           // the list position this lane fetches per step
-    const uint32_t* my_list = off32 + (t0 + my_token) * top_k;
-    float* out = spart + (int64_t)slice * num_tokens * top_k + t0 * top_k;
-    uint32_t mine = my_token < tokens && my_at < top_k ? my_list[my_at] : kBadOffset;
+    for (int n = 0; n < NT; ++n) xq[n] = at.col_ok && n < at.tokens ? *reinterpret_cast<const u32x4_t*>(x + (at.t0 + n) * hidden + at.col) : zero4;
+    const uint32_t* my_list = off32 + (at.t0 + at.my_token) * top_k + at.my_at;
+    float* out = spart + (int64_t)slice * num_tokens * top_k + at.t0 * top_k;
+    Pace pace{&done, blockDim.x / kWave, 0};
+    uint32_t mine = at.lists(0, top_k) ? my_list[0] : kBadOffset;
     for (int k0 = 0; k0 < top_k; k0 += QP) {
-        u32x4_t w[CL];
+        pace.wait();
+        u32x4_t w[U];
 #pragma unroll
-        for (int u = 0; u < CL; ++u) {
-            const uint32_t o = (uint32_t)__builtin_amdgcn_ds_bpermute((u / QL * QP + (u % QL) * PPL + pg) * 4, (int)mine);
-            w[u] = load_row_piece(rsrc, col_ok ? o + col_bytes : kBadOffset);          // as in the slice kernel
+        for (int u = 0; u < U; ++u) {
+            const uint32_t o = (uint32_t)__builtin_amdgcn_ds_bpermute(at.source(u), (int)mine);
+            w[u] = load_row_piece(rsrc, at.col_ok ? o + at.col_bytes : kBadOffset);          // as in the slice kernel
         }
-        const int next = k0 + QP + my_at;
-        mine = my_token < tokens && next < top_k ? my_list[next] : kBadOffset;
-        float part[CL];
+        mine = at.lists(k0 + QP, top_k) ? my_list[k0 + QP] : kBadOffset;
+        float part[U];
 #pragma unroll
-        for (int u = 0; u < CL; ++u) part[u] = dot16<T>(xq[u / QL], w[u], 0.0f);
-        const float total = transpose_sum<CL, 1>(part, c);          // load u = c: token c / QL, position (c % QL) * PPL + pg
-        const int kk = k0 + (c % QL) * PPL + pg;
-        if (c / QL < tokens && kk < top_k) out[(int64_t)(c / QL) * top_k + kk] = total;
+        for (int u = 0; u < U; ++u) part[u] = dot16<T>(xq[u / QL], w[u], 0.0f);
+        float total = transpose_sum<U, 1>(part, at.c);              // gather u = c % U: token u / QL, position (u % QL) * PPL + pg
+        if constexpr (U == 8) total += xor_step<U, 8>(total);
+        const int u = at.c & (U - 1), kk = k0 + (u % QL) * Walk::PPL + at.pg;
+        if (at.c < U && u / QL < at.tokens && kk < top_k) out[(int64_t)(u / QL) * top_k + kk] = total;
+        pace.tick();
     }
 }
 
-template <typename T, int NT>
-__global__ __launch_bounds__(256) void expert_states_ordered_kernel(const float* __restrict__ a, const T* __restrict__ up, uint32_t table_bytes,
-                                                                    const uint32_t* __restrict__ off32, T* __restrict__ out,
-                                                                    int64_t num_tokens, int hidden, int top_k, int num_slices,
-                                                                    int blocks_per_slice, int xcds) {
-    constexpr int V = Elem<T>::kVec, CL = 16, PPL = kWave / CL;
-    constexpr int QL = CL / NT, QP = QL * PPL;
+template <typename T, int NT, int U>
+__global__ __launch_bounds__(kOrderMaxWaves * kWave, 4) void expert_states_ordered_kernel(
+    const float* __restrict__ a, const T* __restrict__ up, uint32_t table_bytes, const uint32_t* __restrict__ off32, T* __restrict__ out,
+    int64_t num_tokens, int hidden, int top_k, int num_slices, int blocks_per_slice, int xcds) {
+    using Walk = OrderedWalk<T, NT, U>;
+    constexpr int QL = Walk::QL, QP = Walk::QP, V = Walk::V;
+    __shared__ uint32_t done;
     int slice, tb;
     if (!slice_of_block(num_slices, blocks_per_slice, xcds, slice, tb)) return;
-    const int lane = lane_id(), wave = (int)(threadIdx.x >> 6);
-    const int c = lane & (CL - 1), pg = lane / CL;
-    const int col = slice * (CL * V) + c * V;
-    const bool col_ok = col < hidden;
-    const uint32_t col_bytes = col_ok ? (uint32_t)col * sizeof(T) : 0u;
+    if (threadIdx.x == 0) done = 0;
+    __syncthreads();
+    const Walk at(slice, tb, num_tokens, hidden);
     const __amdgpu_buffer_rsrc_t rsrc = table_resource(up, table_bytes);
-    const int64_t t0 = ((int64_t)tb * 4 + wave) * NT;
-    if (t0 >= num_tokens) return;                                // whole wave leaves; nobody waits on it
-    const int tokens = (int)(num_tokens - t0 < NT ? num_tokens - t0 : NT);
     float acc[NT][V];
 #pragma unroll
     for (int n = 0; n < NT; ++n)
 #pragma unroll
         for (int v = 0; v < V; ++v) acc[n][v] = 0.0f;
-    const int my_token = lane / QP, my_at = lane % QP;
-    const uint32_t* my_list = off32 + (t0 + my_token) * top_k;
-    const float* my_coef = a + (t0 + my_token) * top_k;
-    bool live = my_token < tokens && my_at < top_k;
-    uint32_t mine = live ? my_list[my_at] : kBadOffset;
-    float mine_a = live ? my_coef[my_at] : 0.0f;
+    const uint32_t* my_list = off32 + (at.t0 + at.my_token) * top_k + at.my_at;
+    const float* my_coef = a + (at.t0 + at.my_token) * top_k + at.my_at;
+    Pace pace{&done, blockDim.x / kWave, 0};
+    bool live = at.lists(0, top_k);
+    uint32_t mine = live ? my_list[0] : kBadOffset;
+    float mine_a = live ? my_coef[0] : 0.0f;
     for (int k0 = 0; k0 < top_k; k0 += QP) {
-        u32x4_t w[CL];
-        float av[CL];
+        pace.wait();
+        u32x4_t w[U];
+        float av[U];
 #pragma unroll
-        for (int u = 0; u < CL; ++u) {
-            const int src = (u / QL * QP + (u % QL) * PPL + pg) * 4;
-            const uint32_t o = (uint32_t)__builtin_amdgcn_ds_bpermute(src, (int)mine);
-            av[u] = __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(src, __builtin_bit_cast(int, mine_a)));
-            w[u] = load_row_piece(rsrc, o + col_bytes);          // zeros for an invalid id (out of bounds)
+        for (int u = 0; u < U; ++u) {
+            const uint32_t o = (uint32_t)__builtin_amdgcn_ds_bpermute(at.source(u), (int)mine);
+            av[u] = __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(at.source(u), __builtin_bit_cast(int, mine_a)));
+            w[u] = load_row_piece(rsrc, o + at.col_bytes);          // zeros for an invalid id (out of bounds)
         }
-        const int next = k0 + QP + my_at;
-        live = my_token < tokens && next < top_k;
-        mine = live ? my_list[next] : kBadOffset;
-        mine_a = live ? my_coef[next] : 0.0f;
+        live = at.lists(k0 + QP, top_k);
+        mine = live ? my_list[k0 + QP] : kBadOffset;
+        mine_a = live ? my_coef[k0 + QP] : 0.0f;
         // fp32 coefficients, as in the row kernel: the loads, not these instructions, set the pace
 #pragma unroll
-        for (int u = 0; u < CL; ++u) axpy16<T>(av[u], w[u], acc[u / QL]);
+        for (int u = 0; u < U; ++u) axpy16<T>(av[u], w[u], acc[u / QL]);
+        pace.tick();
     }
 #pragma unroll
     for (int n = 0; n < NT; ++n) {
@@ -818,7 +857,7 @@ __global__ __launch_bounds__(256) void expert_states_ordered_kernel(const float*
             acc[n][v] += __shfl_xor(acc[n][v], 16, kWave);
             acc[n][v] += __shfl_xor(acc[n][v], 32, kWave);
         }
-        if (pg == 0 && col_ok && n < tokens) *reinterpret_cast<u32x4_t*>(out + (t0 + n) * hidden + col) = pack16<T>(acc[n]);
+        if (at.pg == 0 && at.col_ok && n < at.tokens) *reinterpret_cast<u32x4_t*>(out + (at.t0 + n) * hidden + at.col) = pack16<T>(acc[n]);
     }
 }
 
@@ -830,22 +869,32 @@ int launch_expert_order(const int64_t* indices, uint32_t* off32, uint16_t* place
     return FMOE_OK;
 }
 
-// Tokens per wave: until all of them are resident at once (about 20 waves per CU), at most eight.
-int ordered_tokens_per_wave(int64_t T_) {
-    const int64_t resident = (int64_t)chip_info().cus / chip_info().xcds * 20;
-    int nt = 1;
-    while (nt < 8 && T_ > resident * nt) nt *= 2;
-    return nt;
+// A compute unit holds twenty waves of these kernels, each with one, two or four tokens (eight spill registers).  Tokens per wave: as few
+// as have all tokens resident at once.  Workgroups: all of one size, one per unit, two where its share is more than sixteen waves; a
+// last generation of a few of them would take as long as a full one (2100 x 512 with 64 tokens to a workgroup, 33 for 32 units: 577 us,
+// with 36 tokens 379).  More tokens than are resident go in generations of one workgroup per unit: two of different generations on a
+// unit undo each other's window (16384 x 512, H = 512: 1382 us, 1122 so).  Few waves to a unit have sixteen gathers in flight, not
+// eight (128 x 2500 of 197136 169 for 204 us).
+struct OrderedShape { int tokens, waves; };
+OrderedShape ordered_shape(int64_t T_) {
+    const int64_t units = chip_info().cus / chip_info().xcds, resident = 20;
+    const int64_t share = (T_ + units - 1) / units;              // tokens per unit
+    const int nt = share > 2 * resident ? 4 : (share > resident ? 2 : 1);
+    const int64_t generations = share <= resident * nt ? 1 : (share + kOrderMaxWaves * nt - 1) / (kOrderMaxWaves * nt);
+    const int64_t waves = (share + generations * nt - 1) / (generations * nt);
+    return {nt, (int)(waves > kOrderMaxWaves ? (waves + 1) / 2 : waves)};
 }
+#define FMOE_LAUNCH_ORDERED_AS(KERNEL, NT, U, ...)                                                                            \
+    hipLaunchKernelGGL((KERNEL<T, NT, U>), grid, dim3((unsigned)(shape.waves * kWave)), 0, stream, __VA_ARGS__, T_, H, K, p.num_slices, blocks, p.xcds)
 #define FMOE_LAUNCH_ORDERED(KERNEL, ...)                                                                                      \
     do {                                                                                                                      \
-        const int nt = ordered_tokens_per_wave(T_);                                                                           \
-        const int blocks = (int)((T_ + 4 * nt - 1) / (4 * nt));                                                               \
+        const OrderedShape shape = ordered_shape(T_);                                                                         \
+        const int per = shape.waves * shape.tokens, blocks = (int)((T_ + per - 1) / per);                                     \
         const dim3 grid((unsigned)(p.xcds * slice_grid_rows(p.num_slices, blocks, p.xcds)));                                  \
-        if (nt == 1) hipLaunchKernelGGL((KERNEL<T, 1>), grid, dim3(256), 0, stream, __VA_ARGS__, T_, H, K, p.num_slices, blocks, p.xcds); \
-        else if (nt == 2) hipLaunchKernelGGL((KERNEL<T, 2>), grid, dim3(256), 0, stream, __VA_ARGS__, T_, H, K, p.num_slices, blocks, p.xcds); \
-        else if (nt == 4) hipLaunchKernelGGL((KERNEL<T, 4>), grid, dim3(256), 0, stream, __VA_ARGS__, T_, H, K, p.num_slices, blocks, p.xcds); \
-        else hipLaunchKernelGGL((KERNEL<T, 8>), grid, dim3(256), 0, stream, __VA_ARGS__, T_, H, K, p.num_slices, blocks, p.xcds); \
+        if (shape.tokens == 4) FMOE_LAUNCH_ORDERED_AS(KERNEL, 4, 8, __VA_ARGS__);                                             \
+        else if (shape.tokens == 2) FMOE_LAUNCH_ORDERED_AS(KERNEL, 2, 8, __VA_ARGS__);                                        \
+        else if (shape.waves > 6) FMOE_LAUNCH_ORDERED_AS(KERNEL, 1, 8, __VA_ARGS__);                                          \
+        else FMOE_LAUNCH_ORDERED_AS(KERNEL, 1, 16, __VA_ARGS__);                                                              \
     } while (0)
 
 template <typename T>
@@ -1401,7 +1450,7 @@ bool slices_chosen(int64_t T_, int H, int64_t E, int K, size_t elt) {
 // 10-25 % ahead of whole-row gathers; 8 pairs per expert, 15 % behind): below that the rows are better gathered whole, straight
 // from HBM.
 // Ordered slices pay when the slices of the table do not stay in L2 and 400 tokens name every expert about once or more, so that the
-// gathers in flight (400 to 5000 tokens of an XCD, ordered_tokens_per_wave) meet in a window of the slice.  Measured in bf16, ordered
+// gathers in flight (400 to 2500 tokens of an XCD, ordered_shape) meet in a window of the slice.  Measured in bf16, ordered
 // against the better of whole rows and buckets, us, ids uniform | ids a product-key router selects, whose lists keep less in step:
 //   H 1024, E 102400   1024 tokens x 256 139 for 150 | 145 for 148, x 512 223 for 291 | 252 for 291;  4096 x 256 406 for 573 | 529 for 578,
 //                      x 512 660 for 906 | 977 for 900;  16384 x 512 2807 for 3920 | 4205 for 3854

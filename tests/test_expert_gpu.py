@@ -308,7 +308,9 @@ def test_expert_on_router_produced_ids_at_the_block_size():
 @pytest.mark.parametrize("T,H,E,K", [
     (3, 8, 4, 1), (37, 72, 50, 5),                     # fewer list positions than a step takes; one partial slice
     (641, 136, 700, 33), (1281, 264, 300, 70),         # two and four tokens per wave, the last wave short of tokens
-    (2570, 64, 1000, 130),                             # eight tokens per wave
+    (2570, 64, 1000, 130),                             # generations of one workgroup per compute unit
+    (200, 72, 300, 8), (530, 8, 90, 31), (1000, 64, 300, 9), (2100, 136, 64, 17),      # seven waves; two workgroups per unit with one,
+    # two and four tokens per wave; lists shorter than a step and one position longer; waves without a token
     (70, 1000, 70000, 1100),                           # more positions than the ordering pass has lanes; the automatic choice
 ])
 def test_expert_ordered_lists(dtype, T, H, E, K):
