@@ -365,15 +365,18 @@ template <int N, int STEP> __device__ inline float transpose_sum(const float (&p
     }
 }
 
+// NT tokens of a wave share a step of 64 list positions, 64 / NT of each: lists much shorter than 64, or a little longer than a multiple,
+// would leave most of a step's gathers without a row (slice_tokens chooses).
 // IDS: the row offsets are not prepared yet: they are taken from the int64 ids (an id outside [0, num_experts) gives the
 // out-of-bounds offset) and the workgroups of slice 0 also store them to off32 for the launches that follow.
-template <typename T, int CL, bool IDS = false>
+template <typename T, int CL, int NT, bool IDS = false>
 __global__ __launch_bounds__(256) void expert_scores_slice_kernel(
     const T* __restrict__ x, const T* __restrict__ down, uint32_t table_bytes, const uint32_t* __restrict__ off32,
     float* __restrict__ spart, int64_t num_tokens, int hidden, int top_k, int num_slices, int blocks_per_slice,
     int tokens_per_block, int xcds, const int64_t* __restrict__ ids = nullptr, int64_t num_experts = 0) {
     constexpr int V = Elem<T>::kVec;
     constexpr int PPL = kWave / CL;                         // pairs per wave-wide load
+    constexpr int QL = CL / NT, QP = QL * PPL;              // loads and list positions per token and step
     int slice, tb;
     if (!slice_of_block(num_slices, blocks_per_slice, xcds, slice, tb)) return;
     const int lane = lane_id(), wave = (int)(threadIdx.x >> 6);
@@ -387,34 +390,38 @@ __global__ __launch_bounds__(256) void expert_scores_slice_kernel(
     const int64_t t_begin = (int64_t)tb * tokens_per_block;
     const int64_t t_end = t_begin + tokens_per_block < num_tokens ? t_begin + tokens_per_block : num_tokens;
     float* my_spart = spart + (int64_t)slice * pairs;
+    const int my_token = lane / QP, my_at = lane % QP;      // the list position this lane fetches per step
 
-    for (int64_t t = t_begin + wave; t < t_end; t += 4) {
-        const u32x4_t xq = col_ok ? *reinterpret_cast<const u32x4_t*>(x + t * hidden + col) : zero4;
-        const uint32_t* tok_off = off32 + t * top_k;
-        for (int k0 = 0; k0 < top_k; k0 += kWave) {
-            // one coalesced load brings the row offsets of 64 pairs; lane (pg, c) then needs those of pairs u*PPL+pg
+    for (int64_t t = t_begin + wave * NT; t < t_end; t += 4 * NT) {
+        const int tokens = (int)(t_end - t < NT ? t_end - t : NT);
+        u32x4_t xq[NT];
+#pragma unroll
+        for (int n = 0; n < NT; ++n) xq[n] = col_ok && n < tokens ? *reinterpret_cast<const u32x4_t*>(x + (t + n) * hidden + col) : zero4;
+        const int64_t list = (t + my_token) * top_k + my_at;
+        for (int k0 = 0; k0 < top_k; k0 += QP) {
+            // one coalesced load brings the row offsets of 64 pairs; lane (pg, c) then needs those of positions (u % QL) * PPL + pg
             uint32_t mine = kBadOffset;
-            if constexpr (IDS) {
-                if (k0 + lane < top_k) {
-                    const int64_t e = ids[t * top_k + k0 + lane];
+            if (my_token < tokens && k0 + my_at < top_k) {
+                if constexpr (IDS) {
+                    const int64_t e = ids[list + k0];
                     if (e >= 0 && e < num_experts) mine = (uint32_t)e * (uint32_t)(hidden * (int)sizeof(T));
-                    if (slice == 0) const_cast<uint32_t*>(tok_off)[k0 + lane] = mine;
+                    if (slice == 0) const_cast<uint32_t*>(off32)[list + k0] = mine;
+                } else {
+                    mine = off32[list + k0];
                 }
-            } else {
-                if (k0 + lane < top_k) mine = tok_off[k0 + lane];
             }
             u32x4_t w[CL];
 #pragma unroll
             for (int u = 0; u < CL; ++u) {
-                const uint32_t o = (uint32_t)__builtin_amdgcn_ds_bpermute((u * PPL + pg) * 4, (int)mine);
+                const uint32_t o = (uint32_t)__builtin_amdgcn_ds_bpermute((u / QL * QP + (u % QL) * PPL + pg) * 4, (int)mine);
                 w[u] = load_row_piece(rsrc, col_ok ? o + col_bytes : kBadOffset);      // zeros beyond the row: x is zero there, and so must w be
             }
             float part[CL];
 #pragma unroll
-            for (int u = 0; u < CL; ++u) part[u] = dot16<T>(xq, w[u], 0.0f);
-            const float total = transpose_sum<CL, 1>(part, c);      // pair k0 + c*PPL + pg
-            const int kk = k0 + c * PPL + pg;
-            if (kk < top_k) my_spart[t * top_k + kk] = total;
+            for (int u = 0; u < CL; ++u) part[u] = dot16<T>(xq[u / QL], w[u], 0.0f);
+            const float total = transpose_sum<CL, 1>(part, c);      // load u = c: token c / QL, position (c % QL) * PPL + pg
+            const int kk = k0 + (c % QL) * PPL + pg;
+            if (c / QL < tokens && kk < top_k) my_spart[(t + c / QL) * top_k + kk] = total;
         }
     }
 }
@@ -470,13 +477,15 @@ template <> __device__ inline void axpy16_coef<bf16_t>(float a, u32x4_t w, float
     }
 }
 
-template <typename T, int CL>
-__global__ __launch_bounds__(256) void expert_states_slice_kernel(
+template <typename T, int CL, int NT>
+__global__ __launch_bounds__(256, 4) void expert_states_slice_kernel(
     const float* __restrict__ a, const T* __restrict__ up, uint32_t table_bytes, const uint32_t* __restrict__ off32,
     T* __restrict__ out, int64_t num_tokens, int hidden, int top_k, int num_slices, int blocks_per_slice,
     int tokens_per_block, int xcds) {
     constexpr int V = Elem<T>::kVec;
     constexpr int PPL = kWave / CL;
+    constexpr int QL = CL / NT, QP = QL * PPL;
+    static_assert(QL % 2 == 0, "rows of one token meet in pairs");
     int slice, tb;
     if (!slice_of_block(num_slices, blocks_per_slice, xcds, slice, tb)) return;
     const int lane = lane_id(), wave = (int)(threadIdx.x >> 6);
@@ -487,45 +496,67 @@ __global__ __launch_bounds__(256) void expert_states_slice_kernel(
     const __amdgpu_buffer_rsrc_t rsrc = table_resource(up, table_bytes);
     const int64_t t_begin = (int64_t)tb * tokens_per_block;
     const int64_t t_end = t_begin + tokens_per_block < num_tokens ? t_begin + tokens_per_block : num_tokens;
+    const int my_token = lane / QP, my_at = lane % QP;
 
-    for (int64_t t = t_begin + wave; t < t_end; t += 4) {
-        const uint32_t* tok_off = off32 + t * top_k;
-        const float* tok_a = a + t * top_k;
-        float acc[V];
+    for (int64_t t = t_begin + wave * NT; t < t_end; t += 4 * NT) {
+        const int tokens = (int)(t_end - t < NT ? t_end - t : NT);
+        const int64_t list = (t + my_token) * top_k + my_at;
+        float acc[NT][V];
 #pragma unroll
-        for (int v = 0; v < V; ++v) acc[v] = 0.0f;
-        for (int k0 = 0; k0 < top_k; k0 += kWave) {
-            const bool live = k0 + lane < top_k;
-            const uint32_t mine = live ? tok_off[k0 + lane] : kBadOffset;
-            const float mine_a = live ? tok_a[k0 + lane] : 0.0f;
+        for (int n = 0; n < NT; ++n)
+#pragma unroll
+            for (int v = 0; v < V; ++v) acc[n][v] = 0.0f;
+        for (int k0 = 0; k0 < top_k; k0 += QP) {
+            const bool live = my_token < tokens && k0 + my_at < top_k;
+            const uint32_t mine = live ? off32[list + k0] : kBadOffset;
+            const float mine_a = live ? a[list + k0] : 0.0f;
             u32x4_t w[CL];
             float av[CL];
 #pragma unroll
             for (int u = 0; u < CL; ++u) {
-                const int src = (u * PPL + pg) * 4;
+                const int src = (u / QL * QP + (u % QL) * PPL + pg) * 4;
                 const uint32_t o = (uint32_t)__builtin_amdgcn_ds_bpermute(src, (int)mine);
                 av[u] = __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(src, __builtin_bit_cast(int, mine_a)));
                 w[u] = load_row_piece(rsrc, o + col_bytes);      // zeros for an invalid id (out of bounds)
             }
 #pragma unroll
-            for (int u = 0; u < CL; u += 2) axpy16_pair<T>(av[u], av[u + 1], w[u], w[u + 1], acc);
+            for (int u = 0; u < CL; u += 2) axpy16_pair<T>(av[u], av[u + 1], w[u], w[u + 1], acc[u / QL]);
         }
         // sum the pair groups (lanes c, c+CL, c+2*CL, ... hold the same columns)
 #pragma unroll
-        for (int v = 0; v < V; ++v) {
-            if constexpr (CL == 8) acc[v] += dpp_move<0x128>(acc[v]);             // lanes 8 apart
-            acc[v] += __shfl_xor(acc[v], 16, kWave);
-            acc[v] += __shfl_xor(acc[v], 32, kWave);
+        for (int n = 0; n < NT; ++n) {
+#pragma unroll
+            for (int v = 0; v < V; ++v) {
+                if constexpr (CL == 8) acc[n][v] += dpp_move<0x128>(acc[n][v]);             // lanes 8 apart
+                acc[n][v] += __shfl_xor(acc[n][v], 16, kWave);
+                acc[n][v] += __shfl_xor(acc[n][v], 32, kWave);
+            }
+            if (pg == 0 && col_ok && n < tokens) *reinterpret_cast<u32x4_t*>(out + (t + n) * hidden + col) = pack16<T>(acc[n]);
         }
-        if (pg == 0 && col_ok) *reinterpret_cast<u32x4_t*>(out + t * hidden + col) = pack16<T>(acc);
     }
 }
 
 struct SlicePlan {
-    int chunk_lanes, num_slices, blocks_per_slice, tokens_per_block, xcds;
+    int chunk_lanes, num_slices, tokens, blocks_per_slice, tokens_per_block, xcds;
     unsigned grid;
     size_t off_idx32, off_a, off_spart, off_place, bytes;
 };
+
+// Tokens that share a step of 64 list positions in the slice kernels: as many as save a fifth of the steps, while every compute
+// unit of an XCD has two workgroups.  us with one token to a step and so: 16384 tokens x 16 of 16384 experts 161 -> 88, x 32 171 -> 125; 4096
+// x 16 53 -> 33; 1024 x 32 24.5 -> 20.8; 256 x 1000, where nearly nothing is empty, would go from 63 to 188, and a tenth of the steps does
+// not pay (2274 x 267, training step 324 -> 335).
+int slice_tokens(int64_t T_, int K) {
+    int best = 1, best_steps = 4 * ((K + 63) / 64);
+    for (int nt = 2; nt <= 4 && T_ >= 256 * nt; nt *= 2) {
+        const int steps = 4 / nt * ((K + 64 / nt - 1) / (64 / nt));         // of four tokens
+        if (5 * steps <= 4 * best_steps) {
+            best = nt;
+            best_steps = steps;
+        }
+    }
+    return best;
+}
 
 // A slice is as wide as one XCD's 4 MiB L2 can keep resident: 256 bytes per row up to 16384 rows (fewer passes over
 // the offsets, coefficients and partial sums), 128 bytes beyond.
@@ -536,9 +567,11 @@ SlicePlan plan_slices(int64_t T_, int H, int64_t E, int K, size_t elt, bool orde
     p.chunk_lanes = ordered || E * 256 <= chip.l2_bytes ? 16 : 8;
     const size_t chunk_bytes = (size_t)p.chunk_lanes * 16;
     p.num_slices = (int)((H * elt + chunk_bytes - 1) / chunk_bytes);
-    const int64_t want = (T_ + 3) / 4;                       // at least one token per wave
-    p.blocks_per_slice = (int)(want < 1024 ? want : 1024);   // 256 blocks of 4 waves fill one XCD; a few rounds of them
-    p.tokens_per_block = (int)((T_ + p.blocks_per_slice - 1) / p.blocks_per_slice);
+    p.tokens = slice_tokens(T_, K);
+    const int per_step = 4 * p.tokens;                       // tokens of a workgroup's four waves
+    const int64_t want = (T_ + per_step - 1) / per_step, rounds = (want + 1023) / 1024;      // 256 blocks fill one XCD; a few rounds of them
+    p.blocks_per_slice = (int)((want + rounds - 1) / rounds);
+    p.tokens_per_block = (int)(rounds * per_step);
     p.grid = (unsigned)(p.xcds * slice_grid_rows(p.num_slices, p.blocks_per_slice, p.xcds));
     const size_t pairs = (size_t)T_ * (size_t)K;
     p.off_idx32 = 0;
@@ -554,23 +587,19 @@ template <typename T>
 int launch_slice_scores(const SlicePlan& p, const void* x, const void* table, const uint32_t* off32, float* spart, int64_t T_, int H,
                         int64_t E, int K, hipStream_t stream, const int64_t* ids = nullptr) {
     const uint32_t table_bytes = (uint32_t)(E * (int64_t)H * (int64_t)sizeof(T));
-    if (ids != nullptr) {
-        if (p.chunk_lanes == 16)
-            hipLaunchKernelGGL((expert_scores_slice_kernel<T, 16, true>), dim3(p.grid), dim3(256), 0, stream, (const T*)x,
-                               (const T*)table, table_bytes, off32, spart, T_, H, K, p.num_slices, p.blocks_per_slice,
-                               p.tokens_per_block, p.xcds, ids, E);
-        else
-            hipLaunchKernelGGL((expert_scores_slice_kernel<T, 8, true>), dim3(p.grid), dim3(256), 0, stream, (const T*)x,
-                               (const T*)table, table_bytes, off32, spart, T_, H, K, p.num_slices, p.blocks_per_slice,
-                               p.tokens_per_block, p.xcds, ids, E);
-    } else if (p.chunk_lanes == 16)
-        hipLaunchKernelGGL((expert_scores_slice_kernel<T, 16>), dim3(p.grid), dim3(256), 0, stream, (const T*)x,
-                           (const T*)table, table_bytes, off32, spart, T_, H, K, p.num_slices, p.blocks_per_slice,
-                           p.tokens_per_block, p.xcds, (const int64_t*)nullptr, (int64_t)0);
-    else
-        hipLaunchKernelGGL((expert_scores_slice_kernel<T, 8>), dim3(p.grid), dim3(256), 0, stream, (const T*)x,
-                           (const T*)table, table_bytes, off32, spart, T_, H, K, p.num_slices, p.blocks_per_slice,
-                           p.tokens_per_block, p.xcds, (const int64_t*)nullptr, (int64_t)0);
+#define FMOE_LAUNCH_SCORES(CL, NT, IDS)                                                                                           \
+    hipLaunchKernelGGL((expert_scores_slice_kernel<T, CL, NT, IDS>), dim3(p.grid), dim3(256), 0, stream, (const T*)x, (const T*)table, \
+                       table_bytes, off32, spart, T_, H, K, p.num_slices, p.blocks_per_slice, p.tokens_per_block, p.xcds, ids, E)
+#define FMOE_LAUNCH_SCORES_CL(CL)                                                                \
+    do {                                                                                         \
+        if (p.tokens == 4) { if (ids) FMOE_LAUNCH_SCORES(CL, 4, true); else FMOE_LAUNCH_SCORES(CL, 4, false); }      \
+        else if (p.tokens == 2) { if (ids) FMOE_LAUNCH_SCORES(CL, 2, true); else FMOE_LAUNCH_SCORES(CL, 2, false); } \
+        else { if (ids) FMOE_LAUNCH_SCORES(CL, 1, true); else FMOE_LAUNCH_SCORES(CL, 1, false); }                    \
+    } while (0)
+    if (p.chunk_lanes == 16) FMOE_LAUNCH_SCORES_CL(16);
+    else FMOE_LAUNCH_SCORES_CL(8);
+#undef FMOE_LAUNCH_SCORES
+#undef FMOE_LAUNCH_SCORES_CL
     FMOE_CHECK_LAUNCH("routed experts (slice scores)");
     return FMOE_OK;
 }
@@ -585,12 +614,19 @@ template <typename T>
 int launch_slice_states(const SlicePlan& p, const float* a, const void* table, const uint32_t* off32, void* out, int64_t T_, int H,
                         int64_t E, int K, hipStream_t stream) {
     const uint32_t table_bytes = (uint32_t)(E * (int64_t)H * (int64_t)sizeof(T));
-    if (p.chunk_lanes == 16)
-        hipLaunchKernelGGL((expert_states_slice_kernel<T, 16>), dim3(p.grid), dim3(256), 0, stream, a, (const T*)table,
-                           table_bytes, off32, (T*)out, T_, H, K, p.num_slices, p.blocks_per_slice, p.tokens_per_block, p.xcds);
-    else
-        hipLaunchKernelGGL((expert_states_slice_kernel<T, 8>), dim3(p.grid), dim3(256), 0, stream, a, (const T*)table,
-                           table_bytes, off32, (T*)out, T_, H, K, p.num_slices, p.blocks_per_slice, p.tokens_per_block, p.xcds);
+#define FMOE_LAUNCH_STATES(CL, NT)                                                                                              \
+    hipLaunchKernelGGL((expert_states_slice_kernel<T, CL, NT>), dim3(p.grid), dim3(256), 0, stream, a, (const T*)table, table_bytes, \
+                       off32, (T*)out, T_, H, K, p.num_slices, p.blocks_per_slice, p.tokens_per_block, p.xcds)
+#define FMOE_LAUNCH_STATES_CL(CL)                       \
+    do {                                                \
+        if (p.tokens == 4) FMOE_LAUNCH_STATES(CL, 4);   \
+        else if (p.tokens == 2) FMOE_LAUNCH_STATES(CL, 2); \
+        else FMOE_LAUNCH_STATES(CL, 1);                 \
+    } while (0)
+    if (p.chunk_lanes == 16) FMOE_LAUNCH_STATES_CL(16);
+    else FMOE_LAUNCH_STATES_CL(8);
+#undef FMOE_LAUNCH_STATES
+#undef FMOE_LAUNCH_STATES_CL
     FMOE_CHECK_LAUNCH("routed experts (slice states)");
     return FMOE_OK;
 }
@@ -874,10 +910,12 @@ int launch_expert_order(const int64_t* indices, uint32_t* off32, uint16_t* place
 // last generation of a few of them would take as long as a full one (2100 x 512 with 64 tokens to a workgroup, 33 for 32 units: 577 us,
 // with 36 tokens 379).  More tokens than are resident go in generations of one workgroup per unit: two of different generations on a
 // unit undo each other's window (16384 x 512, H = 512: 1382 us, 1122 so).  Few waves to a unit have sixteen gathers in flight, not
-// eight (128 x 2500 of 197136 169 for 204 us).
+// eight (128 x 2500 of 197136 169 for 204 us).  Where several XCDs share a slice (rows of fewer slices than XCDs) each has its part of the
+// tokens.
 struct OrderedShape { int tokens, waves; };
-OrderedShape ordered_shape(int64_t T_) {
-    const int64_t units = chip_info().cus / chip_info().xcds, resident = 20;
+OrderedShape ordered_shape(int64_t T_, int num_slices) {
+    const int xcds = chip_info().xcds;
+    const int64_t units = chip_info().cus / xcds * (num_slices < xcds ? slice_parts(num_slices, xcds) : 1), resident = 20;
     const int64_t share = (T_ + units - 1) / units;              // tokens per unit
     const int nt = share > 2 * resident ? 4 : (share > resident ? 2 : 1);
     const int64_t generations = share <= resident * nt ? 1 : (share + kOrderMaxWaves * nt - 1) / (kOrderMaxWaves * nt);
@@ -888,7 +926,7 @@ OrderedShape ordered_shape(int64_t T_) {
     hipLaunchKernelGGL((KERNEL<T, NT, U>), grid, dim3((unsigned)(shape.waves * kWave)), 0, stream, __VA_ARGS__, T_, H, K, p.num_slices, blocks, p.xcds)
 #define FMOE_LAUNCH_ORDERED(KERNEL, ...)                                                                                      \
     do {                                                                                                                      \
-        const OrderedShape shape = ordered_shape(T_);                                                                         \
+        const OrderedShape shape = ordered_shape(T_, p.num_slices);                                                                         \
         const int per = shape.waves * shape.tokens, blocks = (int)((T_ + per - 1) / per);                                     \
         const dim3 grid((unsigned)(p.xcds * slice_grid_rows(p.num_slices, blocks, p.xcds)));                                  \
         if (shape.tokens == 4) FMOE_LAUNCH_ORDERED_AS(KERNEL, 4, 8, __VA_ARGS__);                                             \

@@ -336,6 +336,29 @@ def test_expert_ordered_lists(dtype, T, H, E, K):
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("E", [300, 20000])                     # slices of 256 and of 128 bytes
+@pytest.mark.parametrize("T,H,K", [
+    (1027, 136, 5), (1024, 8, 16), (1100, 264, 17), (1029, 72, 48),      # four tokens share a step, one short of positions or a step more
+    (515, 136, 31), (1023, 64, 32), (700, 72, 81),                       # two
+    (511, 136, 32), (1500, 8, 63),                                       # one
+])
+def test_expert_slices_with_several_tokens_to_a_step(dtype, E, T, H, K):
+    from flash_moe import _C
+    from flash_moe.ops.hip.flash_expert import expert_forward
+
+    g = torch.Generator().manual_seed(T + K)
+    x, wd, wu = (torch.randn(n, H, generator=g).mul(s).to(dtype) for n, s in ((T, 1.0), (E, 0.05), (E, 0.05)))
+    idx = torch.randint(0, E, (T, K), generator=g)
+    gates = torch.softmax(torch.randn(T, K, generator=g), -1).to(dtype)
+    idx[0, 0], idx[T - 1, K - 1], idx[T // 2] = -1, E, -7            # ids outside the table; a token without an expert
+    got = expert_forward(*cuda(x, wd, wu, idx, gates), algo=_C.EXPERT_SLICES).cpu()
+    valid = (idx >= 0) & (idx < E)
+    tol = {torch.float32: 2e-6, torch.bfloat16: 5e-3, torch.float16: 6e-4}[dtype]      # as the other schedules' tests
+    assert rel_fro(got, truth64(x, wd, wu, idx.clamp(0, E - 1), gates * valid)) < tol
+    assert (got[T // 2] == 0).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("algo", ["ROWS", "SLICES", "ORDERED"])
 @pytest.mark.parametrize("T,H,E,K", [(70, 72, 300, 5), (40, 8, 20000, 33), (700, 200, 500, 20)])
 def test_expert_infinite_weights_and_a_partial_last_slice(dtype, algo, T, H, E, K):
