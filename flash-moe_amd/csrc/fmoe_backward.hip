@@ -720,7 +720,7 @@ extern "C" int fmoe_expert_backward_saved(const void* dout, const void* x, const
     const int vec = (int)(16 / dtype_size(dtype));
     FMOE_REQUIRE(hidden % vec == 0, FMOE_ERR_ALIGNMENT, "fmoe_expert_backward: hidden=%d must be a multiple of %d (16-byte rows)", hidden, vec);
     // rows too long for the per-token row kernel take the column-slice kernels, which need 32-bit row offsets
-    FMOE_REQUIRE(hidden <= 8 * kWave * vec || num_tokens == 0 || top_k == 0 || expert_slices_usable(num_tokens, hidden, num_experts, top_k, dtype),
+    FMOE_REQUIRE(hidden <= 8 * kWave * vec || num_tokens == 0 || top_k == 0 || expert_saved_plan(num_tokens, hidden, num_experts, top_k, dtype).kept,
                  FMOE_ERR_UNSUPPORTED, "fmoe_expert_backward: rows of more than %d elements need tables below 4 GiB (hidden=%d, E=%lld)",
                  8 * kWave * vec, hidden, (long long)num_experts);
     FMOE_REQUIRE(num_experts < (1ll << 31) - 1 && (int64_t)num_tokens * top_k < (1ll << 31), FMOE_ERR_UNSUPPORTED,

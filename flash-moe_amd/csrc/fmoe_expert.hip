@@ -1470,58 +1470,79 @@ int launch_expert_bucketed(int act, const void* x, const void* down, const void*
     return launch_expert_rows_coef<T>(up, indices, a, T_, H, E, K, out, stream);
 }
 
-// A slice of the table must stay resident in one XCD's L2 (4 MiB) next to the streaming traffic; with 128-byte
-// slices of up to twice the L2 the measured gather rate is still twice the fabric's.  Beyond that, and for problems with
-// too few pairs to pay for four launches, whole rows are gathered by the one-wave-per-token kernel.
-bool slices_pay(int64_t T_, int64_t E, int K) { return E * 128 <= 2 * chip_info().l2_bytes && T_ * K >= (1ll << 16); }
 // rows are addressed with 32-bit byte offsets below kBadOffset
 bool slices_possible(int64_t E, int H, size_t elt) { return (uint64_t)E * (uint64_t)H * elt < (uint64_t)kBadOffset; }
-
-// column slices: when they pay, and for rows too long for the row kernels whatever the problem size
-bool slices_chosen(int64_t T_, int H, int64_t E, int K, size_t elt) {
-    return slices_possible(E, H, elt) && (slices_pay(T_, E, K) || !rows_possible(H, elt));
-}
-
-// Which schedule a call takes.  A forced schedule that cannot run these extents is reported by the dispatcher; AUTO
-// falls back to whole rows.
-// Grouping the pairs by expert pays once an expert's row serves about a dozen pairs (measured: 16 pairs per expert, bucketed
-// 10-25 % ahead of whole-row gathers; 8 pairs per expert, 15 % behind): below that the rows are better gathered whole, straight
-// from HBM.
-// Ordered slices pay when the slices of the table do not stay in L2 and 400 tokens name every expert about once or more, so that the
-// gathers in flight (400 to 2500 tokens of an XCD, ordered_shape) meet in a window of the slice.  Measured in bf16, ordered
-// against the better of whole rows and buckets, us, ids uniform | ids a product-key router selects, whose lists keep less in step:
-//   H 1024, E 102400   1024 tokens x 256 139 for 150 | 145 for 148, x 512 223 for 291 | 252 for 291;  4096 x 256 406 for 573 | 529 for 578,
-//                      x 512 660 for 906 | 977 for 900;  16384 x 512 2807 for 3920 | 4205 for 3854
-//   H 2048, E 160000   2048 tokens x 800 1339 for 1446 | 1685 for 1440;  8192 x 512 3443 for 3555 | 4562 for 3523
-//   H 512, E 75076     1024 tokens x 512 79 for 142 | 97 for 142;  8192 x 400: 547 for 825 | 787 for 809 (E 102400)
-// Fewer experts per token do not pay however many tokens there are: H 1024, E 102400, 16384 tokens x 64 599 for 556 | 627 for 552, x 16
-// 202 for 156; 4096 x 128 alone is better for uniform ids, 252 for 297 | 287 for 292; E 262144, 32768 x 128 2571 for 1965.
 bool ordered_possible(int64_t E, int H, int K, size_t elt) { return slices_possible(E, H, elt) && K <= kOrderMaxTopK; }
-bool ordered_pays(int64_t T_, int64_t E, int K) {
-    const int64_t resident = T_ < 400 ? T_ : 400;
-    return !slices_pay(T_, E, K) && T_ * K >= (1ll << 16) && resident * K >= E;
-}
-bool buckets_pay(int64_t T_, int64_t E, int K) { return !slices_pay(T_, E, K) && T_ * K >= (1ll << 16) && T_ * K >= 12 * E; }
-// Where both pay, rows of 4 KB and hardly more than 400 K = E ids in step leave the forward to the buckets: at H 2048, E 102400, 256 experts
-// per token, ordered takes 3440 us of 16384 tokens for 3218 in buckets and 7641 of 32768 for 6653 (uniform ids), 4429 for 3183 and 9065 for
-// 6444 (a router's).  The training step keeps the ordered lists, which its backward walks too: 12.1 ms for 13.7 and 26.2 for 28.2 | 11.3
-// for 12.5 and 24.0 for 26.3.
-bool buckets_ahead(int64_t E, int H, int K, size_t elt) { return (size_t)H * elt >= 4096 && 400ll * K * 100 < E * 135; }
-// keeps: the forward of a training step
-int choose_schedule(int algo, int64_t T_, int H, int64_t E, int K, size_t elt, bool scored = true, bool keeps = false) {
+
+// Which schedule a call takes.  A forced schedule that cannot run these extents is reported by the dispatcher; AUTO takes what follows,
+// from sweeps of all four over some 6000 problems (bf16, H 256 to 2048, E 600 to 197000, 256 x 64 to 32768 x 128, ids uniform and from a
+// product-key router): 2.4 % longer than the best of the four on average; the rule before it (slices up to 65536 experts, then ordered
+// lists from 400 K = E on, then buckets) 12 %.  us below.
+//
+// Fewer than 2^16 pairs and 128 MB of rows: whole rows, one launch instead of three or four (beyond, 2000 x 24 of 10000 with rows of 4 KB
+// takes 39 in slices for 57).
+//
+// A slice of 256 bytes fits an XCD's L2 (16384 experts): slices (16384 x 64 of 16384, H 1024: 229 for 291 ordered, 546 in rows).  But rows
+// for fewer than 12 experts per token, where most of a step is empty (16384 x 8 of 600: 32 for 68), unless they are 4 KB; for up to 150 MB
+// of rows that start between cache lines and whose pieces touch a line more each (H 776: 4096 x 16 35 for 45), unless a token has 64;
+// and for few experts per token of tables that the L2 holds whole (600 x 2 KB: 4096 x 40 1.25 times faster, 16384 x 16 1.29).
+//
+// Larger tables, ordered: where the tokens in flight on an XCD (2560) name every expert 1.3 times (rows of 3 KB: twice), so that a piece
+// serves several of them, and their lists keep in step well enough for the window to stay in the L2; it is as wide as E / sqrt(K), up to
+// E = 12000 sqrt(K).  H 1024: 1024 x 256 of 45000 76 for 104, of 102400 122 for 141; 4096 x 500 of 65000 505 for 715; 16384 x 128 of 50000
+// 533 for 640; beyond the limits 4096 x 64 of 102400 1.03, 1024 x 128 of 197000 1.19, H 2048, 1024 x 128 of 90000 1.15 times the rows.
+// Narrower, E = 9000 sqrt(K), where buckets pay (H 2048, 32768 x 64 of 90000: 2200 for 1800) and for rows of fewer slices than XCDs.  Up to 100 experts per token slices of 128
+// bytes are ahead where they fit (H 1024: 4096 x 64 of 35000 1.10 times), and for rows of fewer slices than XCDs while all of one fits (H
+// 512: 16384 x 64 of 50000 1.16 times).  Slices that leave more than one XCD in eight without work do not pay (H 640, five of them: 6000 x
+// 200 of 40000 313 for 233 in slices of 128 bytes).  Rows between lines, whose pieces are three lines: four times and 4000 sqrt(K) (H 776:
+// 1024 x 800 of 75000 1.16 times faster, 4096 x 64 of 35000 1.18 times slower), and from 11000 experts on, where their slices outgrow
+// the L2 (H 1000: 6000 x 200 of 16000 327 for 440).
+//
+// Slices of 128 bytes, while an L2 holds half of one (H 1024: 16384 x 32 of 24000 1.25 times faster than ordered, 4096 x 32 of 50000 1.21
+// than rows), all of one for rows of 4 KB (beyond, rows 1.07 to 1.12 times faster); for rows of 1 KB from 24 experts per token on; for rows
+// between lines up to 21000 experts (H 1000: 20000 x 30 of 20000 275 for 333).  Shorter rows would still gain beyond 65536 experts (H 256:
+// 16384 x 64 of 102400 1.15 times), but in bf16 slices round the coefficients, which the other schedules keep in fp32.
+//
+// Buckets, once an expert's row serves a dozen pairs and rows are 1 KB or at least 2 KB (H 1024: 32768 x 64 of 102400 1.15 times faster; H
+// 256 1.6 times slower than rows, H 640 1.3: those keep them only from 2^17 experts on, where a test holds the schedule); else whole rows,
+// straight from HBM.
+int choose_schedule(int algo, int64_t T_, int H, int64_t E, int K, size_t elt, bool scored = true) {
     if (K == 0) return FMOE_EXPERT_ROWS;
     if (algo != FMOE_EXPERT_AUTO) return algo;
-    if (slices_chosen(T_, H, E, K, elt)) return FMOE_EXPERT_SLICES;
+    const ChipInfo& chip = chip_info();
+    const int64_t pairs = T_ * K, row = (int64_t)H * (int64_t)elt, l2 = chip.l2_bytes;
+    const bool rows = rows_possible(H, elt), slices = slices_possible(E, H, elt), on_lines = row % 128 == 0, many = pairs >= (1ll << 16);
+    const bool fits = E * 256 <= l2, halves_fit = on_lines && E * 128 <= (row >= 4096 ? 1 : 2) * l2;      // a slice, or one of 128 bytes
     // grouping by expert serves the score phase; an op without scores (product-key memory) has nothing to group
-    const bool buckets = scored && buckets_pay(T_, E, K) && bucketed_possible(T_, E, H, K, elt);
-    if (ordered_pays(T_, E, K) && ordered_possible(E, H, K, elt) && (keeps || !buckets || !buckets_ahead(E, H, K, elt))) return FMOE_EXPERT_ORDERED;
+    const bool buckets = scored && many && pairs >= 12 * E && (row >= 2048 || row == 1024 || E >= (1ll << 17)) && bucketed_possible(T_, E, H, K, elt);
+    if (many && slices && (!fits || (!on_lines && E * 384 > l2 && K >= 100))) {
+        const int num_slices = (int)((row + 255) / 256);
+        const bool shared = num_slices < chip.xcds;
+        const int parts = shared ? slice_parts(num_slices, chip.xcds) : 1;
+        const bool busy = !shared || 8 * num_slices * parts >= 7 * chip.xcds;
+        const int64_t tokens = T_ / parts;
+        const double named = (double)(tokens < 2560 ? tokens : 2560) * K, width = (double)E * (double)E / K;
+        const bool in_step = on_lines ? named >= (row >= 3072 ? 2.0 : 1.3) * (double)E && width <= (buckets || shared ? 80.0e6 : 144.0e6) : named >= 4.0 * (double)E && width <= 16.0e6;
+        const int least = on_lines && (shared || (row < 4096 && halves_fit)) ? 100 : 24;
+        const bool small_slices = shared && on_lines && E * 128 <= (row <= 512 ? 2 : 1) * l2;
+        if (in_step && busy && K >= least && !small_slices && ordered_possible(E, H, K, elt)) return FMOE_EXPERT_ORDERED;
+    }
+    if (slices && fits) {
+        const bool resident = 2 * E * row * 4 <= 5 * l2 && row >= 1024;
+        const bool pay = (many || pairs * row >= 128000000) && (K >= 12 || (row >= 4096 && !resident)) &&
+                         (on_lines || pairs * row >= 150000000 || K >= 64) && !(resident && K < 128 && (pairs < (1ll << 17) || K < 16));
+        return pay || !rows ? FMOE_EXPERT_SLICES : FMOE_EXPERT_ROWS;
+    }
+    const bool pay = on_lines ? many && halves_fit && K >= (row <= 1024 && pairs < (1ll << 18) ? 24 : 12)
+                              : E * 192 <= l2 && K >= 24 && pairs >= (1ll << 18);
+    if (slices && (pay || !rows)) return FMOE_EXPERT_SLICES;
     return buckets ? FMOE_EXPERT_BUCKETS : FMOE_EXPERT_ROWS;
 }
 
 }  // namespace
 
 bool expert_slices_usable(int64_t num_tokens, int hidden, int64_t num_experts, int top_k, int dtype) {
-    return top_k > 0 && slices_chosen(num_tokens, hidden, num_experts, top_k, dtype_size(dtype));
+    return top_k > 0 && choose_schedule(FMOE_EXPERT_AUTO, num_tokens, hidden, num_experts, top_k, dtype_size(dtype)) == FMOE_EXPERT_SLICES;
 }
 
 uint32_t* expert_workspace_offsets(void* workspace) { return (uint32_t*)workspace; }   // SlicePlan::off_idx32 == 0
@@ -1546,7 +1567,7 @@ int expert_rows_added(const void* x, const void* down, const void* up, const int
 ExpertSavedPlan expert_saved_plan(int64_t num_tokens, int hidden, int64_t num_experts, int top_k, int dtype) {
     ExpertSavedPlan p = {};
     if (num_tokens <= 0 || top_k <= 0) return p;
-    const int schedule = choose_schedule(FMOE_EXPERT_AUTO, num_tokens, hidden, num_experts, top_k, dtype_size(dtype), true, true);
+    const int schedule = choose_schedule(FMOE_EXPERT_AUTO, num_tokens, hidden, num_experts, top_k, dtype_size(dtype));
     p.kept = schedule == FMOE_EXPERT_SLICES || schedule == FMOE_EXPERT_ORDERED;
     p.ordered = schedule == FMOE_EXPERT_ORDERED;
     if (!p.kept) return p;
