@@ -246,6 +246,16 @@ __device__ inline float wave_sum(float v) {
     return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 63));
 }
 
+// The same sum over each half of the lanes, result in the lanes of the half.
+__device__ inline float half_wave_sum(float v) {
+    v = group8_sum(v);
+    v += dpp_move<0x140>(v);
+    v += dpp_move<0x142, 0xA, false>(v);
+    const int lower = __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 31);
+    const int upper = __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 63);
+    return __builtin_bit_cast(float, lane_id() < 32 ? lower : upper);
+}
+
 // Max over the 64 lanes, result in all lanes.
 __device__ inline float wave_max(float v) {
     v = fmaxf(v, dpp_move<0xB1>(v));

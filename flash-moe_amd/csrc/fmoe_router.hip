@@ -163,13 +163,13 @@ __global__ __launch_bounds__(kRouterWaves* kWave) __attribute__((amdgpu_waves_pe
 // OCC: waves per SIMD the register allocation must leave room for.  With more than four tokens per SIMD eight resident
 // waves (at most 64 registers, a few of them spilled for the larger lists) finish sooner than seven, whose eighth token
 // per SIMD would wait for a second round; with at most four tokens per SIMD the unconstrained allocation is faster.
-template <typename T, typename TG, int RK, int RH, int RC, bool FROM_LOGITS, int OCC, bool SMALL = false>
+template <typename T, typename TG, int RK, int RH, int RC, bool FROM_LOGITS, int OCC, bool SMALL, int TOK>
 __global__ __launch_bounds__(kRouterWaves* kWave, OCC) void router_select_kernel(
     const T* __restrict__ lp, int64_t num_tokens, int nk, int top_k, int num_cand, T* __restrict__ scores,
     int64_t* __restrict__ indices, TG* __restrict__ gates, int norm_topk_prob, uint32_t* __restrict__ row_offsets,
     uint32_t row_bytes, const CandidateTable table) {
-    __shared__ SelectLds<RK, RC, kRouterWaves, false> lds;
-    router_select_tokens<T, TG, RK, RH, RC, FROM_LOGITS, SMALL, kRouterWaves, false>(
+    __shared__ SelectLds<RK, RC, kRouterWaves, false, TOK> lds;
+    router_select_tokens<T, TG, RK, RH, RC, FROM_LOGITS, SMALL, kRouterWaves, false, TOK>(
         lp, num_tokens, nk, top_k, num_cand, scores, indices, gates, norm_topk_prob, row_offsets, row_bytes, table, lds, (int)blockIdx.x,
         (int)gridDim.x);
 }
@@ -446,9 +446,12 @@ template <typename T, typename TG, bool FROM_LOGITS>
 int launch_router(const void* lp, int64_t T_, int nk, int K, void* scores, int64_t* indices, void* gates,
                   int norm, uint32_t* row_offsets, uint32_t row_bytes, hipStream_t stream) {
     const int num_cand = count_candidates(K);
-    const int64_t blocks_needed = (T_ + kRouterWaves - 1) / kRouterWaves;
-    const int64_t max_blocks = (int64_t)chip_info().cus * 8;   // a few resident blocks per CU; the kernel loops over tokens
-    const dim3 grid((unsigned)(blocks_needed < max_blocks ? blocks_needed : max_blocks));
+    auto blocks_of = [&](int tokens_of_a_wave) {
+        const int64_t needed = (T_ + kRouterWaves * tokens_of_a_wave - 1) / (kRouterWaves * tokens_of_a_wave);
+        const int64_t most = (int64_t)chip_info().cus * 8;     // a few resident blocks per CU; the kernel loops over tokens
+        return needed < most ? needed : most;
+    };
+    const dim3 grid((unsigned)blocks_of(1));
     const dim3 block(kRouterWaves * kWave);
     if (K > kMaxTopK) {      // the workgroup-per-token kernels; their limits are checked by the callers
         const int64_t big_blocks = T_ < (int64_t)chip_info().cus * 2 ? T_ : (int64_t)chip_info().cus * 2;
@@ -466,39 +469,49 @@ int launch_router(const void* lp, int64_t T_, int nk, int K, void* scores, int64
     }
     // lists that fit the registers of a wave take the threshold selection
     const bool crowded = T_ > (int64_t)chip_info().cus * 4 * kRouterWaves;      // more than four tokens per SIMD
-#define FMOE_LAUNCH_SELECT_OCC(RK_, RH_, RC_, OCC_, SMALL_)                                                                   \
-    hipLaunchKernelGGL((router_select_kernel<T, TG, RK_, RH_, RC_, FROM_LOGITS, OCC_, SMALL_>), grid, block, 0, stream, (const T*)lp, \
-                       T_, nk, K, num_cand, (T*)scores, indices, (TG*)gates, norm, row_offsets, row_bytes, table)
+    const bool in_pairs = T_ >= (int64_t)chip_info().cus * 16 * kRouterWaves;     // sixteen or more
+#define FMOE_LAUNCH_SELECT_OCC(RK_, RH_, RC_, OCC_, SMALL_, TOK_)                                                             \
+    hipLaunchKernelGGL((router_select_kernel<T, TG, RK_, RH_, RC_, FROM_LOGITS, OCC_, SMALL_, TOK_>), dim3((unsigned)blocks_of(TOK_)), \
+                       block, 0, stream, (const T*)lp, T_, nk, K, num_cand, (T*)scores, indices, (TG*)gates, norm, row_offsets, row_bytes, table)
 // Many tokens: one key per lane lets the kernel run in the registers of eight waves per SIMD at no or little spilling (K = 16, nk =
-// 128, 32768 tokens: 36 us against 40 at five waves); the instances of two keys per lane would spill 25 to 59 registers (nk = 512,
-// K = 128: 165 us against 138 without the bound).  Few tokens are one latency chain, spills would lengthen it.
-#define FMOE_LAUNCH_SELECT(RK_, RH_, RC_, SMALL_)                              \
+// 128, 32768 tokens: 36 us against 40 at five waves when it was chosen); the instances of two keys per lane would spill 25 to 59
+// registers (nk = 512, K = 128: 165 us against 138 without the bound).  Few tokens are one latency chain, spills would lengthen it.
+// Two tokens to a wave save a third of the sorting once every wave has two (us, 128 keys, 16 experts: 32768 tokens 29.4 -> 28.0,
+// 16384 16.2 -> 15.6, but 12288 11.9 -> 12.9 and 8192 9.6 -> 10.5).
+#define FMOE_LAUNCH_SELECT(RK_, RH_, RC_)                                      \
     do {                                                                       \
-        if (crowded && RK_ == 1) FMOE_LAUNCH_SELECT_OCC(1, RH_, RC_, 8, SMALL_); \
-        else FMOE_LAUNCH_SELECT_OCC(RK_, RH_, RC_, 1, SMALL_);                 \
+        if (crowded && RK_ == 1) FMOE_LAUNCH_SELECT_OCC(1, RH_, RC_, 8, false, 1); \
+        else FMOE_LAUNCH_SELECT_OCC(RK_, RH_, RC_, 1, false, 1);               \
+    } while (0)
+#define FMOE_LAUNCH_SELECT_SMALL(RH_, RC_)                                     \
+    do {                                                                       \
+        if (in_pairs) FMOE_LAUNCH_SELECT_OCC(1, RH_, RC_, 8, true, 2);         \
+        else if (crowded) FMOE_LAUNCH_SELECT_OCC(1, RH_, RC_, 8, true, 1);     \
+        else FMOE_LAUNCH_SELECT_OCC(1, RH_, RC_, 1, true, 1);                  \
     } while (0)
     if (K <= 128 && nk <= 512) {
         CandidateTable table;
         candidate_table(K, table);
         if (K <= 32 && num_cand <= kWave) {          // up to 19 experts: the candidates are one key per lane
-            if (nk <= 128) FMOE_LAUNCH_SELECT(1, 2, 1, true);
-            else FMOE_LAUNCH_SELECT(1, 8, 1, true);
+            if (nk <= 128) FMOE_LAUNCH_SELECT_SMALL(2, 1);
+            else FMOE_LAUNCH_SELECT_SMALL(8, 1);
         } else if (K <= 32) {
-            if (nk <= 128) FMOE_LAUNCH_SELECT(1, 2, 2, true);
-            else FMOE_LAUNCH_SELECT(1, 8, 2, true);
+            if (nk <= 128) FMOE_LAUNCH_SELECT_SMALL(2, 2);
+            else FMOE_LAUNCH_SELECT_SMALL(8, 2);
         } else if (K <= 64) {
-            if (nk <= 128) FMOE_LAUNCH_SELECT(1, 2, 5, false);
-            else if (nk <= 256) FMOE_LAUNCH_SELECT(1, 4, 5, false);
-            else FMOE_LAUNCH_SELECT(1, 8, 5, false);
+            if (nk <= 128) FMOE_LAUNCH_SELECT(1, 2, 5);
+            else if (nk <= 256) FMOE_LAUNCH_SELECT(1, 4, 5);
+            else FMOE_LAUNCH_SELECT(1, 8, 5);
         } else {
-            if (nk <= 128) FMOE_LAUNCH_SELECT(2, 2, 11, false);
-            else FMOE_LAUNCH_SELECT(2, 8, 11, false);
+            if (nk <= 128) FMOE_LAUNCH_SELECT(2, 2, 11);
+            else FMOE_LAUNCH_SELECT(2, 8, 11);
         }
         FMOE_CHECK_LAUNCH("fmoe_router_topk");
         return FMOE_OK;
     }
 #undef FMOE_LAUNCH_SELECT_OCC
 #undef FMOE_LAUNCH_SELECT
+#undef FMOE_LAUNCH_SELECT_SMALL
 #define FMOE_LAUNCH_ROUTER(R)                                                                                      \
     hipLaunchKernelGGL((router_topk_kernel<T, TG, R, FROM_LOGITS>), grid, block, 0, stream, (const T*)lp, T_, nk, K, \
                        num_cand, (T*)scores, indices, (TG*)gates, norm, row_offsets, row_bytes)

@@ -22,19 +22,23 @@ __device__ inline uint64_t make_key(float score, uint32_t index) {
 __device__ inline float key_score(uint64_t k) { return order_value((uint32_t)(k >> 32)); }
 __device__ inline uint32_t key_index(uint64_t k) { return ~(uint32_t)(k & 0xffffffffu); }
 
-// Value of lane (lane ^ mask) for mask in {1,2,4,8,16,32}; `mask` must be a compile-time constant after inlining.
-// Distances 1, 2 and 8 are single DPP moves.  Distances 4, 16 and 32 would cost 2-4 vector instructions each on the
-// DPP / permlane path; the kernel is bound by vector-ALU issue, so they go through the LDS crossbar instead
+// Value of lane (lane ^ mask) for the masks of a sorting network, a power of two or one less than that; `mask` must be a compile-time
+// constant after inlining.  Distances 1, 2 and 8 and mirrors within a row are single DPP moves.  The others would cost 2-4 vector
+// instructions each on the DPP / permlane path; the kernel is bound by instruction issue, so they go through the LDS crossbar
 // (ds_swizzle / ds_bpermute: no LDS memory is touched, no vector-ALU slot is used, other waves cover the latency).
 __device__ inline uint32_t xor_lane_u32(uint32_t v, int mask, int lane) {
     const int iv = (int)v;
     switch (mask) {
         case 1: return (uint32_t)__builtin_amdgcn_update_dpp(0, iv, 0xB1, 0xF, 0xF, true);    // quad_perm [1,0,3,2]
         case 2: return (uint32_t)__builtin_amdgcn_update_dpp(0, iv, 0x4E, 0xF, 0xF, true);    // quad_perm [2,3,0,1]
+        case 3: return (uint32_t)__builtin_amdgcn_update_dpp(0, iv, 0x1B, 0xF, 0xF, true);    // quad_perm [3,2,1,0]
         case 4: return (uint32_t)__builtin_amdgcn_ds_swizzle(iv, (4 << 10) | 0x1F);          // bit mode: lane ^ 4
+        case 7: return (uint32_t)__builtin_amdgcn_update_dpp(0, iv, 0x141, 0xF, 0xF, true);   // row_half_mirror
         case 8: return (uint32_t)__builtin_amdgcn_update_dpp(0, iv, 0x128, 0xF, 0xF, true);   // row_ror:8
+        case 15: return (uint32_t)__builtin_amdgcn_update_dpp(0, iv, 0x140, 0xF, 0xF, true);  // row_mirror
         case 16: return (uint32_t)__builtin_amdgcn_ds_swizzle(iv, (16 << 10) | 0x1F);        // bit mode: lane ^ 16
-        default: return (uint32_t)__builtin_amdgcn_ds_bpermute((lane ^ 32) << 2, iv);
+        case 31: return (uint32_t)__builtin_amdgcn_ds_swizzle(iv, (31 << 10) | 0x1F);        // bit mode: lane ^ 31
+        default: return (uint32_t)__builtin_amdgcn_ds_bpermute((lane ^ mask) << 2, iv);
     }
 }
 __device__ inline uint64_t xor_lane_u64(uint64_t v, int mask, int lane) {
@@ -44,90 +48,66 @@ __device__ inline uint64_t xor_lane_u64(uint64_t v, int mask, int lane) {
 }
 
 // Position of a key in the wave-wide sequence: p = lane*RK + r.
-// One compare-exchange layer of a bitonic network: partner = p ^ J, blocks of size K alternate direction.
-// Which lanes keep the larger key is a function of the lane number alone, so it is a 64-bit compile-time constant per
-// (layer, register), handed to the selects as a lane mask (inverse ballot): no vector instruction and no live scalar
-// register per layer, where lane-number compares hoisted out of the token loop would be spilled.
-template <int RK> struct LaneMasks { uint64_t m[RK]; };
-template <int RK, int K, bool DESC> constexpr LaneMasks<RK> descending_block_lanes() {
-    LaneMasks<RK> out{};
-    for (int r = 0; r < RK; ++r)
-        for (int l = 0; l < kWave; ++l) out.m[r] |= (uint64_t)((((l * RK + r) & K) == 0) == DESC) << l;
-    return out;
+// One compare-exchange layer: a key and the one at p ^ X, X = J or (the first layer of a stage) 2J - 1, the mirror of its block.  The key
+// with bit J of its position clear keeps the larger one (DESC).  With the mirror every block of a stage runs in one direction, so
+// which lanes keep the larger key takes only six 64-bit constants over all layers; they stay in scalar registers and reach the selects
+// as a lane mask (inverse ballot).  With blocks of alternating direction each layer had a constant of its own: 15 layers of 32 lanes
+// took 45 scalar instructions for 15 now, and the scalar unit was the busiest of the kernel.
+constexpr uint64_t lanes_with_clear(int bit) {
+    uint64_t m = 0;
+    for (int l = 0; l < kWave; ++l) m |= (uint64_t)((l & bit) == 0) << l;
+    return m;
 }
-template <int RK, int K, int J, bool DESC> constexpr LaneMasks<RK> keep_max_lanes() {
-    LaneMasks<RK> out{};
-    for (int r = 0; r < RK; ++r)
-        for (int l = 0; l < kWave; ++l) {
-            const int p = l * RK + r;
-            const bool desc_block = (((p & K) == 0) == DESC), first = (p & J) == 0;
-            out.m[r] |= (uint64_t)(first == desc_block) << l;
-        }
-    return out;
-}
-
-template <int RK, bool DESC, int K, int J>
-__device__ inline void bitonic_layer(uint64_t (&v)[RK], int lane) {
-    if constexpr (J < RK) {
-        constexpr LaneMasks<RK> desc = descending_block_lanes<RK, K, DESC>();
+template <int RK, bool DESC, int J, int X>
+__device__ inline void exchange_layer(uint64_t (&v)[RK], int lane) {
+    if constexpr (X < RK) {
 #pragma unroll
         for (int r = 0; r < RK; ++r) {
             if ((r & J) == 0) {
-                const bool desc_block = __builtin_amdgcn_inverse_ballot_w64(desc.m[r]);
-                const uint64_t a = v[r], b = v[r | J];
-                const uint64_t hi = a > b ? a : b, lo = a > b ? b : a;
-                v[r] = desc_block ? hi : lo;
-                v[r | J] = desc_block ? lo : hi;
+                const uint64_t a = v[r], b = v[r ^ X];
+                const bool swap = DESC ? a < b : a > b;
+                v[r] = swap ? b : a;
+                v[r ^ X] = swap ? a : b;
             }
         }
     } else {
-        constexpr LaneMasks<RK> keep = keep_max_lanes<RK, K, J, DESC>();
+        constexpr uint64_t first = lanes_with_clear(J / RK);         // J is at least RK here
+        const bool keep_max = __builtin_amdgcn_inverse_ballot_w64(DESC ? first : ~first);
+        uint64_t w[RK];
 #pragma unroll
         for (int r = 0; r < RK; ++r) {
-            const uint64_t other = xor_lane_u64(v[r], J / RK, lane);
-            const bool keep_max = __builtin_amdgcn_inverse_ballot_w64(keep.m[r]);
+            const uint64_t other = xor_lane_u64(v[r ^ (X % RK)], X / RK, lane);
             // keep my key if it is the larger one and I keep the max, or the smaller one and I keep the min
-            v[r] = ((v[r] > other) == keep_max) ? v[r] : other;
+            w[r] = ((v[r] > other) == keep_max) ? v[r] : other;
         }
+#pragma unroll
+        for (int r = 0; r < RK; ++r) v[r] = w[r];
     }
 }
 
-// layers J, J/2, ..., 1 of the stage with block size K
-template <int RK, bool DESC, int K, int J>
-__device__ inline void bitonic_stage(uint64_t (&v)[RK], int lane) {
-    bitonic_layer<RK, DESC, K, J>(v, lane);
-    if constexpr (J > 1) bitonic_stage<RK, DESC, K, J / 2>(v, lane);
+// layers J, J/2, ..., 1: sorts blocks of 2J keys that hold a bitonic sequence each
+template <int RK, bool DESC, int J>
+__device__ inline void bitonic_layers(uint64_t (&v)[RK], int lane) {
+    exchange_layer<RK, DESC, J, J>(v, lane);
+    if constexpr (J > 1) bitonic_layers<RK, DESC, J / 2>(v, lane);
 }
-// stages K, 2K, ..., N
-template <int RK, bool DESC, int K>
-__device__ inline void bitonic_stages_from(uint64_t (&v)[RK], int lane) {
-    bitonic_stage<RK, DESC, K, K / 2>(v, lane);
-    if constexpr (K < RK * kWave) bitonic_stages_from<RK, DESC, 2 * K>(v, lane);
+// sorted blocks of K keys out of sorted blocks of K / 2, up to blocks of N
+template <int RK, bool DESC, int N, int K = 2>
+__device__ inline void sort_blocks(uint64_t (&v)[RK], int lane) {
+    exchange_layer<RK, DESC, K / 2, K - 1>(v, lane);
+    if constexpr (K > 2) bitonic_layers<RK, DESC, K / 4>(v, lane);
+    if constexpr (K < N) sort_blocks<RK, DESC, N, 2 * K>(v, lane);
 }
 
 template <int RK, bool DESC>
 __device__ inline void bitonic_sort(uint64_t (&v)[RK], int lane) {
-    bitonic_stages_from<RK, DESC, 2>(v, lane);
-}
-
-// One key per lane: every aligned block of N lanes sorted descending on its own (block size 0 in the last stage: all blocks alike).
-template <int N>
-__device__ inline void bitonic_sort_blocks(uint64_t& v, int lane) {
-    uint64_t a[1] = {v};
-    if constexpr (N >= 4) bitonic_stage<1, true, 2, 1>(a, lane);
-    if constexpr (N >= 8) bitonic_stage<1, true, 4, 2>(a, lane);
-    if constexpr (N >= 16) bitonic_stage<1, true, 8, 4>(a, lane);
-    if constexpr (N >= 32) bitonic_stage<1, true, 16, 8>(a, lane);
-    if constexpr (N >= 64) bitonic_stage<1, true, 32, 16>(a, lane);
-    bitonic_stage<1, true, 0, N / 2>(a, lane);
-    v = a[0];
+    sort_blocks<RK, DESC, RK * kWave>(v, lane);
 }
 
 // v holds a bitonic sequence of N keys; sort it descending.
 template <int RK>
 __device__ inline void bitonic_merge_desc(uint64_t (&v)[RK], int lane) {
-    constexpr int N = RK * kWave;
-    bitonic_stage<RK, true, N, N / 2>(v, lane);
+    bitonic_layers<RK, true, RK * kWave / 2>(v, lane);
 }
 
 // Key at position `pos` of the wave-wide sequence (wave-uniform `pos`).
@@ -153,21 +133,26 @@ __device__ inline uint64_t key_at(const uint64_t (&v)[RK], int pos) {
 // candidate sums tied at the cut the earlier candidate (lower rank in half 0) is taken: where the sorted keys show such a tie, or
 // more than CAP keys tie with the K-th, the keys above that score and then the equal ones in list order are taken again.
 // Up to 32 experts per token (SMALL) CAP is 32 and one sort orders both halves, 32 lanes each.
-// Bound by instruction issue, 4 to 8 tokens per SIMD: at 32768 tokens, 128 keys, 16 experts the kernel took 92 us with the exact
-// search and three 64-lane sorts, now 36; 128 tokens or fewer, 32 experts: 10.3 -> 7.1; 4096 tokens, 64 experts: 16 -> 12.5.
+// Bound by instruction issue, the scalar unit (searches, lane masks) hardly less than the vector units: 32768 tokens, 128 keys, 16
+// experts take 28 us (323 scalar and 294 vector instructions per token), 32 with a constant per layer of the sorts and the search on
+// the vector unit (332 and 472), 92 with the exact search and three 64-lane sorts; 64 experts 51 for 57.  128 tokens or fewer, 32
+// experts: 10.3 -> 7.1 with the threshold, 4096 tokens, 64 experts: 16 -> 12.5 and now 11.0.
 // ------------------------------------------------------------------------------------------------------------
 template <int CTRL> __device__ inline uint32_t dpp_max_step(uint32_t v) {      // lanes without a source read 0
     const uint32_t o = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xF, 0xF, true);
     return v > o ? v : o;
 }
-__device__ inline uint32_t wave_max_u32(uint32_t v) {
+// The largest a and the largest b of the wave: folded onto one half of the lanes each, then reduced together.
+__device__ inline void wave_max_two_u32(uint32_t& a, uint32_t& b) {
+    const auto folded = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+    uint32_t v = folded[0] > folded[1] ? folded[0] : folded[1];
     v = dpp_max_step<0xB1>(v);       // lane ^ 1
     v = dpp_max_step<0x4E>(v);       // lane ^ 2
     v = dpp_max_step<0x141>(v);      // mirrored in 8 lanes
     v = dpp_max_step<0x140>(v);      // mirrored in 16 lanes
-    v = dpp_max_step<0x142>(v);      // lane 15 of a row into the next row
-    v = dpp_max_step<0x143>(v);      // lane 31 into rows 2 and 3
-    return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
+    v = dpp_max_step<0x142>(v);      // lane 15 of a row into the next row: rows 1 and 3 hold the maxima
+    a = (uint32_t)__builtin_amdgcn_readlane((int)v, 31);
+    b = (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
 }
 // RK = registers whose 64 * RK entries cover at least k: their smallest score bounds the K-th largest from below (k entries are at
 // least that large), the largest score of the list bounds it from above, and tau shares the leading bits the two bounds
@@ -183,18 +168,21 @@ __device__ inline uint32_t selecting_score(const uint64_t (&key)[R], int k, int 
         hi = hi > s ? hi : s;
         if (r < RK) lo_inv = lo_inv > ~s ? lo_inv : ~s;        // max of the complements = complement of the min
     }
-    hi = wave_max_u32(hi);
-    const uint32_t lo = ~wave_max_u32(lo_inv);
+    wave_max_two_u32(hi, lo_inv);
+    const uint32_t lo = ~lo_inv;
     const int bits = 32 - __builtin_clz((hi ^ lo) | 1u);         // low bits in which the bounds may differ
     uint32_t tau = bits >= 32 ? 0u : (hi >> bits) << bits;
-    for (int bit = bits - 1; bit >= LOW; --bit) {
-        const uint32_t trial = tau | (1u << bit);
+    uint32_t step = 1u << (bits - 1);
+    while (step >= 1u << LOW) {
+        // on the scalar unit but for a compare per register, one branch per step
+        const uint32_t trial = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tau | step));
         int count = 0;
 #pragma unroll
         for (int r = 0; r < R; ++r)
             count += __builtin_popcountll(__builtin_amdgcn_ballot_w64((uint32_t)(key[r] >> 32) >= trial));
         tau = count >= k ? trial : tau;
-        if (count >= k && count <= cap) break;
+        step = (uint32_t)(count - k) <= (uint32_t)(cap - k) ? 0u : step >> 1;
+        asm("" : "+s"(step));                                    // one exit: the two conditions cost six instructions apart
     }
     if constexpr (LOW > 0) {                                     // make tau a score: the low bits of a negative one are ones
         if (!(tau >> 31)) tau |= (1u << LOW) - 1u;
@@ -247,7 +235,7 @@ __device__ inline void collect_top(const uint64_t (&key)[R], int n, int k, int c
     int base = 0;
 #pragma unroll
     for (int r = 0; r < R; ++r) {
-        if ((m[r] >> lane) & 1) slots[base + lanes_below(m[r])] = key[r];
+        if ((uint32_t)(key[r] >> 32) >= tau) slots[base + lanes_below(m[r])] = key[r];
         base += __builtin_popcountll(m[r]);
     }
     for (int p = base + lane; p < cap; p += kWave) slots[p] = 0ull;
@@ -259,7 +247,7 @@ __device__ inline void sort_slots(const uint64_t* slots, uint64_t (&best)[RK], i
 #pragma unroll
     for (int r = 0; r < RK; ++r) best[r] = slots[lane * RK + r];
     __builtin_amdgcn_wave_barrier();
-    if constexpr (SMALL) bitonic_sort_blocks<32>(best[0], lane);
+    if constexpr (SMALL) sort_blocks<RK, true, kWave / 2>(best, lane);
     else bitonic_sort<RK, true>(best, lane);
 }
 
@@ -278,8 +266,8 @@ inline int candidate_table(int top_k, CandidateTable& table) {
     return used;
 }
 
-template <int RK, int RC, int WAVES, bool PAIRED> struct SelectLds {
-    static constexpr int kTokens = PAIRED ? WAVES / 2 : WAVES;
+template <int RK, int RC, int WAVES, bool PAIRED, int TOK = 1> struct SelectLds {
+    static constexpr int kTokens = PAIRED ? WAVES / 2 : WAVES * TOK;
     uint64_t slot[WAVES][RK * kWave];
     float half_score[kTokens][2][RK * kWave];
     uint32_t half_index[kTokens][2][RK * kWave];
@@ -287,18 +275,19 @@ template <int RK, int RC, int WAVES, bool PAIRED> struct SelectLds {
 };
 
 // WAVES waves per workgroup, a token each; PAIRED: two waves per token (one launch round of few tokens), one per half, the first of
-// them going on with the candidates.
-template <typename T, typename TG, int RK, int RH, int RC, bool FROM_LOGITS, bool SMALL, int WAVES, bool PAIRED>
+// them going on with the candidates.  TOK = 2 (SMALL): two tokens per wave, whose candidates one sort orders, 32 lanes each.
+template <typename T, typename TG, int RK, int RH, int RC, bool FROM_LOGITS, bool SMALL, int WAVES, bool PAIRED, int TOK = 1>
 __device__ __forceinline__ void router_select_tokens(
     const T* __restrict__ lp, int64_t num_tokens, int nk, int top_k, int num_cand, T* __restrict__ scores,
     int64_t* __restrict__ indices, TG* __restrict__ gates, int norm_topk_prob, uint32_t* __restrict__ row_offsets,
-    uint32_t row_bytes, const CandidateTable& table, SelectLds<RK, RC, WAVES, PAIRED>& lds, int block, int blocks) {
+    uint32_t row_bytes, const CandidateTable& table, SelectLds<RK, RC, WAVES, PAIRED, TOK>& lds, int block, int blocks) {
     constexpr int KP = RK * kWave;
     constexpr int LOW = sizeof(T) == 4 ? 0 : __is_same(T, bf16_t) ? 16 : 13;      // fp32 bits below the type's mantissa
     constexpr int CAP = SMALL ? kWave / 2 : KP;
     static_assert(RC * kWave <= kSelectMaxCand, "candidate table");
     static_assert(!SMALL || RK == 1, "one key per lane");
-    constexpr int TOKENS = PAIRED ? WAVES / 2 : WAVES;
+    static_assert(TOK == 1 || (TOK == 2 && SMALL && !PAIRED), "32 lanes per token");
+    constexpr int TOKENS = SelectLds<RK, RC, WAVES, PAIRED, TOK>::kTokens;
     auto& cand = lds.cand;
     auto& half_score = lds.half_score;
     auto& half_index = lds.half_index;
@@ -308,100 +297,112 @@ __device__ __forceinline__ void router_select_tokens(
     __syncthreads();
     const int lane = lane_id();
     const int wave = (int)(threadIdx.x >> 6);
-    const int mine = PAIRED ? wave >> 1 : wave;          // the wave's token of the workgroup
+    const int mine = PAIRED ? wave >> 1 : wave * TOK;    // the wave's (first) token of the workgroup
     const int64_t tokens_total = (int64_t)blocks * TOKENS;
-    const int64_t rounds = PAIRED ? 1 : (num_tokens + tokens_total - 1) / tokens_total;
 
-    for (int64_t round = 0; round < rounds; ++round) {
-        const int64_t token = round * tokens_total + (int64_t)block * TOKENS + mine;
-        if (!PAIRED && token >= num_tokens) continue;    // nothing below synchronises across waves
+    // PAIRED: one round; else nothing below synchronises across waves
+    for (int64_t first = (int64_t)block * TOKENS + mine; PAIRED || first < num_tokens; first += tokens_total) {
+        const bool both = TOK == 2 && first + 1 < num_tokens;
 #pragma unroll
-        for (int h = PAIRED ? __builtin_amdgcn_readfirstlane(wave & 1) : 0; h < 2; ++h) {
-            if (PAIRED && token >= num_tokens) break;
-            const T* row = FROM_LOGITS ? lp + (token * 2 + h) * nk : lp + ((int64_t)h * num_tokens + token) * nk;
-            float v[RH];
+        for (int t = 0; t < TOK; ++t) {
+            const int64_t token = first + t;
+            if (t == 1 && !both) break;
 #pragma unroll
-            for (int r = 0; r < RH; ++r) {
-                const int p = r * kWave + lane;
-                v[r] = p < nk ? Elem<T>::to_f32(row[p]) : 0.0f;
-            }
-            float shift = 0.0f, lse = 0.0f;
-            if (FROM_LOGITS) {
-                float mx = -INFINITY;
+            for (int h = PAIRED ? __builtin_amdgcn_readfirstlane(wave & 1) : 0; h < 2; ++h) {
+                if (PAIRED && token >= num_tokens) break;
+                const T* row = FROM_LOGITS ? lp + (token * 2 + h) * nk : lp + ((int64_t)h * num_tokens + token) * nk;
+                float v[RH];
 #pragma unroll
-                for (int r = 0; r < RH; ++r)
-                    if (r * kWave + lane < nk) mx = fmaxf(mx, v[r]);
-                mx = wave_max(mx);
-                float se = 0.0f;
-#pragma unroll
-                for (int r = 0; r < RH; ++r)
-                    if (r * kWave + lane < nk) se += expf(v[r] - mx);
-                shift = mx;
-                lse = logf(wave_sum(se));
-            }
-            uint64_t key[RH];
-#pragma unroll
-            for (int r = 0; r < RH; ++r) {
-                const int p = r * kWave + lane;
-                key[r] = p < nk ? make_key(FROM_LOGITS ? (v[r] - shift) - lse : v[r], (uint32_t)p) : 0ull;
-            }
-            // the candidates look up ranks below top_k (entries past nk stay key 0)
-            collect_top<RH, RK, FROM_LOGITS ? 0 : LOW>(key, nk, top_k < nk ? top_k : nk, CAP, slot[wave] + (SMALL && !PAIRED ? h * CAP : 0), lane);
-            if (!SMALL || PAIRED || h == 1) {
-                uint64_t best[RK];
-                sort_slots<RK, SMALL>(slot[wave], best, lane);
-#pragma unroll
-                for (int r = 0; r < RK; ++r) {
-                    const int which = SMALL && !PAIRED ? lane / CAP : h, rank = SMALL && !PAIRED ? lane % CAP : lane * RK + r;
-                    half_score[mine][which][rank] = key_score(best[r]);
-                    half_index[mine][which][rank] = key_index(best[r]);
+                for (int r = 0; r < RH; ++r) {
+                    const int p = r * kWave + lane;
+                    v[r] = p < nk ? Elem<T>::to_f32(row[p]) : 0.0f;
                 }
+                float shift = 0.0f, lse = 0.0f;
+                if (FROM_LOGITS) {
+                    float mx = -INFINITY;
+#pragma unroll
+                    for (int r = 0; r < RH; ++r)
+                        if (r * kWave + lane < nk) mx = fmaxf(mx, v[r]);
+                    mx = wave_max(mx);
+                    float se = 0.0f;
+#pragma unroll
+                    for (int r = 0; r < RH; ++r)
+                        if (r * kWave + lane < nk) se += expf(v[r] - mx);
+                    shift = mx;
+                    lse = logf(wave_sum(se));
+                }
+                uint64_t key[RH];
+#pragma unroll
+                for (int r = 0; r < RH; ++r) {
+                    const int p = r * kWave + lane;
+                    key[r] = p < nk ? make_key(FROM_LOGITS ? (v[r] - shift) - lse : v[r], (uint32_t)p) : 0ull;
+                }
+                // the candidates look up ranks below top_k (entries past nk stay key 0)
+                collect_top<RH, RK, FROM_LOGITS ? 0 : LOW>(key, nk, top_k < nk ? top_k : nk, CAP, slot[wave] + (SMALL && !PAIRED ? h * CAP : 0), lane);
+                if (!SMALL || PAIRED || h == 1) {
+                    uint64_t best[RK];
+                    sort_slots<RK, SMALL>(slot[wave], best, lane);
+#pragma unroll
+                    for (int r = 0; r < RK; ++r) {
+                        const int which = SMALL && !PAIRED ? lane / CAP : h, rank = SMALL && !PAIRED ? lane % CAP : lane * RK + r;
+                        half_score[mine + t][which][rank] = key_score(best[r]);
+                        half_index[mine + t][which][rank] = key_index(best[r]);
+                    }
+                }
+                if (PAIRED) break;
             }
-            if (PAIRED) break;
         }
         if (PAIRED) {
             __syncthreads();
-            if ((wave & 1) != 0 || token >= num_tokens) return;
+            if ((wave & 1) != 0 || first >= num_tokens) return;
         }
         __builtin_amdgcn_wave_barrier();
-        uint64_t ckey[RC];
+        uint64_t ckey[TOK][RC];
+        if (SMALL && !both && lane >= CAP) slot[wave][lane] = 0ull;        // the sort's other block
 #pragma unroll
-        for (int r = 0; r < RC; ++r) {
-            const int c = r * kWave + lane;
-            ckey[r] = 0ull;
-            if (c < num_cand) {
-                const int ij = cand[c];
-                const int i = ij & 0xff, j = ij >> 8;
-                const float s = round_through<T>(half_score[mine][0][i] + half_score[mine][1][j]);
-                const uint32_t flat = half_index[mine][0][i] * (uint32_t)nk + half_index[mine][1][j];
-                ckey[r] = make_key(s, flat);
+        for (int t = 0; t < TOK; ++t) {
+            if (t == 1 && !both) break;
+#pragma unroll
+            for (int r = 0; r < RC; ++r) {
+                const int c = r * kWave + lane;
+                ckey[t][r] = 0ull;
+                if (c < num_cand) {
+                    const int ij = cand[c];
+                    const int i = ij & 0xff, j = ij >> 8;
+                    const float s = round_through<T>(half_score[mine + t][0][i] + half_score[mine + t][1][j]);
+                    const uint32_t flat = half_index[mine + t][0][i] * (uint32_t)nk + half_index[mine + t][1][j];
+                    ckey[t][r] = make_key(s, flat);
+                }
             }
+            collect_top<RC, RK, LOW>(ckey[t], num_cand, top_k, CAP, slot[wave] + t * CAP, lane);
         }
         uint64_t best[RK];
-        if (SMALL && lane >= CAP) slot[wave][lane] = 0ull;                 // the sort's other block
-        collect_top<RC, RK, LOW>(ckey, num_cand, top_k, CAP, slot[wave], lane);
         sort_slots<RK, SMALL>(slot[wave], best, lane);
-        {
+#pragma unroll
+        for (int t = 0; t < TOK; ++t) {
+            if (t == 1 && !both) break;
             // a tie across the cut: the first candidates in list order among the equal sums are the ones to keep
-            const uint32_t cut = (uint32_t)(key_at<RK>(best, top_k - 1) >> 32);
-            if (top_k < CAP && cut == (uint32_t)(key_at<RK>(best, top_k) >> 32)) {
-                collect_exactly<RC>(ckey, cut, top_k, CAP, slot[wave], lane);
+            const uint32_t cut = (uint32_t)(key_at<RK>(best, t * CAP + top_k - 1) >> 32);
+            if (top_k < CAP && cut == (uint32_t)(key_at<RK>(best, t * CAP + top_k) >> 32)) {
+                collect_exactly<RC>(ckey[t], cut, top_k, CAP, slot[wave] + t * CAP, lane);
                 sort_slots<RK, SMALL>(slot[wave], best, lane);
             }
         }
+        const int64_t token = TOK == 2 ? first + lane / CAP : first;
+        const int rank = TOK == 2 ? lane % CAP : lane * RK;
+        const int kept = TOK == 2 && lane >= CAP && !both ? 0 : top_k;
         float e[RK];
         float total = 0.0f;
 #pragma unroll
         for (int r = 0; r < RK; ++r) {
-            const int p = lane * RK + r;
-            e[r] = p < top_k ? expf(key_score(best[r])) : 0.0f;
+            e[r] = rank + r < kept ? expf(key_score(best[r])) : 0.0f;
             total += e[r];
         }
-        if (gates != nullptr && norm_topk_prob) total = wave_sum(total);
+        if (gates != nullptr && norm_topk_prob) total = TOK == 2 ? half_wave_sum(total) : wave_sum(total);
 #pragma unroll
         for (int r = 0; r < RK; ++r) {
-            const int p = lane * RK + r;
-            if (p < top_k) {
+            const int p = rank + r;
+            if (p < kept) {
                 const int64_t o = token * top_k + p;
                 scores[o] = Elem<T>::from_f32(key_score(best[r]));
                 indices[o] = (int64_t)key_index(best[r]);
@@ -409,6 +410,7 @@ __device__ __forceinline__ void router_select_tokens(
                 if (gates != nullptr) gates[o] = Elem<TG>::from_f32(norm_topk_prob ? e[r] / total : e[r]);
             }
         }
+        if (PAIRED) break;
     }
 }
 

@@ -17,7 +17,8 @@ def gen(seed):
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("T,nk,K", [(64, 32, 16), (300, 128, 64), (17, 512, 128), (5, 8, 1),
-                                    (6, 9000, 48)])    # more keys than one LDS row pair holds: rows built 4096 keys at a time
+                                    (6, 9000, 48),     # more keys than one LDS row pair holds: rows built 4096 keys at a time
+                                    (8193, 24, 11), (16390, 64, 16), (12301, 25, 5)])   # two, four and three tokens to a wave
 def test_router_backward(dtype, T, nk, K):
     from flash_moe.ops import flash_router_func
     from flash_moe.ops.hip.flash_router import router_topk_backward

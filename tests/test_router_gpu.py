@@ -98,6 +98,7 @@ def test_router_matches_exhaustive_scan_with_lowest_index_ties():
     # a choice of the selection each side of its edges: 19 | 20 and 32 | 33 experts, 128 | 129 and 256 | 257 keys, lists that fill
     # their slots exactly, and enough tokens for the eight-wave instances
     (60, 19, 19), (60, 128, 20), (4200, 128, 16), (60, 129, 32), (60, 32, 32), (60, 33, 33), (60, 256, 64), (4200, 257, 64), (60, 130, 65),
+    (16385, 40, 16), (16384, 300, 32),                          # two tokens to a wave
 ])
 @pytest.mark.parametrize("step", [0.0, 0.25, 8.0])
 def test_router_selection_is_exact_with_ties(dtype, T, nk, K, step):
@@ -150,6 +151,19 @@ def test_router_gates(norm):
     torch.testing.assert_close(g.cpu(), ref, rtol=1e-5, atol=1e-9)
     if norm:
         torch.testing.assert_close(g.sum(-1).cpu(), torch.ones(T), rtol=1e-5, atol=1e-5)
+
+
+@pytest.mark.parametrize("norm", [False, True])
+@pytest.mark.parametrize("nk,K", [(128, 16), (24, 1), (129, 32)])
+def test_router_gates_of_two_tokens_to_a_wave(norm, nk, K):
+    # a token's scores, experts and gates do not depend on how many others the call has (from 16384 tokens on a wave takes two)
+    from flash_moe.ops.hip.flash_router import router_topk_gates
+
+    lp = cuda(orc.make_router_inputs(16387, nk, seed=nk))
+    whole = router_topk_gates(lp, nk, K, with_gates=True, norm_topk_prob=norm)
+    for part in (slice(0, 101), slice(16300, 16387)):
+        for a, b in zip(whole, router_topk_gates(lp[:, part].contiguous(), nk, K, with_gates=True, norm_topk_prob=norm)):
+            assert torch.equal(a[part], b)
 
 
 def test_router_limits_of_the_large_top_k_kernel():
