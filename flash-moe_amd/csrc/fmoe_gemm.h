@@ -577,6 +577,8 @@ template <typename T> constexpr int kSmallAhead = sizeof(T) == 2 ? 1 : 3;
 // the busiest CU has tiles.  The rule picks the shape with the smallest rounds * time: 256 x 256 (8 waves, two per SIMD) once that
 // means fewer rounds, smaller ones so that every CU has a tile, whatever the extents.  (Pricing 256 x 256 at / 66 gave 1675 tokens
 // of 2904 -> 7744 seven rounds of 128 x 128, 227 us; two of 256 x 256 take 157.)
+// Its two groups of waves keep the pipes busier: BM * BN / 108 for the plain products (us: 22464 tokens, 3232 -> 808 147 -> 128; 15029
+// tokens, 3408 -> 1280 166 -> 147); gate/up products, of which half are short in k, gain and lose about alike and stay at / 95.
 // fp32 rows of 128 bytes hold half as many values for matrix pipes an eighth as fast: BM * BN / 15.  The k-splitting kernel
 // costs more per received row, and more so the more CUs receive at once (measured from 64 to 224 workgroups), but its tiles are
 // small enough for a few rows of A.
@@ -592,7 +594,8 @@ template <typename T, int EPI> double tile_cost(int i, int M, int N, int64_t& n)
     n = (int64_t)((M + kTileRows[i] - 1) / kTileRows[i]) * ((N + out_cols - 1) / out_cols);
     const double occupied = n < cus ? (double)n / cus : 1.0;
     const double received = (kTileRows[i] + cols) * (split_k ? 1.45 * (1.0 + occupied) : 1.0);
-    const double multiplied = kTileRows[i] * (double)cols / (sizeof(T) == 4 ? 15.0 : 95.0);
+    const double rate = sizeof(T) == 4 ? 15.0 : (i == kTile256 && EPI == kEpiPlain ? 108.0 : 95.0);
+    const double multiplied = kTileRows[i] * (double)cols / rate;
     return received > multiplied ? received : multiplied;
 }
 template <typename T, int EPI> TileShape choose_tile(int M, int N, int& tiles, double* cost_out = nullptr) {
@@ -631,8 +634,8 @@ template <typename T> SlicePlan plan_slices_of_k(int M, int N, int K) {
     double best_time = (split_k ? 0.8 : 0.9) * whole * k_tiles * kRow;
     // Two 128 x 128 tiles to a compute unit hide each other's latency, by how much depends on the extents in ways the price does not
     // see: of 53 down products that would otherwise be sliced (bf16) 38 would gain, up to a third (1692 tokens, 10576 -> 3968: 192 whole,
-    // 131 in two slices), and 15 lose, up to a seventh (4918 tokens, 3456 -> 864: 41 whole, 47).  0.65 keeps all of them whole.
-    if (shape == kTile128 && tiles > cus) best_time *= 0.65;
+    // 131 in two slices), and 15 lose, up to a seventh (4918 tokens, 3456 -> 864: 41 whole, 47).  0.65 keeps nearly all of them whole.
+    if (shape == kTile128 && tiles > cus) best_time *= sizeof(T) == 2 ? 0.85 : 0.65;
     if (sizeof(T) == 4 && K % 4 != 0) return best;
     for (int i = sizeof(T) == 2 ? kTile256 : kTile128; i <= kTile64; ++i) {
         int64_t n = 0;
@@ -640,7 +643,7 @@ template <typename T> SlicePlan plan_slices_of_k(int M, int N, int K) {
         for (int s = 2; s <= kMaxSlices && n * s <= cus && s * 4 <= k_tiles; ++s) {
             const int share = (k_tiles + s - 1) / s;
             if ((s - 1) * share >= k_tiles) continue;           // a slice would have no k-tile
-            const double time = round * share * kRow + launch + (i == kTile256 ? 7.0 : 0.0) + 8.0e-6 * s * (double)M * N / 6.0;
+            const double time = round * share * kRow + launch + (i == kTile256 ? 5.0 : 0.0) + 8.0e-6 * s * (double)M * N / 6.0;
             if (time < best_time) {
                 best = {i, s};
                 best_time = time;

@@ -70,13 +70,14 @@ __global__ __launch_bounds__(256) void gemm_turned_add_kernel(const float* __res
 }
 
 // Tile shape and slices of k by price (us): a round of tiles costs what the forward's rule says, 2.3 ns per received row and k-tile,
-// plus the stores of its tiles, which nothing hides on 256 x 256 (8.5 us; the smaller tiles overlap them with other workgroups); slices,
-// as long as they are one round, add a launch of 4 us and their planes, written and read at 6 TB/s.
+// plus the stores of its tiles, which nothing hides on 256 x 256 (7 us; the smaller tiles overlap them with other workgroups);
+// slices, as long as they are one round, add a launch of 5 us (fp32 4) and their planes, written and read at 6 TB/s.
 // fp32 tiles are bound by the matrix pipes, which two workgroups of a compute unit keep a tenth busier than one (a k-tile of 128 x 128
 // 2.0 us for 2.25), so slices of 64 x 64 tiles may be two rounds: dx of 1000 tokens, 1024 -> 4096 156 -> 138 in two slices.  64 x 128 has
 // the faults of both its neighbours there and is left out (dx of 2048 tokens 279 for 268 on 64 x 64).
-// The 8.5 us: dq of 32768 tokens, 256 -> 2048 in bf16 takes 66 on 256 x 256 tiles and 54 on 128 x 128; dWd of 384 tokens, 7520 -> 1880, 19
-// for 23.
+// These prices against 186 products timed in every shape and number of slices (bf16): 2.3 % over the best on average, 3.6 with the
+// 256 x 256 tiles at the rate of the forward's and their stores at 8.5; us: dh of 1819 tokens, 1792 -> 4776 52 -> 39, of 4681, 1136 -> 4544
+// 74 -> 58, dWd of 19470 tokens, 1704 -> 640 90 -> 60, dx of 1819 tokens, 4776 -> 1792 90 -> 75; the worst, 1536 x 3072 of 2760, 36 -> 45.
 template <typename T> SlicePlan plan_turned(int M, int N, int K, int segments) {
     const int cus = chip_info().cus, k_tiles = (K + kStageK<T> - 1) / kStageK<T> * segments;
     SlicePlan best = {kTile64, 1};
@@ -84,13 +85,13 @@ template <typename T> SlicePlan plan_turned(int M, int N, int K, int segments) {
     for (int i = sizeof(T) == 4 ? kTile128 : kTile256; i <= kTile64; ++i) {
         int64_t n = 0;
         if (sizeof(T) == 4 && i == kTile64x128) continue;
-        const double row = tile_cost<T, kEpiPlain>(i, M, N, n) * 2.3e-3, stores = i == kTile256 ? 8.5 : 1.0;
+        const double row = tile_cost<T, kEpiPlain>(i, M, N, n) * 2.3e-3, stores = i == kTile256 ? 7.0 : 1.0;
         const int64_t most = sizeof(T) == 4 && i == kTile64 ? 2 * cus : cus;
         for (int s = 1; s <= kMaxSlices && (s == 1 || (n * s <= most && 2 * s <= k_tiles)); ++s) {
             const int share = (k_tiles + s - 1) / s;
             if ((s - 1) * share >= k_tiles) continue;                 // a slice would have no k-tile
             const double shared = sizeof(T) == 4 && n * s > cus ? 0.9 : 1.0;
-            const double time = (double)((n * s + cus - 1) / cus) * (shared * row * share + stores) + (s > 1 ? 4.0 + 8.0e-6 * s * (double)M * N / 6.0 : 0.0);
+            const double time = (double)((n * s + cus - 1) / cus) * (shared * row * share + stores) + (s > 1 ? (sizeof(T) == 4 ? 4.0 : 5.0) + 8.0e-6 * s * (double)M * N / 6.0 : 0.0);
             if (best_time == 0.0 || time < best_time) {
                 best = {i, s};
                 best_time = time;
