@@ -358,7 +358,7 @@ __global__ __launch_bounds__((WAVES > 1 ? WAVES : kBwdWaves) * kWave) void exper
                 coef_up[p] = valid[u] ? act * gate[u] : 0.0f;
                 coef_down[p] = ds;
                 dgates[p] = Elem<T>::from_f32(valid[u] ? da[u] * act : 0.0f);
-                if (valid[u]) atomicAdd(&counts[expert[u]], 1);   // integer histogram: the result does not depend on order
+                if (counts != nullptr && valid[u]) atomicAdd(&counts[expert[u]], 1);   // integer histogram: no order to depend on
             }
         }
     }
@@ -417,7 +417,7 @@ __global__ __launch_bounds__(256) void expert_backward_gate_kernel(
     coef_down[p] = cd;
     if (place != nullptr) coef_list[at] = cd;
     dgates[p] = Elem<T>::from_f32(valid ? u * act : 0.0f);
-    if (valid) atomicAdd(&counts[indices[p]], 1);   // integer histogram: the result does not depend on order
+    if (counts != nullptr && valid) atomicAdd(&counts[indices[p]], 1);   // integer histogram: the result does not depend on order
 }
 
 // A wave takes `span` consecutive experts (lane l holds the end of the l-th one's segment) and a chunk of the columns (NCH * 1024 bytes):
@@ -513,8 +513,9 @@ __global__ __launch_bounds__(kBwdWaves* kWave) void expert_backward_weight_kerne
 
 struct ExpertBwdPlan {
     bool slices, ordered;      // slices: column slices of the tables, on ordered lists or not
+    bool partition;            // the pairs are grouped by expert in two partition passes, nothing is counted on the way
     int num_slices;
-    size_t off_coef_up, off_coef_down, off_pairs, off_counts, off_cursor, off_offsets, off_off32, off_place, off_coef_list, off_spart_s, off_spart_u, bytes;
+    size_t off_coef_up, off_coef_down, off_pairs, off_counts, off_offsets, off_off32, off_place, off_coef_list, off_spart_s, off_spart_u, bytes;
 };
 
 ExpertBwdPlan plan_expert_backward(int64_t T_, int H, int64_t E, int K, int dtype) {
@@ -525,8 +526,9 @@ ExpertBwdPlan plan_expert_backward(int64_t T_, int H, int64_t E, int K, int dtyp
     p.off_coef_up = take(pairs * 4);
     p.off_coef_down = take(pairs * 4);
     p.off_pairs = take(pairs * 4);
-    p.off_counts = take(bucket_workspace_bytes(E));     // per-expert counts, then the fill's cursors, and the scan state
-    p.off_cursor = p.off_counts;
+    p.partition = bucket_partition_pays((int64_t)pairs, E);
+    // the partition's, or per-expert counts, then the fill's cursors, and the scan state
+    p.off_counts = take(p.partition ? bucket_partition_workspace_bytes((int64_t)pairs, E) : bucket_workspace_bytes(E));
     p.off_offsets = take((size_t)(E + 1) * 4);
     const ExpertSavedPlan kept = expert_saved_plan(T_, H, E, K, dtype);
     p.slices = kept.kept;
@@ -555,12 +557,13 @@ int launch_expert_backward(const void* dout, const void* x, const void* down, co
     float* coef_down = (float*)(ws + p.off_coef_down);
     uint32_t* pairs_by_expert = (uint32_t*)(ws + p.off_pairs);
     void* bucket_ws = ws + p.off_counts;
-    int32_t* counts = bucket_counts(bucket_ws);
+    int32_t* counts = p.partition ? nullptr : bucket_counts(bucket_ws);
     int32_t* offsets = (int32_t*)(ws + p.off_offsets);
     const int64_t pairs = T_ * K;
     const int nch = (H / V + kWave - 1) / kWave;
     const dim3 block(kBwdWaves * kWave);
-    if (int rc = bucket_clear(bucket_ws, E, stream)) return rc;
+    if (!p.partition)
+        if (int rc = bucket_clear(bucket_ws, E, stream)) return rc;
     if (p.slices) {
         uint32_t* off32 = (uint32_t*)(ws + p.off_off32);
         uint16_t* place = p.ordered ? (uint16_t*)(ws + p.off_place) : nullptr;
@@ -607,9 +610,11 @@ int launch_expert_backward(const void* dout, const void* x, const void* down, co
         FMOE_CHECK_LAUNCH("fmoe_expert_backward(tokens)");
     }
 
-    // the per-token kernels above counted the pairs of every expert: offsets, segments, each in ascending pair index
-    if (int rc = bucket_scan_fill(indices, bucket_ws, pairs, E, K, offsets, (int32_t*)pairs_by_expert, nullptr, 1u, nullptr, 1u,
-                                  nullptr, 0, 1, stream))
+    // offsets and segments, each in ascending pair index; without the partition the kernels above counted the pairs of every expert
+    if (int rc = p.partition ? bucket_partition(indices, bucket_ws, pairs, E, K, offsets, (int32_t*)pairs_by_expert, nullptr, 1u,
+                                                nullptr, 1u, nullptr, 0, true, stream)
+                             : bucket_scan_fill(indices, bucket_ws, pairs, E, K, offsets, (int32_t*)pairs_by_expert, nullptr, 1u,
+                                                nullptr, 1u, nullptr, 0, 1, stream))
         return rc;
 
     // experts per wave: about a round of 64 pairs, as long as every SIMD keeps four waves

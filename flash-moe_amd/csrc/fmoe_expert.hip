@@ -1415,7 +1415,7 @@ int launch_expert_bucketed(int act, const void* x, const void* down, const void*
     }
     if (bucket_partition_pays(pairs, E)) {
         if (int rc = bucket_partition(indices, ws + p.off_part, pairs, E, K, offsets, sorted_pairs, tokoff, 1u, expoff, 1u, a, 24,
-                                      stream))
+                                      false, stream))
             return rc;
     } else {
         if (int rc = bucket_clear(ws + p.off_bucket, E, stream)) return rc;

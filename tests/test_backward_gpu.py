@@ -309,6 +309,35 @@ def test_expert_backward_c4_tables_fewer_tokens():
         assert fro < GRAD_FRO[dtype], f"{name}: relative Frobenius error {fro:.3e}"
 
 
+@pytest.mark.parametrize("E,ids", [(40000, "spread"), (300, "spread"), (3, "spread"), (5000, "warm"), (5000, "hot")])
+def test_expert_backward_groups_pairs_alike_in_both_ways(E, ids):
+    # 65536 pairs are grouped by two partition passes, 64512 with counters in memory; the last pair of every token names no expert, so
+    # both calls sum the same pairs and, each in ascending pair index, to the same bits.  Segments that a pair ranks itself in, that
+    # are sorted in LDS, that are sorted after a group too large for LDS was written (warm: ten experts of 6450 pairs), and one of
+    # half of all pairs (hot)
+    from flash_moe.ops import flash_expert_func
+
+    T, K, H = 1024, 64, 64
+    indices = torch.randint(0, E, (T, K), generator=gen(E))
+    if ids == "warm":
+        indices = torch.randint(0, 10, (T, K), generator=gen(E))
+    if ids == "hot":
+        indices[torch.rand(T, K, generator=gen(1)) < 0.5] = 7
+    indices[:, -1] = -1
+    x, dout = torch.randn(T, H, generator=gen(2)).cuda(), torch.randn(T, H, generator=gen(3)).cuda()
+    down, up = (torch.randn(E, H, generator=gen(4)) * 0.1).cuda(), (torch.randn(E, H, generator=gen(5)) * 0.1).cuda()
+    gates = torch.rand(T, K, generator=gen(6)).cuda()
+
+    def grads(keep):
+        ws = [down.clone().requires_grad_(True), up.clone().requires_grad_(True)]
+        flash_expert_func(x, *ws, indices[:, :keep].contiguous().cuda(), gates[:, :keep].contiguous()).backward(dout)
+        return ws[0].grad, ws[1].grad
+
+    for a, b in zip(grads(K), grads(K - 1)):
+        assert torch.equal(a, b)
+    assert float(grads(K)[0].abs().max()) > 0
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_expert_backward_column_slices(dtype):
     """Enough pairs (65536) for the column-slice schedule of the per-token part; some ids invalid, some doubled."""
