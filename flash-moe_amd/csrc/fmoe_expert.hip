@@ -542,15 +542,16 @@ struct SlicePlan {
     size_t off_idx32, off_a, off_spart, off_place, bytes;
 };
 
-// Tokens that share a step of 64 list positions in the slice kernels: as many as save a fifth of the steps, while every compute
-// unit of an XCD has two workgroups.  us with one token to a step and so: 16384 tokens x 16 of 16384 experts 161 -> 88, x 32 171 -> 125; 4096
-// x 16 53 -> 33; 1024 x 32 24.5 -> 20.8; 256 x 1000, where nearly nothing is empty, would go from 63 to 188, and a tenth of the steps does
-// not pay (2274 x 267, training step 324 -> 335).
-int slice_tokens(int64_t T_, int K) {
+// Tokens that share a step of 64 list positions in the slice kernels: as many as halve the steps, while every compute unit of an XCD
+// has two workgroups; two also where they save a quarter, on slices of 256 bytes (16 lanes) and enough tokens.  us with one token to a
+// step and so: 16384 tokens x 16 of 16384 experts 161 -> 88, x 32 171 -> 125; 4096 x 16 53 -> 33; 1024 x 32 24.5 -> 20.8; 4000 x 82 8 to 14 %
+// less on 256 bytes, 1100 x 82 up to 6 more, 4000 x 82 on 128 bytes up to 7 more.  Four tokens in three steps for four take 16 to 40 % more
+// (1100 x 40, 1024 columns of 16000 experts), 256 x 1000, where nearly nothing is empty, 188 for 63.
+int slice_tokens(int64_t T_, int K, int chunk_lanes) {
     int best = 1, best_steps = 4 * ((K + 63) / 64);
     for (int nt = 2; nt <= 4 && T_ >= 256 * nt; nt *= 2) {
         const int steps = 4 / nt * ((K + 64 / nt - 1) / (64 / nt));         // of four tokens
-        if (5 * steps <= 4 * best_steps) {
+        if (2 * steps <= best_steps || (nt == 2 && chunk_lanes == 16 && T_ >= 2048 && 4 * steps <= 3 * best_steps)) {
             best = nt;
             best_steps = steps;
         }
@@ -567,7 +568,7 @@ SlicePlan plan_slices(int64_t T_, int H, int64_t E, int K, size_t elt, bool orde
     p.chunk_lanes = ordered || E * 256 <= chip.l2_bytes ? 16 : 8;
     const size_t chunk_bytes = (size_t)p.chunk_lanes * 16;
     p.num_slices = (int)((H * elt + chunk_bytes - 1) / chunk_bytes);
-    p.tokens = slice_tokens(T_, K);
+    p.tokens = slice_tokens(T_, K, p.chunk_lanes);
     const int per_step = 4 * p.tokens;                       // tokens of a workgroup's four waves
     const int64_t want = (T_ + per_step - 1) / per_step, rounds = (want + 1023) / 1024;      // 256 blocks fill one XCD; a few rounds of them
     p.blocks_per_slice = (int)((want + rounds - 1) / rounds);

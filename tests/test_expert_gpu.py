@@ -338,9 +338,9 @@ def test_expert_ordered_lists(dtype, T, H, E, K):
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("E", [300, 20000])                     # slices of 256 and of 128 bytes
 @pytest.mark.parametrize("T,H,K", [
-    (1027, 136, 5), (1024, 8, 16), (1100, 264, 17), (1029, 72, 48),      # four tokens share a step, one short of positions or a step more
-    (515, 136, 31), (1023, 64, 32), (700, 72, 81),                       # two
-    (511, 136, 32), (1500, 8, 63),                                       # one
+    (1027, 136, 5), (1024, 8, 16), (1029, 72, 15),                       # four tokens share a step
+    (515, 136, 31), (1023, 64, 32), (1100, 264, 17), (2100, 72, 81),     # two; the last for a quarter of the steps
+    (511, 136, 32), (1029, 72, 48), (1500, 8, 63),                       # one
 ])
 def test_expert_slices_with_several_tokens_to_a_step(dtype, E, T, H, K):
     from flash_moe import _C
