@@ -12,9 +12,8 @@
 // No floating-point atomics on global memory: every output element is written once and sums run in a fixed order
 // (pairs of an expert in ascending pair index), so gradients are reproducible bit for bit.  The per-token part of the
 // expert backward is one wave per token with the token's rows of x and dout in registers (the layout of the forward
-// row kernel).  The per-expert part needs the pairs grouped by expert: the bucketing stage (fmoe_bucket.hip: integer
-// histogram taken by the per-token kernels, scan, fill, ordering pass) gives each expert one segment listing its pairs in
-// ascending pair index, and the wave that owns the expert walks it in that order.
+// row kernel).  The per-expert part needs the pairs grouped by expert: group_pairs (fmoe_bucket.hip) gives each expert one segment
+// listing its pairs in ascending pair index, and the wave that owns the expert walks it in that order.
 #include "fmoe_common.h"
 #include "fmoe_vec.h"
 
@@ -272,7 +271,7 @@ template <typename T, int NCH, int WAVES>
 __global__ __launch_bounds__((WAVES > 1 ? WAVES : kBwdWaves) * kWave) void expert_backward_token_kernel(
     const T* __restrict__ dout, const T* __restrict__ x, const T* __restrict__ down, const T* __restrict__ up,
     const int64_t* __restrict__ indices, const T* __restrict__ gates, T* __restrict__ dx, T* __restrict__ dgates,
-    float* __restrict__ coef_up, float* __restrict__ coef_down, int32_t* __restrict__ counts, int64_t num_tokens,
+    float* __restrict__ coef_up, float* __restrict__ coef_down, int64_t num_tokens,
     int hidden, int64_t num_experts, int top_k) {
     constexpr int V = Elem<T>::kVec;
     constexpr int PIF = NCH >= 8 ? 1 : (NCH >= 4 ? 2 : 4);   // (down, up) row pairs requested ahead
@@ -304,7 +303,6 @@ __global__ __launch_bounds__((WAVES > 1 ? WAVES : kBwdWaves) * kWave) void exper
         u32x4_t dn[PIF][NCH], uq[PIF][NCH];
         float gate[PIF];
         bool valid[PIF];
-        int64_t expert[PIF];
 #pragma unroll
         for (int u = 0; u < PIF; ++u) {
             const int k = k0 + u;
@@ -318,7 +316,6 @@ __global__ __launch_bounds__((WAVES > 1 ? WAVES : kBwdWaves) * kWave) void exper
             const uint32_t ehi = __builtin_amdgcn_readfirstlane((uint32_t)((uint64_t)e >> 32));
             e = (int64_t)(((uint64_t)ehi << 32) | elo);
             valid[u] = e >= 0 && e < num_experts;
-            expert[u] = e;
             const u32x4_t* drow = reinterpret_cast<const u32x4_t*>(down + (valid[u] ? e : 0) * hidden);
             const u32x4_t* urow = reinterpret_cast<const u32x4_t*>(up + (valid[u] ? e : 0) * hidden);
 #pragma unroll
@@ -358,7 +355,6 @@ __global__ __launch_bounds__((WAVES > 1 ? WAVES : kBwdWaves) * kWave) void exper
                 coef_up[p] = valid[u] ? act * gate[u] : 0.0f;
                 coef_down[p] = ds;
                 dgates[p] = Elem<T>::from_f32(valid[u] ? da[u] * act : 0.0f);
-                if (counts != nullptr && valid[u]) atomicAdd(&counts[expert[u]], 1);   // integer histogram: no order to depend on
             }
         }
     }
@@ -391,14 +387,14 @@ __global__ __launch_bounds__((WAVES > 1 ? WAVES : kBwdWaves) * kWave) void exper
 
 // Column-slice schedule of the per-token part (same kernels as the forward, fmoe_expert.hip): the partial dot products
 // s = <x, down[e]> and u = <dout, up[e]> come per slice; this kernel sums them (or takes the scores the forward kept) and forms
-// every pair's coefficients, gate gradient and histogram entry; dx is then the forward's `states` pass over `down` with coef_down.
+// every pair's coefficients and gate gradient; dx is then the forward's `states` pass over `down` with coef_down.
 // place: NULL, or the (token, k) position of every list position: the states pass then needs coef_down in list order as well.
 template <typename T>
 __global__ __launch_bounds__(256) void expert_backward_gate_kernel(
     const float* __restrict__ spart_s, const float* __restrict__ scores, const float* __restrict__ spart_u,
     const T* __restrict__ gates, const uint32_t* __restrict__ off32, const uint16_t* __restrict__ place,
-    const int64_t* __restrict__ indices, T* __restrict__ dgates, float* __restrict__ coef_up, float* __restrict__ coef_down,
-    float* __restrict__ coef_list, int32_t* __restrict__ counts, int64_t pairs, int num_slices, int top_k) {
+    T* __restrict__ dgates, float* __restrict__ coef_up, float* __restrict__ coef_down, float* __restrict__ coef_list, int64_t pairs,
+    int num_slices, int top_k) {
     const int64_t at = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (at >= pairs) return;
     const int64_t p = place == nullptr ? at : at / top_k * top_k + place[at];
@@ -417,7 +413,6 @@ __global__ __launch_bounds__(256) void expert_backward_gate_kernel(
     coef_down[p] = cd;
     if (place != nullptr) coef_list[at] = cd;
     dgates[p] = Elem<T>::from_f32(valid ? u * act : 0.0f);
-    if (counts != nullptr && valid) atomicAdd(&counts[indices[p]], 1);   // integer histogram: the result does not depend on order
 }
 
 // A wave takes `span` consecutive experts (lane l holds the end of the l-th one's segment) and a chunk of the columns (NCH * 1024 bytes):
@@ -513,9 +508,8 @@ __global__ __launch_bounds__(kBwdWaves* kWave) void expert_backward_weight_kerne
 
 struct ExpertBwdPlan {
     bool slices, ordered;      // slices: column slices of the tables, on ordered lists or not
-    bool partition;            // the pairs are grouped by expert in two partition passes, nothing is counted on the way
     int num_slices;
-    size_t off_coef_up, off_coef_down, off_pairs, off_counts, off_offsets, off_off32, off_place, off_coef_list, off_spart_s, off_spart_u, bytes;
+    size_t off_coef_up, off_coef_down, off_pairs, off_group, off_offsets, off_off32, off_place, off_coef_list, off_spart_s, off_spart_u, bytes;
 };
 
 ExpertBwdPlan plan_expert_backward(int64_t T_, int H, int64_t E, int K, int dtype) {
@@ -526,9 +520,7 @@ ExpertBwdPlan plan_expert_backward(int64_t T_, int H, int64_t E, int K, int dtyp
     p.off_coef_up = take(pairs * 4);
     p.off_coef_down = take(pairs * 4);
     p.off_pairs = take(pairs * 4);
-    p.partition = bucket_partition_pays((int64_t)pairs, E);
-    // the partition's, or per-expert counts, then the fill's cursors, and the scan state
-    p.off_counts = take(p.partition ? bucket_partition_workspace_bytes((int64_t)pairs, E) : bucket_workspace_bytes(E));
+    p.off_group = take(group_pairs_workspace_bytes((int64_t)pairs, E));
     p.off_offsets = take((size_t)(E + 1) * 4);
     const ExpertSavedPlan kept = expert_saved_plan(T_, H, E, K, dtype);
     p.slices = kept.kept;
@@ -556,14 +548,10 @@ int launch_expert_backward(const void* dout, const void* x, const void* down, co
     float* coef_up = (float*)(ws + p.off_coef_up);
     float* coef_down = (float*)(ws + p.off_coef_down);
     uint32_t* pairs_by_expert = (uint32_t*)(ws + p.off_pairs);
-    void* bucket_ws = ws + p.off_counts;
-    int32_t* counts = p.partition ? nullptr : bucket_counts(bucket_ws);
     int32_t* offsets = (int32_t*)(ws + p.off_offsets);
     const int64_t pairs = T_ * K;
     const int nch = (H / V + kWave - 1) / kWave;
     const dim3 block(kBwdWaves * kWave);
-    if (!p.partition)
-        if (int rc = bucket_clear(bucket_ws, E, stream)) return rc;
     if (p.slices) {
         uint32_t* off32 = (uint32_t*)(ws + p.off_off32);
         uint16_t* place = p.ordered ? (uint16_t*)(ws + p.off_place) : nullptr;
@@ -585,7 +573,7 @@ int launch_expert_backward(const void* dout, const void* x, const void* down, co
         if (int rc = expert_slice_scores(dout, up, off32, spart_u, T_, H, E, K, dtype, p.ordered, stream)) return rc;
         hipLaunchKernelGGL((expert_backward_gate_kernel<T>), dim3((unsigned)((pairs + 255) / 256)), dim3(256), 0, stream,
                            (const float*)spart_s, scores, (const float*)spart_u, (const T*)gates, (const uint32_t*)off32,
-                           (const uint16_t*)place, indices, (T*)dgates, coef_up, coef_down, coef_list, counts, pairs, p.num_slices, K);
+                           (const uint16_t*)place, (T*)dgates, coef_up, coef_down, coef_list, pairs, p.num_slices, K);
         FMOE_CHECK_LAUNCH("fmoe_expert_backward(coefficients)");
         if (int rc = expert_slice_states(coef_list, down, off32, dx, T_, H, E, K, dtype, p.ordered, stream)) return rc;
     } else {
@@ -594,7 +582,7 @@ int launch_expert_backward(const void* dout, const void* x, const void* down, co
 #define FMOE_LAUNCH_TOKEN(N, W)                                                                                                       \
         hipLaunchKernelGGL((expert_backward_token_kernel<T, N, W>), dim3((unsigned)(W > 1 ? T_ : (T_ + kBwdWaves - 1) / kBwdWaves)), \
                            dim3((W > 1 ? W : kBwdWaves) * kWave), 0, stream, (const T*)dout, (const T*)x, (const T*)down,            \
-                           (const T*)up, indices, (const T*)gates, (T*)dx, (T*)dgates, coef_up, coef_down, counts, T_, H, E, K)
+                           (const T*)up, indices, (const T*)gates, (T*)dx, (T*)dgates, coef_up, coef_down, T_, H, E, K)
 #define FMOE_LAUNCH_TOKENS(N, MOST)                                      \
         do {                                                             \
             if (waves >= 8) FMOE_LAUNCH_TOKEN(N, MOST);                  \
@@ -610,12 +598,8 @@ int launch_expert_backward(const void* dout, const void* x, const void* down, co
         FMOE_CHECK_LAUNCH("fmoe_expert_backward(tokens)");
     }
 
-    // offsets and segments, each in ascending pair index; without the partition the kernels above counted the pairs of every expert
-    if (int rc = p.partition ? bucket_partition(indices, bucket_ws, pairs, E, K, offsets, (int32_t*)pairs_by_expert, nullptr, 1u,
-                                                nullptr, 1u, nullptr, 0, true, stream)
-                             : bucket_scan_fill(indices, bucket_ws, pairs, E, K, offsets, (int32_t*)pairs_by_expert, nullptr, 1u,
-                                                nullptr, 1u, nullptr, 0, 1, stream))
-        return rc;
+    // offsets and segments, each in ascending pair index
+    if (int rc = group_pairs(indices, ws + p.off_group, pairs, E, K, offsets, (int32_t*)pairs_by_expert, stream)) return rc;
 
     // experts per wave: about a round of 64 pairs, as long as every SIMD keeps four waves
     const int xcds = chip_info().xcds;

@@ -343,8 +343,84 @@ __device__ inline void sort_segment(uint32_t* keys, int n) {
     }
 }
 
-// ASCENDING writes sorted_pairs only (tok and exp NULL).
+// Ascending pair index in every segment of experts [e0, e0 + n_e), whose cursors ends[] stand at the ends of their segments and whose
+// pairs begin at slot `begin`.  in_lds: the pairs are in out_pair (expert e0 + out_low), segment by segment, and go to sorted_pairs;
+// otherwise they are there already, in any order.  CAP: entries of out_pair.
 constexpr int kPartRank = 64;            // longest segment ordered by counting
+template <int CAP>
+__device__ inline void order_segments(const int64_t* __restrict__ indices, int64_t num_pairs, int32_t* __restrict__ sorted_pairs,
+                                      const int32_t* ends, uint32_t* out_pair, const uint16_t* out_low, bool in_lds, int32_t begin,
+                                      int32_t end, int64_t e0, int n_e, int top_k) {
+    constexpr int NT = kPartLocalThreads;
+    __shared__ int32_t long_ones;
+    __shared__ int32_t wave_count[kWalkBatch][NT / kWave];
+    const int tid = (int)threadIdx.x;
+    if (tid == 0) long_ones = in_lds ? 0 : 1;
+    __syncthreads();
+    auto start_of = [&](int j) { return j > 0 ? ends[j - 1] : begin; };
+    if (in_lds) {
+        for (int32_t i = tid; i < end - begin; i += NT) {
+            const uint32_t p = out_pair[i];
+            const int low = out_low[i];
+            const int32_t from = start_of(low), n = ends[low] - from;
+            if (n <= kPartRank) {
+                int rank = 0;
+                for (int q = 0; q < n; ++q) rank += out_pair[from - begin + q] < p ? 1 : 0;
+                sorted_pairs[from + rank] = (int32_t)p;
+            } else {
+                long_ones = 1;
+            }
+        }
+    }
+    __syncthreads();
+    if (long_ones == 0) return;
+    for (int j = 0; j < n_e; ++j) {          // the same for every thread of the workgroup
+        const int32_t from = start_of(j), n = ends[j] - from;
+        if (n <= (in_lds ? kPartRank : 1)) continue;
+        if (n > CAP) {
+            walk_segment<NT / kWave>(indices, num_pairs, e0 + j, from, sorted_pairs, nullptr, top_k, 1u, wave_count);
+            continue;
+        }
+        uint32_t* keys = in_lds ? out_pair + (from - begin) : out_pair;
+        if (!in_lds)
+            for (int i = tid; i < n; i += NT) keys[i] = (uint32_t)sorted_pairs[from + i];
+        __syncthreads();
+        sort_segment(keys, n);
+        for (int i = tid; i < n; i += NT) sorted_pairs[from + i] = (int32_t)keys[i];
+        __syncthreads();
+    }
+}
+
+// Segments of n_e experts from their counts: ends[j] becomes the slot where segment j starts (its cursor), as offsets[e0 + j] does.
+__device__ inline void start_segments(int32_t* ends, int32_t* __restrict__ offsets, int64_t e0, int n_e, int32_t begin,
+                                      int32_t* wave_total) {
+    constexpr int NT = kPartLocalThreads;
+    const int tid = (int)threadIdx.x, lane = tid & (kWave - 1), wave = tid >> 6;
+    // thread t owns experts [t * per, (t + 1) * per)
+    const int per = (n_e + NT - 1) / NT;
+    const int j0 = tid * per < n_e ? tid * per : n_e, j1 = j0 + per < n_e ? j0 + per : n_e;
+    int32_t mine = 0;
+    for (int j = j0; j < j1; ++j) mine += ends[j];
+    int32_t incl = mine;
+#pragma unroll
+    for (int d = 1; d < kWave; d <<= 1) {
+        const int32_t up = __shfl_up(incl, d, kWave);
+        if (lane >= d) incl += up;
+    }
+    if (lane == kWave - 1) wave_total[wave] = incl;
+    __syncthreads();
+    int32_t run = begin + incl - mine;
+    for (int w = 0; w < wave; ++w) run += wave_total[w];
+    for (int j = j0; j < j1; ++j) {
+        const int32_t c = ends[j];
+        offsets[e0 + j] = run;
+        ends[j] = run;
+        run += c;
+    }
+    __syncthreads();
+}
+
+// ASCENDING writes sorted_pairs only (tok and exp NULL).
 template <bool ASCENDING>
 __global__ __launch_bounds__(kPartLocalThreads) void partition_local_kernel(
     const int64_t* __restrict__ indices, int64_t num_pairs, const uint64_t* __restrict__ stage, const int32_t* __restrict__ offs1, int32_t* __restrict__ offsets,
@@ -355,7 +431,7 @@ __global__ __launch_bounds__(kPartLocalThreads) void partition_local_kernel(
     __shared__ uint16_t out_low[kPartLocalCap];
     __shared__ int32_t wave_total[kPartLocalThreads / kWave];
     constexpr int NT = kPartLocalThreads;
-    const int b = (int)blockIdx.x, tid = (int)threadIdx.x, lane = tid & (kWave - 1), wave = tid >> 6;
+    const int b = (int)blockIdx.x, tid = (int)threadIdx.x;
     const int32_t begin = offs1[(int64_t)b * groups], end = offs1[(int64_t)(b + 1) * groups];
     if (b == buckets) {      // the slots after the last segment
         if (tid == 0) offsets[num_experts] = begin;
@@ -375,28 +451,7 @@ __global__ __launch_bounds__(kPartLocalThreads) void partition_local_kernel(
         if (s + NT < end) atomicAdd(&cnt[(uint32_t)v1], 1);
     }
     __syncthreads();
-    // exclusive scan of the counts: thread t owns experts [t * per, (t + 1) * per)
-    const int per = (n_e + NT - 1) / NT;
-    const int j0 = tid * per < n_e ? tid * per : n_e, j1 = j0 + per < n_e ? j0 + per : n_e;
-    int32_t mine = 0;
-    for (int j = j0; j < j1; ++j) mine += cnt[j];
-    int32_t incl = mine;
-#pragma unroll
-    for (int d = 1; d < kWave; d <<= 1) {
-        const int32_t up = __shfl_up(incl, d, kWave);
-        if (lane >= d) incl += up;
-    }
-    if (lane == kWave - 1) wave_total[wave] = incl;
-    __syncthreads();
-    int32_t run = begin + incl - mine;
-    for (int w = 0; w < wave; ++w) run += wave_total[w];
-    for (int j = j0; j < j1; ++j) {
-        const int32_t c = cnt[j];
-        offsets[e0 + j] = run;
-        cnt[j] = run;            // the cursor of expert e0 + j
-        run += c;
-    }
-    __syncthreads();
+    start_segments(cnt, offsets, e0, n_e, begin, wave_total);
     auto emit = [&](int32_t slot, uint32_t p, uint32_t low) {
         const uint32_t e = (uint32_t)e0 + low;
         sorted_pairs[slot] = (int32_t)p;
@@ -423,48 +478,79 @@ __global__ __launch_bounds__(kPartLocalThreads) void partition_local_kernel(
     }
     __syncthreads();
     if constexpr (ASCENDING) {
-        __shared__ int32_t long_ones;
-        __shared__ int32_t wave_count[kWalkBatch][kPartLocalThreads / kWave];
-        if (tid == 0) long_ones = 0;
-        __syncthreads();
-        auto start_of = [&](int j) { return j > 0 ? cnt[j - 1] : begin; };     // the cursors stand at the ends of the segments
-        if (in_lds) {
-            for (int32_t i = tid; i < end - begin; i += NT) {
-                const uint32_t p = out_pair[i];
-                const int low = out_low[i];
-                const int32_t from = start_of(low), n = cnt[low] - from;
-                if (n <= kPartRank) {
-                    int rank = 0;
-                    for (int q = 0; q < n; ++q) rank += out_pair[from - begin + q] < p ? 1 : 0;
-                    sorted_pairs[from + rank] = (int32_t)p;
-                } else {
-                    long_ones = 1;
-                }
-            }
-        } else if (tid == 0) {
-            long_ones = 1;
-        }
-        __syncthreads();
-        if (long_ones == 0) return;
-        for (int j = 0; j < n_e; ++j) {          // the same for every thread of the workgroup
-            const int32_t from = start_of(j), n = cnt[j] - from;
-            if (n <= (in_lds ? kPartRank : 1)) continue;
-            if (n > kPartLocalCap) {
-                walk_segment<kPartLocalThreads / kWave>(indices, num_pairs, e0 + j, from, sorted_pairs, nullptr, top_k, 1u, wave_count);
-                continue;
-            }
-            uint32_t* keys = in_lds ? out_pair + (from - begin) : out_pair;
-            if (!in_lds)
-                for (int i = tid; i < n; i += NT) keys[i] = (uint32_t)sorted_pairs[from + i];
-            __syncthreads();
-            sort_segment(keys, n);
-            for (int i = tid; i < n; i += NT) sorted_pairs[from + i] = (int32_t)keys[i];
-            __syncthreads();
-        }
+        order_segments<kPartLocalCap>(indices, num_pairs, sorted_pairs, cnt, out_pair, out_low, in_lds, begin, end, e0, n_e, top_k);
     } else {
         if (!in_lds) return;
         for (int32_t i = tid; i < end - begin; i += NT) emit(begin + i, out_pair[i], out_low[i]);
     }
+}
+
+// ---- grouping in one launch ---------------------------------------------------------------------------------------------
+// For fewer pairs every workgroup reads all ids (from the L2) and keeps those of its own 2^shift experts: what it counts of lower experts
+// is where its segments begin, the rest happens in LDS as above.  One launch in place of clearing, scan, fill and ordering, and
+// nothing to count elsewhere: 10455 pairs of 4100 experts 15.5 -> 7.1 us.
+constexpr int kOneCap = 4096;            // pairs of a workgroup's experts that are put in order in LDS
+constexpr int kOneBatch = 8;             // loads in flight per thread
+constexpr int kOneMaxGroups = 256;
+
+__global__ __launch_bounds__(kPartLocalThreads) void group_pairs_kernel(const int64_t* __restrict__ indices, int32_t* __restrict__ offsets,
+                                                                       int32_t* __restrict__ sorted_pairs, int64_t num_pairs,
+                                                                       int64_t num_experts, int top_k, int shift) {
+    extern __shared__ int32_t cnt[];     // 1 << shift
+    __shared__ uint32_t out_pair[kOneCap], in_pair[kOneCap];
+    __shared__ uint16_t out_low[kOneCap], in_low[kOneCap];
+    __shared__ int32_t wave_total[kPartLocalThreads / kWave], wave_below[kPartLocalThreads / kWave];
+    __shared__ int32_t mine_s;
+    constexpr int NT = kPartLocalThreads;
+    const int tid = (int)threadIdx.x, lane = tid & (kWave - 1), wave = tid >> 6;
+    const int64_t e0 = (int64_t)blockIdx.x << shift;
+    const int n_e = (int)(num_experts - e0 < (1ll << shift) ? num_experts - e0 : (1ll << shift));
+    for (int j = tid; j < n_e; j += NT) cnt[j] = 0;
+    if (tid == 0) mine_s = 0;
+    __syncthreads();
+    // f(pair, low) for every pair of the workgroup's experts; returns the thread's pairs of lower ones
+    auto scan_ids = [&](auto f) {
+        int32_t below = 0;
+        for (int64_t p0 = tid; p0 < num_pairs; p0 += kOneBatch * NT) {
+            int64_t e[kOneBatch];
+#pragma unroll
+            for (int u = 0; u < kOneBatch; ++u) e[u] = p0 + u * NT < num_pairs ? indices[p0 + u * NT] : -1;
+#pragma unroll
+            for (int u = 0; u < kOneBatch; ++u) {
+                below += e[u] >= 0 && e[u] < e0 ? 1 : 0;
+                if (e[u] >= e0 && e[u] < e0 + n_e) f((uint32_t)(p0 + u * NT), (int)(e[u] - e0));
+            }
+        }
+        return below;
+    };
+    int32_t below = scan_ids([&](uint32_t p, int low) {
+        atomicAdd(&cnt[low], 1);
+        const int32_t at = atomicAdd(&mine_s, 1);
+        if (at < kOneCap) {
+            in_pair[at] = p;
+            in_low[at] = (uint16_t)low;
+        }
+    });
+#pragma unroll
+    for (int d = 1; d < kWave; d <<= 1) below += __shfl_xor(below, d, kWave);
+    if (lane == 0) wave_below[wave] = below;
+    __syncthreads();
+    int32_t begin = 0;
+    for (int w = 0; w < NT / kWave; ++w) begin += wave_below[w];
+    const int32_t mine = mine_s, end = begin + mine;
+    start_segments(cnt, offsets, e0, n_e, begin, wave_total);
+    if (tid == 0 && e0 + n_e == num_experts) offsets[num_experts] = end;
+    const bool in_lds = mine <= kOneCap;
+    if (in_lds)
+        for (int32_t i = tid; i < mine; i += NT) {
+            const int32_t slot = atomicAdd(&cnt[in_low[i]], 1) - begin;
+            out_pair[slot] = in_pair[i];
+            out_low[slot] = in_low[i];
+        }
+    else
+        scan_ids([&](uint32_t p, int low) { sorted_pairs[atomicAdd(&cnt[low], 1)] = (int32_t)p; });
+    __syncthreads();
+    order_segments<kOneCap>(indices, num_pairs, sorted_pairs, cnt, out_pair, out_low, in_lds, begin, end, e0, n_e, top_k);
 }
 
 struct PartitionPlan {
@@ -553,7 +639,35 @@ int bucket_partition(const int64_t* indices, void* workspace, int64_t num_pairs,
     return FMOE_OK;
 }
 
-int32_t* bucket_counts(void* workspace) { return (int32_t*)workspace; }
+// Pairs in ascending index by expert for the weight gradients, the way their number asks for.  `workspace`: group_pairs_workspace_bytes.
+static bool group_in_one(int64_t num_pairs, int64_t num_experts) {
+    return num_pairs < (1ll << 16) && num_experts <= (int64_t)kOneMaxGroups << kPartMaxShift;
+}
+size_t group_pairs_workspace_bytes(int64_t num_pairs, int64_t num_experts) {
+    if (group_in_one(num_pairs, num_experts)) return 0;
+    return bucket_partition_pays(num_pairs, num_experts) ? bucket_partition_workspace_bytes(num_pairs, num_experts)
+                                                         : bucket_workspace_bytes(num_experts);
+}
+int group_pairs(const int64_t* indices, void* workspace, int64_t num_pairs, int64_t num_experts, int top_k, int32_t* offsets,
+                int32_t* sorted_pairs, hipStream_t stream) {
+    if (group_in_one(num_pairs, num_experts)) {
+        int shift = 0;
+        while ((num_experts + (1ll << shift) - 1) >> shift > kOneMaxGroups) ++shift;
+        const unsigned groups = (unsigned)((num_experts + (1ll << shift) - 1) >> shift);
+        hipLaunchKernelGGL(group_pairs_kernel, dim3(groups), dim3(kPartLocalThreads), (size_t)4 << shift, stream, indices, offsets,
+                           sorted_pairs, num_pairs, num_experts, top_k, shift);
+        FMOE_CHECK_LAUNCH("expert bucketing (one launch)");
+        return FMOE_OK;
+    }
+    if (bucket_partition_pays(num_pairs, num_experts))
+        return bucket_partition(indices, workspace, num_pairs, num_experts, top_k, offsets, sorted_pairs, nullptr, 1u, nullptr, 1u,
+                                nullptr, 0, true, stream);
+    if (int rc = bucket_clear(workspace, num_experts, stream)) return rc;
+    if (num_pairs > 0)
+        if (int rc = bucket_histogram(indices, workspace, num_pairs, num_experts, stream)) return rc;
+    return bucket_scan_fill(indices, workspace, num_pairs, num_experts, top_k, offsets, sorted_pairs, nullptr, 1u, nullptr, 1u, nullptr,
+                            0, 1, stream);
+}
 
 int bucket_clear(void* workspace, int64_t num_experts, hipStream_t stream) {
     const BucketPlan p = plan_bucket(num_experts);
@@ -567,7 +681,7 @@ int bucket_clear(void* workspace, int64_t num_experts, hipStream_t stream) {
 int bucket_histogram(const int64_t* indices, void* workspace, int64_t num_pairs, int64_t num_experts, hipStream_t stream) {
     const int64_t blocks = (num_pairs + 255) / 256;
     hipLaunchKernelGGL(bucket_histogram_kernel, dim3((unsigned)(blocks < 4096 ? blocks : 4096)), dim3(256), 0, stream, indices,
-                       bucket_counts(workspace), num_pairs, num_experts);
+                       (int32_t*)workspace, num_pairs, num_experts);
     FMOE_CHECK_LAUNCH("expert bucketing (histogram)");
     return FMOE_OK;
 }

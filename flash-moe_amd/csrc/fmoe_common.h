@@ -148,13 +148,12 @@ bool gemm_nt_dual_usable(int64_t M, int N, int K);
 int gemm_nt_dual(const void* A, const void* B, void* C, float* C32, int M, int N, int K, int dtype, hipStream_t stream);
 
 // Expert-centric bucketing (fmoe_bucket.hip): pairs grouped by expert id.  The workspace holds the per-expert counts
-// (bucket_counts; cleared by bucket_clear, filled by bucket_histogram or by a caller's own kernel) and the scan state.
+// (cleared by bucket_clear, filled by bucket_histogram) and the scan state.
 // bucket_scan_fill turns the counts into offsets [E+1] and writes, per slot of the grouped order, the pair index, and
 // optionally token * tok_scale and expert * exp_scale; `coef_clear` [num_pairs] gets a zero for every pair whose id is
 // outside [0,E); with `pack_shift` the token word also carries the id, shifted left by that many bits (truncated to 32
 // bits); `ordered` puts every segment in ascending pair index (and rewrites the token words without packing).
 size_t bucket_workspace_bytes(int64_t num_experts);
-int32_t* bucket_counts(void* workspace);
 int bucket_clear(void* workspace, int64_t num_experts, hipStream_t stream);
 int bucket_histogram(const int64_t* indices, void* workspace, int64_t num_pairs, int64_t num_experts, hipStream_t stream);
 int bucket_scan_fill(const int64_t* indices, void* workspace, int64_t num_pairs, int64_t num_experts, int top_k,
@@ -169,6 +168,10 @@ size_t bucket_partition_workspace_bytes(int64_t num_pairs, int64_t num_experts);
 int bucket_partition(const int64_t* indices, void* workspace, int64_t num_pairs, int64_t num_experts, int top_k,
                      int32_t* offsets, int32_t* sorted_pairs, uint32_t* tok, uint32_t tok_scale, uint32_t* exp,
                      uint32_t exp_scale, float* coef_clear, int pack_shift, bool ascending, hipStream_t stream);
+// ... and for the weight gradients: segments in ascending pair index by one launch, the partition or the counters (fmoe_bucket.hip).
+size_t group_pairs_workspace_bytes(int64_t num_pairs, int64_t num_experts);
+int group_pairs(const int64_t* indices, void* workspace, int64_t num_pairs, int64_t num_experts, int top_k, int32_t* offsets,
+                int32_t* sorted_pairs, hipStream_t stream);
 
 // Plain library GEMM (rocBLAS, loaded on first use) for the operand layouts of the backward passes; row-major
 // C[M,N] = A[M,K] B[K,N] (kBlasNN) or A[K,M]^T B[K,N] (kBlasTN), C = product + beta * C.  Defined in fmoe_mlp_backward.hip.
