@@ -30,8 +30,7 @@ constexpr int kWideLdsElements = 65536;                          // two buffers 
 
 // Position of tile t in the order each XCD walks: XCD x (workgroup id mod xcds) takes a contiguous run, eight tile-rows at a time.
 __device__ __forceinline__ void wide_tile_at(int t, int num_tiles, int tiles_m, int tiles_n, int xcds, int& tm, int& tn) {
-    const int x = t % xcds, each = num_tiles / xcds, more = num_tiles % xcds;
-    t = x * each + (x < more ? x : more) + t / xcds;
+    t = xcd_run(t, num_tiles, xcds);
     constexpr int GM = 8;
     const int width = GM * tiles_n, group = t / width, first_m = group * GM;
     const int gsz = (tiles_m - first_m) < GM ? (tiles_m - first_m) : GM;

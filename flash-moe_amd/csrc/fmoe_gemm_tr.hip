@@ -29,14 +29,15 @@
 namespace fmoe {
 namespace {
 
-// SLICED: workgroup = slice * tiles + tile, sums to plane `slice` of C (fp32).
+// SLICED: each XCD takes a run of slice * tiles + tile, so that it fetches its slices' part of the operands only, sums to plane `slice` of C
+// (fp32).  dx of 615 tokens, 2072 -> 776 in six slices of 35 tiles 17.5 -> 14 us with both operands far from the compute units.
 template <typename T, bool TA, int BM, int BN, int WAVES_N, int NSTAGE, bool SLICED>
 __global__ __launch_bounds__(2 * WAVES_N * kWave) void gemm_turned_kernel(
     const T* __restrict__ A, int lda, const T* __restrict__ B0, const T* __restrict__ B1, int ldb, T* __restrict__ C, int M, int N, int K,
     int segments, int tiles_m, int tiles_n, int xcds, int slices) {
-    const int tiles = tiles_m * tiles_n, block = (int)blockIdx.x;
+    const int tiles = tiles_m * tiles_n, block = SLICED ? xcd_run((int)blockIdx.x, (int)gridDim.x, xcds) : (int)blockIdx.x;
     gemm_dma_tiles<T, BM, BN, 2, WAVES_N, kStageK<T>, NSTAGE, SLICED ? kEpiPart : kEpiPlain, kSmallAhead<T>, kFragRows<T>, true, SLICED,
-                   TA, true>(A, B0, B1, C, nullptr, M, N, K, tiles_m, tiles_n, xcds, SLICED ? block % tiles : block,
+                   TA, true>(A, B0, B1, C, nullptr, M, N, K, tiles_m, tiles_n, SLICED ? 1 : xcds, SLICED ? block % tiles : block,
                              SLICED ? tiles : (int)gridDim.x, SLICED ? block / tiles : 0, slices, lda, ldb, segments);
 }
 
@@ -44,9 +45,9 @@ template <typename T, bool TA, bool SLICED, bool RAGGED>
 __global__ __launch_bounds__(kWideThreads, 2) void gemm_wide_turned_kernel(
     const T* __restrict__ A, int lda, const T* __restrict__ B0, const T* __restrict__ B1, int ldb, T* __restrict__ C, int M, int N, int K,
     int segments, int tiles_m, int tiles_n, int xcds, int slices) {
-    const int tiles = tiles_m * tiles_n, block = (int)blockIdx.x;
+    const int tiles = tiles_m * tiles_n, block = SLICED ? xcd_run((int)blockIdx.x, (int)gridDim.x, xcds) : (int)blockIdx.x;
     gemm_wide_tiles<T, SLICED ? kEpiPart : kEpiPlain, RAGGED, SLICED, TA, true>(
-        A, B0, B1, C, nullptr, M, N, K, tiles_m, tiles_n, xcds, SLICED ? block % tiles : block, SLICED ? tiles : (int)gridDim.x,
+        A, B0, B1, C, nullptr, M, N, K, tiles_m, tiles_n, SLICED ? 1 : xcds, SLICED ? block % tiles : block, SLICED ? tiles : (int)gridDim.x,
         SLICED ? block / tiles : 0, slices, lda, ldb, segments);
 }
 

@@ -56,18 +56,17 @@ __global__ __launch_bounds__(kWideThreads, 2) void gemm_wide_kernel(const T* __r
 template <typename T>
 __global__ __launch_bounds__(kWideThreads, 2) void gemm_wide_sliced_kernel(const T* __restrict__ A, const T* __restrict__ B, float* __restrict__ planes, int M,
                                                                         int N, int K, int tiles_m, int tiles_n, int xcds, int slices) {
-    const int tiles = tiles_m * tiles_n;
-    gemm_wide_tiles<T, kEpiPart, true, true>(A, B, nullptr, reinterpret_cast<T*>(planes), nullptr, M, N, K, tiles_m, tiles_n, xcds,
-                                             (int)blockIdx.x % tiles, tiles, (int)blockIdx.x / tiles, slices);
+    const int tiles = tiles_m * tiles_n, at = xcd_run((int)blockIdx.x, (int)gridDim.x, xcds);
+    gemm_wide_tiles<T, kEpiPart, true, true>(A, B, nullptr, reinterpret_cast<T*>(planes), nullptr, M, N, K, tiles_m, tiles_n, 1, at % tiles,
+                                             tiles, at / tiles, slices);
 }
 
 template <typename T, int BM, int BN, int WAVES_N, int NSTAGE>
 __global__ __launch_bounds__(2 * WAVES_N * 64) void gemm_sliced_kernel(const T* __restrict__ A, const T* __restrict__ B, float* __restrict__ planes, int M,
                                                           int N, int K, int tiles_m, int tiles_n, int xcds, int slices) {
-    const int tiles = tiles_m * tiles_n;
+    const int tiles = tiles_m * tiles_n, at = xcd_run((int)blockIdx.x, (int)gridDim.x, xcds);
     gemm_dma_tiles<T, BM, BN, 2, WAVES_N, kStageK<T>, NSTAGE, kEpiPart, kSmallAhead<T>, kFragRows<T>, true, true>(
-        A, B, nullptr, reinterpret_cast<T*>(planes), nullptr, M, N, K, tiles_m, tiles_n, xcds, (int)blockIdx.x % tiles, tiles,
-        (int)blockIdx.x / tiles, slices);
+        A, B, nullptr, reinterpret_cast<T*>(planes), nullptr, M, N, K, tiles_m, tiles_n, 1, at % tiles, tiles, at / tiles, slices);
 }
 
 // C = sum of the planes in slice order [+ R]; four elements per thread.

@@ -218,3 +218,29 @@ def test_mlp_on_the_widest_tiles(dtype, T, N, K):
             assert off.norm() < times * tol * want.norm() and (off <= 2 * times * tol * want.abs() + 1e-5 * K).all()
         for buf, rows, at in ((abuf, T, 0), (sbuf, 2 * T, 0), (obuf, T, shift)):
             assert (buf[:8 * N + at] == 7).all() and (buf[(8 + rows) * N + at:] == 7).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("T,H,I", [
+    (337, 2056, 2664),        # more operand bytes than runs of tiles begin at, 3 tile-rows; dx in slices
+    (1154, 392, 784),         # fewer: the order as it is
+    (2200, 1016, 1992),       # several groups of eight tile-rows, the last not full
+])
+def test_mlp_where_tiles_are_no_multiple_of_the_xcds(dtype, T, H, I):
+    """Every tile is formed once, forward and backward, however the XCDs share them out: a left-out tile is wrong by its whole size.
+    Bound: one rounding to the type per stage (2^-9; fp32 sums of I products), three of them one after another in the longest chain."""
+    from flash_moe.ops import flash_mlp_func
+
+    x, *ws = (t.cuda().requires_grad_(True) for t in make(T, H, I, dtype, seed=T + H))
+    dy = torch.randn(T, H, generator=torch.Generator().manual_seed(I)).to("cuda", dtype)
+    y = flash_mlp_func(x, *ws)
+    y.backward(dy)
+    x64, *ws64 = (t.detach().double().requires_grad_(True) for t in (x, *ws))
+    y64 = (torch.nn.functional.silu(x64 @ ws64[0].t()) * (x64 @ ws64[1].t())) @ ws64[2].t()
+    y64.backward(dy.double())
+    tol = 3 * 2.0 ** -9 if dtype == torch.bfloat16 else 2e-5
+    for got, want in [(y.detach(), y64.detach())] + [(a.grad, b.grad) for a, b in zip((x, *ws), (x64, *ws64))]:
+        off, size = got.double() - want, want.norm()
+        assert off.norm() < tol * size
+        rows = off.norm(dim=1)
+        assert (rows < 4 * tol * size / want.shape[0] ** 0.5).all()
