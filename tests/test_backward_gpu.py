@@ -48,6 +48,7 @@ def test_router_backward(dtype, T, nk, K):
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("norm", [False, True])
 @pytest.mark.parametrize("T,nk,K", [(64, 32, 16), (130, 128, 64), (9, 512, 128), (5, 8, 1),
+                                    (7, 129, 64), (7, 128, 65), (7, 256, 128), (6, 257, 128), (6, 256, 129), (3, 1, 1),   # what registers hold
                                     (5, 8192, 64), (6, 20000, 96)])   # the last: rows built 4096 keys at a time
 def test_route_backward(dtype, norm, T, nk, K):
     """Gate gradients -> gradient of the fp32 gate logits, against float64 autograd of log-softmax, pair sums, exp and
