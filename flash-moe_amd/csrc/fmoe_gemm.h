@@ -24,8 +24,8 @@ template <typename T, int N> struct DmaLds {
 // Position of item t of n in the order the XCDs walk: XCD x (workgroup id mod xcds) takes a contiguous run, so that what its items share
 // passes into its L2 once.  A permutation of [0, n) for every n.
 __host__ __device__ __forceinline__ int xcd_run(int t, int n, int xcds) {
-    const int x = t % xcds, each = n / xcds, more = n % xcds;
-    return x * each + (x < more ? x : more) + t / xcds;
+    const uint32_t x = (uint32_t)t % (uint32_t)xcds, each = (uint32_t)n / (uint32_t)xcds, more = (uint32_t)n % (uint32_t)xcds;
+    return (int)(x * each + (x < more ? x : more) + (uint32_t)t / (uint32_t)xcds);
 }
 
 // Products whose number of tiles is no multiple of the XCDs, neither operand turned: runs where the operands are larger than this, two and
@@ -132,7 +132,7 @@ __device__ __forceinline__ void gemm_dma_tiles(
     // run of the tile order, walked 8 tile-rows at a time so that a compact patch shares A and B tiles in the XCD's L2.
     // Turned products take runs whatever their number of tiles: backward passes of 777 tokens, 2048 -> 5464 252 -> 236 us, 8000 tokens,
     // 320 -> 848 125 -> 112, 546 tokens, 1304 -> 2608 106 -> 97, none slower.
-    const bool runs = kTurned || num_tiles % xcds == 0 || ((int64_t)M + (EPI == kEpiSwiGLU ? 2 : 1) * (int64_t)N) * K * (int64_t)sizeof(T) > kRunBytes;
+    const bool runs = kTurned || (uint32_t)num_tiles % (uint32_t)xcds == 0 || ((int64_t)M + (EPI == kEpiSwiGLU ? 2 : 1) * (int64_t)N) * K * (int64_t)sizeof(T) > kRunBytes;
     auto set_tile = [&](int t) {
         if (runs) t = xcd_run(t, num_tiles, xcds);
         constexpr int GM = 8;
