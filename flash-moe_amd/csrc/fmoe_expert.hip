@@ -1493,8 +1493,10 @@ bool ordered_possible(int64_t E, int H, int K, size_t elt) { return slices_possi
 // product-key router): 2.4 % longer than the best of the four on average; the rule before it (slices up to 65536 experts, then ordered
 // lists from 400 K = E on, then buckets) 12 %.  us below.
 //
-// Fewer than 2^16 pairs and 128 MB of rows: whole rows, one launch instead of three or four (beyond, 2000 x 24 of 10000 with rows of 4 KB
-// takes 39 in slices for 57).
+// Fewer than 2^16 pairs and 128 MB of rows: whole rows, one launch instead of three or four.  Beyond, slices take 0.76 times as long as
+// rows in fp16 and 0.64 in fp32 (up to 4096 x 256, rows of 2 to 8 KB, 468 problems; 100 to 128 MB 0.84 and 0.81, 60 to 80 MB 1.06 and 1.01;
+// fp16, H 1984, 2200 x 25 of 4600 41 for 69).  Not in bf16, whose slices round the coefficients that rows keep in fp32; routing weights
+// without a score are bf16 as they come.
 //
 // A slice of 256 bytes fits an XCD's L2 (16384 experts): slices (16384 x 64 of 16384, H 1024: 229 for 291 ordered, 546 in rows).  But rows
 // for fewer than 12 experts per token, where most of a step is empty (16384 x 8 of 600: 32 for 68), unless they are 4 KB; for up to 150 MB
@@ -1520,9 +1522,10 @@ bool ordered_possible(int64_t E, int H, int K, size_t elt) { return slices_possi
 // Buckets, once an expert's row serves a dozen pairs and rows are 1 KB or at least 2 KB (H 1024: 32768 x 64 of 102400 1.15 times faster; H
 // 256 1.6 times slower than rows, H 640 1.3: those keep them only from 2^17 experts on, where a test holds the schedule); else whole rows,
 // straight from HBM.
-int choose_schedule(int algo, int64_t T_, int H, int64_t E, int K, size_t elt, bool scored = true) {
+int choose_schedule(int algo, int64_t T_, int H, int64_t E, int K, int dtype, bool scored = true) {
     if (K == 0) return FMOE_EXPERT_ROWS;
     if (algo != FMOE_EXPERT_AUTO) return algo;
+    const size_t elt = dtype_size(dtype);
     const ChipInfo& chip = chip_info();
     const int64_t pairs = T_ * K, row = (int64_t)H * (int64_t)elt, l2 = chip.l2_bytes;
     const bool rows = rows_possible(H, elt), slices = slices_possible(E, H, elt), on_lines = row % 128 == 0, many = pairs >= (1ll << 16);
@@ -1543,7 +1546,8 @@ int choose_schedule(int algo, int64_t T_, int H, int64_t E, int K, size_t elt, b
     }
     if (slices && fits) {
         const bool resident = 2 * E * row * 4 <= 5 * l2 && row >= 1024;
-        const bool pay = (many || pairs * row >= 128000000) && (K >= 12 || (row >= 4096 && !resident)) &&
+        const bool coef32 = dtype != FMOE_BF16 || !scored;
+        const bool pay = (many || (coef32 && pairs * row >= 128000000)) && (K >= 12 || (row >= 4096 && !resident)) &&
                          (on_lines || pairs * row >= 150000000 || K >= 64) && !(resident && K < 128 && (pairs < (1ll << 17) || K < 16));
         return pay || !rows ? FMOE_EXPERT_SLICES : FMOE_EXPERT_ROWS;
     }
@@ -1556,13 +1560,13 @@ int choose_schedule(int algo, int64_t T_, int H, int64_t E, int K, size_t elt, b
 }  // namespace
 
 bool expert_slices_usable(int64_t num_tokens, int hidden, int64_t num_experts, int top_k, int dtype) {
-    return top_k > 0 && choose_schedule(FMOE_EXPERT_AUTO, num_tokens, hidden, num_experts, top_k, dtype_size(dtype)) == FMOE_EXPERT_SLICES;
+    return top_k > 0 && choose_schedule(FMOE_EXPERT_AUTO, num_tokens, hidden, num_experts, top_k, dtype) == FMOE_EXPERT_SLICES;
 }
 
 uint32_t* expert_workspace_offsets(void* workspace) { return (uint32_t*)workspace; }   // SlicePlan::off_idx32 == 0
 
 bool expert_rows_chosen(int64_t num_tokens, int hidden, int64_t num_experts, int top_k, int dtype) {
-    return choose_schedule(FMOE_EXPERT_AUTO, num_tokens, hidden, num_experts, top_k, dtype_size(dtype)) == FMOE_EXPERT_ROWS;
+    return choose_schedule(FMOE_EXPERT_AUTO, num_tokens, hidden, num_experts, top_k, dtype) == FMOE_EXPERT_ROWS;
 }
 
 int expert_rows_added(const void* x, const void* down, const void* up, const int64_t* indices, const void* gates, int64_t num_tokens,
@@ -1581,7 +1585,7 @@ int expert_rows_added(const void* x, const void* down, const void* up, const int
 ExpertSavedPlan expert_saved_plan(int64_t num_tokens, int hidden, int64_t num_experts, int top_k, int dtype) {
     ExpertSavedPlan p = {};
     if (num_tokens <= 0 || top_k <= 0) return p;
-    const int schedule = choose_schedule(FMOE_EXPERT_AUTO, num_tokens, hidden, num_experts, top_k, dtype_size(dtype));
+    const int schedule = choose_schedule(FMOE_EXPERT_AUTO, num_tokens, hidden, num_experts, top_k, dtype);
     p.kept = schedule == FMOE_EXPERT_SLICES || schedule == FMOE_EXPERT_ORDERED;
     p.ordered = schedule == FMOE_EXPERT_ORDERED;
     if (!p.kept) return p;
@@ -1651,7 +1655,7 @@ extern "C" size_t fmoe_expert_workspace_bytes_algo(int64_t num_tokens, int hidde
     using namespace fmoe;
     if (num_tokens <= 0 || hidden <= 0 || num_experts <= 0 || top_k <= 0 || !dtype_ok(dtype)) return 0;
     const size_t elt = dtype_size(dtype);
-    switch (choose_schedule(algo, num_tokens, hidden, num_experts, top_k, elt)) {
+    switch (choose_schedule(algo, num_tokens, hidden, num_experts, top_k, dtype)) {
         case FMOE_EXPERT_SLICES: return plan_slices(num_tokens, hidden, num_experts, top_k, elt).bytes;
         case FMOE_EXPERT_BUCKETS: return plan_bucketed(num_tokens, hidden, num_experts, top_k, elt).bytes;
         case FMOE_EXPERT_ORDERED: return plan_slices(num_tokens, hidden, num_experts, top_k, elt, true).bytes;
@@ -1671,7 +1675,7 @@ extern "C" size_t fmoe_pkm_workspace_bytes(int64_t num_tokens, int hidden, int64
     using namespace fmoe;
     if (num_tokens <= 0 || hidden <= 0 || num_experts <= 0 || top_k <= 0 || !dtype_ok(dtype)) return 0;
     const size_t elt = dtype_size(dtype);
-    switch (choose_schedule(FMOE_EXPERT_AUTO, num_tokens, hidden, num_experts, top_k, elt, false)) {
+    switch (choose_schedule(FMOE_EXPERT_AUTO, num_tokens, hidden, num_experts, top_k, dtype, false)) {
         case FMOE_EXPERT_SLICES: return plan_slices(num_tokens, hidden, num_experts, top_k, elt).bytes;
         case FMOE_EXPERT_ORDERED: return plan_slices(num_tokens, hidden, num_experts, top_k, elt, true, false).bytes;
         default: return 0;
@@ -1706,7 +1710,7 @@ int expert_dispatch(const char* who, int act, const void* x, const void* down, c
                  (long long)(num_tokens * top_k));
     hipStream_t s = (hipStream_t)stream;
     const size_t elt = dtype_size(dtype);
-    const int schedule = choose_schedule(algo, num_tokens, hidden, num_experts, top_k, elt, act != kActNone);
+    const int schedule = choose_schedule(algo, num_tokens, hidden, num_experts, top_k, dtype, act != kActNone);
     FMOE_REQUIRE(schedule != FMOE_EXPERT_SLICES || slices_possible(num_experts, hidden, elt), FMOE_ERR_UNSUPPORTED,
                  "%s: tables of 4 GiB or more cannot use the column-slice schedule", who);
     FMOE_REQUIRE(schedule != FMOE_EXPERT_BUCKETS || bucketed_possible(num_tokens, num_experts, hidden, top_k, elt),

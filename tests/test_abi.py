@@ -229,6 +229,18 @@ def test_backward_argument_checks():
     assert mb(a, a, a, a, a, a, 8, 64, 128, _C.BF16, a, a, a, a, a, sneed - 1, None) == -7      # with saved products
 
 
+@pytest.mark.parametrize("T,H,E,K", [(1024, 2048, 16384, 32), (1960, 1536, 3481, 31), (521, 2048, 9000, 63), (2047, 2048, 9801, 31)])
+def test_few_bf16_pairs_of_long_rows_keep_fp32_coefficients(T, H, E, K):
+    """Below 2^16 pairs bf16 takes whole rows however many bytes they are, without scratch and with nothing kept for a backward pass: its
+    column slices round the coefficients, fp16's and fp32's do not, and a product-key memory's are routing weights as they came."""
+    lib = _C.lib()
+    assert T * K < 1 << 16 and T * K * H * 2 >= 128000000
+    assert lib.fmoe_expert_workspace_bytes(T, H, E, K, _C.BF16) == lib.fmoe_expert_saved_bytes(T, H, E, K, _C.BF16) == 0
+    for code in (_C.F16, _C.F32):
+        assert lib.fmoe_expert_workspace_bytes(T, H, E, K, code) == lib.fmoe_expert_workspace_bytes_algo(T, H, E, K, code, _C.EXPERT_SLICES)
+    assert lib.fmoe_pkm_workspace_bytes(T, H, E, K, _C.BF16) > 0
+
+
 def test_expert_workspace_is_enough_for_both_forwards():
     """The forward of a training step may take the ordered lists where the other takes buckets: one size for both."""
     lib = _C.lib()
