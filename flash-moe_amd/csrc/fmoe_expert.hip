@@ -1489,39 +1489,51 @@ bool slices_possible(int64_t E, int H, size_t elt) { return (uint64_t)E * (uint6
 bool ordered_possible(int64_t E, int H, int K, size_t elt) { return slices_possible(E, H, elt) && K <= kOrderMaxTopK; }
 
 // Which schedule a call takes.  A forced schedule that cannot run these extents is reported by the dispatcher; AUTO takes what follows,
-// from sweeps of all four over some 6000 problems (bf16, H 256 to 2048, E 600 to 197000, 256 x 64 to 32768 x 128, ids uniform and from a
-// product-key router): 2.4 % longer than the best of the four on average; the rule before it (slices up to 65536 experts, then ordered
-// lists from 400 K = E on, then buckets) 12 %.  us below.
+// from sweeps of all four, H 256 to 2048, E 600 to 260000, 256 x 64 to 32768 x 256, ids uniform and from a product-key router, forward and
+// training step: over 11400 problems in bf16, 5300 in fp16 and 5800 in fp32 it is 2, 3 and 3 % longer than the best of the four on average,
+// in training 1.2 to 2 (below 2^16 pairs 6 and 7 in fp16 and fp32; without scores 3.4 to 4.6, over 4600).  The lines lie at the same bytes
+// in all three types except where fp32 is named: its elements are half as many.  us below, bf16 unless another type is named.
 //
 // Fewer than 2^16 pairs and 128 MB of rows: whole rows, one launch instead of three or four.  Beyond, slices take 0.76 times as long as
 // rows in fp16 and 0.64 in fp32 (up to 4096 x 256, rows of 2 to 8 KB, 468 problems; 100 to 128 MB 0.84 and 0.81, 60 to 80 MB 1.06 and 1.01;
-// fp16, H 1984, 2200 x 25 of 4600 41 for 69).  Not in bf16, whose slices round the coefficients that rows keep in fp32; routing weights
-// without a score are bf16 as they come.
+// fp16, H 1984, 2200 x 25 of 4600 41 for 69), and blocks of up to 2048 tokens, which lose the launch that selection and down product share,
+// 0.89 and 0.90 (50 blocks).  Not in bf16, whose slices round the coefficients that rows keep in fp32; routing weights without a score are
+// bf16 as they come.
 //
 // A slice of 256 bytes fits an XCD's L2 (16384 experts): slices (16384 x 64 of 16384, H 1024: 229 for 291 ordered, 546 in rows).  But rows
-// for fewer than 12 experts per token, where most of a step is empty (16384 x 8 of 600: 32 for 68), unless they are 4 KB; for up to 150 MB
-// of rows that start between cache lines and whose pieces touch a line more each (H 776: 4096 x 16 35 for 45), unless a token has 64;
-// and for few experts per token of tables that the L2 holds whole (600 x 2 KB: 4096 x 40 1.25 times faster, 16384 x 16 1.29).
+// for fewer than 12 experts per token, where most of a step is empty (10 to 12: 1.17 to 1.19 times faster; fp32 fewer than 10), unless they
+// are 4 KB; for up to 150 MB of rows that start between cache lines and whose pieces touch a line more each (H 776: 4096 x 16 35 for 45),
+// unless a token has 64; and for few experts per token of tables that the L2 holds whole (600 x 2 KB: 4096 x 40 1.25 times faster, 16384 x
+// 16 1.29; all types 1.05 to 1.4 up to 64 experts, 0.9 beyond 2^17 pairs of 64 to 128).
 //
 // Larger tables, ordered: where the tokens in flight on an XCD (2560) name every expert 1.3 times (rows of 3 KB: twice), so that a piece
 // serves several of them, and their lists keep in step well enough for the window to stay in the L2; it is as wide as E / sqrt(K), up to
 // E = 12000 sqrt(K).  H 1024: 1024 x 256 of 45000 76 for 104, of 102400 122 for 141; 4096 x 500 of 65000 505 for 715; 16384 x 128 of 50000
 // 533 for 640; beyond the limits 4096 x 64 of 102400 1.03, 1024 x 128 of 197000 1.19, H 2048, 1024 x 128 of 90000 1.15 times the rows.
-// Narrower, E = 9000 sqrt(K), where buckets pay (H 2048, 32768 x 64 of 90000: 2200 for 1800) and for rows of fewer slices than XCDs.  Up to 100 experts per token slices of 128
-// bytes are ahead where they fit (H 1024: 4096 x 64 of 35000 1.10 times), and for rows of fewer slices than XCDs while all of one fits (H
-// 512: 16384 x 64 of 50000 1.16 times).  Slices that leave more than one XCD in eight without work do not pay (H 640, five of them: 6000 x
-// 200 of 40000 313 for 233 in slices of 128 bytes).  Rows between lines, whose pieces are three lines: four times and 4000 sqrt(K) (H 776:
-// 1024 x 800 of 75000 1.16 times faster, 4096 x 64 of 35000 1.18 times slower), and from 11000 experts on, where their slices outgrow
-// the L2 (H 1000: 6000 x 200 of 16000 327 for 440).
+// Narrower, E = 9000 sqrt(K), where buckets pay (H 2048, 32768 x 64 of 90000: 2200 for 1800) and for rows of fewer slices than XCDs.
+// Up to 100 experts per token slices of 128 bytes are ahead where they fit (H 1024: 4096 x 64 of 35000 1.10 times), and for rows of fewer
+// slices than XCDs while all of one fits (H 512: 16384 x 64 of 50000 1.16 times).  Slices that leave more than one XCD in eight without
+// work do not pay against those (H 640, five of them: 6000 x 200 of 40000 313 for 233 in slices of 128 bytes).  Rows between lines, whose
+// pieces are three lines: four times and 4000 sqrt(K) (H 776: 4096 x 64 of 35000 1.18 times slower), and from 11000 experts on, where their
+// slices outgrow the L2 (H 1000: 6000 x 200 of 16000 327 for 440).
+//
+// Where no slice fits (beyond 65536 experts, in rows between lines 21000) ordered lists compete with rows and buckets only, and pay
+// earlier: from every expert named 1.1 times on, in rows between lines four times and up to 5500 sqrt(K) (H 736, 1097 x 816 of 66000 246 for 443;
+// fp16, H 336, 2107 x 881 of 26000 259 for 576).  XCDs without a slice count by the square of their share, on both lines: with six of eight in
+// work the lists are ahead from 2 to 4 times on, with all of them from 1 to 1.3 (H 384, 2172 x 535 of 102000 205 for 356).  Up to 512 tokens
+// of 100 experts or more are too few to fill the chip in rows and walk ordered lists from once on (H 384, 282 x 757 of 121000 57 for 119;
+// fp16, H 256, 286 x 540 of 144000 38 for 82); of 1024 tokens they no longer pay there.
 //
 // Slices of 128 bytes, while an L2 holds half of one (H 1024: 16384 x 32 of 24000 1.25 times faster than ordered, 4096 x 32 of 50000 1.21
-// than rows), all of one for rows of 4 KB (beyond, rows 1.07 to 1.12 times faster); for rows of 1 KB from 24 experts per token on; for rows
-// between lines up to 21000 experts (H 1000: 20000 x 30 of 20000 275 for 333).  Shorter rows would still gain beyond 65536 experts (H 256:
-// 16384 x 64 of 102400 1.15 times), but in bf16 slices round the coefficients, which the other schedules keep in fp32.
+// than rows), all of one for 16-bit rows of 4 KB (beyond, rows 1.07 to 1.12 times faster; fp32 rows of 4 to 8 KB 0.75 to 0.89); for 16-bit
+// rows of 1 KB from 24 experts per token on (12 to 16 1.1 times the rows, fp32 0.85); for rows between lines up to 21000 experts (H 1000:
+// 20000 x 30 of 20000 275 for 333).  Shorter rows would still gain beyond 65536 experts (H 256: 16384 x 64 of 102400 1.15 times), but in
+// bf16 slices round the coefficients, which the other schedules keep in fp32.
 //
-// Buckets, once an expert's row serves a dozen pairs and rows are 1 KB or at least 2 KB (H 1024: 32768 x 64 of 102400 1.15 times faster; H
-// 256 1.6 times slower than rows, H 640 1.3: those keep them only from 2^17 experts on, where a test holds the schedule); else whole rows,
-// straight from HBM.
+// Buckets, once an expert's row serves a dozen pairs and rows are 2 KB, in fp32 1.5 KB; else whole rows, straight from HBM.  Buckets against
+// rows, twelve to sixteen pairs an expert | more, over 1900 problems: bf16 rows of 512 bytes 1.86 | 1.63, 1 KB 1.15 | 1.05, 1152 1.60 | 1.44,
+// 1536 1.27 | 1.16, 1792 1.07 | 1.05, 2 KB 0.96 | 0.88, 4 KB 0.89 | 0.79; fp16 the same; fp32 1 KB 1.01 | 0.98, 1152 1.17 | 1.12, 1408 1.10
+// | 1.02, 1536 0.98 | 0.95, 1792 0.99 | 0.91, 2 KB 0.94 | 0.87.
 int choose_schedule(int algo, int64_t T_, int H, int64_t E, int K, int dtype, bool scored = true) {
     if (K == 0) return FMOE_EXPERT_ROWS;
     if (algo != FMOE_EXPERT_AUTO) return algo;
@@ -1529,29 +1541,38 @@ int choose_schedule(int algo, int64_t T_, int H, int64_t E, int K, int dtype, bo
     const ChipInfo& chip = chip_info();
     const int64_t pairs = T_ * K, row = (int64_t)H * (int64_t)elt, l2 = chip.l2_bytes;
     const bool rows = rows_possible(H, elt), slices = slices_possible(E, H, elt), on_lines = row % 128 == 0, many = pairs >= (1ll << 16);
-    const bool fits = E * 256 <= l2, halves_fit = on_lines && E * 128 <= (row >= 4096 ? 1 : 2) * l2;      // a slice, or one of 128 bytes
+    const bool fp32 = dtype == FMOE_F32, wide = !fp32 && row >= 4096;
+    const bool fits = E * 256 <= l2, halves_fit = on_lines && E * 128 <= (wide ? 1 : 2) * l2;      // a slice, or one of 128 bytes
     // grouping by expert serves the score phase; an op without scores (product-key memory) has nothing to group
-    const bool buckets = scored && many && pairs >= 12 * E && (row >= 2048 || row == 1024 || E >= (1ll << 17)) && bucketed_possible(T_, E, H, K, elt);
-    if (many && slices && (!fits || (!on_lines && E * 384 > l2 && K >= 100))) {
+    const bool buckets = scored && many && pairs >= 12 * E && row >= (fp32 ? 1536 : 2048) && bucketed_possible(T_, E, H, K, elt);
+    if (many && slices && K >= 24 && (!fits || (!on_lines && E * 384 > l2 && K >= 100)) && ordered_possible(E, H, K, elt)) {
         const int num_slices = (int)((row + 255) / 256);
         const bool shared = num_slices < chip.xcds;
         const int parts = shared ? slice_parts(num_slices, chip.xcds) : 1;
-        const bool busy = !shared || 8 * num_slices * parts >= 7 * chip.xcds;
-        const int64_t tokens = T_ / parts;
-        const double named = (double)(tokens < 2560 ? tokens : 2560) * K, width = (double)E * (double)E / K;
-        const bool in_step = on_lines ? named >= (row >= 3072 ? 2.0 : 1.3) * (double)E && width <= (buckets || shared ? 80.0e6 : 144.0e6) : named >= 4.0 * (double)E && width <= 16.0e6;
-        const int least = on_lines && (shared || (row < 4096 && halves_fit)) ? 100 : 24;
-        const bool small_slices = shared && on_lines && E * 128 <= (row <= 512 ? 2 : 1) * l2;
-        if (in_step && busy && K >= least && !small_slices && ordered_possible(E, H, K, elt)) return FMOE_EXPERT_ORDERED;
+        const double in_work = shared ? (double)(num_slices * parts) / chip.xcds : 1.0, width = (double)E * (double)E / K;
+        if (E * (on_lines ? 128 : 384) > 2 * l2) {
+            const double named = (double)(T_ < 2560 ? T_ : 2560) * K, share = in_work * in_work;
+            const double most = on_lines ? (buckets ? 80.0e6 : 144.0e6) : 30.0e6;
+            if ((named * share >= (on_lines ? 1.1 : 4.0) * (double)E && width <= most * share) ||
+                (T_ <= 512 && K >= 100 && named >= (double)E && width <= 144.0e6))
+                return FMOE_EXPERT_ORDERED;
+        } else {
+            const int64_t tokens = T_ / parts;
+            const double named = (double)(tokens < 2560 ? tokens : 2560) * K;
+            const bool in_step = on_lines ? named >= (row >= 3072 ? 2.0 : 1.3) * (double)E && width <= (buckets || shared ? 80.0e6 : 144.0e6) : named >= 4.0 * (double)E && width <= 16.0e6;
+            const int least = on_lines && (shared || (!wide && halves_fit)) ? 100 : 24;
+            const bool small_slices = shared && on_lines && E * 128 <= (row <= 512 ? 2 : 1) * l2;
+            if (in_step && 8 * in_work >= 7 && K >= least && !small_slices) return FMOE_EXPERT_ORDERED;
+        }
     }
+    const int least = fp32 ? 10 : 12;
     if (slices && fits) {
-        const bool resident = 2 * E * row * 4 <= 5 * l2 && row >= 1024;
-        const bool coef32 = dtype != FMOE_BF16 || !scored;
-        const bool pay = (many || (coef32 && pairs * row >= 128000000)) && (K >= 12 || (row >= 4096 && !resident)) &&
+        const bool resident = 2 * E * row * 4 <= 5 * l2 && row >= 1024, coef32 = dtype != FMOE_BF16 || !scored;
+        const bool pay = (many || (coef32 && pairs * row >= 128000000)) && (K >= least || (row >= 4096 && !resident)) &&
                          (on_lines || pairs * row >= 150000000 || K >= 64) && !(resident && K < 128 && (pairs < (1ll << 17) || K < 16));
         return pay || !rows ? FMOE_EXPERT_SLICES : FMOE_EXPERT_ROWS;
     }
-    const bool pay = on_lines ? many && halves_fit && K >= (row <= 1024 && pairs < (1ll << 18) ? 24 : 12)
+    const bool pay = on_lines ? many && halves_fit && K >= (!fp32 && row <= 1024 && pairs < (1ll << 18) ? 24 : least)
                               : E * 192 <= l2 && K >= 24 && pairs >= (1ll << 18);
     if (slices && (pay || !rows)) return FMOE_EXPERT_SLICES;
     return buckets ? FMOE_EXPERT_BUCKETS : FMOE_EXPERT_ROWS;

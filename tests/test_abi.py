@@ -241,6 +241,26 @@ def test_few_bf16_pairs_of_long_rows_keep_fp32_coefficients(T, H, E, K):
     assert lib.fmoe_pkm_workspace_bytes(T, H, E, K, _C.BF16) > 0
 
 
+@pytest.mark.parametrize("T,H,E,K,dtype,schedule", [
+    # grouping by expert: rows from 2 KB on, in fp32 from 1.5 KB, a dozen pairs per expert, however many experts
+    (24600, 256, 131072, 64, "BF16", "ROWS"), (25000, 640, 200000, 96, "F16", "ROWS"), (32768, 512, 102400, 64, "BF16", "ROWS"),
+    (32768, 896, 102400, 64, "BF16", "ROWS"), (32768, 1024, 102400, 64, "BF16", "BUCKETS"), (32768, 1024, 102400, 64, "F16", "BUCKETS"),
+    (32768, 352, 102400, 64, "F32", "ROWS"), (32768, 384, 102400, 64, "F32", "BUCKETS"), (19000, 384, 102400, 64, "F32", "ROWS"),
+    # ordered lists where no slice fits: few tokens with many experts; rows of three, five and six slices; rows between lines
+    (282, 384, 120943, 757, "BF16", "ORDERED"), (286, 256, 144100, 540, "F16", "ORDERED"), (2172, 384, 101688, 535, "F16", "ORDERED"),
+    (1097, 736, 66109, 816, "BF16", "ORDERED"), (2107, 336, 25869, 881, "F16", "ORDERED"), (282, 384, 120943, 400, "BF16", "ROWS"),
+    (3118, 640, 100000, 64, "BF16", "ROWS"), (282, 384, 120943, 99, "BF16", "ROWS"),
+    # slices in fp32: from ten experts per token on, and for rows of 4 KB of more than 32768 experts
+    (16384, 1024, 16000, 9, "F16", "ROWS"), (16384, 480, 16000, 11, "F32", "SLICES"), (16384, 960, 16000, 11, "F16", "ROWS"),
+    (6348, 1216, 53917, 31, "F32", "SLICES"), (7000, 2048, 50000, 31, "BF16", "ROWS"),
+])
+def test_expert_schedule_at_the_lines_of_its_rule(T, H, E, K, dtype, schedule):
+    lib, code = _C.lib(), getattr(_C, dtype)
+    want = lib.fmoe_expert_workspace_bytes_algo(T, H, E, K, code, getattr(_C, "EXPERT_" + schedule))
+    assert lib.fmoe_expert_workspace_bytes(T, H, E, K, code) == want and (want > 0) == (schedule != "ROWS")
+    assert (lib.fmoe_expert_saved_bytes(T, H, E, K, code) > 0) == (schedule in ("SLICES", "ORDERED"))
+
+
 def test_expert_workspace_is_enough_for_both_forwards():
     """The forward of a training step may take the ordered lists where the other takes buckets: one size for both."""
     lib = _C.lib()
