@@ -247,11 +247,14 @@ __global__ __launch_bounds__(kOrderWaves* kWave) void bucket_order_kernel(
 // writes its pairs behind its own offsets), and one workgroup per coarse bucket finishes it in LDS (counts per expert,
 // scan = the expert offsets, slots handed out by LDS cursors).  Pairs with an id outside [0, E) form one more bucket at the
 // end, whose slots are the zeroed tail.  The order inside an expert's segment is whatever the LDS serves first, or (ASCENDING) each
-// segment is put in ascending pair index there: a pair counts the smaller ones of a short segment, a long one is sorted.
+// segment is put in ascending pair index there (order_groups); a bucket that LDS does not hold goes through it in chunks of whole tiles,
+// which lie in ascending order in it, each appended to the segments behind the one before.  8388608 pairs of 102400 experts, 10500 a bucket:
+// 219 us (segment after segment by the whole workgroup 1610); 4194304 of 262144, bucket loads by a bell curve, 128 (1480).
 // Against clearing, counting, filling and ordering with global atomics, us: 524288 pairs of 102400 experts 84 -> 30, 262144 of 16384
 // 38 -> 23.
+constexpr int kPartMaxTile = 8192;
 // pairs per workgroup of the partition passes: long runs per (tile, bucket) for millions of pairs, more workgroups for fewer
-inline int partition_tile(int64_t num_pairs) { return num_pairs >= (1ll << 21) ? 8192 : 2048; }
+inline int partition_tile(int64_t num_pairs) { return num_pairs >= (1ll << 21) ? kPartMaxTile : 2048; }
 constexpr int kPartMaxBuckets = 1024;    // coarse buckets, not counting the one for invalid ids
 constexpr int kPartMaxShift = 13;        // 2^13 experts per coarse bucket: 32 KiB of LDS counters
 
@@ -313,6 +316,7 @@ __global__ __launch_bounds__(kPartThreads) void partition_scatter_kernel(const i
 
 constexpr int kPartLocalThreads = 512;
 constexpr int kPartLocalCap = 8192;      // pairs of a coarse bucket that are put in order in LDS and written out coalesced
+static_assert(kPartMaxTile <= kPartLocalCap, "what a tile gives a bucket fits LDS");
 
 // keys[0 .. n) ascending, by the whole workgroup: a bitonic network whose blocks all run in one direction, so that the places beyond
 // n act as keys above all others without being there.
@@ -343,64 +347,98 @@ __device__ inline void sort_segment(uint32_t* keys, int n) {
     }
 }
 
-// Ascending pair index in every segment of experts [e0, e0 + n_e), whose cursors ends[] stand at the ends of their segments and whose
-// pairs begin at slot `begin`.  in_lds: the pairs are in out_pair (expert e0 + out_low), segment by segment, and go to sorted_pairs;
-// otherwise they are there already, in any order.  CAP: entries of out_pair.
-constexpr int kPartRank = 64;            // longest segment ordered by counting
-template <int CAP>
-__device__ inline void order_segments(const int64_t* __restrict__ indices, int64_t num_pairs, int32_t* __restrict__ sorted_pairs,
-                                      const int32_t* ends, uint32_t* out_pair, const uint16_t* out_low, bool in_lds, int32_t begin,
-                                      int32_t end, int64_t e0, int n_e, int top_k) {
-    constexpr int NT = kPartLocalThreads;
-    __shared__ int32_t long_ones;
-    __shared__ int32_t wave_count[kWalkBatch][NT / kWave];
-    const int tid = (int)threadIdx.x;
-    if (tid == 0) long_ones = in_lds ? 0 : 1;
+// keys[0 .. n), all different and in [lo, lo + span), in ascending order to out[]: by the whole workgroup, a key's place is the number of
+// bits below its own.  A group of 8192 keys takes some 3 us so, in the network above 110.  scratch: kBitsBytes of LDS.
+constexpr int kBitsSpan = 1 << 16, kBitsBytes = kBitsSpan / 8 + kBitsSpan / 16;
+__device__ inline void place_by_bits(const uint32_t* keys, int n, uint32_t lo, int span, int32_t* __restrict__ out, void* scratch) {
+    constexpr int NT = kPartLocalThreads, PER = kBitsSpan / 32 / NT;
+    uint32_t* bits = static_cast<uint32_t*>(scratch);
+    uint16_t* before = reinterpret_cast<uint16_t*>(bits + kBitsSpan / 32);
+    __shared__ int32_t wave_bits[NT / kWave];
+    const int tid = (int)threadIdx.x, lane = tid & (kWave - 1), wave = tid >> 6, words = (span + 31) / 32;
+    for (int w = tid; w < words; w += NT) bits[w] = 0;
     __syncthreads();
-    auto start_of = [&](int j) { return j > 0 ? ends[j - 1] : begin; };
-    if (in_lds) {
-        for (int32_t i = tid; i < end - begin; i += NT) {
-            const uint32_t p = out_pair[i];
-            const int low = out_low[i];
-            const int32_t from = start_of(low), n = ends[low] - from;
-            if (n <= kPartRank) {
-                int rank = 0;
-                for (int q = 0; q < n; ++q) rank += out_pair[from - begin + q] < p ? 1 : 0;
-                sorted_pairs[from + rank] = (int32_t)p;
-            } else {
-                long_ones = 1;
-            }
-        }
+    for (int i = tid; i < n; i += NT) {
+        const uint32_t d = keys[i] - lo;
+        atomicOr(&bits[d >> 5], 1u << (d & 31));
     }
     __syncthreads();
-    if (long_ones == 0) return;
-    for (int j = 0; j < n_e; ++j) {          // the same for every thread of the workgroup
-        const int32_t from = start_of(j), n = ends[j] - from;
-        if (n <= (in_lds ? kPartRank : 1)) continue;
-        if (n > CAP) {
-            walk_segment<NT / kWave>(indices, num_pairs, e0 + j, from, sorted_pairs, nullptr, top_k, 1u, wave_count);
-            continue;
-        }
-        uint32_t* keys = in_lds ? out_pair + (from - begin) : out_pair;
-        if (!in_lds)
-            for (int i = tid; i < n; i += NT) keys[i] = (uint32_t)sorted_pairs[from + i];
-        __syncthreads();
-        sort_segment(keys, n);
-        for (int i = tid; i < n; i += NT) sorted_pairs[from + i] = (int32_t)keys[i];
-        __syncthreads();
+    int32_t mine = 0;
+    for (int w = tid * PER; w < tid * PER + PER && w < words; ++w) mine += __popc(bits[w]);
+    int32_t incl = mine;
+#pragma unroll
+    for (int d = 1; d < kWave; d <<= 1) {
+        const int32_t up = __shfl_up(incl, d, kWave);
+        if (lane >= d) incl += up;
     }
+    if (lane == kWave - 1) wave_bits[wave] = incl;
+    __syncthreads();
+    int32_t run = incl - mine;
+    for (int w = 0; w < wave; ++w) run += wave_bits[w];
+    for (int w = tid * PER; w < tid * PER + PER && w < words; ++w) {
+        before[w] = (uint16_t)run;
+        run += __popc(bits[w]);
+    }
+    __syncthreads();
+    for (int i = tid; i < n; i += NT) {
+        const uint32_t d = keys[i] - lo;
+        out[before[d >> 5] + __popc(bits[d >> 5] & ((1u << (d & 31)) - 1u))] = (int32_t)keys[i];
+    }
+    __syncthreads();
 }
 
-// Segments of n_e experts from their counts: ends[j] becomes the slot where segment j starts (its cursor), as offsets[e0 + j] does.
-__device__ inline void start_segments(int32_t* ends, int32_t* __restrict__ offsets, int64_t e0, int n_e, int32_t begin,
-                                      int32_t* wave_total) {
+// Ascending pair index inside every group of a chunk: its n pairs, of [lo, lo + span), lie in pair[] (expert e0 + low[]) group by group,
+// group j up to group_end(j), and go to sorted_pairs from first_slot(j) on.  A pair of a short group counts the smaller ones (n keys a pair,
+// but without a barrier); long groups, at most CAP / kPartRank, follow one after the other, by their bits where the span allows, which take
+// the place of low[].
+// Longest group that counts, us with 64 | 128 | 256 | 512 | 1024: 262144 pairs of 16384 experts, up to 101 each 194 | 31 | 31 | 31 | 31;
+// 1048576, up to 362 182 | 179 | 179 | 97 | 97; 60000 of 300 34 | 34 | 31 | 24 | 24; 10455 of 4100, one of 698 51 | 33 | 27 | 27 | 37.
+constexpr int kPartRank = 512;
+template <int CAP, typename End, typename Slot>
+__device__ inline void order_groups(uint32_t* pair, uint16_t* low, int n, uint32_t lo, int64_t span, int32_t* __restrict__ sorted_pairs,
+                                    End group_end, Slot first_slot) {
+    constexpr int NT = kPartLocalThreads;
+    static_assert(CAP * sizeof(uint16_t) >= kBitsBytes, "the bits take the place of low[]");
+    __shared__ int32_t long_ones[CAP / kPartRank + 1];
+    __shared__ int32_t num_long;
+    const int tid = (int)threadIdx.x;
+    if (tid == 0) num_long = 0;
+    __syncthreads();
+    for (int i = tid; i < n; i += NT) {
+        const uint32_t p = pair[i];
+        const int j = low[i], from = j > 0 ? group_end(j - 1) : 0, m = group_end(j) - from;
+        if (m <= kPartRank) {
+            int rank = 0;
+#pragma unroll 4
+            for (int q = 0; q < m; ++q) rank += pair[from + q] < p ? 1 : 0;
+            sorted_pairs[first_slot(j) + rank] = (int32_t)p;
+        } else if (i == from) {
+            long_ones[atomicAdd(&num_long, 1)] = j;
+        }
+    }
+    __syncthreads();
+    for (int l = 0; l < num_long; ++l) {          // the same for every thread of the workgroup
+        const int j = long_ones[l], from = j > 0 ? group_end(j - 1) : 0, m = group_end(j) - from;
+        if (span <= kBitsSpan) {
+            place_by_bits(pair + from, m, lo, (int)span, sorted_pairs + first_slot(j), low);
+        } else {
+            sort_segment(pair + from, m);
+            for (int i = tid; i < m; i += NT) sorted_pairs[first_slot(j) + i] = (int32_t)pair[from + i];
+        }
+    }
+    __syncthreads();
+}
+
+// counts[0 .. n_e) becomes where each group starts when the first starts at `begin`; start(j, slot) is called for each.
+template <typename Start>
+__device__ inline void scan_groups(int32_t* counts, int n_e, int32_t begin, int32_t* wave_total, Start start) {
     constexpr int NT = kPartLocalThreads;
     const int tid = (int)threadIdx.x, lane = tid & (kWave - 1), wave = tid >> 6;
-    // thread t owns experts [t * per, (t + 1) * per)
+    // thread t owns groups [t * per, (t + 1) * per)
     const int per = (n_e + NT - 1) / NT;
     const int j0 = tid * per < n_e ? tid * per : n_e, j1 = j0 + per < n_e ? j0 + per : n_e;
     int32_t mine = 0;
-    for (int j = j0; j < j1; ++j) mine += ends[j];
+    for (int j = j0; j < j1; ++j) mine += counts[j];
     int32_t incl = mine;
 #pragma unroll
     for (int d = 1; d < kWave; d <<= 1) {
@@ -412,23 +450,46 @@ __device__ inline void start_segments(int32_t* ends, int32_t* __restrict__ offse
     int32_t run = begin + incl - mine;
     for (int w = 0; w < wave; ++w) run += wave_total[w];
     for (int j = j0; j < j1; ++j) {
-        const int32_t c = ends[j];
-        offsets[e0 + j] = run;
-        ends[j] = run;
+        const int32_t c = counts[j];
+        start(j, run);
+        counts[j] = run;
         run += c;
     }
+    __syncthreads();
+}
+
+// One chunk of a workgroup's pairs, all of them above the chunks before it: the pairs are counted per expert (fill(f) calls f(pair, low)
+// for each of them, twice over), placed group by group and appended in ascending order behind the segments' cursors.
+template <int CAP, typename Fill>
+__device__ inline void append_chunk(uint32_t* pair, uint16_t* low, int32_t* counts, int32_t* cursors, int n, uint32_t lo, int64_t span, int n_e,
+                                    int32_t* __restrict__ sorted_pairs, int32_t* wave_total, Fill fill) {
+    constexpr int NT = kPartLocalThreads;
+    const int tid = (int)threadIdx.x;
+    for (int j = tid; j < n_e; j += NT) counts[j] = 0;
+    __syncthreads();
+    fill([&](uint32_t, int j) { atomicAdd(&counts[j], 1); });
+    __syncthreads();
+    scan_groups(counts, n_e, 0, wave_total, [](int, int32_t) {});
+    fill([&](uint32_t p, int j) {
+        const int32_t slot = atomicAdd(&counts[j], 1);
+        pair[slot] = p;
+        low[slot] = (uint16_t)j;
+    });
+    __syncthreads();
+    order_groups<CAP>(pair, low, n, lo, span, sorted_pairs, [&](int j) { return counts[j]; }, [&](int j) { return cursors[j]; });
+    for (int j = tid; j < n_e; j += NT) cursors[j] += counts[j] - (j > 0 ? counts[j - 1] : 0);
     __syncthreads();
 }
 
 // ASCENDING writes sorted_pairs only (tok and exp NULL).
 template <bool ASCENDING>
 __global__ __launch_bounds__(kPartLocalThreads) void partition_local_kernel(
-    const int64_t* __restrict__ indices, int64_t num_pairs, const uint64_t* __restrict__ stage, const int32_t* __restrict__ offs1, int32_t* __restrict__ offsets,
+    const uint64_t* __restrict__ stage, const int32_t* __restrict__ offs1, int32_t* __restrict__ offsets,
     int32_t* __restrict__ sorted_pairs, uint32_t* __restrict__ tok, uint32_t* __restrict__ exp, int64_t num_experts, int shift,
-    int buckets, int groups, int top_k, uint32_t tok_scale, uint32_t exp_scale, int pack_shift) {
-    extern __shared__ int32_t cnt[];     // 1 << shift
+    int buckets, int groups, int tile, int top_k, uint32_t tok_scale, uint32_t exp_scale, int pack_shift) {
+    extern __shared__ int32_t cnt[];     // 1 << shift; ASCENDING: as many again for the counts of a chunk
     __shared__ uint32_t out_pair[kPartLocalCap];
-    __shared__ uint16_t out_low[kPartLocalCap];
+    __shared__ __attribute__((aligned(16))) uint16_t out_low[kPartLocalCap];
     __shared__ int32_t wave_total[kPartLocalThreads / kWave];
     constexpr int NT = kPartLocalThreads;
     const int b = (int)blockIdx.x, tid = (int)threadIdx.x;
@@ -451,15 +512,47 @@ __global__ __launch_bounds__(kPartLocalThreads) void partition_local_kernel(
         if (s + NT < end) atomicAdd(&cnt[(uint32_t)v1], 1);
     }
     __syncthreads();
-    start_segments(cnt, offsets, e0, n_e, begin, wave_total);
+    scan_groups(cnt, n_e, begin, wave_total, [&](int j, int32_t slot) { offsets[e0 + j] = slot; });
     auto emit = [&](int32_t slot, uint32_t p, uint32_t low) {
         const uint32_t e = (uint32_t)e0 + low;
         sorted_pairs[slot] = (int32_t)p;
         if (tok != nullptr) tok[slot] = (p / (uint32_t)top_k) * tok_scale | (pack_shift ? e << pack_shift : 0u);
         if (exp != nullptr) exp[slot] = e * exp_scale;
     };
-    const bool in_lds = end - begin <= kPartLocalCap;      // else (a few experts took a large share of all pairs): slot by slot
-    for (int32_t s = begin + tid; s < end; s += 2 * NT) {
+    const bool in_lds = end - begin <= kPartLocalCap;
+    if constexpr (ASCENDING) {
+        if (!in_lds) {
+            // the runs that the tiles wrote lie in ascending order here, so as many whole runs as LDS holds are a chunk; a run never
+            // exceeds it (partition_tile)
+            __shared__ int32_t run_s, stop_s;
+            int32_t from = begin;
+            for (int g = 0; g < groups;) {
+                const int last = g + 1 + tid;      // one thread finds the last run of the chunk
+                auto holds = [&](int r) { return r <= groups && offs1[(int64_t)b * groups + r] - from <= kPartLocalCap; };
+                const bool here = holds(last), next = holds(last + 1);
+                if (here && (tid == NT - 1 || !next)) {
+                    run_s = last;
+                    stop_s = offs1[(int64_t)b * groups + last];
+                }
+                __syncthreads();
+                const int run = run_s;
+                const int32_t stop = stop_s;
+                if (stop > from)
+                    append_chunk<kPartLocalCap>(out_pair, out_low, cnt + (1 << shift), cnt, stop - from, (uint32_t)g * (uint32_t)tile,
+                                                (int64_t)(run - g) * tile, n_e, sorted_pairs, wave_total, [&](auto f) {
+                                                    for (int32_t s = from + tid; s < stop; s += NT) {
+                                                        const uint64_t v = stage[s];
+                                                        f((uint32_t)(v >> 32), (int)(uint32_t)v);
+                                                    }
+                                                });
+                g = run;
+                from = stop;
+                __syncthreads();
+            }
+            return;
+        }
+    }
+    for (int32_t s = begin + tid; s < end; s += 2 * NT) {      // not in LDS (a few experts took a large share of all pairs): slot by slot
         const bool two = s + NT < end;
         const uint64_t v0 = stage[s], v1 = two ? stage[s + NT] : 0;
         const int32_t slot0 = atomicAdd(&cnt[(uint32_t)v0], 1);
@@ -478,7 +571,8 @@ __global__ __launch_bounds__(kPartLocalThreads) void partition_local_kernel(
     }
     __syncthreads();
     if constexpr (ASCENDING) {
-        order_segments<kPartLocalCap>(indices, num_pairs, sorted_pairs, cnt, out_pair, out_low, in_lds, begin, end, e0, n_e, top_k);
+        order_groups<kPartLocalCap>(out_pair, out_low, end - begin, 0u, (int64_t)groups * tile, sorted_pairs,
+                                    [&](int j) { return cnt[j] - begin; }, [&](int j) { return j > 0 ? cnt[j - 1] : begin; });
     } else {
         if (!in_lds) return;
         for (int32_t i = tid; i < end - begin; i += NT) emit(begin + i, out_pair[i], out_low[i]);
@@ -489,16 +583,19 @@ __global__ __launch_bounds__(kPartLocalThreads) void partition_local_kernel(
 // For fewer pairs every workgroup reads all ids (from the L2) and keeps those of its own 2^shift experts: what it counts of lower experts
 // is where its segments begin, the rest happens in LDS as above.  One launch in place of clearing, scan, fill and ordering, and
 // nothing to count elsewhere: 10455 pairs of 4100 experts 15.5 -> 7.1 us.
-constexpr int kOneCap = 4096;            // pairs of a workgroup's experts that are put in order in LDS
+// LDS holds 6144 pairs of a workgroup's experts: with 4096 a chunk of those beyond was a single block of ids, and 60000 pairs of which one of
+// 300 experts has a seventh took 114 us for 81.
+constexpr int kOneCap = 6144;
 constexpr int kOneBatch = 8;             // loads in flight per thread
 constexpr int kOneMaxGroups = 256;
 
 __global__ __launch_bounds__(kPartLocalThreads) void group_pairs_kernel(const int64_t* __restrict__ indices, int32_t* __restrict__ offsets,
                                                                        int32_t* __restrict__ sorted_pairs, int64_t num_pairs,
-                                                                       int64_t num_experts, int top_k, int shift) {
-    extern __shared__ int32_t cnt[];     // 1 << shift
+                                                                       int64_t num_experts, int shift) {
+    extern __shared__ int32_t cnt[];     // 1 << shift, and as many again for the counts of a chunk
     __shared__ uint32_t out_pair[kOneCap], in_pair[kOneCap];
-    __shared__ uint16_t out_low[kOneCap], in_low[kOneCap];
+    __shared__ __attribute__((aligned(16))) uint16_t out_low[kOneCap];
+    __shared__ uint16_t in_low[kOneCap];
     __shared__ int32_t wave_total[kPartLocalThreads / kWave], wave_below[kPartLocalThreads / kWave];
     __shared__ int32_t mine_s;
     constexpr int NT = kPartLocalThreads;
@@ -508,13 +605,13 @@ __global__ __launch_bounds__(kPartLocalThreads) void group_pairs_kernel(const in
     for (int j = tid; j < n_e; j += NT) cnt[j] = 0;
     if (tid == 0) mine_s = 0;
     __syncthreads();
-    // f(pair, low) for every pair of the workgroup's experts; returns the thread's pairs of lower ones
-    auto scan_ids = [&](auto f) {
+    // f(pair, low) for every pair of the workgroup's experts in [from, stop); returns the thread's pairs of lower ones
+    auto scan_ids = [&](int64_t from, int64_t stop, auto f) {
         int32_t below = 0;
-        for (int64_t p0 = tid; p0 < num_pairs; p0 += kOneBatch * NT) {
+        for (int64_t p0 = from + tid; p0 < stop; p0 += kOneBatch * NT) {
             int64_t e[kOneBatch];
 #pragma unroll
-            for (int u = 0; u < kOneBatch; ++u) e[u] = p0 + u * NT < num_pairs ? indices[p0 + u * NT] : -1;
+            for (int u = 0; u < kOneBatch; ++u) e[u] = p0 + u * NT < stop ? indices[p0 + u * NT] : -1;
 #pragma unroll
             for (int u = 0; u < kOneBatch; ++u) {
                 below += e[u] >= 0 && e[u] < e0 ? 1 : 0;
@@ -523,7 +620,7 @@ __global__ __launch_bounds__(kPartLocalThreads) void group_pairs_kernel(const in
         }
         return below;
     };
-    int32_t below = scan_ids([&](uint32_t p, int low) {
+    int32_t below = scan_ids(0, num_pairs, [&](uint32_t p, int low) {
         atomicAdd(&cnt[low], 1);
         const int32_t at = atomicAdd(&mine_s, 1);
         if (at < kOneCap) {
@@ -537,20 +634,48 @@ __global__ __launch_bounds__(kPartLocalThreads) void group_pairs_kernel(const in
     __syncthreads();
     int32_t begin = 0;
     for (int w = 0; w < NT / kWave; ++w) begin += wave_below[w];
-    const int32_t mine = mine_s, end = begin + mine;
-    start_segments(cnt, offsets, e0, n_e, begin, wave_total);
-    if (tid == 0 && e0 + n_e == num_experts) offsets[num_experts] = end;
-    const bool in_lds = mine <= kOneCap;
-    if (in_lds)
+    const int32_t mine = mine_s;
+    scan_groups(cnt, n_e, begin, wave_total, [&](int j, int32_t slot) { offsets[e0 + j] = slot; });
+    if (tid == 0 && e0 + n_e == num_experts) offsets[num_experts] = begin + mine;
+    if (mine <= kOneCap) {
         for (int32_t i = tid; i < mine; i += NT) {
             const int32_t slot = atomicAdd(&cnt[in_low[i]], 1) - begin;
             out_pair[slot] = in_pair[i];
             out_low[slot] = in_low[i];
         }
-    else
-        scan_ids([&](uint32_t p, int low) { sorted_pairs[atomicAdd(&cnt[low], 1)] = (int32_t)p; });
-    __syncthreads();
-    order_segments<kOneCap>(indices, num_pairs, sorted_pairs, cnt, out_pair, out_low, in_lds, begin, end, e0, n_e, top_k);
+        __syncthreads();
+        order_groups<kOneCap>(out_pair, out_low, mine, 0u, num_pairs, sorted_pairs, [&](int j) { return cnt[j] - begin; },
+                              [&](int j) { return j > 0 ? cnt[j - 1] : begin; });
+        return;
+    }
+    // more than LDS holds: a chunk takes block after block of ids while the next one surely fits
+    constexpr int kBlock = kOneBatch * NT;
+    static_assert(kBlock <= kOneCap, "a block of ids fits LDS");
+    for (int64_t from = 0; from < num_pairs;) {
+        if (tid == 0) mine_s = 0;
+        __syncthreads();
+        int64_t stop = from;
+        int n = 0;
+        do {
+            const int64_t next = stop + kBlock < num_pairs ? stop + kBlock : num_pairs;
+            scan_ids(stop, next, [&](uint32_t p, int low) {
+                const int32_t at = atomicAdd(&mine_s, 1);
+                in_pair[at] = p;
+                in_low[at] = (uint16_t)low;
+            });
+            __syncthreads();
+            n = mine_s;
+            stop = next;
+            __syncthreads();
+        } while (stop < num_pairs && n + kBlock <= kOneCap);
+        if (n > 0)
+            append_chunk<kOneCap>(out_pair, out_low, cnt + (1 << shift), cnt, n, (uint32_t)from, stop - from, n_e, sorted_pairs, wave_total,
+                                  [&](auto f) {
+                                      for (int i = tid; i < n; i += NT) f(in_pair[i], (int)in_low[i]);
+                                  });
+        from = stop;
+        __syncthreads();
+    }
 }
 
 struct PartitionPlan {
@@ -629,9 +754,9 @@ int bucket_partition(const int64_t* indices, void* workspace, int64_t num_pairs,
                        (const int32_t*)offs1, stage, coef_clear, num_pairs, num_experts, p.shift, p.buckets, p.groups, p.tile);
     FMOE_CHECK_LAUNCH("expert bucketing (partition scatter)");
 #define FMOE_LAUNCH_LOCAL(ASCENDING)                                                                                                    \
-    hipLaunchKernelGGL((partition_local_kernel<ASCENDING>), dim3((unsigned)(p.buckets + 1)), dim3(kPartLocalThreads), (size_t)4 << p.shift, \
-                       stream, indices, num_pairs, (const uint64_t*)stage, (const int32_t*)offs1, offsets, sorted_pairs, tok, exp,      \
-                       num_experts, p.shift, p.buckets, p.groups, top_k, tok_scale, exp_scale, pack_shift)
+    hipLaunchKernelGGL((partition_local_kernel<ASCENDING>), dim3((unsigned)(p.buckets + 1)), dim3(kPartLocalThreads),                   \
+                       (size_t)(ASCENDING ? 8 : 4) << p.shift, stream, (const uint64_t*)stage, (const int32_t*)offs1, offsets,          \
+                       sorted_pairs, tok, exp, num_experts, p.shift, p.buckets, p.groups, p.tile, top_k, tok_scale, exp_scale, pack_shift)
     if (ascending) FMOE_LAUNCH_LOCAL(true);
     else FMOE_LAUNCH_LOCAL(false);
 #undef FMOE_LAUNCH_LOCAL
@@ -654,8 +779,8 @@ int group_pairs(const int64_t* indices, void* workspace, int64_t num_pairs, int6
         int shift = 0;
         while ((num_experts + (1ll << shift) - 1) >> shift > kOneMaxGroups) ++shift;
         const unsigned groups = (unsigned)((num_experts + (1ll << shift) - 1) >> shift);
-        hipLaunchKernelGGL(group_pairs_kernel, dim3(groups), dim3(kPartLocalThreads), (size_t)4 << shift, stream, indices, offsets,
-                           sorted_pairs, num_pairs, num_experts, top_k, shift);
+        hipLaunchKernelGGL(group_pairs_kernel, dim3(groups), dim3(kPartLocalThreads), (size_t)8 << shift, stream, indices, offsets,
+                           sorted_pairs, num_pairs, num_experts, shift);
         FMOE_CHECK_LAUNCH("expert bucketing (one launch)");
         return FMOE_OK;
     }

@@ -310,7 +310,7 @@ def test_expert_backward_c4_tables_fewer_tokens():
         assert fro < GRAD_FRO[dtype], f"{name}: relative Frobenius error {fro:.3e}"
 
 
-@pytest.mark.parametrize("E,ids", [(40000, "spread"), (300, "spread"), (3, "spread"), (5000, "warm"), (5000, "hot")])
+@pytest.mark.parametrize("E,ids", [(40000, "spread"), (300, "spread"), (3, "spread"), (5000, "warm"), (5000, "hot"), (700, "warm")])
 def test_expert_backward_groups_pairs_alike_in_both_ways(E, ids):
     # 65536 pairs are grouped by two partition passes, 64512 in one launch; the last pair of every token names no expert, so both calls
     # sum the same pairs and, each in ascending pair index, to the same bits.  Segments that a pair ranks itself in, that are sorted in
@@ -342,6 +342,49 @@ def test_expert_backward_groups_pairs_alike_in_both_ways(E, ids):
     act = torch.nn.functional.silu(s) * gates[:, :-1].double().cpu()
     dup = torch.zeros(E, H, dtype=torch.float64).index_add_(0, ids64.flatten(), (act[..., None] * d64[:, None]).flatten(0, 1))
     torch.testing.assert_close(whole[1].double().cpu(), dup, rtol=1e-4, atol=1e-5 * float(dup.abs().max()))
+
+
+@pytest.mark.parametrize("T,K,E,power,most_ms", [(16384, 512, 102400, 1, 2.1), (16384, 512, 102400, 3, 60), (16384, 129, 20000, 3, 25),
+                                                 (1024, 64, 1500, 2, 2.1)])
+def test_expert_backward_groups_experts_whose_pairs_exceed_lds(T, K, E, power, most_ms):
+    """Coarse groups of 10000 pairs of 128 experts each; groups of 900000 and experts of 180000 pairs (ids that crowd towards expert 0);
+    tiles of 8192 and of 2048 pairs.  Weight gradients against a float64 sum over the pairs, the same bits twice, and no path on which a
+    workgroup sorts one short segment after the other or walks all ids for a long one (3.5 and 157 ms for the first two; 1.3 and 29
+    without)."""
+    from flash_moe.ops.hip.flash_expert import expert_backward
+
+    H = 8
+    g = torch.Generator(device="cuda").manual_seed(K)
+    idx = (E * torch.rand(T, K, device="cuda", generator=g, dtype=torch.float64) ** power).long().clamp_(0, E - 1)
+    idx[::5, 0] = E
+    x, dout, down, up = (torch.randn(n, H, device="cuda", generator=g) * s for n, s in ((T, 1.0), (T, 1.0), (E, 0.1), (E, 0.1)))
+    gates = torch.rand(T, K, device="cuda", generator=g)
+    args = (dout, x, down, up, idx, gates)
+    got = expert_backward(*args)
+    start, stop = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+    times = []
+    for _ in range(3):
+        start.record()
+        again = expert_backward(*args)
+        stop.record()
+        torch.cuda.synchronize()
+        times.append(start.elapsed_time(stop))
+        assert all(torch.equal(a, b) for a, b in zip(got, again))
+    print(f"\n{T} x {K} of {E}, power {power}: {min(times):.2f} ms")
+    assert min(times) < most_ms, times
+    ddown, dup = (torch.zeros(E, H, device="cuda", dtype=torch.float64) for _ in range(2))
+    for lo in range(0, T, 2048):
+        i, x64, do64, g64 = idx[lo:lo + 2048], x[lo:lo + 2048].double(), dout[lo:lo + 2048].double(), gates[lo:lo + 2048].double()
+        g64 = g64 * (i < E)
+        i = i.clamp(0, E - 1)
+        s = (down[i].double() * x64[:, None]).sum(-1)
+        sig = torch.sigmoid(s)
+        ds = (up[i].double() * do64[:, None]).sum(-1) * g64 * sig * (1 + s * (1 - sig))
+        ddown.index_add_(0, i.flatten(), (ds[..., None] * x64[:, None]).flatten(0, 1))
+        dup.index_add_(0, i.flatten(), ((s * sig * g64)[..., None] * do64[:, None]).flatten(0, 1))
+    # an fp32 sum of n products in one chain is off by up to n * 2^-24 of the sum of their magnitudes; a lost or doubled pair of an expert of
+    # n pairs by 1 / n of it.  Relative to the tensors, whose norm the sums of n such products make, 1e-4 holds for the longest here
+    assert rel_fro(got[1], ddown) < 1e-4 and rel_fro(got[2], dup) < 1e-4
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
