@@ -344,6 +344,37 @@ def test_expert_backward_groups_pairs_alike_in_both_ways(E, ids):
     torch.testing.assert_close(whole[1].double().cpu(), dup, rtol=1e-4, atol=1e-5 * float(dup.abs().max()))
 
 
+@pytest.mark.parametrize("T,K,E", [(64, 10, (1 << 21) + 5), (1024, 64, (1 << 23) + 100)])
+def test_expert_backward_groups_pairs_of_tables_beyond_the_other_ways(T, K, E):
+    """More experts than one launch or the coarse groups of the partition passes can hold (few pairs, and 65536): the pairs are grouped by
+    counters in memory, with segments of one pair, of some hundred (ordered in LDS) and of 8000 (met in order).  Weight gradients
+    against float64 sums, zeros where no token went, the same bits twice."""
+    from flash_moe import _C
+    from flash_moe.ops.hip.flash_expert import expert_backward
+
+    H = 8
+    assert _C.lib().fmoe_expert_backward_workspace_bytes(T, H, E, K, _C.F32) > 8 * E        # a counter and an offset per expert
+    g = torch.Generator(device="cuda").manual_seed(K)
+    idx = torch.randint(0, E, (T, K), device="cuda", generator=g)
+    idx[:, 1], idx[::3, 2], idx[0, 0], idx[1, 0], idx[2, 0] = 77, E - 1, 0, -1, E
+    if K == 64:
+        idx[:, 8:16] = E // 2
+    x, dout = torch.randn(T, H, device="cuda", generator=g), torch.randn(T, H, device="cuda", generator=g)
+    down, up = torch.randn(E, H, device="cuda", generator=g) * 0.1, torch.randn(E, H, device="cuda", generator=g) * 0.1
+    gates = torch.rand(T, K, device="cuda", generator=g)
+    args = (dout, x, down, up, idx, gates)
+    got = expert_backward(*args)
+    assert all(torch.equal(a, b) for a, b in zip(got, expert_backward(*args)))
+    valid = (idx >= 0) & (idx < E)
+    used, at = torch.unique(idx.clamp(0, E - 1), return_inverse=True)
+    leaves = [t.double().cpu().requires_grad_(True) for t in (down[used], up[used])]
+    orc.expert_forward(x.double().cpu(), *leaves, at.cpu(), (gates * valid).double().cpu()).backward(dout.double().cpu())
+    for grad, ref in zip(got[1:3], leaves):
+        assert rel_fro(grad[used], ref.grad) < GRAD_FRO[torch.float32]
+        grad[used] = 0
+        assert not grad.any()
+
+
 @pytest.mark.parametrize("T,K,E,power,most_ms", [(16384, 512, 102400, 1, 2.1), (16384, 512, 102400, 3, 60), (16384, 129, 20000, 3, 25),
                                                  (1024, 64, 1500, 2, 2.1)])
 def test_expert_backward_groups_experts_whose_pairs_exceed_lds(T, K, E, power, most_ms):

@@ -18,6 +18,16 @@ def run(x, wd, wu, idx, g, algo="auto"):
     return expert_forward(*cuda(x, wd, wu, idx, g), algo=ALGOS[algo]).cpu()
 
 
+def taken(T, H, E, K, dtype):
+    """The schedule a call takes by itself, by the scratch it asks for."""
+    from flash_moe import _C
+
+    sizes = [_C.lib().fmoe_expert_workspace_bytes_algo(T, H, E, K, _C.dtype_code(dtype), algo) for algo in range(5)]
+    names = [n for n, algo in (("rows", 1), ("slices", 2), ("buckets", 3), ("ordered", 4)) if sizes[algo] == sizes[0]]
+    assert len(names) == 1
+    return names[0]
+
+
 def truth64(x, wd, wu, idx, g):
     """The oracle evaluated in float64 on the (already rounded) inputs."""
     return orc.expert_forward(x.double(), wd.double(), wu.double(), idx, g.double())
@@ -319,6 +329,7 @@ def test_expert_ordered_lists(dtype, T, H, E, K):
     from flash_moe import _C
     from flash_moe.ops.hip.flash_expert import expert_forward
 
+    assert E < 65537 or taken(T, H, E, K, dtype) == "ordered"
     g = torch.Generator().manual_seed(T + K)
     x, wd, wu = (torch.randn(n, H, generator=g).mul(s).to(dtype) for n, s in ((T, 1.0), (E, 0.05), (E, 0.05)))
     idx = torch.randint(0, E, (T, K), generator=g)
@@ -382,14 +393,20 @@ def test_expert_infinite_weights_and_a_partial_last_slice(dtype, algo, T, H, E, 
     assert rel_fro(got[others], ref) < {torch.float32: 2e-6, torch.bfloat16: 5e-3, torch.float16: 6e-4}[dtype]
 
 
-@pytest.mark.parametrize("dtype,H,K", [(torch.float32, 1024, 166), (torch.bfloat16, 2048, 222), (torch.bfloat16, 2048, 223), (torch.bfloat16, 2040, 166)])
-def test_expert_forward_and_training_step_where_buckets_and_ordered_lists_both_pay(dtype, H, K):
-    """Rows of 4 KB, 400 tokens that name every expert hardly more than once, twelve pairs per expert: without gradients the forward
-    groups by expert, in a training step it walks ordered lists.  One expert per token more, and rows shorter than 4 KB, are ordered
-    in both.  Both against the float64 oracle on a sample."""
+@pytest.mark.parametrize("dtype,T,H,K,schedule", [
+    (torch.float32, 4800, 1024, 166, "ordered"), (torch.bfloat16, 4800, 2048, 222, "ordered"), (torch.bfloat16, 4800, 2048, 223, "ordered"),
+    (torch.bfloat16, 4800, 2040, 166, "ordered"), (torch.bfloat16, 4800, 2040, 140, "rows"),
+    (torch.bfloat16, 15000, 2048, 55, "ordered"), (torch.bfloat16, 15000, 2048, 54, "buckets"),
+    (torch.float32, 15000, 1024, 55, "ordered"), (torch.float32, 15000, 1024, 54, "buckets"),
+])
+def test_expert_forward_and_training_step_where_buckets_and_ordered_lists_both_pay(dtype, T, H, K, schedule):
+    """Rows of 4 KB and twelve pairs per expert: ordered lists while their window is narrow enough, with fewer experts per token the pairs are
+    grouped by expert; rows between cache lines, which are not grouped, are taken whole there.  Without gradients and in a training step,
+    both against the float64 oracle on a sample."""
     from flash_moe.ops import flash_expert_func
 
-    T, E = 4800, 66049
+    E = 66049
+    assert taken(T, H, E, K, dtype) == schedule and T * K >= (12 * E if schedule != "rows" else 0)
     g = torch.Generator().manual_seed(K)
     x, wd, wu = (torch.randn(n, H, generator=g).mul(s).to(dtype) for n, s in ((T, 1.0), (E, 0.05), (E, 0.05)))
     idx = torch.randint(0, E, (T, K), generator=g)
@@ -405,8 +422,10 @@ def test_expert_forward_and_training_step_where_buckets_and_ordered_lists_both_p
         assert rel_fro(out[sample.cuda()], ref) < tol
 
 
-@pytest.mark.parametrize("T,H,E,K", [(64, 128, 256, 8), (300, 264, 700, 230), (70, 64, 66000, 1000)])    # rows, slices, ordered lists
-def test_expert_backward_from_what_the_forward_kept(T, H, E, K):
+@pytest.mark.parametrize("T,H,E,K,schedule", [(64, 128, 256, 8, "rows"), (300, 264, 700, 230, "slices"), (70, 64, 66000, 1000, "ordered"),
+                                             (300, 96, 66000, 300, "ordered"), (513, 40, 66000, 700, "ordered")])
+def test_expert_backward_from_what_the_forward_kept(T, H, E, K, schedule):
+    assert taken(T, H, E, K, torch.float32) == schedule
     # the op's autograd keeps scores and list addresses where its schedule has them; the stand-alone backward recomputes them
     from flash_moe.ops import flash_expert_func
     from flash_moe.ops.hip.flash_expert import expert_backward
