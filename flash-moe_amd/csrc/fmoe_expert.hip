@@ -1685,11 +1685,7 @@ extern "C" size_t fmoe_expert_workspace_bytes_algo(int64_t num_tokens, int hidde
 }
 
 extern "C" size_t fmoe_expert_workspace_bytes(int64_t num_tokens, int hidden, int64_t num_experts, int top_k, int dtype) {
-    // enough for the forward of a training step as well, which may take another schedule
-    const size_t plain = fmoe_expert_workspace_bytes_algo(num_tokens, hidden, num_experts, top_k, dtype, FMOE_EXPERT_AUTO);
-    if (plain == 0 || !fmoe::expert_saved_plan(num_tokens, hidden, num_experts, top_k, dtype).ordered) return plain;
-    const size_t ordered = fmoe_expert_workspace_bytes_algo(num_tokens, hidden, num_experts, top_k, dtype, FMOE_EXPERT_ORDERED);
-    return ordered > plain ? ordered : plain;
+    return fmoe_expert_workspace_bytes_algo(num_tokens, hidden, num_experts, top_k, dtype, FMOE_EXPERT_AUTO);
 }
 
 extern "C" size_t fmoe_pkm_workspace_bytes(int64_t num_tokens, int hidden, int64_t num_experts, int top_k, int dtype) {
@@ -1803,7 +1799,7 @@ extern "C" int fmoe_expert_forward_save(const void* x, const void* down, const v
     const ExpertSavedPlan plan = expert_saved_plan(num_tokens, hidden, num_experts, top_k, dtype);
     if (need) kept = plan.at(saved);
     return expert_dispatch("fmoe_expert_forward_save", kActSilu, x, down, up, indices, gates, num_tokens, hidden, num_experts, top_k, dtype,
-                           out, workspace, workspace_bytes, plan.ordered ? FMOE_EXPERT_ORDERED : FMOE_EXPERT_AUTO, stream, need ? &kept : nullptr);
+                           out, workspace, workspace_bytes, FMOE_EXPERT_AUTO, stream, need ? &kept : nullptr);
 }
 
 extern "C" int fmoe_peer_forward(const void* x, const void* down, const void* up, const void* routing_weights,

@@ -651,9 +651,10 @@ template <typename T> SlicePlan plan_slices_of_k(int M, int N, int K) {
     const double kRow = 2.3e-3, launch = split_k ? 8.5 : 4.0;
     double best_time = (split_k ? 0.8 : 0.9) * whole * k_tiles * kRow;
     // Two 128 x 128 tiles to a compute unit hide each other's latency, by how much depends on the extents in ways the price does not
-    // see: of 53 down products that would otherwise be sliced (bf16) 38 would gain, up to a third (1692 tokens, 10576 -> 3968: 192 whole,
-    // 131 in two slices), and 15 lose, up to a seventh (4918 tokens, 3456 -> 864: 41 whole, 47).  0.65 keeps nearly all of them whole.
-    if (shape == kTile128 && tiles > cus) best_time *= sizeof(T) == 2 ? 0.85 : 0.65;
+    // see.  Of 90 down products in bf16 that the price alone would cut, 0.85 cuts 46, of which 37 gain (0.91 of the time on average, at best
+    // 2510 tokens, 5416 -> 2032: 102 us whole, 71 in slices) and 9 lose (at most 2685 tokens, 4160 -> 1560: 47 whole, 54); of the 44 it keeps
+    // whole 27 would gain (2708 tokens, 4968 -> 1864: 90 whole, 70) and 17 lose, up to a fifth.  No fp32 product comes near.
+    if (shape == kTile128 && tiles > cus) best_time *= 0.85;
     if (sizeof(T) == 4 && K % 4 != 0) return best;
     for (int i = sizeof(T) == 2 ? kTile256 : kTile128; i <= kTile64; ++i) {
         int64_t n = 0;

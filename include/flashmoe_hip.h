@@ -155,12 +155,12 @@ int fmoe_router_forward_noalloc(const void* x, const void* gate_w, void* running
  *   buckets  rows a multiple of 128 bytes; x and each table below 4 GiB; T*K < 2^31 - 4096; T < 2^24 (its second
  *            phase sweeps the experts when the dtype is 16-bit, K <= 256 and E < 2^22; else it gathers whole rows)
  *   ordered  tables below 4 GiB, K <= 65536
- * fmoe_expert_forward picks slices when E*128 bytes fit twice the L2 of one XCD and there are at least 65536 pairs, or
- * when the rows are too long for the row schedule; else ordered when there are at least 65536 pairs and min(T, 400) * K >= E
- * (the tokens in flight then share the table's rows; without gradients rows of 4 KB and more go to buckets while 400 * K is below
- * 1.35 * E and those apply); else buckets when there are at least 65536 pairs and 12 pairs per
- * expert (each table row then serves enough pairs to pay for the grouping) and its limits hold; else rows.  So any
- * hidden size works as long as each table stays below 4 GiB.
+ * fmoe_expert_forward picks by the extents and the dtype, from measurements of all four: slices for tables of which an XCD's L2 holds a
+ * slice, with at least 65536 pairs (fp16 and fp32 also with fewer of at least 128 MB of rows) and a dozen experts per token, or when
+ * the rows are too long for the row schedule; ordered for larger tables whose every expert the tokens in flight name about once or
+ * more; buckets for the largest with at least 65536 pairs, 12 pairs per expert and rows of 2 KB (fp32: 1.5 KB), within its limits;
+ * else rows.  The forward of a training step and its backward take the same.  So any hidden size works as long as each table stays
+ * below 4 GiB.  In bf16 slices round the coefficients silu(.) * gate to bf16; every other schedule and dtype keeps them in fp32.
  */
 size_t fmoe_expert_workspace_bytes(int64_t num_tokens, int hidden, int64_t num_experts, int top_k, int dtype);
 size_t fmoe_expert_workspace_bytes_algo(int64_t num_tokens, int hidden, int64_t num_experts, int top_k, int dtype, int algo);

@@ -262,7 +262,7 @@ def test_expert_schedule_at_the_lines_of_its_rule(T, H, E, K, dtype, schedule):
 
 
 def test_expert_workspace_is_enough_for_both_forwards():
-    """The forward of a training step may take the ordered lists where the other takes buckets: one size for both."""
+    """The forward alone and that of a training step: one size for both."""
     lib = _C.lib()
     for T, H, E, K in ((4800, 2048, 66049, 222), (16384, 2048, 102400, 256), (1024, 1024, 102400, 512), (4096, 1024, 16384, 64)):
         need = lib.fmoe_expert_workspace_bytes(T, H, E, K, _C.BF16)
