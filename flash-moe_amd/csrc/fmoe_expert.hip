@@ -1518,17 +1518,18 @@ bool ordered_possible(int64_t E, int H, int K, size_t elt) { return slices_possi
 // slices outgrow the L2 (H 1000: 6000 x 200 of 16000 327 for 440).
 //
 // Where no slice fits (beyond 65536 experts, in rows between lines 21000) ordered lists compete with rows and buckets only, and pay
-// earlier: from every expert named 1.1 times on, in rows between lines four times and up to 5500 sqrt(K) (H 736, 1097 x 816 of 66000 246 for 443;
-// fp16, H 336, 2107 x 881 of 26000 259 for 576).  XCDs without a slice count by the square of their share, on both lines: with six of eight in
-// work the lists are ahead from 2 to 4 times on, with all of them from 1 to 1.3 (H 384, 2172 x 535 of 102000 205 for 356).  Up to 512 tokens
-// of 100 experts or more are too few to fill the chip in rows and walk ordered lists from once on (H 384, 282 x 757 of 121000 57 for 119;
-// fp16, H 256, 286 x 540 of 144000 38 for 82); of 1024 tokens they no longer pay there.
+// earlier: from every expert named 1.1 times on, in rows between lines four times and up to 5500 sqrt(K) (H 736, 1097 x 816 of 66000 246
+// for 443; fp16, H 336, 2107 x 881 of 26000 259 for 576).  XCDs without a slice count by the square of their share, on both lines: with
+// six of eight in work the lists are ahead from 2 to 4 times on, with all of them from 1 to 1.3 (H 384, 2172 x 535 of 102000 205 for 356).
+// Where 400 tokens, or all where there are fewer, name every expert once and each has 100, ordered lists are ahead whatever the slices and
+// the window (H 384, 282 x 757 of 121000 57 for 119 in rows; fp16, H 256, 286 x 540 of 144000 38 for 82; 26 problems of 260000 to 900000
+// experts, rows of 2 to 4 KB, 0.61 to 0.93 times the buckets, which round the coefficients in bf16 as well).
 //
 // Slices of 128 bytes, while an L2 holds half of one (H 1024: 16384 x 32 of 24000 1.25 times faster than ordered, 4096 x 32 of 50000 1.21
 // than rows), all of one for 16-bit rows of 4 KB (beyond, rows 1.07 to 1.12 times faster; fp32 rows of 4 to 8 KB 0.75 to 0.89); for 16-bit
 // rows of 1 KB from 24 experts per token on (12 to 16 1.1 times the rows, fp32 0.85); for rows between lines up to 21000 experts (H 1000:
 // 20000 x 30 of 20000 275 for 333).  Shorter rows would still gain beyond 65536 experts (H 256: 16384 x 64 of 102400 1.15 times), but in
-// bf16 slices round the coefficients, which the other schedules keep in fp32.
+// bf16 slices round the coefficients, which rows and ordered lists keep in fp32.
 //
 // Buckets, once an expert's row serves a dozen pairs and rows are 2 KB, in fp32 1.5 KB; else whole rows, straight from HBM.  Buckets against
 // rows, twelve to sixteen pairs an expert | more, over 1900 problems: bf16 rows of 512 bytes 1.86 | 1.63, 1 KB 1.15 | 1.05, 1152 1.60 | 1.44,
@@ -1553,8 +1554,7 @@ int choose_schedule(int algo, int64_t T_, int H, int64_t E, int K, int dtype, bo
         if (E * (on_lines ? 128 : 384) > 2 * l2) {
             const double named = (double)(T_ < 2560 ? T_ : 2560) * K, share = in_work * in_work;
             const double most = on_lines ? (buckets ? 80.0e6 : 144.0e6) : 30.0e6;
-            if ((named * share >= (on_lines ? 1.1 : 4.0) * (double)E && width <= most * share) ||
-                (T_ <= 512 && K >= 100 && named >= (double)E && width <= 144.0e6))
+            if ((named * share >= (on_lines ? 1.1 : 4.0) * (double)E && width <= most * share) || (K >= 100 && (T_ < 400 ? T_ : 400) * K >= E))
                 return FMOE_EXPERT_ORDERED;
         } else {
             const int64_t tokens = T_ / parts;

@@ -160,7 +160,8 @@ int fmoe_router_forward_noalloc(const void* x, const void* gate_w, void* running
  * the rows are too long for the row schedule; ordered for larger tables whose every expert the tokens in flight name about once or
  * more; buckets for the largest with at least 65536 pairs, 12 pairs per expert and rows of 2 KB (fp32: 1.5 KB), within its limits;
  * else rows.  The forward of a training step and its backward take the same.  So any hidden size works as long as each table stays
- * below 4 GiB.  In bf16 slices round the coefficients silu(.) * gate to bf16; every other schedule and dtype keeps them in fp32.
+ * below 4 GiB.  In bf16 slices and buckets round the coefficients silu(.) * gate to bf16; rows, ordered and the other dtypes keep
+ * them in fp32.
  */
 size_t fmoe_expert_workspace_bytes(int64_t num_tokens, int hidden, int64_t num_experts, int top_k, int dtype);
 size_t fmoe_expert_workspace_bytes_algo(int64_t num_tokens, int hidden, int64_t num_experts, int top_k, int dtype, int algo);

@@ -250,6 +250,8 @@ def test_few_bf16_pairs_of_long_rows_keep_fp32_coefficients(T, H, E, K):
     (282, 384, 120943, 757, "BF16", "ORDERED"), (286, 256, 144100, 540, "F16", "ORDERED"), (2172, 384, 101688, 535, "F16", "ORDERED"),
     (1097, 736, 66109, 816, "BF16", "ORDERED"), (2107, 336, 25869, 881, "F16", "ORDERED"), (282, 384, 120943, 400, "BF16", "ROWS"),
     (3118, 640, 100000, 64, "BF16", "ROWS"), (282, 384, 120943, 99, "BF16", "ROWS"),
+    # and where 400 tokens name every expert, instead of the grouping, which rounds the coefficients in bf16
+    (8301, 1024, 334092, 1078, "BF16", "ORDERED"), (18039, 1792, 838895, 4030, "BF16", "ORDERED"), (8301, 1024, 334092, 830, "BF16", "BUCKETS"),
     # slices in fp32: from ten experts per token on, and for rows of 4 KB of more than 32768 experts
     (16384, 1024, 16000, 9, "F16", "ROWS"), (16384, 480, 16000, 11, "F32", "SLICES"), (16384, 960, 16000, 11, "F16", "ROWS"),
     (6348, 1216, 53917, 31, "F32", "SLICES"), (7000, 2048, 50000, 31, "BF16", "ROWS"),
