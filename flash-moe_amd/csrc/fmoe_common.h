@@ -179,13 +179,23 @@ enum { kBlasNN = 0, kBlasTN = 1 };
 int blas_gemm(int layout, int M, int N, int K, const void* A, int lda, const void* B, int ldb, void* C, int ldc, float beta,
               int dtype, hipStream_t stream);
 
-// The same products (C is [M,N]) on this library's own kernels (fmoe_gemm_tr.hip), through blas_gemm where those cannot address them.  With B1
-// (NN only) the product has a second range of K values: C = A[:, :K] B0 + A[:, K:2K] B1.  A's rows may be padded (lda) with zeros to
-// whole 16-byte packets.
-int gemm_backward(int layout, int M, int N, int K, const void* A, int lda, const void* B0, const void* B1, int ldb, void* C, int dtype,
-                  void* workspace, size_t workspace_bytes, hipStream_t stream);
-// Scratch of gemm_backward for the sums of a sliced k range (0 when it needs none); segments = 2 with B1, else 1.
+// The same products (C is [M,N]) on this library's own kernels (fmoe_gemm_tr.hip), through blas_gemm where those cannot address them.  With
+// two segments (NN only) the product has a second range of K values: C = A[:, :K] B0 + A[:, K:2K] B1.  A's rows may be padded (lda)
+// with zeros to whole 16-byte packets.
+struct BackwardProduct {
+    int layout, M, N, K, segments;
+    const void* A;
+    int lda;
+    const void *B0, *B1;
+    int ldb;
+    void* C;
+};
+int gemm_backward(const BackwardProduct& product, int dtype, void* workspace, size_t workspace_bytes, hipStream_t stream);
+// Scratch of gemm_backward for the sums of a sliced k range (0 when it needs none).
 size_t gemm_backward_workspace_bytes(int M, int N, int K, int segments, int dtype);
+// Several products that do not depend on each other (at most four share a launch); their pointers do not matter for the scratch.
+int gemm_backward(const BackwardProduct* products, int count, int dtype, void* workspace, size_t workspace_bytes, hipStream_t stream);
+size_t gemm_backward_workspace_bytes(const BackwardProduct* products, int count, int dtype);
 
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 inline size_t dtype_size(int dtype) { return dtype == FMOE_F32 ? 4 : 2; }

@@ -10,7 +10,10 @@
 // and, with few tiles and a long k loop, the length of one chain, which slices of k cut (their sums are added by a second launch, in
 // slice order).  A kernel that turned the operands in registers reached 600 TFLOP/s in bf16 where these reach 1000 to 1300.
 //
-// Against the library's kernels (rocBLAS), us:
+// The MLP's backward forms dWd, dx, dWg and dWu in one launch (gemm_group_kernel): none of them alone is whole rounds of tiles, and two
+// workgroups of different products share a compute unit as well as two of one.
+//
+// Against the library's kernels (rocBLAS), each product alone, us:
 //   bf16  2048 tokens, 4096 -> 16384: dh 187 for 203, dx 414 for 502, dWd 213 for 258, dWg and dWu 418 for 512; 4096 tokens, 1024 -> 4096:
 //         31 for 33, 71 for 79, 39 for 45, 62 for 69; 615 tokens, 776 -> 2072: 8 for 17, 20 for 36, 7 for 17, 11 for 18; 32768 tokens, 2048
 //         -> 8192: 871 for 871, 1501 for 1648, 783 for 944, 1613 for 1891.  Before the waves of a 256 x 256 tile worked in two groups
@@ -51,23 +54,81 @@ __global__ __launch_bounds__(kWideThreads, 2) void gemm_wide_turned_kernel(
         SLICED ? block / tiles : 0, slices, lda, ldb, segments);
 }
 
-// C = sum over the slices, in order; one packet of C per thread
+// Several products in one launch: the workgroups of member i are first .. first + tiles * slices - 1 (first a multiple of the XCDs; ids
+// past the last are spare), one tile or slice of k each, which the dispatcher hands to compute units as they fall free, longest first.
+// us, dWd, dx, dWg and dWu one after the other and together, bf16: 4096 tokens, 1024 -> 4096 190 -> 152; 615 tokens, 776 -> 2072 35.5 ->
+// 23.6; 1000 tokens, 1024 -> 4096 63 -> 49; 130 tokens, 408 -> 1088 17.8 -> 9.4; 5616 tokens, 608 -> 2432 123 -> 82; fp32: 691 tokens, 1056
+// -> 2112 177 -> 133; 103 tokens, 768 -> 1536 33 -> 22.  What is left is what the L2s deliver on 128 x 128 tiles, two to a compute unit
+// (69 GB/s each), and the matrix pipes in fp32.
+struct GroupMember {
+    const void *A, *B0, *B1;
+    void* out;                   // C, or the planes of its slices
+    int lda, ldb, M, N, K, segments, tiles_m, tiles_n, slices, first, a_turned;
+};
+constexpr int kGroupMost = 4;
+struct Group { GroupMember m[kGroupMost]; };
+
+template <typename T, int SHAPE, bool TA, bool SLICED>
+__device__ __forceinline__ void group_tile(const GroupMember& m, int at) {
+    const int tiles = m.tiles_m * m.tiles_n, tile = at % tiles, slice = at / tiles;
+    const T *A = (const T*)m.A, *B0 = (const T*)m.B0, *B1 = (const T*)m.B1;
+    constexpr int EPI = SLICED ? kEpiPart : kEpiPlain;
+    if constexpr (SHAPE == kTile256)
+        gemm_wide_tiles<T, EPI, true, SLICED, TA, true>(A, B0, B1, (T*)m.out, nullptr, m.M, m.N, m.K, m.tiles_m, m.tiles_n, 1, tile, tiles, slice,
+                                                        m.slices, m.lda, m.ldb, m.segments);
+    else
+        gemm_dma_tiles<T, kTileRows[SHAPE], kTileCols[SHAPE], 2, 2, kStageK<T>, 2, EPI, kSmallAhead<T>, kFragRows<T>, true, SLICED, TA, true>(
+            A, B0, B1, (T*)m.out, nullptr, m.M, m.N, m.K, m.tiles_m, m.tiles_n, 1, tile, tiles, slice, m.slices, m.lda, m.ldb, m.segments);
+}
+
+template <typename T, int SHAPE>
+__global__ __launch_bounds__(SHAPE == kTile256 ? kWideThreads : 256, 2) void gemm_group_kernel(const Group g, int members, int xcds) {
+    const int block = (int)blockIdx.x;
+    int i = 0;
+    while (i + 1 < members && block >= g.m[i + 1].first) ++i;
+    const GroupMember& m = g.m[i];
+    const int items = m.tiles_m * m.tiles_n * m.slices, local = block - m.first;
+    if (local >= items) return;
+    const int at = xcd_run(local, items, xcds);
+    if (m.slices > 1) {
+        if (m.a_turned) group_tile<T, SHAPE, true, true>(m, at);
+        else group_tile<T, SHAPE, false, true>(m, at);
+    } else {
+        if (m.a_turned) group_tile<T, SHAPE, true, false>(m, at);
+        else group_tile<T, SHAPE, false, false>(m, at);
+    }
+}
+
+// C = sum over the slices, in order, of one or several products; one packet of C per thread
+struct SumMember { const float* planes; void* C; int64_t packets; int slices, first; };
+struct Sums { SumMember m[kGroupMost]; };
 template <typename T>
-__global__ __launch_bounds__(256) void gemm_turned_add_kernel(const float* __restrict__ planes, T* __restrict__ C, int64_t packets, int slices) {
+__global__ __launch_bounds__(256) void gemm_turned_add_kernel(const Sums g, int members) {
     constexpr int V = Elem<T>::kVec;
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= packets) return;
+    int k = 0;
+    while (k + 1 < members && (int)blockIdx.x >= g.m[k + 1].first) ++k;
+    const SumMember& m = g.m[k];
+    const int64_t i = (int64_t)((int)blockIdx.x - m.first) * blockDim.x + threadIdx.x;
+    if (i >= m.packets) return;
     float v[V];
 #pragma unroll
     for (int e = 0; e < V; ++e) v[e] = 0.0f;
-    for (int s = 0; s < slices; ++s)
+    for (int s = 0; s < m.slices; ++s)
 #pragma unroll
         for (int h = 0; h < V; h += 4) {
-            const f32x4_t p = *reinterpret_cast<const f32x4_t*>(planes + (s * packets + i) * V + h);
+            const f32x4_t p = *reinterpret_cast<const f32x4_t*>(m.planes + (s * m.packets + i) * V + h);
 #pragma unroll
             for (int e = 0; e < 4; ++e) v[h + e] += p[e];
         }
-    reinterpret_cast<u32x4_t*>(C)[i] = pack16<T>(v);
+    reinterpret_cast<u32x4_t*>(m.C)[i] = pack16<T>(v);
+}
+template <typename T> void launch_sums(Sums& g, int members, hipStream_t stream) {
+    int blocks = 0;
+    for (int i = 0; i < members; ++i) {
+        g.m[i].first = blocks;
+        blocks += (int)((g.m[i].packets + 255) / 256);
+    }
+    hipLaunchKernelGGL((gemm_turned_add_kernel<T>), dim3((unsigned)blocks), dim3(256), 0, stream, g, members);
 }
 
 // Tile shape and slices of k by price (us): a round of tiles costs what the forward's rule says, 2.3 ns per received row and k-tile,
@@ -127,9 +188,9 @@ void launch_turned(const void* A, int lda, const void* B0, const void* B1, int l
             case kTile64x128: if constexpr (sizeof(T) == 2) FMOE_SLICED(64, 128, 2, 4); break;
             default: FMOE_SLICED(64, 64, 2, 4); break;
         }
-        const int64_t packets = (int64_t)M * N / Elem<T>::kVec;
-        hipLaunchKernelGGL((gemm_turned_add_kernel<T>), dim3((unsigned)((packets + 255) / 256)), dim3(256), 0, stream, (const float*)planes,
-                           (T*)C, packets, p.slices);
+        Sums g = {};
+        g.m[0] = {planes, C, (int64_t)M * N / Elem<T>::kVec, p.slices, 0};
+        launch_sums<T>(g, 1, stream);
         return;
     }
     switch (p.shape) {
@@ -156,6 +217,171 @@ void launch_turned(const void* A, int lda, const void* B0, const void* B1, int l
 #undef FMOE_WHOLE
 }
 
+// How a group is cut: one tile shape for all, slices of k for each, shape -1: one product after the other.
+struct GroupPlan { int shape, slices[kGroupMost]; };
+
+// Time of `kinds` lots of items (n[i] of time t[i], longest first) on `slots` that take the next item as they fall free.
+inline double time_of_items(const int64_t* n, const double* t, int kinds, int slots) {
+    struct Free { double at; int64_t slots; } f[2 * kGroupMost + 2] = {{0.0, slots}};
+    int lots = 1;
+    double end = 0.0;
+    for (int i = 0; i < kinds; ++i)
+        for (int64_t left = n[i]; left > 0;) {
+            int e = 0;
+            for (int j = 1; j < lots; ++j)
+                if (f[j].at < f[e].at) e = j;
+            const double done = f[e].at + t[i];
+            int64_t take = left < f[e].slots ? left : f[e].slots;
+            if (lots == 1 && take == f[e].slots) {                  // whole rounds at once
+                const int64_t rounds = left / f[e].slots;
+                f[e].at += (double)rounds * t[i];
+                end = f[e].at > end ? f[e].at : end;
+                left -= rounds * f[e].slots;
+                continue;
+            }
+            left -= take;
+            f[e].slots -= take;
+            if (f[e].slots == 0) f[e] = f[--lots];
+            int j = 0;
+            while (j < lots && f[j].at != done) ++j;
+            if (j < lots) f[j].slots += take;
+            else if (lots < 2 * kGroupMost + 2) f[lots++] = {done, take};
+            else f[lots - 1].slots += take;
+            end = done > end ? done : end;
+        }
+    return end;
+}
+
+// Price (us) of a group on tiles of a shape: half (0.4 to 1) of what its items take on slots that hold two workgroups of 128 x 128 (four of
+// 64 x 64) to a compute unit, the rest what they take if the tail were filled, at least the longest chain; per sliced product 4 us and
+// its planes written and read at 6 TB/s.  The rates of a k-tile, with the compute unit full and alone, and the 3.4 % (fp32 2.3) by which the
+// choice misses the best of 72 cuts on average come from 105 backward passes in bf16 (64 to 8192 tokens, 256 to 2048 columns) and 35 in fp32 (there up to
+// 16384, best on 128 x 128 tiles from about 4000 tokens on: 4096 tokens, 1024 -> 4096 1258 us one by one, 1238 on 64 x 64, 1176; 5000, 2048
+// -> 5464 4392, 4291, 4176).  64 x 128 tiles would gain half a percent.  Products over tokens (the weight gradients)
+// are sliced from 2048 tokens on.
+// 16-bit, beyond four rounds of 256 x 256 tiles: each product fills the chip and its persistent workgroups start a tile's loads under the last
+// one's stores: 2048 tokens, 4096 -> 16384 1057 us one by one, 1087 together; 6000 tokens, 1800 -> 7200, three and a half rounds, 734 and 731.
+template <typename T> GroupPlan plan_group(const BackwardProduct* p, int count) {
+    GroupPlan best = {-1, {1, 1, 1, 1}};
+    if (count < 2 || count > kGroupMost) return best;
+    constexpr bool kSingle = sizeof(T) == 4;      // fp32
+    const int cus = chip_info().cus;
+    int64_t wide = 0;
+    int token_cuts = 1;
+    for (int i = 0; i < count; ++i) {
+        if (p[i].layout == kBlasTN && p[i].K >= 2048) token_cuts = 3;
+        wide += (int64_t)((p[i].M + 255) / 256) * ((p[i].N + 255) / 256);
+    }
+    if (!kSingle && wide > 4 * (int64_t)cus) return best;
+    constexpr int kShapes[3] = {kTile256, kTile128, kTile64}, kPer[3] = {1, 2, 4};
+    constexpr double kFull[3] = {1.5, kSingle ? 1.75 : 0.47, kSingle ? 0.475 : 0.225}, kAlone[3] = {1.3, kSingle ? 2.2 : 0.75, kSingle ? 0.6 : 0.3};
+    constexpr double kStores[3] = {6.0, kSingle ? 2.0 : 0.65, kSingle ? 0.2 : 0.1}, kRounds[3] = {0.5, kSingle ? 1.0 : 0.4, kSingle ? 0.5 : 0.4};
+    constexpr int kOver[6] = {1, 2, 3, 4, 6, 8}, kTokens[3] = {1, 2, 4};
+    double best_time = 0.0;
+    for (int z = kSingle ? 1 : 0; z < 3; ++z) {
+        const int shape = kShapes[z];
+        int64_t tiles[kGroupMost];
+        int k_tiles[kGroupMost];
+        for (int i = 0; i < count; ++i) {
+            tiles[i] = (int64_t)((p[i].M + kTileRows[shape] - 1) / kTileRows[shape]) * ((p[i].N + kTileCols[shape] - 1) / kTileCols[shape]);
+            k_tiles[i] = (p[i].K + kStageK<T> - 1) / kStageK<T> * p[i].segments;
+        }
+        for (int over : kOver)
+            for (int cut = 0; cut < token_cuts; ++cut)
+                for (int cut_rest = 0; cut_rest <= cut; ++cut_rest) {
+                    const int first = kTokens[cut], rest = kTokens[cut_rest];
+                    GroupPlan g = {shape, {1, 1, 1, 1}};
+                    int64_t n[kGroupMost];
+                    double t[kGroupMost], work = 0.0, longest = 0.0, planes = 0.0;
+                    bool usable = true, seen = false;
+                    for (int i = 0; i < count && usable; ++i) {
+                        const bool turned = p[i].layout == kBlasTN;
+                        const int s = turned ? (seen ? rest : first) : over, share = (k_tiles[i] + s - 1) / s;
+                        seen = seen || turned;
+                        usable = s == 1 || ((!turned || p[i].K >= 2048) && k_tiles[i] >= 2 * s && (s - 1) * share < k_tiles[i]);
+                        g.slices[i] = s;
+                        int at = i;                                              // longest first
+                        const double item = share * kFull[z] + kStores[z];
+                        while (at > 0 && t[at - 1] < item) {
+                            t[at] = t[at - 1];
+                            n[at] = n[at - 1];
+                            --at;
+                        }
+                        t[at] = item;
+                        n[at] = tiles[i] * s;
+                        work += (double)n[at] * item / cus;
+                        if (share * kAlone[z] > longest) longest = share * kAlone[z];
+                        if (s > 1) planes += 4.0 + 8.0e-6 * s * (double)p[i].M * p[i].N / 6.0;
+                    }
+                    if (!usable || (best.shape >= 0 && (work > longest ? work : longest) + planes >= best_time)) continue;
+                    for (int i = 0; i < count; ++i) t[i] *= kPer[z];
+                    const double mixed = kRounds[z] * time_of_items(n, t, count, kPer[z] * cus) + (1.0 - kRounds[z]) * work;
+                    const double time = (mixed > longest ? mixed : longest) + planes;
+                    if (best.shape < 0 || time < best_time) {
+                        best = g;
+                        best_time = time;
+                    }
+                }
+    }
+    return best;
+}
+
+GroupPlan plan_group_of(const BackwardProduct* p, int count, int dtype) {
+    return dtype == FMOE_F32 ? plan_group<float>(p, count) : plan_group<bf16_t>(p, count);
+}
+size_t group_planes_bytes(const BackwardProduct* p, int count, const GroupPlan& g) {
+    size_t bytes = 0;
+    for (int i = 0; i < count; ++i)
+        if (g.slices[i] > 1) bytes += round_up((size_t)g.slices[i] * p[i].M * p[i].N * sizeof(float), 256);
+    return bytes;
+}
+
+// Whether the kernels here can address a product: whole packets (where M (TN) or K (NN) is none, the rows of A are padded with zeros up to
+// lda) and 32-bit byte offsets inside a descriptor.
+bool addressable(const BackwardProduct& p, int dtype) {
+    const int a_cols = p.layout == kBlasTN ? p.M : p.K * p.segments, vec = dtype == FMOE_F32 ? 4 : 8;
+    const bool packets = p.lda % vec == 0 && p.ldb % vec == 0 && p.N % vec == 0 && (a_cols + vec - 1) / vec * vec <= p.lda &&
+                         (p.segments == 1 || p.K % vec == 0) && aligned16(p.A) && aligned16(p.B0) && aligned16(p.B1) && aligned16(p.C);
+    const double most = dtype == FMOE_F32 ? 5.0e8 : 1.0e9;
+    return packets && (double)p.K * p.ldb < most && (p.layout == kBlasTN ? (double)p.K * p.lda < most : 256.0 * p.lda < most);
+}
+
+template <typename T> void launch_group(const BackwardProduct* p, int count, const GroupPlan& plan, void* workspace, hipStream_t stream) {
+    const int xcds = chip_info().xcds, rows = kTileRows[plan.shape], cols = kTileCols[plan.shape];
+    Group g = {};
+    Sums sums = {};
+    int sliced = 0, blocks = 0, order[kGroupMost];
+    auto share = [&](int i) { return ((p[i].K + kStageK<T> - 1) / kStageK<T> * p[i].segments + plan.slices[i] - 1) / plan.slices[i]; };
+    for (int i = 0; i < count; ++i) {                    // longest first
+        int at = i;
+        while (at > 0 && share(order[at - 1]) < share(i)) {
+            order[at] = order[at - 1];
+            --at;
+        }
+        order[at] = i;
+    }
+    char* planes = (char*)workspace;
+    for (int k = 0; k < count; ++k) {
+        const int i = order[k];
+        const BackwardProduct& q = p[i];
+        g.m[k] = {q.A, q.B0, q.segments > 1 ? q.B1 : q.B0, q.C, q.lda, q.ldb, q.M, q.N, q.K, q.segments, (q.M + rows - 1) / rows, (q.N + cols - 1) / cols,
+                  plan.slices[i], blocks, q.layout == kBlasTN};
+        if (plan.slices[i] > 1) {
+            g.m[k].out = planes;
+            sums.m[sliced++] = {(const float*)planes, q.C, (int64_t)q.M * q.N / Elem<T>::kVec, plan.slices[i], 0};
+            planes += round_up((size_t)plan.slices[i] * q.M * q.N * sizeof(float), 256);
+        }
+        blocks += (g.m[k].tiles_m * g.m[k].tiles_n * plan.slices[i] + xcds - 1) / xcds * xcds;
+    }
+#define FMOE_GO(SHAPE) \
+    hipLaunchKernelGGL((gemm_group_kernel<T, SHAPE>), dim3((unsigned)blocks), dim3((SHAPE) == kTile256 ? kWideThreads : 256), 0, stream, g, count, xcds)
+    if (plan.shape == kTile64) FMOE_GO(kTile64);
+    else if (plan.shape == kTile128) FMOE_GO(kTile128);
+    else if constexpr (sizeof(T) == 2) FMOE_GO(kTile256);
+#undef FMOE_GO
+    if (sliced > 0) launch_sums<T>(sums, sliced, stream);
+}
+
 }  // namespace
 
 size_t gemm_backward_workspace_bytes(int M, int N, int K, int segments, int dtype) {
@@ -163,24 +389,15 @@ size_t gemm_backward_workspace_bytes(int M, int N, int K, int segments, int dtyp
     return slices > 1 ? (size_t)slices * M * N * sizeof(float) : 0;
 }
 
-int gemm_backward(int layout, int M, int N, int K, const void* A, int lda, const void* B0, const void* B1, int ldb, void* C, int dtype,
-                  void* workspace, size_t workspace_bytes, hipStream_t stream) {
-    const int segments = B1 != nullptr ? 2 : 1;
-    // whole packets: where M (TN) or K (NN) is none, the rows of A are padded with zeros up to lda
-    const int a_cols = layout == kBlasTN ? M : K * segments, vec = dtype == FMOE_F32 ? 4 : 8;
-    const bool packets = lda % vec == 0 && ldb % vec == 0 && N % vec == 0 && (a_cols + vec - 1) / vec * vec <= lda &&
-                         (segments == 1 || K % vec == 0) && aligned16(A) && aligned16(B0) && aligned16(B1) && aligned16(C);
-    // 32-bit byte offsets inside a descriptor
-    const double most = dtype == FMOE_F32 ? 5.0e8 : 1.0e9;
-    const bool reach = (double)K * ldb < most && (layout == kBlasTN ? (double)K * lda < most : 256.0 * lda < most);
-    if (packets && reach) {
-        SlicePlan p = dtype == FMOE_F32 ? plan_turned<float>(M, N, K, segments) : plan_turned<bf16_t>(M, N, K, segments);
-        if ((size_t)p.slices * M * N * sizeof(float) > workspace_bytes) p.slices = 1;
+int gemm_backward(const BackwardProduct& q, int dtype, void* workspace, size_t workspace_bytes, hipStream_t stream) {
+    if (addressable(q, dtype)) {
+        SlicePlan p = dtype == FMOE_F32 ? plan_turned<float>(q.M, q.N, q.K, q.segments) : plan_turned<bf16_t>(q.M, q.N, q.K, q.segments);
+        if ((size_t)p.slices * q.M * q.N * sizeof(float) > workspace_bytes) p.slices = 1;
         float* planes = (float*)workspace;
-#define FMOE_TURNED(TT)                                                                                                       \
-    do {                                                                                                                      \
-        if (layout == kBlasTN) launch_turned<TT, true>(A, lda, B0, B1, ldb, C, M, N, K, segments, p, planes, stream);         \
-        else launch_turned<TT, false>(A, lda, B0, B1, ldb, C, M, N, K, segments, p, planes, stream);                          \
+#define FMOE_TURNED(TT)                                                                                                                         \
+    do {                                                                                                                                        \
+        if (q.layout == kBlasTN) launch_turned<TT, true>(q.A, q.lda, q.B0, q.B1, q.ldb, q.C, q.M, q.N, q.K, q.segments, p, planes, stream);     \
+        else launch_turned<TT, false>(q.A, q.lda, q.B0, q.B1, q.ldb, q.C, q.M, q.N, q.K, q.segments, p, planes, stream);                        \
     } while (0)
         switch (dtype) {
             case FMOE_F32: FMOE_TURNED(float); break;
@@ -191,9 +408,38 @@ int gemm_backward(int layout, int M, int N, int K, const void* A, int lda, const
         FMOE_CHECK_LAUNCH("backward product");
         return FMOE_OK;
     }
-    if (int rc = blas_gemm(layout, M, N, K, A, lda, B0, ldb, C, N, 0.0f, dtype, stream)) return rc;
-    if (B1 == nullptr) return FMOE_OK;
-    return blas_gemm(layout, M, N, K, (const char*)A + (size_t)K * dtype_size(dtype), lda, B1, ldb, C, N, 1.0f, dtype, stream);
+    if (int rc = blas_gemm(q.layout, q.M, q.N, q.K, q.A, q.lda, q.B0, q.ldb, q.C, q.N, 0.0f, dtype, stream)) return rc;
+    if (q.segments == 1) return FMOE_OK;
+    return blas_gemm(q.layout, q.M, q.N, q.K, (const char*)q.A + (size_t)q.K * dtype_size(dtype), q.lda, q.B1, q.ldb, q.C, q.N, 1.0f, dtype, stream);
+}
+
+size_t gemm_backward_workspace_bytes(const BackwardProduct* p, int count, int dtype) {
+    const GroupPlan plan = plan_group_of(p, count, dtype);
+    if (plan.shape >= 0) return group_planes_bytes(p, count, plan);
+    size_t most = 0;
+    for (int i = 0; i < count; ++i) {
+        const size_t alone = gemm_backward_workspace_bytes(p[i].M, p[i].N, p[i].K, p[i].segments, dtype);
+        if (alone > most) most = alone;
+    }
+    return most;
+}
+
+int gemm_backward(const BackwardProduct* p, int count, int dtype, void* workspace, size_t workspace_bytes, hipStream_t stream) {
+    const GroupPlan plan = plan_group_of(p, count, dtype);
+    bool together = plan.shape >= 0 && group_planes_bytes(p, count, plan) <= workspace_bytes;
+    for (int i = 0; i < count; ++i) together = together && addressable(p[i], dtype);
+    if (together) {
+        switch (dtype) {
+            case FMOE_F32: launch_group<float>(p, count, plan, workspace, stream); break;
+            case FMOE_BF16: launch_group<bf16_t>(p, count, plan, workspace, stream); break;
+            default: launch_group<f16_t>(p, count, plan, workspace, stream); break;
+        }
+        FMOE_CHECK_LAUNCH("backward products");
+        return FMOE_OK;
+    }
+    for (int i = 0; i < count; ++i)
+        if (int rc = gemm_backward(p[i], dtype, workspace, workspace_bytes, stream)) return rc;
+    return FMOE_OK;
 }
 
 }  // namespace fmoe

@@ -73,6 +73,17 @@ struct MlpBwdPlan {
     size_t off_a, off_b, off_dh, off_h, off_dab, off_part, part_bytes, bytes;
 };
 
+// The products after the SwiGLU gradient, extents only.  adjacent: dWg and dWu follow each other in memory and are one [2I, H] product (49
+// us each alone, 74 together at T = I = 4096, H = 1024).
+int mlp_gradients(int T_, int H, int I, bool adjacent, BackwardProduct (&q)[4]) {
+    const int I2 = 2 * I;
+    q[0] = {kTN, H, I, T_, 1, nullptr, H, nullptr, nullptr, I, nullptr};                     // dWd = dy^T h
+    q[1] = {kNN, T_, H, I, 2, nullptr, I2, nullptr, nullptr, H, nullptr};                    // dx = da Wg + db Wu
+    q[2] = {kTN, adjacent ? I2 : I, H, T_, 1, nullptr, I2, nullptr, nullptr, H, nullptr};    // dWg = da^T x (and dWu)
+    q[3] = {kTN, I, H, T_, 1, nullptr, I2, nullptr, nullptr, H, nullptr};                    // dWu = db^T x
+    return adjacent ? 3 : 4;
+}
+
 // kept: the caller has the products.  Their planes are left out, and h takes the place of dh, element by element as that is read.
 MlpBwdPlan plan_mlp_backward(int64_t T_, int H, int I, int dtype, bool kept) {
     MlpBwdPlan p;
@@ -84,12 +95,13 @@ MlpBwdPlan plan_mlp_backward(int64_t T_, int H, int I, int dtype, bool kept) {
     p.off_dh = take(ti);
     p.off_h = kept ? p.off_dh : take(ti);
     p.off_dab = take(2 * ti);
-    p.part_bytes = 0;
     const int t = (int)T_;
-    for (size_t n : {gemm_backward_workspace_bytes(t, I, H, 1, dtype), gemm_backward_workspace_bytes(H, I, t, 1, dtype),
-                     gemm_backward_workspace_bytes(t, H, I, 2, dtype), gemm_backward_workspace_bytes(2 * I, H, t, 1, dtype),
-                     gemm_backward_workspace_bytes(I, H, t, 1, dtype)})
+    p.part_bytes = gemm_backward_workspace_bytes(t, I, H, 1, dtype);
+    for (bool adjacent : {false, true}) {
+        BackwardProduct q[4];
+        const size_t n = gemm_backward_workspace_bytes(q, mlp_gradients(t, H, I, adjacent, q), dtype);
         if (n > p.part_bytes) p.part_bytes = n;
+    }
     p.off_part = take(p.part_bytes);
     p.bytes = o;
     return p;
@@ -164,22 +176,19 @@ extern "C" int fmoe_mlp_backward(const void* dy, const void* x, const void* gate
         if (rc) return rc;
     }
 
-    rc = gemm_backward(kNN, T_, I, H, dy, H, down_w, nullptr, I, dh, dtype, part, p.part_bytes, s);                        // dh = dy Wd
+    rc = gemm_backward({kNN, T_, I, H, 1, dy, H, down_w, nullptr, I, dh}, dtype, part, p.part_bytes, s);                    // dh = dy Wd
     if (rc) return rc;
     // da and db side by side: one [T, 2I] matrix [da | db], so that products over both are single calls
     char* db = dab + (size_t)I * elt;
     const int I2 = 2 * I;
     rc = launch_swiglu_backward(dh, a, b, dab, db, h, num_tokens, I, I2, I2, dtype, s);
     if (rc) return rc;
-    rc = gemm_backward(kTN, H, I, T_, dy, H, h, nullptr, I, ddown_w, dtype, part, p.part_bytes, s);                         // dWd = dy^T h
-    if (rc) return rc;
-    rc = gemm_backward(kNN, T_, H, I, dab, I2, gate_w, up_w, H, dx, dtype, part, p.part_bytes, s);                          // dx = da Wg + db Wu
-    if (rc) return rc;
     const size_t w_bytes = (size_t)I * H * elt;
-    // the two weight gradients are one [2I, H] product when the caller's buffers follow each other: one 74 us kernel at
-    // T = I = 4096, H = 1024 instead of two of 49 us
-    if ((char*)dup_w == (char*)dgate_w + w_bytes) return gemm_backward(kTN, I2, H, T_, dab, I2, x, nullptr, H, dgate_w, dtype, part, p.part_bytes, s);
-    rc = gemm_backward(kTN, I, H, T_, dab, I2, x, nullptr, H, dgate_w, dtype, part, p.part_bytes, s);                       // dWg = da^T x
-    if (rc) return rc;
-    return gemm_backward(kTN, I, H, T_, db, I2, x, nullptr, H, dup_w, dtype, part, p.part_bytes, s);                        // dWu = db^T x
+    BackwardProduct q[4];
+    const int count = mlp_gradients(T_, H, I, (char*)dup_w == (char*)dgate_w + w_bytes, q);
+    q[0].A = dy, q[0].B0 = h, q[0].C = ddown_w;
+    q[1].A = dab, q[1].B0 = gate_w, q[1].B1 = up_w, q[1].C = dx;
+    q[2].A = dab, q[2].B0 = x, q[2].C = dgate_w;
+    q[3].A = db, q[3].B0 = x, q[3].C = dup_w;
+    return gemm_backward(q, count, dtype, part, p.part_bytes, s);
 }

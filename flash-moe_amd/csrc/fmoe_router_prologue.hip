@@ -730,6 +730,12 @@ struct PrologueBwdPlan {
     size_t off_d16, off_q, off_dq, off_partial, off_sums, off_part, part_bytes, bytes;
 };
 
+// The two products, extents only.
+void prologue_products(int T_, int H, int N, int n_pad, BackwardProduct (&q)[2]) {
+    q[0] = {kBlasTN, N, H, T_, 1, nullptr, n_pad, nullptr, nullptr, H, nullptr};      // dWr = d^T q
+    q[1] = {kBlasNN, T_, H, N, 1, nullptr, n_pad, nullptr, nullptr, H, nullptr};      // dq = d Wr
+}
+
 PrologueBwdPlan plan_prologue_backward(int64_t T_, int H, int nk, int dtype) {
     PrologueBwdPlan p;
     const size_t elt = dtype_size(dtype);
@@ -742,9 +748,9 @@ PrologueBwdPlan plan_prologue_backward(int64_t T_, int H, int nk, int dtype) {
     p.off_dq = take((size_t)T_ * H * elt);
     p.off_partial = take((size_t)kMaxRowBlocks * 2 * H * 4);
     p.off_sums = take((size_t)2 * H * 4);
-    p.part_bytes = gemm_backward_workspace_bytes(2 * nk, H, t, 1, dtype);
-    const size_t dq = gemm_backward_workspace_bytes(t, H, 2 * nk, 1, dtype);
-    if (dq > p.part_bytes) p.part_bytes = dq;
+    BackwardProduct products[2];
+    prologue_products(t, H, 2 * nk, p.n_pad, products);
+    p.part_bytes = gemm_backward_workspace_bytes(products, 2, dtype);
     p.off_part = take(p.part_bytes);
     p.bytes = o;
     return p;
@@ -767,8 +773,12 @@ int launch_prologue_backward(const float* dlogits, const void* x, const void* ga
     hipLaunchKernelGGL((prologue_bwd_prepare_kernel<T>), dim3((unsigned)(T_ * col_blocks)), dim3(256), 0, s, dlogits,
                        (const T*)x, mean_rstd, d16, q, H, N, p.n_pad, col_blocks);
     FMOE_CHECK_LAUNCH("fmoe_router_prologue_backward(prepare)");
-    if (int rc = gemm_backward(kBlasTN, N, H, (int)T_, d16, p.n_pad, q, nullptr, H, dgate_w, dtype, part, p.part_bytes, s)) return rc;   // dWr = d^T q
-    if (int rc = gemm_backward(kBlasNN, (int)T_, H, N, d16, p.n_pad, gate_w, nullptr, H, dq, dtype, part, p.part_bytes, s)) return rc;   // dq = d Wr
+    BackwardProduct products[2];
+    prologue_products((int)T_, H, N, p.n_pad, products);
+    products[0].A = products[1].A = d16;
+    products[0].B0 = q, products[0].C = dgate_w;
+    products[1].B0 = gate_w, products[1].C = dq;
+    if (int rc = gemm_backward(products, 2, dtype, part, p.part_bytes, s)) return rc;
     if (training) {
         const int strips = (H + kWave * V - 1) / (kWave * V);
         hipLaunchKernelGGL((bn_bwd_partial_kernel<T>), dim3((unsigned)rows.row_blocks, (unsigned)strips), dim3(kStatsThreads), 0, s,

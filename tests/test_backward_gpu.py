@@ -752,6 +752,19 @@ def test_mlp_backward_on_the_large_tiles_of_the_turned_products(dtype, T, H, I):
     test_mlp_backward_remainders_of_the_transposing_products(dtype, T, H, I)
 
 
+@pytest.mark.parametrize("dtype,T,H,I", [
+    (torch.bfloat16, 513, 264, 520), (torch.float16, 2600, 264, 264),        # one launch on 64 x 64 tiles: whole; weight gradients in slices
+    (torch.float16, 1000, 1800, 4104), (torch.bfloat16, 5200, 776, 264),     # on 128 x 128: dx in slices; weight gradients in slices
+    (torch.bfloat16, 3000, 520, 1032),                                       # on 128 x 128, whole
+    (torch.float16, 1500, 1544, 5000),                                       # on 256 x 256, dx in slices
+    (torch.float32, 515, 132, 260), (torch.float32, 383, 516, 1544), (torch.float32, 2100, 136, 264),   # whole, dx, weight gradients
+    (torch.float32, 3076, 1284, 3076),                                       # on 128 x 128, dx in slices
+])
+def test_mlp_backward_products_in_one_launch(dtype, T, H, I):
+    """Sizes that take every tile shape and cut of the launch that forms dWd, dx, dWg and dWu together, none a multiple of a tile."""
+    test_mlp_backward_remainders_of_the_transposing_products(dtype, T, H, I)
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("T,H,E,K", [
     (3, 24, 40, 4), (256, 264, 900, 5), (257, 520, 300, 33), (2049, 136, 5000, 9),      # waves per token of the row schedule
