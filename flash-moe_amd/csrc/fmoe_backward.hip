@@ -219,11 +219,13 @@ __global__ __launch_bounds__(kBwdWaves* kWave) void route_backward_kernel(
 // pair is worked out once.  Bound by the latency of a wave's chain, which was four reductions on loads of their own and a 64-bit
 // division for every pair and pass: 4096 tokens of 128 keys and 64 pairs 15.4 -> 10.6 us, 615 tokens
 // of 64 keys and 17 pairs 6.3 -> 4.4.  The sums are those of the other kernel in its order.
-template <typename T, int R, int P>
+// PREPARE: inside the block nobody reads the gradients in fp32: they leave as the prologue's products take them, and with them the token's
+// row of q, whose loads hide in the chain: 4096 tokens, 1024 columns 16.3 us in two launches, 13.6 so; 615 tokens, 776 columns 6.9 -> 5.0.
+template <typename T, int R, int P, bool PREPARE>
 __global__ __launch_bounds__(kBwdWaves* kWave) void route_backward_small_kernel(
     const T* __restrict__ dgates, const int64_t* __restrict__ indices, const float* __restrict__ logits,
     const T* __restrict__ dlogits_extra, int64_t extra_token, int64_t extra_half, float* __restrict__ dlogits,
-    int64_t num_tokens, int nk, int top_k, int norm_topk_prob, int waves_per_block) {
+    int64_t num_tokens, int nk, int top_k, int norm_topk_prob, int waves_per_block, const PrologueOperands to) {
     extern __shared__ float acc_all[];   // [waves_per_block][2 * nk], one private row pair per wave
     const int lane = lane_id();
     const int wave = (int)(threadIdx.x >> 6);
@@ -318,25 +320,48 @@ __global__ __launch_bounds__(kBwdWaves* kWave) void route_backward_small_kernel(
             if (p >= nk) continue;
             float d = got[h][r] - expf((v[h][r] - shift[h]) - lse[h]) * sum[h];
             if (dlogits_extra != nullptr) d += extra[h][r];
-            dlogits[token * 2 * nk + h * nk + p] = d;
+            if constexpr (PREPARE) reinterpret_cast<T*>(to.d)[token * to.n_pad + h * nk + p] = Elem<T>::from_f32(d);
+            else dlogits[token * 2 * nk + h * nk + p] = d;
         }
+    if constexpr (PREPARE) {
+        constexpr int V = Elem<T>::kVec;
+        if (2 * nk + lane < to.n_pad) reinterpret_cast<T*>(to.d)[token * to.n_pad + 2 * nk + lane] = Elem<T>::from_f32(0.0f);
+        for (int c = lane; c < to.hidden / V; c += kWave) {
+            float xv[V], qv[V];
+            unpack16<T>(reinterpret_cast<const u32x4_t*>((const T*)to.x + token * to.hidden)[c], xv);
+#pragma unroll
+            for (int v = 0; v < V; v += 4) {
+                const f32x4_t m = *reinterpret_cast<const f32x4_t*>(to.mean_rstd + c * V + v);
+                const f32x4_t rs = *reinterpret_cast<const f32x4_t*>(to.mean_rstd + to.hidden + c * V + v);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) qv[v + j] = (xv[v + j] - m[j]) * rs[j];
+            }
+            reinterpret_cast<u32x4_t*>((T*)to.q + token * to.hidden)[c] = pack16<T>(qv);
+        }
+    }
 }
 
 template <typename T>
 int launch_route_backward(const void* dgates, const int64_t* indices, const float* logits, const void* dlogits_extra,
-                          int64_t extra_token, int64_t extra_half, float* dlogits, int64_t T_, int nk, int K, int norm, hipStream_t stream) {
+                          int64_t extra_token, int64_t extra_half, float* dlogits, int64_t T_, int nk, int K, int norm, hipStream_t stream,
+                          const PrologueOperands* operands) {
     const int chunk = backward_key_chunk(nk);
     const size_t per_wave = (size_t)2 * chunk * sizeof(float);
     int waves = (int)((48 * 1024) / per_wave);
     waves = waves < 1 ? 1 : (waves > kBwdWaves ? kBwdWaves : waves);
     const unsigned grid = (unsigned)((T_ + waves - 1) / waves);
-#define FMOE_LAUNCH_SMALL(R, P)                                                                                                  \
-    hipLaunchKernelGGL((route_backward_small_kernel<T, R, P>), dim3(grid), dim3(kBwdWaves * kWave), waves * per_wave, stream,    \
-                       (const T*)dgates, indices, logits, (const T*)dlogits_extra, extra_token, extra_half, dlogits, T_, nk, K, norm, waves)
+    const PrologueOperands to = operands != nullptr ? *operands : PrologueOperands{};
+#define FMOE_LAUNCH_SMALL(R, P, PREPARE)                                                                                                    \
+    hipLaunchKernelGGL((route_backward_small_kernel<T, R, P, PREPARE>), dim3(grid), dim3(kBwdWaves * kWave), waves * per_wave, stream,      \
+                       (const T*)dgates, indices, logits, (const T*)dlogits_extra, extra_token, extra_half, dlogits, T_, nk, K, norm, waves, to)
     // what a lane's registers hold; up to 256 keys a row pair also lies in LDS whole, for four waves
-    if (nk <= 2 * kWave && K <= kWave) FMOE_LAUNCH_SMALL(2, 1);
-    else if (nk <= 4 * kWave && K <= 2 * kWave) FMOE_LAUNCH_SMALL(4, 2);
-    else
+    if (nk <= 2 * kWave && K <= kWave) {
+        if (operands != nullptr) FMOE_LAUNCH_SMALL(2, 1, true);
+        else FMOE_LAUNCH_SMALL(2, 1, false);
+    } else if (route_backward_prepares(nk, K)) {
+        if (operands != nullptr) FMOE_LAUNCH_SMALL(4, 2, true);
+        else FMOE_LAUNCH_SMALL(4, 2, false);
+    } else
         hipLaunchKernelGGL((route_backward_kernel<T>), dim3(grid), dim3(kBwdWaves * kWave), waves * per_wave, stream,
                            (const T*)dgates, indices, logits, (const T*)dlogits_extra, extra_token, extra_half, dlogits, T_, nk, K, norm, waves,
                            chunk);
@@ -798,21 +823,23 @@ extern "C" int fmoe_route_backward(const void* dgates, const int64_t* indices, c
                                      top_k, dtype, norm_topk_prob, dlogits_fp32, (hipStream_t)stream);
 }
 
+bool fmoe::route_backward_prepares(int num_keys, int top_k) { return num_keys <= 4 * kWave && top_k <= 2 * kWave; }
+
 int fmoe::route_backward_impl(const void* dgates, const int64_t* indices, const float* logits_fp32, const void* dlogits_extra,
                               int64_t extra_token, int64_t extra_half, int64_t num_tokens, int num_keys, int top_k, int dtype,
-                              int norm_topk_prob, float* dlogits_fp32, hipStream_t s) {
+                              int norm_topk_prob, float* dlogits_fp32, hipStream_t s, const PrologueOperands* operands) {
     using namespace fmoe;
     FMOE_REQUIRE(dtype_ok(dtype), FMOE_ERR_BAD_DTYPE, "fmoe_route_backward: unknown dtype %d", dtype);
     FMOE_REQUIRE(num_tokens >= 0 && num_keys > 0 && top_k >= 0, FMOE_ERR_BAD_SHAPE,
                  "fmoe_route_backward: bad shape T=%lld nk=%d K=%d", (long long)num_tokens, num_keys, top_k);
     FMOE_REQUIRE(num_keys <= 32767, FMOE_ERR_UNSUPPORTED, "fmoe_route_backward: num_keys=%d > 32767", num_keys);
     if (num_tokens == 0) return FMOE_OK;
-    FMOE_REQUIRE(logits_fp32 && dlogits_fp32 && (top_k == 0 || (dgates && indices)), FMOE_ERR_NULL_POINTER,
+    FMOE_REQUIRE(logits_fp32 && (dlogits_fp32 || operands) && (top_k == 0 || (dgates && indices)), FMOE_ERR_NULL_POINTER,
                  "fmoe_route_backward: null tensor pointer");
     switch (dtype) {
-        case FMOE_F32: return launch_route_backward<float>(dgates, indices, logits_fp32, dlogits_extra, extra_token, extra_half, dlogits_fp32, num_tokens, num_keys, top_k, norm_topk_prob, s);
-        case FMOE_BF16: return launch_route_backward<bf16_t>(dgates, indices, logits_fp32, dlogits_extra, extra_token, extra_half, dlogits_fp32, num_tokens, num_keys, top_k, norm_topk_prob, s);
-        default: return launch_route_backward<f16_t>(dgates, indices, logits_fp32, dlogits_extra, extra_token, extra_half, dlogits_fp32, num_tokens, num_keys, top_k, norm_topk_prob, s);
+        case FMOE_F32: return launch_route_backward<float>(dgates, indices, logits_fp32, dlogits_extra, extra_token, extra_half, dlogits_fp32, num_tokens, num_keys, top_k, norm_topk_prob, s, operands);
+        case FMOE_BF16: return launch_route_backward<bf16_t>(dgates, indices, logits_fp32, dlogits_extra, extra_token, extra_half, dlogits_fp32, num_tokens, num_keys, top_k, norm_topk_prob, s, operands);
+        default: return launch_route_backward<f16_t>(dgates, indices, logits_fp32, dlogits_extra, extra_token, extra_half, dlogits_fp32, num_tokens, num_keys, top_k, norm_topk_prob, s, operands);
     }
 }
 

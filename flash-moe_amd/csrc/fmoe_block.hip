@@ -286,10 +286,14 @@ extern "C" int fmoe_block_backward(const void* dout, const void* dlogits, const 
     rc = fmoe_expert_backward_saved(dout, x, down_embed, up_embed, indices, sv + sp.off_gates, sv + sp.off_experts, num_tokens, hidden,
                                     num_experts, top_k, dtype, dx_experts, ddown_embed, dup_embed, dgates, stage, p.stage_bytes, stream);
     if (rc) return rc;
+    const float* mean_rstd = (const float*)(sv + sp.off_stats);
+    const bool prepares = route_backward_prepares(num_keys, top_k);
+    const PrologueOperands operands = prologue_operands(x, mean_rstd, num_tokens, hidden, num_keys, dtype, stage);
     rc = route_backward_impl(dgates, indices, logits32, dlogits, num_keys, num_tokens * num_keys, num_tokens, num_keys, top_k, dtype,
-                             norm_topk_prob, dlogits32, (hipStream_t)stream);
+                             norm_topk_prob, dlogits32, (hipStream_t)stream, prepares ? &operands : nullptr);
     if (rc) return rc;
     // the three token gradients are summed where the last of them is formed
-    return router_prologue_backward_impl(dlogits32, x, router_gate_w, (const float*)(sv + sp.off_stats), training, num_tokens, hidden,
-                                         num_keys, dtype, dx, drouter_gate_w, dx, dx_experts, stage, p.stage_bytes, (hipStream_t)stream);
+    return router_prologue_backward_impl(dlogits32, x, router_gate_w, mean_rstd, training, num_tokens, hidden,
+                                         num_keys, dtype, dx, drouter_gate_w, dx, dx_experts, stage, p.stage_bytes, (hipStream_t)stream,
+                                         prepares);
 }

@@ -92,19 +92,31 @@ int router_forward_impl(const void* x, const void* gate_w, void* running_mean, v
                         void* router_logits, float* logits_fp32, float* scores, int64_t* indices, void* gates,
                         uint32_t* row_offsets, uint32_t row_bytes, void* workspace, size_t workspace_bytes,
                         hipStream_t stream, int split_query = 0, int fixed_scratch = 0, float* mean_rstd_out = nullptr);
-// Arguments of fmoe_router_prologue_backward; addend0 / addend1 [T,H] (either may be NULL, and may be dx itself) are added to
+// What the products of the router prologue's backward read: d, the logits' gradients in the activation dtype (rows of n_pad values, whole
+// packets, zeros beyond 2 nk), and q = round((x - mean) * rstd).
+struct PrologueOperands {
+    void *d, *q;
+    int n_pad, hidden;
+    const void* x;
+    const float* mean_rstd;
+};
+PrologueOperands prologue_operands(const void* x, const float* mean_rstd, int64_t num_tokens, int hidden, int num_keys, int dtype, void* workspace);
+// Arguments of fmoe_router_prologue_backward; operands_ready: prologue_operands of this workspace are in place and stand for dlogits_fp32;
+// addend0 / addend1 [T,H] (either may be NULL, and may be dx itself) are added to
 // dx in fp32 before it is rounded.
 int router_prologue_backward_impl(const float* dlogits_fp32, const void* x, const void* gate_w, const float* mean_rstd,
                                   int training, int64_t num_tokens, int hidden, int num_keys, int dtype, void* dx,
                                   void* dgate_w, const void* addend0, const void* addend1, void* workspace,
-                                  size_t workspace_bytes, hipStream_t stream);
+                                  size_t workspace_bytes, hipStream_t stream, bool operands_ready = false);
 
 // (router_forward_impl: mean_rstd_out [2][H], when given, receives mean and 1/std instead of the workspace.)
 
 // fmoe_route_backward with the strides (in elements) of dlogits_extra per token and per half.
 int route_backward_impl(const void* dgates, const int64_t* indices, const float* logits_fp32, const void* dlogits_extra,
                         int64_t extra_token, int64_t extra_half, int64_t num_tokens, int num_keys, int top_k, int dtype,
-                        int norm_topk_prob, float* dlogits_fp32, hipStream_t stream);
+                        int norm_topk_prob, float* dlogits_fp32, hipStream_t stream, const PrologueOperands* operands = nullptr);
+// ... which writes the prologue's operands in place of dlogits_fp32 if these are given; for extents that it has a kernel for.
+bool route_backward_prepares(int num_keys, int top_k);
 
 // Column-slice schedule of the routed experts on row offsets that are already in place (off32; expert_workspace_offsets is where a
 // caller without a place of its own puts them), `workspace` as fmoe_expert_workspace_bytes describes; scores: NULL, or where the

@@ -759,7 +759,7 @@ PrologueBwdPlan plan_prologue_backward(int64_t T_, int H, int nk, int dtype) {
 template <typename T>
 int launch_prologue_backward(const float* dlogits, const void* x, const void* gate_w, const float* mean_rstd, int training,
                              int64_t T_, int H, int nk, int dtype, void* dx, void* dgate_w, const void* addend0, const void* addend1,
-                             void* workspace, hipStream_t s) {
+                             void* workspace, hipStream_t s, bool operands_ready) {
     constexpr int V = Elem<T>::kVec;
     const PrologueBwdPlan p = plan_prologue_backward(T_, H, nk, dtype);
     const ProloguePlan rows = plan_prologue(T_, H, nk);
@@ -770,9 +770,11 @@ int launch_prologue_backward(const float* dlogits, const void* x, const void* ga
     const int widest = H > p.n_pad ? H : p.n_pad;
     void* part = ws + p.off_part;
     const int col_blocks = ((widest + V - 1) / V + 255) / 256;
-    hipLaunchKernelGGL((prologue_bwd_prepare_kernel<T>), dim3((unsigned)(T_ * col_blocks)), dim3(256), 0, s, dlogits,
-                       (const T*)x, mean_rstd, d16, q, H, N, p.n_pad, col_blocks);
-    FMOE_CHECK_LAUNCH("fmoe_router_prologue_backward(prepare)");
+    if (!operands_ready) {
+        hipLaunchKernelGGL((prologue_bwd_prepare_kernel<T>), dim3((unsigned)(T_ * col_blocks)), dim3(256), 0, s, dlogits,
+                           (const T*)x, mean_rstd, d16, q, H, N, p.n_pad, col_blocks);
+        FMOE_CHECK_LAUNCH("fmoe_router_prologue_backward(prepare)");
+    }
     BackwardProduct products[2];
     prologue_products((int)T_, H, N, p.n_pad, products);
     products[0].A = products[1].A = d16;
@@ -1019,10 +1021,16 @@ extern "C" int fmoe_router_prologue_backward(const float* dlogits_fp32, const vo
                                                dgate_w, nullptr, nullptr, workspace, workspace_bytes, (hipStream_t)stream);
 }
 
+fmoe::PrologueOperands fmoe::prologue_operands(const void* x, const float* mean_rstd, int64_t num_tokens, int hidden, int num_keys, int dtype,
+                                               void* workspace) {
+    const PrologueBwdPlan p = plan_prologue_backward(num_tokens, hidden, num_keys, dtype);
+    return {(char*)workspace + p.off_d16, (char*)workspace + p.off_q, p.n_pad, hidden, x, mean_rstd};
+}
+
 int fmoe::router_prologue_backward_impl(const float* dlogits_fp32, const void* x, const void* gate_w, const float* mean_rstd,
                                         int training, int64_t num_tokens, int hidden, int num_keys, int dtype, void* dx,
                                         void* dgate_w, const void* addend0, const void* addend1, void* workspace,
-                                        size_t workspace_bytes, hipStream_t s) {
+                                        size_t workspace_bytes, hipStream_t s, bool operands_ready) {
     using namespace fmoe;
     FMOE_REQUIRE(dtype_ok(dtype), FMOE_ERR_BAD_DTYPE, "fmoe_router_prologue_backward: unknown dtype %d", dtype);
     FMOE_REQUIRE(num_tokens > 0 && hidden > 0 && num_keys > 0 && num_tokens < (1ll << 24), FMOE_ERR_BAD_SHAPE,
@@ -1030,7 +1038,7 @@ int fmoe::router_prologue_backward_impl(const float* dlogits_fp32, const void* x
     const int vec = (int)(16 / dtype_size(dtype));
     FMOE_REQUIRE(hidden % vec == 0, FMOE_ERR_ALIGNMENT,
                  "fmoe_router_prologue_backward: hidden=%d must be a multiple of %d", hidden, vec);
-    FMOE_REQUIRE(dlogits_fp32 && x && gate_w && mean_rstd && dx && dgate_w, FMOE_ERR_NULL_POINTER,
+    FMOE_REQUIRE((dlogits_fp32 || operands_ready) && x && gate_w && mean_rstd && dx && dgate_w, FMOE_ERR_NULL_POINTER,
                  "fmoe_router_prologue_backward: null tensor pointer");
     FMOE_REQUIRE(aligned16(x) && aligned16(dx) && aligned16(dlogits_fp32) && aligned16(mean_rstd), FMOE_ERR_ALIGNMENT,
                  "fmoe_router_prologue_backward: tensor pointers must be 16-byte aligned");
@@ -1038,8 +1046,8 @@ int fmoe::router_prologue_backward_impl(const float* dlogits_fp32, const void* x
     FMOE_REQUIRE(workspace && workspace_bytes >= need && aligned16(workspace), FMOE_ERR_WORKSPACE,
                  "fmoe_router_prologue_backward: workspace of %zu bytes needed, %zu given", need, workspace_bytes);
     switch (dtype) {
-        case FMOE_F32: return launch_prologue_backward<float>(dlogits_fp32, x, gate_w, mean_rstd, training, num_tokens, hidden, num_keys, dtype, dx, dgate_w, addend0, addend1, workspace, s);
-        case FMOE_BF16: return launch_prologue_backward<bf16_t>(dlogits_fp32, x, gate_w, mean_rstd, training, num_tokens, hidden, num_keys, dtype, dx, dgate_w, addend0, addend1, workspace, s);
-        default: return launch_prologue_backward<f16_t>(dlogits_fp32, x, gate_w, mean_rstd, training, num_tokens, hidden, num_keys, dtype, dx, dgate_w, addend0, addend1, workspace, s);
+        case FMOE_F32: return launch_prologue_backward<float>(dlogits_fp32, x, gate_w, mean_rstd, training, num_tokens, hidden, num_keys, dtype, dx, dgate_w, addend0, addend1, workspace, s, operands_ready);
+        case FMOE_BF16: return launch_prologue_backward<bf16_t>(dlogits_fp32, x, gate_w, mean_rstd, training, num_tokens, hidden, num_keys, dtype, dx, dgate_w, addend0, addend1, workspace, s, operands_ready);
+        default: return launch_prologue_backward<f16_t>(dlogits_fp32, x, gate_w, mean_rstd, training, num_tokens, hidden, num_keys, dtype, dx, dgate_w, addend0, addend1, workspace, s, operands_ready);
     }
 }

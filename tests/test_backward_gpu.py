@@ -544,6 +544,37 @@ def test_block_backward_with_a_key_count_that_is_not_a_multiple_of_four(dtype):
     assert gp["router_gate.weight"].shape == (20, H) and gp["router_gate.weight"].abs().sum() > 0
 
 
+@pytest.mark.parametrize("dtype,H,nk,K", [
+    (torch.bfloat16, 8, 3, 2), (torch.float32, 4, 1, 1),             # one packet to a row, padded rows of d
+    (torch.float16, 776, 65, 17), (torch.bfloat16, 520, 129, 65),    # a packet more than whole waves; either kernel of the registers
+    (torch.bfloat16, 1032, 256, 128), (torch.float32, 264, 256, 64),
+    (torch.bfloat16, 72, 257, 4), (torch.bfloat16, 72, 256, 129),    # beyond them: gradients in fp32 and a launch of their own
+])
+def test_block_backward_operands_from_the_routing_gradient(dtype, H, nk, K):
+    """The routing gradient's kernel writes what the prologue's products read; the composition of ops forms it on its own."""
+    from flash_moe.modules.flash_moe import FlashMoE, FlashMoEConfig
+
+    m = FlashMoE(FlashMoEConfig(H, 64, "silu", nk * nk, K, True)).to(device="cuda", dtype=dtype)
+    with torch.no_grad():
+        m.router_gate.weight.normal_(0.0, 2.0 / H**0.5)
+        m.down_embed.weight.normal_(0.0, H**-0.5)       # scores of order 1: with the default of 1 the gradients pass 65504 in fp16
+        m.up_embed.weight.normal_(0.0, H**-0.5)
+    x = torch.randn(1, 70, H, generator=gen(3)).to(dtype).cuda()
+    wl = (torch.randn(2, 70, nk, generator=gen(7)) * 0.1).cuda()
+    results = []
+    for forward in (m.forward_autograd, m.forward_autograd_ops):
+        for p in m.parameters():
+            p.grad = None
+        m.router_norm.reset_running_stats()
+        xg = x.clone().requires_grad_(True)
+        y, logits = forward(xg)
+        (y.float().square().sum() + (logits.float() * wl).sum()).backward()
+        results.append((xg.grad, m.router_gate.weight.grad.clone()))
+    # both round the same fp32 gradients to the activation dtype; the 16-bit gates that reach them differ in their last bit
+    for a, b in zip(*results):
+        assert torch.isfinite(a).all() and rel_fro(a, b) < {torch.float32: 1e-4, torch.bfloat16: 3e-2, torch.float16: 6e-3}[dtype]
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_mlp_backward_with_saved_products_equals_recomputation(dtype):
     from flash_moe.ops.hip.flash_mlp import mlp_backward, mlp_forward, mlp_forward_saving
