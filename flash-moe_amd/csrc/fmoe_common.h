@@ -102,12 +102,18 @@ struct PrologueOperands {
 };
 PrologueOperands prologue_operands(const void* x, const float* mean_rstd, int64_t num_tokens, int hidden, int num_keys, int dtype, void* workspace);
 // Arguments of fmoe_router_prologue_backward; operands_ready: prologue_operands of this workspace are in place and stand for dlogits_fp32;
-// addend0 / addend1 [T,H] (either may be NULL, and may be dx itself) are added to
-// dx in fp32 before it is rounded.
+// more: token gradients that are added to dx in fp32 before it is rounded, any of them NULL: two tensors [T,H], each of which may be
+// dx itself, and fp32 planes [slices][T,H].
+struct TokenGradients {
+    const void* addend0;
+    const void* addend1;
+    const float* planes;
+    int slices;
+};
 int router_prologue_backward_impl(const float* dlogits_fp32, const void* x, const void* gate_w, const float* mean_rstd,
                                   int training, int64_t num_tokens, int hidden, int num_keys, int dtype, void* dx,
-                                  void* dgate_w, const void* addend0, const void* addend1, void* workspace,
-                                  size_t workspace_bytes, hipStream_t stream, bool operands_ready = false);
+                                  void* dgate_w, const TokenGradients& more, void* workspace, size_t workspace_bytes,
+                                  hipStream_t stream, bool operands_ready = false);
 
 // (router_forward_impl: mean_rstd_out [2][H], when given, receives mean and 1/std instead of the workspace.)
 
@@ -206,8 +212,22 @@ int gemm_backward(const BackwardProduct& product, int dtype, void* workspace, si
 // Scratch of gemm_backward for the sums of a sliced k range (0 when it needs none).
 size_t gemm_backward_workspace_bytes(int M, int N, int K, int segments, int dtype);
 // Several products that do not depend on each other (at most four share a launch); their pointers do not matter for the scratch.
-int gemm_backward(const BackwardProduct* products, int count, int dtype, void* workspace, size_t workspace_bytes, hipStream_t stream);
+// keep: leave the sum of one product's slices to the caller, if it is cut.
+struct KeptPlanes {
+    int product;
+    const float* planes;          // NULL: the product is where it belongs
+    int slices;
+};
+int gemm_backward(const BackwardProduct* products, int count, int dtype, void* workspace, size_t workspace_bytes, hipStream_t stream,
+                  KeptPlanes* keep = nullptr);
 size_t gemm_backward_workspace_bytes(const BackwardProduct* products, int count, int dtype);
+
+// fmoe_mlp_backward with the products kept, whose scratch for slices of k lies apart from its workspace; dx may stay there as planes.
+struct MlpBackwardBytes { size_t workspace, planes; };
+MlpBackwardBytes mlp_backward_bytes(int64_t num_tokens, int hidden, int intermediate, int dtype);
+int mlp_backward_impl(const void* dy, const void* x, const void* gate_w, const void* up_w, const void* down_w, const void* saved_products,
+                      int64_t num_tokens, int hidden, int intermediate, int dtype, void* dx, void* dgate_w, void* dup_w, void* ddown_w,
+                      void* workspace, size_t workspace_bytes, void* planes, KeptPlanes* keep_dx, hipStream_t stream);
 
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 inline size_t dtype_size(int dtype) { return dtype == FMOE_F32 ? 4 : 2; }

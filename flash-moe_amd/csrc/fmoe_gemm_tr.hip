@@ -346,7 +346,8 @@ bool addressable(const BackwardProduct& p, int dtype) {
     return packets && (double)p.K * p.ldb < most && (p.layout == kBlasTN ? (double)p.K * p.lda < most : 256.0 * p.lda < most);
 }
 
-template <typename T> void launch_group(const BackwardProduct* p, int count, const GroupPlan& plan, void* workspace, hipStream_t stream) {
+template <typename T>
+void launch_group(const BackwardProduct* p, int count, const GroupPlan& plan, void* workspace, hipStream_t stream, KeptPlanes* keep) {
     const int xcds = chip_info().xcds, rows = kTileRows[plan.shape], cols = kTileCols[plan.shape];
     Group g = {};
     Sums sums = {};
@@ -368,7 +369,12 @@ template <typename T> void launch_group(const BackwardProduct* p, int count, con
                   plan.slices[i], blocks, q.layout == kBlasTN};
         if (plan.slices[i] > 1) {
             g.m[k].out = planes;
-            sums.m[sliced++] = {(const float*)planes, q.C, (int64_t)q.M * q.N / Elem<T>::kVec, plan.slices[i], 0};
+            if (keep != nullptr && keep->product == i) {
+                keep->planes = (const float*)planes;
+                keep->slices = plan.slices[i];
+            } else {
+                sums.m[sliced++] = {(const float*)planes, q.C, (int64_t)q.M * q.N / Elem<T>::kVec, plan.slices[i], 0};
+            }
             planes += round_up((size_t)plan.slices[i] * q.M * q.N * sizeof(float), 256);
         }
         blocks += (g.m[k].tiles_m * g.m[k].tiles_n * plan.slices[i] + xcds - 1) / xcds * xcds;
@@ -424,15 +430,15 @@ size_t gemm_backward_workspace_bytes(const BackwardProduct* p, int count, int dt
     return most;
 }
 
-int gemm_backward(const BackwardProduct* p, int count, int dtype, void* workspace, size_t workspace_bytes, hipStream_t stream) {
+int gemm_backward(const BackwardProduct* p, int count, int dtype, void* workspace, size_t workspace_bytes, hipStream_t stream, KeptPlanes* keep) {
     const GroupPlan plan = plan_group_of(p, count, dtype);
     bool together = plan.shape >= 0 && group_planes_bytes(p, count, plan) <= workspace_bytes;
     for (int i = 0; i < count; ++i) together = together && addressable(p[i], dtype);
     if (together) {
         switch (dtype) {
-            case FMOE_F32: launch_group<float>(p, count, plan, workspace, stream); break;
-            case FMOE_BF16: launch_group<bf16_t>(p, count, plan, workspace, stream); break;
-            default: launch_group<f16_t>(p, count, plan, workspace, stream); break;
+            case FMOE_F32: launch_group<float>(p, count, plan, workspace, stream, keep); break;
+            case FMOE_BF16: launch_group<bf16_t>(p, count, plan, workspace, stream, keep); break;
+            default: launch_group<f16_t>(p, count, plan, workspace, stream, keep); break;
         }
         FMOE_CHECK_LAUNCH("backward products");
         return FMOE_OK;

@@ -138,11 +138,23 @@ extern "C" size_t fmoe_mlp_backward_saved_workspace_bytes(int64_t num_tokens, in
     return fmoe::plan_mlp_backward(num_tokens, hidden, intermediate, dtype, true).bytes;
 }
 
+fmoe::MlpBackwardBytes fmoe::mlp_backward_bytes(int64_t num_tokens, int hidden, int intermediate, int dtype) {
+    const MlpBwdPlan p = plan_mlp_backward(num_tokens, hidden, intermediate, dtype, true);
+    return {p.off_part, p.part_bytes};
+}
+
 extern "C" int fmoe_mlp_backward(const void* dy, const void* x, const void* gate_w, const void* up_w, const void* down_w,
                                  const void* saved_products, int64_t num_tokens, int hidden, int intermediate, int dtype, void* dx, void* dgate_w, void* dup_w,
                                  void* ddown_w, void* workspace, size_t workspace_bytes, void* stream) {
+    fmoe::clear_error();
+    return fmoe::mlp_backward_impl(dy, x, gate_w, up_w, down_w, saved_products, num_tokens, hidden, intermediate, dtype, dx, dgate_w, dup_w, ddown_w,
+                                   workspace, workspace_bytes, nullptr, nullptr, (hipStream_t)stream);
+}
+
+int fmoe::mlp_backward_impl(const void* dy, const void* x, const void* gate_w, const void* up_w, const void* down_w, const void* saved_products,
+                            int64_t num_tokens, int hidden, int intermediate, int dtype, void* dx, void* dgate_w, void* dup_w, void* ddown_w,
+                            void* workspace, size_t workspace_bytes, void* planes, KeptPlanes* keep_dx, hipStream_t s) {
     using namespace fmoe;
-    clear_error();
     FMOE_REQUIRE(dtype_ok(dtype), FMOE_ERR_BAD_DTYPE, "fmoe_mlp_backward: unknown dtype %d", dtype);
     FMOE_REQUIRE(num_tokens > 0 && hidden > 0 && intermediate > 0, FMOE_ERR_BAD_SHAPE, "fmoe_mlp_backward: bad shape T=%lld H=%d I=%d",
                  (long long)num_tokens, hidden, intermediate);
@@ -153,13 +165,13 @@ extern "C" int fmoe_mlp_backward(const void* dy, const void* x, const void* gate
     FMOE_REQUIRE(dy && x && gate_w && up_w && down_w && dx && dgate_w && dup_w && ddown_w, FMOE_ERR_NULL_POINTER,
                  "fmoe_mlp_backward: null tensor pointer");
     const MlpBwdPlan p = plan_mlp_backward(num_tokens, hidden, intermediate, dtype, saved_products != nullptr);
-    FMOE_REQUIRE(workspace && workspace_bytes >= p.bytes && aligned16(workspace), FMOE_ERR_WORKSPACE,
-                 "fmoe_mlp_backward: workspace of %zu bytes needed, %zu given", p.bytes, workspace_bytes);
-    hipStream_t s = (hipStream_t)stream;
+    const size_t need = planes != nullptr ? p.off_part : p.bytes;
+    FMOE_REQUIRE(workspace && workspace_bytes >= need && aligned16(workspace), FMOE_ERR_WORKSPACE,
+                 "fmoe_mlp_backward: workspace of %zu bytes needed, %zu given", need, workspace_bytes);
     char* ws = (char*)workspace;
     void *a = ws + p.off_a, *b = ws + p.off_b, *dh = ws + p.off_dh, *h = ws + p.off_h;
     char* dab = ws + p.off_dab;
-    void* part = ws + p.off_part;
+    void* part = planes != nullptr ? planes : ws + p.off_part;
     const int T_ = (int)num_tokens, H = hidden, I = intermediate;
     const size_t elt = dtype_size(dtype);
 
@@ -170,9 +182,9 @@ extern "C" int fmoe_mlp_backward(const void* dy, const void* x, const void* gate
         b = (char*)a + (size_t)num_tokens * I * elt;
     } else {
         // recompute them with the forward's NT kernel ("down" form: out[T,N] = act[T,K] W[N,K]^T)
-        rc = fmoe_mlp_down(x, gate_w, num_tokens, I, H, dtype, nullptr, a, stream);
+        rc = fmoe_mlp_down(x, gate_w, num_tokens, I, H, dtype, nullptr, a, s);
         if (rc) return rc;
-        rc = fmoe_mlp_down(x, up_w, num_tokens, I, H, dtype, nullptr, b, stream);
+        rc = fmoe_mlp_down(x, up_w, num_tokens, I, H, dtype, nullptr, b, s);
         if (rc) return rc;
     }
 
@@ -190,5 +202,6 @@ extern "C" int fmoe_mlp_backward(const void* dy, const void* x, const void* gate
     q[1].A = dab, q[1].B0 = gate_w, q[1].B1 = up_w, q[1].C = dx;
     q[2].A = dab, q[2].B0 = x, q[2].C = dgate_w;
     q[3].A = db, q[3].B0 = x, q[3].C = dup_w;
-    return gemm_backward(q, count, dtype, part, p.part_bytes, s);
+    if (keep_dx != nullptr) *keep_dx = {1, nullptr, 0};
+    return gemm_backward(q, count, dtype, part, p.part_bytes, s, keep_dx);
 }

@@ -596,15 +596,16 @@ __global__ __launch_bounds__(256) void prologue_bwd_prepare_kernel(const float* 
     }
 }
 
-// partial: [row_blocks][2][H] = (sum dq, sum dq * xhat) over the block's rows; same geometry as bn_partial_kernel.
+// partial: [row_blocks][2][H] = (sum dq, sum dq * xhat) over the block's rows; geometry of bn_block_stats_kernel: at most
+// kFoldMaxRowBlocks tall blocks, so that the next launch adds them itself.
 template <typename T>
 __global__ __launch_bounds__(kStatsThreads) void bn_bwd_partial_kernel(const T* __restrict__ x, const T* __restrict__ dq,
                                                                       const float* __restrict__ mean_rstd, int64_t num_tokens,
                                                                       int hidden, int rows_per_block, float* __restrict__ partial) {
     constexpr int V = Elem<T>::kVec;
-    __shared__ float red[3][2][kWave * V];
+    __shared__ float red[3][2][8 * V];
     const int lane = lane_id(), wave = (int)(threadIdx.x >> 6);
-    const int col = ((int)blockIdx.y * kWave + lane) * V;
+    const int col = ((int)blockIdx.y * 8 + (lane & 7)) * V;
     const bool col_ok = col < hidden;
     const int64_t r0 = (int64_t)blockIdx.x * rows_per_block;
     const int64_t r1 = r0 + rows_per_block < num_tokens ? r0 + rows_per_block : num_tokens;
@@ -616,18 +617,39 @@ __global__ __launch_bounds__(kStatsThreads) void bn_bwd_partial_kernel(const T* 
         s1[v] = s2[v] = 0.0f;
     }
     if (col_ok) {
-        for (int64_t r = r0 + wave; r < r1; r += 4) {
-            float xv[V], gv[V];
-            unpack16<T>(*reinterpret_cast<const u32x4_t*>(x + r * hidden + col), xv);
-            unpack16<T>(*reinterpret_cast<const u32x4_t*>(dq + r * hidden + col), gv);
+        constexpr int kBatch = 4;                                // rows of x and dq issued together: one memory round trip per batch
+        for (int64_t rb = r0 + wave * 8 + (lane >> 3); rb < r1; rb += 32 * kBatch) {
+            u32x4_t raw[kBatch], raw_dq[kBatch];
 #pragma unroll
-            for (int v = 0; v < V; ++v) {
-                s1[v] += gv[v];
-                s2[v] = __builtin_fmaf(gv[v], (xv[v] - mean[v]) * rstd[v], s2[v]);
+            for (int i = 0; i < kBatch; ++i) {
+                const int64_t r = rb + 32 * i < r1 ? rb + 32 * i : r1 - 1;
+                raw[i] = *reinterpret_cast<const u32x4_t*>(x + r * hidden + col);
+                raw_dq[i] = *reinterpret_cast<const u32x4_t*>(dq + r * hidden + col);
+            }
+#pragma unroll
+            for (int i = 0; i < kBatch; ++i) {
+                if (rb + 32 * i >= r1) continue;
+                float xv[V], gv[V];
+                unpack16<T>(raw[i], xv);
+                unpack16<T>(raw_dq[i], gv);
+#pragma unroll
+                for (int v = 0; v < V; ++v) {
+                    s1[v] += gv[v];
+                    s2[v] = __builtin_fmaf(gv[v], (xv[v] - mean[v]) * rstd[v], s2[v]);
+                }
             }
         }
     }
-    if (wave > 0) {
+    // the 8 row lanes of a wave, then waves 1..3 -> wave 0 through LDS; fixed order
+#pragma unroll
+    for (int v = 0; v < V; ++v) {
+#pragma unroll
+        for (int m = 8; m < kWave; m <<= 1) {
+            s1[v] += __shfl_xor(s1[v], m, kWave);
+            s2[v] += __shfl_xor(s2[v], m, kWave);
+        }
+    }
+    if (wave > 0 && lane < 8) {
 #pragma unroll
         for (int v = 0; v < V; ++v) {
             red[wave - 1][0][lane * V + v] = s1[v];
@@ -635,99 +657,142 @@ __global__ __launch_bounds__(kStatsThreads) void bn_bwd_partial_kernel(const T* 
         }
     }
     __syncthreads();
-    if (wave == 0 && col_ok) {
+    if (wave == 0 && lane < 8 && col_ok) {
+#pragma unroll
+        for (int w = 0; w < 3; ++w)
+#pragma unroll
+            for (int v = 0; v < V; ++v) {
+                s1[v] += red[w][0][lane * V + v];
+                s2[v] += red[w][1][lane * V + v];
+            }
         float* out = partial + (int64_t)blockIdx.x * 2 * hidden;
 #pragma unroll
         for (int v = 0; v < V; ++v) {
-            float a = s1[v], b = s2[v];
-#pragma unroll
-            for (int w = 0; w < 3; ++w) {
-                a += red[w][0][lane * V + v];
-                b += red[w][1][lane * V + v];
-            }
-            out[col + v] = a;
-            out[hidden + col + v] = b;
+            out[col + v] = s1[v];
+            out[hidden + col + v] = s2[v];
         }
     }
 }
 
-// sums[0][c] = sum over row blocks of partial[.][0][c] / T, sums[1][c] likewise: the two column means of the formula.
-// 32 columns to a workgroup, each summed by eight threads with eight loads in flight: bound by two memory round trips (one thread to a
-// column, 16 loads at a time: 7.5 us for 4.9 at 1024 columns and 128 row blocks).
-__global__ __launch_bounds__(256) void bn_bwd_finalize_kernel(const float* __restrict__ partial, int row_blocks, int hidden,
-                                                              float inv_tokens, float* __restrict__ sums) {
-    __shared__ float red[8][32];
-    const int c = (int)(blockIdx.x * 32 + (threadIdx.x & 31)), group = (int)(threadIdx.x >> 5);
-    const bool col_ok = c < 2 * hidden;
-    float acc[8];
-#pragma unroll
-    for (int u = 0; u < 8; ++u) acc[u] = 0.0f;
-    for (int b0 = group; b0 < row_blocks; b0 += 64) {
-        float got[8];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            const int b = b0 + 8 * u < row_blocks ? b0 + 8 * u : row_blocks - 1;      // clamped: every load is unconditional
-            got[u] = partial[(int64_t)b * 2 * hidden + (col_ok ? c : 0)];
-        }
-#pragma unroll
-        for (int u = 0; u < 8; ++u) acc[u] += b0 + 8 * u < row_blocks ? got[u] : 0.0f;
-    }
-    float a = 0.0f;
-#pragma unroll
-    for (int u = 0; u < 8; ++u) a += acc[u];
-    red[group][threadIdx.x & 31] = a;
-    __syncthreads();
-    if (group != 0 || !col_ok) return;
-#pragma unroll
-    for (int g = 1; g < 8; ++g) a += red[g][threadIdx.x];
-    sums[c] = a * inv_tokens;
-}
-
+// dx, and the block's other token gradients added in fp32: addend0 and addend1 (either may be NULL, or dx itself: a thread reads its
+// packet before it writes), and fp32 planes of slices of k (of the MLP's dx, whose sum nobody else needs).
+// A workgroup takes a strip of 64 packets and rows_per_block rows, its waves rows 4 apart.  training: it first adds the blocks'
+// column sums to the two means of the formula, a quarter of the blocks to a wave.  Where a launch of its own had formed the means: 4096
+// tokens, 1024 columns 22.8 us in three launches, 18.7 in two; 615 tokens, 776 columns, with four planes that another launch had
+// added, 17.6 in four and 10.7 in two.
 template <typename T>
 __global__ __launch_bounds__(256) void bn_bwd_apply_kernel(const T* __restrict__ x, const T* __restrict__ dq,
-                                                           const float* __restrict__ mean_rstd, const float* __restrict__ sums,
-                                                           const T* addend0, const T* addend1, T* dx, int hidden,
-                                                           int col_blocks, int training) {
-    constexpr int V = Elem<T>::kVec;
-    const uint32_t row = blockIdx.x / (uint32_t)col_blocks;
-    const int col = ((int)(blockIdx.x % (uint32_t)col_blocks) * 256 + (int)threadIdx.x) * V;
-    if (col >= hidden) return;
-    const int64_t at = (int64_t)row * hidden + col;
-    float xv[V], gv[V], ov[V], mean[V], rstd[V], m1[V], m2[V];
-    unpack16<T>(*reinterpret_cast<const u32x4_t*>(x + at), xv);
-    unpack16<T>(*reinterpret_cast<const u32x4_t*>(dq + at), gv);
-    // the four per-column vectors as 16-byte loads, all requested before any is used
+                                                           const float* __restrict__ mean_rstd, const float* __restrict__ partial,
+                                                           int row_blocks, float inv_tokens, const T* addend0, const T* addend1,
+                                                           const float* __restrict__ planes, int slices, T* dx, int64_t num_tokens,
+                                                           int hidden, int rows_per_block) {
+    constexpr int V = Elem<T>::kVec, kShare = kFoldMaxRowBlocks / 4;
+    __shared__ __attribute__((aligned(16))) float shared_sums[4][2][kWave * V];
+    const int lane = lane_id(), wave = (int)(threadIdx.x >> 6);
+    const int col = ((int)blockIdx.y * kWave + lane) * V;
+    const bool col_ok = col < hidden;
+    const int at_col = col_ok ? col : 0;
+    // a wave's next row is asked for before the current one is worked on, the first before the means
+    const int64_t r0 = (int64_t)blockIdx.x * rows_per_block;
+    const int64_t r1 = r0 + rows_per_block < num_tokens ? r0 + rows_per_block : num_tokens;
+    const T* const rows[4] = {x, dq, addend0 != nullptr ? addend0 : x, addend1 != nullptr ? addend1 : x};
+    u32x4_t raw[4];
+    auto load = [&](int64_t r) {
+        const int64_t at = (r < r1 ? r : r1 - 1) * hidden + at_col;
 #pragma unroll
-    for (int h = 0; h < V / 4; ++h) {
-        const f32x4_t a = *reinterpret_cast<const f32x4_t*>(mean_rstd + col + 4 * h);
-        const f32x4_t b = *reinterpret_cast<const f32x4_t*>(mean_rstd + hidden + col + 4 * h);
-        const f32x4_t c = training ? *reinterpret_cast<const f32x4_t*>(sums + col + 4 * h) : f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-        const f32x4_t d = training ? *reinterpret_cast<const f32x4_t*>(sums + hidden + col + 4 * h) : f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+        for (int i = 0; i < 4; ++i) raw[i] = *reinterpret_cast<const u32x4_t*>(rows[i] + at);
+    };
+    load(r0 + wave);
+    float mean[V], rstd[V], m1[V], m2[V];
+#pragma unroll
+    for (int v = 0; v < V; v += 4) {
+        const f32x4_t a = *reinterpret_cast<const f32x4_t*>(mean_rstd + at_col + v);
+        const f32x4_t b = *reinterpret_cast<const f32x4_t*>(mean_rstd + hidden + at_col + v);
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-            mean[4 * h + j] = a[j];
-            rstd[4 * h + j] = b[j];
-            m1[4 * h + j] = c[j];
-            m2[4 * h + j] = d[j];
+            mean[v + j] = a[j];
+            rstd[v + j] = b[j];
+            m1[v + j] = m2[v + j] = 0.0f;            // evaluation mode: the formula reduces to rstd * dq
         }
     }
-    // evaluation mode: m1 = m2 = 0 and the formula reduces to rstd * dq
+    if (partial != nullptr) {
+        f32x4_t got[kShare][2][V / 4];
 #pragma unroll
-    for (int v = 0; v < V; ++v) ov[v] = rstd[v] * (gv[v] - m1[v] - (xv[v] - mean[v]) * rstd[v] * m2[v]);
-    // the block's other two token gradients; a thread reads its packet of them before it writes dx, which may be one of them
-    for (const T* addend : {addend0, addend1}) {
-        if (addend == nullptr) continue;
-        float av[V];
-        unpack16<T>(*reinterpret_cast<const u32x4_t*>(addend + at), av);
+        for (int u = 0; u < kShare; ++u) {
+            const int b = wave * kShare + u < row_blocks ? wave * kShare + u : 0;      // clamped: every load is unconditional
 #pragma unroll
-        for (int v = 0; v < V; ++v) ov[v] += av[v];
+            for (int h = 0; h < 2; ++h)
+#pragma unroll
+                for (int v = 0; v < V; v += 4) got[u][h][v / 4] = *reinterpret_cast<const f32x4_t*>(partial + (int64_t)(2 * b + h) * hidden + at_col + v);
+        }
+#pragma unroll
+        for (int u = 0; u < kShare; ++u) {
+            if (wave * kShare + u >= row_blocks) continue;
+#pragma unroll
+            for (int v = 0; v < V; ++v) {
+                m1[v] += got[u][0][v / 4][v % 4];
+                m2[v] += got[u][1][v / 4][v % 4];
+            }
+        }
+#pragma unroll
+        for (int v = 0; v < V; v += 4) {
+            *reinterpret_cast<f32x4_t*>(&shared_sums[wave][0][lane * V + v]) = f32x4_t{m1[v], m1[v + 1], m1[v + 2], m1[v + 3]};
+            *reinterpret_cast<f32x4_t*>(&shared_sums[wave][1][lane * V + v]) = f32x4_t{m2[v], m2[v + 1], m2[v + 2], m2[v + 3]};
+        }
+        __syncthreads();
+#pragma unroll
+        for (int v = 0; v < V; v += 4) {
+            f32x4_t a = *reinterpret_cast<const f32x4_t*>(&shared_sums[0][0][lane * V + v]);
+            f32x4_t b = *reinterpret_cast<const f32x4_t*>(&shared_sums[0][1][lane * V + v]);
+#pragma unroll
+            for (int w = 1; w < 4; ++w) {
+                a += *reinterpret_cast<const f32x4_t*>(&shared_sums[w][0][lane * V + v]);
+                b += *reinterpret_cast<const f32x4_t*>(&shared_sums[w][1][lane * V + v]);
+            }
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                m1[v + j] = a[j] * inv_tokens;
+                m2[v + j] = b[j] * inv_tokens;
+            }
+        }
     }
-    *reinterpret_cast<u32x4_t*>(dx + at) = pack16<T>(ov);
+    if (!col_ok) return;
+    for (int64_t r = r0 + wave; r < r1; r += 4) {
+        const int64_t at = r * hidden + col;
+        float xv[V], gv[V], ov[V], more[2][V];
+        unpack16<T>(raw[0], xv);
+        unpack16<T>(raw[1], gv);
+        unpack16<T>(raw[2], more[0]);
+        unpack16<T>(raw[3], more[1]);
+        if (r + 4 < r1) load(r + 4);             // never this row, which may be written in place
+#pragma unroll
+        for (int v = 0; v < V; ++v) ov[v] = rstd[v] * (gv[v] - m1[v] - (xv[v] - mean[v]) * rstd[v] * m2[v]);
+        if (planes != nullptr) {
+            float sum[V];
+#pragma unroll
+            for (int v = 0; v < V; ++v) sum[v] = 0.0f;
+            for (int s = 0; s < slices; ++s)
+#pragma unroll
+                for (int v = 0; v < V; v += 4) {
+                    const f32x4_t p = *reinterpret_cast<const f32x4_t*>(planes + ((int64_t)s * num_tokens + r) * hidden + col + v);
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) sum[v + j] += p[j];
+                }
+#pragma unroll
+            for (int v = 0; v < V; ++v) ov[v] += sum[v];
+        }
+#pragma unroll
+        for (int v = 0; v < V; ++v) {
+            if (addend0 != nullptr) ov[v] += more[0][v];
+            if (addend1 != nullptr) ov[v] += more[1][v];
+        }
+        *reinterpret_cast<u32x4_t*>(dx + at) = pack16<T>(ov);
+    }
 }
 
 struct PrologueBwdPlan {
     int n_pad;            // row length of d in the activation dtype: 2 * nk rounded up to whole packets
-    size_t off_d16, off_q, off_dq, off_partial, off_sums, off_part, part_bytes, bytes;
+    size_t off_d16, off_q, off_dq, off_partial, off_part, part_bytes, bytes;
 };
 
 // The two products, extents only.
@@ -746,8 +811,7 @@ PrologueBwdPlan plan_prologue_backward(int64_t T_, int H, int nk, int dtype) {
     p.off_d16 = take((size_t)T_ * p.n_pad * elt);
     p.off_q = take((size_t)T_ * H * elt);
     p.off_dq = take((size_t)T_ * H * elt);
-    p.off_partial = take((size_t)kMaxRowBlocks * 2 * H * 4);
-    p.off_sums = take((size_t)2 * H * 4);
+    p.off_partial = take((size_t)kFoldMaxRowBlocks * 2 * H * 4);
     BackwardProduct products[2];
     prologue_products(t, H, 2 * nk, p.n_pad, products);
     p.part_bytes = gemm_backward_workspace_bytes(products, 2, dtype);
@@ -758,14 +822,14 @@ PrologueBwdPlan plan_prologue_backward(int64_t T_, int H, int nk, int dtype) {
 
 template <typename T>
 int launch_prologue_backward(const float* dlogits, const void* x, const void* gate_w, const float* mean_rstd, int training,
-                             int64_t T_, int H, int nk, int dtype, void* dx, void* dgate_w, const void* addend0, const void* addend1,
-                             void* workspace, hipStream_t s, bool operands_ready) {
+                             int64_t T_, int H, int nk, int dtype, void* dx, void* dgate_w, const TokenGradients& more, void* workspace,
+                             hipStream_t s, bool operands_ready) {
     constexpr int V = Elem<T>::kVec;
     const PrologueBwdPlan p = plan_prologue_backward(T_, H, nk, dtype);
-    const ProloguePlan rows = plan_prologue(T_, H, nk);
+    const BlockStatsPlan rows = plan_block_stats(T_);
     char* ws = (char*)workspace;
     T *d16 = (T*)(ws + p.off_d16), *q = (T*)(ws + p.off_q), *dq = (T*)(ws + p.off_dq);
-    float *partial = (float*)(ws + p.off_partial), *sums = (float*)(ws + p.off_sums);
+    float* partial = (float*)(ws + p.off_partial);
     const int N = 2 * nk;
     const int widest = H > p.n_pad ? H : p.n_pad;
     void* part = ws + p.off_part;
@@ -782,17 +846,17 @@ int launch_prologue_backward(const float* dlogits, const void* x, const void* ga
     products[1].B0 = gate_w, products[1].C = dq;
     if (int rc = gemm_backward(products, 2, dtype, part, p.part_bytes, s)) return rc;
     if (training) {
-        const int strips = (H + kWave * V - 1) / (kWave * V);
+        const int strips = (H + 8 * V - 1) / (8 * V);
         hipLaunchKernelGGL((bn_bwd_partial_kernel<T>), dim3((unsigned)rows.row_blocks, (unsigned)strips), dim3(kStatsThreads), 0, s,
                            (const T*)x, (const T*)dq, mean_rstd, T_, H, rows.rows_per_block, partial);
         FMOE_CHECK_LAUNCH("fmoe_router_prologue_backward(column sums)");
-        hipLaunchKernelGGL(bn_bwd_finalize_kernel, dim3((unsigned)((2 * H + 31) / 32)), dim3(256), 0, s, (const float*)partial,
-                           rows.row_blocks, H, 1.0f / (float)T_, sums);
-        FMOE_CHECK_LAUNCH("fmoe_router_prologue_backward(finalize)");
     }
-    const int apply_blocks = (H / V + 255) / 256;
-    hipLaunchKernelGGL((bn_bwd_apply_kernel<T>), dim3((unsigned)(T_ * apply_blocks)), dim3(256), 0, s, (const T*)x,
-                       (const T*)dq, mean_rstd, (const float*)sums, (const T*)addend0, (const T*)addend1, (T*)dx, H, apply_blocks, training);
+    // about two workgroups to a compute unit, rows in fours
+    const int64_t strips = (H + kWave * V - 1) / (kWave * V), wanted = 2 * chip_info().cus / strips + 1;
+    const int apply_rows = (int)((T_ + wanted * 4 - 1) / (wanted * 4) * 4);
+    hipLaunchKernelGGL((bn_bwd_apply_kernel<T>), dim3((unsigned)((T_ + apply_rows - 1) / apply_rows), (unsigned)strips), dim3(256), 0, s, (const T*)x,
+                       (const T*)dq, mean_rstd, training ? (const float*)partial : nullptr, rows.row_blocks, 1.0f / (float)T_, (const T*)more.addend0,
+                       (const T*)more.addend1, more.planes, more.slices, (T*)dx, T_, H, apply_rows);
     FMOE_CHECK_LAUNCH("fmoe_router_prologue_backward(apply)");
     return FMOE_OK;
 }
@@ -1018,7 +1082,7 @@ extern "C" int fmoe_router_prologue_backward(const float* dlogits_fp32, const vo
                                              void* dgate_w, void* workspace, size_t workspace_bytes, void* stream) {
     fmoe::clear_error();
     return fmoe::router_prologue_backward_impl(dlogits_fp32, x, gate_w, mean_rstd, training, num_tokens, hidden, num_keys, dtype, dx,
-                                               dgate_w, nullptr, nullptr, workspace, workspace_bytes, (hipStream_t)stream);
+                                               dgate_w, {}, workspace, workspace_bytes, (hipStream_t)stream);
 }
 
 fmoe::PrologueOperands fmoe::prologue_operands(const void* x, const float* mean_rstd, int64_t num_tokens, int hidden, int num_keys, int dtype,
@@ -1029,8 +1093,8 @@ fmoe::PrologueOperands fmoe::prologue_operands(const void* x, const float* mean_
 
 int fmoe::router_prologue_backward_impl(const float* dlogits_fp32, const void* x, const void* gate_w, const float* mean_rstd,
                                         int training, int64_t num_tokens, int hidden, int num_keys, int dtype, void* dx,
-                                        void* dgate_w, const void* addend0, const void* addend1, void* workspace,
-                                        size_t workspace_bytes, hipStream_t s, bool operands_ready) {
+                                        void* dgate_w, const TokenGradients& more, void* workspace, size_t workspace_bytes,
+                                        hipStream_t s, bool operands_ready) {
     using namespace fmoe;
     FMOE_REQUIRE(dtype_ok(dtype), FMOE_ERR_BAD_DTYPE, "fmoe_router_prologue_backward: unknown dtype %d", dtype);
     FMOE_REQUIRE(num_tokens > 0 && hidden > 0 && num_keys > 0 && num_tokens < (1ll << 24), FMOE_ERR_BAD_SHAPE,
@@ -1046,8 +1110,8 @@ int fmoe::router_prologue_backward_impl(const float* dlogits_fp32, const void* x
     FMOE_REQUIRE(workspace && workspace_bytes >= need && aligned16(workspace), FMOE_ERR_WORKSPACE,
                  "fmoe_router_prologue_backward: workspace of %zu bytes needed, %zu given", need, workspace_bytes);
     switch (dtype) {
-        case FMOE_F32: return launch_prologue_backward<float>(dlogits_fp32, x, gate_w, mean_rstd, training, num_tokens, hidden, num_keys, dtype, dx, dgate_w, addend0, addend1, workspace, s, operands_ready);
-        case FMOE_BF16: return launch_prologue_backward<bf16_t>(dlogits_fp32, x, gate_w, mean_rstd, training, num_tokens, hidden, num_keys, dtype, dx, dgate_w, addend0, addend1, workspace, s, operands_ready);
-        default: return launch_prologue_backward<f16_t>(dlogits_fp32, x, gate_w, mean_rstd, training, num_tokens, hidden, num_keys, dtype, dx, dgate_w, addend0, addend1, workspace, s, operands_ready);
+        case FMOE_F32: return launch_prologue_backward<float>(dlogits_fp32, x, gate_w, mean_rstd, training, num_tokens, hidden, num_keys, dtype, dx, dgate_w, more, workspace, s, operands_ready);
+        case FMOE_BF16: return launch_prologue_backward<bf16_t>(dlogits_fp32, x, gate_w, mean_rstd, training, num_tokens, hidden, num_keys, dtype, dx, dgate_w, more, workspace, s, operands_ready);
+        default: return launch_prologue_backward<f16_t>(dlogits_fp32, x, gate_w, mean_rstd, training, num_tokens, hidden, num_keys, dtype, dx, dgate_w, more, workspace, s, operands_ready);
     }
 }

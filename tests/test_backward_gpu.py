@@ -575,6 +575,40 @@ def test_block_backward_operands_from_the_routing_gradient(dtype, H, nk, K):
         assert torch.isfinite(a).all() and rel_fro(a, b) < {torch.float32: 1e-4, torch.bfloat16: 3e-2, torch.float16: 6e-3}[dtype]
 
 
+@pytest.mark.parametrize("dtype,T,H,I", [
+    (torch.bfloat16, 615, 776, 2072), (torch.float32, 383, 516, 1544),     # dx of the MLP in slices of k: added with the other gradients
+    (torch.float16, 2050, 72, 136), (torch.bfloat16, 4101, 520, 264),      # more than one row to a wave, rows beyond the last block
+    (torch.float32, 3, 4, 8),
+])
+def test_block_backward_adds_the_token_gradients(dtype, T, H, I):
+    """dx of the block is the sum of the MLP's, the experts' and the router's, formed where the last of them is."""
+    from flash_moe.modules.flash_moe import FlashMoE, FlashMoEConfig
+    from flash_moe.ops.hip.flash_expert import expert_backward
+    from flash_moe.ops.hip.flash_mlp import mlp_backward
+    from flash_moe.ops.hip.flash_router import route_backward, router_prologue_backward
+
+    m = FlashMoE(FlashMoEConfig(H, I, "silu", 100, 5, False)).to(device="cuda", dtype=dtype)
+    with torch.no_grad():
+        for p in m.parameters():
+            p.copy_((torch.randn(p.shape, generator=gen(p.numel())) * p.shape[-1] ** -0.5).to(dtype))
+    x, dy = (torch.randn(1, T, H, generator=gen(k)).to(dtype).cuda() for k in (1, 2))
+    xg = x.clone().requires_grad_(True)
+    y, logits = m(xg)
+    y.backward(dy)
+    w = [getattr(m, n).weight for n in ("gate_proj", "up_proj", "down_proj", "router_gate", "down_embed", "up_embed")]
+    with torch.no_grad():
+        m.router_norm.reset_running_stats()
+        _, _, indices, gates, logits32 = m.route(x[0], return_logits32=True)
+        x64 = x[0].double()
+        stats = torch.stack((x64.mean(0), (x64.var(0, unbiased=False) + m.router_norm.eps).rsqrt())).float()
+        mlp = mlp_backward(dy[0], x[0], *w[:3])
+        experts = expert_backward(dy[0], x[0], w[4], w[5], indices, gates)
+        router = router_prologue_backward(route_backward(experts[3], indices, logits32, 10, False), x[0], w[3], stats, True)
+    expect = mlp[0].double() + experts[0].double() + router[0].double()
+    # every term may be rounded to the type before the sum here, only the sum there
+    assert rel_fro(xg.grad[0], expect) < {torch.float32: 1e-5, torch.bfloat16: 8e-3, torch.float16: 1e-3}[dtype]
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_mlp_backward_with_saved_products_equals_recomputation(dtype):
     from flash_moe.ops.hip.flash_mlp import mlp_backward, mlp_forward, mlp_forward_saving
