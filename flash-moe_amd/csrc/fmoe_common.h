@@ -222,6 +222,11 @@ int gemm_backward(const BackwardProduct* products, int count, int dtype, void* w
                   KeptPlanes* keep = nullptr);
 size_t gemm_backward_workspace_bytes(const BackwardProduct* products, int count, int dtype);
 
+// da and db (rows ld values apart) and h, all [M,N], of dh = dy Wd, the K-column rows of dy and the forward's products a and b, without dh:
+// true if these extents and types have one launch for it and it has been made.
+bool swiglu_gradient_together(const void* dy, const void* wd, const void* a, const void* b, void* da, void* db, void* h, int M, int N, int K, int ld,
+                              int dtype, hipStream_t stream);
+
 // fmoe_mlp_backward with the products kept, whose scratch for slices of k lies apart from its workspace; dx may stay there as planes.
 struct MlpBackwardBytes { size_t workspace, planes; };
 MlpBackwardBytes mlp_backward_bytes(int64_t num_tokens, int hidden, int intermediate, int dtype);

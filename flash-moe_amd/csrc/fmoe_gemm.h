@@ -5,11 +5,19 @@
 
 #include "fmoe_common.h"
 #include "fmoe_mfma.h"
+#include "fmoe_vec.h"
 
 namespace fmoe {
 namespace {
 
-enum Epilogue { kEpiSwiGLU = 0, kEpiPlain = 1, kEpiDual = 2, kEpiPart = 3 };   // Dual: the product in T and, through R, in fp32
+enum Epilogue { kEpiSwiGLU = 0, kEpiPlain = 1, kEpiDual = 2, kEpiPart = 3, kEpiGradient = 4 };   // Dual: the product in T and, through R, in fp32
+// kEpiGradient: the product is dh = dy Wd and is not stored; with the forward's products a = x Wg^T and b = x Wu^T it becomes the
+// gradients da and db (rows ld apart) and h = silu(a) * b, all [M,N].
+template <typename T> struct GradientPlanes {
+    const T *a, *b;
+    T *da, *db, *h;
+    int ld;
+};
 template <bool B> struct Flag { static constexpr bool value = B; };
 constexpr uint32_t kOutOfRange = 0x80000000u;    // beyond every buffer descriptor here: loads give zeros, stores are dropped
 
@@ -21,6 +29,13 @@ template <typename T, int N> struct DmaLds {
         return stages;
     }
 };
+// The hardware reciprocal (1 ulp) instead of a division: the results are rounded to 16 bits.
+__device__ __forceinline__ void swiglu_gradient(float dc, float a, float b, float& da, float& db, float& h) {
+    const float sig = __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(a * -1.44269504088896340736f)), silu = a * sig;
+    db = dc * silu;
+    da = dc * (silu * (1.0f - sig) + sig) * b;
+    h = silu * b;
+}
 // Position of item t of n in the order the XCDs walk: XCD x (workgroup id mod xcds) takes a contiguous run, so that what its items share
 // passes into its L2 once.  A permutation of [0, n) for every n.
 __host__ __device__ __forceinline__ int xcd_run(int t, int n, int xcds) {
@@ -48,7 +63,7 @@ template <typename T, int BM, int BN, int WAVES_M, int WAVES_N, int BKT, int NST
 __device__ __forceinline__ void gemm_dma_tiles(
     const T* __restrict__ A, const T* __restrict__ B0, const T* __restrict__ B1, T* __restrict__ C,
     const T* __restrict__ R, int M, int N, int K, int tiles_m, int tiles_n, int xcds, int block, int blocks, int slice = 0, int slices = 1,
-    int lda = 0, int ldb = 0, int segments = 1) {
+    int lda = 0, int ldb = 0, int segments = 1, const GradientPlanes<T>& grad = {}) {
     using Shape = MfmaShape<T, FR>;
     using Frag = typename Shape::Frag;
     using Acc = typename Shape::Acc;
@@ -330,7 +345,11 @@ __device__ __forceinline__ void gemm_dma_tiles(
 #pragma unroll
                 for (int i = 0; i < MF; ++i)
 #pragma unroll
-                    for (int j = 0; j < NF; ++j) acc[i][j] = Shape::run(fa[q % RING][i], fb[q % RING][j], acc[i][j]);
+                    for (int j = 0; j < NF; ++j) {
+                        // exchanged, a lane receives four successive columns of C instead of four rows
+                        if constexpr (EPI == kEpiGradient) acc[i][j] = Shape::run(fb[q % RING][j], fa[q % RING][i], acc[i][j]);
+                        else acc[i][j] = Shape::run(fa[q % RING][i], fb[q % RING][j], acc[i][j]);
+                    }
                 // issue order: the LDS reads spread evenly behind the MFMAs
                 constexpr int kPer = (n_reads + kMfmas - 1) / kMfmas;
 #pragma unroll
@@ -355,6 +374,68 @@ __device__ __forceinline__ void gemm_dma_tiles(
                 if (s < k_tiles) issue(s, Lds::at() + s * STAGE);
         }
 
+        if constexpr (EPI == kEpiGradient) {
+            // Lane l has row l % 16 and columns 4 (l / 16) .. + 3 of every fragment; rows of 16 lanes swap words between two fragments so
+            // that loads and stores are of 16 bytes (a lane's eight successive columns of one of them), the arithmetic in the lanes'
+            // own layout.  Offsets in the vector register alone: see fmoe_gemm256.h.
+            static_assert(sizeof(T) == 2 && FR == 16 && TB && !TA && NF % 2 == 0, "gradient epilogue");
+            const int row0 = out_m0 + wm * WM, col0 = out_n0 + wn * WN + (fhalf & 1) * 16 + (fhalf >> 1) * 8;
+            const int rows = M - row0;
+            auto plane = [&](const T* base, int ld) {
+                const int64_t span = rows > 0 ? ((int64_t)(rows - 1) * ld + N) * 2 : 0;
+                return __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(base + (int64_t)row0 * ld), 0, (int)(span < 0x7FFFFFFFll ? span : 0x7FFFFFFFll), 0x00020000);
+            };
+            const auto a_plane = plane(grad.a, N), b_plane = plane(grad.b, N), h_plane = plane(grad.h, N);
+            const auto da_plane = plane(grad.da, grad.ld), db_plane = plane(grad.db, grad.ld);
+            auto swap_rows = [](u32x4_t& w) {
+#pragma unroll
+                for (int e = 0; e < 2; ++e) {
+                    const auto swapped = __builtin_amdgcn_permlane16_swap(w[e], w[2 + e], false, false);
+                    w[e] = swapped[0];
+                    w[2 + e] = swapped[1];
+                }
+            };
+            auto at = [&](int i, int j, int ld) {
+                const int col = col0 + j * FR;
+                return col < N ? ((i * FR + frow) * ld + col) * 2 : (int)kOutOfRange;
+            };
+            u32x4_t ra[MF][NF / 2], rb[MF][NF / 2];
+            auto load = [&](int i) {
+#pragma unroll
+                for (int p = 0; p < NF / 2; ++p) {
+                    ra[i][p] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(a_plane, at(i, 2 * p, N), 0, 0));
+                    rb[i][p] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(b_plane, at(i, 2 * p, N), 0, 0));
+                }
+            };
+#pragma unroll
+            for (int i = 0; i < MF; ++i) load(i);            // all of a and b at once: one memory round trip
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int i = 0; i < MF; ++i) {
+#pragma unroll
+                for (int p = 0; p < NF / 2; ++p) {
+                    float av[8], bv[8], dav[8], dbv[8], hv[8];
+                    swap_rows(ra[i][p]);
+                    swap_rows(rb[i][p]);
+                    unpack16<T>(ra[i][p], av);
+                    unpack16<T>(rb[i][p], bv);
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) {
+                        const float dc = acc[i][2 * p + e / 4][e % 4];
+                        swiglu_gradient(dc, av[e], bv[e], dav[e], dbv[e], hv[e]);
+                    }
+                    u32x4_t out[3] = {pack16<T>(dav), pack16<T>(dbv), pack16<T>(hv)};
+#pragma unroll
+                    for (int k = 0; k < 3; ++k) swap_rows(out[k]);
+                    __builtin_amdgcn_raw_buffer_store_b128(out[0], da_plane, at(i, 2 * p, grad.ld), 0, 0);
+                    __builtin_amdgcn_raw_buffer_store_b128(out[1], db_plane, at(i, 2 * p, grad.ld), 0, 0);
+                    __builtin_amdgcn_raw_buffer_store_b128(out[2], h_plane, at(i, 2 * p, N), 0, 0);
+                }
+            }
+            if (next >= num_tiles) break;
+            tile = next;
+            continue;
+        }
         // D fragment layout (both shapes): lane l, register v holds
         //   row = 8*(v/4) + 4*(l/FR) + (v%4)   (A / M index),   col = l%FR   (B / N index)
         // Buffer addressing: a wave-uniform descriptor of the rows from the wave's first one on, a scalar byte offset

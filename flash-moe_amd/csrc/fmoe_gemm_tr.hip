@@ -54,6 +54,17 @@ __global__ __launch_bounds__(kWideThreads, 2) void gemm_wide_turned_kernel(
         SLICED ? block / tiles : 0, slices, lda, ldb, segments);
 }
 
+// dh = dy Wd and the SwiGLU gradient of it (kEpiGradient): dh makes no way through memory, and is not rounded on it.  us, two launches and
+// one (bf16): 615 tokens, 776 -> 2072 14.6 and 11.5; 4096 tokens, 1024 -> 4096 63 and 54; 300 tokens, 512 -> 1360 9.0 and 6.1; 8000 tokens, 320
+// -> 848 27 and 17.  da, db and h against 64 bits: 1.66e-3 of them, 2.34e-3 with dh rounded.  Bound by the planes, read and written at
+// 6 TB/s, on few columns, by what the L2s deliver to 128 x 128 tiles on many.
+template <typename T, int BM, int BN>
+__global__ __launch_bounds__(256, 2) void gemm_gradient_kernel(const T* __restrict__ dy, const T* __restrict__ wd, const GradientPlanes<T> grad, int M, int N, int K,
+                                                               int tiles_m, int tiles_n, int xcds) {
+    gemm_dma_tiles<T, BM, BN, 2, 2, kStageK<T>, 2, kEpiGradient, kSmallAhead<T>, kFragRows<T>, true, false, false, true>(
+        dy, wd, nullptr, nullptr, nullptr, M, N, K, tiles_m, tiles_n, xcds, (int)blockIdx.x, (int)gridDim.x, 0, 1, K, N, 1, grad);
+}
+
 // Several products in one launch: the workgroups of member i are first .. first + tiles * slices - 1 (first a multiple of the XCDs; ids
 // past the last are spare), one tile or slice of k each, which the dispatcher hands to compute units as they fall free, longest first.
 // us, dWd, dx, dWg and dWu one after the other and together, bf16: 4096 tokens, 1024 -> 4096 190 -> 152; 615 tokens, 776 -> 2072 35.5 ->
@@ -140,7 +151,7 @@ template <typename T> void launch_sums(Sums& g, int members, hipStream_t stream)
 // These prices against 186 products timed in every shape and number of slices (bf16): 2.3 % over the best on average, 3.6 with the
 // 256 x 256 tiles at the rate of the forward's and their stores at 8.5; us: dh of 1819 tokens, 1792 -> 4776 52 -> 39, of 4681, 1136 -> 4544
 // 74 -> 58, dWd of 19470 tokens, 1704 -> 640 90 -> 60, dx of 1819 tokens, 4776 -> 1792 90 -> 75; the worst, 1536 x 3072 of 2760, 36 -> 45.
-template <typename T> SlicePlan plan_turned(int M, int N, int K, int segments) {
+template <typename T> SlicePlan plan_turned(int M, int N, int K, int segments, double* price = nullptr) {
     const int cus = chip_info().cus, k_tiles = (K + kStageK<T> - 1) / kStageK<T> * segments;
     SlicePlan best = {kTile64, 1};
     double best_time = 0.0;
@@ -160,6 +171,7 @@ template <typename T> SlicePlan plan_turned(int M, int N, int K, int segments) {
             }
         }
     }
+    if (price != nullptr) *price = best_time;
     return best;
 }
 
@@ -250,6 +262,37 @@ inline double time_of_items(const int64_t* n, const double* t, int kinds, int sl
             end = done > end ? done : end;
         }
     return end;
+}
+
+// Tile shape of dh = dy Wd with its SwiGLU gradient in one launch, or -1: two launches.  Prices (us): k-tiles at the rate of a full
+// compute unit or of one tile alone, an epilogue's five values of 2 bytes at what a unit gets of 6.6 TB/s; two launches: the product at
+// its own price and six planes at 6.3 TB/s.  Over 83 products timed all ways (16 to 8192 tokens, 256 to 4096 columns) the choice is 1 % behind
+// the best on average; two launches take 20 % more.  Planes beyond 100 MB come from memory, no longer from the cache in front of it, and an
+// epilogue waits for them where a launch that does nothing else streams them (4096 tokens, 1024 -> 4096 67 us in two, 72 to 74 in one,
+// also on 256 x 256 tiles; 59 with the planes at hand).
+int plan_gradient(int M, int N, int K) {
+    const int cus = chip_info().cus, k_tiles = (K + 63) / 64;
+    if ((double)M * N > 1.0e7) return -1;
+    double best_time = 0.0;
+    plan_turned<bf16_t>(M, N, K, 1, &best_time);
+    const double planes = 12.0e-6 * (double)M * N / 6.3 + 2.0;
+    best_time += (planes > 3.8 ? planes : 3.8) + 0.9;
+    int best = -1;
+    for (int shape : {kTile128, kTile64}) {
+        const bool large = shape == kTile128;
+        const int rows = kTileRows[shape], cols = kTileCols[shape], per = large ? 2 : 4;
+        const int64_t n = (int64_t)((M + rows - 1) / rows) * ((N + cols - 1) / cols);
+        const double share = 6550.0 / (n < cus ? n : cus), rate = large && share > 26.0 ? 26.0 : share;     // GB/s of a compute unit
+        const double stores = 10.0e-3 * rows * cols / rate, item = k_tiles * (large ? 0.59 : 0.19) + stores;
+        const double rounds = (double)((n + per * cus - 1) / (per * cus)) * item * per, blend = large ? 0.32 : 0.4;
+        const double alone = k_tiles * (large ? 0.68 : 0.44) + 0.66 * stores, full = n > cus ? blend * rounds + (1.0 - blend) * (double)n * item / cus : 0.0;
+        const double time = (full > alone ? full : alone) + 2.2;
+        if (time < best_time) {
+            best_time = time;
+            best = shape;
+        }
+    }
+    return best;
 }
 
 // Price (us) of a group on tiles of a shape: half (0.4 to 1) of what its items take on slots that hold two workgroups of 128 x 128 (four of
@@ -393,6 +436,32 @@ void launch_group(const BackwardProduct* p, int count, const GroupPlan& plan, vo
 size_t gemm_backward_workspace_bytes(int M, int N, int K, int segments, int dtype) {
     const int slices = (dtype == FMOE_F32 ? plan_turned<float>(M, N, K, segments) : plan_turned<bf16_t>(M, N, K, segments)).slices;
     return slices > 1 ? (size_t)slices * M * N * sizeof(float) : 0;
+}
+
+template <typename T>
+void launch_gradient(const void* dy, const void* wd, const GradientPlanes<T>& grad, int M, int N, int K, int shape, hipStream_t stream) {
+    const int rows = kTileRows[shape], cols = kTileCols[shape], tm = (M + rows - 1) / rows, tn = (N + cols - 1) / cols;
+    const int64_t n = (int64_t)tm * tn, resident = (int64_t)chip_info().cus * (shape == kTile128 ? 2 : 4);
+    const dim3 grid((unsigned)(n < resident ? n : resident));
+#define FMOE_GO(TILE) \
+    hipLaunchKernelGGL((gemm_gradient_kernel<T, TILE, TILE>), grid, dim3(256), 0, stream, (const T*)dy, (const T*)wd, grad, M, N, K, tm, tn, chip_info().xcds)
+    if (shape == kTile64) FMOE_GO(64);
+    else FMOE_GO(128);
+#undef FMOE_GO
+}
+
+bool swiglu_gradient_together(const void* dy, const void* wd, const void* a, const void* b, void* da, void* db, void* h, int M, int N, int K, int ld,
+                              int dtype, hipStream_t stream) {
+    if (dtype == FMOE_F32 || ld > 1 << 21 || !addressable({kBlasNN, M, N, K, 1, dy, K, wd, nullptr, N, h}, dtype) || !aligned16(a) || !aligned16(b) ||
+        !aligned16(da) || !aligned16(db) || ld % 8 != 0)
+        return false;
+    const int shape = plan_gradient(M, N, K);
+    if (shape < 0) return false;
+    if (dtype == FMOE_BF16)
+        launch_gradient<bf16_t>(dy, wd, {(const bf16_t*)a, (const bf16_t*)b, (bf16_t*)da, (bf16_t*)db, (bf16_t*)h, ld}, M, N, K, shape, stream);
+    else
+        launch_gradient<f16_t>(dy, wd, {(const f16_t*)a, (const f16_t*)b, (f16_t*)da, (f16_t*)db, (f16_t*)h, ld}, M, N, K, shape, stream);
+    return true;
 }
 
 int gemm_backward(const BackwardProduct& q, int dtype, void* workspace, size_t workspace_bytes, hipStream_t stream) {

@@ -188,13 +188,17 @@ int fmoe::mlp_backward_impl(const void* dy, const void* x, const void* gate_w, c
         if (rc) return rc;
     }
 
-    rc = gemm_backward({kNN, T_, I, H, 1, dy, H, down_w, nullptr, I, dh}, dtype, part, p.part_bytes, s);                    // dh = dy Wd
-    if (rc) return rc;
     // da and db side by side: one [T, 2I] matrix [da | db], so that products over both are single calls
     char* db = dab + (size_t)I * elt;
     const int I2 = 2 * I;
-    rc = launch_swiglu_backward(dh, a, b, dab, db, h, num_tokens, I, I2, I2, dtype, s);
-    if (rc) return rc;
+    if (swiglu_gradient_together(dy, down_w, a, b, dab, db, h, T_, I, H, I2, dtype, s)) {
+        FMOE_CHECK_LAUNCH("fmoe_mlp_backward(SwiGLU gradient)");
+    } else {
+        rc = gemm_backward({kNN, T_, I, H, 1, dy, H, down_w, nullptr, I, dh}, dtype, part, p.part_bytes, s);                // dh = dy Wd
+        if (rc) return rc;
+        rc = launch_swiglu_backward(dh, a, b, dab, db, h, num_tokens, I, I2, I2, dtype, s);
+        if (rc) return rc;
+    }
     const size_t w_bytes = (size_t)I * H * elt;
     BackwardProduct q[4];
     const int count = mlp_gradients(T_, H, I, (char*)dup_w == (char*)dgate_w + w_bytes, q);

@@ -817,6 +817,31 @@ def test_mlp_backward_on_the_large_tiles_of_the_turned_products(dtype, T, H, I):
     test_mlp_backward_remainders_of_the_transposing_products(dtype, T, H, I)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("T,H,I", [
+    (1, 8, 8), (63, 72, 64), (65, 136, 72), (127, 8, 1032), (1025, 1032, 2056),      # 64 x 64 tiles and their edges, one and many rounds
+    (2049, 72, 1032), (4097, 264, 520),                                              # 128 x 128
+    (129, 3080, 4104),                                                               # two launches
+])
+def test_mlp_backward_swiglu_gradient_in_the_product(dtype, T, H, I):
+    """dh = dy Wd becomes da, db and h where it is formed: the gradients that hang on them, dx on da and db, dWd on h."""
+    from flash_moe.ops.hip.flash_mlp import mlp_backward, mlp_forward_saving
+
+    g = gen(T + H)
+    x, dy = (torch.randn(T, H, generator=g).to(dtype).cuda() for _ in range(2))
+    ws = [(torch.randn(s, generator=g) * s[-1] ** -0.5).to(dtype).cuda() for s in ((I, H), (I, H), (H, I))]
+    saved = mlp_forward_saving(x, *ws)[1]
+    a, b = saved.double()
+    dh, sig = dy.double() @ ws[2].double(), torch.sigmoid(a)
+    h, db = a * sig * b, dh * a * sig
+    da = dh * b * sig * (1 + a * (1 - sig))
+    for kept in (saved, None):                         # the products of the forward, or recomputed
+        dx, dwg, dwu, dwd = mlp_backward(dy, x, *ws, kept)
+        for name, got, ref in (("dwd", dwd, dy.double().t() @ h), ("dx", dx, da @ ws[0].double() + db @ ws[1].double()),
+                               ("dwg", dwg, da.t() @ x.double()), ("dwu", dwu, db.t() @ x.double())):
+            assert rel_fro(got, ref) < GRAD_FRO[dtype], (name, rel_fro(got, ref))
+
+
 @pytest.mark.parametrize("dtype,T,H,I", [
     (torch.bfloat16, 513, 264, 520), (torch.float16, 2600, 264, 264),        # one launch on 64 x 64 tiles: whole; weight gradients in slices
     (torch.float16, 1000, 1800, 4104), (torch.bfloat16, 5200, 776, 264),     # on 128 x 128: dx in slices; weight gradients in slices
