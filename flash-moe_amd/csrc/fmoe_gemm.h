@@ -669,6 +669,10 @@ template <typename T> constexpr int kStageK = 128 / (int)sizeof(T);
 // 32x32x2.
 template <typename T> constexpr int kFragRows = sizeof(T) == 2 ? 16 : 32;
 template <typename T> constexpr int kSmallAhead = sizeof(T) == 2 ? 1 : 3;
+// Gate/up tiles of 64 x 64 hold 32 columns of either, a wave 16 of them: fragments of 16 rows in fp32 too.
+template <typename T, int BN, int EPI> constexpr bool kNarrowPair = sizeof(T) == 4 && BN == 64 && EPI == kEpiSwiGLU;
+template <typename T, int BN, int EPI> constexpr int kTileFrag = kNarrowPair<T, BN, EPI> ? 16 : kFragRows<T>;
+template <typename T, int BN, int EPI> constexpr int kTileAhead = kNarrowPair<T, BN, EPI> ? 1 : kSmallAhead<T>;
 
 // Tile choice.  A workgroup's time per k-tile is the larger of what its CU receives from the L2 ((BM + BN) rows of 128 bytes, at 40
 // to 70 GB/s per CU) and what its matrix pipes take (BM * BN), in units of one received row BM * BN / 95: with every CU busy a
@@ -678,7 +682,9 @@ template <typename T> constexpr int kSmallAhead = sizeof(T) == 2 ? 1 : 3;
 // of 2904 -> 7744 seven rounds of 128 x 128, 227 us; two of 256 x 256 take 157.)
 // Its two groups of waves keep the pipes busier: BM * BN / 108 for the plain products (us: 22464 tokens, 3232 -> 808 147 -> 128; 15029
 // tokens, 3408 -> 1280 166 -> 147); gate/up products, of which half are short in k, gain and lose about alike and stay at / 95.
-// fp32 rows of 128 bytes hold half as many values for matrix pipes an eighth as fast: BM * BN / 15.  The k-splitting kernel
+// fp32 rows of 128 bytes hold half as many values for matrix pipes an eighth as fast: BM * BN / 15, gate/up pairs of 32 columns / 13 (the
+// block, us, on the best of the other tiles and on these: 400 tokens, 512 -> 1024 43.1 -> 35.9; 300, 256 -> 1024 28.1 -> 24.5; 512, 256 -> 1024
+// 33.1 -> 31.6; at / 15 1900 tokens, 640 -> 1704 would take them too, 159 -> 163).  The k-splitting kernel
 // costs more per received row, and more so the more CUs receive at once (measured from 64 to 224 workgroups), but its tiles are
 // small enough for a few rows of A.
 enum TileShape { kTile256, kTile128, kTile64x128, kTile64, kSplit32, kSplit16x32, kSplit16 };
@@ -693,7 +699,7 @@ template <typename T, int EPI> double tile_cost(int i, int M, int N, int64_t& n)
     n = (int64_t)((M + kTileRows[i] - 1) / kTileRows[i]) * ((N + out_cols - 1) / out_cols);
     const double occupied = n < cus ? (double)n / cus : 1.0;
     const double received = (kTileRows[i] + cols) * (split_k ? 1.45 * (1.0 + occupied) : 1.0);
-    const double rate = sizeof(T) == 4 ? 15.0 : (i == kTile256 && EPI == kEpiPlain ? 108.0 : 95.0);
+    const double rate = sizeof(T) == 4 ? (i == kTile64 && EPI == kEpiSwiGLU ? 13.0 : 15.0) : (i == kTile256 && EPI == kEpiPlain ? 108.0 : 95.0);
     const double multiplied = kTileRows[i] * (double)cols / rate;
     return received > multiplied ? received : multiplied;
 }
@@ -702,7 +708,6 @@ template <typename T, int EPI> TileShape choose_tile(int M, int N, int& tiles, d
     TileShape best = kTile128;
     double best_cost = 0.0;
     for (int i = 0; i < 7; ++i) {
-        if (i == kTile64 && EPI == kEpiSwiGLU && sizeof(T) == 4) continue;      // a 32-column wave tile is one fp32 fragment: no gate/up pair
         int64_t n = 0;
         const double round = tile_cost<T, EPI>(i, M, N, n), cost = (double)((n + cus - 1) / cus) * round;
         if (i == 0 || cost < best_cost) {

@@ -33,7 +33,7 @@ template <> struct Mfma32<float> {
         return c;
     }
 };
-template <typename T> constexpr int kMfmaPerRun = sizeof(T) == 4 ? 4 : 1;   // matrix instructions per Mfma32<T>::run
+template <typename T> constexpr int kMfmaPerRun = sizeof(T) == 4 ? 4 : 1;   // matrix instructions per run of either shape
 
 // v_mfma_f32_16x16x32_{bf16,f16}: D[16x16] += A[16x32] * B[32x16].  Lane l supplies row l%16 of A (column l%16 of B) and 8
 // consecutive k values chosen by l/16; it receives D[4*(l/16) + v][l%16] in register v (four registers).  Under the power
@@ -48,19 +48,23 @@ template <> struct Mfma16<f16_t> {
     __device__ static f32x4_t run(Frag a, Frag b, f32x4_t c) { return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0); }
 };
 
+// fp32: v_mfma_f32_16x16x4_f32, the same D layout.  A fragment is one 16-byte LDS read: 4 consecutive k values, lanes of piece l/16 of a
+// 64-byte k-step, instruction q multiplying element q of the four pieces.
+template <> struct Mfma16<float> {
+    using Frag = f32x4_t;
+    __device__ static f32x4_t run(Frag a, Frag b, f32x4_t c) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[q], b[q], c, 0, 0, 0);
+        return c;
+    }
+};
+
 // One step of a 16 x 16 tile from 16-byte packets: lane l holds packet l/16 (of four) of row l%16 on either side, 32 k values for
 // the 16-bit types (one v_mfma_f32_16x16x32), 16 for fp32 (four v_mfma_f32_16x16x4_f32, instruction q multiplying element q of
 // the four packets).  D layout as Mfma16.
 template <typename T> __device__ inline f32x4_t mfma16_packet(u32x4_t a, u32x4_t b, f32x4_t c) {
-    if constexpr (sizeof(T) == 4) {
-        const f32x4_t av = __builtin_bit_cast(f32x4_t, a), bv = __builtin_bit_cast(f32x4_t, b);
-#pragma unroll
-        for (int q = 0; q < 4; ++q) c = __builtin_amdgcn_mfma_f32_16x16x4f32(av[q], bv[q], c, 0, 0, 0);
-        return c;
-    } else {
-        using Frag = typename Mfma16<T>::Frag;
-        return Mfma16<T>::run(__builtin_bit_cast(Frag, a), __builtin_bit_cast(Frag, b), c);
-    }
+    using Frag = typename Mfma16<T>::Frag;
+    return Mfma16<T>::run(__builtin_bit_cast(Frag, a), __builtin_bit_cast(Frag, b), c);
 }
 
 // What the tiled kernel needs to know about a fragment shape: FR = rows (and columns) of a fragment, kChunks = 16-byte
@@ -76,7 +80,7 @@ template <typename T> struct MfmaShape<T, 32> {
 template <typename T> struct MfmaShape<T, 16> {
     using Frag = typename Mfma16<T>::Frag;
     using Acc = f32x4_t;
-    static constexpr int kChunks = 4, kAccRegs = 4, kInstr = 1;
+    static constexpr int kChunks = 4, kAccRegs = 4, kInstr = kMfmaPerRun<T>;
     __device__ static Acc run(Frag a, Frag b, Acc c) { return Mfma16<T>::run(a, b, c); }
 };
 

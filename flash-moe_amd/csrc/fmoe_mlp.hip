@@ -207,9 +207,7 @@ void launch_tiles(const T* A, const T* B0, const T* B1, T* C, const T* R, int M,
         case kSplit16x32: launch_gemm_splitk<T, 1, 2, EPI>(A, B0, B1, C, R, M, N, K, stream); break;
         case kSplit16: launch_gemm_splitk<T, 1, 1, EPI>(A, B0, B1, C, R, M, N, K, stream); break;
         case kTile64x128: launch_gemm_dma<T, 64, 128, 2, 2, KT, 4, EPI, PF, FR, RAGGED>(A, B0, B1, C, R, M, N, K, stream); break;
-        default:
-            if constexpr (EPI != kEpiSwiGLU || sizeof(T) == 2)
-                launch_gemm_dma<T, 64, 64, 2, 2, KT, 4, EPI, PF, FR, RAGGED>(A, B0, B1, C, R, M, N, K, stream);
+        default: launch_gemm_dma<T, 64, 64, 2, 2, KT, 4, EPI, kTileAhead<T, 64, EPI>, kTileFrag<T, 64, EPI>, RAGGED>(A, B0, B1, C, R, M, N, K, stream);
     }
 }
 

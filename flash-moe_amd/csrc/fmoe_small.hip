@@ -56,7 +56,7 @@ __device__ __forceinline__ void product_tiles(const T* A, const T* B0, const T* 
         if constexpr (CUT == kCut256 && sizeof(T) == 2 && EPI == kEpiSwiGLU)
             gemm_wide_tiles<T, EPI, true>(A, B0, B1, C, R, M, N, K, p.tiles_m, p.tiles_n, xcds, block, p.blocks);
         else
-            gemm_dma_tiles<T, S::BM, S::BN, 2, S::kWavesN, kStageK<T>, S::kStages, EPI, kSmallAhead<T>, kFragRows<T>, true>(
+            gemm_dma_tiles<T, S::BM, S::BN, 2, S::kWavesN, kStageK<T>, S::kStages, EPI, kTileAhead<T, S::BN, EPI>, kTileFrag<T, S::BN, EPI>, true>(
                 A, B0, B1, C, R, M, N, K, p.tiles_m, p.tiles_n, xcds, block, p.blocks);
     } else {
         gemm_splitk_tile<T, S::MT, S::MT, EPI>(A, B0, B1, C, R, M, N, K, p.tiles_m, p.tiles_m * p.tiles_n, xcds, block % p.blocks, p.blocks,
@@ -130,9 +130,14 @@ template <typename T, int EPI> Product plan_product(int M, int N) {
 }
 
 // Few tokens: 16 x 16 tiles while they leave compute units free, else 32 x 32.  A compute unit receives about 60 GB/s, so a
-// workgroup that would read more than 256 KB leaves parts of k to others as long as there are compute units without a tile.
+// workgroup that would read more than 256 KB leaves parts of k to others as long as there are compute units without a tile; fp32, whose
+// matrix pipes take as long, from 128 KB on beyond 256 tokens (300 tokens, 1024 -> 256: the block 24.5 -> 21.1 us; 8 tokens, 4096 -> 1024
+// would take 33.3 -> 35.4).
 template <typename T> Product plan_down(int M, int H, int I) {
-    if (M > 256) return plan_product<T, kEpiPart>(M, H);
+    if (M > 256) {
+        const Product whole = plan_product<T, kEpiPart>(M, H);
+        if (sizeof(T) == 2 || whole.cut > kCutSplit32) return whole;
+    }
     const int cus = chip_info().cus;
     Product p;
     p.cut = ((M + 15) / 16) * ((H + 15) / 16) < cus ? kCutSplit16 : kCutSplit32;
@@ -140,7 +145,7 @@ template <typename T> Product plan_down(int M, int H, int I) {
     p.tiles_m = (M + b - 1) / b;
     p.tiles_n = (H + b - 1) / b;
     const int64_t tiles = (int64_t)p.tiles_m * p.tiles_n, bytes = 2 * b * (int64_t)I * (int64_t)sizeof(T);
-    const int64_t wanted = (bytes + (256 << 10) - 1) / (256 << 10), room = cus / tiles;
+    const int64_t most = M > 256 ? 128 << 10 : 256 << 10, wanted = (bytes + most - 1) / most, room = cus / tiles;
     p.slices = (int)(wanted < room ? wanted : room);
     if (p.slices > kSmallMaxSlices) p.slices = kSmallMaxSlices;
     if (p.slices < 1) p.slices = 1;
@@ -169,7 +174,7 @@ int gate_and_up(const void* x, const void* gate_w, const GateStats& st, float* l
     switch (up.cut) {
         case kCutSplit16: FMOE_GO(kCutSplit16); break;
         case kCutSplit32: FMOE_GO(kCutSplit32); break;
-        case kCut64: if constexpr (sizeof(T) == 2) FMOE_GO(kCut64); break;
+        case kCut64: FMOE_GO(kCut64); break;
         case kCut64x128: FMOE_GO(kCut64x128); break;
         case kCut128: FMOE_GO(kCut128); break;
         default: if constexpr (sizeof(T) == 2) FMOE_GO(kCut256); break;

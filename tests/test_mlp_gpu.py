@@ -150,6 +150,12 @@ def test_mlp_remainders_of_every_tile_shape(dtype, T, H, I):
         assert (buf[:8] == 7).all() and (buf[-8:] == 7).all()
 
 
+@pytest.mark.parametrize("T,H,I", [(512, 256, 1024), (385, 516, 1028), (301, 260, 996), (1500, 36, 1060), (400, 4, 992), (393, 100, 1004)])
+def test_mlp_fp32_on_gate_up_tiles_of_32_columns(T, H, I):
+    """64 x 64 tiles of 32 gate and 32 up columns: whole ones, remainders in rows, columns and k, one k-tile and a k tail of one packet."""
+    test_mlp_remainders_of_every_tile_shape(torch.float32, T, H, I)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
 @pytest.mark.parametrize("T,H,I", [(47, 1032, 8200), (129, 520, 4104), (203, 1032, 12296), (300, 2056, 8008), (129, 1001, 4004)])
 @pytest.mark.parametrize("with_residual", [False, True])
