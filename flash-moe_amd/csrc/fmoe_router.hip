@@ -163,13 +163,13 @@ __global__ __launch_bounds__(kRouterWaves* kWave) __attribute__((amdgpu_waves_pe
 // OCC: waves per SIMD the register allocation must leave room for.  With more than four tokens per SIMD eight resident
 // waves (at most 64 registers, a few of them spilled for the larger lists) finish sooner than seven, whose eighth token
 // per SIMD would wait for a second round; with at most four tokens per SIMD the unconstrained allocation is faster.
-template <typename T, typename TG, int RK, int RH, int RC, bool FROM_LOGITS, int OCC, bool SMALL, int TOK>
+template <typename T, typename TG, int RK, int RH, int RC, bool FROM_LOGITS, int OCC, bool SMALL, int TOK, bool REUSE>
 __global__ __launch_bounds__(kRouterWaves* kWave, OCC) void router_select_kernel(
     const T* __restrict__ lp, int64_t num_tokens, int nk, int top_k, int num_cand, T* __restrict__ scores,
     int64_t* __restrict__ indices, TG* __restrict__ gates, int norm_topk_prob, uint32_t* __restrict__ row_offsets,
     uint32_t row_bytes, const CandidateTable table) {
     __shared__ SelectLds<RK, RC, kRouterWaves, false, TOK> lds;
-    router_select_tokens<T, TG, RK, RH, RC, FROM_LOGITS, SMALL, kRouterWaves, false, TOK>(
+    router_select_tokens<T, TG, RK, RH, RC, FROM_LOGITS, SMALL, kRouterWaves, false, TOK, REUSE>(
         lp, num_tokens, nk, top_k, num_cand, scores, indices, gates, norm_topk_prob, row_offsets, row_bytes, table, lds, (int)blockIdx.x,
         (int)gridDim.x);
 }
@@ -470,24 +470,33 @@ int launch_router(const void* lp, int64_t T_, int nk, int K, void* scores, int64
     // lists that fit the registers of a wave take the threshold selection
     const bool crowded = T_ > (int64_t)chip_info().cus * 4 * kRouterWaves;      // more than four tokens per SIMD
     const bool in_pairs = T_ >= (int64_t)chip_info().cus * 16 * kRouterWaves;     // sixteen or more
-#define FMOE_LAUNCH_SELECT_OCC(RK_, RH_, RC_, OCC_, SMALL_, TOK_)                                                             \
-    hipLaunchKernelGGL((router_select_kernel<T, TG, RK_, RH_, RC_, FROM_LOGITS, OCC_, SMALL_, TOK_>), dim3((unsigned)blocks_of(TOK_)), \
-                       block, 0, stream, (const T*)lp, T_, nk, K, num_cand, (T*)scores, indices, (TG*)gates, norm, row_offsets, row_bytes, table)
+#define FMOE_LAUNCH_SELECT_OCC(RK_, RH_, RC_, OCC_, SMALL_, TOK_, REUSE_)                                                     \
+    hipLaunchKernelGGL((router_select_kernel<T, TG, RK_, RH_, RC_, FROM_LOGITS, OCC_, SMALL_, TOK_, REUSE_>),                 \
+                       dim3((unsigned)blocks_of(TOK_)), block, 0, stream, (const T*)lp, T_, nk, K, num_cand, (T*)scores, indices, (TG*)gates, norm, row_offsets, row_bytes, table)
 // Many tokens: one key per lane lets the kernel run in the registers of eight waves per SIMD at no or little spilling (K = 16, nk =
 // 128, 32768 tokens: 36 us against 40 at five waves when it was chosen); the instances of two keys per lane would spill 25 to 59
 // registers (nk = 512, K = 128: 165 us against 138 without the bound).  Few tokens are one latency chain, spills would lengthen it.
-// Two tokens to a wave save a third of the sorting once every wave has two (us, 128 keys, 16 experts: 32768 tokens 29.4 -> 28.0,
-// 16384 16.2 -> 15.6, but 12288 11.9 -> 12.9 and 8192 9.6 -> 10.5).
-#define FMOE_LAUNCH_SELECT(RK_, RH_, RC_)                                      \
-    do {                                                                       \
-        if (crowded && RK_ == 1) FMOE_LAUNCH_SELECT_OCC(1, RH_, RC_, 8, false, 1); \
-        else FMOE_LAUNCH_SELECT_OCC(RK_, RH_, RC_, 1, false, 1);               \
+// Two tokens to a wave save a third of the sorting once every wave has two (us, 128 keys, 16 experts, without REUSE: 32768 tokens 29.4
+// -> 28.0, 16384 16.2 -> 15.6, but 12288 11.9 -> 12.9 and 8192 9.6 -> 10.5).
+// Lists start from the score that served the wave's previous list (REUSE) where a wave has several and at least four slots beyond
+// K are left, eight of 64, so that it often serves again (us, 32768 tokens, without | with, 128 keys: K = 16 28.0 | 22.4, 24 27.5 |
+// 25.5, 28 29.7 | 28.8, 32 35.6 | 36.6, 40 39.1 | 36.7, 50 41.8 | 40.2, 58 44.2 | 44.4, 64 52.2 | 53.9; 512 keys: K = 16 44.1 | 35.1, 24
+// 50.4 | 44.7, 30 56.9 | 56.9, 40 59.7 | 51.0; 10000 tokens, K = 16: 10.5 | 9.75, 6000 8.0 | 7.9).  Two keys per lane gain 0 to 4 %
+// and are left as they are.
+#define FMOE_LAUNCH_SELECT(RK_, RH_, RC_)                                                          \
+    do {                                                                                           \
+        if (crowded && RK_ == 1 && K <= 56) FMOE_LAUNCH_SELECT_OCC(1, RH_, RC_, 8, false, 1, true); \
+        else if (crowded && RK_ == 1) FMOE_LAUNCH_SELECT_OCC(1, RH_, RC_, 8, false, 1, false);     \
+        else FMOE_LAUNCH_SELECT_OCC(RK_, RH_, RC_, 1, false, 1, false);                            \
     } while (0)
-#define FMOE_LAUNCH_SELECT_SMALL(RH_, RC_)                                     \
-    do {                                                                       \
-        if (in_pairs) FMOE_LAUNCH_SELECT_OCC(1, RH_, RC_, 8, true, 2);         \
-        else if (crowded) FMOE_LAUNCH_SELECT_OCC(1, RH_, RC_, 8, true, 1);     \
-        else FMOE_LAUNCH_SELECT_OCC(1, RH_, RC_, 1, true, 1);                  \
+#define FMOE_LAUNCH_SELECT_SMALL(RH_, RC_)                                                         \
+    do {                                                                                           \
+        constexpr bool all_reuse = RC_ == 1;              /* at most 19 experts */                 \
+        if (in_pairs && (all_reuse || K <= 28)) FMOE_LAUNCH_SELECT_OCC(1, RH_, RC_, 8, true, 2, true);      \
+        else if (in_pairs) FMOE_LAUNCH_SELECT_OCC(1, RH_, RC_, 8, true, 2, all_reuse);             \
+        else if (crowded && (all_reuse || K <= 28)) FMOE_LAUNCH_SELECT_OCC(1, RH_, RC_, 8, true, 1, true);  \
+        else if (crowded) FMOE_LAUNCH_SELECT_OCC(1, RH_, RC_, 8, true, 1, all_reuse);              \
+        else FMOE_LAUNCH_SELECT_OCC(1, RH_, RC_, 1, true, 1, false);                               \
     } while (0)
     if (K <= 128 && nk <= 512) {
         CandidateTable table;

@@ -126,7 +126,9 @@ __device__ inline uint64_t key_at(const uint64_t (&v)[RK], int pos) {
 // sizes where a whole list fits the wave's registers (R keys per lane).
 //   1. a score tau that at least K and at most CAP keys reach (CAP: the slots that are sorted), found bit by bit from the top (per
 //      bit one compare per register, the counts come from the ballots on the scalar unit): any such tau will do, so the search
-//      ends after 3 to 9 of the 32 bits, where the exact K-th largest score would take about 22;
+//      ends after 3 to 9 of the 32 bits, where the exact K-th largest score would take about 22.  REUSE: the score that served
+//      the wave's last list of this kind is tried first; lists of a batch resemble each other, and with slots to spare (CAP = 32,
+//      K = 16) it serves nine lists of ten.  Whichever score is found, the result is the same;
 //   2. the keys at or above tau go to slots in LDS (positions from ballot prefix counts);
 //   3. one bitonic sort of the slots on the 64-bit keys; the first K are the result.
 // List order is key index order for a half (position p = r*64 + lane), so ties at the cut go to the lowest index there; among
@@ -134,8 +136,9 @@ __device__ inline uint64_t key_at(const uint64_t (&v)[RK], int pos) {
 // more than CAP keys tie with the K-th, the keys above that score and then the equal ones in list order are taken again.
 // Up to 32 experts per token (SMALL) CAP is 32 and one sort orders both halves, 32 lanes each.
 // Bound by instruction issue, the scalar unit (searches, lane masks) hardly less than the vector units: 32768 tokens, 128 keys, 16
-// experts take 28 us (323 scalar and 294 vector instructions per token), 32 with a constant per layer of the sorts and the search on
-// the vector unit (332 and 472), 92 with the exact search and three 64-lane sorts; 64 experts 51 for 57.  128 tokens or fewer, 32
+// experts take 22.4 us, 28 without REUSE (323 scalar and 294 vector instructions per token: each unit busy two thirds of the time),
+// 32 with a constant per layer of the sorts and the search on the vector unit (332 and 472), 92 with the exact search and three
+// 64-lane sorts; 64 experts 52 for 57.  128 tokens or fewer, 32
 // experts: 10.3 -> 7.1 with the threshold, 4096 tokens, 64 experts: 16 -> 12.5 and now 11.0.
 // ------------------------------------------------------------------------------------------------------------
 template <int CTRL> __device__ inline uint32_t dpp_max_step(uint32_t v) {      // lanes without a source read 0
@@ -216,17 +219,39 @@ __device__ inline void collect_exactly(const uint64_t (&key)[R], uint32_t tau, i
     for (int p = k + lane; p < cap; p += kWave) slots[p] = 0ull;
 }
 
-// At least k of the list's keys, all that reach a common score (or exactly k of them), into slots[0 .. cap), the rest of them 0;
-// cap wave-private LDS entries.  n: keys in the list; unused entries hold key 0 (below every score).
-template <int R, int RK, int LOW>
-__device__ inline void collect_top(const uint64_t (&key)[R], int n, int k, int cap, uint64_t* slots, int lane) {
-    const uint32_t tau = n <= cap ? 1u : selecting_score<R, RK, LOW>(key, k, cap);
-    uint64_t m[R];
+// The registers' lanes whose score reaches tau, and how many they are.
+template <int R>
+__device__ inline int lanes_reaching(const uint64_t (&key)[R], uint32_t tau, uint64_t (&m)[R]) {
     int total = 0;
 #pragma unroll
     for (int r = 0; r < R; ++r) {
         m[r] = __builtin_amdgcn_ballot_w64((uint32_t)(key[r] >> 32) >= tau);
         total += __builtin_popcountll(m[r]);
+    }
+    return total;
+}
+
+// At least k of the list's keys, all that reach a common score (or exactly k of them), into slots[0 .. cap), the rest of them 0;
+// cap wave-private LDS entries.  n: keys in the list; unused entries hold key 0 (below every score).
+// REUSE: seen is a score that selected from a list of this kind before (0: none yet; 1 where n <= cap), replaced when another had
+// to be searched for.  It stays in a vector register: the scalar registers of eight waves are all taken, and on them it cost 2 us of 25.
+template <int R, int RK, int LOW, bool REUSE>
+__device__ inline void collect_top(const uint64_t (&key)[R], int n, int k, int cap, uint64_t* slots, int lane, uint32_t& seen) {
+    uint64_t m[R];
+    uint32_t tau;
+    int total;
+    if constexpr (REUSE) {
+        tau = seen;
+        total = lanes_reaching<R>(key, tau, m);
+        if (n > cap && (uint32_t)(total - k) > (uint32_t)(cap - k)) {
+            tau = selecting_score<R, RK, LOW>(key, k, cap);
+            total = lanes_reaching<R>(key, tau, m);
+            seen = tau;
+            asm("" : "+v"(seen));
+        }
+    } else {
+        tau = n <= cap ? 1u : selecting_score<R, RK, LOW>(key, k, cap);
+        total = lanes_reaching<R>(key, tau, m);
     }
     if (total > cap) {                    // more ties with the k-th score than there are slots
         collect_exactly<R>(key, tau, k, cap, slots, lane);
@@ -276,7 +301,7 @@ template <int RK, int RC, int WAVES, bool PAIRED, int TOK = 1> struct SelectLds 
 
 // WAVES waves per workgroup, a token each; PAIRED: two waves per token (one launch round of few tokens), one per half, the first of
 // them going on with the candidates.  TOK = 2 (SMALL): two tokens per wave, whose candidates one sort orders, 32 lanes each.
-template <typename T, typename TG, int RK, int RH, int RC, bool FROM_LOGITS, bool SMALL, int WAVES, bool PAIRED, int TOK = 1>
+template <typename T, typename TG, int RK, int RH, int RC, bool FROM_LOGITS, bool SMALL, int WAVES, bool PAIRED, int TOK = 1, bool REUSE = false>
 __device__ __forceinline__ void router_select_tokens(
     const T* __restrict__ lp, int64_t num_tokens, int nk, int top_k, int num_cand, T* __restrict__ scores,
     int64_t* __restrict__ indices, TG* __restrict__ gates, int norm_topk_prob, uint32_t* __restrict__ row_offsets,
@@ -299,6 +324,8 @@ __device__ __forceinline__ void router_select_tokens(
     const int wave = (int)(threadIdx.x >> 6);
     const int mine = PAIRED ? wave >> 1 : wave * TOK;    // the wave's (first) token of the workgroup
     const int64_t tokens_total = (int64_t)blocks * TOKENS;
+    uint32_t seen[3] = {nk <= CAP ? 1u : 0u, nk <= CAP ? 1u : 0u, num_cand <= CAP ? 1u : 0u};   // half 0, half 1, candidates
+    if constexpr (REUSE) asm("" : "+v"(seen[0]), "+v"(seen[1]), "+v"(seen[2]));
 
     // PAIRED: one round; else nothing below synchronises across waves
     for (int64_t first = (int64_t)block * TOKENS + mine; PAIRED || first < num_tokens; first += tokens_total) {
@@ -338,7 +365,8 @@ __device__ __forceinline__ void router_select_tokens(
                     key[r] = p < nk ? make_key(FROM_LOGITS ? (v[r] - shift) - lse : v[r], (uint32_t)p) : 0ull;
                 }
                 // the candidates look up ranks below top_k (entries past nk stay key 0)
-                collect_top<RH, RK, FROM_LOGITS ? 0 : LOW>(key, nk, top_k < nk ? top_k : nk, CAP, slot[wave] + (SMALL && !PAIRED ? h * CAP : 0), lane);
+                collect_top<RH, RK, FROM_LOGITS ? 0 : LOW, REUSE>(key, nk, top_k < nk ? top_k : nk, CAP, slot[wave] + (SMALL && !PAIRED ? h * CAP : 0), lane, seen[h]);
+                if (REUSE && h == 0 && seen[1] == 0u) seen[1] = seen[0];
                 if (!SMALL || PAIRED || h == 1) {
                     uint64_t best[RK];
                     sort_slots<RK, SMALL>(slot[wave], best, lane);
@@ -374,7 +402,7 @@ __device__ __forceinline__ void router_select_tokens(
                     ckey[t][r] = make_key(s, flat);
                 }
             }
-            collect_top<RC, RK, LOW>(ckey[t], num_cand, top_k, CAP, slot[wave] + t * CAP, lane);
+            collect_top<RC, RK, LOW, REUSE>(ckey[t], num_cand, top_k, CAP, slot[wave] + t * CAP, lane, seen[2]);
         }
         uint64_t best[RK];
         sort_slots<RK, SMALL>(slot[wave], best, lane);

@@ -166,6 +166,33 @@ def test_router_gates_of_two_tokens_to_a_wave(norm, nk, K):
             assert torch.equal(a[part], b)
 
 
+@pytest.mark.parametrize("T,nk,K", [
+    (16387, 128, 16), (16386, 100, 20), (16385, 200, 28), (4200, 128, 19), (4100, 512, 28),      # starting from the wave's last score ...
+    (8200, 128, 56), (4100, 300, 33), (4100, 65, 40),
+    (16387, 128, 29), (4200, 128, 57), (8195, 20, 16),                                            # ... not, and lists that need none
+])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_router_lists_that_do_not_resemble_the_last_one(T, nk, K, dtype):
+    # neighbouring lists of other scale, of a few values, of one value, with infinities and of nothing but NaN: scores and experts are
+    # bit for bit those of calls of at most 64 tokens, in which every wave has one token and searches for itself
+    from flash_moe.ops import flash_router_func
+
+    lp = cuda(orc.make_router_inputs(T, nk, seed=T + K, log_probs=False))
+    t = torch.arange(T, device="cuda")
+    lp *= torch.tensor([1.0, 1.0, 100.0, 1e-3, 1.0, -3.0, 1e30], device="cuda")[t % 7][None, :, None]
+    lp[:, t % 11 == 3] = lp[:, t % 11 == 3].round()
+    lp[0, t % 13 == 5] = 0.5
+    lp[1, t % 17 == 2, : nk // 2] = float("-inf")
+    lp[:, t % 19 == 4] = float("nan")
+    lp = lp.to(dtype)
+    s, i = flash_router_func(lp, nk, K)
+    bits = torch.int32 if dtype == torch.float32 else torch.int16
+    for lo in list(range(0, 512, 64)) + [T - 64]:
+        a, b = flash_router_func(lp[:, lo:lo + 64].contiguous(), nk, K)
+        assert torch.equal(s[lo:lo + 64].view(bits), a.view(bits))
+        assert torch.equal(i[lo:lo + 64], b)
+
+
 def test_router_limits_of_the_large_top_k_kernel():
     from flash_moe.ops import flash_router_func
 
