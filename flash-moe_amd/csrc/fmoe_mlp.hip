@@ -25,6 +25,7 @@
 // gemm_splitk_kernel; fp32 whose rows are no multiples of 16 bytes takes a plain FMA kernel.
 #include "fmoe_common.h"
 #include "fmoe_gemm.h"
+#include "fmoe_gemm128.h"
 #include "fmoe_gemm256.h"
 
 namespace fmoe {
@@ -59,6 +60,14 @@ __global__ __launch_bounds__(kWideThreads, 2) void gemm_wide_sliced_kernel(const
     const int tiles = tiles_m * tiles_n, at = xcd_run((int)blockIdx.x, (int)gridDim.x, xcds);
     gemm_wide_tiles<T, kEpiPart, true, true>(A, B, nullptr, reinterpret_cast<T*>(planes), nullptr, M, N, K, tiles_m, tiles_n, 1, at % tiles,
                                              tiles, at / tiles, slices);
+}
+
+// tiles_m * tiles_n workgroups
+template <typename T>
+__global__ __launch_bounds__(256, 1) void gemm_solo_kernel(const T* __restrict__ A, const T* __restrict__ B, T* __restrict__ C, const T* __restrict__ R, int M,
+                                                           int N, int K, int tiles_m, int tiles_n, int xcds) {
+    __shared__ __attribute__((aligned(1024))) T lds[4 * kSoloStage];
+    gemm_solo_tile<T>(A, B, C, R, M, N, K, tiles_m, tiles_n, xcds, (int)blockIdx.x, lds);
 }
 
 template <typename T, int BM, int BN, int WAVES_N, int NSTAGE>
@@ -184,7 +193,8 @@ void launch_gemm_splitk(const T* A, const T* B0, const T* B1, T* C, const T* R, 
 }
 
 // 128 x 128 and smaller tiles: 4 waves that read half a k-tile of fragments ahead (a whole one in fp32), one workgroup per CU
-// with four stages in flight, or (128 x 128) two per CU with two stages when there are more tiles than CUs.
+// with four stages in flight, or (128 x 128) two per CU with two stages when there are more tiles than CUs; 128 x 128 tiles of a long k
+// loop that all have a CU to themselves: fmoe_gemm128.h.
 template <typename T, int EPI, bool RAGGED>
 void launch_tiles(const T* A, const T* B0, const T* B1, T* C, const T* R, int M, int N, int K, hipStream_t stream) {
     constexpr int KT = kStageK<T>, PF = kSmallAhead<T>, FR = kFragRows<T>;
@@ -200,6 +210,13 @@ void launch_tiles(const T* A, const T* B0, const T* B1, T* C, const T* R, int M,
             else launch_gemm_dma<T, 256, 256, 2, 4, KT, 2, EPI, 1, FR, RAGGED>(A, B0, B1, C, R, M, N, K, stream);
             break;
         case kTile128:
+            if constexpr (sizeof(T) == 2 && EPI == kEpiPlain) {
+                if (tiles <= chip_info().cus && K > (kSoloTiles - 1) * 64 && aligned16(C) && aligned16(R)) {
+                    hipLaunchKernelGGL((gemm_solo_kernel<T>), dim3((unsigned)tiles), dim3(256), 0, stream, A, B0, C, R, M, N, K, (M + 127) / 128,
+                                       (N + 127) / 128, chip_info().xcds);
+                    break;
+                }
+            }
             if (tiles <= chip_info().cus) launch_gemm_dma<T, 128, 128, 2, 2, KT, 4, EPI, PF, FR, RAGGED>(A, B0, B1, C, R, M, N, K, stream);
             else launch_gemm_dma<T, 128, 128, 2, 2, KT, 2, EPI, PF, FR, RAGGED>(A, B0, B1, C, R, M, N, K, stream);
             break;

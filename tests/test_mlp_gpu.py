@@ -156,6 +156,27 @@ def test_mlp_fp32_on_gate_up_tiles_of_32_columns(T, H, I):
     test_mlp_remainders_of_every_tile_shape(torch.float32, T, H, I)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("T,H,I", [
+    (4096, 1024, 1536), (2000, 1928, 1480), (3900, 1000, 1544), (1100, 2960, 1608), (3001, 1000, 2664),     # 24, 24, 25, 26 and 42 k-tiles
+    (2000, 1928, 1472),                                                                                   # the last before them
+])
+def test_mlp_down_on_tiles_whose_k_the_waves_divide(dtype, T, H, I):
+    """128 x 128 tiles that one wave each multiplies a quarter of k of: whole ones and remainders in every extent, guard rows around the
+    output, with a residual and without, and in place of it."""
+    test_mlp_remainders_of_every_tile_shape(dtype, T, H, I)
+    from flash_moe import _C
+
+    act, wd, res = (torch.randn(*s, device="cuda").to(dtype) for s in ((T, I), (H, I), (T, H)))
+    wd *= 0.02
+    L, code, stream = _C.lib(), _C.dtype_code(dtype), _C.current_stream(act.device)
+    tol, product = {torch.bfloat16: 6e-3, torch.float16: 8e-4}[dtype], act.double() @ wd.double().t()
+    plain, added = torch.empty_like(res), res.clone()
+    _C.check(L.fmoe_mlp_down(_C.ptr(act), _C.ptr(wd), T, H, I, code, None, _C.ptr(plain), stream), "down")
+    _C.check(L.fmoe_mlp_down(_C.ptr(act), _C.ptr(wd), T, H, I, code, _C.ptr(added), _C.ptr(added), stream), "down")
+    assert rel_fro(plain, product) < tol and rel_fro(added, product + res.double()) < tol
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
 @pytest.mark.parametrize("T,H,I", [(47, 1032, 8200), (129, 520, 4104), (203, 1032, 12296), (300, 2056, 8008), (129, 1001, 4004)])
 @pytest.mark.parametrize("with_residual", [False, True])
