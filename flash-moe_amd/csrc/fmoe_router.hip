@@ -479,10 +479,10 @@ int launch_router(const void* lp, int64_t T_, int nk, int K, void* scores, int64
 // Two tokens to a wave save a third of the sorting once every wave has two (us, 128 keys, 16 experts, without REUSE: 32768 tokens 29.4
 // -> 28.0, 16384 16.2 -> 15.6, but 12288 11.9 -> 12.9 and 8192 9.6 -> 10.5).
 // Lists start from the score that served the wave's previous list (REUSE) where a wave has several and at least four slots beyond
-// K are left, eight of 64, so that it often serves again (us, 32768 tokens, without | with, 128 keys: K = 16 28.0 | 22.4, 24 27.5 |
-// 25.5, 28 29.7 | 28.8, 32 35.6 | 36.6, 40 39.1 | 36.7, 50 41.8 | 40.2, 58 44.2 | 44.4, 64 52.2 | 53.9; 512 keys: K = 16 44.1 | 35.1, 24
-// 50.4 | 44.7, 30 56.9 | 56.9, 40 59.7 | 51.0; 10000 tokens, K = 16: 10.5 | 9.75, 6000 8.0 | 7.9).  Two keys per lane gain 0 to 4 %
-// and are left as they are.
+// K are left, eight of 64, so that it often serves again (us with the sorts on integers, 32768 tokens, without | with, 128 keys: K = 16
+// 28.0 | 22.4, 24 27.5 | 25.5, 28 29.7 | 28.8, 32 35.6 | 36.6, 40 39.1 | 36.7, 50 41.8 | 40.2, 58 44.2 | 44.4, 64 52.2 | 53.9; 512 keys:
+// K = 16 44.1 | 35.1, 24 50.4 | 44.7, 30 56.9 | 56.9, 40 59.7 | 51.0; 10000 tokens, K = 16: 10.5 | 9.75, 6000 8.0 | 7.9).  Two keys per
+// lane gain 0 to 4 % and are left as they are.
 #define FMOE_LAUNCH_SELECT(RK_, RH_, RC_)                                                          \
     do {                                                                                           \
         if (crowded && RK_ == 1 && K <= 56) FMOE_LAUNCH_SELECT_OCC(1, RH_, RC_, 8, false, 1, true); \

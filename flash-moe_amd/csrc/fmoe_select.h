@@ -130,16 +130,16 @@ __device__ inline uint64_t key_at(const uint64_t (&v)[RK], int pos) {
 //      the wave's last list of this kind is tried first; lists of a batch resemble each other, and with slots to spare (CAP = 32,
 //      K = 16) it serves nine lists of ten.  Whichever score is found, the result is the same;
 //   2. the keys at or above tau go to slots in LDS (positions from ballot prefix counts);
-//   3. one bitonic sort of the slots on the 64-bit keys; the first K are the result.
+//   3. one bitonic sort of the slots (num_keys is at most 512: pairs have 18 bits); the first K are the result.
 // List order is key index order for a half (position p = r*64 + lane), so ties at the cut go to the lowest index there; among
 // candidate sums tied at the cut the earlier candidate (lower rank in half 0) is taken: where the sorted keys show such a tie, or
 // more than CAP keys tie with the K-th, the keys above that score and then the equal ones in list order are taken again.
 // Up to 32 experts per token (SMALL) CAP is 32 and one sort orders both halves, 32 lanes each.
 // Bound by instruction issue, the scalar unit (searches, lane masks) hardly less than the vector units: 32768 tokens, 128 keys, 16
-// experts take 22.4 us, 28 without REUSE (323 scalar and 294 vector instructions per token: each unit busy two thirds of the time),
-// 32 with a constant per layer of the sorts and the search on the vector unit (332 and 472), 92 with the exact search and three
-// 64-lane sorts; 64 experts 52 for 57.  128 tokens or fewer, 32
-// experts: 10.3 -> 7.1 with the threshold, 4096 tokens, 64 experts: 16 -> 12.5 and now 11.0.
+// experts take 20.3 us, 22.4 with sorts on integers, 28 also without REUSE (323 scalar and 294 vector instructions per token: each unit
+// busy two thirds of the time), 32 with a constant per layer of the sorts and the search on the vector unit (332 and 472), 92 with the
+// exact search and three 64-lane sorts; 64 experts 46.6 for 57.  128 tokens or fewer, 32 experts: 10.3 -> 7.1 with the threshold, 4096
+// tokens, 64 experts: 16 -> 12.5, 11.0 and now 9.9.
 // ------------------------------------------------------------------------------------------------------------
 template <int CTRL> __device__ inline uint32_t dpp_max_step(uint32_t v) {      // lanes without a source read 0
     const uint32_t o = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xF, 0xF, true);
@@ -266,14 +266,82 @@ __device__ inline void collect_top(const uint64_t (&key)[R], int n, int k, int c
     for (int p = base + lane; p < cap; p += kWave) slots[p] = 0ull;
 }
 
+// The network for lists whose indexes fit 20 bits: a key is the score's 32 bits and those 20 as the mantissa of a positive normal
+// double, (hi, lo).  In a layer the lanes that keep the smaller key hold theirs with the sign set; then both lanes of a pair keep
+// max(mine, -other): one v_max_f64 and one XOR of the signs into the next layer's, where 64-bit integers take a compare, a scalar XOR
+// with the lane mask and two selects that wait for it.  us, integers | doubles: 32768 tokens, 128 keys, K = 16 22.4 | 20.3, 64 52.3 |
+// 46.6, 512 keys, K = 16 35.0 | 33.7, 100 107 | 95.5, 128 138 | 126; 4096 tokens, 128 keys, K = 64 10.9 | 9.9.
+template <int RK> constexpr int sign_bit(int J) {           // lane bit whose set lanes hold negated keys in layer J; -1: none
+    int b = -1;
+    for (int l = J / RK; l > 0; l >>= 1) ++b;
+    return b;
+}
+template <int FROM, int TO> __device__ inline void turn_sign(uint32_t& hi, int lane) {
+    if constexpr (FROM != TO) {
+        uint32_t m = 0u;
+        if constexpr (FROM >= 0) m ^= (uint32_t)lane << (31 - FROM);
+        if constexpr (TO >= 0) m ^= (uint32_t)lane << (31 - TO);
+        hi ^= m & 0x80000000u;
+    }
+}
+template <int RK, int J, int X, int FROM>
+__device__ inline void signed_layer(uint32_t (&hi)[RK], uint32_t (&lo)[RK], int lane) {
+    constexpr int TO = sign_bit<RK>(J);
+#pragma unroll
+    for (int r = 0; r < RK; ++r) turn_sign<FROM, TO>(hi[r], lane);
+    auto value = [&](uint32_t h, uint32_t l) { return __builtin_bit_cast(double, ((uint64_t)h << 32) | l); };
+    double w[RK];
+#pragma unroll
+    for (int r = 0; r < RK; ++r) {
+        const double a = value(hi[r], lo[r]);
+        if constexpr (X < RK) {
+            const double b = value(hi[r ^ X], lo[r ^ X]);
+            if ((r & J) == 0) asm("v_max_f64 %0, %1, %2" : "=v"(w[r]) : "v"(a), "v"(b));
+            else asm("v_min_f64 %0, %1, %2" : "=v"(w[r]) : "v"(a), "v"(b));
+        } else {
+            const double b = value(xor_lane_u32(hi[r ^ (X % RK)], X / RK, lane), xor_lane_u32(lo[r ^ (X % RK)], X / RK, lane));
+            asm("v_max_f64 %0, %1, -%2" : "=v"(w[r]) : "v"(a), "v"(b));
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < RK; ++r) {
+        const uint64_t u = __builtin_bit_cast(uint64_t, w[r]);
+        hi[r] = (uint32_t)(u >> 32);
+        lo[r] = (uint32_t)u;
+    }
+}
+template <int RK, int J>
+__device__ inline void signed_layers(uint32_t (&hi)[RK], uint32_t (&lo)[RK], int lane) {
+    signed_layer<RK, J, J, sign_bit<RK>(2 * J)>(hi, lo, lane);
+    if constexpr (J > 1) signed_layers<RK, J / 2>(hi, lo, lane);
+}
+template <int RK, int N, int K = 2>
+__device__ inline void signed_blocks(uint32_t (&hi)[RK], uint32_t (&lo)[RK], int lane) {
+    signed_layer<RK, K / 2, K - 1, K == 2 ? -1 : sign_bit<RK>(1)>(hi, lo, lane);
+    if constexpr (K > 2) signed_layers<RK, K / 4>(hi, lo, lane);
+    if constexpr (K < N) signed_blocks<RK, N, 2 * K>(hi, lo, lane);
+    else
+#pragma unroll
+        for (int r = 0; r < RK; ++r) turn_sign<sign_bit<RK>(1), -1>(hi[r], lane);
+}
+
+// Indexes below 2^20.
 template <int RK, bool SMALL>
 __device__ inline void sort_slots(const uint64_t* slots, uint64_t (&best)[RK], int lane) {
     __builtin_amdgcn_wave_barrier();      // LDS operations of one wave complete in order; keep the compiler from moving them
 #pragma unroll
     for (int r = 0; r < RK; ++r) best[r] = slots[lane * RK + r];
     __builtin_amdgcn_wave_barrier();
-    if constexpr (SMALL) sort_blocks<RK, true, kWave / 2>(best, lane);
-    else bitonic_sort<RK, true>(best, lane);
+    uint32_t hi[RK], lo[RK];
+#pragma unroll
+    for (int r = 0; r < RK; ++r) {
+        const uint32_t score = (uint32_t)(best[r] >> 32);
+        hi[r] = __builtin_amdgcn_alignbit(0x400u, score, 12);
+        lo[r] = (score << 20) | ((uint32_t)best[r] & 0xfffffu);
+    }
+    signed_blocks<RK, SMALL ? kWave / 2 : RK * kWave>(hi, lo, lane);
+#pragma unroll
+    for (int r = 0; r < RK; ++r) best[r] = ((uint64_t)__builtin_amdgcn_alignbit(hi[r], lo[r], 20) << 32) | (lo[r] | 0xfff00000u);
 }
 
 // The candidate pairs (rank in half 0) | (rank in half 1) << 8, listed by rank in half 0: the list depends on top_k only,

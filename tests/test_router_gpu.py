@@ -193,6 +193,34 @@ def test_router_lists_that_do_not_resemble_the_last_one(T, nk, K, dtype):
         assert torch.equal(i[lo:lo + 64], b)
 
 
+@pytest.mark.parametrize("T,K", [(40, 16), (40, 64), (40, 128), (4200, 19), (4200, 60), (16385, 32)])
+def test_router_sorts_the_largest_pair_indexes(T, K):
+    # 512 keys, the best of them last: pair indexes up to 2^18 - 1, in runs of equal scores, with infinities of either sign, zeros of
+    # either sign apart, against a stable sort of the candidates on the CPU
+    from flash_moe.ops import flash_router_func
+
+    nk = 512
+    g = torch.Generator().manual_seed(T + K)
+    lp = (torch.randn(2, T, nk, generator=g) * 2).round() / 2 + torch.arange(nk) // 64
+    lp[lp == 0] = 0.25
+    lp[:, 1, -1] = 100.0                                       # the last pair of all, in a token without infinities
+    lp[0, ::3, -1] = float("inf")
+    lp[1, ::5, : nk // 2] = float("-inf")
+    s, i = flash_router_func(cuda(lp), nk, K)
+    s, i = s.cpu(), i.cpu()
+    top, ids = lp[:, :64].sort(dim=-1, descending=True, stable=True)
+    pairs = [(a, b) for a in range(K) for b in range(K // (a + 1))]
+    a, b = torch.tensor([p[0] for p in pairs]), torch.tensor([p[1] for p in pairs])
+    sums, flat = top[0][:, a] + top[1][:, b], ids[0][:, a] * nk + ids[1][:, b]
+    kept = sums.sort(dim=-1, descending=True, stable=True)[1][:, :K]
+    sums, flat = sums.gather(-1, kept), flat.gather(-1, kept)
+    order = flat.sort(-1)[1]
+    order = order.gather(-1, sums.gather(-1, order).sort(dim=-1, descending=True, stable=True)[1])
+    n = min(T, 64)
+    assert torch.equal(s[:n], sums.gather(-1, order)) and torch.equal(i[:n], flat.gather(-1, order))
+    assert i.max() == nk * nk - 1 and torch.equal(s, lp[0].gather(-1, i // nk) + lp[1].gather(-1, i % nk))
+
+
 def test_router_limits_of_the_large_top_k_kernel():
     from flash_moe.ops import flash_router_func
 
