@@ -14,6 +14,8 @@
 // expert backward is one wave per token with the token's rows of x and dout in registers (the layout of the forward
 // row kernel).  The per-expert part needs the pairs grouped by expert: group_pairs (fmoe_bucket.hip) gives each expert one segment
 // listing its pairs in ascending pair index, and the wave that owns the expert walks it in that order.
+#include <type_traits>
+
 #include "fmoe_common.h"
 #include "fmoe_vec.h"
 
@@ -411,7 +413,7 @@ template <typename T, int NCH, int WAVES>
 __global__ __launch_bounds__((WAVES > 1 ? WAVES : kBwdWaves) * kWave) void expert_backward_token_kernel(
     const T* __restrict__ dout, const T* __restrict__ x, const T* __restrict__ down, const T* __restrict__ up,
     const int64_t* __restrict__ indices, const T* __restrict__ gates, T* __restrict__ dx, T* __restrict__ dgates,
-    float* __restrict__ coef_up, float* __restrict__ coef_down, int64_t num_tokens,
+    float2* __restrict__ coef, int64_t num_tokens,
     int hidden, int64_t num_experts, int top_k) {
     constexpr int V = Elem<T>::kVec;
     constexpr int PIF = NCH >= 8 ? 1 : (NCH >= 4 ? 2 : 4);   // (down, up) row pairs requested ahead
@@ -492,8 +494,7 @@ __global__ __launch_bounds__((WAVES > 1 ? WAVES : kBwdWaves) * kWave) void exper
             for (int c = 0; c < NCH; ++c) axpy16<T>(ds, dn[u][c], acc[c]);
             if (lane == 0 && k < top_k) {
                 const int64_t p = token * top_k + k;
-                coef_up[p] = valid[u] ? act * gate[u] : 0.0f;
-                coef_down[p] = ds;
+                coef[p] = float2{valid[u] ? act * gate[u] : 0.0f, ds};
                 dgates[p] = Elem<T>::from_f32(valid[u] ? da[u] * act : 0.0f);
             }
         }
@@ -527,13 +528,14 @@ __global__ __launch_bounds__((WAVES > 1 ? WAVES : kBwdWaves) * kWave) void exper
 
 // Column-slice schedule of the per-token part (same kernels as the forward, fmoe_expert.hip): the partial dot products
 // s = <x, down[e]> and u = <dout, up[e]> come per slice; this kernel sums them (or takes the scores the forward kept) and forms
-// every pair's coefficients and gate gradient; dx is then the forward's `states` pass over `down` with coef_down.
-// place: NULL, or the (token, k) position of every list position: the states pass then needs coef_down in list order as well.
+// every pair's coefficients and gate gradient; dx is then the forward's `states` pass over `down` with
+// coef_list, the coefficients of `down` in list order.  place: NULL (list order is pair order), or the (token, k) position of every list
+// position.
 template <typename T>
 __global__ __launch_bounds__(256) void expert_backward_gate_kernel(
     const float* __restrict__ spart_s, const float* __restrict__ scores, const float* __restrict__ spart_u,
     const T* __restrict__ gates, const uint32_t* __restrict__ off32, const uint16_t* __restrict__ place,
-    T* __restrict__ dgates, float* __restrict__ coef_up, float* __restrict__ coef_down, float* __restrict__ coef_list, int64_t pairs,
+    T* __restrict__ dgates, float2* __restrict__ coef, float* __restrict__ coef_list, int64_t pairs,
     int num_slices, int top_k) {
     const int64_t at = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (at >= pairs) return;
@@ -548,10 +550,9 @@ __global__ __launch_bounds__(256) void expert_backward_gate_kernel(
     const float gate = Elem<T>::to_f32(gates[p]);
     const float sig = 1.0f / (1.0f + __expf(-s));
     const float act = s * sig;
-    coef_up[p] = valid ? act * gate : 0.0f;
     const float cd = valid ? u * gate * (sig * (1.0f + s * (1.0f - sig))) : 0.0f;
-    coef_down[p] = cd;
-    if (place != nullptr) coef_list[at] = cd;
+    coef[p] = float2{valid ? act * gate : 0.0f, cd};
+    coef_list[at] = cd;
     dgates[p] = Elem<T>::from_f32(valid ? u * act : 0.0f);
 }
 
@@ -564,8 +565,7 @@ __global__ __launch_bounds__(256) void expert_backward_gate_kernel(
 // Where x and dout fit the L2 whole, chunks of two packets per lane save walking the lists twice.
 template <typename T, int NCH>
 __global__ __launch_bounds__(kBwdWaves* kWave) void expert_backward_weight_kernel(
-    const T* __restrict__ dout, const T* __restrict__ x, const float* __restrict__ coef_up,
-    const float* __restrict__ coef_down, const uint32_t* __restrict__ pairs, const int32_t* __restrict__ offsets,
+    const T* __restrict__ dout, const T* __restrict__ x, const float2* __restrict__ coef, const uint32_t* __restrict__ pairs, const int32_t* __restrict__ offsets,
     T* __restrict__ ddown, T* __restrict__ dup, int hidden, int64_t num_experts, int top_k, int span, int units, int chunks, int xcds) {
     constexpr int V = Elem<T>::kVec, PIF = 8 / NCH;
     const int lane = lane_id();
@@ -614,7 +614,8 @@ __global__ __launch_bounds__(kBwdWaves* kWave) void expert_backward_weight_kerne
         const int n = end - done < kWave ? end - done : kWave;
         const uint32_t mine = pairs[done + (lane < n ? lane : n - 1)];
         const uint32_t tok = mine / (uint32_t)top_k;
-        const float cu = coef_up[mine], cd = coef_down[mine];
+        const float2 both = coef[mine];
+        const float cu = both.x, cd = both.y;
         u32x4_t xq[PIF][NCH], gq[PIF][NCH];
         auto load = [&](int j, u32x4_t (&xr)[NCH], u32x4_t (&gr)[NCH]) {
             const int64_t t = (int64_t)(uint32_t)__builtin_amdgcn_readlane((int)tok, j < n ? j : n - 1);
@@ -646,10 +647,112 @@ __global__ __launch_bounds__(kBwdWaves* kWave) void expert_backward_weight_kerne
     }
 }
 
+// ---- the same where 1-KB chunks of x and dout do not fit an L2 -------------------------------------------------------------------
+// A wave's quarters of 16 lanes take spans of experts of their own and 256 bytes of the columns, so that an XCD's chunk of x and dout is a
+// quarter as large.  With four times the chunks the lists are walked as often, so pair_entries_kernel first puts what a pair needs in
+// list order: the byte offset of its token's rows and its two coefficients.  A round is 16 pairs of each quarter, the next rounds' entries
+// and PIF pairs' pieces are requested ahead.  Sums run in ascending pair index here too: the gradients are the same bit for bit.
+// Bound by what the L2s deliver (1 KB chunks: a third of the lines missed at 4096 tokens).  Expert forward and backward, us, 1-KB chunks |
+// quarters, ids uniform and of a product-key router: 4096 tokens x 64 pairs, 16384 experts, 1024 columns 252 | 219 and 220 | 219; 16384 x
+// 64 1047 | 868 and 746 | 748; 8192 x 64, 65536 experts, 512 columns 417 | 380 and 367 | 355.  Where the chunks do fit, quarters only walk
+// the lists more often: 2048 x 32, 2048 columns 165 | 166 and 161 | 170.  8 pairs ahead instead of 4 leave three waves per SIMD: 226.
+__global__ __launch_bounds__(256) void pair_entries_kernel(const float2* __restrict__ coef, const uint32_t* __restrict__ pairs,
+                                                          const int32_t* __restrict__ offsets, int64_t num_experts, uint32_t top_k,
+                                                          uint32_t row_bytes, u32x4_t* __restrict__ entries) {
+    const int at = (int)(blockIdx.x * 256u + threadIdx.x);
+    if (at >= offsets[num_experts]) return;
+    const uint32_t pair = pairs[at];
+    const float2 c = coef[pair];
+    entries[at] = u32x4_t{pair / top_k * row_bytes, __float_as_uint(c.x), __float_as_uint(c.y), 0u};
+}
+
+template <int J> __device__ inline uint32_t row_lane(uint32_t v) {          // lane J's value in each row of 16 lanes (row_newbcast)
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x150 + J, 0xF, 0xF, true);
+}
+template <int N, typename F> __device__ __forceinline__ void static_for(F f) {
+    if constexpr (N > 0) {
+        static_for<N - 1>(f);
+        f(std::integral_constant<int, N - 1>{});
+    }
+}
+
+// span <= 16; num_tokens * hidden values of x are below 2 GB.
+template <typename T>
+__global__ __launch_bounds__(kBwdWaves* kWave) void expert_backward_weight_quarters_kernel(
+    const T* __restrict__ dout, const T* __restrict__ x, const u32x4_t* __restrict__ entries, const int32_t* __restrict__ offsets,
+    T* __restrict__ ddown, T* __restrict__ dup, int64_t num_tokens, int hidden, int64_t num_experts, int span, int units, int chunks, int xcds) {
+    constexpr int V = Elem<T>::kVec, PIF = 4;
+    const int lane = lane_id(), quarter = lane & 48, ql = lane & 15;
+    const int item = ((int)blockIdx.x % xcds) * ((int)gridDim.x / xcds) + (int)blockIdx.x / xcds;      // chunk-major
+    if (item >= units * chunks) return;
+    const int64_t e0 = (((int64_t)(item % units) * kBwdWaves + (threadIdx.x >> 6)) * 4 + (lane >> 4)) * span;
+    const int count = num_experts - e0 < span ? (num_experts > e0 ? (int)(num_experts - e0) : 0) : span;
+    const int packet = item / units * 16 + ql;
+    const bool live = packet < hidden / V;                    // lanes past the row read its first packet and store nothing
+    const uint32_t column = (uint32_t)(live ? packet : 0) * 16u;
+    const int bytes = (int)(num_tokens * hidden * (int64_t)sizeof(T));
+    const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(x), 0, bytes, 0x00020000);
+    const __amdgpu_buffer_rsrc_t gr = __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(dout), 0, bytes, 0x00020000);
+    float acc_d[V], acc_u[V];
+#pragma unroll
+    for (int v = 0; v < V; ++v) acc_d[v] = acc_u[v] = 0.0f;
+
+    const int ends = count > 0 ? offsets[e0 + (ql < count ? ql + 1 : count)] : 0;      // lane ql of a quarter: of its ql-th expert
+    const int begin = count > 0 ? offsets[e0] : 0, end = count > 0 ? offsets[e0 + count] : 0;
+    int longest = 0;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const int n = __builtin_amdgcn_readlane(end - begin, q * 16);
+        longest = n > longest ? n : longest;
+    }
+    const int first_end = __shfl(ends, quarter);
+    int cur = 0, cur_end = count > 0 ? first_end : -1;        // -1: every row of the quarter has left
+    auto flush = [&](int pos) {                               // rows of the experts whose segments end at list position `pos`
+        while (__builtin_amdgcn_ballot_w64(cur_end == pos) != 0ull) {
+            if (cur_end == pos) {
+                if (live) {
+                    reinterpret_cast<u32x4_t*>(ddown + (e0 + cur) * hidden)[packet] = pack16<T>(acc_d);
+                    reinterpret_cast<u32x4_t*>(dup + (e0 + cur) * hidden)[packet] = pack16<T>(acc_u);
+                }
+#pragma unroll
+                for (int v = 0; v < V; ++v) acc_d[v] = acc_u[v] = 0.0f;
+                ++cur;
+            }
+            const int next = __shfl(ends, quarter + (cur < 15 ? cur : 15));
+            cur_end = cur < count ? next : -1;
+        }
+    };
+    flush(begin);
+    auto round_at = [&](int r) {                              // entries past the quarter's list: nothing is fetched, zeros are added
+        const int at = begin + r * 16 + ql;
+        return at < end ? entries[at] : u32x4_t{0x80000000u, 0u, 0u, 0u};
+    };
+    u32x4_t now = round_at(0), next = round_at(1), xq[PIF], gq[PIF];
+    auto load = [&](auto j, const u32x4_t& of, u32x4_t& xv, u32x4_t& gv) {
+        const int at = (int)(row_lane<decltype(j)::value>(of[0]) + column);
+        xv = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(xr, at, 0, 0));
+        gv = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(gr, at, 0, 0));
+    };
+    static_for<PIF>([&](auto j) { load(j, now, xq[j], gq[j]); });
+    for (int r = 0; r * 16 < longest; ++r) {
+        const u32x4_t after = round_at(r + 2);
+        static_for<16>([&](auto j) {
+            constexpr int J = decltype(j)::value, S = J % PIF;
+            axpy16<T>(__uint_as_float(row_lane<J>(now[2])), xq[S], acc_d);
+            axpy16<T>(__uint_as_float(row_lane<J>(now[1])), gq[S], acc_u);
+            flush(begin + r * 16 + J + 1);
+            load(std::integral_constant<int, (J + PIF) % 16>{}, J + PIF < 16 ? now : next, xq[S], gq[S]);
+        });
+        now = next;
+        next = after;
+    }
+}
+
 struct ExpertBwdPlan {
     bool slices, ordered;      // slices: column slices of the tables, on ordered lists or not
+    bool quarters;             // weight gradients by quarter waves: chunks of 1 KB of x and dout exceed an L2
     int num_slices;
-    size_t off_coef_up, off_coef_down, off_pairs, off_group, off_offsets, off_off32, off_place, off_coef_list, off_spart_s, off_spart_u, bytes;
+    size_t off_coef, off_entries, off_pairs, off_group, off_offsets, off_off32, off_place, off_coef_list, off_spart_s, off_spart_u, bytes;
 };
 
 ExpertBwdPlan plan_expert_backward(int64_t T_, int H, int64_t E, int K, int dtype) {
@@ -657,8 +760,10 @@ ExpertBwdPlan plan_expert_backward(int64_t T_, int H, int64_t E, int K, int dtyp
     const size_t pairs = (size_t)T_ * K;
     size_t o = 0;
     auto take = [&](size_t n) { const size_t at = o; o = round_up(o + n, 256); return at; };
-    p.off_coef_up = take(pairs * 4);
-    p.off_coef_down = take(pairs * 4);
+    p.off_coef = take(pairs * 8);
+    const int64_t row = (int64_t)H * (int64_t)dtype_size(dtype);
+    p.quarters = pairs > 0 && 2 * T_ * (row < 1024 ? row : 1024) > chip_info().l2_bytes && T_ * row < (1ll << 31);
+    p.off_entries = take(p.quarters ? pairs * 16 : 0);
     p.off_pairs = take(pairs * 4);
     p.off_group = take(group_pairs_workspace_bytes((int64_t)pairs, E));
     p.off_offsets = take((size_t)(E + 1) * 4);
@@ -670,7 +775,7 @@ ExpertBwdPlan plan_expert_backward(int64_t T_, int H, int64_t E, int K, int dtyp
     if (p.slices) {
         p.off_off32 = take(pairs * 4);
         p.off_place = take(p.ordered ? pairs * 2 : 0);
-        p.off_coef_list = take(p.ordered ? pairs * 4 : 0);
+        p.off_coef_list = take(pairs * 4);
         p.off_spart_s = take((size_t)p.num_slices * pairs * 4);
         p.off_spart_u = take((size_t)p.num_slices * pairs * 4);
     }
@@ -685,8 +790,7 @@ int launch_expert_backward(const void* dout, const void* x, const void* down, co
     constexpr int V = Elem<T>::kVec;
     const ExpertBwdPlan p = plan_expert_backward(T_, H, E, K, dtype);
     char* ws = (char*)workspace;
-    float* coef_up = (float*)(ws + p.off_coef_up);
-    float* coef_down = (float*)(ws + p.off_coef_down);
+    float2* coef = (float2*)(ws + p.off_coef);          // of every pair: of its row of dup, of its row of ddown
     uint32_t* pairs_by_expert = (uint32_t*)(ws + p.off_pairs);
     int32_t* offsets = (int32_t*)(ws + p.off_offsets);
     const int64_t pairs = T_ * K;
@@ -697,7 +801,7 @@ int launch_expert_backward(const void* dout, const void* x, const void* down, co
         uint16_t* place = p.ordered ? (uint16_t*)(ws + p.off_place) : nullptr;
         float* spart_s = (float*)(ws + p.off_spart_s);
         float* spart_u = (float*)(ws + p.off_spart_u);
-        float* coef_list = p.ordered ? (float*)(ws + p.off_coef_list) : coef_down;
+        float* coef_list = (float*)(ws + p.off_coef_list);
         const float* scores = nullptr;
         if (saved != nullptr) {
             const ExpertSaved kept = expert_saved_plan(T_, H, E, K, dtype).at(saved);
@@ -713,7 +817,7 @@ int launch_expert_backward(const void* dout, const void* x, const void* down, co
         if (int rc = expert_slice_scores(dout, up, off32, spart_u, T_, H, E, K, dtype, p.ordered, stream)) return rc;
         hipLaunchKernelGGL((expert_backward_gate_kernel<T>), dim3((unsigned)((pairs + 255) / 256)), dim3(256), 0, stream,
                            (const float*)spart_s, scores, (const float*)spart_u, (const T*)gates, (const uint32_t*)off32,
-                           (const uint16_t*)place, (T*)dgates, coef_up, coef_down, coef_list, pairs, p.num_slices, K);
+                           (const uint16_t*)place, (T*)dgates, coef, coef_list, pairs, p.num_slices, K);
         FMOE_CHECK_LAUNCH("fmoe_expert_backward(coefficients)");
         if (int rc = expert_slice_states(coef_list, down, off32, dx, T_, H, E, K, dtype, p.ordered, stream)) return rc;
     } else {
@@ -722,7 +826,7 @@ int launch_expert_backward(const void* dout, const void* x, const void* down, co
 #define FMOE_LAUNCH_TOKEN(N, W)                                                                                                       \
         hipLaunchKernelGGL((expert_backward_token_kernel<T, N, W>), dim3((unsigned)(W > 1 ? T_ : (T_ + kBwdWaves - 1) / kBwdWaves)), \
                            dim3((W > 1 ? W : kBwdWaves) * kWave), 0, stream, (const T*)dout, (const T*)x, (const T*)down,            \
-                           (const T*)up, indices, (const T*)gates, (T*)dx, (T*)dgates, coef_up, coef_down, T_, H, E, K)
+                           (const T*)up, indices, (const T*)gates, (T*)dx, (T*)dgates, coef, T_, H, E, K)
 #define FMOE_LAUNCH_TOKENS(N, MOST)                                      \
         do {                                                             \
             if (waves >= 8) FMOE_LAUNCH_TOKEN(N, MOST);                  \
@@ -752,10 +856,27 @@ int launch_expert_backward(const void* dout, const void* x, const void* down, co
     const int64_t units = (E + span * kBwdWaves - 1) / (span * kBwdWaves);
 #define FMOE_LAUNCH_WEIGHT(N)                                                                                                             \
     hipLaunchKernelGGL((expert_backward_weight_kernel<T, N>), dim3((unsigned)((units * chunks + xcds - 1) / xcds * xcds)), block, 0, stream, \
-                       (const T*)dout, (const T*)x, (const float*)coef_up, (const float*)coef_down, (const uint32_t*)pairs_by_expert,     \
+                       (const T*)dout, (const T*)x, (const float2*)coef, (const uint32_t*)pairs_by_expert,     \
                        (const int32_t*)offsets, (T*)ddown, (T*)dup, H, E, K, (int)span, (int)units, chunks, xcds)
-    if (resident && nch > 1) FMOE_LAUNCH_WEIGHT(2);
-    else FMOE_LAUNCH_WEIGHT(1);
+    if (p.quarters) {
+        const int quarters = (H / V + 15) / 16;
+        u32x4_t* entries = (u32x4_t*)(ws + p.off_entries);
+        hipLaunchKernelGGL(pair_entries_kernel, dim3((unsigned)((pairs + 255) / 256)), dim3(256), 0, stream, (const float2*)coef,
+                           (const uint32_t*)pairs_by_expert, (const int32_t*)offsets, E, (uint32_t)K, (uint32_t)(H * sizeof(T)), entries);
+        FMOE_CHECK_LAUNCH("fmoe_expert_backward(entries)");
+        span = pairs > 0 ? 64 * E / pairs : 16;
+        const int64_t most_q = E * quarters / (chip_info().cus * 64);
+        if (span > most_q) span = most_q;
+        span = span < 1 ? 1 : (span > 16 ? 16 : span);
+        const int64_t units_q = (E + span * kBwdWaves * 4 - 1) / (span * kBwdWaves * 4);
+        hipLaunchKernelGGL((expert_backward_weight_quarters_kernel<T>), dim3((unsigned)((units_q * quarters + xcds - 1) / xcds * xcds)), block, 0,
+                           stream, (const T*)dout, (const T*)x, (const u32x4_t*)entries, (const int32_t*)offsets, (T*)ddown, (T*)dup, T_, H, E,
+                           (int)span, (int)units_q, quarters, xcds);
+    } else if (resident && nch > 1) {
+        FMOE_LAUNCH_WEIGHT(2);
+    } else {
+        FMOE_LAUNCH_WEIGHT(1);
+    }
 #undef FMOE_LAUNCH_WEIGHT
     FMOE_CHECK_LAUNCH("fmoe_expert_backward(weights)");
     return FMOE_OK;

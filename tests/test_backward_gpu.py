@@ -879,3 +879,37 @@ def test_expert_backward_edges_of_the_waves_and_spans(dtype, T, H, E, K):
     out.backward(dy.double())
     for name, a, leaf in zip(("dx", "ddown", "dup", "dgates"), got, leaves):
         assert rel_fro(a, leaf.grad) < GRAD_FRO[dtype], name
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("T,H,E,K,first", [
+    (4100, 136, 900, 9, 0), (2060, 520, 20000, 7, 0),  # rows below 1 KB; experts without pairs, several spans to a quarter
+    (2050, 1544, 333, 3, 0),                           # the last chunk partial, spans of one
+    (4099, 520, 3, 2, 0), (2200, 1032, 50, 5, 47),     # fewer experts than quarters; lists of very different lengths
+])
+def test_expert_weight_gradients_by_quarter_waves(dtype, T, H, E, K, first):
+    """Chunks of x and dout beyond an L2, with ids out of range among the pairs (they count for nothing)."""
+    from flash_moe.ops.hip.flash_expert import expert_backward
+
+    g = gen(T + H)
+    x, dy = (torch.randn(T, H, generator=g).to(dtype).cuda() for _ in range(2))
+    wd, wu = (torch.randn(E, H, generator=g).mul(0.05).to(dtype).cuda() for _ in range(2))
+    idx = torch.randint(0, E, (T, K), generator=g).clamp_min(first).cuda()
+    idx[5::97, 0] = E
+    gates = torch.softmax(torch.randn(T, K, generator=g), -1).to(dtype).cuda()
+    got = expert_backward(dy, x, wd, wu, idx, gates)
+    valid = idx < E
+    leaves = [t.double().requires_grad_(True) for t in (x, wd, wu, gates)]
+    out = torch.zeros(T, H, device="cuda", dtype=torch.float64)
+    for k in range(K):
+        e = idx[:, k].clamp(max=E - 1)
+        s = (leaves[0] * leaves[1][e]).sum(-1)
+        out = out + (torch.nn.functional.silu(s) * leaves[3][:, k] * valid[:, k])[:, None] * leaves[2][e]
+    out.backward(dy.double())
+    for name, a, leaf in zip(("dx", "ddown", "dup", "dgates"), got, leaves):
+        assert rel_fro(a, leaf.grad) < GRAD_FRO[dtype], name
+    unused = torch.ones(E, dtype=torch.bool, device="cuda")
+    unused[idx[valid]] = False
+    assert (got[1][unused] == 0).all() and (got[2][unused] == 0).all()
+    for a, b in zip(expert_backward(dy, x, wd, wu, idx, gates), got):
+        assert torch.equal(a, b)
