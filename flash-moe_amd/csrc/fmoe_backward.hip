@@ -761,6 +761,7 @@ ExpertBwdPlan plan_expert_backward(int64_t T_, int H, int64_t E, int K, int dtyp
     size_t o = 0;
     auto take = [&](size_t n) { const size_t at = o; o = round_up(o + n, 256); return at; };
     p.off_coef = take(pairs * 8);
+    p.off_coef_list = take(pairs * 4);
     const int64_t row = (int64_t)H * (int64_t)dtype_size(dtype);
     p.quarters = pairs > 0 && 2 * T_ * (row < 1024 ? row : 1024) > chip_info().l2_bytes && T_ * row < (1ll << 31);
     p.off_entries = take(p.quarters ? pairs * 16 : 0);
@@ -771,11 +772,10 @@ ExpertBwdPlan plan_expert_backward(int64_t T_, int H, int64_t E, int K, int dtyp
     p.slices = kept.kept;
     p.ordered = kept.ordered;
     p.num_slices = p.slices ? expert_slice_count(T_, H, E, K, dtype, p.ordered) : 0;
-    p.off_off32 = p.off_place = p.off_coef_list = p.off_spart_s = p.off_spart_u = o;
+    p.off_off32 = p.off_place = p.off_spart_s = p.off_spart_u = o;
     if (p.slices) {
         p.off_off32 = take(pairs * 4);
         p.off_place = take(p.ordered ? pairs * 2 : 0);
-        p.off_coef_list = take(pairs * 4);
         p.off_spart_s = take((size_t)p.num_slices * pairs * 4);
         p.off_spart_u = take((size_t)p.num_slices * pairs * 4);
     }
