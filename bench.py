@@ -192,8 +192,8 @@ LAUNCHES = {
     "expert_c5": ["partition_count_kernel", "bucket_scan_kernel", "partition_scatter_kernel", "partition_local_kernel",
                   "expert_band_copy_kernel", "expert_scores_bucketed_kernel", "expert_gate_sorted_kernel",
                   "expert_owner_sort_kernel", "expert_states_sweep_kernel"],
-    "mlp_gate_up": ["gemm_dma_kernel<256x256 tiles, SwiGLU epilogue>"],
-    "mlp_down": ["gemm_dma_kernel<128x128 tiles, residual epilogue>"],
+    "mlp_gate_up": ["gemm_wide_kernel<256x256 tiles, SwiGLU epilogue>"],
+    "mlp_down": ["gemm_solo_kernel<128x128 tiles, residual epilogue>"],
 }
 
 

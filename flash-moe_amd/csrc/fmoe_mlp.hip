@@ -8,7 +8,8 @@
 //      and up products never go to memory.
 //   2. down: plain epilogue, optional residual add (the routed-expert output in the block).
 //
-// 256 x 256 tiles of the 16-bit types are gemm_wide_kernel's (fmoe_gemm256.h).  The other tiles (gemm_dma_kernel; they and those of
+// 256 x 256 tiles of the 16-bit types are gemm_wide_kernel's (fmoe_gemm256.h), 128 x 128 ones that have a compute unit each
+// gemm_solo_kernel's (fmoe_gemm128.h).  The other tiles (gemm_dma_kernel; they and those of
 // gemm_splitk_kernel are in fmoe_gemm.h) go global -> LDS
 // directly (global_load_lds_dwordx4, no staging registers) into NSTAGE LDS stages, issued NSTAGE-1 k-tiles
 // ahead of their use; one workgroup barrier per k-tile; MFMA fragments (v_mfma_f32_16x16x32 for the 16-bit types) are

@@ -1,11 +1,12 @@
 // Backward of the shared SwiGLU MLP  y = (silu(x Wg^T) * (x Wu^T)) Wd^T  for gfx950.
 //
 // The forward keeps the gate and up products a, b if it was asked to (fmoe_mlp_gate_up_save); without them they are recomputed here
-// (two launches of the forward's own NT GEMM).  The SwiGLU gradient is the fused elementwise kernel of fmoe_backward.hip, which also
-// rebuilds h = silu(a) * b for dWd.  Written in place of dh it costs 2 us in a training step of 4096 tokens of 1024 -> 4096 in
-// bf16 (743 us); keeping it from the forward instead would make the largest tensor a training step holds half as large again.  The
-// remaining products are plain GEMMs in layouts the forward never needs (A B and A^T B): gemm_backward (fmoe_gemm_tr.hip).  What its
-// kernels cannot address goes to rocBLAS, which is loaded on first use so that nothing else depends on it:
+// (two launches of the forward's own NT GEMM).  The SwiGLU gradient is formed where dh is, in the epilogue of its product
+// (swiglu_gradient_together, fmoe_gemm_tr.hip), or, for planes beyond the memory-side cache, in the fused elementwise kernel of
+// fmoe_backward.hip; both also rebuild h = silu(a) * b for dWd, which costs 2 us in a training step of 4096 tokens of 1024 -> 4096 in
+// bf16; keeping it from the forward instead would make the largest tensor a training step holds half as large again.  The remaining
+// products are plain GEMMs in layouts the forward never needs (A B and A^T B): gemm_backward (fmoe_gemm_tr.hip), in one launch where that
+// is the cheaper way.  What its kernels cannot address goes to rocBLAS, which is loaded on first use so that nothing else depends on it:
 //     dh  = dy Wd              [T,H][H,I]
 //     dWd = dy^T h             [T,H]^T [T,I]
 //     dx  = da Wg + db Wu      [T,I][I,H] twice, the second accumulating

@@ -1,5 +1,5 @@
 // Torch binding of the FlashMoE library: argument checks, output and workspace allocation, the current stream and the autograd
-// nodes, natively.  One Python call per op; everything below it (a training step makes about thirty launches and as many
+// nodes, natively.  One Python call per op; everything below it (a training step makes 13 to 25 launches and a dozen
 // allocations) runs without the interpreter, and the backward without the GIL.  The kernels are reached through the C ABI
 // (include/flashmoe_hip.h) only.
 //
