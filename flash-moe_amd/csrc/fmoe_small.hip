@@ -87,11 +87,17 @@ __global__ __launch_bounds__(kSelectDownWaves<CUT> * kWave) void select_and_down
     constexpr int kWaves = kSelectDownWaves<CUT>;
     using Lds = SelectLds<1, RC, kWaves, true>;
     char* lds = launch_lds<T, CUT, kEpiPart, (int)sizeof(Lds)>();
-    const int block = (int)blockIdx.x, down_blocks = down.blocks * down.slices;
-    if (block >= down_blocks)
+    // fp32 products on the k-splitting tiles keep their compute unit's matrix pipes busy for the whole launch: the selections, chains of
+    // latency, start before them and end beside them.  The block, us, product | selections first: 512 tokens, 256 -> 1024 31.4 | 29.1;
+    // 1000, 256 -> 1024 35.7 | 33.4; 400, 512 -> 1024 34.6 | 32.7.  On larger tiles, more of which wait for a place, and in 16 bits the
+    // product goes first: fp32, 1500 tokens, 512 -> 1360 90.8 | 110.7; fp16, 999 tokens, 1000 -> 2664 57.8 | 62.1.
+    constexpr bool kSelectFirst = sizeof(T) == 4 && CUT < kCut64;
+    const int down_blocks = down.blocks * down.slices, select_blocks = (int)gridDim.x - down_blocks;
+    const int block = (int)blockIdx.x - (kSelectFirst ? select_blocks : 0);         // of the product; the others are selections
+    if (block < 0 || block >= down_blocks)
         router_select_tokens<float, T, 1, RH, RC, true, SMALL, kWaves, true>(
             logits32, num_tokens, nk, top_k, num_cand, scores, indices, gates, norm_topk_prob, nullptr, 0u, table,
-            *reinterpret_cast<Lds*>(lds), block - down_blocks, (int)gridDim.x - down_blocks);
+            *reinterpret_cast<Lds*>(lds), kSelectFirst ? (int)blockIdx.x : block - down_blocks, select_blocks);
     else
         product_tiles<T, CUT, kEpiPart>(act, wd, nullptr, reinterpret_cast<T*>(sums), nullptr, M, H, I, down, xcds, block, lds);
 }

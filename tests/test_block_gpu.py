@@ -240,6 +240,12 @@ def test_block_of_few_tokens(dtype, training, T, H, I, E, K):
     assert rel_fro(y.view(T, H)[sample.cuda()], want) < {torch.float32: 3e-6, torch.bfloat16: 6e-3, torch.float16: 8e-4}[dtype]
 
 
+@pytest.mark.parametrize("T,H,I,E,K", [(1000, 256, 1024, 1024, 16), (997, 40, 516, 17000, 33), (2, 136, 264, 100, 7), (509, 264, 520, 20000, 12)])
+def test_block_of_few_tokens_fp32_selections_before_the_down_product(T, H, I, E, K):
+    """Selections dispatched ahead of the k-splitting tiles: nearly as many as those, a last one of fewer tokens, a single one."""
+    test_block_of_few_tokens(torch.float32, T % 2 == 0, T, H, I, E, K)
+
+
 @pytest.mark.parametrize("T,H,I,E,K", [(300, 256, 1024, 1024, 16), (257, 72, 2060, 400, 9), (400, 512, 1032, 2500, 16), (333, 36, 4100, 100, 3)])
 def test_block_of_few_tokens_fp32_down_in_slices_of_k(T, H, I, E, K):
     """More than 256 tokens: 32 x 32 tiles whose k other workgroups share, beside gate/up tiles of 32 columns."""
