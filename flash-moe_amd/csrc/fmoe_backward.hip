@@ -653,9 +653,10 @@ __global__ __launch_bounds__(kBwdWaves* kWave) void expert_backward_weight_kerne
 // list order: the byte offset of its token's rows and its two coefficients.  A round is 16 pairs of each quarter, the next rounds' entries
 // and PIF pairs' pieces are requested ahead.  Sums run in ascending pair index here too: the gradients are the same bit for bit.
 // Bound by what the L2s deliver (1 KB chunks: a third of the lines missed at 4096 tokens).  Expert forward and backward, us, 1-KB chunks |
-// quarters, ids uniform and of a product-key router: 4096 tokens x 64 pairs, 16384 experts, 1024 columns 252 | 219 and 220 | 219; 16384 x
-// 64 1047 | 868 and 746 | 748; 8192 x 64, 65536 experts, 512 columns 417 | 380 and 367 | 355.  Where the chunks do fit, quarters only walk
-// the lists more often: 2048 x 32, 2048 columns 165 | 166 and 161 | 170.  8 pairs ahead instead of 4 leave three waves per SIMD: 226.
+// quarters, ids uniform and of a product-key router: 4096 tokens x 64 pairs, 16384 experts, 1024 columns 252 | 212 and 220 | 212; 16384 x
+// 64 1047 | 865 and 746 | 744; 8192 x 64, 65536 experts, 512 columns, router 367 | 352.  Where the chunks do fit, quarters only walk the
+// lists more often: 2048 x 32, 2048 columns 165 | 166 and 161 | 170.  8 pairs ahead instead of 4, or five waves per SIMD instead of four,
+// were slower (214 to 220), as were entries that every lane loads, for which no wait stands at the end of a round (214; 16384 tokens 891).
 __global__ __launch_bounds__(256) void pair_entries_kernel(const float2* __restrict__ coef, const uint32_t* __restrict__ pairs,
                                                           const int32_t* __restrict__ offsets, int64_t num_experts, uint32_t top_k,
                                                           uint32_t row_bytes, u32x4_t* __restrict__ entries) {
@@ -707,20 +708,26 @@ __global__ __launch_bounds__(kBwdWaves* kWave) void expert_backward_weight_quart
     }
     const int first_end = __shfl(ends, quarter);
     int cur = 0, cur_end = count > 0 ? first_end : -1;        // -1: every row of the quarter has left
-    auto flush = [&](int pos) {                               // rows of the experts whose segments end at list position `pos`
-        while (__builtin_amdgcn_ballot_w64(cur_end == pos) != 0ull) {
-            if (cur_end == pos) {
-                if (live) {
-                    reinterpret_cast<u32x4_t*>(ddown + (e0 + cur) * hidden)[packet] = pack16<T>(acc_d);
-                    reinterpret_cast<u32x4_t*>(dup + (e0 + cur) * hidden)[packet] = pack16<T>(acc_u);
-                }
-#pragma unroll
-                for (int v = 0; v < V; ++v) acc_d[v] = acc_u[v] = 0.0f;
-                ++cur;
+    // Rows of the experts whose segments end at list position `pos`.  The sums are cleared by a select, not under a branch of some lanes: with
+    // that the compiler kept a second copy of them at every position, 34 of 90 vector instructions.
+    auto flush = [&](int pos) {
+        bool ends_here = cur_end == pos;
+        if (__builtin_amdgcn_ballot_w64(ends_here) == 0ull) return;
+        do {
+            if (ends_here && live) {
+                reinterpret_cast<u32x4_t*>(ddown + (e0 + cur) * hidden)[packet] = pack16<T>(acc_d);
+                reinterpret_cast<u32x4_t*>(dup + (e0 + cur) * hidden)[packet] = pack16<T>(acc_u);
             }
+#pragma unroll
+            for (int v = 0; v < V; ++v) {
+                acc_d[v] = ends_here ? 0.0f : acc_d[v];
+                acc_u[v] = ends_here ? 0.0f : acc_u[v];
+            }
+            cur += ends_here ? 1 : 0;
             const int next = __shfl(ends, quarter + (cur < 15 ? cur : 15));
             cur_end = cur < count ? next : -1;
-        }
+            ends_here = cur_end == pos;
+        } while (__builtin_amdgcn_ballot_w64(ends_here) != 0ull);
     };
     flush(begin);
     auto round_at = [&](int r) {                              // entries past the quarter's list: nothing is fetched, zeros are added
