@@ -47,8 +47,9 @@ __device__ __forceinline__ void gemm_solo_tile(const T* __restrict__ A, const T*
     auto issue = [&](int kt, int r) {                                             // load r of 32 of k-tile kt
         const int c = r & 1 ? chunk ^ 4 : chunk;
         const uint32_t at = (uint32_t)((r & 15) * 8 + lrow) * row_bytes + (uint32_t)c * 16u;
+        // past the last k-tile the scalar offset is 0: with one row of A left it would pass the descriptor's end by itself
         __builtin_amdgcn_raw_ptr_buffer_load_lds(r < 16 ? ar : br, (__attribute__((address_space(3))) void*)(stage + r * 512), 16,
-                                                 (int)(kt * 64 + c * 8 < K ? at : kOutOfRange), kt * 128, 0, 0);
+                                                 (int)(kt * 64 + c * 8 < K ? at : kOutOfRange), kt < k_tiles ? kt * 128 : 0, 0, 0);
     };
     const int frow = lane & 15, fhalf = lane >> 4;
     const char* from = reinterpret_cast<const char*>(stage) + frow * 128;

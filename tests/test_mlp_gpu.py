@@ -160,10 +160,13 @@ def test_mlp_fp32_on_gate_up_tiles_of_32_columns(T, H, I):
 @pytest.mark.parametrize("T,H,I", [
     (4096, 1024, 1536), (2000, 1928, 1480), (3900, 1000, 1544), (1100, 2960, 1608), (3001, 1000, 2664),     # 24, 24, 25, 26 and 42 k-tiles
     (2000, 1928, 1472),                                                                                   # the last before them
+    (3969, 1000, 1536), (3969, 1000, 1544), (1025, 3080, 1736),    # one row in the last tiles: 24, 25 and 28 k-tiles
+    (3970, 1000, 1544),                                            # and two
 ])
 def test_mlp_down_on_tiles_whose_k_the_waves_divide(dtype, T, H, I):
     """128 x 128 tiles that one wave each multiplies a quarter of k of: whole ones and remainders in every extent, guard rows around the
     output, with a residual and without, and in place of it."""
+    assert ((T + 127) // 128) * ((H + 127) // 128) <= 256          # a compute unit to each of these tiles
     test_mlp_remainders_of_every_tile_shape(dtype, T, H, I)
     from flash_moe import _C
 
