@@ -211,7 +211,8 @@ struct BackwardProduct {
 int gemm_backward(const BackwardProduct& product, int dtype, void* workspace, size_t workspace_bytes, hipStream_t stream);
 // Scratch of gemm_backward for the sums of a sliced k range (0 when it needs none).
 size_t gemm_backward_workspace_bytes(int M, int N, int K, int segments, int dtype);
-// Several products that do not depend on each other (at most four share a launch); their pointers do not matter for the scratch.
+// Several products (at most four share a launch); their pointers do not matter for the scratch.  None reads another's result; one
+// whose result takes the place of what others read or write is formed after those before it, in a launch of its own like all of them.
 // keep: leave the sum of one product's slices to the caller, if it is cut.
 struct KeptPlanes {
     int product;

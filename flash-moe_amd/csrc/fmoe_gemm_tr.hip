@@ -389,6 +389,26 @@ bool addressable(const BackwardProduct& p, int dtype) {
     return packets && (double)p.K * p.ldb < most && (p.layout == kBlasTN ? (double)p.K * p.lda < most : 256.0 * p.lda < most);
 }
 
+// Whether a product's result lies on what another one reads or writes: a caller may ask for gradients in the place of tensors that only
+// earlier products need (dx in that of dy, a weight's gradient in that of the weight), which one launch would write while others read.
+bool in_place(const BackwardProduct* p, int count, int dtype) {
+    const int64_t elt = (int64_t)dtype_size(dtype);
+    struct Span { const char* at; int64_t bytes; };
+    auto rows = [&](const void* base, int64_t n, int64_t ld, int64_t cols) { return Span{(const char*)base, ((n - 1) * ld + cols) * elt}; };
+    for (int i = 0; i < count; ++i) {
+        const Span c = rows(p[i].C, p[i].M, p[i].N, p[i].N);
+        for (int j = 0; j < count; ++j) {
+            if (j == i) continue;
+            const BackwardProduct& q = p[j];
+            const Span other[4] = {q.layout == kBlasTN ? rows(q.A, q.K, q.lda, q.M) : rows(q.A, q.M, q.lda, (int64_t)q.K * q.segments),
+                                   rows(q.B0, q.K, q.ldb, q.N), rows(q.segments > 1 ? q.B1 : q.B0, q.K, q.ldb, q.N), rows(q.C, q.M, q.N, q.N)};
+            for (const Span& o : other)
+                if (c.at < o.at + o.bytes && o.at < c.at + c.bytes) return true;
+        }
+    }
+    return false;
+}
+
 template <typename T>
 void launch_group(const BackwardProduct* p, int count, const GroupPlan& plan, void* workspace, hipStream_t stream, KeptPlanes* keep) {
     const int xcds = chip_info().xcds, rows = kTileRows[plan.shape], cols = kTileCols[plan.shape];
@@ -503,6 +523,7 @@ int gemm_backward(const BackwardProduct* p, int count, int dtype, void* workspac
     const GroupPlan plan = plan_group_of(p, count, dtype);
     bool together = plan.shape >= 0 && group_planes_bytes(p, count, plan) <= workspace_bytes;
     for (int i = 0; i < count; ++i) together = together && addressable(p[i], dtype);
+    together = together && !in_place(p, count, dtype);
     if (together) {
         switch (dtype) {
             case FMOE_F32: launch_group<float>(p, count, plan, workspace, stream, keep); break;

@@ -378,6 +378,8 @@ int fmoe_swiglu_backward(const void* dc, const void* a, const void* b, int64_t r
  * cannot address (beyond 2 GB, or not whole 16-byte packets) are rocBLAS calls (loaded on first use; FMOE_ERR_LIBRARY if
  * unavailable).  When dup_w starts where dgate_w ends (one [2I,H] buffer) the two weight gradients
  * are formed as one product (faster; the sums may differ in the last bit from two products); separate buffers work as well.
+ * dx may be dy, and a weight's gradient that weight (in place); no other tensors may overlap.  In place the products are launched one
+ * after the other instead of together.
  * Workspace: fmoe_mlp_backward_workspace_bytes() is enough for either kind of call, fmoe_mlp_backward_saved_workspace_bytes() (half
  * of it: three [T,I] planes and what slices of k need) for one with saved_products. */
 size_t fmoe_mlp_backward_workspace_bytes(int64_t num_tokens, int hidden, int intermediate, int dtype);

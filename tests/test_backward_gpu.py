@@ -855,6 +855,41 @@ def test_mlp_backward_products_in_one_launch(dtype, T, H, I):
     test_mlp_backward_remainders_of_the_transposing_products(dtype, T, H, I)
 
 
+@pytest.mark.parametrize("stacked", [False, True])
+@pytest.mark.parametrize("dtype,T,H,I", [
+    (torch.bfloat16, 513, 264, 520), (torch.float16, 2600, 264, 264),        # products that would share a launch: whole; in slices of k
+    (torch.bfloat16, 129, 3080, 4104), (torch.float32, 383, 516, 1544),
+    (torch.bfloat16, 300, 2048, 11008),                                      # and products that would not
+])
+def test_mlp_backward_in_place(dtype, T, H, I, stacked):
+    """dx in the place of dy and each weight's gradient in that of the weight, which only products before them read."""
+    from flash_moe import _C
+    from flash_moe.ops.hip.flash_mlp import mlp_backward, mlp_forward_saving
+
+    g = gen(T + I)
+    x, dy = (torch.randn(T, H, generator=g).to(dtype).cuda() for _ in range(2))
+    both = (torch.randn(2, I, H, generator=g) * 0.05).to(dtype).cuda()
+    wg, wu = both if stacked else (both[0].clone(), both[1].clone())
+    wd = (torch.randn(H, I, generator=g) * 0.05).to(dtype).cuda()
+    saved = mlp_forward_saving(x, wg, wu, wd)[1]
+    want = mlp_backward(dy, x, wg, wu, wd, saved)
+    L, code, stream = _C.lib(), _C.dtype_code(dtype), _C.current_stream(x.device)
+    need = L.fmoe_mlp_backward_saved_workspace_bytes(T, H, I, code)
+    ws = torch.empty(need, device="cuda", dtype=torch.uint8)
+    others = [torch.empty_like(t) for t in (dy, wg, wu, wd)]
+    for places in ((0,), (1, 2), (3,), (0, 1, 2, 3)):                        # which of dx, dWg, dWu, dWd lie on dy and the weights
+        held = torch.stack((wg, wu)) if stacked else (wg.clone(), wu.clone())
+        tensors = [dy.clone(), held[0], held[1], wd.clone()]
+        out = [tensors[i] if i in places else others[i] for i in range(4)]
+        _C.check(L.fmoe_mlp_backward(_C.ptr(tensors[0]), _C.ptr(x), *map(_C.ptr, tensors[1:]), _C.ptr(saved), T, H, I, code, *map(_C.ptr, out),
+                                     _C.ptr(ws), need, stream), "in place")
+        for name, a, b in zip(("dx", "dgate", "dup", "ddown"), out, want):
+            # the same products, their sums cut differently: two roundings to the type apart at most; in fp32 two sums of up to n terms,
+            # each off by the random walk of n roundings of 2^-24
+            n = max(T, 2 * I)
+            assert rel_fro(a, b) < {torch.float32: 2 * n ** 0.5 * 2.0 ** -24, torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[dtype], (places, name)
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("T,H,E,K", [
     (3, 24, 40, 4), (256, 264, 900, 5), (257, 520, 300, 33), (2049, 136, 5000, 9),      # waves per token of the row schedule
