@@ -591,11 +591,13 @@ __global__ __launch_bounds__(kBwdWaves* kWave) void expert_backward_weight_kerne
     };
     clear();
 
+    // list positions are unsigned: a round may end past the 2^31 - 1 pairs that a call may have
     const int ends = offsets[e0 + (lane < count ? lane + 1 : count)];
-    const int begin = __builtin_amdgcn_readfirstlane(offsets[e0]), end = __builtin_amdgcn_readlane(ends, count - 1);
-    int cur = 0, cur_end = __builtin_amdgcn_readlane(ends, 0);
+    const uint32_t begin = (uint32_t)__builtin_amdgcn_readfirstlane(offsets[e0]), end = (uint32_t)__builtin_amdgcn_readlane(ends, count - 1);
+    int cur = 0;
+    uint32_t cur_end = (uint32_t)__builtin_amdgcn_readlane(ends, 0);
     // rows of the experts whose segments end at list position `pos`
-    auto flush = [&](int pos) {
+    auto flush = [&](uint32_t pos) {
         while (cur < count && cur_end == pos) {
 #pragma unroll
             for (int c = 0; c < NCH; ++c) {
@@ -606,12 +608,12 @@ __global__ __launch_bounds__(kBwdWaves* kWave) void expert_backward_weight_kerne
             }
             clear();
             ++cur;
-            cur_end = __builtin_amdgcn_readlane(ends, cur < count ? cur : count - 1);
+            cur_end = (uint32_t)__builtin_amdgcn_readlane(ends, cur < count ? cur : count - 1);
         }
     };
     flush(begin);
-    for (int done = begin; done < end; done += kWave) {
-        const int n = end - done < kWave ? end - done : kWave;
+    for (uint32_t done = begin; done < end; done += kWave) {
+        const int n = end - done < (uint32_t)kWave ? (int)(end - done) : kWave;
         const uint32_t mine = pairs[done + (lane < n ? lane : n - 1)];
         const uint32_t tok = mine / (uint32_t)top_k;
         const float2 both = coef[mine];
@@ -639,7 +641,7 @@ __global__ __launch_bounds__(kBwdWaves* kWave) void expert_backward_weight_kerne
                         axpy16<T>(sd, xq[u][c], acc_d[c]);
                         axpy16<T>(su, gq[u][c], acc_u[c]);
                     }
-                    flush(done + j + 1);
+                    flush(done + (uint32_t)j + 1u);
                 }
                 load(j + PIF, xq[u], gq[u]);
             }
@@ -657,11 +659,15 @@ __global__ __launch_bounds__(kBwdWaves* kWave) void expert_backward_weight_kerne
 // 64 1047 | 865 and 746 | 744; 8192 x 64, 65536 experts, 512 columns, router 367 | 352.  Where the chunks do fit, quarters only walk the
 // lists more often: 2048 x 32, 2048 columns 165 | 166 and 161 | 170.  8 pairs ahead instead of 4, or five waves per SIMD instead of four,
 // were slower (214 to 220), as were entries that every lane loads, for which no wait stands at the end of a round (214; 16384 tokens 891).
+// Unsigned: the last workgroup's threads may lie past the 2^31 - 1 pairs that a call may have.
+__host__ __device__ constexpr auto list_position(uint32_t block, uint32_t thread) { return block * 256u + thread; }
+static_assert(list_position(0x7fffffffu / 256u, 255u) > 0x7ffffffeu && list_position(0x7fffffffu / 256u, 255u) < 0xffffffffu, "the last list position");
+
 __global__ __launch_bounds__(256) void pair_entries_kernel(const float2* __restrict__ coef, const uint32_t* __restrict__ pairs,
                                                           const int32_t* __restrict__ offsets, int64_t num_experts, uint32_t top_k,
                                                           uint32_t row_bytes, u32x4_t* __restrict__ entries) {
-    const int at = (int)(blockIdx.x * 256u + threadIdx.x);
-    if (at >= offsets[num_experts]) return;
+    const uint32_t at = list_position(blockIdx.x, threadIdx.x);
+    if (at >= (uint32_t)offsets[num_experts]) return;
     const uint32_t pair = pairs[at];
     const float2 c = coef[pair];
     entries[at] = u32x4_t{pair / top_k * row_bytes, __float_as_uint(c.x), __float_as_uint(c.y), 0u};
@@ -698,19 +704,22 @@ __global__ __launch_bounds__(kBwdWaves* kWave) void expert_backward_weight_quart
 #pragma unroll
     for (int v = 0; v < V; ++v) acc_d[v] = acc_u[v] = 0.0f;
 
-    const int ends = count > 0 ? offsets[e0 + (ql < count ? ql + 1 : count)] : 0;      // lane ql of a quarter: of its ql-th expert
-    const int begin = count > 0 ? offsets[e0] : 0, end = count > 0 ? offsets[e0 + count] : 0;
-    int longest = 0;
+    // Positions count from the quarter's first pair, unsigned: the wave walks on to the end of its longest list.
+    const uint32_t begin = count > 0 ? (uint32_t)offsets[e0] : 0u, length = count > 0 ? (uint32_t)offsets[e0 + count] - begin : 0u;
+    const uint32_t ends = count > 0 ? (uint32_t)offsets[e0 + (ql < count ? ql + 1 : count)] - begin : 0u;      // lane ql of a quarter: of its ql-th expert
+    uint32_t longest = 0u;
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-        const int n = __builtin_amdgcn_readlane(end - begin, q * 16);
+        const uint32_t n = (uint32_t)__builtin_amdgcn_readlane((int)length, q * 16);
         longest = n > longest ? n : longest;
     }
-    const int first_end = __shfl(ends, quarter);
-    int cur = 0, cur_end = count > 0 ? first_end : -1;        // -1: every row of the quarter has left
-    // Rows of the experts whose segments end at list position `pos`.  The sums are cleared by a select, not under a branch of some lanes: with
+    constexpr uint32_t kNone = 0xffffffffu;                   // every row of the quarter has left
+    const uint32_t first_end = (uint32_t)__shfl((int)ends, quarter);
+    int cur = 0;
+    uint32_t cur_end = count > 0 ? first_end : kNone;
+    // Rows of the experts whose segments end at position `pos`.  The sums are cleared by a select, not under a branch of some lanes: with
     // that the compiler kept a second copy of them at every position, 34 of 90 vector instructions.
-    auto flush = [&](int pos) {
+    auto flush = [&](uint32_t pos) {
         bool ends_here = cur_end == pos;
         if (__builtin_amdgcn_ballot_w64(ends_here) == 0ull) return;
         do {
@@ -724,30 +733,30 @@ __global__ __launch_bounds__(kBwdWaves* kWave) void expert_backward_weight_quart
                 acc_u[v] = ends_here ? 0.0f : acc_u[v];
             }
             cur += ends_here ? 1 : 0;
-            const int next = __shfl(ends, quarter + (cur < 15 ? cur : 15));
-            cur_end = cur < count ? next : -1;
+            const uint32_t next = (uint32_t)__shfl((int)ends, quarter + (cur < 15 ? cur : 15));
+            cur_end = cur < count ? next : kNone;
             ends_here = cur_end == pos;
         } while (__builtin_amdgcn_ballot_w64(ends_here) != 0ull);
     };
-    flush(begin);
-    auto round_at = [&](int r) {                              // entries past the quarter's list: nothing is fetched, zeros are added
-        const int at = begin + r * 16 + ql;
-        return at < end ? entries[at] : u32x4_t{0x80000000u, 0u, 0u, 0u};
+    flush(0u);
+    auto round_at = [&](uint32_t first) {                     // entries past the quarter's list: nothing is fetched, zeros are added
+        const uint32_t at = first + (uint32_t)ql;
+        return at < length ? entries[begin + at] : u32x4_t{0x80000000u, 0u, 0u, 0u};
     };
-    u32x4_t now = round_at(0), next = round_at(1), xq[PIF], gq[PIF];
+    u32x4_t now = round_at(0u), next = round_at(16u), xq[PIF], gq[PIF];
     auto load = [&](auto j, const u32x4_t& of, u32x4_t& xv, u32x4_t& gv) {
         const int at = (int)(row_lane<decltype(j)::value>(of[0]) + column);
         xv = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(xr, at, 0, 0));
         gv = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(gr, at, 0, 0));
     };
     static_for<PIF>([&](auto j) { load(j, now, xq[j], gq[j]); });
-    for (int r = 0; r * 16 < longest; ++r) {
-        const u32x4_t after = round_at(r + 2);
+    for (uint32_t done = 0u; done < longest; done += 16u) {
+        const u32x4_t after = round_at(done + 32u);
         static_for<16>([&](auto j) {
             constexpr int J = decltype(j)::value, S = J % PIF;
             axpy16<T>(__uint_as_float(row_lane<J>(now[2])), xq[S], acc_d);
             axpy16<T>(__uint_as_float(row_lane<J>(now[1])), gq[S], acc_u);
-            flush(begin + r * 16 + J + 1);
+            flush(done + (uint32_t)J + 1u);
             load(std::integral_constant<int, (J + PIF) % 16>{}, J + PIF < 16 ? now : next, xq[S], gq[S]);
         });
         now = next;
