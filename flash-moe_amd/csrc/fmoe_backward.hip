@@ -659,6 +659,8 @@ __global__ __launch_bounds__(kBwdWaves* kWave) void expert_backward_weight_kerne
 // 64 1047 | 865 and 746 | 744; 8192 x 64, 65536 experts, 512 columns, router 367 | 352.  Where the chunks do fit, quarters only walk the
 // lists more often: 2048 x 32, 2048 columns 165 | 166 and 161 | 170.  8 pairs ahead instead of 4, or five waves per SIMD instead of four,
 // were slower (214 to 220), as were entries that every lane loads, for which no wait stands at the end of a round (214; 16384 tokens 891).
+// One expert that every token names, 4096 tokens x 8 of 8192: 690 | 491, its list a chain of additions for either.  Which calls take them:
+// quarter_waves.
 // Unsigned: the last workgroup's threads may lie past the 2^31 - 1 pairs that a call may have.
 __host__ __device__ constexpr auto list_position(uint32_t block, uint32_t thread) { return block * 256u + thread; }
 static_assert(list_position(0x7fffffffu / 256u, 255u) > 0x7ffffffeu && list_position(0x7fffffffu / 256u, 255u) < 0xffffffffu, "the last list position");
@@ -766,10 +768,23 @@ __global__ __launch_bounds__(kBwdWaves* kWave) void expert_backward_weight_quart
 
 struct ExpertBwdPlan {
     bool slices, ordered;      // slices: column slices of the tables, on ordered lists or not
-    bool quarters;             // weight gradients by quarter waves: chunks of 1 KB of x and dout exceed an L2
+    bool quarters;             // weight gradients by quarter waves
     int num_slices;
     size_t off_coef, off_entries, off_pairs, off_group, off_offsets, off_off32, off_place, off_coef_list, off_spart_s, off_spart_u, bytes;
 };
+
+// Weight gradients by quarter waves: 1-KB chunks of x and dout exceed an L2, and what that saves is more than the entries' launch and the
+// shorter reads cost.  Expert backward, us, whole waves | quarters, over 425 sizes (2100 to 20000 tokens, 64 to 524288 experts, 4 to 64 per
+// token; the rule is 0.3 % behind the better of the two on average, quarters everywhere 2.7 %, nowhere 7.2 %):
+//   64 pairs to an expert and more, few waves that walk long lists: 3000 tokens x 32, 512 experts, 1024 columns 102 | 94; 64 experts 334 | 254;
+//   rows of 256 bytes and less, of which a whole wave has idle lanes: 20000 x 16 of 4096, 64 columns 97 | 81;
+//   else where the chunks exceed an L2 by two fifths (2868 tokens of 1 KB), for 48 K pairs and one and a half to an expert: 16384 x 16 of 16384,
+//   1024 columns 317 | 268.  Below them: 2100 x 32 of 8192, 512 columns 66 | 69; x 4 25 | 31; 16384 x 16 of 262144, 1024 columns 565 | 630.
+inline bool quarter_waves(int64_t tokens, int64_t row, int64_t experts, int64_t pairs) {
+    const int64_t chunks = 2 * tokens * (row < 1024 ? row : 1024), l2 = chip_info().l2_bytes;
+    if (pairs == 0 || chunks <= l2 || tokens * row >= (1ll << 31)) return false;
+    return pairs / 64 >= experts || row <= 256 || (5 * chunks >= 7 * l2 && pairs >= 3 << 14 && 2 * pairs >= 3 * experts);
+}
 
 ExpertBwdPlan plan_expert_backward(int64_t T_, int H, int64_t E, int K, int dtype) {
     ExpertBwdPlan p;
@@ -778,8 +793,7 @@ ExpertBwdPlan plan_expert_backward(int64_t T_, int H, int64_t E, int K, int dtyp
     auto take = [&](size_t n) { const size_t at = o; o = round_up(o + n, 256); return at; };
     p.off_coef = take(pairs * 8);
     p.off_coef_list = take(pairs * 4);
-    const int64_t row = (int64_t)H * (int64_t)dtype_size(dtype);
-    p.quarters = pairs > 0 && 2 * T_ * (row < 1024 ? row : 1024) > chip_info().l2_bytes && T_ * row < (1ll << 31);
+    p.quarters = quarter_waves(T_, (int64_t)H * (int64_t)dtype_size(dtype), E, (int64_t)pairs);
     p.off_entries = take(p.quarters ? pairs * 16 : 0);
     p.off_pairs = take(pairs * 4);
     p.off_group = take(group_pairs_workspace_bytes((int64_t)pairs, E));

@@ -263,6 +263,22 @@ def test_expert_schedule_at_the_lines_of_its_rule(T, H, E, K, dtype, schedule):
     assert (lib.fmoe_expert_saved_bytes(T, H, E, K, code) > 0) == (schedule in ("SLICES", "ORDERED"))
 
 
+@pytest.mark.parametrize("quarters,whole,dtype", [
+    ((4096, 512, 256, 4), (4096, 512, 257, 4), "BF16"),                # 64 pairs to an expert
+    ((20000, 128, 5000, 2), (20000, 136, 5000, 2), "BF16"), ((20000, 64, 5000, 2), (20000, 68, 5000, 2), "F32"),      # rows of 256 bytes
+    ((2868, 512, 1024, 18), (2867, 512, 1024, 18), "F16"),             # chunks of x and dout that exceed an L2 by two fifths
+    ((2868, 4096, 2048, 18), (2867, 4096, 2048, 18), "BF16"),          # ... of which longer rows have more
+    ((4096, 512, 8192, 12), (4095, 512, 8192, 12), "BF16"),            # 48 K pairs
+    ((4096, 1024, 43690, 16), (4096, 1024, 43691, 16), "BF16"),        # one and a half to an expert
+])
+def test_expert_weight_gradients_by_quarter_waves_at_the_lines_of_their_rule(quarters, whole, dtype):
+    """Their entries are 16 bytes of scratch to a pair."""
+    lib, code = _C.lib(), getattr(_C, dtype)
+    more, less = (lib.fmoe_expert_backward_workspace_bytes(*c, code) for c in (quarters, whole))
+    pairs = quarters[0] * quarters[3]
+    assert 15 * pairs < more - less < 17 * pairs
+
+
 def test_expert_workspace_is_enough_for_both_forwards():
     """The forward alone and that of a training step: one size for both."""
     lib = _C.lib()

@@ -754,6 +754,23 @@ def test_expert_backward_with_skewed_routing_is_exact_and_quick():
     elapsed = time.perf_counter() - t0
     assert all(torch.equal(a, b) for a, b in zip(got, again))
     assert elapsed < 0.05, f"{elapsed * 1e3:.1f} ms for a backward with one 8192-pair segment"
+    # and against the same call on ids without such an expert: what it adds is its chain of 8192 additions, about 120 ns each in either
+    # kernel of the weight gradients (twice that allowed)
+    uniform = args[:4] + (torch.stack([torch.randperm(E - 1, generator=g)[:K] + 1 for _ in range(T)]).cuda(),) + args[5:]
+
+    def call_us(call):
+        times = []
+        for _ in range(7):
+            a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            a.record()
+            expert_backward(*call)
+            b.record()
+            b.synchronize()
+            times.append(a.elapsed_time(b) * 1e3)
+        return sorted(times)[3]
+
+    skewed, even = call_us(args), call_us(uniform)
+    assert skewed - even < 2 * 0.12 * T, f"{skewed:.0f} us with a segment of {T} pairs, {even:.0f} without"
     # the hot expert's rows against float64: ddown[0] = sum_t ds_t x_t, dup[0] = sum_t silu(s_t) g_t dout_t
     x64, wd64, wu64, g64, do64 = (t.double() for t in (x, wd, wu, gates, dout))
     s = x64 @ wd64[0]
@@ -921,6 +938,8 @@ def test_expert_backward_edges_of_the_waves_and_spans(dtype, T, H, E, K):
     (4100, 136, 900, 9, 0), (2060, 520, 20000, 7, 0),  # rows below 1 KB; experts without pairs, several spans to a quarter
     (2050, 1544, 333, 3, 0),                           # the last chunk partial, spans of one
     (4099, 520, 3, 2, 0), (2200, 1032, 50, 5, 47),     # fewer experts than quarters; lists of very different lengths
+    (4100, 264, 900, 13, 0), (3000, 520, 33000, 17, 0), (3001, 1544, 333, 17, 0),      # the first three with the pairs that they take
+    (20001, 40, 5000, 3, 0),                           # rows shorter than a quarter's chunk
 ])
 def test_expert_weight_gradients_by_quarter_waves(dtype, T, H, E, K, first):
     """Chunks of x and dout beyond an L2, with ids out of range among the pairs (they count for nothing)."""
