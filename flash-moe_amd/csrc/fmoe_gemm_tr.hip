@@ -302,6 +302,10 @@ int plan_gradient(int M, int N, int K) {
 // 16384, best on 128 x 128 tiles from about 4000 tokens on: 4096 tokens, 1024 -> 4096 1258 us one by one, 1238 on 64 x 64, 1176; 5000, 2048
 // -> 5464 4392, 4291, 4176).  64 x 128 tiles would gain half a percent.  Products over tokens (the weight gradients)
 // are sliced from 2048 tokens on.
+// A group must be cheaper than its products one by one, whose price is plan_turned's and a launch of 4 us for each but the first (fp32,
+// whose prices fit less well: a fifth more, and 4 us each).  Few tiles over many tokens are not: alone, a product may be cut into 16 slices.
+// Where groups were formed at any price, 32768 tokens, 256 columns, 24 keys, us: two launches 76, one 125, fp32 114 and 214; MLP, 65536
+// tokens, 128 -> 344 171 and 247.  Of 316 such calls (256 to 65536 tokens) the choice is 0.1 % behind the better way on average, 8 % at most.
 // 16-bit, beyond four rounds of 256 x 256 tiles: each product fills the chip and its persistent workgroups start a tile's loads under the last
 // one's stores: 2048 tokens, 4096 -> 16384 1057 us one by one, 1087 together; 6000 tokens, 1800 -> 7200, three and a half rounds, 734 and 731.
 template <typename T> GroupPlan plan_group(const BackwardProduct* p, int count) {
@@ -320,7 +324,12 @@ template <typename T> GroupPlan plan_group(const BackwardProduct* p, int count) 
     constexpr double kFull[3] = {1.5, kSingle ? 1.75 : 0.47, kSingle ? 0.475 : 0.225}, kAlone[3] = {1.3, kSingle ? 2.2 : 0.75, kSingle ? 0.6 : 0.3};
     constexpr double kStores[3] = {6.0, kSingle ? 2.0 : 0.65, kSingle ? 0.2 : 0.1}, kRounds[3] = {0.5, kSingle ? 1.0 : 0.4, kSingle ? 0.5 : 0.4};
     constexpr int kOver[6] = {1, 2, 3, 4, 6, 8}, kTokens[3] = {1, 2, 4};
-    double best_time = 0.0;
+    double best_time = kSingle ? 4.0 * count : 4.0 * (count - 1);          // one by one
+    for (int i = 0; i < count; ++i) {
+        double alone = 0.0;
+        plan_turned<T>(p[i].M, p[i].N, p[i].K, p[i].segments, &alone);
+        best_time += (kSingle ? 1.2 : 1.0) * alone;
+    }
     for (int z = kSingle ? 1 : 0; z < 3; ++z) {
         const int shape = kShapes[z];
         int64_t tiles[kGroupMost];
@@ -356,11 +365,11 @@ template <typename T> GroupPlan plan_group(const BackwardProduct* p, int count) 
                         if (share * kAlone[z] > longest) longest = share * kAlone[z];
                         if (s > 1) planes += 4.0 + 8.0e-6 * s * (double)p[i].M * p[i].N / 6.0;
                     }
-                    if (!usable || (best.shape >= 0 && (work > longest ? work : longest) + planes >= best_time)) continue;
+                    if (!usable || (work > longest ? work : longest) + planes >= best_time) continue;
                     for (int i = 0; i < count; ++i) t[i] *= kPer[z];
                     const double mixed = kRounds[z] * time_of_items(n, t, count, kPer[z] * cus) + (1.0 - kRounds[z]) * work;
                     const double time = (mixed > longest ? mixed : longest) + planes;
-                    if (best.shape < 0 || time < best_time) {
+                    if (time < best_time) {
                         best = g;
                         best_time = time;
                     }

@@ -279,6 +279,16 @@ def test_expert_weight_gradients_by_quarter_waves_at_the_lines_of_their_rule(qua
     assert 15 * pairs < more - less < 17 * pairs
 
 
+@pytest.mark.parametrize("T,H,nk,dtype,slices", [(32768, 256, 24, "BF16", 16), (32768, 256, 24, "F32", 16), (8192, 512, 64, "BF16", 12), (4096, 256, 24, "F32", 8)])
+def test_backward_products_of_few_tiles_over_many_tokens_are_cut_as_if_alone(T, H, nk, dtype, slices):
+    """A launch shared with another product leaves a weight gradient at most four slices of the tokens, fp32 sums of [2 nk, H] each."""
+    lib, code, elt = _C.lib(), getattr(_C, dtype), 4 if dtype == "F32" else 2
+    operands = T * elt * (2 * nk + 2 * H)
+    assert lib.fmoe_router_prologue_backward_workspace_bytes(T, H, nk, code) >= operands + slices * 2 * nk * H * 4
+    # and one that takes the shared launch keeps to them
+    assert lib.fmoe_router_prologue_backward_workspace_bytes(2048, 1024, 128, code) < 2048 * elt * (2 * 128 + 2 * 1024) + 5 * 2 * 128 * 1024 * 4
+
+
 def test_expert_workspace_is_enough_for_both_forwards():
     """The forward alone and that of a training step: one size for both."""
     lib = _C.lib()
