@@ -596,8 +596,7 @@ __global__ __launch_bounds__(256) void prologue_bwd_prepare_kernel(const float* 
     }
 }
 
-// partial: [row_blocks][2][H] = (sum dq, sum dq * xhat) over the block's rows; geometry of bn_block_stats_kernel: at most
-// kFoldMaxRowBlocks tall blocks, so that the next launch adds them itself.
+// partial: [row_blocks][2][H] = (sum dq, sum dq * xhat) over the block's rows; strips of bn_block_stats_kernel.
 template <typename T>
 __global__ __launch_bounds__(kStatsThreads) void bn_bwd_partial_kernel(const T* __restrict__ x, const T* __restrict__ dq,
                                                                       const float* __restrict__ mean_rstd, int64_t num_tokens,
@@ -674,9 +673,39 @@ __global__ __launch_bounds__(kStatsThreads) void bn_bwd_partial_kernel(const T* 
     }
 }
 
+// The row blocks' column sums added, 32 columns to a workgroup, eight threads to a column: [2][H] after the row blocks.
+__global__ __launch_bounds__(256) void bn_bwd_fold_kernel(const float* __restrict__ partial, int row_blocks, int hidden, float* __restrict__ sums) {
+    __shared__ float red[8][32];
+    const int c = (int)(blockIdx.x * 32 + (threadIdx.x & 31)), group = (int)(threadIdx.x >> 5);
+    const bool col_ok = c < 2 * hidden;
+    float acc[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) acc[u] = 0.0f;
+    for (int b0 = group; b0 < row_blocks; b0 += 64) {
+        float got[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            const int b = b0 + 8 * u < row_blocks ? b0 + 8 * u : row_blocks - 1;      // clamped: every load is unconditional
+            got[u] = partial[(int64_t)b * 2 * hidden + (col_ok ? c : 0)];
+        }
+#pragma unroll
+        for (int u = 0; u < 8; ++u) acc[u] += b0 + 8 * u < row_blocks ? got[u] : 0.0f;
+    }
+    float a = 0.0f;
+#pragma unroll
+    for (int u = 0; u < 8; ++u) a += acc[u];
+    red[group][threadIdx.x & 31] = a;
+    __syncthreads();
+    if (group != 0 || !col_ok) return;
+#pragma unroll
+    for (int g = 1; g < 8; ++g) a += red[g][threadIdx.x];
+    sums[c] = a;
+}
+
 // dx, and the block's other token gradients added in fp32: addend0 and addend1 (either may be NULL, or dx itself: a thread reads its
 // packet before it writes), and fp32 planes of slices of k (of the MLP's dx, whose sum nobody else needs).
-// A workgroup takes a strip of 64 packets and rows_per_block rows, its waves rows 4 apart.  training: it first adds the blocks'
+// A workgroup takes a strip of 2^lane_bits packets (64, or what a shorter row has) and rows_per_block rows, its waves 64 lanes of them, the
+// four steps apart.  training: it first adds the blocks'
 // column sums to the two means of the formula, a quarter of the blocks to a wave.  Where a launch of its own had formed the means: 4096
 // tokens, 1024 columns 22.8 us in three launches, 18.7 in two; 615 tokens, 776 columns, with four planes that another launch had
 // added, 17.6 in four and 10.7 in two.
@@ -685,11 +714,12 @@ __global__ __launch_bounds__(256) void bn_bwd_apply_kernel(const T* __restrict__
                                                            const float* __restrict__ mean_rstd, const float* __restrict__ partial,
                                                            int row_blocks, float inv_tokens, const T* addend0, const T* addend1,
                                                            const float* __restrict__ planes, int slices, T* dx, int64_t num_tokens,
-                                                           int hidden, int rows_per_block) {
+                                                           int hidden, int rows_per_block, int lane_bits) {
     constexpr int V = Elem<T>::kVec, kShare = kFoldMaxRowBlocks / 4;
     __shared__ __attribute__((aligned(16))) float shared_sums[4][2][kWave * V];
     const int lane = lane_id(), wave = (int)(threadIdx.x >> 6);
-    const int col = ((int)blockIdx.y * kWave + lane) * V;
+    const int wave_rows = kWave >> lane_bits, step = 4 * wave_rows;
+    const int col = ((int)blockIdx.y * kWave + (lane & ((1 << lane_bits) - 1))) * V;
     const bool col_ok = col < hidden;
     const int at_col = col_ok ? col : 0;
     // a wave's next row is asked for before the current one is worked on, the first before the means
@@ -702,7 +732,8 @@ __global__ __launch_bounds__(256) void bn_bwd_apply_kernel(const T* __restrict__
 #pragma unroll
         for (int i = 0; i < 4; ++i) raw[i] = *reinterpret_cast<const u32x4_t*>(rows[i] + at);
     };
-    load(r0 + wave);
+    const int64_t first = r0 + wave * wave_rows + (lane >> lane_bits);
+    load(first);
     float mean[V], rstd[V], m1[V], m2[V];
 #pragma unroll
     for (int v = 0; v < V; v += 4) {
@@ -757,14 +788,14 @@ __global__ __launch_bounds__(256) void bn_bwd_apply_kernel(const T* __restrict__
         }
     }
     if (!col_ok) return;
-    for (int64_t r = r0 + wave; r < r1; r += 4) {
+    for (int64_t r = first; r < r1; r += step) {
         const int64_t at = r * hidden + col;
         float xv[V], gv[V], ov[V], more[2][V];
         unpack16<T>(raw[0], xv);
         unpack16<T>(raw[1], gv);
         unpack16<T>(raw[2], more[0]);
         unpack16<T>(raw[3], more[1]);
-        if (r + 4 < r1) load(r + 4);             // never this row, which may be written in place
+        if (r + step < r1) load(r + step);             // never this row, which may be written in place
 #pragma unroll
         for (int v = 0; v < V; ++v) ov[v] = rstd[v] * (gv[v] - m1[v] - (xv[v] - mean[v]) * rstd[v] * m2[v]);
         if (planes != nullptr) {
@@ -790,7 +821,22 @@ __global__ __launch_bounds__(256) void bn_bwd_apply_kernel(const T* __restrict__
     }
 }
 
+// Row blocks of the batch-norm gradient's column sums.  Up to kFoldMaxRowBlocks of them the last launch adds itself; where few strips leave
+// compute units idle so, as many as fill the chip, if their rows are fewer by what a launch that adds them takes (250; 1000 where there is
+// a workgroup for every other compute unit already).
+struct ColumnSumsPlan { int row_blocks, rows_per_block; bool folded; };
+ColumnSumsPlan plan_column_sums(int64_t T_, int H, int vec) {
+    const BlockStatsPlan few = plan_block_stats(T_);
+    const int64_t strips = (H + 8 * vec - 1) / (8 * vec), wanted = 2 * chip_info().cus / strips, most = (T_ + 127) / 128;
+    int64_t rb = wanted < most ? wanted : most;
+    if (rb > kMaxRowBlocks) rb = kMaxRowBlocks;
+    const int rows = rb > kFoldMaxRowBlocks ? (int)((T_ + rb - 1) / rb) : few.rows_per_block;
+    if (few.rows_per_block - rows < (strips * kFoldMaxRowBlocks <= chip_info().cus / 2 ? 250 : 1000)) return {few.row_blocks, few.rows_per_block, false};
+    return {(int)((T_ + rows - 1) / rows), rows, true};
+}
+
 struct PrologueBwdPlan {
+    ColumnSumsPlan sums;
     int n_pad;            // row length of d in the activation dtype: 2 * nk rounded up to whole packets
     size_t off_d16, off_q, off_dq, off_partial, off_part, part_bytes, bytes;
 };
@@ -811,7 +857,8 @@ PrologueBwdPlan plan_prologue_backward(int64_t T_, int H, int nk, int dtype) {
     p.off_d16 = take((size_t)T_ * p.n_pad * elt);
     p.off_q = take((size_t)T_ * H * elt);
     p.off_dq = take((size_t)T_ * H * elt);
-    p.off_partial = take((size_t)kFoldMaxRowBlocks * 2 * H * 4);
+    p.sums = plan_column_sums(T_, H, vec);
+    p.off_partial = take((size_t)(p.sums.row_blocks + 1) * 2 * H * 4);
     BackwardProduct products[2];
     prologue_products(t, H, 2 * nk, p.n_pad, products);
     p.part_bytes = gemm_backward_workspace_bytes(products, 2, dtype);
@@ -826,7 +873,6 @@ int launch_prologue_backward(const float* dlogits, const void* x, const void* ga
                              hipStream_t s, bool operands_ready) {
     constexpr int V = Elem<T>::kVec;
     const PrologueBwdPlan p = plan_prologue_backward(T_, H, nk, dtype);
-    const BlockStatsPlan rows = plan_block_stats(T_);
     char* ws = (char*)workspace;
     T *d16 = (T*)(ws + p.off_d16), *q = (T*)(ws + p.off_q), *dq = (T*)(ws + p.off_dq);
     float* partial = (float*)(ws + p.off_partial);
@@ -847,16 +893,27 @@ int launch_prologue_backward(const float* dlogits, const void* x, const void* ga
     if (int rc = gemm_backward(products, 2, dtype, part, p.part_bytes, s)) return rc;
     if (training) {
         const int strips = (H + 8 * V - 1) / (8 * V);
-        hipLaunchKernelGGL((bn_bwd_partial_kernel<T>), dim3((unsigned)rows.row_blocks, (unsigned)strips), dim3(kStatsThreads), 0, s,
-                           (const T*)x, (const T*)dq, mean_rstd, T_, H, rows.rows_per_block, partial);
+        hipLaunchKernelGGL((bn_bwd_partial_kernel<T>), dim3((unsigned)p.sums.row_blocks, (unsigned)strips), dim3(kStatsThreads), 0, s,
+                           (const T*)x, (const T*)dq, mean_rstd, T_, H, p.sums.rows_per_block, partial);
         FMOE_CHECK_LAUNCH("fmoe_router_prologue_backward(column sums)");
     }
-    // about two workgroups to a compute unit, rows in fours
-    const int64_t strips = (H + kWave * V - 1) / (kWave * V), wanted = 2 * chip_info().cus / strips + 1;
-    const int apply_rows = (int)((T_ + wanted * 4 - 1) / (wanted * 4) * 4);
+    int row_blocks = p.sums.row_blocks;
+    if (training && p.sums.folded) {
+        float* sums = partial + (size_t)row_blocks * 2 * H;
+        hipLaunchKernelGGL(bn_bwd_fold_kernel, dim3((unsigned)((2 * H + 31) / 32)), dim3(256), 0, s, (const float*)partial, row_blocks, H, sums);
+        FMOE_CHECK_LAUNCH("fmoe_router_prologue_backward(row blocks)");
+        partial = sums;
+        row_blocks = 1;
+    }
+    // about two workgroups to a compute unit
+    const int packets = H / V;
+    int lane_bits = 6;
+    while (lane_bits > 0 && packets <= 1 << (lane_bits - 1)) --lane_bits;
+    const int64_t strips = (packets + kWave - 1) / kWave, wanted = 2 * chip_info().cus / strips + 1, step = 4 * (kWave >> lane_bits);
+    const int apply_rows = (int)((T_ + wanted * step - 1) / (wanted * step) * step);
     hipLaunchKernelGGL((bn_bwd_apply_kernel<T>), dim3((unsigned)((T_ + apply_rows - 1) / apply_rows), (unsigned)strips), dim3(256), 0, s, (const T*)x,
-                       (const T*)dq, mean_rstd, training ? (const float*)partial : nullptr, rows.row_blocks, 1.0f / (float)T_, (const T*)more.addend0,
-                       (const T*)more.addend1, more.planes, more.slices, (T*)dx, T_, H, apply_rows);
+                       (const T*)dq, mean_rstd, training ? (const float*)partial : nullptr, row_blocks, 1.0f / (float)T_, (const T*)more.addend0,
+                       (const T*)more.addend1, more.planes, more.slices, (T*)dx, T_, H, apply_rows, lane_bits);
     FMOE_CHECK_LAUNCH("fmoe_router_prologue_backward(apply)");
     return FMOE_OK;
 }
