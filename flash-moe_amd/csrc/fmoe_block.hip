@@ -67,6 +67,8 @@ SavedPlan plan_saved(int64_t T_, int H, int I, int nk, int64_t E, int K, int dty
 
 struct BlockBackwardPlan {
     size_t off_dgates, off_dlogits32, off_dx_experts, off_planes, off_stage, stage_bytes, bytes;
+    MlpBackwardPlan mlp;
+    PrologueBackwardPlan prologue;
 };
 
 // The stages run one after the other on one stream, so they share one scratch area, but for the MLP's slices of k: the last stage adds
@@ -79,13 +81,13 @@ BlockBackwardPlan plan_block_backward(int64_t T_, int H, int I, int nk, int64_t 
     p.off_dgates = take((size_t)T_ * K * elt);
     p.off_dlogits32 = take((size_t)T_ * 2 * nk * 4);
     p.off_dx_experts = take((size_t)T_ * H * elt);
-    const MlpBackwardBytes mlp = mlp_backward_bytes(T_, H, I, dtype);
-    p.off_planes = take(mlp.planes > 0 ? mlp.planes : 256);
-    p.stage_bytes = mlp.workspace;
+    p.mlp = plan_mlp_backward(T_, H, I, dtype, true);
+    p.prologue = plan_prologue_backward(T_, H, nk, dtype);
+    p.off_planes = take(p.mlp.part_bytes > 0 ? p.mlp.part_bytes : 256);
+    p.stage_bytes = p.mlp.off_part;
     const size_t experts = fmoe_expert_backward_workspace_bytes(T_, H, E, K, dtype);
-    const size_t prologue = fmoe_router_prologue_backward_workspace_bytes(T_, H, nk, dtype);
     if (experts > p.stage_bytes) p.stage_bytes = experts;
-    if (prologue > p.stage_bytes) p.stage_bytes = prologue;
+    if (p.prologue.bytes > p.stage_bytes) p.stage_bytes = p.prologue.bytes;
     p.off_stage = take(p.stage_bytes);
     p.bytes = o;
     return p;
@@ -285,19 +287,19 @@ extern "C" int fmoe_block_backward(const void* dout, const void* dlogits, const 
     float* dlogits32 = (float*)(ws + p.off_dlogits32);
     KeptPlanes kept = {};
     int rc = mlp_backward_impl(dout, x, gate_proj_w, up_proj_w, down_proj_w, sv + sp.off_products, num_tokens, hidden, intermediate, dtype, dx,
-                               dgate_proj_w, dup_proj_w, ddown_proj_w, stage, p.stage_bytes, ws + p.off_planes, &kept, (hipStream_t)stream);
+                               dgate_proj_w, dup_proj_w, ddown_proj_w, p.mlp, stage, p.stage_bytes, ws + p.off_planes, &kept, (hipStream_t)stream);
     if (rc) return rc;
     rc = fmoe_expert_backward_saved(dout, x, down_embed, up_embed, indices, sv + sp.off_gates, sv + sp.off_experts, num_tokens, hidden,
                                     num_experts, top_k, dtype, dx_experts, ddown_embed, dup_embed, dgates, stage, p.stage_bytes, stream);
     if (rc) return rc;
     const float* mean_rstd = (const float*)(sv + sp.off_stats);
     const bool prepares = route_backward_prepares(num_keys, top_k);
-    const PrologueOperands operands = prologue_operands(x, mean_rstd, num_tokens, hidden, num_keys, dtype, stage);
+    const PrologueOperands operands = prologue_operands(x, mean_rstd, hidden, p.prologue, stage);
     rc = route_backward_impl(dgates, indices, logits32, dlogits, num_keys, num_tokens * num_keys, num_tokens, num_keys, top_k, dtype,
                              norm_topk_prob, dlogits32, (hipStream_t)stream, prepares ? &operands : nullptr);
     if (rc) return rc;
     // the three token gradients are summed where the last of them is formed
     return router_prologue_backward_impl(dlogits32, x, router_gate_w, mean_rstd, training, num_tokens, hidden,
-                                         num_keys, dtype, dx, drouter_gate_w, {kept.planes ? nullptr : dx, dx_experts, kept.planes, kept.slices}, stage,
-                                         p.stage_bytes, (hipStream_t)stream, prepares);
+                                         num_keys, dtype, dx, drouter_gate_w, {kept.planes ? nullptr : dx, dx_experts, kept.planes, kept.slices}, p.prologue,
+                                         stage, p.stage_bytes, (hipStream_t)stream, prepares);
 }

@@ -100,7 +100,8 @@ struct PrologueOperands {
     const void* x;
     const float* mean_rstd;
 };
-PrologueOperands prologue_operands(const void* x, const float* mean_rstd, int64_t num_tokens, int hidden, int num_keys, int dtype, void* workspace);
+struct PrologueBackwardPlan;
+PrologueOperands prologue_operands(const void* x, const float* mean_rstd, int hidden, const PrologueBackwardPlan& plan, void* workspace);
 // Arguments of fmoe_router_prologue_backward; operands_ready: prologue_operands of this workspace are in place and stand for dlogits_fp32;
 // more: token gradients that are added to dx in fp32 before it is rounded, any of them NULL: two tensors [T,H], each of which may be
 // dx itself, and fp32 planes [slices][T,H].
@@ -112,7 +113,7 @@ struct TokenGradients {
 };
 int router_prologue_backward_impl(const float* dlogits_fp32, const void* x, const void* gate_w, const float* mean_rstd,
                                   int training, int64_t num_tokens, int hidden, int num_keys, int dtype, void* dx,
-                                  void* dgate_w, const TokenGradients& more, void* workspace, size_t workspace_bytes,
+                                  void* dgate_w, const TokenGradients& more, const PrologueBackwardPlan& plan, void* workspace, size_t workspace_bytes,
                                   hipStream_t stream, bool operands_ready = false);
 
 // (router_forward_impl: mean_rstd_out [2][H], when given, receives mean and 1/std instead of the workspace.)
@@ -211,29 +212,52 @@ struct BackwardProduct {
 int gemm_backward(const BackwardProduct& product, int dtype, void* workspace, size_t workspace_bytes, hipStream_t stream);
 // Scratch of gemm_backward for the sums of a sliced k range (0 when it needs none).
 size_t gemm_backward_workspace_bytes(int M, int N, int K, int segments, int dtype);
-// Several products (at most four share a launch); their pointers do not matter for the scratch.  None reads another's result; one
+// Several products (at most four share a launch); their pointers do not matter for the plan and the scratch.  None reads another's result; one
 // whose result takes the place of what others read or write is formed after those before it, in a launch of its own like all of them.
 // keep: leave the sum of one product's slices to the caller, if it is cut.
+// The plan is a search of 1 to 4 us on the host, so callers make it once for their size and their launches.
+constexpr int kGroupMost = 4;
+struct GroupPlan {
+    int shape;                    // of every tile; -1: one product after the other
+    int slices[kGroupMost];       // of k, of each product
+};
+GroupPlan plan_products(const BackwardProduct* products, int count, int dtype);
 struct KeptPlanes {
     int product;
     const float* planes;          // NULL: the product is where it belongs
     int slices;
 };
-int gemm_backward(const BackwardProduct* products, int count, int dtype, void* workspace, size_t workspace_bytes, hipStream_t stream,
-                  KeptPlanes* keep = nullptr);
-size_t gemm_backward_workspace_bytes(const BackwardProduct* products, int count, int dtype);
+int gemm_backward(const BackwardProduct* products, int count, const GroupPlan& plan, int dtype, void* workspace, size_t workspace_bytes,
+                  hipStream_t stream, KeptPlanes* keep = nullptr);
+size_t gemm_backward_workspace_bytes(const BackwardProduct* products, int count, const GroupPlan& plan, int dtype);
 
 // da and db (rows ld values apart) and h, all [M,N], of dh = dy Wd, the K-column rows of dy and the forward's products a and b, without dh:
 // true if these extents and types have one launch for it and it has been made.
 bool swiglu_gradient_together(const void* dy, const void* wd, const void* a, const void* b, void* da, void* db, void* h, int M, int N, int K, int ld,
                               int dtype, hipStream_t stream);
 
-// fmoe_mlp_backward with the products kept, whose scratch for slices of k lies apart from its workspace; dx may stay there as planes.
-struct MlpBackwardBytes { size_t workspace, planes; };
-MlpBackwardBytes mlp_backward_bytes(int64_t num_tokens, int hidden, int intermediate, int dtype);
+// Workspace and launches of fmoe_mlp_backward.  kept: the caller has the products; their planes are left out, and h takes the place of dh,
+// element by element as that is read.
+struct MlpBackwardPlan {
+    size_t off_a, off_b, off_dh, off_h, off_dab, off_part, part_bytes, bytes;
+    GroupPlan gradients;          // of the products after the SwiGLU gradient
+};
+MlpBackwardPlan plan_mlp_backward(int64_t num_tokens, int hidden, int intermediate, int dtype, bool kept);
+// ... and of fmoe_router_prologue_backward.
+struct PrologueBackwardPlan {
+    int row_blocks, rows_per_block;
+    bool folded;                  // a launch of its own adds the row blocks' column sums
+    int n_pad;                    // row length of d in the activation dtype: 2 * nk rounded up to whole packets
+    size_t off_d16, off_q, off_dq, off_partial, off_part, part_bytes, bytes;
+    GroupPlan products;
+};
+PrologueBackwardPlan plan_prologue_backward(int64_t num_tokens, int hidden, int num_keys, int dtype);
+
+// fmoe_mlp_backward by a plan of these extents.  planes: NULL, or plan.part_bytes for slices of k apart from the workspace (plan.off_part bytes
+// then), where dx may stay as planes.
 int mlp_backward_impl(const void* dy, const void* x, const void* gate_w, const void* up_w, const void* down_w, const void* saved_products,
                       int64_t num_tokens, int hidden, int intermediate, int dtype, void* dx, void* dgate_w, void* dup_w, void* ddown_w,
-                      void* workspace, size_t workspace_bytes, void* planes, KeptPlanes* keep_dx, hipStream_t stream);
+                      const MlpBackwardPlan& plan, void* workspace, size_t workspace_bytes, void* planes, KeptPlanes* keep_dx, hipStream_t stream);
 
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 inline size_t dtype_size(int dtype) { return dtype == FMOE_F32 ? 4 : 2; }

@@ -76,7 +76,6 @@ struct GroupMember {
     void* out;                   // C, or the planes of its slices
     int lda, ldb, M, N, K, segments, tiles_m, tiles_n, slices, first, a_turned;
 };
-constexpr int kGroupMost = 4;
 struct Group { GroupMember m[kGroupMost]; };
 
 template <typename T, int SHAPE, bool TA, bool SLICED>
@@ -229,9 +228,6 @@ void launch_turned(const void* A, int lda, const void* B0, const void* B1, int l
 #undef FMOE_WHOLE
 }
 
-// How a group is cut: one tile shape for all, slices of k for each, shape -1: one product after the other.
-struct GroupPlan { int shape, slices[kGroupMost]; };
-
 // Time of `kinds` lots of items (n[i] of time t[i], longest first) on `slots` that take the next item as they fall free.
 inline double time_of_items(const int64_t* n, const double* t, int kinds, int slots) {
     struct Free { double at; int64_t slots; } f[2 * kGroupMost + 2] = {{0.0, slots}};
@@ -378,9 +374,6 @@ template <typename T> GroupPlan plan_group(const BackwardProduct* p, int count) 
     return best;
 }
 
-GroupPlan plan_group_of(const BackwardProduct* p, int count, int dtype) {
-    return dtype == FMOE_F32 ? plan_group<float>(p, count) : plan_group<bf16_t>(p, count);
-}
 size_t group_planes_bytes(const BackwardProduct* p, int count, const GroupPlan& g) {
     size_t bytes = 0;
     for (int i = 0; i < count; ++i)
@@ -517,8 +510,11 @@ int gemm_backward(const BackwardProduct& q, int dtype, void* workspace, size_t w
     return blas_gemm(q.layout, q.M, q.N, q.K, (const char*)q.A + (size_t)q.K * dtype_size(dtype), q.lda, q.B1, q.ldb, q.C, q.N, 1.0f, dtype, stream);
 }
 
-size_t gemm_backward_workspace_bytes(const BackwardProduct* p, int count, int dtype) {
-    const GroupPlan plan = plan_group_of(p, count, dtype);
+GroupPlan plan_products(const BackwardProduct* p, int count, int dtype) {
+    return dtype == FMOE_F32 ? plan_group<float>(p, count) : plan_group<bf16_t>(p, count);
+}
+
+size_t gemm_backward_workspace_bytes(const BackwardProduct* p, int count, const GroupPlan& plan, int dtype) {
     if (plan.shape >= 0) return group_planes_bytes(p, count, plan);
     size_t most = 0;
     for (int i = 0; i < count; ++i) {
@@ -528,8 +524,8 @@ size_t gemm_backward_workspace_bytes(const BackwardProduct* p, int count, int dt
     return most;
 }
 
-int gemm_backward(const BackwardProduct* p, int count, int dtype, void* workspace, size_t workspace_bytes, hipStream_t stream, KeptPlanes* keep) {
-    const GroupPlan plan = plan_group_of(p, count, dtype);
+int gemm_backward(const BackwardProduct* p, int count, const GroupPlan& plan, int dtype, void* workspace, size_t workspace_bytes, hipStream_t stream,
+                  KeptPlanes* keep) {
     bool together = plan.shape >= 0 && group_planes_bytes(p, count, plan) <= workspace_bytes;
     for (int i = 0; i < count; ++i) together = together && addressable(p[i], dtype);
     together = together && !in_place(p, count, dtype);

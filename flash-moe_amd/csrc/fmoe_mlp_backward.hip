@@ -70,10 +70,6 @@ int rocblas_for_device(rocblas_handle* out) {
 
 constexpr int kNN = kBlasNN, kTN = kBlasTN;
 
-struct MlpBwdPlan {
-    size_t off_a, off_b, off_dh, off_h, off_dab, off_part, part_bytes, bytes;
-};
-
 // The products after the SwiGLU gradient, extents only.  adjacent: dWg and dWu follow each other in memory and are one [2I, H] product (49
 // us each alone, 74 together at T = I = 4096, H = 1024).
 int mlp_gradients(int T_, int H, int I, bool adjacent, BackwardProduct (&q)[4]) {
@@ -85,9 +81,28 @@ int mlp_gradients(int T_, int H, int I, bool adjacent, BackwardProduct (&q)[4]) 
     return adjacent ? 3 : 4;
 }
 
-// kept: the caller has the products.  Their planes are left out, and h takes the place of dh, element by element as that is read.
-MlpBwdPlan plan_mlp_backward(int64_t T_, int H, int I, int dtype, bool kept) {
-    MlpBwdPlan p;
+// How they are cut: planned for adjacent buffers; dWg and dWu apart are each cut as the product of both.
+GroupPlan cut_of(const GroupPlan& gradients, bool adjacent) {
+    GroupPlan g = gradients;
+    if (!adjacent) g.slices[3] = g.slices[2];
+    return g;
+}
+
+int check_extents(int64_t num_tokens, int hidden, int intermediate, int dtype) {
+    FMOE_REQUIRE(dtype_ok(dtype), FMOE_ERR_BAD_DTYPE, "fmoe_mlp_backward: unknown dtype %d", dtype);
+    FMOE_REQUIRE(num_tokens > 0 && hidden > 0 && intermediate > 0, FMOE_ERR_BAD_SHAPE, "fmoe_mlp_backward: bad shape T=%lld H=%d I=%d",
+                 (long long)num_tokens, hidden, intermediate);
+    FMOE_REQUIRE(num_tokens < (1ll << 31), FMOE_ERR_UNSUPPORTED, "fmoe_mlp_backward: T=%lld >= 2^31", (long long)num_tokens);
+    const int vec = (int)(16 / dtype_size(dtype));
+    FMOE_REQUIRE(hidden % vec == 0 && intermediate % vec == 0, FMOE_ERR_ALIGNMENT,
+                 "fmoe_mlp_backward: hidden=%d and intermediate=%d must be multiples of %d (16-byte rows)", hidden, intermediate, vec);
+    return FMOE_OK;
+}
+
+}  // namespace
+
+MlpBackwardPlan plan_mlp_backward(int64_t T_, int H, int I, int dtype, bool kept) {
+    MlpBackwardPlan p;
     const size_t ti = (size_t)T_ * I * dtype_size(dtype);
     size_t o = 0;
     auto take = [&](size_t n) { const size_t at = o; o = round_up(o + n, 256); return at; };
@@ -98,17 +113,17 @@ MlpBwdPlan plan_mlp_backward(int64_t T_, int H, int I, int dtype, bool kept) {
     p.off_dab = take(2 * ti);
     const int t = (int)T_;
     p.part_bytes = gemm_backward_workspace_bytes(t, I, H, 1, dtype);
+    BackwardProduct q[4];
+    p.gradients = plan_products(q, mlp_gradients(t, H, I, true, q), dtype);
     for (bool adjacent : {false, true}) {
-        BackwardProduct q[4];
-        const size_t n = gemm_backward_workspace_bytes(q, mlp_gradients(t, H, I, adjacent, q), dtype);
+        const int count = mlp_gradients(t, H, I, adjacent, q);
+        const size_t n = gemm_backward_workspace_bytes(q, count, cut_of(p.gradients, adjacent), dtype);
         if (n > p.part_bytes) p.part_bytes = n;
     }
     p.off_part = take(p.part_bytes);
     p.bytes = o;
     return p;
 }
-
-}  // namespace
 
 // Row-major product through the column-major library: C^T = B^T A^T, where a row-major [r,c] array is the
 // column-major [c,r] one.  fp32 accumulation; A, B and C have the element type `dtype`.
@@ -139,33 +154,24 @@ extern "C" size_t fmoe_mlp_backward_saved_workspace_bytes(int64_t num_tokens, in
     return fmoe::plan_mlp_backward(num_tokens, hidden, intermediate, dtype, true).bytes;
 }
 
-fmoe::MlpBackwardBytes fmoe::mlp_backward_bytes(int64_t num_tokens, int hidden, int intermediate, int dtype) {
-    const MlpBwdPlan p = plan_mlp_backward(num_tokens, hidden, intermediate, dtype, true);
-    return {p.off_part, p.part_bytes};
-}
-
 extern "C" int fmoe_mlp_backward(const void* dy, const void* x, const void* gate_w, const void* up_w, const void* down_w,
                                  const void* saved_products, int64_t num_tokens, int hidden, int intermediate, int dtype, void* dx, void* dgate_w, void* dup_w,
                                  void* ddown_w, void* workspace, size_t workspace_bytes, void* stream) {
-    fmoe::clear_error();
-    return fmoe::mlp_backward_impl(dy, x, gate_w, up_w, down_w, saved_products, num_tokens, hidden, intermediate, dtype, dx, dgate_w, dup_w, ddown_w,
-                                   workspace, workspace_bytes, nullptr, nullptr, (hipStream_t)stream);
+    using namespace fmoe;
+    clear_error();
+    if (int rc = check_extents(num_tokens, hidden, intermediate, dtype)) return rc;
+    return mlp_backward_impl(dy, x, gate_w, up_w, down_w, saved_products, num_tokens, hidden, intermediate, dtype, dx, dgate_w, dup_w, ddown_w,
+                             plan_mlp_backward(num_tokens, hidden, intermediate, dtype, saved_products != nullptr), workspace, workspace_bytes, nullptr,
+                             nullptr, (hipStream_t)stream);
 }
 
 int fmoe::mlp_backward_impl(const void* dy, const void* x, const void* gate_w, const void* up_w, const void* down_w, const void* saved_products,
                             int64_t num_tokens, int hidden, int intermediate, int dtype, void* dx, void* dgate_w, void* dup_w, void* ddown_w,
-                            void* workspace, size_t workspace_bytes, void* planes, KeptPlanes* keep_dx, hipStream_t s) {
+                            const MlpBackwardPlan& p, void* workspace, size_t workspace_bytes, void* planes, KeptPlanes* keep_dx, hipStream_t s) {
     using namespace fmoe;
-    FMOE_REQUIRE(dtype_ok(dtype), FMOE_ERR_BAD_DTYPE, "fmoe_mlp_backward: unknown dtype %d", dtype);
-    FMOE_REQUIRE(num_tokens > 0 && hidden > 0 && intermediate > 0, FMOE_ERR_BAD_SHAPE, "fmoe_mlp_backward: bad shape T=%lld H=%d I=%d",
-                 (long long)num_tokens, hidden, intermediate);
-    FMOE_REQUIRE(num_tokens < (1ll << 31), FMOE_ERR_UNSUPPORTED, "fmoe_mlp_backward: T=%lld >= 2^31", (long long)num_tokens);
-    const int vec = (int)(16 / dtype_size(dtype));
-    FMOE_REQUIRE(hidden % vec == 0 && intermediate % vec == 0, FMOE_ERR_ALIGNMENT,
-                 "fmoe_mlp_backward: hidden=%d and intermediate=%d must be multiples of %d (16-byte rows)", hidden, intermediate, vec);
+    if (int rc = check_extents(num_tokens, hidden, intermediate, dtype)) return rc;
     FMOE_REQUIRE(dy && x && gate_w && up_w && down_w && dx && dgate_w && dup_w && ddown_w, FMOE_ERR_NULL_POINTER,
                  "fmoe_mlp_backward: null tensor pointer");
-    const MlpBwdPlan p = plan_mlp_backward(num_tokens, hidden, intermediate, dtype, saved_products != nullptr);
     const size_t need = planes != nullptr ? p.off_part : p.bytes;
     FMOE_REQUIRE(workspace && workspace_bytes >= need && aligned16(workspace), FMOE_ERR_WORKSPACE,
                  "fmoe_mlp_backward: workspace of %zu bytes needed, %zu given", need, workspace_bytes);
@@ -202,11 +208,12 @@ int fmoe::mlp_backward_impl(const void* dy, const void* x, const void* gate_w, c
     }
     const size_t w_bytes = (size_t)I * H * elt;
     BackwardProduct q[4];
-    const int count = mlp_gradients(T_, H, I, (char*)dup_w == (char*)dgate_w + w_bytes, q);
+    const bool adjacent = (char*)dup_w == (char*)dgate_w + w_bytes;
+    const int count = mlp_gradients(T_, H, I, adjacent, q);
     q[0].A = dy, q[0].B0 = h, q[0].C = ddown_w;
     q[1].A = dab, q[1].B0 = gate_w, q[1].B1 = up_w, q[1].C = dx;
     q[2].A = dab, q[2].B0 = x, q[2].C = dgate_w;
     q[3].A = db, q[3].B0 = x, q[3].C = dup_w;
     if (keep_dx != nullptr) *keep_dx = {1, nullptr, 0};
-    return gemm_backward(q, count, dtype, part, p.part_bytes, s, keep_dx);
+    return gemm_backward(q, count, cut_of(p.gradients, adjacent), dtype, part, p.part_bytes, s, keep_dx);
 }

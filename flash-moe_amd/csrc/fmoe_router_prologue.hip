@@ -835,20 +835,26 @@ ColumnSumsPlan plan_column_sums(int64_t T_, int H, int vec) {
     return {(int)((T_ + rows - 1) / rows), rows, true};
 }
 
-struct PrologueBwdPlan {
-    ColumnSumsPlan sums;
-    int n_pad;            // row length of d in the activation dtype: 2 * nk rounded up to whole packets
-    size_t off_d16, off_q, off_dq, off_partial, off_part, part_bytes, bytes;
-};
-
 // The two products, extents only.
 void prologue_products(int T_, int H, int N, int n_pad, BackwardProduct (&q)[2]) {
     q[0] = {kBlasTN, N, H, T_, 1, nullptr, n_pad, nullptr, nullptr, H, nullptr};      // dWr = d^T q
     q[1] = {kBlasNN, T_, H, N, 1, nullptr, n_pad, nullptr, nullptr, H, nullptr};      // dq = d Wr
 }
 
-PrologueBwdPlan plan_prologue_backward(int64_t T_, int H, int nk, int dtype) {
-    PrologueBwdPlan p;
+int check_prologue_backward(int64_t num_tokens, int hidden, int num_keys, int dtype) {
+    FMOE_REQUIRE(dtype_ok(dtype), FMOE_ERR_BAD_DTYPE, "fmoe_router_prologue_backward: unknown dtype %d", dtype);
+    FMOE_REQUIRE(num_tokens > 0 && hidden > 0 && num_keys > 0 && num_tokens < (1ll << 24), FMOE_ERR_BAD_SHAPE,
+                 "fmoe_router_prologue_backward: bad shape T=%lld H=%d nk=%d", (long long)num_tokens, hidden, num_keys);
+    const int vec = (int)(16 / dtype_size(dtype));
+    FMOE_REQUIRE(hidden % vec == 0, FMOE_ERR_ALIGNMENT,
+                 "fmoe_router_prologue_backward: hidden=%d must be a multiple of %d", hidden, vec);
+    return FMOE_OK;
+}
+
+}  // namespace
+
+PrologueBackwardPlan plan_prologue_backward(int64_t T_, int H, int nk, int dtype) {
+    PrologueBackwardPlan p;
     const size_t elt = dtype_size(dtype);
     size_t o = 0;
     auto take = [&](size_t n) { const size_t at = o; o = round_up(o + n, 256); return at; };
@@ -857,22 +863,27 @@ PrologueBwdPlan plan_prologue_backward(int64_t T_, int H, int nk, int dtype) {
     p.off_d16 = take((size_t)T_ * p.n_pad * elt);
     p.off_q = take((size_t)T_ * H * elt);
     p.off_dq = take((size_t)T_ * H * elt);
-    p.sums = plan_column_sums(T_, H, vec);
-    p.off_partial = take((size_t)(p.sums.row_blocks + 1) * 2 * H * 4);
+    const ColumnSumsPlan sums = plan_column_sums(T_, H, vec);
+    p.row_blocks = sums.row_blocks;
+    p.rows_per_block = sums.rows_per_block;
+    p.folded = sums.folded;
+    p.off_partial = take((size_t)(p.row_blocks + 1) * 2 * H * 4);
     BackwardProduct products[2];
     prologue_products(t, H, 2 * nk, p.n_pad, products);
-    p.part_bytes = gemm_backward_workspace_bytes(products, 2, dtype);
+    p.products = plan_products(products, 2, dtype);
+    p.part_bytes = gemm_backward_workspace_bytes(products, 2, p.products, dtype);
     p.off_part = take(p.part_bytes);
     p.bytes = o;
     return p;
 }
 
+namespace {
+
 template <typename T>
 int launch_prologue_backward(const float* dlogits, const void* x, const void* gate_w, const float* mean_rstd, int training,
-                             int64_t T_, int H, int nk, int dtype, void* dx, void* dgate_w, const TokenGradients& more, void* workspace,
-                             hipStream_t s, bool operands_ready) {
+                             int64_t T_, int H, int nk, int dtype, void* dx, void* dgate_w, const TokenGradients& more, const PrologueBackwardPlan& p,
+                             void* workspace, hipStream_t s, bool operands_ready) {
     constexpr int V = Elem<T>::kVec;
-    const PrologueBwdPlan p = plan_prologue_backward(T_, H, nk, dtype);
     char* ws = (char*)workspace;
     T *d16 = (T*)(ws + p.off_d16), *q = (T*)(ws + p.off_q), *dq = (T*)(ws + p.off_dq);
     float* partial = (float*)(ws + p.off_partial);
@@ -890,15 +901,15 @@ int launch_prologue_backward(const float* dlogits, const void* x, const void* ga
     products[0].A = products[1].A = d16;
     products[0].B0 = q, products[0].C = dgate_w;
     products[1].B0 = gate_w, products[1].C = dq;
-    if (int rc = gemm_backward(products, 2, dtype, part, p.part_bytes, s)) return rc;
+    if (int rc = gemm_backward(products, 2, p.products, dtype, part, p.part_bytes, s)) return rc;
     if (training) {
         const int strips = (H + 8 * V - 1) / (8 * V);
-        hipLaunchKernelGGL((bn_bwd_partial_kernel<T>), dim3((unsigned)p.sums.row_blocks, (unsigned)strips), dim3(kStatsThreads), 0, s,
-                           (const T*)x, (const T*)dq, mean_rstd, T_, H, p.sums.rows_per_block, partial);
+        hipLaunchKernelGGL((bn_bwd_partial_kernel<T>), dim3((unsigned)p.row_blocks, (unsigned)strips), dim3(kStatsThreads), 0, s,
+                           (const T*)x, (const T*)dq, mean_rstd, T_, H, p.rows_per_block, partial);
         FMOE_CHECK_LAUNCH("fmoe_router_prologue_backward(column sums)");
     }
-    int row_blocks = p.sums.row_blocks;
-    if (training && p.sums.folded) {
+    int row_blocks = p.row_blocks;
+    if (training && p.folded) {
         float* sums = partial + (size_t)row_blocks * 2 * H;
         hipLaunchKernelGGL(bn_bwd_fold_kernel, dim3((unsigned)((2 * H + 31) / 32)), dim3(256), 0, s, (const float*)partial, row_blocks, H, sums);
         FMOE_CHECK_LAUNCH("fmoe_router_prologue_backward(row blocks)");
@@ -1137,38 +1148,32 @@ extern "C" size_t fmoe_router_prologue_backward_workspace_bytes(int64_t num_toke
 extern "C" int fmoe_router_prologue_backward(const float* dlogits_fp32, const void* x, const void* gate_w, const float* mean_rstd,
                                              int training, int64_t num_tokens, int hidden, int num_keys, int dtype, void* dx,
                                              void* dgate_w, void* workspace, size_t workspace_bytes, void* stream) {
-    fmoe::clear_error();
-    return fmoe::router_prologue_backward_impl(dlogits_fp32, x, gate_w, mean_rstd, training, num_tokens, hidden, num_keys, dtype, dx,
-                                               dgate_w, {}, workspace, workspace_bytes, (hipStream_t)stream);
+    using namespace fmoe;
+    clear_error();
+    if (int rc = check_prologue_backward(num_tokens, hidden, num_keys, dtype)) return rc;
+    return router_prologue_backward_impl(dlogits_fp32, x, gate_w, mean_rstd, training, num_tokens, hidden, num_keys, dtype, dx, dgate_w, {},
+                                         plan_prologue_backward(num_tokens, hidden, num_keys, dtype), workspace, workspace_bytes, (hipStream_t)stream);
 }
 
-fmoe::PrologueOperands fmoe::prologue_operands(const void* x, const float* mean_rstd, int64_t num_tokens, int hidden, int num_keys, int dtype,
-                                               void* workspace) {
-    const PrologueBwdPlan p = plan_prologue_backward(num_tokens, hidden, num_keys, dtype);
+fmoe::PrologueOperands fmoe::prologue_operands(const void* x, const float* mean_rstd, int hidden, const PrologueBackwardPlan& p, void* workspace) {
     return {(char*)workspace + p.off_d16, (char*)workspace + p.off_q, p.n_pad, hidden, x, mean_rstd};
 }
 
 int fmoe::router_prologue_backward_impl(const float* dlogits_fp32, const void* x, const void* gate_w, const float* mean_rstd,
                                         int training, int64_t num_tokens, int hidden, int num_keys, int dtype, void* dx,
-                                        void* dgate_w, const TokenGradients& more, void* workspace, size_t workspace_bytes,
+                                        void* dgate_w, const TokenGradients& more, const PrologueBackwardPlan& p, void* workspace, size_t workspace_bytes,
                                         hipStream_t s, bool operands_ready) {
     using namespace fmoe;
-    FMOE_REQUIRE(dtype_ok(dtype), FMOE_ERR_BAD_DTYPE, "fmoe_router_prologue_backward: unknown dtype %d", dtype);
-    FMOE_REQUIRE(num_tokens > 0 && hidden > 0 && num_keys > 0 && num_tokens < (1ll << 24), FMOE_ERR_BAD_SHAPE,
-                 "fmoe_router_prologue_backward: bad shape T=%lld H=%d nk=%d", (long long)num_tokens, hidden, num_keys);
-    const int vec = (int)(16 / dtype_size(dtype));
-    FMOE_REQUIRE(hidden % vec == 0, FMOE_ERR_ALIGNMENT,
-                 "fmoe_router_prologue_backward: hidden=%d must be a multiple of %d", hidden, vec);
+    if (int rc = check_prologue_backward(num_tokens, hidden, num_keys, dtype)) return rc;
     FMOE_REQUIRE((dlogits_fp32 || operands_ready) && x && gate_w && mean_rstd && dx && dgate_w, FMOE_ERR_NULL_POINTER,
                  "fmoe_router_prologue_backward: null tensor pointer");
     FMOE_REQUIRE(aligned16(x) && aligned16(dx) && aligned16(dlogits_fp32) && aligned16(mean_rstd), FMOE_ERR_ALIGNMENT,
                  "fmoe_router_prologue_backward: tensor pointers must be 16-byte aligned");
-    const size_t need = plan_prologue_backward(num_tokens, hidden, num_keys, dtype).bytes;
-    FMOE_REQUIRE(workspace && workspace_bytes >= need && aligned16(workspace), FMOE_ERR_WORKSPACE,
-                 "fmoe_router_prologue_backward: workspace of %zu bytes needed, %zu given", need, workspace_bytes);
+    FMOE_REQUIRE(workspace && workspace_bytes >= p.bytes && aligned16(workspace), FMOE_ERR_WORKSPACE,
+                 "fmoe_router_prologue_backward: workspace of %zu bytes needed, %zu given", p.bytes, workspace_bytes);
     switch (dtype) {
-        case FMOE_F32: return launch_prologue_backward<float>(dlogits_fp32, x, gate_w, mean_rstd, training, num_tokens, hidden, num_keys, dtype, dx, dgate_w, more, workspace, s, operands_ready);
-        case FMOE_BF16: return launch_prologue_backward<bf16_t>(dlogits_fp32, x, gate_w, mean_rstd, training, num_tokens, hidden, num_keys, dtype, dx, dgate_w, more, workspace, s, operands_ready);
-        default: return launch_prologue_backward<f16_t>(dlogits_fp32, x, gate_w, mean_rstd, training, num_tokens, hidden, num_keys, dtype, dx, dgate_w, more, workspace, s, operands_ready);
+        case FMOE_F32: return launch_prologue_backward<float>(dlogits_fp32, x, gate_w, mean_rstd, training, num_tokens, hidden, num_keys, dtype, dx, dgate_w, more, p, workspace, s, operands_ready);
+        case FMOE_BF16: return launch_prologue_backward<bf16_t>(dlogits_fp32, x, gate_w, mean_rstd, training, num_tokens, hidden, num_keys, dtype, dx, dgate_w, more, p, workspace, s, operands_ready);
+        default: return launch_prologue_backward<f16_t>(dlogits_fp32, x, gate_w, mean_rstd, training, num_tokens, hidden, num_keys, dtype, dx, dgate_w, more, p, workspace, s, operands_ready);
     }
 }
