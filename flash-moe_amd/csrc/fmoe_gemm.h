@@ -691,8 +691,7 @@ enum TileShape { kTile256, kTile128, kTile64x128, kTile64, kSplit32, kSplit16x32
 constexpr int kTileRows[7] = {256, 128, 64, 64, 32, 16, 16}, kTileCols[7] = {256, 128, 128, 64, 32, 32, 16};
 
 // Workgroups of tile i, and the time of a round of them per k-tile.
-template <typename T, int EPI> double tile_cost(int i, int M, int N, int64_t& n) {
-    const int cus = chip_info().cus;
+template <typename T, int EPI> double tile_cost(int i, int M, int N, int cus, int64_t& n) {
     const bool split_k = i >= kSplit32;
     const int out_cols = EPI == kEpiSwiGLU && !split_k ? kTileCols[i] / 2 : kTileCols[i];
     const int cols = EPI == kEpiSwiGLU ? 2 * out_cols : out_cols;
@@ -709,7 +708,7 @@ template <typename T, int EPI> TileShape choose_tile(int M, int N, int& tiles, d
     double best_cost = 0.0;
     for (int i = 0; i < 7; ++i) {
         int64_t n = 0;
-        const double round = tile_cost<T, EPI>(i, M, N, n), cost = (double)((n + cus - 1) / cus) * round;
+        const double round = tile_cost<T, EPI>(i, M, N, cus, n), cost = (double)((n + cus - 1) / cus) * round;
         if (i == 0 || cost < best_cost) {
             best = (TileShape)i;
             best_cost = cost;
@@ -744,7 +743,7 @@ template <typename T> SlicePlan plan_slices_of_k(int M, int N, int K) {
     if (sizeof(T) == 4 && K % 4 != 0) return best;
     for (int i = sizeof(T) == 2 ? kTile256 : kTile128; i <= kTile64; ++i) {
         int64_t n = 0;
-        const double round = tile_cost<T, kEpiPlain>(i, M, N, n);
+        const double round = tile_cost<T, kEpiPlain>(i, M, N, cus, n);
         for (int s = 2; s <= kMaxSlices && n * s <= cus && s * 4 <= k_tiles; ++s) {
             const int share = (k_tiles + s - 1) / s;
             if ((s - 1) * share >= k_tiles) continue;           // a slice would have no k-tile

@@ -157,7 +157,7 @@ template <typename T> SlicePlan plan_turned(int M, int N, int K, int segments, d
     for (int i = sizeof(T) == 4 ? kTile128 : kTile256; i <= kTile64; ++i) {
         int64_t n = 0;
         if (sizeof(T) == 4 && i == kTile64x128) continue;
-        const double row = tile_cost<T, kEpiPlain>(i, M, N, n) * 2.3e-3, stores = i == kTile256 ? 7.0 : 1.0;
+        const double row = tile_cost<T, kEpiPlain>(i, M, N, cus, n) * 2.3e-3, stores = i == kTile256 ? 7.0 : 1.0;
         const int64_t most = sizeof(T) == 4 && i == kTile64 ? 2 * cus : cus;
         for (int s = 1; s <= kMaxSlices && (s == 1 || (n * s <= most && 2 * s <= k_tiles)); ++s) {
             const int share = (k_tiles + s - 1) / s;
