@@ -245,7 +245,7 @@ struct MlpBackwardPlan {
 MlpBackwardPlan plan_mlp_backward(int64_t num_tokens, int hidden, int intermediate, int dtype, bool kept);
 // ... and of fmoe_router_prologue_backward.
 struct PrologueBackwardPlan {
-    int row_blocks, rows_per_block;
+    int row_blocks, rows_per_block, lane_bits;      // of the batch-norm gradient's column sums, and the packets of a row side by side
     bool folded;                  // a launch of its own adds the row blocks' column sums
     int n_pad;                    // row length of d in the activation dtype: 2 * nk rounded up to whole packets
     size_t off_d16, off_q, off_dq, off_partial, off_part, part_bytes, bytes;

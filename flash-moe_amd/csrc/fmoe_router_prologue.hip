@@ -596,15 +596,17 @@ __global__ __launch_bounds__(256) void prologue_bwd_prepare_kernel(const float* 
     }
 }
 
-// partial: [row_blocks][2][H] = (sum dq, sum dq * xhat) over the block's rows; strips of bn_block_stats_kernel.
+// partial: [row_blocks][2][H] = (sum dq, sum dq * xhat) over the block's rows.  A workgroup takes a strip of 2^lane_bits packets, a wave 64
+// lanes of its rows, rows 256 >> lane_bits apart.
 template <typename T>
 __global__ __launch_bounds__(kStatsThreads) void bn_bwd_partial_kernel(const T* __restrict__ x, const T* __restrict__ dq,
                                                                       const float* __restrict__ mean_rstd, int64_t num_tokens,
-                                                                      int hidden, int rows_per_block, float* __restrict__ partial) {
+                                                                      int hidden, int rows_per_block, int lane_bits, float* __restrict__ partial) {
     constexpr int V = Elem<T>::kVec;
-    __shared__ float red[3][2][8 * V];
+    __shared__ float red[3][2][kWave * V];
     const int lane = lane_id(), wave = (int)(threadIdx.x >> 6);
-    const int col = ((int)blockIdx.y * 8 + (lane & 7)) * V;
+    const int width = 1 << lane_bits, wave_rows = kWave >> lane_bits, step = 4 * wave_rows;
+    const int col = ((int)blockIdx.y * width + (lane & (width - 1))) * V;
     const bool col_ok = col < hidden;
     const int64_t r0 = (int64_t)blockIdx.x * rows_per_block;
     const int64_t r1 = r0 + rows_per_block < num_tokens ? r0 + rows_per_block : num_tokens;
@@ -617,17 +619,17 @@ __global__ __launch_bounds__(kStatsThreads) void bn_bwd_partial_kernel(const T* 
     }
     if (col_ok) {
         constexpr int kBatch = 4;                                // rows of x and dq issued together: one memory round trip per batch
-        for (int64_t rb = r0 + wave * 8 + (lane >> 3); rb < r1; rb += 32 * kBatch) {
+        for (int64_t rb = r0 + wave * wave_rows + (lane >> lane_bits); rb < r1; rb += step * kBatch) {
             u32x4_t raw[kBatch], raw_dq[kBatch];
 #pragma unroll
             for (int i = 0; i < kBatch; ++i) {
-                const int64_t r = rb + 32 * i < r1 ? rb + 32 * i : r1 - 1;
+                const int64_t r = rb + step * i < r1 ? rb + step * i : r1 - 1;
                 raw[i] = *reinterpret_cast<const u32x4_t*>(x + r * hidden + col);
                 raw_dq[i] = *reinterpret_cast<const u32x4_t*>(dq + r * hidden + col);
             }
 #pragma unroll
             for (int i = 0; i < kBatch; ++i) {
-                if (rb + 32 * i >= r1) continue;
+                if (rb + step * i >= r1) continue;
                 float xv[V], gv[V];
                 unpack16<T>(raw[i], xv);
                 unpack16<T>(raw_dq[i], gv);
@@ -639,16 +641,14 @@ __global__ __launch_bounds__(kStatsThreads) void bn_bwd_partial_kernel(const T* 
             }
         }
     }
-    // the 8 row lanes of a wave, then waves 1..3 -> wave 0 through LDS; fixed order
+    // the row lanes of a wave, then waves 1..3 -> wave 0 through LDS; fixed order
+    for (int m = width; m < kWave; m <<= 1)
 #pragma unroll
-    for (int v = 0; v < V; ++v) {
-#pragma unroll
-        for (int m = 8; m < kWave; m <<= 1) {
+        for (int v = 0; v < V; ++v) {
             s1[v] += __shfl_xor(s1[v], m, kWave);
             s2[v] += __shfl_xor(s2[v], m, kWave);
         }
-    }
-    if (wave > 0 && lane < 8) {
+    if (wave > 0 && lane < width) {
 #pragma unroll
         for (int v = 0; v < V; ++v) {
             red[wave - 1][0][lane * V + v] = s1[v];
@@ -656,7 +656,7 @@ __global__ __launch_bounds__(kStatsThreads) void bn_bwd_partial_kernel(const T* 
         }
     }
     __syncthreads();
-    if (wave == 0 && lane < 8 && col_ok) {
+    if (wave == 0 && lane < width && col_ok) {
 #pragma unroll
         for (int w = 0; w < 3; ++w)
 #pragma unroll
@@ -821,18 +821,28 @@ __global__ __launch_bounds__(256) void bn_bwd_apply_kernel(const T* __restrict__
     }
 }
 
-// Row blocks of the batch-norm gradient's column sums.  Up to kFoldMaxRowBlocks of them the last launch adds itself; where few strips leave
-// compute units idle so, as many as fill the chip, if their rows are fewer by what a launch that adds them takes (250; 1000 where there is
-// a workgroup for every other compute unit already).
-struct ColumnSumsPlan { int row_blocks, rows_per_block; bool folded; };
-ColumnSumsPlan plan_column_sums(int64_t T_, int H, int vec) {
+// Packets of a row that a wave's lanes have side by side: 64, or what a shorter row has.
+int row_lane_bits(int packets) {
+    int bits = 6;
+    while (bits > 0 && packets <= 1 << (bits - 1)) --bits;
+    return bits;
+}
+
+// Row blocks of the batch-norm gradient's column sums.  Few tokens: at most kFoldMaxRowBlocks of them on strips of 8 packets, which the last
+// launch adds.  From 16384 on that leaves rows of few strips on few compute units and reads each row in pieces of 128 bytes: as many row
+// blocks as fill the chip on strips of a wave's width, added by a launch of their own.  The router prologue's backward in bf16, 32 keys, two
+// launches | three: 12000 tokens, 512 columns 51.2 | 53.5, 64 columns 39.6 | 38.2; 8192, 512 46.0 | 48.5; 16384, 64 58 | 45; 32768, 512 102 | 88.
+constexpr int64_t kThreeLaunches = 16384;
+struct ColumnSumsPlan { int row_blocks, rows_per_block, lane_bits; bool folded; };
+ColumnSumsPlan plan_column_sums(int64_t T_, int packets) {
     const BlockStatsPlan few = plan_block_stats(T_);
-    const int64_t strips = (H + 8 * vec - 1) / (8 * vec), wanted = 2 * chip_info().cus / strips, most = (T_ + 127) / 128;
+    if (T_ < kThreeLaunches) return {few.row_blocks, few.rows_per_block, 3, false};
+    const int bits = row_lane_bits(packets);
+    const int64_t strips = (packets + (1 << bits) - 1) >> bits, wanted = 2 * chip_info().cus / strips + 1, most = (T_ + 31) / 32;
     int64_t rb = wanted < most ? wanted : most;
     if (rb > kMaxRowBlocks) rb = kMaxRowBlocks;
-    const int rows = rb > kFoldMaxRowBlocks ? (int)((T_ + rb - 1) / rb) : few.rows_per_block;
-    if (few.rows_per_block - rows < (strips * kFoldMaxRowBlocks <= chip_info().cus / 2 ? 250 : 1000)) return {few.row_blocks, few.rows_per_block, false};
-    return {(int)((T_ + rows - 1) / rows), rows, true};
+    const int rows = (int)((T_ + rb - 1) / rb);
+    return {(int)((T_ + rows - 1) / rows), rows, bits, true};
 }
 
 // The two products, extents only.
@@ -863,9 +873,10 @@ PrologueBackwardPlan plan_prologue_backward(int64_t T_, int H, int nk, int dtype
     p.off_d16 = take((size_t)T_ * p.n_pad * elt);
     p.off_q = take((size_t)T_ * H * elt);
     p.off_dq = take((size_t)T_ * H * elt);
-    const ColumnSumsPlan sums = plan_column_sums(T_, H, vec);
+    const ColumnSumsPlan sums = plan_column_sums(T_, (H + vec - 1) / vec);
     p.row_blocks = sums.row_blocks;
     p.rows_per_block = sums.rows_per_block;
+    p.lane_bits = sums.lane_bits;
     p.folded = sums.folded;
     p.off_partial = take((size_t)(p.row_blocks + 1) * 2 * H * 4);
     BackwardProduct products[2];
@@ -903,9 +914,9 @@ int launch_prologue_backward(const float* dlogits, const void* x, const void* ga
     products[1].B0 = gate_w, products[1].C = dq;
     if (int rc = gemm_backward(products, 2, p.products, dtype, part, p.part_bytes, s)) return rc;
     if (training) {
-        const int strips = (H + 8 * V - 1) / (8 * V);
+        const int strips = (H / V + (1 << p.lane_bits) - 1) >> p.lane_bits;
         hipLaunchKernelGGL((bn_bwd_partial_kernel<T>), dim3((unsigned)p.row_blocks, (unsigned)strips), dim3(kStatsThreads), 0, s,
-                           (const T*)x, (const T*)dq, mean_rstd, T_, H, p.rows_per_block, partial);
+                           (const T*)x, (const T*)dq, mean_rstd, T_, H, p.rows_per_block, p.lane_bits, partial);
         FMOE_CHECK_LAUNCH("fmoe_router_prologue_backward(column sums)");
     }
     int row_blocks = p.row_blocks;
@@ -917,9 +928,7 @@ int launch_prologue_backward(const float* dlogits, const void* x, const void* ga
         row_blocks = 1;
     }
     // about two workgroups to a compute unit
-    const int packets = H / V;
-    int lane_bits = 6;
-    while (lane_bits > 0 && packets <= 1 << (lane_bits - 1)) --lane_bits;
+    const int packets = H / V, lane_bits = row_lane_bits(packets);
     const int64_t strips = (packets + kWave - 1) / kWave, wanted = 2 * chip_info().cus / strips + 1, step = 4 * (kWave >> lane_bits);
     const int apply_rows = (int)((T_ + wanted * step - 1) / (wanted * step) * step);
     hipLaunchKernelGGL((bn_bwd_apply_kernel<T>), dim3((unsigned)((T_ + apply_rows - 1) / apply_rows), (unsigned)strips), dim3(256), 0, s, (const T*)x,

@@ -578,7 +578,7 @@ def test_block_backward_operands_from_the_routing_gradient(dtype, H, nk, K):
 @pytest.mark.parametrize("dtype,T,H,I", [
     (torch.bfloat16, 615, 776, 2072), (torch.float32, 383, 516, 1544),     # dx of the MLP in slices of k: added with the other gradients
     (torch.float16, 2050, 72, 136), (torch.bfloat16, 4101, 520, 264),      # more than one row to a wave, rows beyond the last block
-    (torch.float32, 3, 4, 8), (torch.bfloat16, 8200, 72, 136),
+    (torch.float32, 3, 4, 8), (torch.bfloat16, 16400, 72, 136),
 ])
 def test_block_backward_adds_the_token_gradients(dtype, T, H, I):
     """dx of the block is the sum of the MLP's, the experts' and the router's, formed where the last of them is."""
@@ -698,7 +698,7 @@ def test_mlp_backward_with_adjacent_and_separate_buffers(dtype, stacked_weights,
 @pytest.mark.parametrize("T,H,nk", [(256, 128, 16), (1000, 1024, 128), (65, 64, 8), (256, 128, 32), (1024, 1024, 128),
                                     (128, 64, 10), (70, 64, 6), (64, 128, 30), (40, 32, 81),
                                     # column sums of more row blocks than the last launch adds; rows of one packet, two, nine and 65
-                                    (9000, 8, 3), (8200, 72, 12), (33000, 520, 5)])
+                                    (16384, 8, 3), (17000, 72, 12), (33000, 520, 5)])
 def test_router_prologue_backward(dtype, training, T, H, nk):
     """Batch norm + gate product: gradients of the input and of the gate weights against float64 autograd."""
     from flash_moe.ops.hip.flash_router import router_prologue
