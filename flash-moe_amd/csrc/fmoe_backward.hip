@@ -792,7 +792,6 @@ ExpertBwdPlan plan_expert_backward(int64_t T_, int H, int64_t E, int K, int dtyp
     size_t o = 0;
     auto take = [&](size_t n) { const size_t at = o; o = round_up(o + n, 256); return at; };
     p.off_coef = take(pairs * 8);
-    p.off_coef_list = take(pairs * 4);
     p.quarters = quarter_waves(T_, (int64_t)H * (int64_t)dtype_size(dtype), E, (int64_t)pairs);
     p.off_entries = take(p.quarters ? pairs * 16 : 0);
     p.off_pairs = take(pairs * 4);
@@ -802,8 +801,9 @@ ExpertBwdPlan plan_expert_backward(int64_t T_, int H, int64_t E, int K, int dtyp
     p.slices = kept.kept;
     p.ordered = kept.ordered;
     p.num_slices = p.slices ? expert_slice_count(T_, H, E, K, dtype, p.ordered) : 0;
-    p.off_off32 = p.off_place = p.off_spart_s = p.off_spart_u = o;
+    p.off_off32 = p.off_place = p.off_coef_list = p.off_spart_s = p.off_spart_u = o;
     if (p.slices) {
+        p.off_coef_list = take(pairs * 4);
         p.off_off32 = take(pairs * 4);
         p.off_place = take(p.ordered ? pairs * 2 : 0);
         p.off_spart_s = take((size_t)p.num_slices * pairs * 4);

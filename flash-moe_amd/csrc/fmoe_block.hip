@@ -79,7 +79,7 @@ BlockBackwardPlan plan_block_backward(int64_t T_, int H, int I, int nk, int64_t 
     size_t o = 0;
     auto take = [&](size_t n) { const size_t at = o; o = round_up(o + n, 256); return at; };
     p.off_dgates = take((size_t)T_ * K * elt);
-    p.off_dlogits32 = take((size_t)T_ * 2 * nk * 4);
+    p.off_dlogits32 = take(route_backward_prepares(nk, K) ? 0 : (size_t)T_ * 2 * nk * 4);
     p.off_dx_experts = take((size_t)T_ * H * elt);
     p.mlp = plan_mlp_backward(T_, H, I, dtype, true);
     p.prologue = plan_prologue_backward(T_, H, nk, dtype);

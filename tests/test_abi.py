@@ -199,7 +199,11 @@ def test_backward_argument_checks():
     assert sb(a, None, a, 4, 64, _C.BF16, a, a, None) == -1
     assert sb(None, None, None, 0, 64, _C.BF16, None, None, None) == 0
     need = lib.fmoe_expert_backward_workspace_bytes(8, 64, 256, 4, _C.BF16)
-    assert need >= 8 * 4 * 24 + 257 * 4 and need % 256 == 0
+    # rows: two fp32 coefficients and a place in its expert's list for every pair, the lists' ends; with slices one of the
+    # coefficients, the row's offset and two partial scores to a slice for every pair besides
+    assert need >= 8 * 4 * (8 + 4) + 257 * 4 and need % 256 == 0
+    sliced = lib.fmoe_expert_backward_workspace_bytes(4096, 1024, 16384, 64, _C.BF16)
+    assert sliced >= 4096 * 64 * (8 + 4 + 4 + 4 + 2 * 8 * 4) + 16385 * 4 and sliced % 256 == 0
     eb = lib.fmoe_expert_backward
 
     def ecall(T=8, H=64, E=256, K=4, dtype=_C.BF16, dout=a, ws=a, ws_bytes=need):
@@ -297,6 +301,18 @@ def test_expert_workspace_is_enough_for_both_forwards():
         assert need >= lib.fmoe_expert_workspace_bytes_algo(T, H, E, K, _C.BF16, _C.EXPERT_AUTO)
         if K > 64:
             assert need >= lib.fmoe_expert_workspace_bytes_algo(T, H, E, K, _C.BF16, _C.EXPERT_ORDERED)
+
+
+def test_backward_scratch_holds_only_what_its_schedule_writes():
+    """The row schedule of the experts has no list of coefficients; the block keeps no fp32 gradients of the logits where the routing
+    gradient leaves as the gate's products read it (up to 256 keys and 128 experts)."""
+    lib = _C.lib()
+    T, H, E, K = 2048, 256, 4096, 8
+    pairs, group = T * K, lib.fmoe_expert_backward_workspace_bytes(0, H, E, K, _C.BF16)
+    assert group == 0 and lib.fmoe_expert_saved_bytes(T, H, E, K, _C.BF16) == 0             # rows
+    assert lib.fmoe_expert_backward_workspace_bytes(T, H, E, K, _C.BF16) < pairs * (8 + 4) + (E + 1) * 4 + 4 * 256
+    few, many = (lib.fmoe_block_backward_workspace_bytes(4096, 64, 64, nk, 257 * 257, 4, _C.BF16) for nk in (256, 257))
+    assert 4096 * 2 * 257 * 4 <= many - few
 
 
 def test_training_keeps_two_planes_of_the_intermediate_width():
