@@ -575,6 +575,51 @@ def test_block_backward_operands_from_the_routing_gradient(dtype, H, nk, K):
         assert torch.isfinite(a).all() and rel_fro(a, b) < {torch.float32: 1e-4, torch.bfloat16: 3e-2, torch.float16: 6e-3}[dtype]
 
 
+@pytest.mark.parametrize("dtype,T,H,nk,K", [
+    (torch.bfloat16, 70, 8, 3, 2), (torch.float32, 70, 4, 1, 1), (torch.float16, 300, 776, 65, 17), (torch.bfloat16, 70, 520, 129, 65),
+    (torch.bfloat16, 333, 1032, 256, 128), (torch.float32, 1030, 264, 256, 64), (torch.bfloat16, 2100, 72, 256, 4),
+])
+def test_block_backward_rounds_the_routing_gradient_as_the_launch_of_its_own(dtype, T, H, nk, K):
+    """The gate weights' gradient of the block against fmoe_route_backward and fmoe_router_prologue_backward on the block's own gate
+    gradients, logits and statistics: the same operands of the same products, so the same bits."""
+    from flash_moe import _C
+
+    I, E, g = 64, nk * nk, gen(T + H)
+    rand = lambda *s, std=1.0: (torch.randn(*s, generator=g) * std).to(dtype).cuda()
+    x, dy, dl = rand(T, H), rand(T, H), rand(2, T, nk, std=0.1)
+    w = [rand(*s, std=s[-1] ** -0.5) for s in ((I, H), (I, H), (H, I), (2 * nk, H), (E, H), (E, H))]
+    rm, rv, nbt = torch.zeros(H, device="cuda", dtype=dtype), torch.ones(H, device="cuda", dtype=dtype), torch.zeros((), device="cuda", dtype=torch.int64)
+    L, code, stream, p = _C.lib(), _C.dtype_code(dtype), _C.current_stream(x.device), _C.ptr
+    ext = (T, H, I, nk, E, K, code)
+    saved, ws, ws2 = (torch.zeros(f(*ext), device="cuda", dtype=torch.uint8)
+                      for f in (L.fmoe_block_saved_bytes, L.fmoe_block_workspace_bytes, L.fmoe_block_backward_workspace_bytes))
+    out, logits = torch.empty_like(x), rand(T, 2 * nk)
+    _C.check(L.fmoe_block_forward_save(p(x), *map(p, w), p(rm), p(rv), p(nbt), code, 1, 0.1, 1e-5, T, H, I, E, nk, K, code, 1, p(out), p(logits),
+                                       p(saved), saved.numel(), p(ws), ws.numel(), stream), "forward")
+    dx, dwg, dwu, dwd, dwr, ded, deu = (torch.empty_like(t) for t in (x, *w))
+    _C.check(L.fmoe_block_backward(p(dy), p(dl), p(x), *map(p, w), p(saved), 1, T, H, I, E, nk, K, code, 1, p(dx), p(dwg), p(dwu), p(dwd), p(dwr),
+                                   p(ded), p(deu), p(ws2), ws2.numel(), stream), "backward")
+
+    def at(buffer, offset, shape, dtype):
+        n = torch.Size(shape).numel() * dtype.itemsize
+        return buffer[offset:offset + n].view(dtype).view(shape), offset + (n + 255) // 256 * 256
+
+    # what the forward keeps begins with the logits, the ids, the gates and the statistics, the backward's scratch with the gate gradients
+    logits32, o = at(saved, 0, (T, 2 * nk), torch.float32)
+    ids, o = at(saved, o, (T, K), torch.int64)
+    _, o = at(saved, o, (T, K), dtype)
+    stats, _ = at(saved, o, (2, H), torch.float32)
+    dgates, _ = at(ws2, 0, (T, K), dtype)
+    dlogits32, alone, dx_router = torch.empty(T, 2 * nk, device="cuda"), torch.empty_like(dwr), torch.empty_like(x)
+    extra = dl.transpose(0, 1).reshape(T, 2 * nk).contiguous()
+    _C.check(L.fmoe_route_backward(p(dgates), p(ids), p(logits32), p(extra), T, nk, K, code, 1, p(dlogits32), stream), "route")
+    need = L.fmoe_router_prologue_backward_workspace_bytes(T, H, nk, code)
+    ws3 = torch.empty(need, device="cuda", dtype=torch.uint8)
+    _C.check(L.fmoe_router_prologue_backward(p(dlogits32), p(x), p(w[3]), p(stats), 1, T, H, nk, code, p(dx_router), p(alone), p(ws3), need, stream),
+             "prologue")
+    assert dlogits32.abs().sum() > 0 and torch.equal(dwr, alone)
+
+
 @pytest.mark.parametrize("dtype,T,H,I", [
     (torch.bfloat16, 615, 776, 2072), (torch.float32, 383, 516, 1544),     # dx of the MLP in slices of k: added with the other gradients
     (torch.float16, 2050, 72, 136), (torch.bfloat16, 4101, 520, 264),      # more than one row to a wave, rows beyond the last block
@@ -859,6 +904,39 @@ def test_mlp_backward_swiglu_gradient_in_the_product(dtype, T, H, I):
         for name, got, ref in (("dwd", dwd, dy.double().t() @ h), ("dx", dx, da @ ws[0].double() + db @ ws[1].double()),
                                ("dwg", dwg, da.t() @ x.double()), ("dwu", dwu, db.t() @ x.double())):
             assert rel_fro(got, ref) < GRAD_FRO[dtype], (name, rel_fro(got, ref))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("T,H,I", [
+    (1, 8, 8), (63, 72, 64), (65, 136, 72), (127, 8, 1032), (1025, 1032, 2056),      # 64 x 64 tiles and their edges, one and many rounds
+    (2049, 72, 1032), (4097, 264, 520),                                              # 128 x 128
+])
+def test_mlp_backward_rounds_the_swiglu_gradient_once(dtype, T, H, I):
+    """da, db and h as the products after them read them, from the scratch that begins with h and [da | db]: sums of H products in fp32 and
+    one rounding, at most 2^-8 (2^-11) of a value and 1.66e-3 (2.1e-4) of many in the 2-norm, below 2^-9 (2^-12); with dh rounded on the way
+    it would be 2.3e-3 (2.9e-4) of da and db."""
+    from flash_moe import _C
+
+    g = gen(T + I)
+    rand = lambda *s, std=1.0: (torch.randn(*s, generator=g) * std).to(dtype).cuda()
+    x, dy, saved = rand(T, H), rand(T, H), rand(2, T, I)
+    wg, wu, wd = rand(I, H, std=H**-0.5), rand(I, H, std=H**-0.5), rand(H, I)
+    L, code, p = _C.lib(), _C.dtype_code(dtype), _C.ptr
+    need = L.fmoe_mlp_backward_saved_workspace_bytes(T, H, I, code)
+    ws = torch.empty(need, device="cuda", dtype=torch.uint8)
+    out = [torch.empty_like(t) for t in (dy, wg, wu, wd)]
+    _C.check(L.fmoe_mlp_backward(p(dy), p(x), p(wg), p(wu), p(wd), p(saved), T, H, I, code, *map(p, out), p(ws), need, _C.current_stream(x.device)), "mlp")
+    plane = T * I * 2
+    h = ws[:plane].view(dtype).view(T, I)
+    dab = ws[(plane + 255) // 256 * 256:][:2 * plane].view(dtype).view(T, 2 * I)
+    a, b = saved.double()
+    dh, sig = dy.double() @ wd.double(), torch.sigmoid(a)
+    once = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[dtype]
+    for name, got, want in (("h", h, a * sig * b), ("db", dab[:, I:], dh * a * sig), ("da", dab[:, :I], dh * b * sig * (1 + a * (1 - sig)))):
+        # beside it: the fp32 sums, and half a step of fp16 below its normal range
+        slack = 1e-6 * want.abs().max() + 2.0 ** -25
+        assert ((got.double() - want).abs() <= 1.001 * once * want.abs() + slack).all(), name
+        assert T * I < 4096 or rel_fro(got, want) < once / 2, (name, rel_fro(got, want))
 
 
 @pytest.mark.parametrize("dtype,T,H,I", [
