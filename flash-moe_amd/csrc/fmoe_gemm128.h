@@ -10,7 +10,7 @@
 // half as often, but share them.  Requests in one go before the matrix instructions cost 1 % on average, one every fourth instruction
 // 4 %; requesting A's rows while B's are still read gained nothing, nor did this way for slices of k, or for more tiles than CUs (two
 // workgroups of shared tiles to a CU hide each other's waits: 8192 tokens, 4096 -> 1024 65 us, 74 this way).
-// us, down products in bf16, before | now: 4096 tokens, 4096 -> 1024 37.1 | 34.7; 2048 tokens, 8192 -> 2048 67.1 | 62.2; 3000 tokens,
+// us, down products in bf16, repeated alone, before | now (in the README block, behind the gate/up product, 48.8 | 43): 4096 tokens, 4096 -> 1024 37.1 | 34.7; 2048 tokens, 8192 -> 2048 67.1 | 62.2; 3000 tokens,
 // 2664 -> 1000 34.7 | 31.3; 2500 tokens, 3736 -> 1400 45.3 | 40.9; error against float64 as before.
 #pragma once
 

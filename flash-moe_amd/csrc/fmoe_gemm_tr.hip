@@ -67,7 +67,8 @@ __global__ __launch_bounds__(256, 2) void gemm_gradient_kernel(const T* __restri
 
 // Several products in one launch: the workgroups of member i are first .. first + tiles * slices - 1 (first a multiple of the XCDs; ids
 // past the last are spare), one tile or slice of k each, which the dispatcher hands to compute units as they fall free, longest first.
-// us, dWd, dx, dWg and dWu one after the other and together, bf16: 4096 tokens, 1024 -> 4096 190 -> 152; 615 tokens, 776 -> 2072 35.5 ->
+// us, dWd, dx, dWg and dWu one after the other and together, repeated alone, bf16: 4096 tokens, 1024 -> 4096 190 -> 152 (161 to 177 in a
+// training step, behind what moves its operands out of the L2s); 615 tokens, 776 -> 2072 35.5 ->
 // 23.6; 1000 tokens, 1024 -> 4096 63 -> 49; 130 tokens, 408 -> 1088 17.8 -> 9.4; 5616 tokens, 608 -> 2432 123 -> 82; fp32: 691 tokens, 1056
 // -> 2112 177 -> 133; 103 tokens, 768 -> 1536 33 -> 22.  What is left is what the L2s deliver on 128 x 128 tiles, two to a compute unit
 // (69 GB/s each), and the matrix pipes in fp32.
@@ -294,7 +295,7 @@ int plan_gradient(int M, int N, int K) {
 // Price (us) of a group on tiles of a shape: half (0.4 to 1) of what its items take on slots that hold two workgroups of 128 x 128 (four of
 // 64 x 64) to a compute unit, the rest what they take if the tail were filled, at least the longest chain; per sliced product 4 us and
 // its planes written and read at 6 TB/s.  The rates of a k-tile, with the compute unit full and alone, and the 3.4 % (fp32 2.3) by which the
-// choice misses the best of 72 cuts on average come from 105 backward passes in bf16 (64 to 8192 tokens, 256 to 2048 columns) and 35 in fp32 (there up to
+// choice misses the best of 72 cuts on average come from 105 backward passes in bf16 (64 to 8192 tokens, 256 to 2048 columns) and 44 in fp32 (there up to
 // 16384, best on 128 x 128 tiles from about 4000 tokens on: 4096 tokens, 1024 -> 4096 1258 us one by one, 1238 on 64 x 64, 1176; 5000, 2048
 // -> 5464 4392, 4291, 4176).  64 x 128 tiles would gain half a percent.  Products over tokens (the weight gradients)
 // are sliced from 2048 tokens on.

@@ -1,6 +1,7 @@
 // The FlashMoE block for a few tokens (a generation step, a short prompt), gfx950: stages that do not depend on each other share a
-// launch, the larger grid first, because each of them is bound by its own latency (4 to 9 us for work that the memory would
-// deliver in 1 to 4) or leaves compute units idle.
+// launch, because each of them is bound by its own latency (4 to 9 us for work that the memory would deliver in 1 to 4) or leaves compute
+// units idle.  The MLP's product is dispatched first, but for fp32 down products on the k-splitting tiles, which the selections precede
+// (kSelectFirst).
 //   gate_and_up_kernel       logits = BatchNorm(x) Wr^T   beside   act = silu(x Wg^T) * (x Wu^T)
 //   select_and_down_kernel   product-key selection and gates   beside   the fp32 sums of act Wd^T
 //   expert_token_kernel (fmoe_expert.hip)   the routed experts, plus those sums -> out
